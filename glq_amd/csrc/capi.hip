@@ -2154,7 +2154,7 @@ extern "C" int glqh_e8_quantize(const float *x, const float *table_f32, const fl
 
 int glqh_viterbi_init(void);
 size_t glqh_viterbi_scratch_bytes(int K, int64_t n_tiles);
-int glqh_launch_viterbi(const float *tiles, int64_t n_tiles, int K, uint8_t *scratch, int32_t *states,
+int glqh_launch_viterbi(const float *tiles, int64_t n_tiles, int64_t ld, int K, void *scratch, int32_t *states,
                         float *hat, hipStream_t stream);
 
 extern "C" size_t glqh_trellis_quantize_workspace_bytes(int K, int64_t n_tiles) {
@@ -2171,10 +2171,32 @@ extern "C" int glqh_trellis_quantize_tiles(const float *tiles, int64_t n_tiles, 
     GLQH_REQUIRE(n_tiles >= 1, "trellis quantize: n_tiles=%lld", (long long)n_tiles);
     const size_t need = glqh_viterbi_scratch_bytes(K, n_tiles);
     GLQH_REQUIRE(ws && ws_bytes >= need, "trellis quantize: workspace of %zu bytes needed, got %zu", need, ws_bytes);
-    return glqh_launch_viterbi(tiles, n_tiles, K, (uint8_t *)ws, states_out, hat_out, (hipStream_t)stream);
+    return glqh_launch_viterbi(tiles, n_tiles, 0, K, ws, states_out, hat_out, (hipStream_t)stream);
+}
+
+extern "C" size_t glqh_trellis_quantize_matrix_workspace_bytes(int K, int64_t m, int64_t n) {
+    if (K < 1 || K > 4 || m < 16 || n < 16) return 0;
+    glqh_init();
+    const int64_t tiles = (m / 16) * (n / 16);
+    return glqh_viterbi_scratch_bytes(K, tiles) + (size_t)tiles * 256 * sizeof(int32_t);
 }
 
 int glqh_launch_pack_states(const int32_t *states, int64_t m, int64_t n, int K, void *packed, hipStream_t stream);
+
+extern "C" int glqh_trellis_quantize_matrix(const float *w, int64_t m, int64_t n, int K, void *packed_out, float *recon_out,
+                                            void *ws, size_t ws_bytes, void *stream) {
+    GLQH_INIT();
+    GLQH_REQUIRE(w && packed_out && recon_out, "trellis quantize: null pointer");
+    GLQH_REQUIRE(K >= 1 && K <= 4, "trellis encoder supports K (bits/weight) 1-4, got %d", K);
+    GLQH_REQUIRE(glqh_trellis_kernel_supported(m, n), "trellis pack: m %% 32 and n %% 64 must be 0 (m=%lld, n=%lld)",
+                 (long long)m, (long long)n);
+    const size_t need = glqh_trellis_quantize_matrix_workspace_bytes(K, m, n);
+    GLQH_REQUIRE(ws && ws_bytes >= need, "trellis quantize: workspace of %zu bytes needed, got %zu", need, ws_bytes);
+    const int64_t tiles = (m / 16) * (n / 16);
+    int32_t *states = (int32_t *)((char *)ws + glqh_viterbi_scratch_bytes(K, tiles));   // a multiple of 64 KB
+    int rc = glqh_launch_viterbi(w, tiles, n, K, ws, states, recon_out, (hipStream_t)stream);
+    return rc ? rc : glqh_launch_pack_states(states, m, n, K, packed_out, (hipStream_t)stream);
+}
 
 extern "C" int glqh_trellis_pack_states(const int32_t *states, int64_t m, int64_t n, int K, void *packed_out,
                                         void *stream) {

@@ -6,18 +6,21 @@
 // bits in (state' = (state << K | b) & 0xFFFF) and costs (lut[state'] - x)^2.  With
 // G = 2^(16-K), the predecessors of state' are the 2^K states k*G + (state' >> K), so only
 //     best_i[g] = min_k ( err_{i-1}[k*G + g] + best_{i-1}[(k*G + g) >> K] ),  lowest k on ties,
-// has to be carried from step to step (G floats, double-buffered in LDS); the arg-min k per
-// (step, g) goes to a scratch slab in global memory for the backtrack.  The search runs twice
+// has to be carried from step to step (G floats in LDS).  The search runs twice
 // (glq/trellis.py:479-482): on the sequence rolled by T/2 without constraints, then on the
 // sequence itself with first and last state tied to the overlap the first pass found.
 // All arithmetic is fp32 with separate subtract, multiply and add (no contraction), the
-// input is rounded to fp16 first (glq/trellis.py:468), lut = decode_3inst computed on the fly.
+// input is rounded to fp16 first (glq/trellis.py:468).
 //
-// One workgroup (16 waves) per tile at a time; workgroups are persistent and walk the tiles
-// with a fixed stride, each owning one scratch slab.  At K = 1 the two buffers of G = 32768
-// floats do not fit the LDS together: the new costs of a step go through a slab of global
-// scratch (each thread reads back what it wrote itself) into the one LDS buffer once every
-// thread has finished reading the old ones.
+// What bounds it is vector-ALU issue: 65536 states per step, 510 steps per tile.  A workgroup
+// therefore keeps the whole table in registers, two fp16 values to a register (v_fma_mix_f32
+// subtracts the input from either half with fp32 rounding), and a state costs 3.5 instructions:
+// subtract, multiply, add, half a three-way minimum.  The arg-min is not tracked: every
+// `VT_DEPTH`-th cost row goes to scratch and the backtrack, one wave, recomputes the 2^(K*depth)
+// costs below its state for `depth` steps at a time.  2048 x 2048 weights at K = 4: 165 ms (hash per
+// state and step, compare and two selects per state, a byte of arg-min per step and group) -> 69.6 ms,
+// vector ALUs issuing in 74 % of the cycles at 2.4 GHz (30.8 M instructions per SIMD, of which 29.9 M
+// are the 3.5 per state).
 #include "common.h"
 #include "trellis_device.h"
 
@@ -25,7 +28,6 @@
 
 namespace {
 
-constexpr int VT_THREADS = 1024;
 constexpr int VT_T = 256;
 
 struct vt_best {
@@ -33,121 +35,283 @@ struct vt_best {
     int state;
 };
 
-// One pass.  x: T inputs in LDS; best: 2*G floats in LDS; from_k: T*G bytes of scratch;
-// overlap < 0: unconstrained.  Returns, in `states` (LDS, T ints), the best state sequence.
+// A thread owns UNITS units of LOWS neighbouring groups that share their predecessors' groups
+// (g >> K): unit u holds groups u*LOWS .. u*LOWS + LOWS-1 under predecessor group hi(u), and
+// neighbouring threads own neighbouring units, so that cost reads are conflict-free and cost
+// writes are whole 8..32-byte runs.  512 threads and at most 128 registers for K >= 2: two
+// workgroups per CU, one of which computes while the other's single wave walks back.  At K = 1 the
+// cost row alone is 128 KB of LDS: one workgroup of 1024.
 template <int K>
-__device__ __forceinline__ void viterbi_pass(const float *x, float *best, uint8_t *__restrict__ from_k,
-                                             float *__restrict__ spill, int overlap, int *states,
-                                             vt_best *red) {
-    constexpr int G = 1 << (16 - K);
-    constexpr int NK = 1 << K;
-    constexpr int PER = G / VT_THREADS;                       // groups per thread
-    const float inf = __builtin_inff();
-    constexpr bool ONE_BUF = K == 1;
-    float *cur = best, *nxt = ONE_BUF ? spill : best + G;
-    for (int g = threadIdx.x; g < G; g += VT_THREADS) cur[g] = (overlap < 0 || g == overlap) ? 0.0f : inf;
-    __syncthreads();
-    for (int i = 1; i < VT_T; ++i) {
-        const float xi = x[i - 1];
-#pragma unroll 1
-        for (int u = 0; u < PER; ++u) {
-            const int g = threadIdx.x + u * VT_THREADS;
-            float bc = 0.0f;
-            int bk = 0;
-#pragma unroll
-            for (int k = 0; k < NK; ++k) {
-                const int s = k * G + g;
-                const float d = (float)tr_weight((uint32_t)s) - xi;
-                const float e = d * d;
-                const float c = e + cur[s >> K];
-                if (k == 0 || c < bc) { bc = c; bk = k; }
-            }
-            nxt[g] = bc;
-            from_k[(int64_t)i * G + g] = (uint8_t)bk;
-        }
-        __syncthreads();
-        if constexpr (ONE_BUF) {
-#pragma unroll 4
-            for (int u = 0; u < PER; ++u) cur[threadIdx.x + u * VT_THREADS] = nxt[threadIdx.x + u * VT_THREADS];
-            __syncthreads();
-        } else {
-            float *t = cur; cur = nxt; nxt = t;
-        }
-    }
-    // final costs, with the tail-biting mask on the low 16-K bits; lowest state on ties
-    {
-        const float xi = x[VT_T - 1];
-        float bc = inf;
-        int bs = 0x7fffffff;
-#pragma unroll 1
-        for (int u = 0; u < PER; ++u) {
-            const int g = threadIdx.x + u * VT_THREADS;
-#pragma unroll
-            for (int k = 0; k < NK; ++k) {
-                const int s = k * G + g;
-                const float d = (float)tr_weight((uint32_t)s) - xi;
-                const float e = d * d;
-                float c = e + cur[s >> K];
-                if (overlap >= 0 && g != overlap) c = inf;
-                if (c < bc || (c == bc && s < bs)) { bc = c; bs = s; }
-            }
-        }
-        // wave, then workgroup reduction of (cost, state)
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) {
-            const float oc = __shfl_xor(bc, o, GLQH_WAVE);
-            const int os = __shfl_xor(bs, o, GLQH_WAVE);
-            if (oc < bc || (oc == bc && os < bs)) { bc = oc; bs = os; }
-        }
-        if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = vt_best{bc, bs};
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            vt_best b = red[0];
-            for (int w = 1; w < VT_THREADS / 64; ++w)
-                if (red[w].cost < b.cost || (red[w].cost == b.cost && red[w].state < b.state)) b = red[w];
-            // every state is infinite only if the constraint is unsatisfiable, which the
-            // first pass rules out; argmin of an all-inf row is state 0 in the reference
-            int s = b.state == 0x7fffffff ? 0 : b.state;
-            states[VT_T - 1] = s;
-            for (int i = VT_T - 1; i > 0; --i) {              // backtrack
-                const int g = s >> K;
-                const uint8_t kk = __hip_atomic_load(from_k + (int64_t)i * G + g, __ATOMIC_RELAXED,
-                                                     __HIP_MEMORY_SCOPE_AGENT);   // written by other waves
-                s = g + ((int)kk << (16 - K));
-                states[i - 1] = s;
-            }
-        }
-        __syncthreads();
-    }
+struct vt_cfg {
+    static constexpr int G = 1 << (16 - K), NK = 1 << K;
+    static constexpr int THREADS = K == 1 ? 1024 : 512;
+    static constexpr int PER = G / THREADS;                    // groups per thread
+    static constexpr int LOWS = K == 4 ? 8 : NK;               // K = 4: two threads per predecessor group
+    static constexpr int UNITS = PER / LOWS;
+    static constexpr int HI = G >> K;                          // predecessor groups
+    // two cost rows where they fit the LDS twice per CU, else one (every thread reads, then all write)
+    static constexpr bool TWO_ROWS = K >= 3;
+    static constexpr int ROWS = TWO_ROWS ? 2 : 1;
+    // steps per stored cost row: 16 KB of cost rows per step at most (8 KB at K = 4), 64 or 256 leaves
+    static constexpr int DEPTH = K == 1 ? 8 : K == 2 ? 4 : 2;
+};
+
+// LDS only: a __syncthreads() would also wait for the cost rows on their way to scratch
+__device__ __forceinline__ void vt_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// (float)half - x, rounded once; exact halves of a packed register, x the same for the whole wave
+__device__ __forceinline__ float vt_sub_lo(f16x2 w, float x) {
+    float d;
+    asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel:[0,0,0] op_sel_hi:[1,0,0]" : "=v"(d) : "v"(w), "s"(x));
+    return d;
+}
+__device__ __forceinline__ float vt_sub_hi(f16x2 w, float x) {
+    float d;
+    asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(d) : "v"(w), "s"(x));
+    return d;
 }
 
+__device__ __forceinline__ float vt_err(int s, float x) {
+    const float d = (float)tr_weight((uint32_t)s) - x;
+    return d * d;
+}
+
+// States i-1 .. i-D from state s of step i (one wave): the costs of the NK^D paths into s from the
+// cost row of step i-D, minimised level by level, lowest k on ties.  cost, pick: 256 words each of LDS.
+template <int K, int D>
+__device__ __forceinline__ int vt_back(int i, int s, const float *__restrict__ row, const float *x, float *cost,
+                                       int *pick, int *states) {
+    constexpr int G = vt_cfg<K>::G, NK = vt_cfg<K>::NK;
+    constexpr int LEAVES = 1 << (K * D);
+    int lane = threadIdx.x & 63;
+    asm volatile("" : "+v"(lane));                             // keeps what follows from it out of the callers' registers
+    // state reached from s by the digits of p (e digits, most significant first)
+    auto walk = [&](int p, int e) {
+        int st = s;
+        for (int q = e - 1; q >= 0; --q) st = (st >> K) + ((p >> (K * q)) & (NK - 1)) * G;
+        return st;
+    };
+#pragma unroll
+    for (int r = 0; r < (LEAVES + 63) / 64; ++r) {
+        const int p = lane + 64 * r;
+        if (p < LEAVES) {
+            const int st = walk(p, D);
+            // rows were written by other waves of this workgroup: past the L1
+            const float b = __hip_atomic_load(row + (st >> K), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            cost[p] = vt_err(st, x[i - D]) + b;
+        }
+    }
+    __builtin_amdgcn_wave_barrier();
+    int base = 0;                                              // pick: level D first, then D-1, ...
+#pragma unroll
+    for (int e = D; e >= 1; --e) {
+        const int groups = 1 << (K * (e - 1));
+        float nc[2];
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+            const int p = lane + 64 * r;
+            if (p < groups) {
+                float bc = cost[p * NK];
+                int bk = 0;
+#pragma unroll
+                for (int k = 1; k < NK; ++k) {
+                    const float c = cost[p * NK + k];
+                    if (c < bc) { bc = c; bk = k; }
+                }
+                pick[base + p] = bk;
+                nc[r] = e > 1 ? vt_err(walk(p, e - 1), x[i - e + 1]) + bc : bc;
+            }
+        }
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int r = 0; r < 2; ++r)
+            if (lane + 64 * r < groups) cost[lane + 64 * r] = nc[r];
+        __builtin_amdgcn_wave_barrier();
+        base += groups;
+    }
+    // the picks from the top: level 1 is the last one stored
+    int p = 0;
+#pragma unroll
+    for (int e = 1; e <= D; ++e) {
+        base -= 1 << (K * (e - 1));
+        p = p * NK + pick[base + p];
+        const int st = walk(p, e);
+        if (lane == 0) states[i - e] = st;
+        if (e == D) s = st;
+    }
+    __builtin_amdgcn_wave_barrier();
+    return __builtin_amdgcn_readfirstlane(s);
+}
+
+// One pass.  x: T inputs in LDS; best: ROWS * G floats in LDS; hist: cost rows of steps 0, DEPTH,
+// 2*DEPTH, ... in scratch; overlap < 0: unconstrained.  Leaves the best state sequence in `states`
+// (LDS), from step `first` on.
 template <int K>
-__global__ void __launch_bounds__(VT_THREADS)
-viterbi_kernel(const float *__restrict__ tiles, int64_t n_tiles, uint8_t *__restrict__ scratch,
+__device__ __forceinline__ void viterbi_pass(const f16x2 (&w)[32768 / vt_cfg<K>::THREADS], const float *x, float *best,
+                                             float *__restrict__ hist, int overlap, int first, int *states, vt_best *red,
+                                             float *cost, int *pick) {
+    using C = vt_cfg<K>;
+    constexpr int G = C::G, NK = C::NK, LOWS = C::LOWS, UNITS = C::UNITS, D = C::DEPTH;
+    const int tid = threadIdx.x;
+    const float inf = __builtin_inff();
+    float *cur = best, *nxt = C::TWO_ROWS ? best + G : best;
+    for (int g = tid; g < G; g += C::THREADS) {
+        const float v = (overlap < 0 || g == overlap) ? 0.0f : inf;
+        cur[g] = v;
+        if (first == 0) hist[g] = v;
+    }
+    vt_barrier();
+    auto hi_of = [&](int q) { return K == 4 ? tid >> 1 : tid + q * C::THREADS; };
+    float xn = x[0];                                           // a step's input, read a step ahead
+#pragma unroll 1
+    for (int i = 1; i < VT_T; ++i) {
+        const float xi = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, xn)));
+        xn = x[i];
+        float *row = (i % D == 0 && i >= first - D) ? hist + (int64_t)(i / D) * G : nullptr;   // uniform
+        float c[UNITS][NK];
+        auto load = [&](int q) {
+#pragma unroll
+            for (int k = 0; k < NK; ++k) c[q][k] = cur[k * C::HI + hi_of(q)];
+        };
+        if constexpr (!C::TWO_ROWS) {
+#pragma unroll
+            for (int q = 0; q < UNITS; ++q) load(q);
+            vt_barrier();
+        }
+#pragma unroll
+        for (int q = 0; q < UNITS; ++q) {
+            if constexpr (C::TWO_ROWS) load(q);
+            float m[LOWS];
+#pragma unroll
+            for (int j = 0; j < LOWS; j += 2) {
+                float a[NK], b[NK];
+#pragma unroll
+                for (int k = 0; k < NK; ++k) {
+                    const f16x2 wk = w[(k * UNITS + q) * (LOWS / 2) + j / 2];
+                    const float d0 = vt_sub_lo(wk, xi), d1 = vt_sub_hi(wk, xi);
+                    a[k] = d0 * d0 + c[q][k];
+                    b[k] = d1 * d1 + c[q][k];
+                }
+                float ma = a[0], mb = b[0];
+                if constexpr (NK == 2) {
+                    ma = __builtin_fminf(ma, a[1]);
+                    mb = __builtin_fminf(mb, b[1]);
+                } else {
+#pragma unroll
+                    for (int k = 1; k + 1 < NK; k += 2) {
+                        ma = __builtin_fminf(__builtin_fminf(ma, a[k]), a[k + 1]);
+                        mb = __builtin_fminf(__builtin_fminf(mb, b[k]), b[k + 1]);
+                    }
+                    ma = __builtin_fminf(ma, a[NK - 1]);
+                    mb = __builtin_fminf(mb, b[NK - 1]);
+                }
+                m[j] = ma;
+                m[j + 1] = mb;
+                __builtin_amdgcn_sched_barrier(0);             // one pair of groups at a time: no spills in this loop
+            }
+            const int g = (tid + q * C::THREADS) * LOWS;
+            if constexpr (LOWS == 2) {
+                *(f32x2 *)(nxt + g) = f32x2{m[0], m[1]};
+                if (row) *(f32x2 *)(row + g) = f32x2{m[0], m[1]};
+            } else {
+#pragma unroll
+                for (int j = 0; j < LOWS; j += 4) {
+                    const f32x4 v = {m[j], m[j + 1], m[j + 2], m[j + 3]};
+                    *(f32x4 *)(nxt + g + j) = v;
+                    if (row) *(f32x4 *)(row + g + j) = v;
+                }
+            }
+        }
+        vt_barrier();
+        if constexpr (C::TWO_ROWS) { float *t = cur; cur = nxt; nxt = t; }
+    }
+    // final costs, with the tail-biting mask on the low 16-K bits; lowest state on ties
+    const float xl = x[VT_T - 1];
+    float bc = inf;
+    int bs = 0x7fffffff;
+#pragma unroll 1
+    for (int s = tid; s < 65536; s += C::THREADS) {
+        float c = vt_err(s, xl) + cur[s >> K];
+        if (overlap >= 0 && (s & (G - 1)) != overlap) c = inf;
+        if (c < bc || (c == bc && s < bs)) { bc = c; bs = s; }
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        const float oc = __shfl_xor(bc, o, GLQH_WAVE);
+        const int os = __shfl_xor(bs, o, GLQH_WAVE);
+        if (oc < bc || (oc == bc && os < bs)) { bc = oc; bs = os; }
+    }
+    if ((tid & 63) == 0) red[tid >> 6] = vt_best{bc, bs};
+    __syncthreads();                                           // and every stored cost row has arrived
+    if (tid < GLQH_WAVE) {
+        vt_best b = red[0];
+        for (int v = 1; v < C::THREADS / 64; ++v)
+            if (red[v].cost < b.cost || (red[v].cost == b.cost && red[v].state < b.state)) b = red[v];
+        // every state is infinite only if the constraint is unsatisfiable, which the
+        // first pass rules out; argmin of an all-inf row is state 0 in the reference
+        int s = __builtin_amdgcn_readfirstlane(b.state == 0x7fffffff ? 0 : b.state);
+        if (tid == 0) states[VT_T - 1] = s;
+        constexpr int REST = (VT_T - 1) % D;                   // steps above the last stored row
+        int i = VT_T - 1;
+        s = vt_back<K, REST>(i, s, hist + (int64_t)((i - REST) / D) * G, x, cost, pick, states);
+        i -= REST;
+#pragma unroll 1
+        for (; i > first; i -= D) s = vt_back<K, D>(i, s, hist + (int64_t)(i / D - 1) * G, x, cost, pick, states);
+    }
+    __syncthreads();
+}
+
+// Position (row * 16 + col) of trellis step t = 8l + j inside its 16x16 tile (glq/trellis.py:99-101).
+__device__ __forceinline__ int64_t vt_step_pos(int t, int64_t ld) {
+    const int l = t >> 3, j = t & 7;
+    return (int64_t)((l >> 2) + 8 * ((j >> 1) & 1)) * ld + 2 * (l & 3) + 8 * (j >> 2) + (j & 1);
+}
+
+// Persistent workgroups walk the tiles with a fixed stride, each owning one slab of cost rows.
+// ld > 0: tiles_in and hat_out are (m, n) matrices of row length ld, the tiles their 16x16 blocks in
+// row-major order; ld == 0: (tiles, 256) rows in step order.
+template <int K>
+__global__ void __launch_bounds__(vt_cfg<K>::THREADS, 4)
+viterbi_kernel(const float *__restrict__ tiles_in, int64_t n_tiles, int64_t ld, float *__restrict__ scratch,
                int32_t *__restrict__ states_out, float *__restrict__ hat_out) {
-    constexpr int G = 1 << (16 - K);
-    extern __shared__ float best[];                            // 2 * G floats (G at K = 1)
-    __shared__ float x[VT_T], xr[VT_T];
-    __shared__ int states[VT_T];
-    __shared__ vt_best red[VT_THREADS / 64];
-    uint8_t *from_k = scratch + (int64_t)blockIdx.x * VT_T * G;
-    // K = 1: the spill slabs follow the back-pointer slabs of all workgroups
-    float *spill = K == 1 ? (float *)(scratch + (int64_t)gridDim.x * VT_T * G) + (int64_t)blockIdx.x * G : nullptr;
+    using C = vt_cfg<K>;
+    constexpr int G = C::G;
+    extern __shared__ float best[];                            // ROWS * G floats
+    __shared__ float x[VT_T], xr[VT_T], cost[VT_T];
+    __shared__ int states[VT_T], pick[VT_T];
+    __shared__ vt_best red[C::THREADS / 64];
+    const int tid = threadIdx.x;
+    float *hist = scratch + (int64_t)blockIdx.x * (VT_T / C::DEPTH) * G;
+    f16x2 w[32768 / C::THREADS];
+#pragma unroll
+    for (int k = 0; k < C::NK; ++k)
+#pragma unroll
+        for (int q = 0; q < C::UNITS; ++q)
+#pragma unroll
+            for (int j = 0; j < C::LOWS; j += 2) {
+                const uint32_t s = (uint32_t)(k * G + (tid + q * C::THREADS) * C::LOWS + j);
+                f16x2 v = {tr_weight(s), tr_weight(s + 1)};
+                asm volatile("" : "+v"(v));                    // finished here: neither spilled half-done nor recomputed
+                w[(k * C::UNITS + q) * (C::LOWS / 2) + j / 2] = v;
+            }
     for (int64_t tile = blockIdx.x; tile < n_tiles; tile += gridDim.x) {
-        if (threadIdx.x < VT_T) {
-            const float v = (float)(f16)tiles[tile * VT_T + threadIdx.x];
-            x[threadIdx.x] = v;
-            xr[(threadIdx.x + VT_T / 2) & (VT_T - 1)] = v;    // np.roll(x, T/2)
+        const int64_t per_row = ld >> 4;
+        const int64_t at = ld ? (tile / per_row) * 16 * ld + (tile % per_row) * 16 : tile * VT_T;
+        const int64_t pos = ld ? at + vt_step_pos(tid & 255, ld) : at + (tid & 255);
+        if (tid < VT_T) {
+            const float v = (float)(f16)tiles_in[pos];
+            x[tid] = v;
+            xr[(tid + VT_T / 2) & (VT_T - 1)] = v;             // np.roll(x, T/2)
         }
         __syncthreads();
-        viterbi_pass<K>(xr, best, from_k, spill, -1, states, red);
+        viterbi_pass<K>(w, xr, best, hist, -1, VT_T / 2, states, red, cost, pick);
         const int overlap = states[VT_T / 2] >> K;
         __syncthreads();
-        viterbi_pass<K>(x, best, from_k, spill, overlap, states, red);
-        if (threadIdx.x < VT_T) {
-            const int s = states[threadIdx.x];
-            states_out[tile * VT_T + threadIdx.x] = s;
-            hat_out[tile * VT_T + threadIdx.x] = (float)tr_weight((uint32_t)s);
+        viterbi_pass<K>(w, x, best, hist, overlap, 0, states, red, cost, pick);
+        if (tid < VT_T) {
+            const int s = states[tid];
+            states_out[tile * VT_T + tid] = s;
+            hat_out[pos] = (float)tr_weight((uint32_t)s);
         }
         __syncthreads();
     }
@@ -239,48 +403,47 @@ int acs_launch(const float *cost, const void *x, const float *lut, float *cost_o
 }
 
 template <int K>
-int vt_launch(const float *tiles, int64_t n_tiles, uint8_t *scratch, int grid, int32_t *states, float *hat,
+int vt_launch(const float *tiles, int64_t n_tiles, int64_t ld, void *scratch, int grid, int32_t *states, float *hat,
               hipStream_t stream) {
-    constexpr size_t lds = (K == 1 ? 1 : 2) * sizeof(float) * ((size_t)1 << (16 - K));
-    hipLaunchKernelGGL(viterbi_kernel<K>, dim3((unsigned)grid), dim3(VT_THREADS), lds, stream, tiles, n_tiles,
-                       scratch, states, hat);
+    constexpr size_t lds = vt_cfg<K>::ROWS * sizeof(float) * (size_t)vt_cfg<K>::G;
+    hipLaunchKernelGGL(viterbi_kernel<K>, dim3((unsigned)grid), dim3(vt_cfg<K>::THREADS), lds, stream, tiles, n_tiles, ld,
+                       (float *)scratch, states, hat);
     GLQH_LAUNCH_CHECK("viterbi launch");
     return 0;
 }
 
-template <typename Kn>
-int vt_set_lds(Kn kernel, size_t bytes) {
-    return glqh_check_hip(hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                              (int)bytes),
+template <int K>
+int vt_set_lds() {
+    return glqh_check_hip(hipFuncSetAttribute((const void *)viterbi_kernel<K>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                              (int)(vt_cfg<K>::ROWS * sizeof(float) * vt_cfg<K>::G)),
                           "viterbi attribute");
 }
 
 }  // namespace
 
-int glqh_viterbi_init(void) {
-    return vt_set_lds(viterbi_kernel<1>, 4 * 32768) || vt_set_lds(viterbi_kernel<2>, 2 * 4 * 16384) || vt_set_lds(viterbi_kernel<3>, 2 * 4 * 8192) ||
-           vt_set_lds(viterbi_kernel<4>, 2 * 4 * 4096);
-}
+int glqh_viterbi_init(void) { return vt_set_lds<1>() || vt_set_lds<2>() || vt_set_lds<3>() || vt_set_lds<4>(); }
 
-// persistent workgroups: one per CU (K = 2 fills the LDS of a CU), two for K >= 3
+// persistent workgroups: two per CU, one at K = 1 (its cost row fills the LDS)
 int glqh_viterbi_grid(int K, int64_t n_tiles) {
-    int64_t g = (int64_t)glqh_device_cus() * (K >= 3 ? 2 : 1);
+    const int64_t g = (int64_t)glqh_device_cus() * (K >= 2 ? 2 : 1);
     return (int)(n_tiles < g ? n_tiles : g);
 }
 
 size_t glqh_viterbi_scratch_bytes(int K, int64_t n_tiles) {
-    const size_t G = (size_t)1 << (16 - K);
-    return (size_t)glqh_viterbi_grid(K, n_tiles) * (VT_T * G + (K == 1 ? G * sizeof(float) : 0));
+    const size_t row = sizeof(float) << (16 - K);
+    const int depth = K == 1 ? vt_cfg<1>::DEPTH : K == 2 ? vt_cfg<2>::DEPTH : K == 3 ? vt_cfg<3>::DEPTH : vt_cfg<4>::DEPTH;
+    return (size_t)glqh_viterbi_grid(K, n_tiles) * (VT_T / depth) * row;
 }
 
-int glqh_launch_viterbi(const float *tiles, int64_t n_tiles, int K, uint8_t *scratch, int32_t *states,
+// ld: 0 for tiles in step order, else the row length of the (m, n) matrices `tiles` and `hat`
+int glqh_launch_viterbi(const float *tiles, int64_t n_tiles, int64_t ld, int K, void *scratch, int32_t *states,
                         float *hat, hipStream_t stream) {
     const int grid = glqh_viterbi_grid(K, n_tiles);
     switch (K) {
-    case 1: return vt_launch<1>(tiles, n_tiles, scratch, grid, states, hat, stream);
-    case 2: return vt_launch<2>(tiles, n_tiles, scratch, grid, states, hat, stream);
-    case 3: return vt_launch<3>(tiles, n_tiles, scratch, grid, states, hat, stream);
-    case 4: return vt_launch<4>(tiles, n_tiles, scratch, grid, states, hat, stream);
+    case 1: return vt_launch<1>(tiles, n_tiles, ld, scratch, grid, states, hat, stream);
+    case 2: return vt_launch<2>(tiles, n_tiles, ld, scratch, grid, states, hat, stream);
+    case 3: return vt_launch<3>(tiles, n_tiles, ld, scratch, grid, states, hat, stream);
+    case 4: return vt_launch<4>(tiles, n_tiles, ld, scratch, grid, states, hat, stream);
     }
     return glqh_fail("trellis encoder supports K (bits/weight) 1-4, got %d", K);
 }

@@ -1189,6 +1189,13 @@ def trellis_quantize_matrix(W_rht, K):
     """Normalised RHT-domain weight (m, n) -> (trellis_packed, reconstruction (m, n) fp32):
     tiles -> tail-biting Viterbi -> pack (the identity-Hessian case of
     quantize_layer_trellis_rht, glq/trellis.py:649-688)."""
+    lib = _lib.load()
     m, n = W_rht.shape
-    hat, states = trellis_quantize_tiles(trellis_matrix_to_tiles(W_rht.to(torch.float32)), K)
-    return trellis_pack_states(states, m, n, K), trellis_tiles_to_matrix(hat, m, n)
+    W = W_rht.to(torch.float32).contiguous()
+    _chk(W, "W_rht", torch.float32)
+    packed = torch.empty(((m // 16) * (n // 16), 16 * int(K)), dtype=torch.int16, device=W.device)
+    recon = torch.empty_like(W)
+    with torch.cuda.device(W.device):
+        ws = _ws(lib.glqh_trellis_quantize_matrix_workspace_bytes(int(K), m, n), W.device)
+        check(lib.glqh_trellis_quantize_matrix(_p(W), m, n, int(K), _p(packed), _p(recon), _p(ws), ws.numel(), _stream()))
+    return packed, recon

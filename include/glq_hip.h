@@ -469,6 +469,14 @@ size_t glqh_trellis_quantize_workspace_bytes(int K, int64_t n_tiles);
 int glqh_trellis_quantize_tiles(const float *tiles, int64_t n_tiles, int K, int32_t *states_out,
                                 float *hat_out, void *ws, size_t ws_bytes, void *stream);
 
+size_t glqh_trellis_quantize_matrix_workspace_bytes(int K, int64_t m, int64_t n);
+
+/* The same search over the 16x16 tiles of a row-major (m, n) fp32 matrix: packed_out in the kernel layout
+ * ((m/16)(n/16), 16K int16), recon_out (m, n) fp32.  quantize_layer_trellis_rht with an identity Hessian
+ * (glq/trellis.py:649-688). */
+int glqh_trellis_quantize_matrix(const float *w, int64_t m, int64_t n, int K, void *packed_out, float *recon_out,
+                                 void *ws, size_t ws_bytes, void *stream);
+
 /* One add-compare-select step of that search on cost rows in memory, for callers that
  * drive the search step by step: cost (B, 65536) fp32 -> cost_out (B, 65536) fp32 and
  * prev_out (B, 2^(16-K)) int32, with x (B) fp16 the step's inputs and lut (65536) fp32 the

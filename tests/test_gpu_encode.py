@@ -111,3 +111,21 @@ def test_quantize_matrix_round_trip():
     assert np.array_equal(packed.cpu().numpy(), O.pack_layer_from_states(st_ref, m, n, K))
     err = float(((recon.cpu() - W) ** 2).sum() / (W ** 2).sum())
     assert err < 0.02, err
+
+
+@pytest.mark.parametrize("K,m,n", [(1, 32, 64), (2, 96, 64), (3, 32, 320), (4, 64, 192)])
+def test_quantize_matrix_equals_the_tile_route(K, m, n):
+    """The entry that reads and writes whole matrices against tiles -> search -> pack -> matrix, bit for bit, with
+    inputs that leave a tile's costs tied (a constant block) and large ones."""
+    from glq_amd import ext
+    say("quantize matrix", K, m, n)
+    W = torch.randn(m, n, generator=torch.Generator().manual_seed(K)) * 0.9
+    W[:16, :16] = 0.25
+    W[16:, 16:] *= 4.0
+    W = W.to(DEV)
+    packed, recon = ext.trellis_quantize_matrix(W, K)
+    hat, states = ext.trellis_quantize_tiles(ext.trellis_matrix_to_tiles(W), K)
+    assert torch.equal(packed, ext.trellis_pack_states(states, m, n, K))
+    assert torch.equal(recon, ext.trellis_tiles_to_matrix(hat, m, n))
+    if K > 1:                                            # the dequantizer takes 2..4 bits
+        assert torch.equal(ext.glq_decompress_trellis_3inst_cuda(packed, m, n).float(), recon)
