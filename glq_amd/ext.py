@@ -1083,6 +1083,54 @@ def glq_fused_linear_block_diag_cuda(x, sv, su, qidxs, codebook, wscale, in_feat
 
 
 # ---- encode side ----------------------------------------------------------------------
+_SHELL_PLANS = _DerivedCache()
+_SHELL_COUNTS = (1, 240, 2160, 6720, 17520, 30240)            # E8 points of norm 0, 2, .. 10
+# Tables of a few hundred rows (the secondary table of 3 bpw has 256) are walked in as little time.
+_SHELL_MIN_ROWS = 4096
+
+
+class _ShellPlan:
+    """What the search on the whole shell table needs beside it, derived once per table: fp32 rows and norms, the
+    hash of the rows, matrix operands of the rows of norm 12.  `ok` is False for any other table."""
+
+    def __init__(self, codebook, norms):
+        lib = _lib.load()
+        # copies: the cache must not keep alive the tensors whose end drops its entry
+        self.table = codebook.to(torch.float32, copy=True).contiguous()
+        self.norms = (self.table * self.table).sum(-1) if norms is None else norms.to(torch.float32, copy=True).contiguous()
+        self.given = None if norms is None else weakref.ref(norms.untyped_storage())
+        self.ok = False
+        if self.table.shape[0] < _SHELL_MIN_ROWS or self.norms.numel() != self.table.shape[0]:
+            return
+        i32 = dict(dtype=torch.int32, device=self.table.device)
+        n = self.table.shape[0]
+        keys, vals, counts = torch.empty(1 << 17, **i32), torch.empty(1 << 17, **i32), torch.empty(8, **i32)
+        rem_rows = torch.empty(n + 64, **i32)
+        check(lib.glqh_e8_shell_index(_p(self.table), _p(self.norms), n, _p(keys), _p(vals), _p(counts), _p(rem_rows),
+                                      _stream()))
+        counts = counts.tolist()
+        if tuple(counts[:6]) != _SHELL_COUNTS or counts[7] != 0:
+            return
+        self.n_rem = counts[6]
+        ops = torch.empty(max(1, -(-self.n_rem // 64)) * 1024, dtype=torch.float16, device=self.table.device)
+        check(lib.glqh_e8_shell_operands(_p(self.table), _p(rem_rows), self.n_rem, _p(ops), _stream()))
+        self.keys, self.vals, self.rem_rows, self.ops = keys, vals, rem_rows[:-(-self.n_rem // 64) * 64].clone(), ops
+        self.ok = True
+
+
+def _shell_plan(codebook, norms):
+    """The plan of a table, made on its first use outside stream capture; None where there is none."""
+    if codebook.dim() != 2 or codebook.shape[1] != 8 or not _SHELL_MIN_ROWS <= codebook.shape[0] <= 65536:
+        return None
+    extra = () if norms is None else _skey(norms)
+    plan = _SHELL_PLANS.get(codebook, extra)
+    if plan is None or (norms is not None and plan.given() is not norms.untyped_storage()):
+        if torch.cuda.is_current_stream_capturing():
+            return None
+        plan = _SHELL_PLANS.put(codebook, _ShellPlan(codebook, norms), extra)
+    return plan if plan.ok else None
+
+
 def e8_quantize(x, codebook, codebook_norms=None, return_decoded=True):
     """E8ShellCodebook.quantize (glq/codebook.py:227-278) on the GPU: nearest row of
     `codebook` (K, 8) for every row of x (N, 8), lowest index on ties.  fp32 arithmetic in
@@ -1092,13 +1140,20 @@ def e8_quantize(x, codebook, codebook_norms=None, return_decoded=True):
         raise RuntimeError(f"x must be (N, 8), got {tuple(x.shape)}")
     xf = x.contiguous().to(torch.float32)
     _chk(xf, "x", torch.float32)
-    cb = codebook.contiguous().to(torch.float32)
-    norms = (cb * cb).sum(-1) if codebook_norms is None else codebook_norms.contiguous().to(torch.float32)
     N = xf.shape[0]
     idx = torch.empty(N, dtype=torch.int64, device=x.device)
     dec = torch.empty(N, 8, dtype=torch.float32, device=x.device) if return_decoded else None
     if N:
         with torch.cuda.device(x.device):
+            plan = _shell_plan(codebook, codebook_norms)
+            if plan is not None:
+                ws = _ws(lib.glqh_e8_shell_workspace_bytes(N), x.device)
+                check(lib.glqh_e8_shell_quantize(
+                    _p(xf), N, _p(plan.table), _p(plan.norms), plan.table.shape[0], _p(plan.keys), _p(plan.vals),
+                    _p(plan.ops), _p(plan.rem_rows), plan.n_rem, _p(idx), _p(dec), _p(ws), ws.numel(), _stream()))
+                return dec, idx
+            cb = codebook.contiguous().to(torch.float32)
+            norms = (cb * cb).sum(-1) if codebook_norms is None else codebook_norms.contiguous().to(torch.float32)
             check(lib.glqh_e8_quantize(_p(xf), _p(cb), _p(norms), N, cb.shape[0], _p(idx), _p(dec), _stream()))
     return dec, idx
 

@@ -31,6 +31,8 @@ def test_e8_quantize_matches_oracle_indices():
     bad = np.nonzero(idx != idx_ref)[0]
     assert bad.size == 0, (bad[:5], idx[bad[:5]], idx_ref[bad[:5]])
     assert np.array_equal(dec.cpu().numpy(), dec_ref)
+    # the walk over the rows, which tables that are not the whole shell table take
+    assert np.array_equal(ext.e8_quantize(t(X), t(cb[:65000]))[1].cpu().numpy(), O.e8_quantize(X, cb[:65000])[1])
     # secondary table of the 3 bpw recipe
     _, i2_ref = O.e8_quantize(X[:1000], cb[:256])
     _, i2 = ext.e8_quantize(t(X[:1000]), t(cb[:256]))
@@ -51,6 +53,38 @@ def test_e8_quantize_residual_stage_and_size():
     assert np.array_equal(i1.cpu().numpy(), j1) and np.array_equal(i2.cpu().numpy(), j2)
     again = ext.e8_quantize(t(X), t(cb))[1]
     assert torch.equal(i1, again)
+
+
+@pytest.mark.parametrize("N,scale", [(1, 1.0), (255, 3.0), (257, 0.3), (5000, 1.5), (70001, 1.0), (262145, 1.0)])
+def test_e8_quantize_on_the_shell_table_equals_the_table_walk(N, scale):
+    """The search by the table's symmetry against the kernel that walks all rows (pinned on the oracle above through
+    tables it does not recognise), at sizes around a workgroup's and past the switch to 512 vectors per workgroup:
+    random vectors, exact ties (zeros, equal and opposite entries, midpoints of rows), vectors far outside the table,
+    and some that are not finite."""
+    from glq_amd import _lib, ext
+    say("e8 shell search", N, scale)
+    g = torch.Generator().manual_seed(N)
+    cb = torch.from_numpy(O.e8_table())
+    X = torch.randn(N, 8, generator=g) * scale
+    pick = torch.randint(0, N, (8, max(1, N // 50)), generator=g)
+    X[pick[0]] = (X[pick[0]] * 2).round() / 2                    # on or near the half-integer grid
+    X[pick[1]] = 0.5 * (cb[torch.randint(0, 65536, pick[1].shape, generator=g)] + cb[torch.randint(0, 65536, pick[1].shape, generator=g)])
+    X[pick[2], 1] = -X[pick[2], 0]
+    X[pick[3]] *= 5.0
+    X[pick[4]] = cb[torch.randint(56881, 65536, pick[4].shape, generator=g)] * 1.05
+    for j, bad in enumerate((float("nan"), float("inf"), 3e38, 1e-42)):
+        X[pick[5, j % pick.shape[1]], j % 8] = bad
+    X, cb = X.to(DEV), cb.to(DEV)
+    dec, idx = ext.e8_quantize(X, cb)
+    norms = (cb * cb).sum(-1)
+    walk, wdec = torch.empty_like(idx), torch.empty_like(dec)
+    _lib.check(_lib.load().glqh_e8_quantize(X.data_ptr(), cb.data_ptr(), norms.data_ptr(), N, 65536, walk.data_ptr(),
+                                            wdec.data_ptr(), torch.cuda.current_stream().cuda_stream))
+    assert torch.equal(idx, walk), int((idx != walk).sum())
+    assert torch.equal(dec, wdec)
+    assert torch.equal(ext.e8_quantize(X, cb, norms)[1], walk)   # the caller's norms
+    norms[5] += 0.5                                              # a table that no longer qualifies, same memory
+    assert ext._shell_plan(cb, norms) is None
 
 
 @pytest.mark.parametrize("K", [1, 2, 3, 4])
