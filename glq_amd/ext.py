@@ -66,6 +66,24 @@ def _e8_dense_route(B, n_pad, folded=False):
     return B > limit or (B > 16 and int(n_pad) % (32 if folded else 256) != 0)
 
 
+_host = None
+
+
+def host():
+    """The native host path (csrc/host.cpp), bound to the loaded library on first use."""
+    global _host
+    if _host is None:
+        lib = _lib.load()
+        try:
+            from . import _glq_host
+        except ImportError as e:
+            raise RuntimeError(f"glq_amd/_glq_host.so cannot be imported ({e}): build it with "
+                               "glq_amd/csrc/build.sh") from e
+        _glq_host.bind(lib._handle, globals())
+        _host = _glq_host
+    return _host
+
+
 def _p(t):
     return C.c_void_p(t.data_ptr()) if t is not None else C.c_void_p(0)
 
@@ -364,6 +382,10 @@ def _trellis_dense(x, sv, su, packed, packed2, blocks_n, blocks_m, bn_meta, bm_m
 def glq_fused_linear_trellis_3inst_cuda(x, sv, su, trellis_packed, blocks_n, blocks_m,
                                         blocks_n_meta, blocks_m_meta, wscale, in_features,
                                         out_features, n_pad, m_pad, out_dtype=None):
+    y = (_host or host()).trellis_linear(x, sv, su, trellis_packed, None, blocks_n, blocks_m, blocks_n_meta,
+                                         blocks_m_meta, wscale, 0.0, in_features, out_features, n_pad, m_pad, out_dtype)
+    if y is not None:
+        return y
     return _fused_trellis(x, sv, su, trellis_packed, None, blocks_n, blocks_m, blocks_n_meta,
                           blocks_m_meta, wscale, 0.0, in_features, out_features, n_pad, m_pad,
                           None, None, out_dtype)
@@ -376,6 +398,11 @@ def glq_fused_linear_trellis_3inst_rvq2_cuda(x, sv, su, trellis_packed, trellis_
     if trellis_packed2 is None or trellis_packed2.numel() == 0:
         raise RuntimeError("trellis RVQ stage 2 is half-configured: trellis_packed2 is absent "
                            f"but inv_resid_scale2 = {inv_resid_scale2}")
+    y = (_host or host()).trellis_linear(x, sv, su, trellis_packed, trellis_packed2, blocks_n, blocks_m, blocks_n_meta,
+                                         blocks_m_meta, wscale, inv_resid_scale2, in_features, out_features, n_pad, m_pad,
+                                         out_dtype)
+    if y is not None:
+        return y
     return _fused_trellis(x, sv, su, trellis_packed, trellis_packed2, blocks_n, blocks_m,
                           blocks_n_meta, blocks_m_meta, wscale, inv_resid_scale2, in_features,
                           out_features, n_pad, m_pad, None, None, out_dtype)
@@ -551,6 +578,14 @@ def glq_fused_moe_trellis_3inst_cuda(x, topk_ids, topk_weights,
     host call with the routing read on the device (argument order of the reference's binding,
     glq/csrc/glq_bindings.cpp:509-525; glq/csrc/glq_cuda.cu:5030-5250).  Returns (num_tokens,
     hidden) in the input's 16-bit dtype (the reference returns fp16)."""
+    y = (_host or host()).moe(
+        x, topk_ids, topk_weights, w13_trellis_packed, w13_trellis_packed2, w13_SU, w13_SV, w13_Wscale,
+        w13_inv_resid_scale2, w2_trellis_packed, w2_trellis_packed2, w2_SU, w2_SV, w2_Wscale, w2_inv_resid_scale2,
+        hidden_size, intermediate_size, w13_out_features, n_pad_w13, m_pad_w13, n_pad_w2, m_pad_w2, blocks_n_w13,
+        blocks_m_w13, blocks_n_w13_meta, blocks_m_w13_meta, blocks_n_w2, blocks_m_w2, blocks_n_w2_meta, blocks_m_w2_meta,
+        activation_type, out_dtype)
+    if y is not None:
+        return y
     lib = _lib.load()
     _chk(x, "x", (torch.float16, torch.bfloat16))
     if x.dim() != 2 or x.shape[1] != int(hidden_size):
@@ -898,6 +933,24 @@ def _e8_folded(B, qidxs, t1, q2, t2, q3, q4):
     if len(tables) == 2:
         f.halves2, f.n_halves2 = halves[1][0].data_ptr(), halves[1][0].shape[0]
     return f, keep
+
+
+def e8_plan_parts(stages, cb, cb2):
+    """What the native forward of a prepared layer keeps: packed tables, folded streams of the index tensors `stages`
+    (None: not all of them exist) and the tables of half codewords."""
+    t1 = _primary_table(cb)
+    t2 = _packed_table(cb2) if len(stages) > 1 else None
+    streams = []
+    for s, q in enumerate(stages):
+        t = t2 if s == 1 else t1
+        hit = _FOLD_STREAMS.get(q, (t.data_ptr(),))
+        if hit is None or hit[0]() is not t:
+            return t1, t2, None, None, None
+        streams.append((hit[1], hit[2]))
+    halves = [_FOLD_TABLES.get(t) for t in ([t1] + ([t2] if t2 is not None and t2 is not t1 else []))]
+    if any(h is None or h[0] is None for h in halves):
+        return t1, t2, None, None, None
+    return t1, t2, streams, halves[0][0], halves[1][0] if len(halves) == 2 else None
 
 
 def _primary_table(codebook):

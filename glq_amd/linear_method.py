@@ -89,6 +89,7 @@ class MergedTrellisLinear:
     KV-shared layers do."""
 
     glq_is_trellis = True
+    _fast = None        # native form of the grouped calls (csrc/host.cpp), made by the first of them
 
     def __init__(self, in_features, shard_sizes, bpw=4):
         self.glq_in_features = int(in_features)
@@ -137,6 +138,7 @@ class MergedTrellisLinear:
             device = next(t.device for t in self.trellis_packed._shard_data + self.SV._shard_data
                           if t.device.type == "cuda")
         device = torch.device(device)
+        self._fast = None
         for name in ("trellis_packed", "trellis_packed2", "inv_resid_scale2", "tlut", "SU", "SV", "Wscale"):
             sh = getattr(self, name)
             for i, t in enumerate(sh._shard_data):
@@ -199,6 +201,11 @@ class MergedTrellisLinear:
     def apply(self, x, bias=None):
         """(.., in_features) -> (.., sum(shard_sizes)) in x's dtype: the call sequence of
         `_glq_apply_trellis` plus the bias add of `GLQLinearMethod.apply`."""
+        fast = self._fast
+        if fast is not None and bias is None and _GLQ_MERGED_GROUPED and not torch.compiler.is_compiling():
+            y = fast(self.__dict__, x)
+            if y is not None:
+                return y
         if self._glq_trellis_meta is None:
             raise RuntimeError("process_weights_after_loading() must run before apply()")
         shape = x.shape
@@ -232,12 +239,20 @@ class MergedTrellisLinear:
         return ({self.trellis_packed.get_shard(i).shape[1] for i in n} == {64} and
                 len({self.trellis_packed2.get_shard(i).shape[1] for i in n}) == 1)
 
+    def _make_native(self, ext, two_stage):
+        if self._fast is None:
+            m0 = self._glq_trellis_meta[0]
+            self._fast = ext.host().group_plan(m0["in"], m0["n_pad"], m0["_bn"], m0["_bnm"],
+                                               [(m["wscale"], m["inv_rs2"], m["out"], m["m_pad"])
+                                                for m in self._glq_trellis_meta], two_stage)
+
     def _apply_2d(self, x):
         _apply = E8RHTLinear._trellis_linear_apply
         metas = self._glq_trellis_meta
         if _GLQ_MERGED_GROUPED and x.dtype in (torch.float16, torch.bfloat16) and self._grouped_rvq2_ok(x.shape[0]):
             from . import ext
             m0 = metas[0]
+            self._make_native(ext, True)
             return ext.glq_fused_linear_trellis_3inst_group_rvq2(
                 x.contiguous(), [(self.SV.get_shard(i), self.SU.get_shard(i), self.trellis_packed.get_shard(i),
                                   self.trellis_packed2.get_shard(i), m["wscale"], m["inv_rs2"], m["out"], m["m_pad"])
@@ -246,6 +261,7 @@ class MergedTrellisLinear:
         if _GLQ_MERGED_GROUPED and x.dtype in (torch.float16, torch.bfloat16) and self._grouped_ok(x.shape[0]):
             from . import ext
             m0 = metas[0]
+            self._make_native(ext, False)
             return ext.glq_fused_linear_trellis_3inst_group(
                 x.contiguous(), [(self.SV.get_shard(i), self.SU.get_shard(i), self.trellis_packed.get_shard(i),
                                   m["wscale"], m["out"], m["m_pad"]) for i, m in enumerate(metas)],

@@ -46,6 +46,8 @@ _MAX_TOKENS_PER_CALL = 32768
 _GLQ_FUSED_TRELLIS_ENABLED = os.environ.get("GLQ_FUSED_TRELLIS", "1") != "0"
 
 class E8RHTLinear(nn.Module):
+    _fast = None        # native form of forward (csrc/host.cpp), made by the first forward, dropped with _scalars
+
     def __init__(self, in_features: int, out_features: int, bias: bool = False,
                  block_diagonal: bool = False, codebook_type: str = "e8_shell"):
         super().__init__()
@@ -88,7 +90,7 @@ class E8RHTLinear(nn.Module):
 
         self.codebook = None
         self.codebook2 = None
-        self._scalars = None                 # host copies of Wscale / residual scales
+        self._scalars = self._fast = None    # host copies of Wscale / residual scales
         self._prepared_for = None            # identity of the buffers the load-time step last saw
         self._trellis_has_kernel = True
         self._rebuild_meta()
@@ -113,7 +115,7 @@ class E8RHTLinear(nn.Module):
         self.codebook, self.codebook2 = codebook, codebook2
         if self._is_trellis:
             self._trellis_has_kernel = getattr(codebook, "has_kernel", True)
-        self._scalars = None
+        self._scalars = self._fast = None
         self._prepared_for = None
 
     def _load_from_state_dict(self, state_dict, prefix, local_metadata, strict, missing_keys,
@@ -157,7 +159,7 @@ class E8RHTLinear(nn.Module):
                 for suffix in ("inv_resid_scale", "inv_resid_scale2", "inv_resid_scale3"):
                     if prefix + suffix not in state_dict:
                         state_dict[prefix + suffix] = torch.zeros((), dtype=torch.float32)
-        self._scalars = None
+        self._scalars = self._fast = None
         super()._load_from_state_dict(state_dict, prefix, local_metadata, strict, missing_keys,
                                       unexpected_keys, error_msgs)
 
@@ -191,7 +193,7 @@ class E8RHTLinear(nn.Module):
         dev = self.SV.device
         if dev.type != "cuda":
             raise RuntimeError("E8RHTLinear.prepare() needs the buffers on the GPU")
-        self._scalars = None
+        self._scalars = self._fast = None
         sc = self._resolve(dev, prepare=False)
         held = 0
         if not self._is_trellis:
@@ -294,6 +296,12 @@ class E8RHTLinear(nn.Module):
         x = x2d if x2d.dtype in (torch.float16, torch.bfloat16) else x2d.half()
         x = x.contiguous()
         has_s2 = trellis_packed2 is not None and trellis_packed2.numel() > 0
+        if _GLQ_FUSED_TRELLIS_ENABLED and bias is None and x.dtype == out_dtype and not torch.compiler.is_compiling():
+            y = ext.host().trellis_linear(x, SV, SU, trellis_packed, trellis_packed2 if has_s2 else None, blocks_n, blocks_m,
+                                          blocks_n_meta, blocks_m_meta, float(wscale), float(inv_resid_scale2) if has_s2 else 0.0,
+                                          in_features, out_features, n_pad, m_pad, out_dtype)
+            if y is not None:
+                return y
         ops = torch.ops.glq if hasattr(torch.ops, "glq") else None
         if not _GLQ_FUSED_TRELLIS_ENABLED:
             x_rht = torch.empty((x.shape[0], n_pad), dtype=torch.float16, device=x.device)
@@ -324,7 +332,28 @@ class E8RHTLinear(nn.Module):
             y = y + bias.unsqueeze(0).to(out_dtype)
         return y
 
+    def _native(self, ext, sc):
+        """The native forward: scalars, block sizes and, for a shell layer, tables and folded streams as they are now.
+        The buffers themselves are read again on every call."""
+        h, bd = ext.host(), self._is_trellis or self.block_diagonal
+        args = (self.in_features, self.out_features, self.n_pad, self.m_pad, list(self.blocks_n), list(self.blocks_m),
+                self._blocks_n_meta_gpu if bd else None, self._blocks_m_meta_gpu if bd else None, sc["wscale"])
+        if self._is_trellis:
+            return h.trellis_plan(*args, sc["inv2"])
+        n = sc["n_stages"]
+        cb, cb2 = self._tables(self.SV.device, n)
+        qs = [self.Qidxs, self.Qidxs2, self.Qidxs3, self.Qidxs4]
+        if any(t.is_inference() for t in qs + [cb] + ([cb2] if cb2 is not None else [])):
+            return None                                # tensors that do not count their changes
+        t1, t2, streams, h1, h2 = ext.e8_plan_parts(qs[:n], cb, cb2)
+        return h.shell_plan(*args, *sc["inv"], n, self.codebook, self.codebook2, cb, cb2, t1, t2, qs, streams, h1, h2)
+
     def forward(self, x: torch.Tensor) -> torch.Tensor:
+        fast = self._fast
+        if fast is not None and _GLQ_FUSED_TRELLIS_ENABLED and not torch.compiler.is_compiling():
+            y = fast(self.__dict__, x)
+            if y is not None:
+                return y
         if not x.is_cuda:
             raise RuntimeError("E8RHTLinear (glq_amd) runs on the GPU only: there is no CPU path")
         from . import ext
@@ -351,6 +380,8 @@ class E8RHTLinear(nn.Module):
                 sc["wscale"], self.in_features, self.out_features, self.n_pad, self.m_pad,
                 bias=self.bias, out_dtype=x.dtype, trellis_packed2=self.trellis_packed2,
                 inv_resid_scale2=sc["inv2"])
+            if fast is None:
+                self._fast = self._native(ext, sc)
             return y.reshape(*shape[:-1], self.out_features)
 
         n = sc["n_stages"]
@@ -372,6 +403,8 @@ class E8RHTLinear(nn.Module):
         else:
             y = ext.glq_fused_linear_cuda(*common, int(math.log2(self.n_pad)),
                                           int(math.log2(self.m_pad)), *tail, out_dtype=xin.dtype)
+        if fast is None:
+            self._fast = self._native(ext, sc)
         if y.dtype != x.dtype:
             y = y.to(x.dtype)
         if self.bias is not None:

@@ -1,0 +1,119 @@
+"""The native host path (csrc/host.cpp) against the Python route of the same calls: equal bit for bit where it
+serves a call, None -- and the Python route -- where something is not what it recognises (needs an MI355X)."""
+import copy
+
+import pytest
+import torch
+
+from tests.gpu_util import DEV, e8_table_f16, say
+
+pytestmark = pytest.mark.gpu
+
+
+def _bits(g, *shape):
+    return torch.randint(-32768, 32768, shape, generator=g, device=DEV, dtype=torch.int16)
+
+
+def _signs(g, n):
+    return (torch.randint(0, 2, (n,), generator=g, device=DEV) * 2 - 1).half()
+
+
+def _layer(kind, out_f, in_f, bias):
+    from glq_amd.quantized_linear import E8RHTLinear
+    g = torch.Generator(device=DEV).manual_seed(out_f + in_f)
+    if kind.startswith("trellis"):
+        lin = E8RHTLinear(in_f, out_f, bias=bias, codebook_type="trellis").to(DEV)
+        tiles = (out_f // 16) * (in_f // 16)
+        lin.trellis_packed = _bits(g, tiles, 64)
+        if kind == "trellis2":
+            lin.trellis_packed2, lin.inv_resid_scale2 = _bits(g, tiles, 32), torch.tensor(0.3, device=DEV)
+    else:
+        lin = E8RHTLinear(in_f, out_f, bias=bias, block_diagonal=kind != "shell_pow2").to(DEV)
+        for s in range(int(kind == "shell2") + 1):
+            setattr(lin, ("Qidxs", "Qidxs2")[s], _bits(g, lin.m_pad, lin.n_pad // 8))
+        if kind == "shell2":
+            lin.inv_resid_scale = torch.tensor(1 / 3.0, device=DEV)
+        lin.set_codebook(e8_table_f16(), e8_table_f16())
+    lin.SU, lin.SV, lin.Wscale = _signs(g, lin.m_pad), _signs(g, lin.n_pad), torch.tensor(0.02, device=DEV)
+    if bias:
+        lin.bias = torch.randn(out_f, generator=g, device=DEV).half()
+    return lin
+
+
+@pytest.mark.parametrize("kind,out_f,in_f,bias,dtype,shape", [
+    ("trellis", 512, 2048, False, torch.bfloat16, (1,)), ("trellis", 96, 192, True, torch.float16, (2, 3)),
+    ("trellis2", 160, 128, True, torch.bfloat16, (37,)), ("shell", 960, 960, True, torch.float16, (5,)),
+    ("shell2", 2048, 2304, False, torch.bfloat16, (1, 4)), ("shell2", 2048, 2304, False, torch.bfloat16, (65,)),
+    ("shell_pow2", 100, 200, True, torch.float16, (3,))])
+def test_native_forward_equals_the_python_route(kind, out_f, in_f, bias, dtype, shape):
+    say("native forward", kind, out_f, in_f, bias, dtype, shape)
+    lin = _layer(kind, out_f, in_f, bias)
+    lin.prepare()
+    x = torch.randn(*shape, in_f, generator=torch.Generator().manual_seed(3)).to(DEV, dtype)
+    assert lin._fast is None
+    ref = lin(x)                                                 # the Python route, which makes the native form
+    y = lin._fast(lin.__dict__, x)
+    assert y is not None and y.shape == ref.shape and y.dtype == ref.dtype and torch.equal(y, ref)
+    assert torch.equal(lin(x), ref)
+    # what it leaves to the Python route
+    assert lin._fast(lin.__dict__, x.float()) is None and lin._fast(lin.__dict__, x.cpu()) is None
+    assert lin._fast(lin.__dict__, x[..., :0]) is None and lin._fast(lin.__dict__, x[:0]) is None
+    if x.numel() > in_f:
+        assert lin._fast(lin.__dict__, x.transpose(0, -1)) is None
+    assert lin(x.float()).dtype == torch.float32
+    # buffers are read on every call, copies make their own plan
+    if not bias:
+        su = lin.SU
+        lin.SU = -su
+        assert torch.equal(lin(x), -ref)
+        lin.SU = su
+    twin = copy.deepcopy(lin)
+    assert twin._fast is None and torch.equal(twin(x), ref)
+
+
+def test_native_shell_forward_notices_changed_indices_and_released_streams():
+    from glq_amd import ext
+    say("native shell forward, changed buffers")
+    lin = _layer("shell2", 2048, 2304, False)
+    lin.prepare()
+    x = torch.randn(2, 2304, generator=torch.Generator().manual_seed(1)).to(DEV, torch.bfloat16)
+    lin(x)
+    assert lin._fast(lin.__dict__, x) is not None
+    ext.e8_release(lin.Qidxs, lin.Qidxs2)                        # the plan does not keep the streams alive
+    assert lin._fast(lin.__dict__, x) is None
+    lin.prepare()
+    y = lin(x)
+    lin.Qidxs.add_(1)
+    assert lin._fast(lin.__dict__, x) is None
+    assert not torch.equal(lin(x), y)
+
+
+@pytest.mark.parametrize("bpw,B", [(4, 1), (4, 9), (4, 100), (6, 1), (6, 40)])
+def test_native_merged_forward_equals_the_python_route(bpw, B):
+    from glq_amd import linear_method as LM
+    say("native merged", bpw, B)
+    lins = [_layer("trellis2" if bpw == 6 else "trellis", m, 192, False) for m in (96, 64, 64)]
+    ml = LM.MergedTrellisLinear.from_linears(lins, bpw=bpw).process_weights_after_loading(DEV)
+    x = torch.randn(B, 192, generator=torch.Generator().manual_seed(B)).to(DEV, torch.bfloat16)
+    ref = ml.apply(x)
+    y = ml._fast(ml.__dict__, x)
+    assert y is not None and torch.equal(y, ref)
+    bias = torch.randn(224, generator=torch.Generator().manual_seed(0)).to(DEV)
+    assert torch.equal(ml.apply(x, bias), ref + bias.to(ref.dtype))
+    ml.trellis_packed._shard_data[1] = torch.zeros(0, dtype=torch.int16, device=DEV)    # an unloaded shard
+    assert ml._fast(ml.__dict__, x) is None
+
+
+def test_dispatch_modes_take_the_python_route():
+    from torch.utils._python_dispatch import TorchDispatchMode
+    say("native forward under a dispatch mode")
+
+    class Count(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+    lin = _layer("trellis", 64, 64, False)
+    x = torch.randn(1, 64, generator=torch.Generator().manual_seed(0)).to(DEV, torch.bfloat16)
+    ref = lin(x)
+    with Count():
+        assert lin._fast(lin.__dict__, x) is None
+        assert torch.equal(lin(x), ref)
