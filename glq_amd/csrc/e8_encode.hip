@@ -72,22 +72,21 @@ e8_quantize_kernel(const float *__restrict__ x, const float *__restrict__ table,
 // Which row the table walk above would return depends on fp32 rounding only where two distances are
 // closer than what rounding can move them; `es_margin` bounds that: 128 roundings of
 // 12 + 2 sqrt(12) |x|, where the walk's own sums take 9, the ones here 12 and the place bits in y 16,
-// all twice for a difference.  Vectors inside it (a few in 10^4 of N(0, 1)), and any that are not
-// finite or large, take the table walk, spread over the whole chip (e8_slow_kernel): same indices always.
+// all twice for a difference.  A vector with a second point inside the margin, or with a point of
+// norm 12 that may be nearer (a fifth of N(0, 1)), has all of them listed: orbit by orbit, every
+// point follows from a nearer one by a simple reflection, so the points within reach form a tree
+// that a workgroup walks in its LDS, 2.5 of them on average.  Those that the table holds are compared
+// by the walk's own arithmetic, lowest row on ties: the walk's answer, always.  Vectors that are not
+// finite, or have too many points in reach for the list, take the walk itself (e8_walk_kernel).
 //
-// The part of shell 12 that the table holds has no symmetry: vectors for which some point of the
-// full shell would be nearer (a quarter of N(0, 1)) meet its rows on the matrix cores, f16 codewords against x as
-// two f16 parts (22 bits), and the winning 32 rows are then compared exactly.
-//
-// 524288 vectors of N(0, 1): 12.06 ms (walk) -> 0.098 ms (70 us, of which the rows of norm 12 are most,
-// + 28 us for the walk of the 200 left over); 960 vectors: 12.7 ms -> 21 us, latency.
-typedef f16 f16x8v __attribute__((ext_vector_type(8)));
-typedef float f32x16v __attribute__((ext_vector_type(16)));
-
+// 524288 vectors of N(0, 1): 12.06 ms (walk) -> 98 us (points of norm 12 on the matrix cores, all 8655 rows for
+// every vector they may win) -> 34 us (points in reach only; 38 MB in and out, 8 us); 960 vectors 12.7 ms ->
+// 14 us, latency.
 constexpr int ES_THREADS = 256;
 constexpr int ES_SLOTS = 1 << 17;                              // hash slots for at most 65536 keys
 constexpr uint32_t ES_EMPTY = 0xFFFFFFFFu;
-constexpr int ES_CHUNK = 128;                                  // vectors of one pass over shell 12
+constexpr int ES_CHUNK = 128;                                  // vectors whose points are listed together,
+constexpr int ES_LIST = 3072;                                  // and the points: 2.5 each at unit scale, up to 106 far out
 constexpr int ES_SPLIT = 128;                                  // parts of the table in the exact walk
 
 __device__ __forceinline__ uint32_t es_hash(uint32_t code) { return (code * 2654435761u) >> 15; }
@@ -100,10 +99,10 @@ es_clear_kernel(uint32_t *__restrict__ keys, int *__restrict__ counts) {
 }
 
 // counts[s]: distinct rows of norm 2s (s = 0..6) that are E8 points with that norm in `norms`;
-// rows of norm 12 also go to rem_rows.  counts[7]: everything else.
+// counts[7]: everything else.
 __global__ void __launch_bounds__(256)
 es_index_kernel(const float *__restrict__ table, const float *__restrict__ norms, int n, uint32_t *__restrict__ keys,
-                int *__restrict__ vals, int *__restrict__ counts, int *__restrict__ rem_rows) {
+                int *__restrict__ vals, int *__restrict__ counts) {
     const int r = blockIdx.x * 256 + threadIdx.x;
     if (r >= n) return;
     uint32_t code = 0, odd = 0;
@@ -134,28 +133,8 @@ es_index_kernel(const float *__restrict__ table, const float *__restrict__ norms
 #pragma unroll 1
     for (int q = 0; q < 8; ++q) {
         const unsigned long long who = __ballot(s == q);
-        if (s != q) continue;
-        const int first = __builtin_ctzll(who), lane = threadIdx.x & 63;
-        int at = 0;
-        if (lane == first) at = atomicAdd(counts + q, __builtin_popcountll(who));
-        at = __builtin_amdgcn_readlane(at, first) + __builtin_popcountll(who & ((1ull << lane) - 1));
-        if (q == 6) rem_rows[at] = r;
+        if (s == q && (int)(threadIdx.x & 63) == __builtin_ctzll(who)) atomicAdd(counts + q, __builtin_popcountll(who));
     }
-}
-
-// MFMA operands of the rows of shell 12, 32 to a tile: lanes 0..31 hold a row's eight values, lanes
-// 32..63 the same times 2^-11, for the low parts of x.  Rows past n_rem are zeros (index -1).
-__global__ void __launch_bounds__(256)
-es_operands_kernel(const float *__restrict__ table, int *__restrict__ rem_rows, int n_rem, int n_tiles, f16 *__restrict__ ops) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= n_tiles * 64) return;
-    const int at = (i >> 6) * 32 + (i & 31);
-    const float scale = (i & 32) ? 1.0f / 2048.0f : 1.0f;
-    f16x8v v;
-#pragma unroll
-    for (int d = 0; d < 8; ++d) v[d] = at < n_rem ? (f16)(table[(int64_t)rem_rows[at] * 8 + d] * scale) : (f16)0.0f;
-    *(f16x8v *)(ops + (int64_t)i * 8) = v;
-    if (at >= n_rem && !(i & 32)) rem_rows[at] = -1;
 }
 
 // the walk's distance of one row
@@ -166,17 +145,17 @@ __device__ __forceinline__ float es_dist(const float x[8], const float *__restri
     return __builtin_fmaf(-2.0f, dot, norm) + 0.0f;            // + 0: one zero
 }
 
+// (distance, row) in the walk's order
+__device__ __forceinline__ unsigned long long es_key(float dist, int row) {
+    uint32_t b = __builtin_bit_cast(uint32_t, dist);
+    b = (b >> 31) ? ~b : b | 0x80000000u;                      // ordered like the floats
+    return (unsigned long long)b << 32 | (uint32_t)row;
+}
+
 __device__ __forceinline__ void es_load(const float *__restrict__ x, int64_t v, float xv[8]) {
     const f32x4v a = *(const f32x4v *)(x + v * 8), b = *(const f32x4v *)(x + v * 8 + 4);
     xv[0] = a.x; xv[1] = a.y; xv[2] = a.z; xv[3] = a.w;
     xv[4] = b.x; xv[5] = b.y; xv[6] = b.z; xv[7] = b.w;
-}
-
-__device__ __forceinline__ float es_margin(const float xv[8]) {
-    float q = 0.0f;
-#pragma unroll
-    for (int d = 0; d < 8; ++d) q += xv[d] * xv[d];
-    return (12.0f + 6.93f * __builtin_sqrtf(q)) * 0x1p-17f;
 }
 
 struct es_args {
@@ -184,15 +163,25 @@ struct es_args {
     int64_t N;
     const uint32_t *keys;
     const int *vals;
-    const f16 *ops;
-    const int *rem_rows;
-    int n_groups, n_entries;                                   // groups: pairs of 32-row tiles
+    int n_entries;
     int64_t *idx_out;
     float *dec_out;                                            // may be null
-    int *slow_count;                                           // per workgroup of the first kernel
-    int *slow_list, *slow_arrive;                              // N each
-    unsigned long long *slow_key;                              // N
+    int *walk_count;                                           // per workgroup of the first kernel
+    int *walk_list, *walk_arrive;                              // N each
+    unsigned long long *walk_key;                              // N
 };
+
+// row of a codeword (2 c + 6 in a nibble per coordinate), -1 if the table does not hold it
+__device__ __forceinline__ int es_row(const es_args &a, uint32_t code) {
+    uint32_t h = es_hash(code), k = a.keys[h];
+    int row = a.vals[h];                                       // asked for together; unset where the key is empty
+    for (int probe = 0; k != code && k != ES_EMPTY && probe < ES_SLOTS; ++probe) {
+        h = (h + 1) & (ES_SLOTS - 1);
+        k = a.keys[h];
+        row = a.vals[h];
+    }
+    return k == code ? row : -1;
+}
 
 __device__ __forceinline__ void es_store(const es_args &a, int64_t v, int row) {
     a.idx_out[v] = row;
@@ -204,119 +193,172 @@ __device__ __forceinline__ void es_store(const es_args &a, int64_t v, int row) {
     }
 }
 
-// p of an orbit: 2 p_r + 1 in nibble r - 1
+// x in its dominant chamber: k_r = |x| and, in the low three bits, its place (2^-20 of the value at most),
+// descending; signs of x by place; the last of the order carries the product of the signs
+struct es_vec {
+    uint32_t k[8], signs;
+    bool flip;
+    float y[8], margin;
+};
+
+// false: not finite, or large enough for a sum to leave fp32
+__device__ __forceinline__ bool es_sort(const float xv[8], es_vec &s) {
+    float total = 0.0f, q = 0.0f;
+    s.signs = 0;
+#pragma unroll
+    for (int d = 0; d < 8; ++d) {
+        const uint32_t b = __builtin_bit_cast(uint32_t, xv[d]);
+        s.signs |= (b >> 31) << d;
+        s.k[d] = (b & 0x7ffffff8u) | (uint32_t)d;
+        total += __builtin_fabsf(xv[d]);
+        q += xv[d] * xv[d];
+    }
+    s.margin = (12.0f + 6.93f * __builtin_sqrtf(q)) * 0x1p-17f;
+#define ES_X(i, j) { const uint32_t hi = s.k[i] > s.k[j] ? s.k[i] : s.k[j], lo = s.k[i] > s.k[j] ? s.k[j] : s.k[i]; s.k[i] = hi; s.k[j] = lo; }
+    ES_X(0, 1) ES_X(2, 3) ES_X(4, 5) ES_X(6, 7)
+    ES_X(0, 2) ES_X(1, 3) ES_X(4, 6) ES_X(5, 7)
+    ES_X(1, 2) ES_X(5, 6) ES_X(0, 4) ES_X(3, 7)
+    ES_X(1, 5) ES_X(2, 6)
+    ES_X(1, 4) ES_X(3, 6)
+    ES_X(2, 4) ES_X(3, 5)
+    ES_X(3, 4)
+#undef ES_X
+#pragma unroll
+    for (int d = 0; d < 8; ++d) s.y[d] = __builtin_bit_cast(float, s.k[d] & ~7u);
+    s.flip = __builtin_popcount(s.signs) & 1;
+    if (s.flip) s.y[7] = -s.y[7];
+    return total < 1e15f;
+}
+
+// a point in that order: 2 c_r + 6 in nibble r
 constexpr uint32_t es_p(int a, int b, int c, int d, int e, int f, int g, int h) {
-    return (uint32_t)(a + 1) | (uint32_t)(b + 1) << 4 | (uint32_t)(c + 1) << 8 | (uint32_t)(d + 1) << 12 |
-           (uint32_t)(e + 1) << 16 | (uint32_t)(f + 1) << 20 | (uint32_t)(g + 1) << 24 | (uint32_t)(h + 1) << 28;
+    return (uint32_t)(a + 6) | (uint32_t)(b + 6) << 4 | (uint32_t)(c + 6) << 8 | (uint32_t)(d + 6) << 12 |
+           (uint32_t)(e + 6) << 16 | (uint32_t)(f + 6) << 20 | (uint32_t)(g + 6) << 24 | (uint32_t)(h + 6) << 28;
+}
+
+__device__ __forceinline__ int es_q(uint32_t p, int r) { return (int)((p >> (4 * r)) & 15u) - 6; }
+
+// the codeword in x's own order
+__device__ __forceinline__ uint32_t es_code(uint32_t p, const uint32_t k[8], uint32_t signs, bool flip) {
+    uint32_t code = 0;
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+        const uint32_t i = k[r] & 7u;
+        bool neg = (signs >> i) & 1u;
+        if (r == 7) neg = neg != flip;
+        const int q = es_q(p, r);
+        code |= (uint32_t)(6 + (neg ? -q : q)) << (4 * i);
+    }
+    return code;
+}
+
+// f(distance - |x|^2 of the orbit's nearest point, that point) for the orbits of the full shells ...
+template <typename F>
+__device__ __forceinline__ void es_orbits(const float y[8], F f) {
+    const float s2 = y[0] + y[1], s3 = s2 + y[2], s4 = s3 + y[3], s5 = s4 + y[4], s6 = s5 + y[5], s7 = s6 + y[6];
+    const float s8 = s7 + y[7], t8 = s7 - y[7];
+    f(0.0f, es_p(0, 0, 0, 0, 0, 0, 0, 0));
+    f(2.0f - 2.0f * s2, es_p(2, 2, 0, 0, 0, 0, 0, 0));
+    f(2.0f - s8, es_p(1, 1, 1, 1, 1, 1, 1, 1));
+    f(4.0f - 4.0f * y[0], es_p(4, 0, 0, 0, 0, 0, 0, 0));
+    f(4.0f - 2.0f * s4, es_p(2, 2, 2, 2, 0, 0, 0, 0));
+    f(4.0f - t8 - 2.0f * y[0], es_p(3, 1, 1, 1, 1, 1, 1, -1));
+    f(6.0f - 2.0f * (s3 + y[0]), es_p(4, 2, 2, 0, 0, 0, 0, 0));
+    f(6.0f - 2.0f * s6, es_p(2, 2, 2, 2, 2, 2, 0, 0));
+    f(6.0f - s8 - 2.0f * s2, es_p(3, 3, 1, 1, 1, 1, 1, 1));
+    f(8.0f - 4.0f * s2, es_p(4, 4, 0, 0, 0, 0, 0, 0));
+    f(8.0f - 2.0f * (s5 + y[0]), es_p(4, 2, 2, 2, 2, 0, 0, 0));
+    f(8.0f - 2.0f * s8, es_p(2, 2, 2, 2, 2, 2, 2, 2));
+    f(8.0f - 2.0f * t8, es_p(2, 2, 2, 2, 2, 2, 2, -2));
+    f(8.0f - t8 - 2.0f * s3, es_p(3, 3, 3, 1, 1, 1, 1, -1));
+    f(8.0f - s8 - 4.0f * y[0], es_p(5, 1, 1, 1, 1, 1, 1, 1));
+    f(10.0f - 2.0f * (s2 + 2.0f * y[0]), es_p(6, 2, 0, 0, 0, 0, 0, 0));
+    f(10.0f - 2.0f * (s4 + s2), es_p(4, 4, 2, 2, 0, 0, 0, 0));
+    f(10.0f - 2.0f * (s7 + y[0]), es_p(4, 2, 2, 2, 2, 2, 2, 0));
+    f(10.0f - s8 - 2.0f * s4, es_p(3, 3, 3, 3, 1, 1, 1, 1));
+    f(10.0f - t8 - 2.0f * (s2 + y[0]), es_p(5, 3, 1, 1, 1, 1, 1, -1));
+}
+
+// ... and of the shell of norm 12, of which the table holds a part
+template <typename F>
+__device__ __forceinline__ void es_orbits_12(const float y[8], F f) {
+    const float s2 = y[0] + y[1], s3 = s2 + y[2], s4 = s3 + y[3], s5 = s4 + y[4], s6 = s5 + y[5], s7 = s6 + y[6];
+    const float s8 = s7 + y[7], t8 = s7 - y[7];
+    f(12.0f - 4.0f * s3, es_p(4, 4, 4, 0, 0, 0, 0, 0));
+    f(12.0f - 2.0f * (s6 + s2), es_p(4, 4, 2, 2, 2, 2, 0, 0));
+    f(12.0f - 2.0f * (s4 + 2.0f * y[0]), es_p(6, 2, 2, 2, 0, 0, 0, 0));
+    f(12.0f - t8 - 2.0f * s5, es_p(3, 3, 3, 3, 3, 1, 1, -1));
+    f(12.0f - s8 - 2.0f * (s3 + y[0]), es_p(5, 3, 3, 1, 1, 1, 1, 1));
+}
+
+// f(gap, child) for the children of point p in its orbit's tree whose distance is at most `room` more than p's: a
+// simple reflection that takes p further away, and is the first to bring the child back.
+template <typename F>
+__device__ __forceinline__ void es_children(uint32_t p, const float y[8], float room, F f) {
+    int q[8];
+#pragma unroll
+    for (int r = 0; r < 8; ++r) q[r] = es_q(p, r);
+    bool before = true;                                        // the pairs ahead of (i - 1, i) descend
+#pragma unroll
+    for (int i = 0; i < 7; ++i) {
+        if (i >= 2) before = before && q[i - 2] >= q[i - 1];
+        const float gap = (float)(q[i] - q[i + 1]) * (y[i] - y[i + 1]);
+        if (before && q[i] > q[i + 1] && (i == 0 || q[i - 1] >= q[i + 1]) && gap <= room) {
+            const uint32_t d = ((p >> (4 * i)) ^ (p >> (4 * i + 4))) & 15u;
+            f(gap, p ^ (d << (4 * i)) ^ (d << (4 * i + 4)));
+        }
+    }
+    const float gap = (float)(q[6] + q[7]) * (y[6] + y[7]);
+    if (before && q[4] >= q[5] && q[5] >= -q[7] && q[6] >= q[7] && q[6] + q[7] > 0 && gap <= room)
+        f(gap, (p & 0x00FFFFFFu) | (uint32_t)(6 - q[7]) << 24 | (uint32_t)(6 - q[6]) << 28);
 }
 
 template <int V>                                               // vectors of a workgroup
-__global__ void __launch_bounds__(ES_THREADS, 3)
+__global__ void __launch_bounds__(ES_THREADS, 4)
 e8_shell_kernel(const es_args a) {
-    __shared__ int n_flag, n_slow, n_exact;
-    __shared__ unsigned short flag_v[V], exact_j[ES_CHUNK];
-    __shared__ float flag_a[V], flag_m[V];                     // distance and margin
-    __shared__ int flag_row[V], exact_group[ES_CHUNK];
-    __shared__ float m1s[8][ES_CHUNK], m2s[8][ES_CHUNK];
-    __shared__ int ids[8][ES_CHUNK];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    __shared__ int n_flag, n_walk, n_list;
+    __shared__ unsigned short flags[V];
+    __shared__ uint32_t list_p[ES_LIST], sk[ES_CHUNK][8];
+    __shared__ unsigned char list_j[ES_LIST];
+    __shared__ float list_room[ES_LIST];
+    __shared__ uint32_t s_signs[ES_CHUNK];                     // bit 8: flip, bit 9: left to the walk
+    __shared__ unsigned long long best[ES_CHUNK];
+    const int tid = threadIdx.x;
     const int64_t v0 = (int64_t)blockIdx.x * V;
-    if (tid == 0) n_flag = n_slow = 0;
+    if (tid == 0) n_flag = n_walk = 0;
     __syncthreads();
-    auto slow = [&](int local) {
-        const int64_t at = v0 + atomicAdd(&n_slow, 1);
-        a.slow_list[at] = local;
-        a.slow_arrive[at] = 0;
-        a.slow_key[at] = 0xFF800000ull << 32;                  // +inf, row 0: the walk's start
+    auto walk = [&](int local) {
+        const int64_t at = v0 + atomicAdd(&n_walk, 1);
+        a.walk_list[at] = local;
+        a.walk_arrive[at] = 0;
+        a.walk_key[at] = es_key(__builtin_inff(), 0);          // the walk's start
     };
 #pragma unroll 1
     for (int local = tid; local < V && v0 + local < a.N; local += ES_THREADS) {
         const int64_t v = v0 + local;
         float xv[8];
         es_load(a.x, v, xv);
-        uint32_t k[8], signs = 0;
-        float total = 0.0f;
-#pragma unroll
-        for (int d = 0; d < 8; ++d) {
-            const uint32_t b = __builtin_bit_cast(uint32_t, xv[d]);
-            signs |= (b >> 31) << d;
-            k[d] = (b & 0x7ffffff8u) | (uint32_t)d;            // |x| and its place: 2^-20 of the value at most
-            total += __builtin_fabsf(xv[d]);
-        }
-        if (!(total < 4096.0f)) { slow(local); continue; }     // f16 parts below; infinities and NaN
-        const float margin = es_margin(xv);
-        // descending, 19 exchanges
-#define ES_X(i, j) { const uint32_t hi = k[i] > k[j] ? k[i] : k[j], lo = k[i] > k[j] ? k[j] : k[i]; k[i] = hi; k[j] = lo; }
-        ES_X(0, 1) ES_X(2, 3) ES_X(4, 5) ES_X(6, 7)
-        ES_X(0, 2) ES_X(1, 3) ES_X(4, 6) ES_X(5, 7)
-        ES_X(1, 2) ES_X(5, 6) ES_X(0, 4) ES_X(3, 7)
-        ES_X(1, 5) ES_X(2, 6)
-        ES_X(1, 4) ES_X(3, 6)
-        ES_X(2, 4) ES_X(3, 5)
-        ES_X(3, 4)
-#undef ES_X
-        float y[8];
-#pragma unroll
-        for (int d = 0; d < 8; ++d) y[d] = __builtin_bit_cast(float, k[d] & ~7u);
-        const bool flip = __builtin_popcount(signs) & 1;
-        if (flip) y[7] = -y[7];
-        const float s2 = y[0] + y[1], s3 = s2 + y[2], s4 = s3 + y[3], s5 = s4 + y[4], s6 = s5 + y[5], s7 = s6 + y[6];
-        const float s8 = s7 + y[7], t8 = s7 - y[7];
-        float b1 = 0.0f, b2 = __builtin_inff();                // the origin
-        uint32_t p = es_p(0, 0, 0, 0, 0, 0, 0, 0);
-        auto orbit = [&](float score, uint32_t code) {
-            b2 = __builtin_amdgcn_fmed3f(b1, b2, score);
-            if (score < b1) p = code;
-            b1 = __builtin_fminf(b1, score);
-        };
-        orbit(2.0f - 2.0f * s2, es_p(2, 2, 0, 0, 0, 0, 0, 0));
-        orbit(2.0f - s8, es_p(1, 1, 1, 1, 1, 1, 1, 1));
-        orbit(4.0f - 4.0f * y[0], es_p(4, 0, 0, 0, 0, 0, 0, 0));
-        orbit(4.0f - 2.0f * s4, es_p(2, 2, 2, 2, 0, 0, 0, 0));
-        orbit(4.0f - t8 - 2.0f * y[0], es_p(3, 1, 1, 1, 1, 1, 1, -1));
-        orbit(6.0f - 2.0f * (s3 + y[0]), es_p(4, 2, 2, 0, 0, 0, 0, 0));
-        orbit(6.0f - 2.0f * s6, es_p(2, 2, 2, 2, 2, 2, 0, 0));
-        orbit(6.0f - s8 - 2.0f * s2, es_p(3, 3, 1, 1, 1, 1, 1, 1));
-        orbit(8.0f - 4.0f * s2, es_p(4, 4, 0, 0, 0, 0, 0, 0));
-        orbit(8.0f - 2.0f * (s5 + y[0]), es_p(4, 2, 2, 2, 2, 0, 0, 0));
-        orbit(8.0f - 2.0f * s8, es_p(2, 2, 2, 2, 2, 2, 2, 2));
-        orbit(8.0f - 2.0f * t8, es_p(2, 2, 2, 2, 2, 2, 2, -2 + 0));
-        orbit(8.0f - t8 - 2.0f * s3, es_p(3, 3, 3, 1, 1, 1, 1, -1));
-        orbit(8.0f - s8 - 4.0f * y[0], es_p(5, 1, 1, 1, 1, 1, 1, 1));
-        orbit(10.0f - 2.0f * (s2 + 2.0f * y[0]), es_p(6, 2, 0, 0, 0, 0, 0, 0));
-        orbit(10.0f - 2.0f * (s4 + s2), es_p(4, 4, 2, 2, 0, 0, 0, 0));
-        orbit(10.0f - 2.0f * (s7 + y[0]), es_p(4, 2, 2, 2, 2, 2, 2, 0));
-        orbit(10.0f - s8 - 2.0f * s4, es_p(3, 3, 3, 3, 1, 1, 1, 1));
-        orbit(10.0f - t8 - 2.0f * (s2 + y[0]), es_p(5, 3, 1, 1, 1, 1, 1, -1));
-        // the full shell of norm 12, of which the table holds a part
-        float b12 = 12.0f - 4.0f * s3;
-        b12 = __builtin_fminf(b12, 12.0f - 2.0f * (s6 + s2));
-        b12 = __builtin_fminf(b12, 12.0f - 2.0f * (s4 + 2.0f * y[0]));
-        b12 = __builtin_fminf(b12, 12.0f - t8 - 2.0f * s5);
-        b12 = __builtin_fminf(b12, 12.0f - s8 - 2.0f * (s3 + y[0]));
-        // gap to the other rows: other orbits, and the simple reflections of p on its own
-        float gap = b2 - b1;
+        es_vec s;
+        if (!es_sort(xv, s)) { walk(local); continue; }
+        float b1 = __builtin_inff(), b2 = b1, b12 = b1;
+        uint32_t p = 0;
+        es_orbits(s.y, [&](float d, uint32_t code) {
+            b2 = __builtin_amdgcn_fmed3f(b1, b2, d);
+            if (d < b1) p = code;
+            b1 = __builtin_fminf(b1, d);
+        });
+        es_orbits_12(s.y, [&](float d, uint32_t) { b12 = __builtin_fminf(b12, d); });
+        float gap = __builtin_fminf(b2, b12) - b1;             // to other orbits, and to p's own by a reflection
         int q[8];
 #pragma unroll
-        for (int r = 0; r < 8; ++r) q[r] = (int)((p >> (4 * r)) & 15u) - 1;
-        if (q[7] == 14) q[7] = -2;                             // the one entry below -1
+        for (int r = 0; r < 8; ++r) q[r] = es_q(p, r);
 #pragma unroll
         for (int r = 0; r < 7; ++r)
-            if (q[r] != q[r + 1]) gap = __builtin_fminf(gap, (float)(q[r] - q[r + 1]) * (y[r] - y[r + 1]));
-        if (q[6] + q[7] != 0) gap = __builtin_fminf(gap, (float)(q[6] + q[7]) * (y[6] + y[7]));
-        if (!(gap > margin)) { slow(local); continue; }
-        uint32_t code = 0;
-#pragma unroll
-        for (int r = 0; r < 8; ++r) {
-            const uint32_t i = k[r] & 7u;
-            bool neg = (signs >> i) & 1u;
-            if (r == 7) neg = neg != flip;
-            code |= (uint32_t)(6 + (neg ? -q[r] : q[r])) << (4 * i);
-        }
-        uint32_t h = es_hash(code);
-        for (int probe = 0; a.keys[h] != code && probe < ES_SLOTS; ++probe) h = (h + 1) & (ES_SLOTS - 1);
-        const int row = a.vals[h];
-        a.idx_out[v] = row;
+            if (q[r] != q[r + 1]) gap = __builtin_fminf(gap, (float)(q[r] - q[r + 1]) * (s.y[r] - s.y[r + 1]));
+        if (q[6] + q[7] != 0) gap = __builtin_fminf(gap, (float)(q[6] + q[7]) * (s.y[6] + s.y[7]));
+        if (!(gap > s.margin)) { flags[atomicAdd(&n_flag, 1)] = (unsigned short)local; continue; }
+        const uint32_t code = es_code(p, s.k, s.signs, s.flip);
+        a.idx_out[v] = es_row(a, code);
         if (a.dec_out) {
             f32x4v lo, hi;
 #pragma unroll
@@ -327,144 +369,91 @@ e8_shell_kernel(const es_args a) {
             *(f32x4v *)(a.dec_out + v * 8) = lo;
             *(f32x4v *)(a.dec_out + v * 8 + 4) = hi;
         }
-        if (b12 < b1 + 2.0f * margin) {
-            const int j = atomicAdd(&n_flag, 1);
-            flag_v[j] = (unsigned short)local;
-            flag_a[j] = b1;
-            flag_m[j] = 2.0f * margin;
-            flag_row[j] = row;
-        }
     }
     __syncthreads();
     const int nf = n_flag;
-    for (int c0 = 0; c0 < nf; c0 += ES_CHUNK) {
-        if (tid == 0) n_exact = 0;
-        f16x8v bop[4];
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            const int j = c0 + 32 * t + (lane & 31);
+    // 128 vectors at a time, or 32 where many have points in reach: those have many each
+    const int step = nf * 2 < V ? ES_CHUNK : 32;
+    for (int c0 = 0; c0 < nf; c0 += step) {
+        const int nc = nf - c0 < step ? nf - c0 : step;
+        if (tid == 0) n_list = 0;
+        __syncthreads();
+        auto push = [&](uint32_t p, int j, float room) {
+            const int at = atomicAdd(&n_list, 1);
+            if (at < ES_LIST) {
+                list_p[at] = p;
+                list_j[at] = (unsigned char)j;
+                list_room[at] = room;
+            } else atomicOr(&s_signs[j], 512u);
+        };
+        if (tid < nc) {                                        // the nearest points of the orbits in reach
             float xv[8];
-            if (j < nf) es_load(a.x, v0 + flag_v[j], xv);
+            es_load(a.x, v0 + flags[c0 + tid], xv);
+            es_vec s;
+            es_sort(xv, s);
+#pragma unroll
+            for (int r = 0; r < 8; ++r) sk[tid][r] = s.k[r];
+            s_signs[tid] = s.signs | (s.flip ? 256u : 0u);
+            best[tid] = ~0ull;
+            float b1 = __builtin_inff();
+            es_orbits(s.y, [&](float d, uint32_t) { b1 = __builtin_fminf(b1, d); });
+            const float reach = b1 + s.margin;
+            auto seed = [&](float d, uint32_t code) { if (d <= reach) push(code, tid, reach - d); };
+            es_orbits(s.y, seed);
+            es_orbits_12(s.y, seed);
+        }
+        __syncthreads();
+        for (int done = 0, n = n_list < ES_LIST ? n_list : ES_LIST; done < n;) {     // level by level
+            __syncthreads();
+            for (int e = done + tid; e < n; e += ES_THREADS) {
+                const int j = list_j[e];
+                const float room = list_room[e];
+                float y[8];
+#pragma unroll
+                for (int r = 0; r < 8; ++r) y[r] = __builtin_bit_cast(float, sk[j][r] & ~7u);
+                if (s_signs[j] & 256u) y[7] = -y[7];
+                es_children(list_p[e], y, room, [&](float gap, uint32_t child) { push(child, j, room - gap); });
+            }
+            __syncthreads();
+            done = n;
+            n = n_list < ES_LIST ? n_list : ES_LIST;
+        }
+        const int n = n_list < ES_LIST ? n_list : ES_LIST;
+        for (int e = tid; e < n; e += ES_THREADS) {
+            const int j = list_j[e];
+            uint32_t k[8];
+#pragma unroll
+            for (int r = 0; r < 8; ++r) k[r] = sk[j][r];
+            float xv[8], c[8];
+            es_load(a.x, v0 + flags[c0 + j], xv);
+            const uint32_t code = es_code(list_p[e], k, s_signs[j], (s_signs[j] >> 8) & 1u);
+            const int row = es_row(a, code);
+            if (row < 0) continue;
+            int n4 = 0;
 #pragma unroll
             for (int d = 0; d < 8; ++d) {
-                const float f = j < nf ? xv[d] : 0.0f;
-                f16 hi = (f16)f;
-                if (__builtin_fabsf(f) < 0x1p-13f) hi = (f16)0.0f;      // no subnormal operands
-                bop[t][d] = lane < 32 ? hi : (f16)((f - (float)hi) * 2048.0f);
+                const int q = es_q(code, d);
+                c[d] = 0.5f * (float)q;
+                n4 += q * q;
             }
-        }
-        float m1[4], m2[4];
-        int id[4];
-#pragma unroll
-        for (int t = 0; t < 4; ++t) { m1[t] = m2[t] = -__builtin_inff(); id[t] = 0; }
-        const f16x8v *ops = (const f16x8v *)a.ops + lane;
-        // row tiles requested two steps ahead (a step's products take less than a round trip to the L2)
-        f16x8v nx[2][2];
-        auto request = [&](int slot, int g) {
-            const int64_t at = (int64_t)(g < a.n_groups ? g : 0) * 128;
-            nx[slot][0] = ops[at];
-            nx[slot][1] = ops[at + 64];
-        };
-        if (wave < a.n_groups) { request(0, wave); request(1, wave + 4); }
-        auto step = [&](int slot, int g) {
-            const f16x8v a0 = nx[slot][0], a1 = nx[slot][1];
-            request(slot, g + 8);
-            __builtin_amdgcn_sched_barrier(0);                 // the requests stay up here
-            const f32x16v zero = {};
-            const int tiles = (nf - c0 + 31) >> 5;             // of vectors; 4 and more: all of them
-            f32x16v d0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(a0, bop[0], zero, 0, 0, 0);
-            f32x16v d1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(a1, bop[0], zero, 0, 0, 0);
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {                      // the next products run under this maximum
-                if (t >= tiles) break;
-                f32x16v e0, e1;
-                if (t < 3) {
-                    e0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(a0, bop[t + 1], zero, 0, 0, 0);
-                    e1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(a1, bop[t + 1], zero, 0, 0, 0);
-                }
-                __builtin_amdgcn_sched_barrier(0);
-                float m = __builtin_fmaxf(d0[0], d1[0]);
-#pragma unroll
-                for (int i = 1; i < 16; ++i) m = __builtin_fmaxf(__builtin_fmaxf(m, d0[i]), d1[i]);
-                m2[t] = __builtin_amdgcn_fmed3f(m1[t], m2[t], m);
-                if (m > m1[t]) id[t] = g;
-                m1[t] = __builtin_fmaxf(m1[t], m);
-                d0 = e0;
-                d1 = e1;
-            }
-            __builtin_amdgcn_sched_barrier(0);
-        };
-#pragma unroll 1
-        for (int g = wave; g < a.n_groups; g += 8) {
-            step(0, g);
-            if (g + 4 < a.n_groups) step(1, g + 4);
-        }
-        const int part = wave * 2 + (lane >> 5);
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            m1s[part][32 * t + (lane & 31)] = m1[t];
-            m2s[part][32 * t + (lane & 31)] = m2[t];
-            ids[part][32 * t + (lane & 31)] = id[t] * 2 + (lane >> 5);
+            atomicMin(&best[j], es_key(es_dist(xv, c, 0.25f * (float)n4), row));
         }
         __syncthreads();
-        if (tid < ES_CHUNK && c0 + tid < nf) {
-            float w1 = m1s[0][tid], w2 = m2s[0][tid];
-            int wid = ids[0][tid];
-#pragma unroll
-            for (int q = 1; q < 8; ++q) {
-                const float o1 = m1s[q][tid];
-                w2 = __builtin_fmaxf(__builtin_fmaxf(w2, m2s[q][tid]), __builtin_fminf(w1, o1));
-                if (o1 > w1) { w1 = o1; wid = ids[q][tid]; }
-            }
-            const int local = flag_v[c0 + tid];
-            const float margin = flag_m[c0 + tid], best = flag_a[c0 + tid];
-            const float d1 = 12.0f - 2.0f * w1, d2 = 12.0f - 2.0f * w2;
-            if (d1 <= best + margin) {
-                if (d2 <= __builtin_fminf(d1, best) + margin) slow(local);
-                else {
-                    const int e = atomicAdd(&n_exact, 1);
-                    exact_j[e] = (unsigned short)(c0 + tid);
-                    exact_group[e] = wid;
-                }
-            }
-        }
-        __syncthreads();
-        // the 32 rows of the winning half pair of tiles, a lane each, and the row of the full shells
-        const int ne = n_exact;
-        for (int e = tid >> 5; e < ne; e += ES_THREADS / 32) {
-            const int j = exact_j[e], grp = exact_group[e], i = lane & 31;
-            const int64_t v = v0 + flag_v[j];
-            float xv[8];
-            es_load(a.x, v, xv);
-            const int at = (grp >> 1) * 64 + (i >> 4) * 32 + 8 * ((i >> 2) & 3) + 4 * (grp & 1) + (i & 3);
-            int row = a.rem_rows[at];
-            const f16x8v c16 = ((const f16x8v *)a.ops)[(at >> 5) * 64 + (at & 31)];   // the row's values, exactly
-            float c[8];
-#pragma unroll
-            for (int q = 0; q < 8; ++q) c[q] = (float)c16[q];
-            float d = es_dist(xv, c, 12.0f);
-            if (row < 0) { d = __builtin_inff(); row = 0x7fffffff; }
-            const int fr = flag_row[j];
-            const float fd = es_dist(xv, a.table + (int64_t)fr * 8, a.norms[fr]);
-            if (fd < d || (fd == d && fr < row)) { d = fd; row = fr; }
-#pragma unroll
-            for (int o = 16; o > 0; o >>= 1) {
-                const float od = __shfl_xor(d, o, 64);
-                const int orow = __shfl_xor(row, o, 64);
-                if (od < d || (od == d && orow < row)) { d = od; row = orow; }
-            }
-            if (i == 0 && row != fr) es_store(a, v, row);
+        if (tid < nc) {
+            const int local = flags[c0 + tid];
+            if (s_signs[tid] & 512u) walk(local);
+            else es_store(a, v0 + local, (int)(uint32_t)best[tid]);
         }
         __syncthreads();
     }
-    if (tid == 0) a.slow_count[blockIdx.x] = n_slow;
+    if (tid == 0) a.walk_count[blockIdx.x] = n_walk;
 }
 
 // The table walk for the vectors left over, 64 at a time, a lane each: workgroup (64 vectors, part of
 // the table), its waves walking a quarter of the part.  The lowest (distance, row) of a part goes to the
 // vector's 64-bit minimum; the last part to arrive writes the row.
 __global__ void __launch_bounds__(ES_THREADS)
-e8_slow_kernel(const es_args a, int n_src, int per_src) {
+e8_walk_kernel(const es_args a, int n_src, int per_src) {
     constexpr int ROWS = 65536 / ES_SPLIT;                     // of one part, at most
     __shared__ int sums[4];
     __shared__ int64_t item[64];                               // the vector's list position
@@ -476,7 +465,7 @@ e8_slow_kernel(const es_args a, int n_src, int per_src) {
     const int per = (n_src + ES_THREADS - 1) / ES_THREADS;
     const int s0 = min(tid * per, n_src), s1 = min(s0 + per, n_src);
     int mine = 0;
-    for (int s = s0; s < s1; ++s) mine += a.slow_count[s];
+    for (int s = s0; s < s1; ++s) mine += a.walk_count[s];
     int first = mine;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
@@ -498,7 +487,7 @@ e8_slow_kernel(const es_args a, int n_src, int per_src) {
         if (first < base + 64 && first + mine > base) {
             int rank = first;
             for (int s = s0; s < s1; ++s)
-                for (int j = 0, c = a.slow_count[s]; j < c; ++j, ++rank)
+                for (int j = 0, c = a.walk_count[s]; j < c; ++j, ++rank)
                     if (rank >= base && rank < base + 64) item[rank - base] = (int64_t)s * per_src + j;
         }
         const int r0 = (int)((int64_t)a.n_entries * part / ES_SPLIT), n = (int)((int64_t)a.n_entries * (part + 1) / ES_SPLIT) - r0;
@@ -511,7 +500,7 @@ e8_slow_kernel(const es_args a, int n_src, int per_src) {
         __syncthreads();
         const bool on = base + lane < total;
         const int64_t at = item[on ? lane : 0];
-        const int64_t v = at / per_src * per_src + a.slow_list[at];
+        const int64_t v = at / per_src * per_src + a.walk_list[at];
         float xv[8], best = __builtin_inff();
         es_load(a.x, v, xv);
         int row = 0;
@@ -521,26 +510,24 @@ e8_slow_kernel(const es_args a, int n_src, int per_src) {
             const float d = es_dist(xv, (const float *)rows[i], row_norm[i]);
             if (d < best) { best = d; row = r0 + i; }
         }
-        uint32_t b = __builtin_bit_cast(uint32_t, best);
-        b = (b >> 31) ? ~b : b | 0x80000000u;                  // ordered like the floats
-        keys[wave][lane] = (unsigned long long)b << 32 | (uint32_t)row;
+        keys[wave][lane] = es_key(best, row);
         __syncthreads();
         if (wave == 0 && on) {
             unsigned long long key = keys[0][lane];
             for (int o = 1; o < 4; ++o) key = keys[o][lane] < key ? keys[o][lane] : key;
             // the minimum has been taken before the arrival is counted: its old value is waited for
-            const unsigned long long old = atomicMin(a.slow_key + at, key);
+            const unsigned long long old = atomicMin(a.walk_key + at, key);
             asm volatile("" ::"v"(old));
             __builtin_amdgcn_s_waitcnt(0);
-            if (atomicAdd(a.slow_arrive + at, 1) == ES_SPLIT - 1)
-                es_store(a, v, (int)(uint32_t)__hip_atomic_load(a.slow_key + at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+            if (atomicAdd(a.walk_arrive + at, 1) == ES_SPLIT - 1)
+                es_store(a, v, (int)(uint32_t)__hip_atomic_load(a.walk_key + at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
         }
         __syncthreads();
     }
 }
 
-// Vectors per workgroup: few while the chip is not filled, so that shell 12 is passed once with one tile of
-// them; more when it is, for fewer reads of the shell.
+// Vectors per workgroup: few while the chip is not filled, for latency; more when it is, so that the vectors with
+// more than one point in reach fill the threads that list the points.
 int es_per_wg(int64_t N) {
     const int64_t cus = glqh_device_cus();
     return N <= 2 * 64 * cus ? 64 : N < 4 * 256 * cus ? 256 : 512;
@@ -560,43 +547,33 @@ int glqh_launch_e8_quantize(const float *x, const float *table, const float *nor
 }
 
 int glqh_launch_e8_shell_index(const float *table, const float *norms, int n, uint32_t *keys, int *vals, int *counts,
-                               int *rem_rows, hipStream_t stream) {
+                               hipStream_t stream) {
     hipLaunchKernelGGL(es_clear_kernel, dim3(ES_SLOTS / 256), dim3(256), 0, stream, keys, counts);
     hipLaunchKernelGGL(es_index_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, table, norms, n, keys, vals,
-                       counts, rem_rows);
+                       counts);
     GLQH_LAUNCH_CHECK("e8 shell index launch");
-    return 0;
-}
-
-int glqh_launch_e8_shell_operands(const float *table, int *rem_rows, int n_rem, void *ops, hipStream_t stream) {
-    const int tiles = ((n_rem + 63) / 64) * 2;
-    if (tiles == 0) return 0;
-    hipLaunchKernelGGL(es_operands_kernel, dim3((unsigned)((tiles * 64 + 255) / 256)), dim3(256), 0, stream, table, rem_rows,
-                       n_rem, tiles, (f16 *)ops);
-    GLQH_LAUNCH_CHECK("e8 shell operands launch");
     return 0;
 }
 
 size_t glqh_e8_shell_ws_bytes(int64_t N) { return (size_t)N * 16 + (size_t)((N + 63) / 64) * 4; }
 
 int glqh_launch_e8_shell_quantize(const float *x, int64_t N, const float *table, const float *norms, int n_entries,
-                                  const uint32_t *keys, const int *vals, const void *ops, const int *rem_rows, int n_rem,
-                                  int64_t *idx_out, float *dec_out, void *ws, hipStream_t stream) {
+                                  const uint32_t *keys, const int *vals, int64_t *idx_out, float *dec_out, void *ws,
+                                  hipStream_t stream) {
     const int per = es_per_wg(N);
     const int64_t wgs = (N + per - 1) / per;
-    GLQH_REQUIRE(wgs <= 2147483647ll && N <= 2147483647ll, "e8 quantize: too many vectors");
+    GLQH_REQUIRE(N <= 2147483647ll, "e8 quantize: too many vectors");
     es_args a;
-    a.x = x; a.table = table; a.norms = norms; a.N = N; a.keys = keys; a.vals = vals; a.ops = (const f16 *)ops;
-    a.rem_rows = rem_rows; a.n_groups = (n_rem + 63) / 64; a.n_entries = n_entries; a.idx_out = idx_out; a.dec_out = dec_out;
-    a.slow_key = (unsigned long long *)ws;
-    a.slow_list = (int *)(a.slow_key + N);
-    a.slow_arrive = a.slow_list + N;
-    a.slow_count = a.slow_arrive + N;
+    a.x = x; a.table = table; a.norms = norms; a.N = N; a.keys = keys; a.vals = vals; a.n_entries = n_entries;
+    a.idx_out = idx_out; a.dec_out = dec_out;
+    a.walk_key = (unsigned long long *)ws;
+    a.walk_list = (int *)(a.walk_key + N);
+    a.walk_arrive = a.walk_list + N;
+    a.walk_count = a.walk_arrive + N;
     if (per == 512) hipLaunchKernelGGL(e8_shell_kernel<512>, dim3((unsigned)wgs), dim3(ES_THREADS), 0, stream, a);
     else if (per == 256) hipLaunchKernelGGL(e8_shell_kernel<256>, dim3((unsigned)wgs), dim3(ES_THREADS), 0, stream, a);
     else hipLaunchKernelGGL(e8_shell_kernel<64>, dim3((unsigned)wgs), dim3(ES_THREADS), 0, stream, a);
-    const int grid = 2 * glqh_device_cus();
-    hipLaunchKernelGGL(e8_slow_kernel, dim3((unsigned)grid), dim3(ES_THREADS), 0, stream, a, (int)wgs, per);
+    hipLaunchKernelGGL(e8_walk_kernel, dim3(2 * glqh_device_cus()), dim3(ES_THREADS), 0, stream, a, (int)wgs, per);
     GLQH_LAUNCH_CHECK("e8 shell quantize launch");
     return 0;
 }

@@ -41,6 +41,8 @@ struct {
     decltype(&glqh_fused_linear_trellis_3inst_group_rvq2) group_rvq2;
     decltype(&glqh_fused_moe_trellis_workspace_bytes) moe_ws;
     decltype(&glqh_fused_moe_trellis_3inst) moe;
+    decltype(&glqh_e8_shell_workspace_bytes) shell_ws;
+    decltype(&glqh_e8_shell_quantize) shell_quantize;
 } L;
 
 PyObject *g_ext = nullptr;                                     // glq_amd.ext's globals: its switches are read per call
@@ -615,6 +617,34 @@ PyObject *py_moe(PyObject *, PyObject *const *a, Py_ssize_t n) {
     });
 }
 
+// ---- E8 codewords ----------------------------------------------------------------------------
+// shell_quantize(x, table, norms, keys, vals, return_decoded) -> (decoded | None, indices)
+PyObject *py_shell_quantize(PyObject *, PyObject *const *a, Py_ssize_t n) {
+    NONE_UNLESS(n == 6 && !modes());
+    const at::Tensor *x = gpu(a[0], at::kFloat), *table = gpu(a[1], at::kFloat), *norms = gpu(a[2], at::kFloat);
+    const at::Tensor *keys = gpu(a[3], at::kInt), *vals = gpu(a[4], at::kInt);
+    NONE_UNLESS(x && table && norms && keys && vals && x->dim() == 2 && x->size(1) == 8 && x->size(0) >= 1);
+    NONE_UNLESS(same_device(*x, {table, norms, keys, vals}));
+    const int decoded = PyObject_IsTrue(a[5]);
+    NONE_UNLESS(decoded >= 0);
+    const int64_t N = x->size(0);
+    return guarded([&]() -> PyObject * {
+        c10::DeviceGuard guard(x->device());
+        at::Tensor idx(at::detail::empty_cuda({N}, at::kLong, x->device(), std::nullopt)), dec;
+        if (decoded) dec = like(*x, 8, at::kFloat);
+        int rc;
+        {
+            no_gil unlocked;
+            scratch ws(L.shell_ws(N));
+            rc = L.shell_quantize(x->const_data_ptr<float>(), N, table->const_data_ptr<float>(), norms->const_data_ptr<float>(), table->size(0),
+                                  (const uint32_t *)keys->const_data_ptr(), vals->const_data_ptr<int32_t>(), idx.mutable_data_ptr<int64_t>(),
+                                  decoded ? dec.mutable_data_ptr<float>() : nullptr, ws.p.get(), ws.bytes, stream_of(*x));
+        }
+        if (rc) return failed();
+        return Py_BuildValue("(NN)", decoded ? THPVariable_Wrap(std::move(dec)) : Py_NewRef(Py_None), THPVariable_Wrap(std::move(idx)));
+    });
+}
+
 // ---- module ------------------------------------------------------------------------------------
 // bind(handle of the library, glq_amd.ext's globals)
 PyObject *py_bind(PyObject *, PyObject *args) {
@@ -636,6 +666,8 @@ PyObject *py_bind(PyObject *, PyObject *args) {
     sym(L.group_rvq2, "glqh_fused_linear_trellis_3inst_group_rvq2");
     sym(L.moe_ws, "glqh_fused_moe_trellis_workspace_bytes");
     sym(L.moe, "glqh_fused_moe_trellis_3inst");
+    sym(L.shell_ws, "glqh_e8_shell_workspace_bytes");
+    sym(L.shell_quantize, "glqh_e8_shell_quantize");
     if (PyErr_Occurred()) return nullptr;
     if (!g_oom) {
         PyObject *torch = PyImport_ImportModule("torch");
@@ -652,6 +684,7 @@ PyMethodDef methods[] = {
     {"bind", py_bind, METH_VARARGS, "bind(library handle, globals of glq_amd.ext)"},
     {"trellis_linear", (PyCFunction)(void *)py_trellis_linear, METH_FASTCALL, "fused trellis linear, or None"},
     {"moe", (PyCFunction)(void *)py_moe, METH_FASTCALL, "routed trellis experts, or None"},
+    {"shell_quantize", (PyCFunction)(void *)py_shell_quantize, METH_FASTCALL, "codewords of the whole shell table, or None"},
     {"trellis_plan", py_trellis_plan, METH_VARARGS, "forward of a trellis E8RHTLinear"},
     {"shell_plan", py_shell_plan, METH_VARARGS, "forward of a shell E8RHTLinear"},
     {"group_plan", py_group_plan, METH_VARARGS, "forward of a merged trellis layer"},

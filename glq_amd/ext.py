@@ -1143,14 +1143,14 @@ _SHELL_MIN_ROWS = 4096
 
 
 class _ShellPlan:
-    """What the search on the whole shell table needs beside it, derived once per table: fp32 rows and norms, the
-    hash of the rows, matrix operands of the rows of norm 12.  `ok` is False for any other table."""
+    """What the search on the whole shell table needs beside it, derived once per table: fp32 rows and norms
+    and the hash of the rows.  `ok` is False for any other table."""
 
     def __init__(self, codebook, norms):
         lib = _lib.load()
         # copies: the cache must not keep alive the tensors whose end drops its entry
         self.table = codebook.to(torch.float32, copy=True).contiguous()
-        self.norms = (self.table * self.table).sum(-1) if norms is None else norms.to(torch.float32, copy=True).contiguous()
+        self.norms = (self.table * self.table).sum(-1) if norms is None else norms.to(self.table, copy=True).contiguous()
         self.given = None if norms is None else weakref.ref(norms.untyped_storage())
         self.ok = False
         if self.table.shape[0] < _SHELL_MIN_ROWS or self.norms.numel() != self.table.shape[0]:
@@ -1158,21 +1158,36 @@ class _ShellPlan:
         i32 = dict(dtype=torch.int32, device=self.table.device)
         n = self.table.shape[0]
         keys, vals, counts = torch.empty(1 << 17, **i32), torch.empty(1 << 17, **i32), torch.empty(8, **i32)
-        rem_rows = torch.empty(n + 64, **i32)
-        check(lib.glqh_e8_shell_index(_p(self.table), _p(self.norms), n, _p(keys), _p(vals), _p(counts), _p(rem_rows),
-                                      _stream()))
+        check(lib.glqh_e8_shell_index(_p(self.table), _p(self.norms), n, _p(keys), _p(vals), _p(counts), _stream()))
         counts = counts.tolist()
         if tuple(counts[:6]) != _SHELL_COUNTS or counts[7] != 0:
             return
-        self.n_rem = counts[6]
-        ops = torch.empty(max(1, -(-self.n_rem // 64)) * 1024, dtype=torch.float16, device=self.table.device)
-        check(lib.glqh_e8_shell_operands(_p(self.table), _p(rem_rows), self.n_rem, _p(ops), _stream()))
-        self.keys, self.vals, self.rem_rows, self.ops = keys, vals, rem_rows[:-(-self.n_rem // 64) * 64].clone(), ops
+        self.keys, self.vals = keys, vals
         self.ok = True
+
+
+_SHELL_SEEN = {}                     # (id, id) of table and norms -> what they were, and the plan found for them
 
 
 def _shell_plan(codebook, norms):
     """The plan of a table, made on its first use outside stream capture; None where there is none."""
+    if codebook.is_inference() or (norms is not None and norms.is_inference()):
+        return None                                            # tensors that do not count their changes
+    hit = _SHELL_SEEN.get((id(codebook), id(norms)))
+    if hit is not None and hit[0]() is codebook and hit[1] == codebook._version and hit[2] == codebook.data_ptr() and (
+            norms is None or (hit[3]() is norms and hit[4] == norms._version and hit[5] == norms.data_ptr())):
+        return hit[6]
+    plan = _find_shell_plan(codebook, norms)
+    if plan is not None:
+        if len(_SHELL_SEEN) >= 64:
+            _SHELL_SEEN.clear()
+        _SHELL_SEEN[(id(codebook), id(norms))] = (
+            weakref.ref(codebook), codebook._version, codebook.data_ptr(),
+            *((None, 0, 0) if norms is None else (weakref.ref(norms), norms._version, norms.data_ptr())), plan)
+    return plan
+
+
+def _find_shell_plan(codebook, norms):
     if codebook.dim() != 2 or codebook.shape[1] != 8 or not _SHELL_MIN_ROWS <= codebook.shape[0] <= 65536:
         return None
     extra = () if norms is None else _skey(norms)
@@ -1188,9 +1203,16 @@ def e8_quantize(x, codebook, codebook_norms=None, return_decoded=True):
     """E8ShellCodebook.quantize (glq/codebook.py:227-278) on the GPU: nearest row of
     `codebook` (K, 8) for every row of x (N, 8), lowest index on ties.  fp32 arithmetic in
     coordinate order, the reference's CPU branch.  Returns (decoded fp32 (N, 8), idx int64)."""
-    lib = _lib.load()
     if x.dim() != 2 or x.shape[1] != 8:
         raise RuntimeError(f"x must be (N, 8), got {tuple(x.shape)}")
+    if x.is_cuda and x.shape[0] and codebook.device == x.device:
+        with torch.cuda.device(x.device):
+            plan = _shell_plan(codebook, codebook_norms)
+        if plan is not None:
+            got = host().shell_quantize(x.contiguous().to(torch.float32), plan.table, plan.norms, plan.keys, plan.vals, return_decoded)
+            if got is not None:
+                return got
+    lib = _lib.load()
     xf = x.contiguous().to(torch.float32)
     _chk(xf, "x", torch.float32)
     N = xf.shape[0]
@@ -1198,13 +1220,6 @@ def e8_quantize(x, codebook, codebook_norms=None, return_decoded=True):
     dec = torch.empty(N, 8, dtype=torch.float32, device=x.device) if return_decoded else None
     if N:
         with torch.cuda.device(x.device):
-            plan = _shell_plan(codebook, codebook_norms)
-            if plan is not None:
-                ws = _ws(lib.glqh_e8_shell_workspace_bytes(N), x.device)
-                check(lib.glqh_e8_shell_quantize(
-                    _p(xf), N, _p(plan.table), _p(plan.norms), plan.table.shape[0], _p(plan.keys), _p(plan.vals),
-                    _p(plan.ops), _p(plan.rem_rows), plan.n_rem, _p(idx), _p(dec), _p(ws), ws.numel(), _stream()))
-                return dec, idx
             cb = codebook.contiguous().to(torch.float32)
             norms = (cb * cb).sum(-1) if codebook_norms is None else codebook_norms.contiguous().to(torch.float32)
             check(lib.glqh_e8_quantize(_p(xf), _p(cb), _p(norms), N, cb.shape[0], _p(idx), _p(dec), _stream()))

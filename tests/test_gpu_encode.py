@@ -55,7 +55,7 @@ def test_e8_quantize_residual_stage_and_size():
     assert torch.equal(i1, again)
 
 
-@pytest.mark.parametrize("N,scale", [(1, 1.0), (255, 3.0), (257, 0.3), (5000, 1.5), (70001, 1.0), (262145, 1.0)])
+@pytest.mark.parametrize("N,scale", [(1, 1.0), (255, 3.0), (257, 0.3), (5000, 1.5), (20001, 4.0), (70001, 1.0), (40000, 100.0), (262145, 1.0)])
 def test_e8_quantize_on_the_shell_table_equals_the_table_walk(N, scale):
     """The search by the table's symmetry against the kernel that walks all rows (pinned on the oracle above through
     tables it does not recognise), at sizes around a workgroup's and past the switch to 512 vectors per workgroup:
