@@ -1375,9 +1375,9 @@ struct moe_plan {
 
 // From this many (token, choice) slots on the rows are grouped by expert and every expert's stream is read
 // once per 16 of its rows; below, every slot reads its expert's stream for itself (no routing launch, no
-// separate input transforms).  The grouped form pays three more launches and wins once slots share experts:
-// measured on 128 experts of 2048 -> 2 x 768 -> 2048 with 8 choices, 64 slots 79.7 (per slot) against 84.4 us
-// (grouped), 128 slots 135.9 against 107.6, 512 slots 466 against 147.  GLQ_MOE_GROUP_MIN overrides (read once).
+// separate input transforms).  The grouped form pays three more launches and wins once slots share experts: measured on 128 experts of
+// 2048 -> 2 x 768 -> 2048 with 8 choices, 32 slots 51.7 (per slot) against 54.7 us (grouped), 48 slots 69.0 / 67.8,
+// 64 slots 81.3 / 72.3, 88 slots 105.1 / 78.3.  GLQ_MOE_GROUP_MIN overrides (read once).
 static int64_t moe_group_min(int64_t n_experts) {
     static const int64_t v = [] {
         const char *e = getenv("GLQ_MOE_GROUP_MIN");
@@ -1385,7 +1385,7 @@ static int64_t moe_group_min(int64_t n_experts) {
         return (int64_t)(x > 0 ? x : 0);
     }();
     if (v > 0) return v;
-    const int64_t d = 3 * n_experts / 4;
+    const int64_t d = 3 * n_experts / 8;
     return d < 16 ? 16 : d;
 }
 

@@ -616,21 +616,28 @@ struct tr_moe_group_args {
     int n_slots, x_div;
 };
 
-// One pass over the K slot for NT tiles of 16 of the expert's rows, positions [t0, t0 + 16 NT) of its run in perm.
-template <int R, int NT, int R2 = 0>
+// One pass over the K slot for NT tiles of TP of the expert's rows, positions [t0, t0 + TP NT) of its run in perm.
+// TP = 4 (NT = 1): an expert of few rows stages a quarter of the operand slots; lanes past the fourth row read a
+// zeroed block behind the chunk.
+template <int R, int NT, int R2 = 0, int TP = 16>
 __device__ __forceinline__ void moe_group_pass(const tr_moe_group_args &g, const f16 *__restrict__ x, int m, int k,
                                                int kp0, int kp1, int CH, const uint8_t *lane_base, const mma_lane a,
                                                int wave, int o0, int cnt, int t0, float pscale, int kslot,
                                                u32x4 *xs_lds, int *slotmap, const uint8_t *lane_base2 = nullptr) {
-    constexpr int TPS = mma_tps<16>();
+    constexpr int TPS = mma_tps<TP>(), CL = 4 * TP;
     constexpr int REC = 4 * R;
     constexpr int RB = R2 > 0 ? R2 : 1, REC2 = 4 * RB;
     constexpr int G = mma_red_groups<NT>();                      // row groups per round of the final sum
-    constexpr int PER_WAVE = G * NT * 256;
+    constexpr int PER_WAVE = G * NT * 4 * CL;
     uint32_t *xs = (uint32_t *)xs_lds;
-    float *red = (float *)xs_lds;                                // [TR_WAVES][G][NT][4][64]
+    float *red = (float *)xs_lds;                                // [TR_WAVES][G][NT][4][CL]
+    const bool live = TP == 16 || a.tokl < TP;
+    u32x4 *zero_blk = xs_lds + CH * (NT * 8 * TPS);
     __syncthreads();                                             // the previous pass is done with slotmap and red
-    if (threadIdx.x < 16 * NT)
+    if constexpr (TP < 16) {
+        if (threadIdx.x < 8 * TPS) zero_blk[threadIdx.x] = u32x4{0u, 0u, 0u, 0u};
+    }
+    if (threadIdx.x < TP * NT)
         slotmap[threadIdx.x] = t0 + (int)threadIdx.x < cnt ? g.perm[o0 + t0 + threadIdx.x] : -1;
     int kp = kp0 + wave;
     tr_record<R> cur = {};
@@ -648,9 +655,9 @@ __device__ __forceinline__ void moe_group_pass(const tr_moe_group_args &g, const
         const int c1 = min(c0 + CH, kp1), n = c1 - c0;
         fht_barrier<true>();                                     // slotmap written / previous chunk consumed
         // one item = 32 bytes of one row: columns 16 ks .. 16 ks + 15 of k-pair c0 + u
-        for (int idx = threadIdx.x; idx < 32 * NT * n; idx += TR_THREADS) {
+        for (int idx = threadIdx.x; idx < 2 * TP * NT * n; idx += TR_THREADS) {
             const int ks = idx & 1, u = (idx >> 1) % n, tk = (idx >> 1) / n;
-            const int tt = tk >> 4, tl = tk & 15;
+            const int tt = tk / TP, tl = tk % TP;
             const int sl = slotmap[tk];
             const f16 *p = x + (int64_t)(sl < 0 ? 0 : sl / g.x_div) * k + 32 * (c0 + u) + 16 * ks;
             u32x4 l0 = *(const u32x4 *)p, l1 = *(const u32x4 *)(p + 8);
@@ -669,9 +676,9 @@ __device__ __forceinline__ void moe_group_pass(const tr_moe_group_args &g, const
                 nxt = tr_load_record<R>(lane_base + (int64_t)(kp + TR_WAVES) * 32 * REC);
                 if constexpr (R2 > 0) nxtb = tr_load_record<RB>(lane_base2 + (int64_t)(kp + TR_WAVES) * 32 * REC2);
             }
-            const u32x4 *xsl = xs_lds + ((kp - c0) * NT * 8 + a.q) * TPS + a.tokl;
-            acc = mma_record<R, 16, NT>(cur, a.next1, a.next2, xsl, acc);
-            if constexpr (R2 > 0) accb = mma_record<RB, 16, NT>(curb, a.next1, a.next2, xsl, accb);
+            const u32x4 *xsl = live ? xs_lds + ((kp - c0) * NT * 8 + a.q) * TPS + a.tokl : zero_blk;
+            acc = mma_record<R, TP, NT>(cur, a.next1, a.next2, xsl, acc);
+            if constexpr (R2 > 0) accb = mma_record<RB, TP, NT>(curb, a.next1, a.next2, xsl, accb);
             cur = nxt;
             curb = nxtb;
         }
@@ -687,22 +694,22 @@ __device__ __forceinline__ void moe_group_pass(const tr_moe_group_args &g, const
 #pragma unroll
     for (int s0 = 0; s0 < 4; s0 += G) {
         __syncthreads();
-        {
-            const int cl = a.q * 16 + a.tokl;
+        if (live) {
+            const int cl = a.q * TP + a.tokl;
 #pragma unroll
             for (int sg = 0; sg < G; ++sg)
 #pragma unroll
                 for (int tt = 0; tt < NT; ++tt)
 #pragma unroll
                     for (int r = 0; r < 4; ++r)
-                        red[wave * PER_WAVE + ((sg * NT + tt) * 4 + r) * 64 + cl] = acc.v[s0 + sg][tt][r];
+                        red[wave * PER_WAVE + ((sg * NT + tt) * 4 + r) * CL + cl] = acc.v[s0 + sg][tt][r];
         }
         __syncthreads();
         for (int i2 = threadIdx.x; i2 < PER_WAVE; i2 += TR_THREADS) {
-            const int cl = i2 & 63, r = (i2 >> 6) & 3, tt = (i2 >> 8) % NT, sg = (i2 >> 8) / NT;
-            const int i = 4 * (cl >> 4) + r;
+            const int cl = i2 % CL, r = (i2 / CL) & 3, tt = (i2 / (4 * CL)) % NT, sg = (i2 / (4 * CL)) / NT;
+            const int i = 4 * (cl / TP) + r;
             const int row = 64 * blockIdx.x + 32 * (i >> 3) + (i & 7) + 8 * (s0 + sg);
-            const int sl = slotmap[16 * tt + (cl & 15)];
+            const int sl = slotmap[TP * tt + (cl % TP)];
             if (sl < 0 || row >= m) continue;
             float v = red[i2];
 #pragma unroll
@@ -712,13 +719,14 @@ __device__ __forceinline__ void moe_group_pass(const tr_moe_group_args &g, const
     }
 }
 
-// Chunk lengths (k-pairs staged per barrier pair) of the passes with one, two and four row tiles.
+// Chunk lengths (k-pairs staged per barrier pair) of the passes with one, two and four row tiles, and of the pass
+// with four rows.
 struct moe_chunks {
-    int ch1, ch2, ch4;
+    int ch1, ch2, ch4, ch_few;
 };
 
-// WIDE = false: passes of 16 rows only (few rows per expert: the registers of the wide passes would cost
-// occupancy for nothing).
+// WIDE = false: passes of 16 rows, or of four for an expert with no more (few rows per expert: the registers of the
+// wide passes would cost occupancy for nothing, and so would their LDS).
 template <int R, bool WIDE, int R2 = 0>
 __global__ void __launch_bounds__(TR_THREADS)
 tr_mma_moe_grouped_kernel(tr_moe_group_args g, const f16 *__restrict__ x, int m, int k, int S, moe_chunks ch) {
@@ -746,6 +754,16 @@ tr_mma_moe_grouped_kernel(tr_moe_group_args g, const f16 *__restrict__ x, int m,
 
     // The stream is read once per pass: as many of the expert's rows per pass as there are, up to 64.
     for (int t0 = 0; t0 < cnt;) {
+        if constexpr (!WIDE) {
+            if (cnt - t0 <= 4) {
+                moe_group_pass<R, 1, R2, 4>(g, x, m, k, kp0, kp1, ch.ch_few, lane_base, a, wave, o0, cnt, t0, pscale, kslot, xs_lds, slotmap, lane_base2);
+                return;
+            }
+            if (cnt - t0 <= 8) {
+                moe_group_pass<R, 1, R2, 8>(g, x, m, k, kp0, kp1, ch.ch_few / 2, lane_base, a, wave, o0, cnt, t0, pscale, kslot, xs_lds, slotmap, lane_base2);
+                return;
+            }
+        }
         const int rem = WIDE ? cnt - t0 : 0;
         if (rem > 32) {
             moe_group_pass<R, 4, R2>(g, x, m, k, kp0, kp1, ch.ch4, lane_base, a, wave, o0, cnt, t0, pscale, kslot, xs_lds, slotmap, lane_base2);
@@ -1149,6 +1167,9 @@ int glqh_moe_grouped_wide(int n_slots, int n_experts) {
     return (int64_t)n_slots >= (int64_t)moe_wide_min_rows() * n_experts;
 }
 
+// k-pairs per chunk of the pass with four rows: one 32-byte item per thread (and 16 KB of LDS, what the 16-row pass takes)
+constexpr int MOE_FEW_CHUNK = 32;
+
 // packed2 (with stride2_bytes, R2; R = 4; passes of 16 rows only): stacked experts, both streams in the same passes,
 // the second one's sums times pscale_dev[expert] added in registers.  (With the passes of up to 64 rows the second
 // set of accumulators costs the occupancy: 166 registers, 256 tokens of 6 bpw experts 421 -> 578 us; those keep a
@@ -1168,15 +1189,22 @@ int glqh_launch_trellis_mma_moe_grouped(const void *packed, int64_t stride_bytes
     GLQH_REQUIRE(!(packed2 && wide), "routed experts: two streams per pass are served with passes of 16 rows only");
     // chunk of the one-tile pass as in tr_mma_kernel; the wider passes take what the same LDS holds
     moe_chunks ch;
-    ch.ch1 = mma_chunk_cap<16, 1>();
+    // (without the wide passes eight k-pairs a chunk: half the LDS, twice the waves; 128 slots of 128 experts 85 -> 80 us
+    // in the two decode launches, with four k-pairs 91)
+    ch.ch1 = wide ? mma_chunk_cap<16, 1>() : 8;
     ch.ch2 = std::max(4, (ch.ch1 / 2) & ~3);
     ch.ch4 = std::max(4, (ch.ch1 / 4) & ~3);
     const int s4 = (S + 3) & ~3;
     ch.ch1 = std::min(ch.ch1, s4);
     ch.ch2 = std::min(ch.ch2, s4);
     ch.ch4 = std::min(ch.ch4, s4);
-    size_t lds = std::max({(size_t)ch.ch1 * mma_slot_bytes(16, 1), (size_t)ch.ch2 * mma_slot_bytes(16, 2),
-                           (size_t)ch.ch4 * mma_slot_bytes(16, 4), (size_t)mma_red_bytes<16, 4>()});
+    ch.ch_few = std::min(MOE_FEW_CHUNK, (s4 + 7) & ~7);
+    size_t lds = std::max((size_t)ch.ch1 * mma_slot_bytes(16, 1), (size_t)mma_red_bytes<16, 1>());
+    if (wide)
+        lds = std::max({lds, (size_t)ch.ch2 * mma_slot_bytes(16, 2), (size_t)ch.ch4 * mma_slot_bytes(16, 4),
+                        (size_t)mma_red_bytes<16, 4>()});
+    else
+        lds = std::max({lds, (size_t)(ch.ch_few + 1) * mma_slot_bytes(4, 1), (size_t)(ch.ch_few / 2 + 1) * mma_slot_bytes(8, 1)});
     tr_moe_group_args g = {(const uint8_t *)packed, stride_bytes, (const uint8_t *)packed2, stride2_bytes, perm, offs,
                            pscale_dev, part, n_slots, x_div};
     const dim3 grid((unsigned)((m + 63) / 64), (unsigned)ksplit, (unsigned)n_experts);

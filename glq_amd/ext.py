@@ -1179,7 +1179,7 @@ def _shell_plan(codebook, norms):
         return hit[6]
     plan = _find_shell_plan(codebook, norms)
     if plan is not None:
-        if len(_SHELL_SEEN) >= 64:
+        if len(_SHELL_SEEN) >= 8:                              # bounded: an entry keeps its plan
             _SHELL_SEEN.clear()
         _SHELL_SEEN[(id(codebook), id(norms))] = (
             weakref.ref(codebook), codebook._version, codebook.data_ptr(),
