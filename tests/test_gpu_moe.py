@@ -217,7 +217,7 @@ def test_refusals(ext):
                                                  (256, 128, 200, 3, 0), (320, 192, 300, 2, 2), (256, 128, 530, 2, 0),
                                                  (256, 128, 1100, 4, 0), (320, 192, 600, 2, 2)])
 def test_many_slots_grouped_by_expert(ext, hidden, inter, T, K, K2):
-    """From max(16, 3/4 of the experts) slots on the rows are grouped by expert.  Skewed routing: every token's first choice is
+    """From max(16, 3/8 of the experts) slots on the rows are grouped by expert.  Skewed routing: every token's first choice is
     expert 2 (more than two tiles of 16 rows for it), expert 5 gets nothing, some ids are out of range.  From an
     average of 12 rows per expert on, a pass over an expert's stream takes up to 64 of its rows: the cases give
     expert 2 one pass of 16 (T = 16), of 32 (24), of 64 (33, 40), 64 + 32 (90) and 64 + 16 (80) rows.  From 48 rows
@@ -241,6 +241,22 @@ def test_many_slots_grouped_by_expert(ext, hidden, inter, T, K, K2):
     worst = max(rel(y[i], ref[i]) for i in range(T))
     assert worst < 3 * TOL, worst                            # no single token is off
     assert torch.equal(y, ext.glq_fused_moe_trellis_3inst_cuda(x.to(DEV), t(ids), t(w), *a))
+
+
+@pytest.mark.parametrize("hidden,inter,K2", [(1088, 128, 0), (256, 64, 2)])
+def test_experts_of_four_five_eight_and_nine_rows(ext, hidden, inter, K2):
+    """The decode pass takes four, eight or sixteen of an expert's rows by how many it has; 1088 columns are 34
+    k-pairs, more than one staged chunk of any of the passes, the last one partial."""
+    say("moe few rows", hidden, inter, K2)
+    ex = experts(5, hidden, inter, 4, K2, seed=6)
+    ids = np.random.default_rng(0).permutation(np.repeat([0, 1, 2, 3, 4], [4, 5, 8, 9, 1])).astype(np.int64)[:, None]
+    T = ids.shape[0]
+    rng = np.random.default_rng(1)
+    w = rng.random((T, 1)).astype(np.float32)
+    x = torch.from_numpy(rng.standard_normal((T, hidden)).astype(np.float32)).bfloat16()
+    y = ext.glq_fused_moe_trellis_3inst_cuda(x.to(DEV), t(ids), t(w), *ex.device_args(0))
+    ref = ex.oracle(x.float().numpy(), ids, w, 0)
+    assert max(rel(y[i], ref[i]) for i in range(T)) < 2 * TOL
 
 
 @pytest.mark.parametrize("hidden,inter", [(256, 4096), (8192, 128)])
