@@ -135,7 +135,7 @@ template <> __device__ __forceinline__ void store8<uint16_t>(uint16_t *p, const 
     *(u32x4 *)p = w;
 }
 
-// blockIdx.x = block, blockIdx.y = token.  Requires canonical blocks of 8..8192 points, 16-byte
+// Requires canonical blocks of 8..8192 points, 16-byte
 // aligned rows of x (x_stride % 8 == 0 elements for 16-bit types) and out.  The transform runs
 // in registers (fht_wave<E>): thread t of 512 holds elements E*t .. E*t+E-1 of the block (E = 16
 // for 8192 points, 8 below), log2(E) butterfly levels stay in the thread, six run across the
@@ -173,20 +173,21 @@ __device__ __forceinline__ void reg_gather_runs(float (&v)[E], int log_len, floa
     }
 }
 
-// What a thread of a whole-block workgroup does.  Blocks of 1024 points and more: one token (row) per
-// workgroup, thread te = tid.  Blocks of at most 512 points are transformed inside one wave (eight elements
-// per thread, no exchange through LDS), so a workgroup takes 4096 / bs tokens at once: thread tid works on
-// token tid / (bs / 8) of them as thread te = tid % (bs / 8), with staging space of its own.
+// What a thread of a whole-block workgroup does.  A workgroup of 2^(lwg - 3) threads holds 2^lwg points, eight per
+// thread (a block of 8192: sixteen): smaller blocks are 2^lwg / bs tokens (rows) at once, thread tid working on
+// token tid / (bs / 8) of them as thread te = tid % (bs / 8), with exchange and staging space of its own in LDS.
+// (One token of 1024 points per workgroup left three quarters of its threads without elements: 1360 tokens x
+// 1984 points out 15.2 -> 6.0 us.)
 struct wide_role {
     int te, tok, nthr, lds_off;                              // tok: the token's number inside the workgroup
     bool active;                                             // false: past the workgroup's tokens
 };
 
-__device__ __forceinline__ wide_role wide_role_of(const rht_slice &blk, int ntok) {
+__device__ __forceinline__ wide_role wide_role_of(const rht_slice &blk, int lwg, int ntok) {
     wide_role r;
     const int tid = threadIdx.x;
-    if (blk.log_bs > 9) {
-        r.te = tid; r.tok = 0; r.nthr = REG_THREADS; r.lds_off = 0; r.active = true;
+    if (blk.log_bs >= lwg) {
+        r.te = tid; r.tok = 0; r.nthr = 1 << (lwg - 3); r.lds_off = 0; r.active = true;
     } else {
         const int lthr = blk.log_bs - 3;
         r.te = tid & ((1 << lthr) - 1);
@@ -197,9 +198,76 @@ __device__ __forceinline__ wide_role wide_role_of(const rht_slice &blk, int ntok
     }
     return r;
 }
-constexpr int WIDE_SMALL_LOG = 9;                            // blocks up to 512 points: 4096 / bs tokens per workgroup
-// LDS for the staging of a small block's tokens (layout 2: blocks of 32 points and more)
-constexpr size_t WIDE_SMALL_LDS = (size_t)(4096 + 512 + 8 * 128) * sizeof(float);
+// Points per workgroup: 4096 where there is work for two such workgroups per CU, fewer (a power of two, at least
+// the largest block: every block is one workgroup's) where they would leave CUs without one.
+constexpr int WIDE_LOG_WG = 12, WIDE_LOG_WG_MIN = 9;
+int wide_log_wg(int log_max, int64_t B, int64_t total) {
+    int lwg = WIDE_LOG_WG;
+    while (lwg > WIDE_LOG_WG_MIN && lwg > log_max && ((B * total) >> lwg) < 512) --lwg;
+    return lwg;
+}
+// LDS: the largest block, or the tokens of the smallest one that goes through LDS (from 32 points in layout 2,
+// 1024 otherwise)
+size_t wide_lds_bytes(int log_max, int lwg, bool small_staged) {
+    const size_t n = (size_t)1 << std::max(log_max, lwg);
+    return (n + n / 8 + (small_staged ? 8 << (lwg - 5) : 8 * 4) + 16) * sizeof(float);
+}
+
+// Which block of which tokens a workgroup takes.  The grid holds, for one block of the row after the other
+// (the largest first, so that the tail of the launch is made of small pieces), ceil(B / tokens per workgroup)
+// workgroups.  XCD_RUNS (the token-fast layouts): workgroup L runs on XCD L % 8, and blocks of one token per
+// workgroup give XCD r the tokens r * ceil(B / 8) ..., in order: the 64-byte pieces of neighbouring tokens share
+// a 128-byte line, which is then completed inside one L2 instead of written back in parts (smaller blocks
+// complete their lines inside the workgroup).
+struct wide_work {
+    rht_slice blk;
+    int row0, ntok;                                          // ntok <= 0: nothing to do (uniform)
+};
+template <bool XCD_RUNS>
+__host__ __device__ __forceinline__ int wide_sets(int log_bs, int lwg, int B) {
+    const int lt = log_bs < lwg ? lwg - log_bs : 0, n = (B + (1 << lt) - 1) >> lt;
+    return XCD_RUNS ? (n + 7) & ~7 : n;
+}
+template <bool XCD_RUNS>
+int64_t wide_grid(int canon, int lwg, int B) {
+    int64_t n = 0;
+    for (int l = 0; l < 31; ++l)
+        if (canon >> l & 1) n += wide_sets<XCD_RUNS>(l, lwg, B);
+    return n;
+}
+template <bool XCD_RUNS>
+__device__ __forceinline__ wide_work wide_work_of(const glqh_meta_args margs, float single_norm, int lwg, int B) {
+    wide_work w;
+    int L = blockIdx.x;
+    uint32_t rem = (uint32_t)margs.canon;
+    int log_bs = 31 - __builtin_clz(rem), n = wide_sets<XCD_RUNS>(log_bs, lwg, B);
+    while (L >= n) {                                         // uniform; the grid ends with the last block
+        L -= n;
+        rem &= ~(1u << log_bs);
+        log_bs = 31 - __builtin_clz(rem);
+        n = wide_sets<XCD_RUNS>(log_bs, lwg, B);
+    }
+    w.blk.off = margs.canon - (int)rem;
+    w.blk.bs = 1 << log_bs;
+    w.blk.log_bs = w.blk.log_len = log_bs;
+    w.blk.r = 0;
+    w.blk.nsub = 1;
+    w.blk.live = true;
+    w.blk.norm = (margs.canon & (margs.canon - 1)) == 0 && single_norm != 0.0f ? single_norm : rsqrt_pow2(log_bs);
+    if (log_bs < lwg) {
+        const int lt = lwg - log_bs;
+        w.row0 = L << lt;
+        w.ntok = min(1 << lt, B - w.row0);
+    } else if (XCD_RUNS) {
+        const int per_xcd = (B + 7) >> 3;
+        w.row0 = (L & 7) * per_xcd + (L >> 3);
+        w.ntok = w.row0 < B ? 1 : 0;
+    } else {
+        w.row0 = L;
+        w.ntok = 1;
+    }
+    return w;
+}
 
 // LAYOUT of the transformed row: 0 = row-major (out + token * n_pad); 1 and 2 = the tile kernels'
 // operand layouts out[col / 32][token][4][8]: 32 columns of one token are 64 contiguous bytes, as
@@ -211,7 +279,7 @@ __device__ __forceinline__ void input_rht_wide_body(const XT *__restrict__ x, in
                                                    int in_features, int n_pad, int Mp, int token,
                                                    const rht_slice &blk, float *s, const wide_role role) {
     // te: the thread's number among those of its token; st: the token's staging space in LDS
-    const int tid = threadIdx.x, te = role.te;
+    const int te = role.te;
     const bool active = role.active && E * te < blk.bs;
     float *st = s + role.lds_off;
     const int i = E * te;
@@ -234,7 +302,7 @@ __device__ __forceinline__ void input_rht_wide_body(const XT *__restrict__ x, in
 #pragma unroll
         for (int e = 0; e < E; ++e) v[e] *= sf[e];
     }
-    fht_wave<E>(v, blk.log_len, s, tid);
+    fht_wave<E>(v, blk.log_len, st, te);
     if constexpr (LAYOUT == 2) {
         // every element through LDS, then one 16-byte slot (k-pair, q) per thread and round
         constexpr int LE = fht_wave_log<E>::v;
@@ -259,7 +327,7 @@ __device__ __forceinline__ void input_rht_wide_body(const XT *__restrict__ x, in
         }
         return;
     }
-    reg_gather_runs<E>(v, blk.log_len, s, tid, active);
+    reg_gather_runs<E>(v, blk.log_len, st, te, active);
     if (active) {
 #pragma unroll
         for (int e = 0; e < E; ++e) v[e] *= blk.norm;
@@ -277,45 +345,21 @@ __device__ __forceinline__ void input_rht_wide_body(const XT *__restrict__ x, in
     }
 }
 
-// blocks of 8192 points take 16 elements per thread, smaller ones 8 (all 512 threads busy on 4096).
-// One-dimensional grid: workgroup L runs on XCD L % 8, XCD r owns tokens r * ceil(B / 8) ..., and the
-// workgroups of an XCD come in sets of eight that take the same block of eight consecutive tokens: in the
-// token-fast layouts the 16-byte pieces of eight consecutive tokens share a 128-byte line, which is then
-// completed inside one L2 instead of written back in eight parts; and the blocks of a row differ in size
-// (11008 = 8192 + 2048 + 512 + 256), so dealing a token's four blocks to neighbouring workgroups, which go
-// to the four shader engines of an XCD in turn, put every 8192-point block on the same engine
-// (4096 x 11008: 112 -> 70 us; rows of one or three blocks: no change).
+// blocks of 8192 points take 16 elements per thread, smaller ones 8 (all 512 threads busy on 4096)
 template <typename XT, typename OT, int LAYOUT>
 __global__ void __launch_bounds__(REG_THREADS)
 input_rht_wide_kernel(const XT *__restrict__ x, int64_t x_stride, const f16 *__restrict__ sv,
-                     OT *__restrict__ out, int in_features, int n_pad, int Mp, int B, int n_blocks,
+                     OT *__restrict__ out, int in_features, int n_pad, int Mp, int B, int lwg,
                      glqh_meta_args margs, float single_norm) {
     extern __shared__ float s[];
-    const int L = blockIdx.x, per_xcd = (B + 7) >> 3;
-    const int j = L >> 3;
-    const int member = j & 7, rest = j >> 3, g = rest / n_blocks;
-    const rht_slice blk = rht_slice_of(margs, single_norm, rest % n_blocks);
-    if (blk.log_bs <= WIDE_SMALL_LOG) {
-        // one workgroup of 4096 / bs / 8 sets takes all their tokens (the eight members in turn, so that the
-        // work reaches every shader engine), the others retire
-        const int lsets = 12 - blk.log_bs - 3;
-        if ((g & ((1 << lsets) - 1)) != 0 || member != ((g >> lsets) & 7)) return;
-        const int t_in = g * 8, tok0 = (L & 7) * per_xcd + t_in;
-        if (t_in >= per_xcd || tok0 >= B) return;
-        const int ntok = min(8 << lsets, min(per_xcd - t_in, B - tok0));
-        const wide_role role = wide_role_of(blk, ntok);
-        input_rht_wide_body<8, XT, OT, LAYOUT>(x, x_stride, sv, out, in_features, n_pad, Mp,
-                                               tok0 + min(role.tok, ntok - 1), blk, s, role);
-        return;
-    }
-    const int t_in = g * 8 + member;                          // token, counted inside the XCD's share
-    const int token = (L & 7) * per_xcd + t_in;
-    if (token >= B || t_in >= per_xcd) return;                // uniform over the workgroup
-    const wide_role role = wide_role_of(blk, 1);
-    if (blk.log_bs > 12)
-        input_rht_wide_body<16, XT, OT, LAYOUT>(x, x_stride, sv, out, in_features, n_pad, Mp, token, blk, s, role);
+    const wide_work w = wide_work_of<true>(margs, single_norm, lwg, B);
+    if (w.ntok <= 0) return;
+    const wide_role role = wide_role_of(w.blk, lwg, w.ntok);
+    const int token = w.row0 + min(role.tok, w.ntok - 1);
+    if (w.blk.log_bs > 12)
+        input_rht_wide_body<16, XT, OT, LAYOUT>(x, x_stride, sv, out, in_features, n_pad, Mp, token, w.blk, s, role);
     else
-        input_rht_wide_body<8, XT, OT, LAYOUT>(x, x_stride, sv, out, in_features, n_pad, Mp, token, blk, s, role);
+        input_rht_wide_body<8, XT, OT, LAYOUT>(x, x_stride, sv, out, in_features, n_pad, Mp, token, w.blk, s, role);
 }
 
 // The same rows under several sign vectors in one launch, trellis operand layout out (layers of a group that were
@@ -328,31 +372,16 @@ struct rht_in_wide_multi {
 template <typename XT>
 __global__ void __launch_bounds__(REG_THREADS)
 input_rht_wide_multi_kernel(const XT *__restrict__ x, int64_t x_stride, rht_in_wide_multi mg, int in_features, int n_pad,
-                            int Mp, int B, int n_blocks, glqh_meta_args margs, float single_norm) {
+                            int Mp, int B, int lwg, glqh_meta_args margs, float single_norm) {
     extern __shared__ float s[];
     const f16 *sv = mg.sv[blockIdx.y];
     f16 *out = mg.out[blockIdx.y];
-    const int L = blockIdx.x, per_xcd = (B + 7) >> 3;
-    const int j = L >> 3;
-    const int member = j & 7, rest = j >> 3, g = rest / n_blocks;
-    const rht_slice blk = rht_slice_of(margs, single_norm, rest % n_blocks);
-    if (blk.log_bs <= WIDE_SMALL_LOG) {
-        const int lsets = 12 - blk.log_bs - 3;
-        if ((g & ((1 << lsets) - 1)) != 0 || member != ((g >> lsets) & 7)) return;
-        const int t_in = g * 8, tok0 = (L & 7) * per_xcd + t_in;
-        if (t_in >= per_xcd || tok0 >= B) return;
-        const int ntok = min(8 << lsets, min(per_xcd - t_in, B - tok0));
-        const wide_role role = wide_role_of(blk, ntok);
-        input_rht_wide_body<8, XT, f16, 2>(x, x_stride, sv, out, in_features, n_pad, Mp, tok0 + min(role.tok, ntok - 1), blk, s,
-                                           role);
-        return;
-    }
-    const int t_in = g * 8 + member;
-    const int token = (L & 7) * per_xcd + t_in;
-    if (token >= B || t_in >= per_xcd) return;                // uniform over the workgroup
-    const wide_role role = wide_role_of(blk, 1);
-    if (blk.log_bs > 12) input_rht_wide_body<16, XT, f16, 2>(x, x_stride, sv, out, in_features, n_pad, Mp, token, blk, s, role);
-    else input_rht_wide_body<8, XT, f16, 2>(x, x_stride, sv, out, in_features, n_pad, Mp, token, blk, s, role);
+    const wide_work w = wide_work_of<true>(margs, single_norm, lwg, B);
+    if (w.ntok <= 0) return;
+    const wide_role role = wide_role_of(w.blk, lwg, w.ntok);
+    const int token = w.row0 + min(role.tok, w.ntok - 1);
+    if (w.blk.log_bs > 12) input_rht_wide_body<16, XT, f16, 2>(x, x_stride, sv, out, in_features, n_pad, Mp, token, w.blk, s, role);
+    else input_rht_wide_body<8, XT, f16, 2>(x, x_stride, sv, out, in_features, n_pad, Mp, token, w.blk, s, role);
 }
 
 // v = the transformed sums of elements E * tid .. E * tid + E - 1 of block `blk`, row b (before the
@@ -406,16 +435,10 @@ __device__ __forceinline__ void output_wide_load(float (&v)[E], const glqh_ysrc 
 }
 
 template <int E>
-__device__ __forceinline__ void output_wide_transform(float (&v)[E], const rht_slice &blk, float *s, int tid, bool active) {
-    fht_wave<E>(v, blk.log_len, s, tid);
-    reg_gather_runs<E>(v, blk.log_len, s, tid, active);
-}
-
-template <int E>
-__device__ __forceinline__ void output_wide_values(float (&v)[E], const glqh_ysrc &src, int64_t b, int m_pad,
-                                                   const rht_slice &blk, float *s, int tid, bool active, int te) {
-    output_wide_load<E>(v, src, b, m_pad, blk, active, te);
-    output_wide_transform<E>(v, blk, s, tid, active);
+__device__ __forceinline__ void output_wide_transform(float (&v)[E], const rht_slice &blk, float *s, const wide_role &role,
+                                                      bool active) {
+    fht_wave<E>(v, blk.log_len, s + role.lds_off, role.te);
+    reg_gather_runs<E>(v, blk.log_len, s + role.lds_off, role.te, active);
 }
 
 template <int E, typename YT>
@@ -423,10 +446,10 @@ __device__ __forceinline__ void output_rht_wide_body(const glqh_ysrc &src, const
                                                     YT *__restrict__ y, int64_t y_stride, int out_features,
                                                     int m_pad, const rht_slice &blk, float *s, int64_t b,
                                                     const wide_role role) {
-    const int tid = threadIdx.x;
     const bool active = role.active && E * role.te < blk.bs;
     float v[E];
-    output_wide_values<E>(v, src, b, m_pad, blk, s, tid, active, role.te);
+    output_wide_load<E>(v, src, b, m_pad, blk, active, role.te);
+    output_wide_transform<E>(v, blk, s, role, active);
     const int row = blk.off + E * role.te;
     if (active && row < out_features) {
         float f[E];
@@ -449,30 +472,14 @@ __device__ __forceinline__ void output_rht_wide_body(const glqh_ysrc &src, const
 template <typename YT>
 __global__ void __launch_bounds__(REG_THREADS)
 output_rht_wide_kernel(glqh_ysrc src, const f16 *__restrict__ su, YT *__restrict__ y, int64_t y_stride,
-                      int out_features, int m_pad, int B, int n_blocks, glqh_meta_args margs, float single_norm) {
+                      int out_features, int m_pad, int B, int lwg, glqh_meta_args margs,
+                      float single_norm) {
     extern __shared__ float s[];
-    // Workgroup L runs on XCD L % 8 and, inside it, on shader engine (L / 8) % 4: the 64 workgroups that
-    // follow each other take the same block of 64 consecutive rows, so that the large blocks of a row of
-    // several (11008 = 8192 + 2048 + 512 + 256) reach every engine.  Dealt out block by block, a row of four
-    // blocks put every 8192-point block on the same engine of each XCD: 4096 x 11008 127 -> 72 us.
-    const int L = blockIdx.x, xcd = L & 7, member = (L >> 3) & 7, rest = L >> 6, g = rest / n_blocks;
-    const rht_slice blk = rht_slice_of(margs, single_norm, rest % n_blocks);
-    const int r0 = g * 64 + member * 8;                       // first row of the eight workgroups (member, 0..7)
-    if (blk.log_bs <= WIDE_SMALL_LOG) {
-        // one workgroup of every 4096 / bs rows takes them all (the XCDs in turn), the others retire
-        const int lt = 12 - blk.log_bs, T = 1 << lt;
-        if ((r0 & (T - 1)) != 0 || xcd != ((r0 >> lt) & 7) || r0 >= B) return;
-        const int ntok = min(T, B - r0);
-        const wide_role role = wide_role_of(blk, ntok);
-        output_rht_wide_body<8, YT>(src, su, y, y_stride, out_features, m_pad, blk, s,
-                                    (int64_t)r0 + min(role.tok, ntok - 1), role);
-        return;
-    }
-    const int64_t b = (int64_t)r0 + xcd;
-    if (b >= B) return;                                       // uniform over the workgroup
-    const wide_role role = wide_role_of(blk, 1);
-    if (blk.log_bs > 12) output_rht_wide_body<16, YT>(src, su, y, y_stride, out_features, m_pad, blk, s, b, role);
-    else output_rht_wide_body<8, YT>(src, su, y, y_stride, out_features, m_pad, blk, s, b, role);
+    const wide_work w = wide_work_of<false>(margs, single_norm, lwg, B);
+    const wide_role role = wide_role_of(w.blk, lwg, w.ntok);
+    const int64_t b = w.row0 + min(role.tok, w.ntok - 1);
+    if (w.blk.log_bs > 12) output_rht_wide_body<16, YT>(src, su, y, y_stride, out_features, m_pad, w.blk, s, b, role);
+    else output_rht_wide_body<8, YT>(src, su, y, y_stride, out_features, m_pad, w.blk, s, b, role);
 }
 
 template <typename YT, bool PARTS>
@@ -721,16 +728,16 @@ namespace {
 // layout 0: rows of n_pad; 1 / 2: the tile kernels' token-fast blocks with Mp padded tokens (fp16 only)
 int launch_input_rht_wide(const void *x, int x_dtype, int64_t x_stride, const void *sv, void *out, int out_dtype,
                           int layout, int64_t Mp, int64_t B, int64_t in_features, int64_t n_pad,
-                          const glqh_meta_args &margs, int n_blocks, int64_t max_bs, float rsqrt_n,
-                          hipStream_t stream) {
-    const int64_t wgs = 64 * (((B + 7) / 8 + 7) / 8) * n_blocks;
+                          const glqh_meta_args &margs, int64_t max_bs, float rsqrt_n, hipStream_t stream) {
+    const int lwg = wide_log_wg(ilog2(max_bs), B, n_pad);
+    const int64_t wgs = wide_grid<true>(margs.canon, lwg, (int)B);
     GLQH_REQUIRE(wgs <= 2147483647ll, "input_rht: too many blocks");
-    const dim3 wgrid((unsigned)wgs);
-    const size_t lds = std::max(rht_reg_lds_bytes(ilog2(max_bs)), layout == 2 ? WIDE_SMALL_LDS : (size_t)0);
+    const dim3 wgrid((unsigned)wgs), wthreads(1u << (lwg - 3));
+    const size_t lds = wide_lds_bytes(ilog2(max_bs), lwg, layout == 2);
 #define GLQH_INW_LAUNCH(XT, OT, LAYOUT)                                                             \
-    hipLaunchKernelGGL((input_rht_wide_kernel<XT, OT, LAYOUT>), wgrid, dim3(REG_THREADS), lds, stream, \
+    hipLaunchKernelGGL((input_rht_wide_kernel<XT, OT, LAYOUT>), wgrid, wthreads, lds, stream, \
                        (const XT *)x, x_stride, (const f16 *)sv, (OT *)out, (int)in_features,       \
-                       (int)n_pad, (int)Mp, (int)B, n_blocks, margs, rsqrt_n)
+                       (int)n_pad, (int)Mp, (int)B, lwg, margs, rsqrt_n)
 #define GLQH_INW_X(OT, LAYOUT)                                                                      \
     do {                                                                                            \
         if (x_dtype == GLQH_F16) GLQH_INW_LAUNCH(f16, OT, LAYOUT);                                  \
@@ -772,7 +779,7 @@ int glqh_launch_input_rht_blocked(const void *x, int x_dtype, int64_t x_stride, 
     if (max_bs > (1 << WIDE_LOG_MAX) || (n_pad & 31) != 0) return -1;
     if (!aligned16(x) || !aligned16(xb) || !aligned16(sv) || (x_stride * x_size) % 16 != 0) return -1;
     return launch_input_rht_wide(x, x_dtype, x_stride, sv, xb, GLQH_F16, layout, Mp, B, in_features, n_pad, margs,
-                                 (int)n_blocks, max_bs, 0.0f, stream);
+                                 max_bs, 0.0f, stream);
 }
 
 int glqh_launch_input_rht(const void *x, int x_dtype, int64_t x_stride, const void *sv,
@@ -805,7 +812,7 @@ int glqh_launch_input_rht(const void *x, int x_dtype, int64_t x_stride, const vo
     if (rht_wide_ok(B, margs, n_pad, max_bs) && aligned16(x) && aligned16(out) && aligned16(sv) &&
         (x_stride * x_size) % 16 == 0 && (n_pad * o_size) % 16 == 0)
         return launch_input_rht_wide(x, x_dtype, x_stride, sv, out, out_dtype, 0, 0, B, in_features, n_pad, margs,
-                                     (int)n_blocks, max_bs, rsqrt_n, stream);
+                                     max_bs, rsqrt_n, stream);
     const int log_slice = rht_log_slice(B);
     const int spb = rht_slices_per_block(max_bs, log_slice);
     GLQH_REQUIRE(n_blocks * spb <= 2147483647ll, "input_rht: too many slices");
@@ -855,18 +862,18 @@ int glqh_launch_input_rht_blocked_multi(const void *x, int x_dtype, int64_t x_st
         mg.sv[i] = (const f16 *)sv[j];
         mg.out[i] = (f16 *)xb[j];
     }
-    const int64_t wgs = 64 * (((B + 7) / 8 + 7) / 8) * n_blocks;
+    const int lwg = wide_log_wg(ilog2(max_bs), B * n, n_pad);
+    const int64_t wgs = wide_grid<true>(margs.canon, lwg, (int)B);
     if (wgs > 2147483647ll) return -1;
     glqh_range range("input_rht");
-    const dim3 wgrid((unsigned)wgs, (unsigned)n);
-    const size_t lds = std::max(rht_reg_lds_bytes(ilog2(max_bs)), WIDE_SMALL_LDS);
+    const dim3 wgrid((unsigned)wgs, (unsigned)n), wthreads(1u << (lwg - 3));
+    const size_t lds = wide_lds_bytes(ilog2(max_bs), lwg, true);
     if (x_dtype == GLQH_F16)
-        hipLaunchKernelGGL((input_rht_wide_multi_kernel<f16>), wgrid, dim3(REG_THREADS), lds, stream, (const f16 *)x, x_stride,
-                           mg, (int)in_features, (int)n_pad, (int)Mp, (int)B, (int)n_blocks, margs, 0.0f);
+        hipLaunchKernelGGL((input_rht_wide_multi_kernel<f16>), wgrid, wthreads, lds, stream, (const f16 *)x, x_stride,
+                           mg, (int)in_features, (int)n_pad, (int)Mp, (int)B, lwg, margs, 0.0f);
     else
-        hipLaunchKernelGGL((input_rht_wide_multi_kernel<uint16_t>), wgrid, dim3(REG_THREADS), lds, stream,
-                           (const uint16_t *)x, x_stride, mg, (int)in_features, (int)n_pad, (int)Mp, (int)B, (int)n_blocks,
-                           margs, 0.0f);
+        hipLaunchKernelGGL((input_rht_wide_multi_kernel<uint16_t>), wgrid, wthreads, lds, stream,
+                           (const uint16_t *)x, x_stride, mg, (int)in_features, (int)n_pad, (int)Mp, (int)B, lwg, margs, 0.0f);
     GLQH_LAUNCH_CHECK("input_rht group launch");
     return 0;
 }
@@ -913,8 +920,8 @@ int glqh_launch_input_rht_multi(const void *x, int x_dtype, int64_t x_stride, co
 namespace {
 // The whole-block kernels for canonical blocks and many rows; -1 (nothing launched) when they do not apply.
 int launch_output_rht_wide(const glqh_ysrc &src, const void *su, void *y, int y_dtype, int64_t y_stride, int64_t B,
-                           int64_t out_features, int64_t m_pad, const glqh_meta_args &margs, int64_t n_blocks,
-                           int64_t max_bs, float rsqrt_m, hipStream_t stream) {
+                           int64_t out_features, int64_t m_pad, const glqh_meta_args &margs, int64_t max_bs,
+                           float rsqrt_m, hipStream_t stream) {
     const int y_size = y_dtype == GLQH_F32 ? 4 : 2;
     const int pq = src.part_f16 ? 8 : 4;                     // elements per 16 bytes of partial sums
     const bool src_ok = src.nparts == 0
@@ -927,12 +934,12 @@ int launch_output_rht_wide(const glqh_ysrc &src, const void *su, void *y, int y_
     if (!(rht_wide_ok(Bw, margs, m_pad, max_bs) && src_ok && aligned16(y) && aligned16(su) &&
           (y_stride * y_size) % 16 == 0))
         return -1;
-    dim3 wgrid((unsigned)(64 * ((B + 63) / 64) * n_blocks));
-    const size_t lds = rht_reg_lds_bytes(ilog2(max_bs));
+    const int lwg = wide_log_wg(ilog2(max_bs), B, m_pad);
+    const dim3 wgrid((unsigned)wide_grid<false>(margs.canon, lwg, (int)B)), wthreads(1u << (lwg - 3));
+    const size_t lds = wide_lds_bytes(ilog2(max_bs), lwg, false);
 #define GLQH_OUTW_LAUNCH(YT)                                                                        \
-    hipLaunchKernelGGL((output_rht_wide_kernel<YT>), wgrid, dim3(REG_THREADS), lds, stream, src,    \
-                       (const f16 *)su, (YT *)y, y_stride, (int)out_features, (int)m_pad, (int)B, (int)n_blocks, margs, \
-                       rsqrt_m)
+    hipLaunchKernelGGL((output_rht_wide_kernel<YT>), wgrid, wthreads, lds, stream, src,             \
+                       (const f16 *)su, (YT *)y, y_stride, (int)out_features, (int)m_pad, (int)B, lwg, margs, rsqrt_m)
     if (y_dtype == GLQH_F16) GLQH_OUTW_LAUNCH(f16);
     else if (y_dtype == GLQH_BF16) GLQH_OUTW_LAUNCH(uint16_t);
     else GLQH_OUTW_LAUNCH(float);
@@ -952,7 +959,7 @@ int glqh_launch_output_rht_canon_wide(const glqh_ysrc &src, const void *su, void
         if (m_pad & ((int64_t)1 << bit)) blocks[n++] = (int64_t)1 << bit;
     glqh_meta_args margs;
     if (n == 0 || !glqh_fill_meta_args(&margs, n > 1 ? blocks : nullptr, n > 1 ? n : 1, m_pad)) return -1;
-    return launch_output_rht_wide(src, su, y, y_dtype, y_stride, B, out_features, m_pad, margs, n, blocks[0], 0.0f, stream);
+    return launch_output_rht_wide(src, su, y, y_dtype, y_stride, B, out_features, m_pad, margs, blocks[0], 0.0f, stream);
 }
 
 int glqh_launch_output_rht(const glqh_ysrc &src, const void *su, void *y, int y_dtype,
@@ -988,8 +995,8 @@ int glqh_launch_output_rht(const glqh_ysrc &src, const void *su, void *y, int y_
     if (meta_dev && !blocks_host) margs.canon = 0;         // shard-batched call: device meta only
     else if (!glqh_fill_meta_args(&margs, blocks_host, n_blocks, m_pad)) margs.canon = 0;
     {
-        const int rc = launch_output_rht_wide(src, su, y, y_dtype, y_stride, B, out_features, m_pad, margs, n_blocks,
-                                              max_bs, rsqrt_m, stream);
+        const int rc = launch_output_rht_wide(src, su, y, y_dtype, y_stride, B, out_features, m_pad, margs, max_bs,
+                                              rsqrt_m, stream);
         if (rc >= 0) return rc;
     }
     GLQH_REQUIRE(!src.part_f16, "output_rht: fp16 partial sums need the whole-block kernels (more than 32 tokens, "
@@ -1078,8 +1085,7 @@ moe_output_rht_kernel(moe_out_args a, f16 *__restrict__ h, int64_t h_stride, glq
     else output_rht_wide_body<8, f16>(src, su, h, h_stride, a.out_features, a.m_pad, blk, s, slot, role);
 }
 
-// The same for many slots, dealt out like output_rht_wide_kernel's rows: eight slots per workgroup group on the
-// eight XCDs, blocks of up to 512 rows with 4096 / bs slots per workgroup.  A thread's slot decides its signs and
+// The same for many slots, dealt out like output_rht_wide_kernel's rows.  A thread's slot decides its signs and
 // scale; slots of an invalid expert read nothing (their sums were never written) and get zeros.
 template <int E>
 __device__ __forceinline__ void moe_output_wide_row(const moe_out_args &a, f16 *__restrict__ h, int64_t h_stride,
@@ -1100,24 +1106,14 @@ __device__ __forceinline__ void moe_output_wide_row(const moe_out_args &a, f16 *
 }
 
 __global__ void __launch_bounds__(REG_THREADS)
-moe_output_rht_wide_kernel(moe_out_args a, f16 *__restrict__ h, int64_t h_stride, int n_blocks, glqh_meta_args margs) {
+moe_output_rht_wide_kernel(moe_out_args a, f16 *__restrict__ h, int64_t h_stride, int lwg,
+                           glqh_meta_args margs) {
     extern __shared__ float s[];
-    const int L = blockIdx.x, xcd = L & 7, member = (L >> 3) & 7, rest = L >> 6, g = rest / n_blocks;
-    const rht_slice blk = rht_slice_of(margs, 0.0f, rest % n_blocks);
-    const int r0 = g * 64 + member * 8, B = a.n_slots;
-    if (blk.log_bs <= WIDE_SMALL_LOG) {
-        const int lt = 12 - blk.log_bs, T = 1 << lt;
-        if ((r0 & (T - 1)) != 0 || xcd != ((r0 >> lt) & 7) || r0 >= B) return;
-        const int ntok = min(T, B - r0);
-        const wide_role role = wide_role_of(blk, ntok);
-        moe_output_wide_row<8>(a, h, h_stride, blk, s, (int64_t)r0 + min(role.tok, ntok - 1), role);
-        return;
-    }
-    const int64_t b = (int64_t)r0 + xcd;
-    if (b >= B) return;                                       // uniform over the workgroup
-    const wide_role role = wide_role_of(blk, 1);
-    if (blk.log_bs > 12) moe_output_wide_row<16>(a, h, h_stride, blk, s, b, role);
-    else moe_output_wide_row<8>(a, h, h_stride, blk, s, b, role);
+    const wide_work w = wide_work_of<false>(margs, 0.0f, lwg, a.n_slots);
+    const wide_role role = wide_role_of(w.blk, lwg, w.ntok);
+    const int64_t slot = w.row0 + min(role.tok, w.ntok - 1);
+    if (w.blk.log_bs > 12) moe_output_wide_row<16>(a, h, h_stride, w.blk, s, slot, role);
+    else moe_output_wide_row<8>(a, h, h_stride, w.blk, s, slot, role);
 }
 
 __device__ __forceinline__ float moe_gate(float g, int act) {
@@ -1174,7 +1170,7 @@ moe_mid_kernel(moe_mid_args a, f16 *__restrict__ out, glqh_meta_args m13, glqh_m
         if (bi + 1 < a.nb13) request(nxt, rht_slice_of(m13, 0.0f, bi + 1));
         if (bi) __syncthreads();                                 // the previous block is done with the exchange space
         const bool active = 8 * tid < blk.bs;
-        output_wide_transform<8>(cur.v, blk, s, tid, active);
+        output_wide_transform<8>(cur.v, blk, s, role, active);
         const int row = blk.off + 8 * tid;
         if (active && row < a.o.out_features) {
             float w[8];
@@ -1212,7 +1208,6 @@ template <int E, typename YT>
 __device__ __forceinline__ void moe_final_row(const moe_out_args &a, const float *__restrict__ topk_w, int top_k,
                                               YT *__restrict__ out, int64_t out_stride, const rht_slice &blk, float *s,
                                               int64_t token, const wide_role role) {
-    const int tid = threadIdx.x;
     const bool active = role.active && E * role.te < blk.bs;
     const int row = blk.off + E * role.te;
     float acc[E];
@@ -1243,7 +1238,7 @@ __device__ __forceinline__ void moe_final_row(const moe_out_args &a, const float
     for (int c = 0; c < top_k; ++c) {
         if (c + 1 < top_k) request(nxt, c + 1);
         if (c) __syncthreads();                                  // the previous choice is done with the exchange space
-        output_wide_transform<E>(cur.v, blk, s, tid, active && cur.valid);
+        output_wide_transform<E>(cur.v, blk, s, role, active && cur.valid);
         if (active && cur.valid && row < a.out_features) {
 #pragma unroll
             for (int j = 0; j < E; ++j) acc[j] += cur.w * (float)(f16)(cur.v[j] * (blk.norm * cur.f[j]));
@@ -1268,29 +1263,18 @@ __device__ __forceinline__ void moe_final_row(const moe_out_args &a, const float
 template <typename YT, bool BIG>
 __global__ void __launch_bounds__(REG_THREADS)
 moe_final_kernel(moe_out_args a, const float *__restrict__ topk_w, int top_k, int num_tokens, YT *__restrict__ out,
-                 int64_t out_stride, int n_blocks, glqh_meta_args margs) {
+                 int64_t out_stride, int lwg, glqh_meta_args margs) {
     extern __shared__ float s[];
-    const int L = blockIdx.x, xcd = L & 7, member = (L >> 3) & 7, rest = L >> 6, g = rest / n_blocks;
-    const rht_slice blk = rht_slice_of(margs, 0.0f, rest % n_blocks);
-    const int r0 = g * 64 + member * 8, B = num_tokens;
-    if (blk.log_bs <= WIDE_SMALL_LOG) {
-        const int lt = 12 - blk.log_bs, T = 1 << lt;
-        if ((r0 & (T - 1)) != 0 || xcd != ((r0 >> lt) & 7) || r0 >= B) return;
-        const int ntok = min(T, B - r0);
-        const wide_role role = wide_role_of(blk, ntok);
-        moe_final_row<8, YT>(a, topk_w, top_k, out, out_stride, blk, s, (int64_t)r0 + min(role.tok, ntok - 1), role);
-        return;
-    }
-    const int64_t b = (int64_t)r0 + xcd;
-    if (b >= B) return;                                       // uniform over the workgroup
-    const wide_role role = wide_role_of(blk, 1);
+    const wide_work w = wide_work_of<false>(margs, 0.0f, lwg, num_tokens);
+    const wide_role role = wide_role_of(w.blk, lwg, w.ntok);
+    const int64_t b = w.row0 + min(role.tok, w.ntok - 1);
     if constexpr (BIG) {
-        if (blk.bs > 8 * (int)blockDim.x) {
-            moe_final_row<16, YT>(a, topk_w, top_k, out, out_stride, blk, s, b, role);
+        if (w.blk.log_bs > 12) {
+            moe_final_row<16, YT>(a, topk_w, top_k, out, out_stride, w.blk, s, b, role);
             return;
         }
     }
-    moe_final_row<8, YT>(a, topk_w, top_k, out, out_stride, blk, s, b, role);
+    moe_final_row<8, YT>(a, topk_w, top_k, out, out_stride, w.blk, s, b, role);
 }
 
 // out[slot][i] = act(h[slot][i]) * h[slot][intermediate + i]: 0 SiLU, 1 GELU (tanh form), 2 squared ReLU
@@ -1474,12 +1458,15 @@ int glqh_launch_moe_output_rht(const float *part, int ks, int part_f16, int n_sl
     const moe_out_args a = {part, ks, part_f16, n_slots, n_experts, topk_ids, (const f16 *)su_base, wscale_dev,
                             (int)out_features, (int)m_pad};
     const int nb = __builtin_popcountll((unsigned long long)m_pad);
-    if (n_slots >= MOE_OUT_WIDE_MIN)
-        hipLaunchKernelGGL(moe_output_rht_wide_kernel, dim3((unsigned)(64 * ((n_slots + 63) / 64) * nb)), dim3(REG_THREADS),
-                           rht_reg_lds_bytes(ilog2(max_bs)), stream, a, (f16 *)h_f16, h_stride, nb, margs);
-    else
+    if (n_slots >= MOE_OUT_WIDE_MIN) {
+        const int lwg = wide_log_wg(ilog2(max_bs), n_slots, m_pad);
+        hipLaunchKernelGGL(moe_output_rht_wide_kernel, dim3((unsigned)wide_grid<false>(margs.canon, lwg, n_slots)),
+                           dim3(1u << (lwg - 3)), wide_lds_bytes(ilog2(max_bs), lwg, false), stream, a, (f16 *)h_f16,
+                           h_stride, lwg, margs);
+    } else {
         hipLaunchKernelGGL(moe_output_rht_kernel, dim3((unsigned)nb, (unsigned)n_slots), dim3(REG_THREADS),
                            rht_reg_lds_bytes(ilog2(max_bs)), stream, a, (f16 *)h_f16, h_stride, margs);
+    }
     GLQH_LAUNCH_CHECK("routed-expert output_rht launch");
     return 0;
 }
@@ -1576,19 +1563,15 @@ int glqh_launch_moe_final(const float *part, int ks, int part_f16, int num_token
                  "routed experts: unaligned rows");
     const moe_out_args a = {part, ks, part_f16, num_tokens * top_k, n_experts, topk_ids, (const f16 *)su_base, wscale_dev,
                             (int)out_features, (int)m_pad};
-    const int nb = __builtin_popcountll((unsigned long long)m_pad);
-    const dim3 grid((unsigned)(64 * ((num_tokens + 63) / 64) * nb));
-    const size_t lds = rht_reg_lds_bytes(ilog2(max_bs));
-    // rows without small blocks (which take several tokens per workgroup of 512 threads): as many threads as the
-    // largest block has groups of eight elements
     // (sixteen elements per thread on half as many threads: slower, the whole call of 32768 slots x 2048 rows 701 -> 714 us
     // -- the registers of two choices in flight cost occupancy)
-    int threads = REG_THREADS;
-    if ((m_pad & 1023) == 0 && max_bs <= 2048) threads = (int)(max_bs / 8);
+    const int lwg = wide_log_wg(ilog2(max_bs), num_tokens, m_pad);
+    const dim3 grid((unsigned)wide_grid<false>(margs.canon, lwg, num_tokens)), threads(1u << (lwg - 3));
+    const size_t lds = wide_lds_bytes(ilog2(max_bs), lwg, false);
 #define GLQH_MOE_FINAL(YT, BIG)                                                                                  \
-    hipLaunchKernelGGL((moe_final_kernel<YT, BIG>), grid, dim3((unsigned)threads), lds, stream, a, topk_w, top_k, num_tokens, \
-                       (YT *)out, out_stride, nb, margs)
-    const bool big = max_bs > 8 * threads;
+    hipLaunchKernelGGL((moe_final_kernel<YT, BIG>), grid, threads, lds, stream, a, topk_w, top_k, num_tokens,             \
+                       (YT *)out, out_stride, lwg, margs)
+    const bool big = max_bs > (1 << 12);
     if (out_dtype == GLQH_F16) { if (big) GLQH_MOE_FINAL(f16, true); else GLQH_MOE_FINAL(f16, false); }
     else { if (big) GLQH_MOE_FINAL(uint16_t, true); else GLQH_MOE_FINAL(uint16_t, false); }
 #undef GLQH_MOE_FINAL

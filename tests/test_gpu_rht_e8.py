@@ -59,6 +59,25 @@ def test_input_output_rht_blockdiag(ext, n, inf, dtype, B):
         assert rel(y, x.float().numpy()) < 5e-3
 
 
+@pytest.mark.parametrize("B", [65, 67, 1027])   # odd counts; 1027: several tokens of every block per workgroup
+@pytest.mark.parametrize("n", [1024, 1568, 2048, 3616, 4096 + 2048 + 1024 + 8])
+def test_many_token_rows_of_small_and_middle_blocks(ext, n, B):
+    from glq_amd import hadamard as H
+    say("many-token rht", n, B)
+    blocks = O.block_decompose(n)
+    rng = np.random.default_rng(n + B)
+    x = torch.randn(B, n).to(torch.bfloat16)
+    sv = np.where(rng.random(n) < 0.5, -1.0, 1.0).astype(np.float16)
+    out = torch.empty(B, n, dtype=torch.float32, device=DEV)
+    y = torch.empty(B, n, dtype=torch.bfloat16, device=DEV)
+    meta = H.pack_block_meta(blocks).to(DEV)
+    ext.glq_input_rht_blockdiag_cuda(x.to(DEV), t(sv), out, n, n, torch.tensor(blocks), meta)
+    ref = O.block_diag_fht(x.float().numpy() * sv.astype(np.float32)[None], blocks)
+    assert np.allclose(out.cpu().numpy(), ref, rtol=1e-5, atol=2e-5)
+    ext.glq_output_rht_blockdiag_cuda(out, t(sv), y, n, n, torch.tensor(blocks), meta)
+    assert rel(y, x.float().numpy()) < 5e-3          # H(H(x sv)) sv == x
+
+
 def test_rht_refusals(ext):
     x = torch.zeros(1, 96, dtype=torch.float16, device=DEV)
     sv = torch.ones(96, dtype=torch.float16, device=DEV)
