@@ -891,27 +891,28 @@ static int tr_group_many(const void *x, int x_dtype, int64_t x_stride, int64_t B
     for (int i = 0; i < n_shards; ++i) wscales[i] = (float)shards[i].wscale;
     if (glqh_launch_trellis_tile_group(xb, B, packed, R, m_pads, n_shards, n_pad, parts, f16_sums ? 1 : 0, st, wscales)) return 1;
     for (int i = 0; i < n_shards; ++i) {
-        const glqh_trellis_shard &sh = shards[i];
-        glqh_ysrc src = {};
-        src.nparts = 1;
-        src.part = parts[i];
-        src.part_kstride = B * sh.m_pad;
-        src.ksplit = ks;
-        src.part_f16 = f16_sums;
-        src.scale[0] = f16_sums ? 1.0f : (float)sh.wscale;
-        const int64_t ys = y_stride > 0 ? y_stride : sh.out_features;   // y_stride 0: every layer's rows packed
-        int rc = glqh_launch_output_rht_canon_wide(src, sh.su_f16, sh.y, y_dtype, ys, B, sh.out_features, sh.m_pad, st);
-        if (rc > 0) return 1;
-        if (rc < 0) {
-            GLQH_REQUIRE(!f16_sums, "trellis group: layer %d: output blocks not served by the whole-block transform", i);
-            // canonical blocks above 8192 rows: the sliced kernels of the grouped launcher
-            const float *pt[1] = {parts[i]};
-            const void *sus[1] = {sh.su_f16};
-            const float sc[1] = {(float)sh.wscale};
-            void *yl[1] = {sh.y};
-            if (glqh_launch_output_rht_group(pt, sus, yl, sc, &sh.m_pad, &sh.out_features, 1, y_dtype, ys, B, ks, st))
-                return 1;
-        }
+    const void *sus[TR_GROUP_MANY_MAX];
+    void *ys[TR_GROUP_MANY_MAX];
+    int64_t outs[TR_GROUP_MANY_MAX];
+    float scales[TR_GROUP_MANY_MAX];
+    int kss[TR_GROUP_MANY_MAX];
+        sus[i] = shards[i].su_f16;
+        ys[i] = shards[i].y;
+        outs[i] = shards[i].out_features;
+        scales[i] = f16_sums ? 1.0f : wscales[i];
+        kss[i] = ks;
+    }
+    const float *const *pt = parts;
+    const int rc = glqh_launch_output_rht_wide_group(pt, sus, ys, scales, m_pads, outs, kss, n_shards, f16_sums, y_dtype, y_stride, B, st);
+    if (rc >= 0) return rc;
+    // one by one; a layer with canonical blocks above 8192 rows: the sliced kernels of the grouped launcher
+    GLQH_REQUIRE(!f16_sums, "trellis group: output blocks not served by the whole-block transform");
+    for (int i = 0; i < n_shards; ++i) {
+        const int one = glqh_launch_output_rht_wide_group(pt + i, sus + i, ys + i, scales + i, m_pads + i, outs + i, kss + i, 1, 0,
+                                                          y_dtype, y_stride, B, st);
+        if (one > 0 || (one < 0 && glqh_launch_output_rht_group(pt + i, sus + i, ys + i, scales + i, m_pads + i, outs + i, 1,
+                                                                y_dtype, y_stride > 0 ? y_stride : outs[i], B, ks, st)))
+            return 1;
     }
     return 0;
 }
@@ -985,18 +986,15 @@ static int tr_group_transform_blocked(const void *x, int x_dtype, int64_t x_stri
 static int tr_group_finish(const tr_group_ctx &c, int n_shards, int64_t B, int y_dtype, int64_t y_stride, hipStream_t st) {
     if (B > TR_GROUP_SMALL_MAX && c.ks == 0) {
         for (int i = 0; i < n_shards; ++i) {
-            glqh_ysrc src = {};
-            src.nparts = 1;
-            src.part = c.parts[i];
-            src.part_kstride = B * c.m_pads[i];
-            src.ksplit = c.ks_layer[i];
-            src.scale[0] = c.scale[i];
-            if (glqh_launch_output_rht_canon_wide(src, c.su[i], c.ys[i], y_dtype, y_stride, B, c.outs[i], c.m_pads[i], st) != 0) {
-                const float *pt[1] = {c.parts[i]};
-                if (glqh_launch_output_rht_group(pt, &c.su[i], &c.ys[i], &c.scale[i], &c.m_pads[i], &c.outs[i], 1, y_dtype,
-                                                 y_stride, B, c.ks_layer[i], st))
-                    return 1;
-            }
+        const float *const *pt = c.parts;
+        const int rc = glqh_launch_output_rht_wide_group(pt, c.su, c.ys, c.scale, c.m_pads, c.outs, c.ks_layer, n_shards, 0,
+                                                         y_dtype, y_stride, B, st);
+        if (rc >= 0) return rc;
+            const int one = glqh_launch_output_rht_wide_group(pt + i, c.su + i, c.ys + i, c.scale + i, c.m_pads + i, c.outs + i,
+                                                              c.ks_layer + i, 1, 0, y_dtype, y_stride, B, st);
+            if (one > 0 || (one < 0 && glqh_launch_output_rht_group(pt + i, c.su + i, c.ys + i, c.scale + i, c.m_pads + i,
+                                                                    c.outs + i, 1, y_dtype, y_stride, B, c.ks_layer[i], st)))
+                return 1;
         }
         return 0;
     }

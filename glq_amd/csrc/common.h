@@ -149,8 +149,10 @@ int glqh_launch_output_rht(const glqh_ysrc &src, const void *su, void *y, int y_
                            int64_t n_blocks, int64_t max_bs_hint, float rsqrt_m,
                            hipStream_t stream);
 
-int glqh_launch_output_rht_canon_wide(const glqh_ysrc &src, const void *su, void *y, int y_dtype, int64_t y_stride,
-                                      int64_t B, int64_t out_features, int64_t m_pad, hipStream_t stream);
+int glqh_launch_output_rht_wide_group(const float *const part[], const void *const su[], void *const y[],
+                                      const float scale[], const int64_t m_pad[], const int64_t out_features[],
+                                      const int ksplit[], int n, int part_f16, int y_dtype, int64_t y_stride, int64_t B,
+                                      hipStream_t stream);
 
 // out[tok, row] = (accum ? out : 0) + scale * sum_s part[s * kstride + tok * m + row]
 int glqh_launch_reduce_splits(const float *part, int ksplit, int64_t kstride, int64_t B, int64_t m,

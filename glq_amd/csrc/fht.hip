@@ -488,6 +488,44 @@ output_rht_body(const glqh_ysrc &src, const f16 *__restrict__ su, YT *__restrict
                 int out_features, int m_pad, const glqh_block_meta *__restrict__ meta,
                 glqh_meta_args margs, float single_norm, int spb, int log_slice, float *s) {
     const rht_slice blk = rht_get_slice(meta, margs, single_norm, spb, log_slice);
+// The same for the layers of a group (canonical blocks of m_pad, one sum per K slot), one launch: blockIdx.y is the
+// layer.  One launch per layer left the tail of each beside the start of the next, and 4 us per launch where the
+// layers are small: 512 tokens x (14336, 14336) 25 -> 17.5 us, 1130 x (1088, 512, 512) 13.7 -> 6.7.
+struct rht_out_wide_layer {
+    const float *part;
+    const f16 *su;
+    void *y;
+    int64_t y_stride;
+    float scale;
+    int ksplit, m_pad, out_features, nwg;
+};
+struct rht_out_wide_group {
+    rht_out_wide_layer l[GLQH_MAX_GROUP];
+};
+template <typename YT>
+__global__ void __launch_bounds__(REG_THREADS)
+output_rht_wide_group_kernel(rht_out_wide_group g, int part_f16, int B, int lwg) {
+    extern __shared__ float s[];
+    const rht_out_wide_layer &a = g.l[blockIdx.y];
+    if ((int)blockIdx.x >= a.nwg) return;
+    glqh_ysrc src = {};
+    src.part = a.part;
+    src.part_kstride = (int64_t)B * a.m_pad;
+    src.ksplit = a.ksplit;
+    src.part_f16 = part_f16;
+    src.scale[0] = a.scale;
+    src.nparts = 1;
+    glqh_meta_args margs;
+    margs.canon = a.m_pad;
+    const wide_work w = wide_work_of<false>(margs, 0.0f, lwg, B);
+    const wide_role role = wide_role_of(w.blk, lwg, w.ntok);
+    const int64_t b = w.row0 + min(role.tok, w.ntok - 1);
+    if (w.blk.log_bs > 12)
+        output_rht_wide_body<16, YT>(src, a.su, (YT *)a.y, a.y_stride, a.out_features, a.m_pad, w.blk, s, b, role);
+    else
+        output_rht_wide_body<8, YT>(src, a.su, (YT *)a.y, a.y_stride, a.out_features, a.m_pad, w.blk, s, b, role);
+}
+
     if (!blk.live) return;
     const int64_t b = blockIdx.y;
     const int base = blk.off + (blk.r << blk.log_len);
@@ -727,6 +765,9 @@ bool aligned16(const void *p) { return ((uintptr_t)p & 15) == 0; }
 namespace {
 // layout 0: rows of n_pad; 1 / 2: the tile kernels' token-fast blocks with Mp padded tokens (fp16 only)
 int launch_input_rht_wide(const void *x, int x_dtype, int64_t x_stride, const void *sv, void *out, int out_dtype,
+// output side: whole blocks per workgroup also from 32 tokens on when the rows are many (whole linear,
+// 64 tokens: 11008 x 2048 56.9 -> 45.3 us, 14336 x 4096 70.4 -> 61.6; 2048 x 11008 41.5 -> 43.7)
+int64_t wide_rows(int64_t B, int64_t m_pad) { return ((B >= 32 && m_pad >= 8192) || B > 32) ? 65 : B; }
                           int layout, int64_t Mp, int64_t B, int64_t in_features, int64_t n_pad,
                           const glqh_meta_args &margs, int64_t max_bs, float rsqrt_n, hipStream_t stream) {
     const int lwg = wide_log_wg(ilog2(max_bs), B, n_pad);
@@ -928,10 +969,7 @@ int launch_output_rht_wide(const glqh_ysrc &src, const void *su, void *y, int y_
         ? (aligned16(src.direct) && src.stride % 4 == 0)
         : (aligned16(src.part) && m_pad % pq == 0 && src.part_kstride % pq == 0 && src.part_sstride % pq == 0 &&
            (!src.copy_out || (aligned16(src.copy_out) && src.copy_stride % 4 == 0)));
-    // whole blocks per workgroup also from 32 tokens on when the rows are many (whole linear,
-    // 64 tokens: 11008 x 2048 56.9 -> 45.3 us, 14336 x 4096 70.4 -> 61.6; 2048 x 11008 41.5 -> 43.7)
-    const int64_t Bw = ((B >= 32 && m_pad >= 8192) || B > 32) ? 65 : B;
-    if (!(rht_wide_ok(Bw, margs, m_pad, max_bs) && src_ok && aligned16(y) && aligned16(su) &&
+    if (!(rht_wide_ok(wide_rows(B, m_pad), margs, m_pad, max_bs) && src_ok && aligned16(y) && aligned16(su) &&
           (y_stride * y_size) % 16 == 0))
         return -1;
     const int lwg = wide_log_wg(ilog2(max_bs), B, m_pad);
@@ -949,17 +987,50 @@ int launch_output_rht_wide(const glqh_ysrc &src, const void *su, void *y, int y_
 }
 }  // namespace
 
-// Output transform of a layer whose blocks are the canonical ones of m_pad (descending powers of two), many rows:
-// the whole-block kernels.  -1 (nothing launched) when they do not apply (a block above 8192 rows, alignment).
-int glqh_launch_output_rht_canon_wide(const glqh_ysrc &src, const void *su, void *y, int y_dtype, int64_t y_stride,
-                                      int64_t B, int64_t out_features, int64_t m_pad, hipStream_t stream) {
-    int64_t blocks[64];
-    int n = 0;
-    for (int bit = 62; bit >= 0; --bit)
-        if (m_pad & ((int64_t)1 << bit)) blocks[n++] = (int64_t)1 << bit;
-    glqh_meta_args margs;
-    if (n == 0 || !glqh_fill_meta_args(&margs, n > 1 ? blocks : nullptr, n > 1 ? n : 1, m_pad)) return -1;
-    return launch_output_rht_wide(src, su, y, y_dtype, y_stride, B, out_features, m_pad, margs, blocks[0], 0.0f, stream);
+// Output transforms of n layers whose blocks are the canonical ones of their m_pad (descending powers of two), many
+// rows: the whole-block kernel, one launch.  y_stride 0: every layer's rows packed.  -1 (nothing launched) when it
+// does not apply to one of them (a block above 8192 rows, alignment).
+int glqh_launch_output_rht_wide_group(const float *const part[], const void *const su[], void *const y[],
+                                      const float scale[], const int64_t m_pad[], const int64_t out_features[],
+                                      const int ksplit[], int n, int part_f16, int y_dtype, int64_t y_stride, int64_t B,
+                                      hipStream_t stream) {
+    if (n < 1 || n > GLQH_MAX_GROUP || B < 1 || B > 65535) return -1;
+    const int y_size = y_dtype == GLQH_F32 ? 4 : 2;
+    rht_out_wide_group g = {};
+    int64_t points = 0;
+    int log_max = 0;
+    for (int i = 0; i < n; ++i) {
+        const int64_t ys = y_stride > 0 ? y_stride : out_features[i];
+        const int lm = 63 - __builtin_clzll((unsigned long long)m_pad[i]);
+        glqh_meta_args margs;
+        margs.canon = (int)m_pad[i];
+        if (!part[i] || !su[i] || !y[i] || m_pad[i] < 8 || m_pad[i] > 0x7fffffffll || out_features[i] < 1 ||
+            out_features[i] > m_pad[i] || !rht_wide_ok(wide_rows(B, m_pad[i]), margs, m_pad[i], (int64_t)1 << lm) ||
+            !aligned16(part[i]) || !aligned16(su[i]) || !aligned16(y[i]) || (ys * y_size) % 16 != 0)
+            return -1;
+        g.l[i] = {part[i], (const f16 *)su[i], y[i], ys, scale[i], ksplit[i], (int)m_pad[i], (int)out_features[i], 0};
+        points += m_pad[i];
+        log_max = lm > log_max ? lm : log_max;
+    }
+    glqh_range range("output_rht");
+    const int lwg = wide_log_wg(log_max, B, points);
+    int64_t most = 0;
+    for (int i = 0; i < n; ++i) {
+        const int64_t nwg = wide_grid<false>(g.l[i].m_pad, lwg, (int)B);
+        if (nwg > 2147483647ll) return -1;
+        g.l[i].nwg = (int)nwg;
+        most = nwg > most ? nwg : most;
+    }
+    const dim3 grid((unsigned)most, (unsigned)n), threads(1u << (lwg - 3));
+    const size_t lds = wide_lds_bytes(log_max, lwg, false);
+#define GLQH_OUTWG_LAUNCH(YT) \
+    hipLaunchKernelGGL((output_rht_wide_group_kernel<YT>), grid, threads, lds, stream, g, part_f16, (int)B, lwg)
+    if (y_dtype == GLQH_F16) GLQH_OUTWG_LAUNCH(f16);
+    else if (y_dtype == GLQH_BF16) GLQH_OUTWG_LAUNCH(uint16_t);
+    else GLQH_OUTWG_LAUNCH(float);
+#undef GLQH_OUTWG_LAUNCH
+    GLQH_LAUNCH_CHECK("output_rht group launch");
+    return 0;
 }
 
 int glqh_launch_output_rht(const glqh_ysrc &src, const void *su, void *y, int y_dtype,
@@ -1032,8 +1103,7 @@ int glqh_output_rht_wide_eligible(int64_t B, const int64_t *blocks_host, int64_t
         return 0;
     }
     if (!glqh_fill_meta_args(&margs, n_blocks > 1 ? blocks_host : nullptr, n_blocks > 1 ? n_blocks : 1, m_pad)) return 0;
-    const int64_t Bw = ((B >= 32 && m_pad >= 8192) || B > 32) ? 65 : B;
-    return rht_wide_ok(Bw, margs, m_pad, max_bs) ? 1 : 0;
+    return rht_wide_ok(wide_rows(B, m_pad), margs, m_pad, max_bs) ? 1 : 0;
 }
 
 int glqh_rht_init(void) { return 0; }
