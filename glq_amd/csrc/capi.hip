@@ -30,6 +30,7 @@ int glqh_launch_e8_tile(const void *x_f16, void *xb_scratch, int64_t M, const vo
                         int64_t n_pad, float *part, hipStream_t stream, const glqh_e8_folded *fold, int out_f16 = 0,
                         float f16_scale = 1.0f);
 int glqh_e8_tile_f16_sums_ok(int64_t M, int fold, int64_t m_pad);
+int64_t glqh_e8_tile_pad_cols(int64_t n_pad, int fold);
 // Above 16 tokens the weights are decoded once per 128 x 512 tile instead of once per 16 tokens.
 #define GLQH_E8_SMALL_BATCH 16
 static int e8_tile_ks(int64_t m_pad, int64_t n_pad, int64_t B, int nstages, bool fold) {
@@ -87,7 +88,7 @@ int glqh_launch_input_rht_blocked_multi(const void *x, int x_dtype, int64_t x_st
 // input transform straight into a tile kernel's operand layout (fht.hip); -1 = not eligible, nothing launched
 int glqh_launch_input_rht_blocked(const void *x, int x_dtype, int64_t x_stride, const void *sv, void *xb,
                                   int layout, int64_t Mp, int64_t B, int64_t in_features, int64_t n_pad,
-                                  const int64_t *blocks_host, int64_t n_blocks, hipStream_t stream);
+                                  const int64_t *blocks_host, int64_t n_blocks, hipStream_t stream, int64_t pad_cols = 0);
 
 // Plan for activations already in the transformed domain: up to 16 tokens share one pass over
 // the packed stream with K split by shape only; larger batches use the tile kernels, which
@@ -890,12 +891,12 @@ static int tr_group_many(const void *x, int x_dtype, int64_t x_stride, int64_t B
     float wscales[TR_GROUP_MANY_MAX];                          // fp16 sums carry the layer's scale already
     for (int i = 0; i < n_shards; ++i) wscales[i] = (float)shards[i].wscale;
     if (glqh_launch_trellis_tile_group(xb, B, packed, R, m_pads, n_shards, n_pad, parts, f16_sums ? 1 : 0, st, wscales)) return 1;
-    for (int i = 0; i < n_shards; ++i) {
     const void *sus[TR_GROUP_MANY_MAX];
     void *ys[TR_GROUP_MANY_MAX];
     int64_t outs[TR_GROUP_MANY_MAX];
     float scales[TR_GROUP_MANY_MAX];
     int kss[TR_GROUP_MANY_MAX];
+    for (int i = 0; i < n_shards; ++i) {
         sus[i] = shards[i].su_f16;
         ys[i] = shards[i].y;
         outs[i] = shards[i].out_features;
@@ -985,11 +986,11 @@ static int tr_group_transform_blocked(const void *x, int x_dtype, int64_t x_stri
 // layer when their slot counts differ.
 static int tr_group_finish(const tr_group_ctx &c, int n_shards, int64_t B, int y_dtype, int64_t y_stride, hipStream_t st) {
     if (B > TR_GROUP_SMALL_MAX && c.ks == 0) {
-        for (int i = 0; i < n_shards; ++i) {
         const float *const *pt = c.parts;
         const int rc = glqh_launch_output_rht_wide_group(pt, c.su, c.ys, c.scale, c.m_pads, c.outs, c.ks_layer, n_shards, 0,
                                                          y_dtype, y_stride, B, st);
         if (rc >= 0) return rc;
+        for (int i = 0; i < n_shards; ++i) {
             const int one = glqh_launch_output_rht_wide_group(pt + i, c.su + i, c.ys + i, c.scale + i, c.m_pads + i, c.outs + i,
                                                               c.ks_layer + i, 1, 0, y_dtype, y_stride, B, st);
             if (one > 0 || (one < 0 && glqh_launch_output_rht_group(pt + i, c.su + i, c.ys + i, c.scale + i, c.m_pads + i,
@@ -2073,7 +2074,7 @@ extern "C" int glqh_fused_linear_e8_folded(const void *x, int x_dtype, int64_t x
     if (tks > 0)
         blocked = glqh_launch_input_rht_blocked(x, x_dtype, x_stride, sv_f16, (char *)ws + xb + tile_part, 1,
                                                 glqh_e8_tile_padded_tokens(B, sg.n), B, in_features, n_pad,
-                                                blocks_n, n_blocks_n, st);
+                                                blocks_n, n_blocks_n, st, glqh_e8_tile_pad_cols(n_pad, folded != nullptr));
     if (blocked > 0) return 1;
     if (blocked != 0 &&
         glqh_launch_input_rht(x, x_dtype, x_stride, sv_f16, x_rht, GLQH_F16, B, in_features, n_pad,

@@ -644,9 +644,9 @@ e8_tile_small_kernel(const et_args a) {
 }
 
 // (M, n_pad) row-major fp16 -> (n_pad / 32, Mp, 4, 8): 64 tokens x 16 blocks per workgroup through
-// LDS, reads in runs of 256 bytes, writes in runs of 4 KB.
+// LDS, reads in runs of 256 bytes, writes in runs of 4 KB.  Columns n_pad .. width - 1 are written as zeros.
 __global__ void __launch_bounds__(256)
-e8_pack_blocked_kernel(const f16 *__restrict__ x, f16 *__restrict__ xb, int M, int Mp, int n_pad) {
+e8_pack_blocked_kernel(const f16 *__restrict__ x, f16 *__restrict__ xb, int M, int Mp, int n_pad, int width) {
     __shared__ u32x4 tile[16][65];
     const int tok0 = blockIdx.x * 64, kb0 = blockIdx.y * 16, nblk = n_pad >> 3;
     const int t = threadIdx.x;
@@ -654,13 +654,14 @@ e8_pack_blocked_kernel(const f16 *__restrict__ x, f16 *__restrict__ xb, int M, i
     for (int r = 0; r < 4; ++r) {
         const int tl = r * 16 + (t >> 4), kb = t & 15;
         const int tok = min(tok0 + tl, M - 1), b = min(kb0 + kb, nblk - 1);
-        tile[kb][tl] = *(const u32x4 *)(x + (int64_t)tok * n_pad + 8 * b);
+        const u32x4 w = *(const u32x4 *)(x + (int64_t)tok * n_pad + 8 * b);
+        tile[kb][tl] = kb0 + kb < nblk ? w : u32x4{0u, 0u, 0u, 0u};
     }
     __syncthreads();
 #pragma unroll
     for (int r = 0; r < 4; ++r) {                               // group of four blocks r: 64 tokens x 64 bytes contiguous
         const int tl = t >> 2, pos = t & 3, kb = 4 * r + pos;
-        if (tok0 + tl < M && kb0 + kb < nblk)
+        if (tok0 + tl < M && kb0 + kb < (width >> 3))
             *(u32x4 *)(xb + ((((int64_t)(kb0 + kb) >> 2) * Mp + tok0 + tl) * 4 + pos) * 8) = tile[kb][tl];
     }
 }
@@ -820,12 +821,8 @@ int glqh_e8_tile_ksplit(int64_t m_pad, int64_t n_pad, int64_t M, int nstages, in
     return et_make_plan(m_pad, n_pad, M, nstages, &p) ? p.KS : 0;
 }
 
-namespace {
-__global__ void __launch_bounds__(256) et_zero_kernel(u32x4 *__restrict__ p, int64_t n16) {
-    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n16; i += (int64_t)gridDim.x * 256)
-        p[i] = u32x4{0u, 0u, 0u, 0u};
-}
-}  // namespace
+// zero columns that the blocked activations need behind their n_pad ones (folded streams)
+int64_t glqh_e8_tile_pad_cols(int64_t n_pad, int fold) { return fold && n_pad >= 32 && (n_pad & 31) == 0 ? et_width(n_pad) - n_pad : 0; }
 
 // fp16 sums are written by the large tiles of the folded form only
 int glqh_e8_tile_f16_sums_ok(int64_t M, int fold, int64_t m_pad) { return fold && M > ET_SMALL_TOKENS && m_pad % 8 == 0; }
@@ -833,7 +830,8 @@ int glqh_e8_tile_f16_sums_ok(int64_t M, int fold, int64_t m_pad) { return fold &
 // part[(slot * M + token) * m_pad + row] = sum over the slot's columns of x[token, k] * W[row, k],
 // W = cb[q0] + rel[0] * cb2[q1] + rel[1] * cb[q2] + rel[2] * cb[q3] (nstages terms), unscaled (fp32), or
 // times f16_scale and rounded to fp16 with out_f16 (glqh_e8_tile_f16_sums_ok).
-// x_f16 is (M, n_pad) row-major; xb_scratch takes its repacked copy (glqh_e8_tile_xb_bytes).
+// x_f16 is (M, n_pad) row-major; xb_scratch takes its repacked copy (glqh_e8_tile_xb_bytes).  x_f16 NULL: xb_scratch
+// holds the blocked layout already, the zero columns (glqh_e8_tile_pad_cols) included.
 // tokens of the blocked activation layout: M padded to whole workgroup tiles
 int64_t glqh_e8_tile_padded_tokens(int64_t M, int nstages) { return et_padded_tokens(M, nstages); }
 
@@ -849,17 +847,10 @@ int glqh_launch_e8_tile(const void *x_f16, void *xb_scratch, int64_t M, const vo
     if (fold && n_pad >= 32 && (n_pad & 31) == 0) n_pad = et_width(n_pad);
     if (!et_make_plan(m_pad, n_pad, M, nstages, &p))
         return glqh_fail("e8 tile kernel: shape not eligible (n_pad %% 256, or %% 32 on folded streams)");
-    if (n_pad != n_cols) {                                     // zero activations for the padding columns
-        const int64_t Mp = et_padded_tokens(M, nstages);
-        const int64_t n16 = (n_pad - n_cols) / 32 * Mp * 4;    // 16-byte slots of the k-pairs past the row
-        hipLaunchKernelGGL(et_zero_kernel, dim3((unsigned)((n16 + 255) / 256 < 1024 ? (n16 + 255) / 256 : 1024)), dim3(256), 0,
-                           stream, (u32x4 *)((f16 *)xb_scratch + n_cols / 32 * Mp * 32), n16);
-        GLQH_LAUNCH_CHECK("e8 tile padding launch");
-    }
-    if (x_f16) {                                               // NULL: xb_scratch already holds the blocked layout
-        hipLaunchKernelGGL(e8_pack_blocked_kernel, dim3((unsigned)((M + 63) / 64), (unsigned)((n_cols / 8 + 15) / 16)),
+    if (x_f16) {
+        hipLaunchKernelGGL(e8_pack_blocked_kernel, dim3((unsigned)((M + 63) / 64), (unsigned)((n_pad / 8 + 15) / 16)),
                            dim3(256), 0, stream, (const f16 *)x_f16, (f16 *)xb_scratch, (int)M,
-                           (int)et_padded_tokens(M, nstages), (int)n_cols);
+                           (int)et_padded_tokens(M, nstages), (int)n_cols, (int)n_pad);
         GLQH_LAUNCH_CHECK("e8 pack launch");
     }
     et_args a;

@@ -349,11 +349,17 @@ __device__ __forceinline__ void input_rht_wide_body(const XT *__restrict__ x, in
 template <typename XT, typename OT, int LAYOUT>
 __global__ void __launch_bounds__(REG_THREADS)
 input_rht_wide_kernel(const XT *__restrict__ x, int64_t x_stride, const f16 *__restrict__ sv,
-                     OT *__restrict__ out, int in_features, int n_pad, int Mp, int B, int lwg,
+                     OT *__restrict__ out, int in_features, int n_pad, int Mp, int B, int lwg, int pad_cols,
                      glqh_meta_args margs, float single_norm) {
     extern __shared__ float s[];
     const wide_work w = wide_work_of<true>(margs, single_norm, lwg, B);
     if (w.ntok <= 0) return;
+    if (LAYOUT == 1 && w.blk.off == 0) {                     // zero columns behind the row (a launch of their own: 4 us)
+        for (int i = threadIdx.x; i < (pad_cols >> 3) * w.ntok; i += blockDim.x) {
+            const int tok = (i >> 2) % w.ntok, kp = (n_pad >> 5) + (i >> 2) / w.ntok;
+            *(u32x4 *)(out + (((int64_t)kp * Mp + w.row0 + tok) * 4 + (i & 3)) * 8) = u32x4{0u, 0u, 0u, 0u};
+        }
+    }
     const wide_role role = wide_role_of(w.blk, lwg, w.ntok);
     const int token = w.row0 + min(role.tok, w.ntok - 1);
     if (w.blk.log_bs > 12)
@@ -482,12 +488,6 @@ output_rht_wide_kernel(glqh_ysrc src, const f16 *__restrict__ su, YT *__restrict
     else output_rht_wide_body<8, YT>(src, su, y, y_stride, out_features, m_pad, w.blk, s, b, role);
 }
 
-template <typename YT, bool PARTS>
-__device__ __forceinline__ void
-output_rht_body(const glqh_ysrc &src, const f16 *__restrict__ su, YT *__restrict__ y, int64_t y_stride,
-                int out_features, int m_pad, const glqh_block_meta *__restrict__ meta,
-                glqh_meta_args margs, float single_norm, int spb, int log_slice, float *s) {
-    const rht_slice blk = rht_get_slice(meta, margs, single_norm, spb, log_slice);
 // The same for the layers of a group (canonical blocks of m_pad, one sum per K slot), one launch: blockIdx.y is the
 // layer.  One launch per layer left the tail of each beside the start of the next, and 4 us per launch where the
 // layers are small: 512 tokens x (14336, 14336) 25 -> 17.5 us, 1130 x (1088, 512, 512) 13.7 -> 6.7.
@@ -526,6 +526,12 @@ output_rht_wide_group_kernel(rht_out_wide_group g, int part_f16, int B, int lwg)
         output_rht_wide_body<8, YT>(src, a.su, (YT *)a.y, a.y_stride, a.out_features, a.m_pad, w.blk, s, b, role);
 }
 
+template <typename YT, bool PARTS>
+__device__ __forceinline__ void
+output_rht_body(const glqh_ysrc &src, const f16 *__restrict__ su, YT *__restrict__ y, int64_t y_stride,
+                int out_features, int m_pad, const glqh_block_meta *__restrict__ meta,
+                glqh_meta_args margs, float single_norm, int spb, int log_slice, float *s) {
+    const rht_slice blk = rht_get_slice(meta, margs, single_norm, spb, log_slice);
     if (!blk.live) return;
     const int64_t b = blockIdx.y;
     const int base = blk.off + (blk.r << blk.log_len);
@@ -759,17 +765,18 @@ bool rht_wide_ok(int64_t B, const glqh_meta_args &margs, int64_t total, int64_t 
     if (B <= 64 || margs.canon == 0 || max_bs > (1 << WIDE_LOG_MAX)) return false;
     return (total & 7) == 0;                                 // smallest block >= 8
 }
+// output side: whole blocks per workgroup also from 32 tokens on when the rows are many (whole linear,
+// 64 tokens: 11008 x 2048 56.9 -> 45.3 us, 14336 x 4096 70.4 -> 61.6; 2048 x 11008 41.5 -> 43.7)
+int64_t wide_rows(int64_t B, int64_t m_pad) { return ((B >= 32 && m_pad >= 8192) || B > 32) ? 65 : B; }
 bool aligned16(const void *p) { return ((uintptr_t)p & 15) == 0; }
 }  // namespace
 
 namespace {
-// layout 0: rows of n_pad; 1 / 2: the tile kernels' token-fast blocks with Mp padded tokens (fp16 only)
+// layout 0: rows of n_pad; 1 / 2: the tile kernels' token-fast blocks with Mp padded tokens (fp16 only), layout 1
+// followed by pad_cols columns of zeros (a multiple of 32)
 int launch_input_rht_wide(const void *x, int x_dtype, int64_t x_stride, const void *sv, void *out, int out_dtype,
-// output side: whole blocks per workgroup also from 32 tokens on when the rows are many (whole linear,
-// 64 tokens: 11008 x 2048 56.9 -> 45.3 us, 14336 x 4096 70.4 -> 61.6; 2048 x 11008 41.5 -> 43.7)
-int64_t wide_rows(int64_t B, int64_t m_pad) { return ((B >= 32 && m_pad >= 8192) || B > 32) ? 65 : B; }
                           int layout, int64_t Mp, int64_t B, int64_t in_features, int64_t n_pad,
-                          const glqh_meta_args &margs, int64_t max_bs, float rsqrt_n, hipStream_t stream) {
+                          const glqh_meta_args &margs, int64_t max_bs, float rsqrt_n, hipStream_t stream, int pad_cols = 0) {
     const int lwg = wide_log_wg(ilog2(max_bs), B, n_pad);
     const int64_t wgs = wide_grid<true>(margs.canon, lwg, (int)B);
     GLQH_REQUIRE(wgs <= 2147483647ll, "input_rht: too many blocks");
@@ -778,7 +785,7 @@ int64_t wide_rows(int64_t B, int64_t m_pad) { return ((B >= 32 && m_pad >= 8192)
 #define GLQH_INW_LAUNCH(XT, OT, LAYOUT)                                                             \
     hipLaunchKernelGGL((input_rht_wide_kernel<XT, OT, LAYOUT>), wgrid, wthreads, lds, stream, \
                        (const XT *)x, x_stride, (const f16 *)sv, (OT *)out, (int)in_features,       \
-                       (int)n_pad, (int)Mp, (int)B, lwg, margs, rsqrt_n)
+                       (int)n_pad, (int)Mp, (int)B, lwg, pad_cols, margs, rsqrt_n)
 #define GLQH_INW_X(OT, LAYOUT)                                                                      \
     do {                                                                                            \
         if (x_dtype == GLQH_F16) GLQH_INW_LAUNCH(f16, OT, LAYOUT);                                  \
@@ -796,13 +803,13 @@ int64_t wide_rows(int64_t B, int64_t m_pad) { return ((B >= 32 && m_pad >= 8192)
 }
 }  // namespace
 
-// The input transform written straight into a tile kernel's operand layout (layout 1: E8, 2:
-// trellis; Mp padded tokens).  Returns -1 without launching when the call does not qualify
+// The input transform written straight into a tile kernel's operand layout (layout 1: E8, with pad_cols columns of
+// zeros behind the row; 2: trellis; Mp padded tokens).  Returns -1 without launching when the call does not qualify
 // (non-canonical blocks, blocks over 8192 points, unaligned rows): the caller then transforms into
 // rows and lets the tile launcher repack.
 int glqh_launch_input_rht_blocked(const void *x, int x_dtype, int64_t x_stride, const void *sv, void *xb,
                                   int layout, int64_t Mp, int64_t B, int64_t in_features, int64_t n_pad,
-                                  const int64_t *blocks_host, int64_t n_blocks, hipStream_t stream) {
+                                  const int64_t *blocks_host, int64_t n_blocks, hipStream_t stream, int64_t pad_cols) {
     glqh_range range("input_rht");
     if (!x || !sv || !xb || B < 1 || in_features < 1 || in_features > n_pad) return -1;
     if (x_dtype != GLQH_F16 && x_dtype != GLQH_BF16 && x_dtype != GLQH_F32) return -1;
@@ -820,7 +827,7 @@ int glqh_launch_input_rht_blocked(const void *x, int x_dtype, int64_t x_stride, 
     if (max_bs > (1 << WIDE_LOG_MAX) || (n_pad & 31) != 0) return -1;
     if (!aligned16(x) || !aligned16(xb) || !aligned16(sv) || (x_stride * x_size) % 16 != 0) return -1;
     return launch_input_rht_wide(x, x_dtype, x_stride, sv, xb, GLQH_F16, layout, Mp, B, in_features, n_pad, margs,
-                                 max_bs, 0.0f, stream);
+                                 max_bs, 0.0f, stream, (int)pad_cols);
 }
 
 int glqh_launch_input_rht(const void *x, int x_dtype, int64_t x_stride, const void *sv,
