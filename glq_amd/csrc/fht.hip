@@ -130,8 +130,10 @@ template <> __device__ __forceinline__ void store8<f16>(f16 *p, const float *f) 
 template <> __device__ __forceinline__ void store8<uint16_t>(uint16_t *p, const float *f) {  // bf16
     u32x4 w;
 #pragma unroll
-    for (int e = 0; e < 4; ++e)
-        w[e] = (uint32_t)f32_to_bf16_bits(f[2 * e]) | ((uint32_t)f32_to_bf16_bits(f[2 * e + 1]) << 16);
+    for (int e = 0; e < 4; ++e) {
+        const bf16x2 b = {(__bf16)f[2 * e], (__bf16)f[2 * e + 1]};
+        w[e] = __builtin_bit_cast(uint32_t, b);
+    }
     *(u32x4 *)p = w;
 }
 
