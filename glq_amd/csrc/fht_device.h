@@ -133,7 +133,7 @@ struct lds_writeback {                                   // last pass: results s
 // them is paid in full (4+ cycles each, nothing to overlap with).  Here thread tid holds E
 // consecutive elements, E*tid .. E*tid+E-1, of a 2^log_n-point vector in registers:
 // log2(E) butterfly levels stay inside the thread, up to six run across the lanes of the
-// wave (DPP quad permutes, ds_swizzle, ds_bpermute: no LDS storage, no barrier), and up to
+// wave (DPP and the permlane swaps: vector instructions only), and up to
 // log2(E) more, across waves, take one exchange through LDS.  log2(E) <= log_n <=
 // 6 + 2*log2(E); threads tid >= n/E carry don't-care values but must make the call.
 //
@@ -156,26 +156,86 @@ __device__ __forceinline__ int fht_wave_index(int log_n, int tid, int q) {
     return log_n > LE + 6 ? tid + (q << (log_n - LE)) : tid * E + q;
 }
 
-// value of the lane whose number differs in bit K
+// Butterfly levels across lanes.  Bits 0..3: v += sgn * v[lane ^ (1 << K)] with sgn = -1 in the upper lane of a pair,
+// one v_fmac_f32_dpp per element (bit 2, which no single DPP control reaches, mirrors each eight lanes first and then
+// each four: lane ^ 7 ^ 3).  In the upper lanes that is own - partner where the transform has partner - own: the
+// signs of a lane's levels multiply and are set right at the end (fht_lane_signs), which is exact.  Bits 4 and 5:
+// v_permlane16_swap / v_permlane32_swap exchange the halves of two registers, after which both lanes' values of one
+// element are in one lane; the butterfly, and the same swap back.  (ds_swizzle and ds_bpermute for bits 2..5 put
+// four trips through the LDS pipe into the chain of every short transform and kept that pipe busy in the long ones:
+// 65-launch decode step 621 -> 608 us, 4096 tokens x (4096 -> 14336) 502 -> 496.)
+// DPP and the swaps read a register no sooner than two wait states after a vector instruction wrote it.  The
+// compiler neither adds them inside inline assembly nor sees what that writes: hence the s_nop before every group,
+// and after those whose results a compiler-made DPP move (bit 2) or swap (bit 4) reads.
+#define GLQH_DPP_FMAC4(S0, S1, S2, S3, SGN, CTRL)                                                        \
+    "s_nop 1\n\tv_fmac_f32_dpp %0, " S0 ", " SGN " " CTRL " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t" \
+    "v_fmac_f32_dpp %1, " S1 ", " SGN " " CTRL " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"             \
+    "v_fmac_f32_dpp %2, " S2 ", " SGN " " CTRL " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"             \
+    "v_fmac_f32_dpp %3, " S3 ", " SGN " " CTRL " row_mask:0xf bank_mask:0xf bound_ctrl:1"
+#define GLQH_DPP_OUTS "+&v"(v[0]), "+&v"(v[1]), "+&v"(v[2]), "+&v"(v[3])
 template <int K>
-__device__ __forceinline__ float fht_lane_partner(float v, int swap32_addr) {
-    const int b = __builtin_bit_cast(int, v);
-    int o;
-    if constexpr (K == 0) o = __builtin_amdgcn_mov_dpp(b, 0xB1, 0xF, 0xF, true);        // quad_perm [1,0,3,2]
-    else if constexpr (K == 1) o = __builtin_amdgcn_mov_dpp(b, 0x4E, 0xF, 0xF, true);   // quad_perm [2,3,0,1]
-    else if constexpr (K < 5) o = __builtin_amdgcn_ds_swizzle(b, ((1 << K) << 10) | 0x1F);  // xor mask, 32-lane groups
-    else o = __builtin_amdgcn_ds_bpermute(swap32_addr, b);
-    return __builtin_bit_cast(float, o);
+__device__ __forceinline__ void fht_dpp_fmac4(float *v, const float *o, float sgn) {
+    if constexpr (K == 0)
+        asm(GLQH_DPP_FMAC4("%0", "%1", "%2", "%3", "%4", "quad_perm:[1,0,3,2]") : GLQH_DPP_OUTS : "v"(sgn));
+    else if constexpr (K == 1)
+        asm(GLQH_DPP_FMAC4("%0", "%1", "%2", "%3", "%4", "quad_perm:[2,3,0,1]") "\n\ts_nop 1" : GLQH_DPP_OUTS : "v"(sgn));
+    else if constexpr (K == 2)
+        asm(GLQH_DPP_FMAC4("%4", "%5", "%6", "%7", "%8", "quad_perm:[3,2,1,0]") : GLQH_DPP_OUTS
+            : "v"(o[0]), "v"(o[1]), "v"(o[2]), "v"(o[3]), "v"(sgn));
+    else
+        asm(GLQH_DPP_FMAC4("%0", "%1", "%2", "%3", "%4", "row_ror:8") "\n\ts_nop 1" : GLQH_DPP_OUTS : "v"(sgn));
+}
+#undef GLQH_DPP_OUTS
+#undef GLQH_DPP_FMAC4
+
+__device__ __forceinline__ float fht_half_mirror(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x141, 0xF, 0xF, true));
+}
+
+// lower / upper halves (K = 5: of the wave, K = 4: of each 32 lanes) of b and a trade places
+template <int K>
+__device__ __forceinline__ void fht_half_swap(float &a, float &b) {
+    const uint32_t ua = __builtin_bit_cast(uint32_t, a), ub = __builtin_bit_cast(uint32_t, b);
+    const auto r = K == 5 ? __builtin_amdgcn_permlane32_swap(ua, ub, false, false)
+                          : __builtin_amdgcn_permlane16_swap(ua, ub, false, false);
+    const uint32_t r0 = r[0], r1 = r[1];
+    a = __builtin_bit_cast(float, r0);
+    b = __builtin_bit_cast(float, r1);
 }
 
 template <int K, int E>
-__device__ __forceinline__ void fht_lane_level(float (&v)[E], int lane, int swap32_addr) {
-    const float sgn = ((lane >> K) & 1) ? -1.0f : 1.0f;      // upper element of the pair: partner - own
-    float o[E];
+__device__ __forceinline__ void fht_lane_level(float (&v)[E], int lane) {
+    if constexpr (K < 4) {
+        const float sgn = ((lane >> K) & 1) ? -1.0f : 1.0f;
+        if constexpr (K == 2) {
+            float o[E];
 #pragma unroll
-    for (int j = 0; j < E; ++j) o[j] = fht_lane_partner<K>(v[j], swap32_addr);
+            for (int j = 0; j < E; ++j) o[j] = fht_half_mirror(v[j]);
 #pragma unroll
-    for (int j = 0; j < E; ++j) v[j] = __builtin_fmaf(v[j], sgn, o[j]);   // exact: one rounding, like the add
+            for (int j = 0; j < E; j += 4) fht_dpp_fmac4<K>(v + j, o + j, sgn);
+        } else {
+#pragma unroll
+            for (int j = 0; j < E; j += 4) fht_dpp_fmac4<K>(v + j, v + j, sgn);
+        }
+    } else {
+#pragma unroll
+        for (int j = 0; j < E; j += 2) {
+            fht_half_swap<K>(v[j], v[j + 1]);
+            const float a = v[j], b = v[j + 1];
+            v[j] = a + b;
+            v[j + 1] = a - b;
+            fht_half_swap<K>(v[j], v[j + 1]);
+        }
+    }
+}
+
+// the signs that the levels over lane bits 0 .. min(lane_bits, 4) - 1 left open
+template <int E>
+__device__ __forceinline__ void fht_lane_signs(float (&v)[E], int lane, int lane_bits) {
+    const int mask = (1 << min(lane_bits, 4)) - 1;
+    const uint32_t flip = (uint32_t)__builtin_popcount(lane & mask) << 31;
+#pragma unroll
+    for (int j = 0; j < E; ++j) v[j] = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, v[j]) ^ flip);
 }
 
 template <int E, bool ALWAYS_SYNC = false, bool LDS_ONLY = false>
@@ -194,13 +254,13 @@ __device__ __forceinline__ void fht_wave(float (&v)[E], int log_n, float *xchg, 
     }
     const int lane = tid & 63;
     const int lane_bits = min(log_n - LE, 6);                // uniform
-    const int swap32_addr = (lane ^ 32) << 2;
-    if (lane_bits > 0) fht_lane_level<0>(v, lane, swap32_addr);
-    if (lane_bits > 1) fht_lane_level<1>(v, lane, swap32_addr);
-    if (lane_bits > 2) fht_lane_level<2>(v, lane, swap32_addr);
-    if (lane_bits > 3) fht_lane_level<3>(v, lane, swap32_addr);
-    if (lane_bits > 4) fht_lane_level<4>(v, lane, swap32_addr);
-    if (lane_bits > 5) fht_lane_level<5>(v, lane, swap32_addr);
+    if (lane_bits > 0) fht_lane_level<0>(v, lane);
+    if (lane_bits > 1) fht_lane_level<1>(v, lane);
+    if (lane_bits > 2) fht_lane_level<2>(v, lane);
+    if (lane_bits > 3) fht_lane_level<3>(v, lane);
+    if (lane_bits > 4) fht_lane_level<4>(v, lane);
+    if (lane_bits > 5) fht_lane_level<5>(v, lane);
+    fht_lane_signs(v, lane, lane_bits);
     if (log_n <= LE + 6) {
         if constexpr (ALWAYS_SYNC) fht_barrier<LDS_ONLY>();   // the barrier the longer transforms take
         return;
