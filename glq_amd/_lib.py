@@ -63,6 +63,7 @@ SIGNATURES = {
     "glqh_e8_fold_indices": (c_int, [c_vp, c_i64, c_i64, c_vp, c_i64, c_vp, c_vp, c_vp]),
     "glqh_e8_folded_count": (c_i64, [c_i64, c_i64]),
     "glqh_e8_fold_eligible": (c_int, [c_i64, c_i64, c_i64]),
+    "glqh_e8_few_eligible": (c_int, [c_i64, c_i64, c_i64]),
     "glqh_e8_decompress": (
         c_int, [c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_i64, c_dbl, c_dbl, c_dbl, c_i64, c_i64,
                 c_vp, c_vp]),

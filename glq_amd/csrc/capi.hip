@@ -30,6 +30,11 @@ int glqh_launch_e8_tile(const void *x_f16, void *xb_scratch, int64_t M, const vo
                         int64_t n_pad, float *part, hipStream_t stream, const glqh_e8_folded *fold, int out_f16 = 0,
                         float f16_scale = 1.0f);
 int glqh_e8_tile_f16_sums_ok(int64_t M, int fold, int64_t m_pad);
+int glqh_e8_few_init(void);
+int glqh_e8_few_ksplit(int64_t m_pad, int64_t n_pad, int64_t B, int nstages, int fused);
+int glqh_launch_e8_few(const void *x, int x_dtype, int64_t x_stride, const void *sv, int64_t B, int64_t in_features,
+                       const glqh_e8_folded *fold, int nstages, int64_t m_pad, int64_t n_pad, const float *pscale, float *part,
+                       int direct, hipStream_t stream);
 int64_t glqh_e8_tile_pad_cols(int64_t n_pad, int fold);
 // Above 16 tokens the weights are decoded once per 128 x 512 tile instead of once per 16 tokens.
 #define GLQH_E8_SMALL_BATCH 16
@@ -242,7 +247,7 @@ extern "C" int glqh_init(void) {
             return;
         }
         g_cus = prop.multiProcessorCount;
-        g_init_rc = glqh_rht_init() || glqh_e8_init() || glqh_e8_tile_init() || glqh_trellis_init() || glqh_trellis_tile_init() || glqh_trellis_mma_init() || glqh_viterbi_init();
+        g_init_rc = glqh_rht_init() || glqh_e8_init() || glqh_e8_tile_init() || glqh_e8_few_init() || glqh_trellis_init() || glqh_trellis_tile_init() || glqh_trellis_mma_init() || glqh_viterbi_init();
     });
     if (g_init_rc != 0 && g_err[0] == 0) glqh_fail("libglq_hip initialisation failed earlier");
     if (g_init_rc != 0) return g_init_rc;
@@ -1834,12 +1839,16 @@ extern "C" int glqh_e8_fold_table(const uint32_t *table, int64_t n_entries, void
     return 0;
 }
 
-int glqh_e8_mma_ksplit(int64_t m_pad, int64_t n_pad, int64_t B, int64_t n1, int fold);
+int glqh_e8_mma_ksplit(int64_t m_pad, int64_t n_pad, int64_t B, int64_t n1);
 
 extern "C" int glqh_e8_fold_eligible(int64_t m_pad, int64_t n_pad, int64_t B) {
     if (glqh_init() != 0 || m_pad < 1 || n_pad < 8 || (n_pad & 7) || B < 1) return 0;
     if (B > GLQH_E8_SMALL_BATCH) return glqh_e8_tile_ksplit(m_pad, n_pad, B, 1, 1) > 0 ? 1 : 0;   // the many-token kernel
-    return glqh_e8_mma_ksplit(m_pad, n_pad, B, 65536, 1) > 0 ? 1 : 0;
+    return glqh_e8_mma_ksplit(m_pad, n_pad, B, 65536) > 0 && glqh_e8_few_ksplit(m_pad, n_pad, B, 1, 0) > 0 ? 1 : 0;
+}
+
+extern "C" int glqh_e8_few_eligible(int64_t m_pad, int64_t n_pad, int64_t B) {
+    return glqh_init() == 0 && glqh_e8_few_ksplit(m_pad, n_pad, B, 1, 0) > 0 ? 1 : 0;
 }
 
 extern "C" int64_t glqh_e8_folded_count(int64_t rows, int64_t cols) {
@@ -1908,11 +1917,12 @@ static size_t e8_part_bytes(int64_t m_pad, int64_t n_pad, int64_t B) {
     if (tks > 0)                                                 // + the repacked activations
         tile = align256((size_t)tks * B * m_pad * sizeof(float)) + align256(glqh_e8_tile_xb_bytes(n_pad, B));
     if (tks > 0 && e8_tile_ks(m_pad, n_pad, B, 1, false) > 0) return tile;
-    int ks = glqh_e8_pick_ksplit(m_pad, n_pad, B, 0);
-    const int ksf = glqh_e8_pick_ksplit(m_pad, n_pad, B, 1);       // on folded streams
-    if (ksf > ks) ks = ksf;
+    const int ks = glqh_e8_pick_ksplit(m_pad, n_pad, B);
     const size_t plain = align256((size_t)ks * 4 * B * m_pad * sizeof(float));
-    return plain > tile ? plain : tile;
+    // folded streams: the few-token kernel, with and without its own transform
+    const int kf = std::max(glqh_e8_few_ksplit(m_pad, n_pad, B, 1, 0), glqh_e8_few_ksplit(m_pad, n_pad, B, 1, 1));
+    const size_t few = align256((size_t)kf * 4 * B * m_pad * sizeof(float));
+    return std::max(std::max(plain, tile), few);
 }
 
 extern "C" size_t glqh_e8_matmul_workspace_bytes(int64_t m_pad, int64_t n_pad, int64_t B) {
@@ -1956,17 +1966,17 @@ extern "C" int glqh_e8_dequant_matmul_folded(const void *x_f16, int64_t B, const
             return 1;
         return glqh_launch_reduce_splits(part, tks, B * m_pad, B, m_pad, (float)wscale, out, m_pad, 0, st);
     }
-    // folded streams with K inside the workgroups: the kernel writes the finished sums itself
-    if (folded && glqh_e8_mma_direct_ok(m_pad, n_pad, B, sg.n))
-        return glqh_launch_e8_partial(x_f16, B, sg.q, sg.n, table1, table2 ? table2 : table1, table2 ? n_entries2 : 65536,
-                                      m_pad, n_pad, 1, out, st, sg.scale, folded, 1);
-    const int ks = glqh_e8_pick_ksplit(m_pad, n_pad, B, folded != nullptr);
+    const int few = folded ? glqh_e8_few_ksplit(m_pad, n_pad, B, sg.n, 0) : 0;
+    if (few == 1)                                              // K inside the workgroups: the kernel writes the finished sums
+        return glqh_launch_e8_few(x_f16, GLQH_F16, n_pad, nullptr, B, n_pad, folded, sg.n, m_pad, n_pad, sg.scale, out, 1, st);
+    const int ks = few > 0 ? few : glqh_e8_pick_ksplit(m_pad, n_pad, B);
     const size_t need = (size_t)ks * sg.n * B * m_pad * sizeof(float);
     GLQH_REQUIRE(ws && ws_bytes >= need, "e8 matmul: workspace of %zu bytes needed, got %zu", need, ws_bytes);
     // every stage's partial sums are written already multiplied by that stage's scale: one
     // reduction over ks * stages plain slots instead of one launch per stage
-    if (glqh_launch_e8_partial(x_f16, B, sg.q, sg.n, table1, table2 ? table2 : table1,
-                               table2 ? n_entries2 : 65536, m_pad, n_pad, ks, part, st, sg.scale, folded))
+    if (few > 0 ? glqh_launch_e8_few(x_f16, GLQH_F16, n_pad, nullptr, B, n_pad, folded, sg.n, m_pad, n_pad, sg.scale, part, 0, st)
+                : glqh_launch_e8_partial(x_f16, B, sg.q, sg.n, table1, table2 ? table2 : table1, table2 ? n_entries2 : 65536,
+                                         m_pad, n_pad, ks, part, st, sg.scale))
         return 1;
     return glqh_launch_reduce_splits(part, ks * sg.n, B * m_pad, B, m_pad, 1.0f, out, m_pad, 0, st);
 }
@@ -2060,7 +2070,8 @@ extern "C" int glqh_fused_linear_e8_folded(const void *x, int x_dtype, int64_t x
     GLQH_REQUIRE(in_features <= n_pad && out_features <= m_pad, "fused e8 linear: features exceed padded dims");
     const size_t xb = align256((size_t)B * n_pad * sizeof(f16));
     const int tks = e8_tile_ks(m_pad, n_pad, B, sg.n, folded != nullptr);
-    const int ks = tks > 0 ? tks : glqh_e8_pick_ksplit(m_pad, n_pad, B, folded != nullptr);
+    const int few_rows = folded && tks <= 0 ? glqh_e8_few_ksplit(m_pad, n_pad, B, sg.n, 0) : 0;   // on transformed rows
+    const int ks = tks > 0 ? tks : few_rows > 0 ? few_rows : glqh_e8_pick_ksplit(m_pad, n_pad, B);
     const size_t tile_part = align256((size_t)ks * B * m_pad * sizeof(float));
     const size_t need = tks > 0 ? xb + tile_part + glqh_e8_tile_xb_bytes(n_pad, B)
                                 : xb + (size_t)ks * sg.n * B * m_pad * sizeof(float);
@@ -2069,6 +2080,26 @@ extern "C" int glqh_fused_linear_e8_folded(const void *x, int x_dtype, int64_t x
     hipStream_t st = (hipStream_t)stream;
     f16 *x_rht = (f16 *)ws;
     float *part = (float *)((char *)ws + xb);
+    // Up to 16 tokens on folded streams, rows short enough for every workgroup to transform them itself, canonical
+    // blocks on both sides: one launch from the activations to the sums of all stages, one finishing launch.
+    if (folded && tks <= 0 && (x_dtype == GLQH_F16 || x_dtype == GLQH_BF16) && ((uintptr_t)x & 15) == 0 &&
+        ((uintptr_t)sv_f16 & 15) == 0 && (x_stride & 7) == 0 && in_features >= 2 && in_features % 2 == 0) {
+        glqh_meta_args cn, cm;
+        const int few = glqh_e8_few_ksplit(m_pad, n_pad, B, sg.n, 1);
+        if (few > 0 && ws_bytes >= xb + (size_t)few * sg.n * B * m_pad * sizeof(float) &&
+            glqh_fill_meta_args(&cn, n_blocks_n > 1 ? blocks_n : nullptr, n_blocks_n > 1 ? n_blocks_n : 1, n_pad) &&
+            cn.canon == n_pad &&
+            glqh_fill_meta_args(&cm, n_blocks_m > 1 ? blocks_m : nullptr, n_blocks_m > 1 ? n_blocks_m : 1, m_pad) &&
+            cm.canon == m_pad) {
+            if (glqh_launch_e8_few(x, x_dtype, x_stride, sv_f16, B, in_features, folded, sg.n, m_pad, n_pad, sg.scale, part, 0, st))
+                return 1;
+            const float *pt[1] = {part};
+            const void *sus[1] = {su_f16};
+            void *ys[1] = {y};
+            const float sc[1] = {1.0f};
+            return glqh_launch_output_rht_group(pt, sus, ys, sc, &m_pad, &out_features, 1, y_dtype, y_stride, B, few * sg.n, st);
+        }
+    }
     // tile kernel: the transform writes the kernel's blocked operand layout itself where it can
     int blocked = -1;
     if (tks > 0)
@@ -2113,9 +2144,10 @@ extern "C" int glqh_fused_linear_e8_folded(const void *x, int x_dtype, int64_t x
     const bool canon_out = B <= 16 && glqh_fill_meta_args(&canon_m, n_blocks_m > 1 ? blocks_m : nullptr,
                                                           n_blocks_m > 1 ? n_blocks_m : 1, m_pad) &&
                            canon_m.canon == m_pad;
-    if (glqh_launch_e8_partial(x_rht, B, sg.q, sg.n, table1, table2 ? table2 : table1,
-                               table2 ? n_entries2 : 65536, m_pad, n_pad, ks, part, st, canon_out ? sg.scale : nullptr,
-                               folded))
+    const float *scales = canon_out ? sg.scale : nullptr;
+    if (few_rows > 0 ? glqh_launch_e8_few(x_rht, GLQH_F16, n_pad, nullptr, B, n_pad, folded, sg.n, m_pad, n_pad, scales, part, 0, st)
+                     : glqh_launch_e8_partial(x_rht, B, sg.q, sg.n, table1, table2 ? table2 : table1, table2 ? n_entries2 : 65536,
+                                              m_pad, n_pad, ks, part, st, scales))
         return 1;
     if (canon_out) {
         const float *pt[1] = {part};

@@ -30,7 +30,7 @@
 // are served by that XCD's L2.  K is split into slots only while the tiles alone would leave CUs
 // idle; partial sums [slot][token][row] are combined in slot order by the consumer.
 //
-// FOLD: the same kernel on the folded streams (glqh_e8_fold_table / glqh_e8_fold_indices, e8_mma.hip):
+// FOLD: the same kernel on the folded streams (glqh_e8_fold_table / glqh_e8_fold_indices, e8_few.hip):
 // an index is two 11-bit half-codeword numbers, the table of half codewords as finished fp16 values
 // (at most 16 KB per table) sits in LDS whole, and a lookup is two 8-byte LDS reads whose result is
 // the operand: no table word comes from L2, nothing is expanded, 128 KB of table fill per workgroup

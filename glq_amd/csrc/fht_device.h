@@ -204,9 +204,9 @@ __device__ __forceinline__ void fht_half_swap(float &a, float &b) {
 }
 
 template <int K, int E>
-__device__ __forceinline__ void fht_lane_level(float (&v)[E], int lane) {
+__device__ __forceinline__ void fht_lane_level(float (&v)[E], int lane, bool on = true) {   // on, per lane: only below bit 4
     if constexpr (K < 4) {
-        const float sgn = ((lane >> K) & 1) ? -1.0f : 1.0f;
+        const float sgn = on ? (((lane >> K) & 1) ? -1.0f : 1.0f) : 0.0f;
         if constexpr (K == 2) {
             float o[E];
 #pragma unroll
@@ -238,9 +238,8 @@ __device__ __forceinline__ void fht_lane_signs(float (&v)[E], int lane, int lane
     for (int j = 0; j < E; ++j) v[j] = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, v[j]) ^ flip);
 }
 
-template <int E, bool ALWAYS_SYNC = false, bool LDS_ONLY = false>
-__device__ __forceinline__ void fht_wave(float (&v)[E], int log_n, float *xchg, int tid) {
-    constexpr int LE = fht_wave_log<E>::v;
+template <int E>
+__device__ __forceinline__ void fht_thread_levels(float (&v)[E]) {
 #pragma unroll
     for (int h = 1; h < E; h <<= 1) {
 #pragma unroll
@@ -252,6 +251,30 @@ __device__ __forceinline__ void fht_wave(float (&v)[E], int log_n, float *xchg, 
             }
         }
     }
+}
+
+// Blocks of 16..512 points side by side in one wave, sixteen elements per lane: log_bs is the lane's own block's.
+// Blocks are aligned to their size, so a lane's partner at a level below its block's size is in the same block; a
+// lane whose block is smaller takes no part in the level.
+__device__ __forceinline__ void fht_lanes_ragged(float (&v)[16], int log_bs, int lane) {
+    fht_thread_levels<16>(v);
+    fht_lane_level<0>(v, lane, log_bs > 4);
+    fht_lane_level<1>(v, lane, log_bs > 5);
+    fht_lane_level<2>(v, lane, log_bs > 6);
+    fht_lane_level<3>(v, lane, log_bs > 7);
+    fht_lane_signs(v, lane, log_bs - 4);
+    float o[16];
+#pragma unroll
+    for (int j = 0; j < 16; ++j) o[j] = v[j];
+    fht_lane_level<4>(o, lane);
+#pragma unroll
+    for (int j = 0; j < 16; ++j) v[j] = log_bs > 8 ? o[j] : v[j];
+}
+
+template <int E, bool ALWAYS_SYNC = false, bool LDS_ONLY = false>
+__device__ __forceinline__ void fht_wave(float (&v)[E], int log_n, float *xchg, int tid) {
+    constexpr int LE = fht_wave_log<E>::v;
+    fht_thread_levels<E>(v);
     const int lane = tid & 63;
     const int lane_bits = min(log_n - LE, 6);                // uniform
     if (lane_bits > 0) fht_lane_level<0>(v, lane);

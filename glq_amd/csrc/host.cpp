@@ -36,6 +36,7 @@ struct {
     decltype(&glqh_fused_linear_e8_workspace_bytes) e8_ws;
     decltype(&glqh_fused_linear_e8_folded) e8;
     decltype(&glqh_e8_fold_eligible) fold_eligible;
+    decltype(&glqh_e8_few_eligible) few_eligible;
     decltype(&glqh_fused_linear_trellis_group_workspace_bytes) group_ws;
     decltype(&glqh_fused_linear_trellis_3inst_group) group;
     decltype(&glqh_fused_linear_trellis_3inst_group_rvq2) group_rvq2;
@@ -325,8 +326,10 @@ PyObject *forward_shell(const plan_t &p, PyObject *self, PyObject *buffers, cons
     glqh_e8_folded f = {};
     std::vector<c10::intrusive_ptr<c10::TensorImpl>> keep;
     bool folded = false;
-    if (!(B > fold_most || (B > 16 && p.n_pad % 32 != 0)) && setting(s_fold, 0) && L.fold_eligible(p.m_pad, p.n_pad, B)) {
-        NONE_UNLESS(p.folded);
+    bool wants = !(B > fold_most || (B > 16 && p.n_pad % 32 != 0)) && setting(s_fold, 0);
+    if (wants && L.fold_eligible(p.m_pad, p.n_pad, B)) NONE_UNLESS(p.folded);
+    else wants = wants && p.folded && L.few_eligible(p.m_pad, p.n_pad, B);   // a small layer: on its indices if not prepared
+    if (wants) {
         for (int s = 0; s < p.stages; ++s) {
             auto lo = p.lo[s].lock(), hi = p.hi[s].lock();
             NONE_UNLESS(lo && hi);
@@ -661,6 +664,7 @@ PyObject *py_bind(PyObject *, PyObject *args) {
     sym(L.e8_ws, "glqh_fused_linear_e8_workspace_bytes");
     sym(L.e8, "glqh_fused_linear_e8_folded");
     sym(L.fold_eligible, "glqh_e8_fold_eligible");
+    sym(L.few_eligible, "glqh_e8_few_eligible");
     sym(L.group_ws, "glqh_fused_linear_trellis_group_workspace_bytes");
     sym(L.group, "glqh_fused_linear_trellis_3inst_group");
     sym(L.group_rvq2, "glqh_fused_linear_trellis_3inst_group_rvq2");

@@ -873,7 +873,8 @@ def e8_prepare(qidxs, codebook, qidxs2=None, codebook2=None, qidxs3=None, qidxs4
     stages += [(q, t1) for q in (qidxs3, qidxs4) if not _absent(q)]
     M, nblk = qidxs.shape
     lib = _lib.load()
-    if not E8_FOLD or not any(lib.glqh_e8_fold_eligible(M, nblk * 8, B) for B in (1, 4, 16, 17, 64)):
+    if not E8_FOLD or not (any(lib.glqh_e8_fold_eligible(M, nblk * 8, B) for B in (1, 4, 16, 17, 64)) or
+                           lib.glqh_e8_few_eligible(M, nblk * 8, 1)):
         return 0
     need = sum(3 * lib.glqh_e8_folded_count(q.shape[0], q.shape[1]) for q, t in stages
                if _FOLD_STREAMS.get(q, (t.data_ptr(),)) is None)
@@ -898,15 +899,17 @@ def e8_release(*qidxs):
             del _FOLD_STREAMS._d[k]
 
 
-def _e8_folded(B, qidxs, t1, q2, t2, q3, q4):
+def _e8_folded(B, qidxs, t1, q2, t2, q3, q4, linear=False):
     """The folded streams of a layer as the C struct (and what must stay alive during the call), or
     (None, None) when the call would not read them or `e8_prepare` has not made them.  Looks up
-    only: nothing is allocated, launched or synchronized here, so it is safe under stream capture."""
+    only: nothing is allocated, launched or synchronized here, so it is safe under stream capture.
+    linear: the call is the fused linear, which reads them at a few tokens of a small layer too."""
     M, nblk = qidxs.shape
     if not E8_FOLD or not qidxs.is_contiguous():
         return None, None
     lib = _lib.load()
-    if not lib.glqh_e8_fold_eligible(M, nblk * 8, B):
+    wanted = lib.glqh_e8_fold_eligible(M, nblk * 8, B)
+    if not wanted and not (linear and lib.glqh_e8_few_eligible(M, nblk * 8, B)):
         return None, None
     stages = [(qidxs, t1)] + ([(q2, t2)] if q2 is not None else []) + [(q, t1) for q in (q3, q4) if q is not None]
     keep, f = [], _E8Folded()
@@ -914,7 +917,7 @@ def _e8_folded(B, qidxs, t1, q2, t2, q3, q4):
         hit = _FOLD_STREAMS.get(q, (t.data_ptr(),))
         if hit is None or hit[0]() is not t:
             key = (qidxs.data_ptr(), tuple(qidxs.shape))
-            if key not in _fold_warned and len(_fold_warned) < 4096:
+            if wanted and key not in _fold_warned and len(_fold_warned) < 4096:
                 _fold_warned.add(key)
                 warnings.warn(f"E8 layer {M}x{nblk * 8} was not prepared (glq_amd.ext.e8_prepare / "
                               "E8RHTLinear.prepare): it runs on its indices, which is slower at 1-4096 "
@@ -1094,7 +1097,7 @@ def _fused_e8(x, sv, su, qidxs, codebook, wscale, in_features, out_features, n_p
     folded, keep = None, None
     if not _e8_dense_route(B, n_pad, True):
         with torch.cuda.device(x.device):
-            folded, keep = _e8_folded(B, qidxs, t1, q2, t2, q3, q4)
+            folded, keep = _e8_folded(B, qidxs, t1, q2, t2, q3, q4, linear=True)
     if _e8_dense_route(B, n_pad, folded is not None):
         x_rht = torch.empty((B, int(n_pad)), dtype=torch.float16, device=x.device)
         glq_input_rht_blockdiag_cuda(x, sv, x_rht, in_features, n_pad, blocks_n, bn_meta)

@@ -338,9 +338,14 @@ typedef struct {
 int glqh_e8_fold_table(const uint32_t *table, int64_t n_entries, void *halves_out, int64_t capacity,
                        uint32_t *map_out, int64_t *n_halves_out, void *stream);
 
-/* 1 when a product of this shape and token count reads the folded streams (the LDS-table
+/* 1 when a product of this shape and token count reads the folded streams (the few-token
  * kernel or, above 16 tokens, the tile kernel serves it), 0 when they would go unused. */
 int glqh_e8_fold_eligible(int64_t m_pad, int64_t n_pad, int64_t B);
+
+/* 1 when the fused linear of this shape and token count reads them as well: up to 16 tokens
+ * whose input transform and product share a launch (small layers, which
+ * glqh_e8_fold_eligible leaves to the gather kernel, included). */
+int glqh_e8_few_eligible(int64_t m_pad, int64_t n_pad, int64_t B);
 
 /* Entries of a folded stream of a (rows, cols) index matrix: rows padded to 16, cols to 32. */
 int64_t glqh_e8_folded_count(int64_t rows, int64_t cols);

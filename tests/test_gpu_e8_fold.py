@@ -254,6 +254,35 @@ def test_fused_linear_at_many_tokens_on_folded_streams(ext, m, n, B, stages):
         assert rel(y, want) < TOL
 
 
+# rows that a workgroup transforms itself: one segment and its small blocks, blocks of 1024, 2048, 4096 and 8192, more
+# segments than waves, a row past the last and one with an odd end (rows transformed by a launch of their own), K slots
+@pytest.mark.parametrize("m,n,inf,B", [(40, 64, 64, 1), (1000, 960, 960, 5), (96, 1024, 1022, 4), (2080, 1088, 1080, 16),
+                                       (512, 3136, 3136, 2), (4128, 7232, 7232, 1), (264, 12352, 12350, 1),
+                                       (128, 12352, 12352, 3), (256, 2048, 2047, 2), (5000, 4096, 4096, 3)])
+@pytest.mark.parametrize("stages,dtype", [(1, torch.bfloat16), (2, torch.float16), (3, torch.bfloat16), (4, torch.float16)])
+def test_fused_linear_at_few_tokens_on_folded_streams(ext, m, n, inf, B, stages, dtype):
+    say("e8 folded fused linear, few tokens", m, n, inf, B, stages, dtype)
+    from glq_amd import hadamard as H
+    q = [t(a) for a in _indices(m, n, stages, m + n + stages)]
+    su, sv = O.rht_signs(m, n, 42)
+    bn, bm = O.block_decompose(n), O.block_decompose(m)
+    cb = e8_table_f16()
+    inv = [1 / 3.0, 1 / 9.0, 1 / 27.0]
+    extra = []
+    for s in range(1, 4):
+        extra += [q[s] if s < stages else None, cb if s < stages else None, inv[s - 1] if s < stages else 0.0]
+    qs = q + [None] * (4 - stages)
+    assert ext.e8_prepare(qs[0], cb, qs[1], cb, qs[2], qs[3]) > 0
+    x = torch.randn(B, inf, generator=torch.Generator().manual_seed(B)).to(dtype).to(DEV)
+    y = ext.glq_fused_linear_block_diag_cuda(
+        x, t(sv.astype(np.float16)), t(su.astype(np.float16)), q[0], cb, 0.02, inf, m, n, m, torch.tensor(bn), torch.tensor(bm),
+        H.pack_block_meta(bn).to(DEV), H.pack_block_meta(bm).to(DEV), *extra, out_dtype=dtype)
+    W = sum(O.e8_table()[q[s].cpu().numpy().view(np.uint16).astype(np.int64)].reshape(m, n) * (3.0 ** -s)
+            for s in range(stages)).astype(np.float32) * np.float32(0.02)
+    want = O.linear_forward_rht(x.float().cpu().numpy(), W, su.astype(np.float32), sv.astype(np.float32), bn, bm, inf, m)
+    assert rel(y, want) < TOL, rel(y, want)
+
+
 def test_fresh_views_of_the_indices_hit_the_one_fold(ext):
     """A caller that passes a new view object of the same index memory on every call (a shard of a
     stacked tensor, `.view()`) finds the one folded copy: nothing is folded again, nothing dropped."""
