@@ -293,7 +293,7 @@ __device__ __forceinline__ void tr_tile_body(const tt_args &a, const tt_group &g
                 for (int d = ds0; d < ds1; ++d) {
                     const tr_record<R> p3 = load_rec(d + 3);
                     const tr_record<RB> p3b = load_rec2(d + 3);
-                    emit_both(p1, p1b, abuf + (((d - ds0) & 1) ^ 1) * TT_BUF);
+                    if (d + 1 < ds1) emit_both(p1, p1b, abuf + (((d - ds0) & 1) ^ 1) * TT_BUF);   // uniform
                     tt_barrier();
                     p1 = p2;
                     p2 = p3;
@@ -627,7 +627,7 @@ tr_tile_small_kernel(const tt_args a) {
 #pragma unroll
                         for (int kk = 0; kk < PF; ++kk) ring[kk] = frag(kk);
                         load_b(b[(dd + 3) & 3], d0 + dd + 3);
-                        emit(rc[dd], rcb[dd], wr + dd * TT_BUF);   // operands of the next group (unused after the last)
+                        if (d0 + 4 + dd < ds1) emit(rc[dd], rcb[dd], wr + dd * TT_BUF);   // operands of the next group, uniform
                         if (d0 + dd < ds1) {                    // uniform: a slot need not be whole groups
 #pragma unroll
                             for (int kk = 0; kk < NK; ++kk) {
