@@ -293,7 +293,8 @@ __device__ __forceinline__ void tr_tile_body(const tt_args &a, const tt_group &g
                 for (int d = ds0; d < ds1; ++d) {
                     const tr_record<R> p3 = load_rec(d + 3);
                     const tr_record<RB> p3b = load_rec2(d + 3);
-                    if (d + 1 < ds1) emit_both(p1, p1b, abuf + (((d - ds0) & 1) ^ 1) * TT_BUF);   // uniform
+                    // (the last one goes unused; a branch around it: 96 tokens and more 1-3 % slower)
+                    emit_both(p1, p1b, abuf + (((d - ds0) & 1) ^ 1) * TT_BUF);
                     tt_barrier();
                     p1 = p2;
                     p2 = p3;
@@ -525,7 +526,8 @@ tr_moe_tiles_kernel(const int *__restrict__ offs, int n_experts, int tile_tok, i
 // Here: TG = 2 or 4 token groups of 16 NTW tokens; wave w takes token group w % TG and the operands
 // w / TG + (8 / TG) j, j < TG, of each half-step -- 2 TG operand reads and 2 TG NTW MFMAs per wave and step,
 // every product computed once.  The operands of a whole group of four steps (256 columns) are decoded into one
-// of two 64 KB buffers while the previous group is multiplied out of the other; decoding is as above (wave w:
+// of two 64 KB buffers while the previous group is multiplied out of the other, none past the K slot (a slot of 11
+// steps decoded 16: 2048 x 11008 at 37 tokens, 4 + 2 bits, the kernel 21.6 -> 18.8 us); decoding is as above (wave w:
 // block pair w >> 2, k-pair (w >> 1) & 1, m-tile w & 1).  Same K slots and order of summation as above.
 constexpr size_t TT_SMALL_LDS = (size_t)8 * TT_BUF * 16;       // 128 KB
 
