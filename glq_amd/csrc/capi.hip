@@ -77,10 +77,11 @@ int glqh_launch_trellis_tile(const void *x_f16, void *xb_scratch, int64_t M, con
                              hipStream_t stream, int out_f16 = 0, const void *packed2 = nullptr, int R2 = 0,
                              float rs2 = 0.0f);
 int64_t glqh_trellis_tile_padded_tokens(int64_t M);
-int glqh_trellis_tile_group_ksplit(const int64_t *m, int n_layers, int64_t k, int64_t M);
+int glqh_trellis_tile_group_ksplit(const int64_t *m, int n_layers, int64_t k, int64_t M, int two_stage);
 int glqh_launch_trellis_tile_group(const void *const xb[], int64_t M, const void *const packed[], int R,
                                    const int64_t m[], int n_layers, int64_t k, float *const out[], int out_f16,
-                                   hipStream_t stream, const float f16_scale[] = nullptr);
+                                   hipStream_t stream, const float f16_scale[] = nullptr,
+                                   const void *const packed2[] = nullptr, int R2 = 0, const float rs2[] = nullptr);
 int glqh_launch_trellis_pack(const void *x_f16, void *xb, int64_t M, int64_t k, hipStream_t stream);
 int64_t glqh_e8_tile_padded_tokens(int64_t M, int nstages);
 // several sign vectors on the same few rows in one launch (fht.hip); -1 = not eligible, nothing launched
@@ -742,7 +743,8 @@ extern "C" size_t glqh_fused_linear_trellis_group_workspace_bytes(int64_t B, int
         // them, and the partial sums of the largest K split a group of these rows can get (fp32)
         glqh_init();
         const int64_t one[1] = {TT_GROUP_ROWS_FLOOR};
-        const int ks = glqh_trellis_tile_group_ksplit(one, 1, n_pad, B);
+        const int ks = std::max(glqh_trellis_tile_group_ksplit(one, 1, n_pad, B, 0),
+                                glqh_trellis_tile_group_ksplit(one, 1, n_pad, B, 1));   // (single-stage and stacked layers)
         return (size_t)n_shards * (256 + align256(glqh_trellis_tile_xb_bytes(n_pad, B))) +
                align256((size_t)B * n_pad * sizeof(f16)) + align256((size_t)ks * B * total_m_pad * sizeof(float));
     }
@@ -791,14 +793,63 @@ extern "C" size_t glqh_fused_linear_trellis_group_workspace_bytes(int64_t B, int
     return (size_t)n_shards * 256 + (stacked > most ? stacked : most);
 }
 
-// Decode launch of a group: checks, K plan, partial-sum layout in ws.  On return parts[i] holds
-// layer i's [slot][token][row] fp32 partial sums and *ks_out the slot count.
+// the second stage of stacked layer i of a group (first: it sets the group's rate *R2)
+static int tr_check_stage2(const glqh_trellis_stage2 &s2, int i, int R1, int64_t m_pad, int64_t n_pad, bool first, int *R2) {
+    GLQH_REQUIRE(s2.packed2, "trellis two-stage group: null pointer in shard %d", i);
+    GLQH_REQUIRE(s2.inv_resid_scale2 != 0.0, "trellis two-stage group: shard %d has a second stream but inv_resid_scale2 = 0", i);
+    int Ri;
+    if (tr_bits_from_packed(s2.packed2_cols, 1, &Ri) || tr_check_shape(m_pad, n_pad, s2.packed2_rows)) return 1;
+    GLQH_REQUIRE(R1 == 4, "trellis two-stage group: first stages of 4 bits/weight, shard %d has %d", i, R1);
+    GLQH_REQUIRE(first || Ri == *R2, "trellis two-stage group: second stages of %d and %d bits/weight cannot share a launch", *R2, Ri);
+    *R2 = Ri;
+    return 0;
+}
+
+// x under every distinct sign vector of a group in the tile kernels' blocked layout, buffer j at ws + j * xbb (more than
+// 16 tokens): one launch for all of them where the whole-block transform serves the call, else one per sign vector,
+// by rows (x_rows) and repacked where it cannot write the layout.  xb_of[i] = layer i's buffer.
+static int tr_group_blocked(const void *x, int x_dtype, int64_t x_stride, int64_t B, const void *const sv[], int n_shards,
+                            const int64_t *blocks_n, int64_t n_blocks_n, const glqh_block_meta *bn_meta_dev,
+                            int64_t in_features, int64_t n_pad, void *ws, size_t xbb, f16 *x_rows, const void *xb_of[],
+                            hipStream_t st) {
+    const void *dsv[GLQH_MAX_SHARDS];
+    void *dout[GLQH_MAX_SHARDS];
+    int nd = 0;
+    for (int i = 0; i < n_shards; ++i) {
+        int j = 0;
+        while (j < nd && dsv[j] != sv[i]) ++j;
+        if (j == nd) {
+            dsv[nd] = sv[i];
+            dout[nd] = (char *)ws + (size_t)nd * xbb;
+            ++nd;
+        }
+        xb_of[i] = dout[j];
+    }
+    const int64_t Mp = glqh_trellis_tile_padded_tokens(B);
+    if (nd > 1) {
+        const int rc = glqh_launch_input_rht_blocked_multi(x, x_dtype, x_stride, dsv, dout, nd, Mp, B, in_features, n_pad, blocks_n,
+                                                           n_blocks_n, st);
+        if (rc >= 0) return rc;
+    }
+    for (int j = 0; j < nd; ++j) {
+        const int rc = glqh_launch_input_rht_blocked(x, x_dtype, x_stride, dsv[j], dout[j], 2, Mp, B, in_features, n_pad, blocks_n,
+                                                     n_blocks_n, st);
+        if (rc > 0) return 1;
+        if (rc < 0 && (glqh_launch_input_rht(x, x_dtype, x_stride, dsv[j], x_rows, GLQH_F16, B, in_features, n_pad, bn_meta_dev,
+                                             blocks_n, n_blocks_n, 0.0f, st) ||
+                       glqh_launch_trellis_pack(x_rows, dout[j], B, n_pad, st)))
+            return 1;
+    }
+    return 0;
+}
+
 // Layers that read the same activations, many tokens (prefill of fused q/k/v, gate/up): per distinct sign vector
 // one input transform straight into the tile kernel's layout, ONE launch of the tile kernel over the row tiles of
 // all layers (small layers do not fill the chip one by one: 512 tokens x (2048 -> 2048 + 512 + 512): 16 + 4 + 4
 // row tiles), then every layer's output transform from fp16 sums.
+// stage2: stacked layers (first stages of 4 bits/weight, second stages of one rate), both streams into one operand.
 static int tr_group_many(const void *x, int x_dtype, int64_t x_stride, int64_t B, const glqh_trellis_shard *shards,
-                         int n_shards, const int64_t *blocks_n, int64_t n_blocks_n, const glqh_block_meta *bn_meta_dev,
+                         const glqh_trellis_stage2 *stage2, int n_shards, const int64_t *blocks_n, int64_t n_blocks_n, const glqh_block_meta *bn_meta_dev,
                          int64_t in_features, int64_t n_pad, int y_dtype, int64_t y_stride, void *ws, size_t ws_bytes,
                          hipStream_t st) {
     GLQH_REQUIRE(x && shards && ws, "trellis group: null pointer");
@@ -809,9 +860,10 @@ static int tr_group_many(const void *x, int x_dtype, int64_t x_stride, int64_t B
     GLQH_REQUIRE(in_features >= 1 && in_features <= n_pad && n_pad % 64 == 0, "trellis group: bad in_features / n_pad");
     GLQH_REQUIRE(n_blocks_n > 1 ? (bn_meta_dev != nullptr && blocks_n != nullptr) : (n_pad & (n_pad - 1)) == 0,
                  "trellis group: input block sizes missing");
-    int R = 0;
+    int R = 0, R2 = 0;
     int64_t total = 0, m_pads[TR_GROUP_MANY_MAX];
-    const void *packed[TR_GROUP_MANY_MAX];
+    const void *packed[TR_GROUP_MANY_MAX], *packed2[TR_GROUP_MANY_MAX], *sv[TR_GROUP_MANY_MAX];
+    float rs2[TR_GROUP_MANY_MAX];
     for (int i = 0; i < n_shards; ++i) {
         const glqh_trellis_shard &sh = shards[i];
         GLQH_REQUIRE(sh.sv_f16 && sh.packed && sh.su_f16 && sh.y, "trellis group: null pointer in shard %d", i);
@@ -819,12 +871,18 @@ static int tr_group_many(const void *x, int x_dtype, int64_t x_stride, int64_t B
         if (tr_bits_from_packed(sh.packed_cols, 0, &Ri) || tr_check_shape(sh.m_pad, n_pad, sh.packed_rows)) return 1;
         GLQH_REQUIRE(i == 0 || Ri == R, "trellis group: shards of %d and %d bits/weight cannot share a launch", R, Ri);
         R = Ri;
+        if (stage2) {
+            if (tr_check_stage2(stage2[i], i, R, sh.m_pad, n_pad, i == 0, &R2)) return 1;
+            packed2[i] = stage2[i].packed2;
+            rs2[i] = (float)stage2[i].inv_resid_scale2;
+        }
+        sv[i] = sh.sv_f16;
         GLQH_REQUIRE(sh.out_features >= 1 && sh.out_features <= sh.m_pad, "trellis group: out_features exceeds m_pad");
         m_pads[i] = sh.m_pad;
         packed[i] = sh.packed;
         total += sh.m_pad;
     }
-    const int ks = glqh_trellis_tile_group_ksplit(m_pads, n_shards, n_pad, B);
+    const int ks = glqh_trellis_tile_group_ksplit(m_pads, n_shards, n_pad, B, stage2 != nullptr);
     const size_t xb_one = align256(glqh_trellis_tile_xb_bytes(n_pad, B));
     const size_t rows = align256((size_t)B * n_pad * sizeof(f16));
     const size_t need = (size_t)n_shards * xb_one + rows + align256((size_t)ks * B * total * sizeof(float));
@@ -832,7 +890,6 @@ static int tr_group_many(const void *x, int x_dtype, int64_t x_stride, int64_t B
     char *base = (char *)ws;
     f16 *x_rows = (f16 *)(base + (size_t)n_shards * xb_one);
     char *pbase = base + (size_t)n_shards * xb_one + rows;
-    const int64_t Mp = glqh_trellis_tile_padded_tokens(B);
     const void *xb[TR_GROUP_MANY_MAX];
     float *parts[TR_GROUP_MANY_MAX];
     // fp16 sums need the whole-block output kernels for every layer (canonical blocks of at most 8192 rows)
@@ -848,54 +905,18 @@ static int tr_group_many(const void *x, int x_dtype, int64_t x_stride, int64_t B
     }
     const size_t esz = f16_sums ? sizeof(f16) : sizeof(float);
     size_t poff = 0;
-    // all distinct sign vectors in one transform launch where it applies (layer i's activations in buffer i)
-    int all = -1;
-    {
-        const void *dsv[GLQH_MAX_SHARDS];
-        void *dout[GLQH_MAX_SHARDS];
-        int nd = 0;
-        for (int i = 0; i < n_shards; ++i) {
-            int j = 0;
-            while (j < nd && dsv[j] != shards[i].sv_f16) ++j;
-            if (j == nd) {
-                dsv[nd] = shards[i].sv_f16;
-                dout[nd] = base + (size_t)i * xb_one;
-                ++nd;
-            }
-        }
-        if (nd > 1)
-            all = glqh_launch_input_rht_blocked_multi(x, x_dtype, x_stride, dsv, dout, nd, Mp, B, in_features, n_pad, blocks_n,
-                                                      n_blocks_n, st);
-        if (all > 0) return 1;
-    }
     for (int i = 0; i < n_shards; ++i) {
-        // layers quantized with the same sign vector share one transform of x
-        int same = -1;
-        for (int j = 0; j < i; ++j)
-            if (shards[j].sv_f16 == shards[i].sv_f16) { same = j; break; }
-        if (same >= 0) {
-            xb[i] = xb[same];
-        } else if (all == 0) {
-            xb[i] = base + (size_t)i * xb_one;
-        } else {
-            void *dst = base + (size_t)i * xb_one;
-            const int rc = glqh_launch_input_rht_blocked(x, x_dtype, x_stride, shards[i].sv_f16, dst, 2, Mp, B, in_features,
-                                                         n_pad, blocks_n, n_blocks_n, st);
-            if (rc > 0) return 1;
-            if (rc < 0) {                                        // rows first, then repacked
-                if (glqh_launch_input_rht(x, x_dtype, x_stride, shards[i].sv_f16, x_rows, GLQH_F16, B, in_features, n_pad,
-                                          bn_meta_dev, blocks_n, n_blocks_n, 0.0f, st) ||
-                    glqh_launch_trellis_pack(x_rows, dst, B, n_pad, st))
-                    return 1;
-            }
-            xb[i] = dst;
-        }
         parts[i] = (float *)(pbase + poff);
         poff += align256((size_t)ks * B * m_pads[i] * esz);
     }
+    if (tr_group_blocked(x, x_dtype, x_stride, B, sv, n_shards, blocks_n, n_blocks_n, bn_meta_dev, in_features, n_pad, base, xb_one,
+                         x_rows, xb, st))
+        return 1;
     float wscales[TR_GROUP_MANY_MAX];                          // fp16 sums carry the layer's scale already
     for (int i = 0; i < n_shards; ++i) wscales[i] = (float)shards[i].wscale;
-    if (glqh_launch_trellis_tile_group(xb, B, packed, R, m_pads, n_shards, n_pad, parts, f16_sums ? 1 : 0, st, wscales)) return 1;
+    if (glqh_launch_trellis_tile_group(xb, B, packed, R, m_pads, n_shards, n_pad, parts, f16_sums ? 1 : 0, st, wscales,
+                                       stage2 ? packed2 : nullptr, R2, rs2))
+        return 1;
     const void *sus[TR_GROUP_MANY_MAX];
     void *ys[TR_GROUP_MANY_MAX];
     int64_t outs[TR_GROUP_MANY_MAX];
@@ -925,13 +946,44 @@ static int tr_group_many(const void *x, int x_dtype, int64_t x_stride, int64_t B
 
 struct tr_group_ctx {
     int R, ks, fi_mode;
-    int ks_layer[GLQH_MAX_SHARDS];                             // 17..64 tokens: every layer's own slot count (ks = 0 when they differ)
+    int ks_layer[GLQH_MAX_SHARDS];                             // 17..64 tokens: ks, per layer
     int64_t m_pads[GLQH_MAX_SHARDS], outs[GLQH_MAX_SHARDS];
     const void *su[GLQH_MAX_SHARDS];
     void *ys[GLQH_MAX_SHARDS];
     float scale[GLQH_MAX_SHARDS];
     float *parts[GLQH_MAX_SHARDS];
 };
+
+// 17..64 tokens: one transform of x per distinct sign vector into the tile kernels' layout (one launch where it
+// applies), the row tiles of all layers in one launch of the small-tile kernel under one K plan, sums left for the
+// finishing launch.  packed2: stacked layers, both streams into one operand.
+static int tr_group_tiles(const void *x, int x_dtype, int64_t x_stride, int64_t B, const void *const sv[], const void *const packed[],
+                          int R, const void *const packed2[], int R2, const float rs2[], int n_shards, const int64_t *blocks_n,
+                          int64_t n_blocks_n, const glqh_block_meta *bn_meta_dev, int64_t in_features, int64_t n_pad, void *ws,
+                          size_t ws_bytes, hipStream_t st, tr_group_ctx *c) {
+    const size_t xbb = align256(glqh_trellis_tile_xb_bytes(n_pad, B)), xrm = align256((size_t)B * n_pad * sizeof(f16));
+    static_assert(GLQH_MAX_SHARDS <= TR_GROUP_MANY_MAX, "a group of layers fits one launch of the tile kernels");
+    c->ks = glqh_trellis_tile_group_ksplit(c->m_pads, n_shards, n_pad, B, packed2 != nullptr);
+    size_t sums = 0;
+    for (int i = 0; i < n_shards; ++i) {
+        c->ks_layer[i] = c->ks;
+        sums += align256((size_t)c->ks * B * c->m_pads[i] * sizeof(float));
+    }
+    const size_t need = (size_t)n_shards * xbb + xrm + sums;
+    GLQH_REQUIRE(ws && ws_bytes >= need, "trellis group: workspace of %zu bytes needed, got %zu", need, ws_bytes);
+    char *p = (char *)ws + (size_t)n_shards * xbb + xrm;
+    for (int i = 0; i < n_shards; ++i) {
+        c->parts[i] = (float *)p;
+        p += align256((size_t)c->ks * B * c->m_pads[i] * sizeof(float));
+    }
+    c->R = R; c->fi_mode = 0;
+    const void *xb_of[GLQH_MAX_SHARDS];
+    if (tr_group_blocked(x, x_dtype, x_stride, B, sv, n_shards, blocks_n, n_blocks_n, bn_meta_dev, in_features, n_pad, ws, xbb,
+                         (f16 *)((char *)ws + (size_t)n_shards * xbb), xb_of, st))
+        return 1;
+    glqh_range range("dequant_matmul");
+    return glqh_launch_trellis_tile_group(xb_of, B, packed, R, c->m_pads, n_shards, n_pad, c->parts, 0, st, nullptr, packed2, R2, rs2);
+}
 
 // x under every distinct sign vector of a group of layers, fp16 rows at ws + j * xb_one (few tokens): one launch for
 // all of them where the small-batch kernel serves the call, one per sign vector otherwise.  x_of[i] = layer i's rows.
@@ -964,50 +1016,20 @@ static int tr_group_transform(const void *x, int x_dtype, int64_t x_stride, int6
     return 0;
 }
 
-// 17..64 tokens: x under every distinct sign vector of a group straight into the tile kernels' layout, buffer j at
-// ws + j * xbb, in one launch.  0: done, xb_of[i] = layer i's buffer; -1: not applicable, nothing launched.
-static int tr_group_transform_blocked(const void *x, int x_dtype, int64_t x_stride, int64_t B, const void *const sv[],
-                                      int n_shards, const int64_t *blocks_n, int64_t n_blocks_n, int64_t in_features,
-                                      int64_t n_pad, void *ws, size_t xbb, void *xb_of[], hipStream_t st) {
-    const void *dsv[GLQH_MAX_SHARDS];
-    void *dout[GLQH_MAX_SHARDS];
-    int nd = 0;
-    for (int i = 0; i < n_shards; ++i) {
-        int j = 0;
-        while (j < nd && dsv[j] != sv[i]) ++j;
-        if (j == nd) {
-            dsv[nd] = sv[i];
-            dout[nd] = (char *)ws + (size_t)nd * xbb;
-            ++nd;
-        }
-        xb_of[i] = dout[j];
-    }
-    if (nd < 2) return -1;
-    return glqh_launch_input_rht_blocked_multi(x, x_dtype, x_stride, dsv, dout, nd, glqh_trellis_tile_padded_tokens(B), B,
-                                               in_features, n_pad, blocks_n, n_blocks_n, st);
-}
-
-// One finishing launch for all layers of a group; at 17..64 tokens, where every layer has its own K plan, one per
-// layer when their slot counts differ.
+// One finishing launch for all layers of a group; at 33..64 tokens the whole-block transforms where they apply.
 static int tr_group_finish(const tr_group_ctx &c, int n_shards, int64_t B, int y_dtype, int64_t y_stride, hipStream_t st) {
-    if (B > TR_GROUP_SMALL_MAX && c.ks == 0) {
+    if (B > TR_GROUP_SMALL_MAX) {
         const float *const *pt = c.parts;
         const int rc = glqh_launch_output_rht_wide_group(pt, c.su, c.ys, c.scale, c.m_pads, c.outs, c.ks_layer, n_shards, 0,
                                                          y_dtype, y_stride, B, st);
         if (rc >= 0) return rc;
-        for (int i = 0; i < n_shards; ++i) {
-            const int one = glqh_launch_output_rht_wide_group(pt + i, c.su + i, c.ys + i, c.scale + i, c.m_pads + i, c.outs + i,
-                                                              c.ks_layer + i, 1, 0, y_dtype, y_stride, B, st);
-            if (one > 0 || (one < 0 && glqh_launch_output_rht_group(pt + i, c.su + i, c.ys + i, c.scale + i, c.m_pads + i,
-                                                                    c.outs + i, 1, y_dtype, y_stride, B, c.ks_layer[i], st)))
-                return 1;
-        }
-        return 0;
     }
     return glqh_launch_output_rht_group(c.parts, c.su, c.ys, c.scale, c.m_pads, c.outs, n_shards, y_dtype, y_stride,
                                         B, c.ks, st);
 }
 
+// Decode launch of a group: checks, K plan, partial-sum layout in ws.  On return parts[i] holds
+// layer i's [slot][token][row] fp32 partial sums and *ks_out the slot count.
 static int tr_group_decode(const void *x, int x_dtype, int64_t x_stride, int64_t B,
                            const glqh_trellis_shard *shards, int n_shards, const int64_t *blocks_n,
                            int64_t n_blocks_n, const glqh_block_meta *bn_meta_dev, int64_t in_features,
@@ -1051,55 +1073,9 @@ static int tr_group_decode(const void *x, int x_dtype, int64_t x_stride, int64_t
         total += sh.m_pad;
     }
     int steps = 0, ks = 0;
-    if (B > TR_GROUP_SMALL_MAX) {
-        // 17..64 tokens: one transform launch per distinct sign vector, straight into the tile kernel's layout where
-        // it can, one launch of the small-tile kernel per layer (its own K plan), sums left for the finishing launch
-        const size_t xbb = align256(glqh_trellis_tile_xb_bytes(n_pad, B)), xrm = align256((size_t)B * n_pad * sizeof(f16));
-        size_t sums = 0;
-        bool same = true;
-        for (int i = 0; i < n_shards; ++i) {
-            c->ks_layer[i] = glqh_trellis_tile_ksplit(c->m_pads[i], n_pad, B);
-            same = same && c->ks_layer[i] == c->ks_layer[0];
-            sums += align256((size_t)c->ks_layer[i] * B * c->m_pads[i] * sizeof(float));
-        }
-        const size_t need = (size_t)n_shards * xbb + xrm + sums;
-        GLQH_REQUIRE(ws && ws_bytes >= need, "trellis group: workspace of %zu bytes needed, got %zu", need, ws_bytes);
-        void *xb = ws;
-        f16 *x_rht = (f16 *)((char *)ws + (size_t)n_shards * xbb);
-        char *p = (char *)ws + (size_t)n_shards * xbb + xrm;
-        c->R = R; c->ks = same ? c->ks_layer[0] : 0; c->fi_mode = 0;
-        void *xb_of[GLQH_MAX_SHARDS];
-        const int all = tr_group_transform_blocked(x, x_dtype, x_stride, B, sv, n_shards, blocks_n, n_blocks_n, in_features,
-                                                   n_pad, ws, xbb, xb_of, st);
-        if (all > 0) return 1;
-        int blocked = -1;
-        for (int i = 0; i < n_shards; ++i) {
-            if (all == 0) {                                    // every sign vector's activations are in place
-                c->parts[i] = (float *)p;
-                p += align256((size_t)c->ks_layer[i] * B * c->m_pads[i] * sizeof(float));
-                glqh_range range("dequant_matmul");
-                if (glqh_launch_trellis_tile(nullptr, xb_of[i], B, packed[i], R, c->m_pads[i], n_pad, c->parts[i], 0, 1.0f, 0,
-                                             0, st, 0))
-                    return 1;
-                continue;
-            }
-            if (i == 0 || sv[i] != sv[i - 1]) {
-                blocked = glqh_launch_input_rht_blocked(x, x_dtype, x_stride, sv[i], xb, 2, glqh_trellis_tile_padded_tokens(B),
-                                                        B, in_features, n_pad, blocks_n, n_blocks_n, st);
-                if (blocked > 0) return 1;
-                if (blocked != 0 && glqh_launch_input_rht(x, x_dtype, x_stride, sv[i], x_rht, GLQH_F16, B, in_features, n_pad,
-                                                          bn_meta_dev, blocks_n, n_blocks_n, 0.0f, st))
-                    return 1;
-            }
-            c->parts[i] = (float *)p;
-            p += align256((size_t)c->ks_layer[i] * B * c->m_pads[i] * sizeof(float));
-            glqh_range range("dequant_matmul");
-            if (glqh_launch_trellis_tile(blocked == 0 ? nullptr : x_rht, xb, B, packed[i], R, c->m_pads[i], n_pad, c->parts[i],
-                                         0, 1.0f, 0, 0, st, 0))
-                return 1;
-        }
-        return 0;
-    }
+    if (B > TR_GROUP_SMALL_MAX)
+        return tr_group_tiles(x, x_dtype, x_stride, B, sv, packed, R, nullptr, 0, nullptr, n_shards, blocks_n, n_blocks_n, bn_meta_dev,
+                              in_features, n_pad, ws, ws_bytes, st, c);
     if (tr_group_plain(total, n_pad, B)) {
         // one K plan for all layers (that of the tallest), so that the finishing launch sees one slot count
         int64_t mmax = 0;
@@ -1152,7 +1128,7 @@ extern "C" int glqh_fused_linear_trellis_3inst_group(const void *x, int x_dtype,
     GLQH_REQUIRE(y_stride > 0 || B > TR_GROUP_MANY_MIN, "trellis group: y_stride 0 (packed rows per layer) needs more than %lld tokens",
                  (long long)TR_GROUP_MANY_MIN);
     if (B > TR_GROUP_MANY_MIN)
-        return tr_group_many(x, x_dtype, x_stride, B, shards, n_shards, blocks_n, n_blocks_n, bn_meta_dev, in_features,
+        return tr_group_many(x, x_dtype, x_stride, B, shards, nullptr, n_shards, blocks_n, n_blocks_n, bn_meta_dev, in_features,
                              n_pad, y_dtype, y_stride, ws, ws_bytes, st);
     tr_group_ctx c;
     if (tr_group_decode(x, x_dtype, x_stride, B, shards, n_shards, blocks_n, n_blocks_n, bn_meta_dev, in_features,
@@ -1202,15 +1178,10 @@ extern "C" int glqh_fused_linear_trellis_3inst_group_rvq2(const void *x, int x_d
     for (int i = 0; i < n_shards; ++i) {
         const glqh_trellis_shard &sh = shards[i];
         const glqh_trellis_stage2 &s2 = stage2[i];
-        GLQH_REQUIRE(sh.sv_f16 && sh.packed && sh.su_f16 && sh.y && s2.packed2, "trellis two-stage group: null pointer in shard %d", i);
-        GLQH_REQUIRE(s2.inv_resid_scale2 != 0.0, "trellis two-stage group: shard %d has a second stream but inv_resid_scale2 = 0", i);
-        int R1, Ri;
+        GLQH_REQUIRE(sh.sv_f16 && sh.packed && sh.su_f16 && sh.y, "trellis two-stage group: null pointer in shard %d", i);
+        int R1;
         if (tr_bits_from_packed(sh.packed_cols, 0, &R1) || tr_check_shape(sh.m_pad, n_pad, sh.packed_rows)) return 1;
-        if (tr_bits_from_packed(s2.packed2_cols, 1, &Ri) || tr_check_shape(sh.m_pad, n_pad, s2.packed2_rows)) return 1;
-        GLQH_REQUIRE(R1 == 4, "trellis two-stage group: first stages of 4 bits/weight, shard %d has %d", i, R1);
-        GLQH_REQUIRE(i == 0 || Ri == R2, "trellis two-stage group: second stages of %d and %d bits/weight cannot share a launch",
-                     R2, Ri);
-        R2 = Ri;
+        if (tr_check_stage2(s2, i, R1, sh.m_pad, n_pad, i == 0, &R2)) return 1;
         GLQH_REQUIRE(sh.out_features >= 1 && sh.out_features <= sh.m_pad, "trellis two-stage group: out_features exceeds m_pad");
         c.m_pads[i] = sh.m_pad; c.outs[i] = sh.out_features;
         packed[i] = sh.packed; packed2[i] = s2.packed2; rs2[i] = (float)s2.inv_resid_scale2;
@@ -1220,53 +1191,10 @@ extern "C" int glqh_fused_linear_trellis_3inst_group_rvq2(const void *x, int x_d
     }
     int steps = 0, ks = 0;
     if (B > TR_GROUP_SMALL_MAX) {
-        // 17..64 tokens: one transform launch per distinct sign vector, one launch of the small-tile kernel per layer,
-        // which decodes both streams into one operand, finishing as for single-stage layers
         GLQH_REQUIRE(tr_fuse_stages_enabled(), "trellis two-stage group: more than 16 tokens need both streams in one operand");
-        const size_t xbb = align256(glqh_trellis_tile_xb_bytes(n_pad, B)), xrm = align256((size_t)B * n_pad * sizeof(f16));
-        size_t sums = 0;
-        bool same = true;
-        for (int i = 0; i < n_shards; ++i) {
-            c.ks_layer[i] = glqh_trellis_tile_ksplit(c.m_pads[i], n_pad, B, 1);
-            same = same && c.ks_layer[i] == c.ks_layer[0];
-            sums += align256((size_t)c.ks_layer[i] * B * c.m_pads[i] * sizeof(float));
-        }
-        const size_t need = (size_t)n_shards * xbb + xrm + sums;
-        GLQH_REQUIRE(ws && ws_bytes >= need, "trellis two-stage group: workspace of %zu bytes needed, got %zu", need, ws_bytes);
-        void *xb = ws;
-        f16 *x_rht = (f16 *)((char *)ws + (size_t)n_shards * xbb);
-        char *p = (char *)ws + (size_t)n_shards * xbb + xrm;
-        c.ks = same ? c.ks_layer[0] : 0;
-        void *xb_of[GLQH_MAX_SHARDS];
-        const int all = tr_group_transform_blocked(x, x_dtype, x_stride, B, sv, n_shards, blocks_n, n_blocks_n, in_features,
-                                                   n_pad, ws, xbb, xb_of, st);
-        if (all > 0) return 1;
-        int blocked = -1;
-        for (int i = 0; i < n_shards; ++i) {
-            if (all == 0) {                                    // every sign vector's activations are in place
-                c.parts[i] = (float *)p;
-                p += align256((size_t)c.ks_layer[i] * B * c.m_pads[i] * sizeof(float));
-                glqh_range range("dequant_matmul");
-                if (glqh_launch_trellis_tile(nullptr, xb_of[i], B, packed[i], 4, c.m_pads[i], n_pad, c.parts[i], 0, 1.0f, 0, 0,
-                                             st, 0, packed2[i], R2, rs2[i]))
-                    return 1;
-                continue;
-            }
-            if (i == 0 || sv[i] != sv[i - 1]) {
-                blocked = glqh_launch_input_rht_blocked(x, x_dtype, x_stride, sv[i], xb, 2, glqh_trellis_tile_padded_tokens(B),
-                                                        B, in_features, n_pad, blocks_n, n_blocks_n, st);
-                if (blocked > 0) return 1;
-                if (blocked != 0 && glqh_launch_input_rht(x, x_dtype, x_stride, sv[i], x_rht, GLQH_F16, B, in_features, n_pad,
-                                                          bn_meta_dev, blocks_n, n_blocks_n, 0.0f, st))
-                    return 1;
-            }
-            c.parts[i] = (float *)p;
-            p += align256((size_t)c.ks_layer[i] * B * c.m_pads[i] * sizeof(float));
-            glqh_range range("dequant_matmul");
-            if (glqh_launch_trellis_tile(blocked == 0 ? nullptr : x_rht, xb, B, packed[i], 4, c.m_pads[i], n_pad, c.parts[i], 0,
-                                         1.0f, 0, 0, st, 0, packed2[i], R2, rs2[i]))
-                return 1;
-        }
+        if (tr_group_tiles(x, x_dtype, x_stride, B, sv, packed, 4, packed2, R2, rs2, n_shards, blocks_n, n_blocks_n, bn_meta_dev,
+                           in_features, n_pad, ws, ws_bytes, st, &c))
+            return 1;
         return tr_group_finish(c, n_shards, B, y_dtype, y_stride, st);
     }
     if (B > 1) {

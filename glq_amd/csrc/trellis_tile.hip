@@ -68,8 +68,26 @@ struct tt_group {
     float *out[TT_MAX_GROUP];
     int m[TT_MAX_GROUP], rt0[TT_MAX_GROUP];
     float scale[TT_MAX_GROUP];                     // factor of the layer's fp16 sums (its Wscale)
+    const uint8_t *packed2[TT_MAX_GROUP];          // stacked layers (kernels with R2 > 0): residual streams and scales
+    float rs2[TT_MAX_GROUP];
     int n;
 };
+
+// the layer of a group that owns row tile rt, and the tile's number inside it
+struct tt_layer {
+    const uint8_t *packed, *packed2;
+    const f16 *xb;
+    float *out, scale, rs2;
+    int m, rt;
+};
+__device__ __forceinline__ tt_layer tt_group_layer(const tt_group &g, int rt) {
+    tt_layer l = {g.packed[0], g.packed2[0], g.xb[0], g.out[0], g.scale[0], g.rs2[0], g.m[0], rt};
+#pragma unroll
+    for (int j = 1; j < TT_MAX_GROUP; ++j)
+        if (j < g.n && rt >= g.rt0[j])
+            l = {g.packed[j], g.packed2[j], g.xb[j], g.out[j], g.scale[j], g.rs2[j], g.m[j], rt - g.rt0[j]};
+    return l;
+}
 
 // Routed experts of a mixture-of-experts layer with many rows per expert (glq/csrc/glq_trellis.cu:1475-1540 is the
 // reference's grouped kernel; its caller loops over whole per-expert linears beyond 256 tokens,
@@ -204,20 +222,17 @@ __device__ __forceinline__ void tr_tile_body(const tt_args &a, const tt_group &g
         // fp16 sums leave times the layer's scale: an unscaled sum over a long row of large activations can pass
         // the fp16 range where the scaled one, of the size of the layer's output, does not
         float f16sc = a.scale;
+        const uint8_t *lpacked2 = a.packed2;
+        float lrs2 = a.rs2;
         if constexpr (GROUP) {
-            int first = 0;
-            lm = g.m[0]; lpacked = g.packed[0]; lxb = g.xb[0]; lout = g.out[0]; f16sc = g.scale[0];
-#pragma unroll
-            for (int j = 1; j < TT_MAX_GROUP; ++j)
-                if (j < g.n && rt >= g.rt0[j]) { first = g.rt0[j]; lm = g.m[j]; lpacked = g.packed[j]; lxb = g.xb[j]; lout = g.out[j]; f16sc = g.scale[j]; }
-            rt -= first;
+            const tt_layer y = tt_group_layer(g, rt);
+            rt = y.rt; lm = y.m; lpacked = y.packed; lxb = y.xb; lout = y.out; f16sc = y.scale;
+            if constexpr (R2 > 0) { lpacked2 = y.packed2; lrs2 = y.rs2; }
         }
         const int mpairs = lm >> 5;
         int tok0 = tt0 * (MW * 16 * NTW) + (PC ? wave & 3 : wave) * 16 * NTW, limit = a.M;
         float osc = 1.0f;
         bool active = true;                                     // uniform over the wave
-        const uint8_t *lpacked2 = a.packed2;
-        float lrs2 = a.rs2;
         if constexpr (MOE) {
             // a run of the table may be longer than this kernel's tile (a stacked expert's streams are decoded
             // into one operand in tiles of at most 256 positions): TT workgroup tiles per run, in order
@@ -470,6 +485,19 @@ tr_tile_group_kernel(const tt_args a, const tt_group g) {
     tr_tile_body<R, NTW, TT_GROUP>(a, g, tt_moe{});
 }
 
+// stacked layers of a group
+template <int R2, int NTW>
+__global__ void __launch_bounds__(TT_THREADS)
+tr_tile_group_rvq_kernel(const tt_args a, const tt_group g) {
+    tr_tile_body<4, NTW, TT_GROUP, R2>(a, g, tt_moe{});
+}
+
+template <int R2, int NTW>
+__global__ void __launch_bounds__(TT_THREADS)
+tr_tile_group_rvq_pc_kernel(const tt_args a, const tt_group g) {
+    tr_tile_body<4, NTW, TT_GROUP, R2, true>(a, g, tt_moe{});
+}
+
 template <int R, int NTW>
 __global__ void __launch_bounds__(TT_THREADS)
 tr_tile_moe_kernel(const tt_args a, const tt_moe mo) {
@@ -531,15 +559,14 @@ tr_moe_tiles_kernel(const int *__restrict__ offs, int n_experts, int tile_tok, i
 // block pair w >> 2, k-pair (w >> 1) & 1, m-tile w & 1).  Same K slots and order of summation as above.
 constexpr size_t TT_SMALL_LDS = (size_t)8 * TT_BUF * 16;       // 128 KB
 
-template <int R, int TG, int NTW, int R2 = 0>
-__global__ void __launch_bounds__(TT_THREADS)
-tr_tile_small_kernel(const tt_args a) {
+template <int R, int TG, int NTW, int R2, bool GROUP>
+__device__ __forceinline__ void tr_tile_small_body(const tt_args &a, const tt_group &g) {
     constexpr int RG = TT_FRAGS / TG;                          // operand groups
     constexpr int RB = R2 > 0 ? R2 : 1, REC2 = 4 * RB;         // R2 > 0: a stacked layer, both streams into one operand
     extern __shared__ u32x4 abuf[];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int i = lane & 15, q = lane >> 4;
-    const int nkp = a.k >> 5, nds = a.k >> 6, mpairs = a.m >> 5;
+    const int nkp = a.k >> 5, nds = a.k >> 6;
     constexpr int REC = 4 * R;
     const int tg = wave % TG, rg = wave / TG;
 
@@ -551,29 +578,31 @@ tr_tile_small_kernel(const tt_args a) {
 
     const int nitems = a.KS * a.RT;                            // one token tile
     for (int item = blockIdx.x; item < nitems; item += gridDim.x) {
-        const int rt = item % a.RT, slot = item / a.RT;
-        const int r0 = rt * TT_ROWS;
+        const int slot = item / a.RT;
+        tt_layer y = {a.packed, a.packed2, a.xb, a.out, 1.0f, a.rs2, a.m, item % a.RT};
+        if constexpr (GROUP) y = tt_group_layer(g, y.rt);
+        const int rt = y.rt, r0 = rt * TT_ROWS, mpairs = y.m >> 5;
         const int ds0 = slot * a.slot_ds, ds1 = min(ds0 + a.slot_ds, nds);
         const int nquads = (ds1 - ds0 + 3) >> 2;
 
         const int mp = min(2 * (2 * rt + unit) + hm, mpairs - 1);
-        const uint8_t *rec_base = a.packed + ((int64_t)mp * nkp * 32 + l) * REC + (int64_t)kpi * 32 * REC;
+        const uint8_t *rec_base = y.packed + ((int64_t)mp * nkp * 32 + l) * REC + (int64_t)kpi * 32 * REC;
         auto load_rec = [&](int d) {                            // the record of k-pair 2d + kpi
             return tr_load_record<R>(rec_base + (int64_t)min(d, ds1 - 1) * 64 * REC);
         };
-        const uint8_t *rec_base2 = R2 > 0 ? a.packed2 + ((int64_t)mp * nkp * 32 + l) * REC2 + (int64_t)kpi * 32 * REC2 : nullptr;
+        const uint8_t *rec_base2 = R2 > 0 ? y.packed2 + ((int64_t)mp * nkp * 32 + l) * REC2 + (int64_t)kpi * 32 * REC2 : nullptr;
         auto load_rec2 = [&](int d) {
             tr_record<RB> r = {};
             if constexpr (R2 > 0) r = tr_load_record<RB>(rec_base2 + (int64_t)min(d, ds1 - 1) * 64 * REC2);
             return r;
         };
         auto emit = [&](const tr_record<R> r, const tr_record<RB> rb, u32x4 *dst) {
-            if constexpr (R2 > 0) tt_emit2<R, RB>(r, rb, a.rs2, unit, kpi, ms, next1, next2, lane, dst);
+            if constexpr (R2 > 0) tt_emit2<R, RB>(r, rb, y.rs2, unit, kpi, ms, next1, next2, lane, dst);
             else tt_emit<R>(r, unit, kpi, ms, next1, next2, lane, dst);
         };
         // multiply role: token 16 * tt + i of the wave's token group
         const int64_t bstep = (int64_t)a.Mp * 32;               // elements from one k-pair to the next
-        const f16 *xrow = a.xb + (int64_t)(16 * NTW * tg + i) * 32 + q * 8;
+        const f16 *xrow = y.xb + (int64_t)(16 * NTW * tg + i) * 32 + q * 8;
         auto load_b = [&](u32x4 (&bb)[NTW][2], int d) {
             d = min(d, ds1 - 1);
 #pragma unroll
@@ -658,11 +687,11 @@ tr_tile_small_kernel(const tt_args a) {
             for (int j = 0; j < TG; ++j) {
                 const int f = rg + RG * j;
                 const int row = r0 + 64 * (f >> 2) + 8 * (f & 3) + rlane;
-                if (row >= a.m) continue;                       // m is a multiple of 32: whole groups of four
+                if (row >= y.m) continue;                       // m is a multiple of 32: whole groups of four
                 if (!a.direct) {
-                    *(f32x4 *)(a.out + ((int64_t)slot * a.M + tok) * a.m + row) = acc[j][tt];
+                    *(f32x4 *)(y.out + ((int64_t)slot * a.M + tok) * y.m + row) = acc[j][tt];
                 } else {
-                    float *o = a.out + (int64_t)tok * a.out_stride + row;
+                    float *o = y.out + (int64_t)tok * a.out_stride + row;
                     if ((a.out_stride & 3) == 0) {
                         f32x4 v = acc[j][tt] * a.scale;
                         if (a.accum) v += *(f32x4 *)o;
@@ -675,6 +704,20 @@ tr_tile_small_kernel(const tt_args a) {
             }
         }
     }
+}
+
+template <int R, int TG, int NTW, int R2 = 0>
+__global__ void __launch_bounds__(TT_THREADS)
+tr_tile_small_kernel(const tt_args a) {
+    tr_tile_small_body<R, TG, NTW, R2, false>(a, tt_group{});
+}
+
+// the layers of a group: one launch instead of one per layer, most of which leave CUs idle ((2048, 512, 512) x 2048
+// at 20 tokens, 4 bits, kernels 21.8 -> 7.8 us, whole call 30 -> 16; (5248, 640, 640) x 5248, 4 + 2 bits, 62 -> 32)
+template <int R, int TG, int NTW, int R2 = 0>
+__global__ void __launch_bounds__(TT_THREADS)
+tr_tile_small_group_kernel(const tt_args a, const tt_group g) {
+    tr_tile_small_body<R, TG, NTW, R2, true>(a, g);
 }
 
 // (M, k) row-major fp16 -> xb[k-pair][token][q][8]: slot q of a k-pair takes columns
@@ -873,6 +916,10 @@ int tt_init_R() {
            tt_set_lds(tr_tile_moe_rvq_pc_kernel<R, 2>) || tt_set_lds(tr_tile_moe_rvq_pc_kernel<R, 4>) ||
            tt_set_lds(tr_tile_group_kernel<R, 1>) || tt_set_lds(tr_tile_group_kernel<R, 2>) ||
            tt_set_lds(tr_tile_small_kernel<4, 2, 1, R>) || tt_set_lds(tr_tile_small_kernel<4, 4, 1, R>) ||
+           tt_set_lds(tr_tile_small_group_kernel<R, 2, 1>) || tt_set_lds(tr_tile_small_group_kernel<R, 4, 1>) ||
+           tt_set_lds(tr_tile_small_group_kernel<4, 2, 1, R>) || tt_set_lds(tr_tile_small_group_kernel<4, 4, 1, R>) ||
+           tt_set_lds(tr_tile_group_rvq_kernel<R, 1>) || tt_set_lds(tr_tile_group_rvq_kernel<R, 2>) ||
+           tt_set_lds(tr_tile_group_rvq_pc_kernel<R, 2>) || tt_set_lds(tr_tile_group_rvq_pc_kernel<R, 4>) ||
            tt_set_lds(tr_tile_rvq_kernel<R, 1>) || tt_set_lds(tr_tile_rvq_kernel<R, 2>) ||
            tt_set_lds(tr_tile_moe_rvq_kernel<R, 1>) || tt_set_lds(tr_tile_moe_rvq_kernel<R, 2>) ||
            tt_set_lds(tr_tile_group_kernel<R, 4>) || tt_set_lds(tr_tile_moe_kernel<R, 1>) ||
@@ -1003,59 +1050,71 @@ int glqh_launch_trellis_tile(const void *x_f16, void *xb_scratch, int64_t M, con
     }
 }
 
-// ---- several layers in one launch (many tokens) ---------------------------------------------------
+// ---- several layers in one launch (more than 16 tokens) -------------------------------------------
 namespace {
-void tt_make_group_plan(const int64_t *m, int n_layers, int64_t k, int64_t M, tt_plan *p) {
-    int64_t rt = 0, mtot = 0;
-    for (int l = 0; l < n_layers; ++l) {
-        rt += (m[l] + TT_ROWS - 1) / TT_ROWS;
-        mtot += m[l];
-    }
-    tt_make_plan(TT_ROWS * rt, k, M, p);                        // same rule, on the row tiles of all layers
-    (void)mtot;
+void tt_make_group_plan(const int64_t *m, int n_layers, int64_t k, int64_t M, int two_stage, tt_plan *p) {
+    int64_t rt = 0;
+    for (int l = 0; l < n_layers; ++l) rt += (m[l] + TT_ROWS - 1) / TT_ROWS;
+    tt_make_plan(TT_ROWS * rt, k, M, p, two_stage ? 2 : 4);     // same rule, on the row tiles of all layers
 }
 
+#define GLQH_TTG(...)                                                                                      \
+    hipLaunchKernelGGL((__VA_ARGS__), dim3((unsigned)p.grid), dim3(TT_THREADS), a.M <= 64 ? TT_SMALL_LDS : TT_LDS, stream, a, g)
 template <int R>
 int tt_launch_group_R(const tt_plan &p, const tt_args &a, const tt_group &g, hipStream_t stream) {
-#define GLQH_TTG(NTW)                                                                                      \
-    hipLaunchKernelGGL((tr_tile_group_kernel<R, NTW>), dim3((unsigned)p.grid), dim3(TT_THREADS), TT_LDS, stream, a, g)
-#define GLQH_TTGP(NTW)                                                                                     \
-    hipLaunchKernelGGL((tr_tile_group_pc_kernel<R, NTW>), dim3((unsigned)p.grid), dim3(TT_THREADS), TT_LDS, stream, a, g)
-    if (tt_split_roles(p, 8) && p.NTW == 1) GLQH_TTGP(2);
-    else if (tt_split_roles(p, 8)) GLQH_TTGP(4);
-    else if (p.NTW == 1) GLQH_TTG(1);
-    else if (p.NTW == 2) GLQH_TTG(2);
-    else GLQH_TTG(4);
-#undef GLQH_TTG
-#undef GLQH_TTGP
+    if (a.M <= 32) GLQH_TTG(tr_tile_small_group_kernel<R, 2, 1>);
+    else if (a.M <= 64) GLQH_TTG(tr_tile_small_group_kernel<R, 4, 1>);
+    else if (tt_split_roles(p, 8) && p.NTW == 1) GLQH_TTG(tr_tile_group_pc_kernel<R, 2>);
+    else if (tt_split_roles(p, 8)) GLQH_TTG(tr_tile_group_pc_kernel<R, 4>);
+    else if (p.NTW == 1) GLQH_TTG(tr_tile_group_kernel<R, 1>);
+    else if (p.NTW == 2) GLQH_TTG(tr_tile_group_kernel<R, 2>);
+    else GLQH_TTG(tr_tile_group_kernel<R, 4>);
     GLQH_LAUNCH_CHECK("trellis tile group launch");
     return 0;
 }
+
+template <int R2>
+int tt_launch_group_rvq(const tt_plan &p, const tt_args &a, const tt_group &g, hipStream_t stream) {
+    if (a.M <= 32) GLQH_TTG(tr_tile_small_group_kernel<4, 2, 1, R2>);
+    else if (a.M <= 64) GLQH_TTG(tr_tile_small_group_kernel<4, 4, 1, R2>);
+    else if (tt_split_roles(p, 8) && p.NTW == 1) GLQH_TTG(tr_tile_group_rvq_pc_kernel<R2, 2>);
+    else if (tt_split_roles(p, 8)) GLQH_TTG(tr_tile_group_rvq_pc_kernel<R2, 4>);
+    else if (p.NTW == 1) GLQH_TTG(tr_tile_group_rvq_kernel<R2, 1>);
+    else GLQH_TTG(tr_tile_group_rvq_kernel<R2, 2>);
+    GLQH_LAUNCH_CHECK("trellis two-stage tile group launch");
+    return 0;
+}
+#undef GLQH_TTG
 }  // namespace
 
-int glqh_trellis_tile_group_ksplit(const int64_t *m, int n_layers, int64_t k, int64_t M) {
+int glqh_trellis_tile_group_ksplit(const int64_t *m, int n_layers, int64_t k, int64_t M, int two_stage) {
     tt_plan p;
-    tt_make_group_plan(m, n_layers, k, M, &p);
+    tt_make_group_plan(m, n_layers, k, M, two_stage, &p);
     return p.KS;
 }
 
-// Layers l < n_layers (at most 4) of the same width k and bits/weight against the same M > 64 tokens: partial
-// sums out[l][(slot * M + token) * m[l] + row] (fp16 with out_f16, then times f16_scale[l] if given), K slots from
-// glqh_trellis_tile_group_ksplit.
+// Layers l < n_layers (at most 4) of the same width k and bits/weight against the same M > 16 tokens: partial
+// sums out[l][(slot * M + token) * m[l] + row] (fp16 with out_f16 at more than 64 tokens, then times f16_scale[l] if
+// given), K slots from glqh_trellis_tile_group_ksplit.
 // xb[l]: the layer's activations in the blocked layout (glqh_trellis_tile_padded_tokens(M) tokens).
+// packed2 (with R2, rs2): the residual stages of stacked layers, first stages of 4 bits/weight.
 int glqh_launch_trellis_tile_group(const void *const xb[], int64_t M, const void *const packed[], int R,
                                    const int64_t m[], int n_layers, int64_t k, float *const out[], int out_f16,
-                                   hipStream_t stream, const float f16_scale[]) {
+                                   hipStream_t stream, const float f16_scale[], const void *const packed2[], int R2,
+                                   const float rs2[]) {
     GLQH_REQUIRE(n_layers >= 1 && n_layers <= TT_MAX_GROUP, "trellis tile group: %d layers (1..%d)", n_layers, TT_MAX_GROUP);
-    GLQH_REQUIRE(M > 64, "trellis tile group: more than 64 tokens");
+    GLQH_REQUIRE(M > 16 && (M > 64 || !out_f16), "trellis tile group: more than 16 tokens (64 for fp16 sums)");
+    GLQH_REQUIRE(!packed2 || R == 4, "trellis tile group: two streams in one operand need first stages of 4 bits/weight");
     tt_plan p;
-    tt_make_group_plan(m, n_layers, k, M, &p);
+    tt_make_group_plan(m, n_layers, k, M, packed2 != nullptr, &p);
     tt_args a = {};
     tt_group g = {};
     g.n = n_layers;
     int rt = 0;
     for (int l = 0; l < n_layers; ++l) {
         g.packed[l] = (const uint8_t *)packed[l];
+        g.packed2[l] = packed2 ? (const uint8_t *)packed2[l] : nullptr;
+        g.rs2[l] = packed2 ? rs2[l] : 0.0f;
         g.xb[l] = (const f16 *)xb[l];
         g.out[l] = out[l];
         g.scale[l] = out_f16 && f16_scale ? f16_scale[l] : 1.0f;
@@ -1072,6 +1131,15 @@ int glqh_launch_trellis_tile_group(const void *const xb[], int64_t M, const void
     a.KS = p.KS;
     a.slot_ds = p.slot_ds;
     a.out_f16 = out_f16;
+    if (packed2) {
+        switch (R2) {
+        case 1: return tt_launch_group_rvq<1>(p, a, g, stream);
+        case 2: return tt_launch_group_rvq<2>(p, a, g, stream);
+        case 3: return tt_launch_group_rvq<3>(p, a, g, stream);
+        case 4: return tt_launch_group_rvq<4>(p, a, g, stream);
+        }
+        return glqh_fail("trellis tile kernel: second stage of 1-4 bits/weight, got %d", R2);
+    }
     switch (R) {
     case 1: return tt_launch_group_R<1>(p, a, g, stream);
     case 2: return tt_launch_group_R<2>(p, a, g, stream);

@@ -71,6 +71,37 @@ def test_grouped_many_tokens(ms, n, B, K, shared_sv):
         off += m
 
 
+@pytest.mark.parametrize("ms,n,B,bits,shared_sv", [
+    ((2048, 512, 512), 2048, 17, (4,), False), ((1088, 32), 2368, 32, (3,), True), ((160, 320, 2336, 64), 1088, 33, (2,), False),
+    ((11008, 96), 576, 64, (4,), False), ((512, 1088), 704, 20, (4, 2), False), ((2048, 512, 512), 2048, 64, (4, 4), True),
+    ((160, 96), 128, 37, (4, 1), False),
+])
+def test_grouped_few_dozen_tokens(ms, n, B, bits, shared_sv):
+    from glq_amd import ext, hadamard as H
+    say("grouped few dozen tokens", ms, n, B, bits, shared_sv)
+    layers, bn, bn_meta = _layers(ms, n, bits[0], 3, shared_sv)
+    x = (torch.randn(B, n, generator=torch.Generator().manual_seed(5)) * 0.7).to(torch.bfloat16).to(DEV)
+    sv0 = t(layers[0]["sv"])
+    shards, ones = [], []
+    for i, l in enumerate(layers):
+        sv, su, p1, bm = sv0 if shared_sv else t(l["sv"]), t(l["su"]), t(l["packed"]), O.block_decompose(l["m"])
+        p2 = t(O.random_packed(l["m"], n, bits[1], 70 + i)) if len(bits) > 1 else None
+        shards.append((sv, su, p1) + ((p2, l["wscale"], 0.3) if p2 is not None else (l["wscale"],)) + (l["m"], l["m"]))
+        dims = (torch.tensor(bn), torch.tensor(bm), bn_meta, H.pack_block_meta(bm).to(DEV), l["wscale"])
+        if p2 is not None:
+            one = ext.glq_fused_linear_trellis_3inst_rvq2_cuda(x, sv, su, p1, p2, *dims, 0.3, n, l["m"], n, l["m"],
+                                                               out_dtype=torch.bfloat16)
+        else:
+            one = ext.glq_fused_linear_trellis_3inst_cuda(x, sv, su, p1, *dims, n, l["m"], n, l["m"], out_dtype=torch.bfloat16)
+        ones.append(one)
+    call = ext.glq_fused_linear_trellis_3inst_group_rvq2 if len(bits) > 1 else ext.glq_fused_linear_trellis_3inst_group
+    y = call(x, shards, torch.tensor(bn), bn_meta, n, n, out_dtype=torch.bfloat16)
+    off = 0
+    for m, one in zip(ms, ones):                                 # the layer on its own: another K split at most
+        assert rel(y[:, off:off + m], one.float().cpu().numpy()) < 4e-3
+        off += m
+
+
 def test_grouped_many_tokens_refusals():
     from glq_amd import ext
     say("grouped many tokens refusals")
