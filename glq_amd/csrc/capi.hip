@@ -1138,7 +1138,7 @@ extern "C" int glqh_fused_linear_trellis_3inst_group(const void *x, int x_dtype,
     return tr_group_finish(c, n_shards, B, y_dtype, y_stride, st);
 }
 
-// The same for stacked (two-stage) layers at one token: every layer's two streams decoded by one launch
+// The same for stacked (two-stage) layers: every layer's two streams decoded into one operand
 // (first stage 4 bits/weight, the second stages of one rate), finished like single-stage layers.
 extern "C" int glqh_fused_linear_trellis_3inst_group_rvq2(const void *x, int x_dtype, int64_t x_stride, int64_t B,
                                                           const glqh_trellis_shard *shards,
@@ -1152,11 +1152,15 @@ extern "C" int glqh_fused_linear_trellis_3inst_group_rvq2(const void *x, int x_d
     GLQH_REQUIRE(x && shards && stage2, "trellis two-stage group: null pointer");
     GLQH_REQUIRE(n_shards >= 1 && n_shards <= GLQH_MAX_SHARDS, "trellis two-stage group: %d shards (1..%d)", n_shards,
                  GLQH_MAX_SHARDS);
-    GLQH_REQUIRE(B >= 1 && B <= TR_GROUP_MANY_MIN, "trellis two-stage group: B=%lld (the grouped two-stage call serves 1..64 tokens)",
-                 (long long)B);
+    GLQH_REQUIRE(B >= 1, "trellis two-stage group: B=%lld", (long long)B);
     GLQH_REQUIRE(x_dtype == GLQH_F16 || x_dtype == GLQH_BF16, "trellis two-stage group: x must be f16 or bf16");
     GLQH_REQUIRE(in_features >= 1 && in_features <= n_pad, "trellis two-stage group: in_features exceeds n_pad");
     GLQH_REQUIRE(y_stride > 0, "trellis two-stage group: y_stride must be positive");
+    if (B > TR_GROUP_MANY_MIN) {
+        GLQH_REQUIRE(tr_fuse_stages_enabled(), "trellis two-stage group: more than 16 tokens need both streams in one operand");
+        return tr_group_many(x, x_dtype, x_stride, B, shards, stage2, n_shards, blocks_n, n_blocks_n, bn_meta_dev, in_features, n_pad,
+                             y_dtype, y_stride, ws, ws_bytes, st);
+    }
     const bool pow2_n = (n_pad & (n_pad - 1)) == 0;
     GLQH_REQUIRE(n_blocks_n > 1 ? (bn_meta_dev != nullptr && blocks_n != nullptr) : pow2_n,
                  "trellis two-stage group: input block sizes missing");

@@ -49,7 +49,7 @@ struct {
 PyObject *g_ext = nullptr;                                     // glq_amd.ext's globals: its switches are read per call
 PyObject *g_oom = nullptr;                                     // torch.OutOfMemoryError
 PyObject *s_buffers, *s_SV, *s_SU, *s_tp, *s_tp2, *s_tlut, *s_bias, *s_codebook, *s_codebook2, *s_shards;
-PyObject *s_q[4], *s_dense, *s_tmax, *s_smax, *s_fold, *s_emax, *s_efmax;
+PyObject *s_q[4], *s_dense, *s_fuse, *s_tmax, *s_smax, *s_fold, *s_emax, *s_efmax;
 
 constexpr int64_t MOST_TOKENS = 32768;                         // _MAX_TOKENS_PER_CALL
 
@@ -377,7 +377,11 @@ PyObject *shard_list(PyObject *self, PyObject *name, size_t n) {
 PyObject *forward_group(const plan_t &p, PyObject *self, const at::Tensor &x) {
     const size_t n = p.shards.size();
     const int64_t B = x.numel() / p.in;
-    NONE_UNLESS(B >= 1 && B <= MOST_TOKENS && (!p.two_stage || B <= 64));
+    NONE_UNLESS(B >= 1 && B <= MOST_TOKENS);
+    // stacked shards at many tokens: the conditions of MergedTrellisLinear._grouped_rvq2_many_ok
+    if (p.two_stage && B > 64)
+        NONE_UNLESS(B <= std::min(setting(s_tmax, 0), setting(s_smax, 0)) && PyDict_GetItem(g_ext, s_dense) == Py_False &&
+                    PyDict_GetItem(g_ext, s_fuse) == Py_True);
     PyObject *svs = shard_list(self, s_SV, n), *sus = shard_list(self, s_SU, n), *ps = shard_list(self, s_tp, n), *ps2 = shard_list(self, s_tp2, n);
     NONE_UNLESS(svs && sus && ps && ps2);
     glqh_trellis_shard sh[GLQH_MAX_SHARDS] = {};
@@ -711,7 +715,7 @@ PyMODINIT_FUNC PyInit__glq_host(void) {
         {&s_buffers, "_buffers"}, {&s_SV, "SV"}, {&s_SU, "SU"}, {&s_tp, "trellis_packed"}, {&s_tp2, "trellis_packed2"},
         {&s_tlut, "tlut"}, {&s_bias, "bias"}, {&s_codebook, "codebook"}, {&s_codebook2, "codebook2"}, {&s_shards, "_shard_data"},
         {&s_q[0], "Qidxs"}, {&s_q[1], "Qidxs2"}, {&s_q[2], "Qidxs3"}, {&s_q[3], "Qidxs4"}, {&s_dense, "TRELLIS_DENSE"},
-        {&s_tmax, "TRELLIS_BATCH_MAX"}, {&s_smax, "TRELLIS_STACKED_BATCH_MAX"}, {&s_fold, "E8_FOLD"}, {&s_emax, "E8_BATCH_MAX"},
+        {&s_fuse, "TRELLIS_FUSE_STAGES"}, {&s_tmax, "TRELLIS_BATCH_MAX"}, {&s_smax, "TRELLIS_STACKED_BATCH_MAX"}, {&s_fold, "E8_FOLD"}, {&s_emax, "E8_BATCH_MAX"},
         {&s_efmax, "E8_FOLD_BATCH_MAX"}};
     for (auto &n : names)
         if (!(*n.p = PyUnicode_InternFromString(n.s))) return nullptr;

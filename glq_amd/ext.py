@@ -48,6 +48,8 @@ TRELLIS_BATCH_MAX = max(1, int(os.environ.get("GLQ_TRELLIS_BATCH_MAX", "8192")))
 # 766 / 597 at 4096, 1581 / 1191 and 1528 / 1051 at 8192 (4096 x 4096: 126 / 140 at 2048, 229 / 203 at 4096).
 # They take the library route above the smaller of the two limits.
 TRELLIS_STACKED_BATCH_MAX = max(1, int(os.environ.get("GLQ_TRELLIS_BATCH_MAX", "2048")))
+# the library decodes both stages of a stacked layer into one operand (it reads the same variable)
+TRELLIS_FUSE_STAGES = not os.environ.get("GLQ_TRELLIS_FUSE_STAGES", "").startswith("0")
 # GLQ_TRELLIS_DENSE (set to anything) sends every fused trellis call to that dense route, the
 # reference's A/B switch of the same name (glq/csrc/glq_trellis.cu:1023-1029, 1269).
 TRELLIS_DENSE = "GLQ_TRELLIS_DENSE" in os.environ
@@ -475,12 +477,12 @@ class _TrellisStage2(C.Structure):
 
 def glq_fused_linear_trellis_3inst_group_rvq2(x, shards, blocks_n, blocks_n_meta, in_features, n_pad,
                                               out_dtype=None):
-    """The grouped call for stacked (two-stage) layers at 1..64 tokens: the decode step of fused q/k/v or
+    """The grouped call for stacked (two-stage) layers: fused q/k/v or
     gate/up of a 5-8 bpw checkpoint, whose per-shard loop in the reference is
     fused_linear_trellis_3inst_yrht_rvq2 per shard + output_rht_shards (glq_vllm/linear_method.py:664-710).
-    One token: one decode launch for both streams of every shard; 2..64: one transform launch per distinct
-    sign vector and one decode launch per shard (the small-batch kernel to 16 tokens, the small-tile kernel
-    above); one finishing launch either way.
+    One token: one decode launch for both streams of every shard; 2..16: one transform launch for all sign
+    vectors and one decode launch per shard (the small-batch kernel); above: one launch of the tile kernel over
+    the row tiles of all shards; one finishing launch.
 
     shards: sequence of (sv, su, trellis_packed, trellis_packed2, wscale, inv_resid_scale2, out_features,
     m_pad); first stages of 4 bpw, second stages of one common rate.  Returns (B, sum(out_features)).

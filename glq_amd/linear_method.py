@@ -239,6 +239,13 @@ class MergedTrellisLinear:
         return ({self.trellis_packed.get_shard(i).shape[1] for i in n} == {64} and
                 len({self.trellis_packed2.get_shard(i).shape[1] for i in n}) == 1)
 
+    def _grouped_rvq2_many_ok(self, B):
+        """The same shards at more tokens, up to those from which a whole linear decompresses and multiplies with the
+        library."""
+        from . import ext
+        return B > 64 and B <= min(ext.TRELLIS_BATCH_MAX, ext.TRELLIS_STACKED_BATCH_MAX) and not ext.TRELLIS_DENSE and \
+            ext.TRELLIS_FUSE_STAGES and self._grouped_rvq2_ok(64)
+
     def _make_native(self, ext, two_stage):
         if self._fast is None:
             m0 = self._glq_trellis_meta[0]
@@ -249,7 +256,8 @@ class MergedTrellisLinear:
     def _apply_2d(self, x):
         _apply = E8RHTLinear._trellis_linear_apply
         metas = self._glq_trellis_meta
-        if _GLQ_MERGED_GROUPED and x.dtype in (torch.float16, torch.bfloat16) and self._grouped_rvq2_ok(x.shape[0]):
+        if _GLQ_MERGED_GROUPED and x.dtype in (torch.float16, torch.bfloat16) and \
+                (self._grouped_rvq2_ok(x.shape[0]) or self._grouped_rvq2_many_ok(x.shape[0])):
             from . import ext
             m0 = metas[0]
             self._make_native(ext, True)
@@ -268,9 +276,9 @@ class MergedTrellisLinear:
                 m0["_bn"], m0["_bnm"], m0["in"], m0["n_pad"], out_dtype=x.dtype)
         if self.glq_is_fused:
             s4b = self._glq_s4b
-            # from 64 tokens on, shards the grouped call does not take (stacked, mixed, more than four) run as
-            # whole fused linears, concatenated: their sums stay fp16 between the tile kernel and the output
-            # transform and stacked shards take the library route above 2048 tokens, which a shared fp32 y_rht
+            # from 64 tokens on, shards the grouped calls do not take (mixed, more than four, stacked ones at more than
+            # 2048 tokens) run as whole fused linears, concatenated: their sums stay fp16 between the tile kernel and
+            # the output transform and stacked shards take the library route above 2048 tokens, which a shared fp32 y_rht
             # rules out (gate/up 4096 -> 2 x 14336 at 6 bpw, 512 / 2048 / 4096 tokens: 334 / 1262 / 2407 -> 251 /
             # 935 / 1509 us; q/k/v 160 / 339 / 634 -> 116 / 247 / 436)
             whole = _GLQ_MERGED_GROUPED and x.shape[0] >= 64

@@ -75,8 +75,10 @@ def test_grouped_many_tokens(ms, n, B, K, shared_sv):
     ((2048, 512, 512), 2048, 17, (4,), False), ((1088, 32), 2368, 32, (3,), True), ((160, 320, 2336, 64), 1088, 33, (2,), False),
     ((11008, 96), 576, 64, (4,), False), ((512, 1088), 704, 20, (4, 2), False), ((2048, 512, 512), 2048, 64, (4, 4), True),
     ((160, 96), 128, 37, (4, 1), False),
+    ((512, 1088), 704, 65, (4, 2), False), ((2048, 512, 512), 2048, 200, (4, 4), False), ((1184, 96), 2368, 300, (4, 3), True),
+    ((4096, 32), 576, 700, (4, 1), False),
 ])
-def test_grouped_few_dozen_tokens(ms, n, B, bits, shared_sv):
+def test_grouped_few_dozen_tokens_and_stacked_layers(ms, n, B, bits, shared_sv):
     from glq_amd import ext, hadamard as H
     say("grouped few dozen tokens", ms, n, B, bits, shared_sv)
     layers, bn, bn_meta = _layers(ms, n, bits[0], 3, shared_sv)
