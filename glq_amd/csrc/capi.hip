@@ -45,6 +45,10 @@ static int e8_tile_ks(int64_t m_pad, int64_t n_pad, int64_t B, int nstages, bool
 int glqh_trellis_mma_fusein_plan(int64_t wgs_rows, int64_t k, int64_t B, int *S_out, int *ksplit_out);
 int glqh_launch_trellis_mma_rvq(const void *x_f16, int64_t B, const void *packed, const void *packed2, int R2, float rs2,
                                 int64_t m, int64_t k, int S, int ksplit, float *part, hipStream_t stream);
+int64_t glqh_trellis_mma_group_rows(const int64_t m[], int n);
+int glqh_launch_trellis_mma_group(const f16 *const x[], int64_t B, const void *const packed[], int R,
+                                  const void *const packed2[], int R2, const float rs2[], const int64_t m[], int n, int64_t k,
+                                  int S, int ksplit, float *const part[], hipStream_t stream);
 int glqh_launch_trellis_mma_fusein_rvq(const void *const packed[], const void *const packed2[], int R2, const float rs2[],
                                        const void *const sv[], float *const part[], const int64_t m[], int n_layers,
                                        const void *x, int x_dtype, int64_t x_stride, int64_t k, int64_t in_features,
@@ -703,28 +707,28 @@ extern "C" int glqh_fused_linear_trellis_3inst_noalloc(
 }
 
 // ---- grouped trellis linears -------------------------------------------------------
-// Two to four tokens on a large group: every workgroup of the fused-input launch repeats the
-// transform of all tokens, and one transform launch + one plain GEMV per layer is faster
-// (gate/up 4096 -> 2 x 14336 at four tokens: 63 us folded, 46 us as separate per-layer calls).
-static bool tr_group_plain(int64_t total_m_pad, int64_t n_pad, int64_t B) {
+// Few tokens of a group: one transform launch and one launch of the small-batch kernel over the strips of all layers, or
+// the fused-input launch, every workgroup of which repeats the transform of all tokens for its K slot (as many terms per
+// element as its Hadamard block has slices).  Whole grouped call, kernel us, folded / separate:
+//   4 bits, 1 token   2048-wide q/k/v 10.3 / 13.9, 3072 13.9 / 14.0, 4096 17.4 / 17.6, 5248 20.1 / 18.0, 8192 30.0 / 28.3;
+//                     gate/up 2048 -> 2 x 11008 17.0 / 20.2, 3392 -> 2 x 7040 20.8 / 20.0, 4096 -> 2 x 8192 22.6 / 23.2
+//   4 + 2, 1 token    3072 16.6 / 17.0, 4096 23.1 / 21.2, 5248 26.5 / 23.5; 3392 -> 2 x 7040 30.0 / 27.5
+//   4 bits, 2 tokens  960 14.3 / 12.2, 2048 12.8 / 13.3, 3072 18.3 / 14.4; 1024 -> 2 x 2560 11.6 / 12.8,
+//                     2048 -> 2 x 11008 19.6 / 20.9, 3392 -> 2 x 7040 25.1 / 20.8
+//   4 bits, 4 tokens  960 18.0 / 12.6, 2048 15.8 / 13.4; 2048 -> 2 x 11008 22.5 / 21.5
+// and one token of single-stage groups above 96M weights (4096 -> 2 x 14336: 37.4 / 33.9), below 32M (11008 -> 2048, a
+// group of one: 14.3 / 18) never.  The fused-input launches
+// serve up to four tokens, one of stacked layers.
+static bool tr_group_plain(int64_t total_m_pad, int64_t n_pad, int64_t B, bool stacked) {
+    if (!tr_fuse_input_enabled() || B > 4 || (stacked && B > 1)) return true;
     const int64_t w = total_m_pad * n_pad;
-    // q/k/v of a 4096-wide model (25M weights): 22.1 / 25.6 / 28.5 us folded at 2 / 3 / 4 tokens,
-    // 24.5 / 24.5 / 25.1 us separate; gate/up 2048 -> 2 x 11008 (45M): 19-22 us folded, 25-26 separate
-    // Checked on nine other groups (q/k/v and gate/up of 2048- to 8192-wide models, 1-4 tokens, folded /
-    // separate, us): one token folds with a gain of 5-8 us up to 50M weights (gate/up 3072 -> 2 x 8192: 18.1 /
-    // 24.4) and loses above 96M (4096 -> 2 x 14336: 37.4 / 33.9; 8192 -> 2 x 28672: 103.9 / 92.3; 5120 -> 2 x 13824
-    // ties); three and four tokens on q/k/v of a 3072-wide model lose 1-4 us folded (21.7 / 20.5, 24.4 / 20.2),
-    // which the rule below does not catch.
-    if (!tr_fuse_input_enabled()) return true;
-    if (B > 4) return true;                                  // 5..16 tokens: the fused-input launches serve up to four
-    if (B == 1) return w > ((int64_t)96 << 20);
-    return w > ((int64_t)48 << 20) || (B >= 3 && n_pad >= 4096 && w > ((int64_t)16 << 20));
+    if (B == 1) return (n_pad > 3072 && (stacked || n_pad != 4096) && w > ((int64_t)32 << 20)) || (!stacked && w > ((int64_t)96 << 20));
+    return B > 2 || n_pad > 2048 || (n_pad & (n_pad - 1)) != 0;
 }
 // The grouped call at many tokens: more than 64 tokens, at most four layers.  The K split of a group is at most
 // that of a single 128-row layer of the same width (fewer row tiles, more slots).
 constexpr int64_t TR_GROUP_MANY_MIN = 64;
-// 5..16 tokens: one transform launch per distinct sign vector, one small-batch decode launch per layer under the
-// K plan of the tallest, one finishing launch for all layers (no K-slot sum launches, no shared fp32 buffer)
+// up to 16 tokens: the small-batch kernel; above: the tile kernels
 constexpr int64_t TR_GROUP_SMALL_MAX = 16;
 constexpr int TR_GROUP_MANY_MAX = 4;
 constexpr int64_t TT_GROUP_ROWS_FLOOR = 128;
@@ -774,23 +778,13 @@ extern "C" size_t glqh_fused_linear_trellis_group_workspace_bytes(int64_t B, int
     int ks2 = 0;
     if (!glqh_trellis_fusein_plan(total_m_pad, n_pad, B, &steps, &ks)) return 0;
     if (glqh_trellis_mma_fusein_plan((total_m_pad + 63) / 64, n_pad, B, &steps, &ks2) && ks2 > ks) ks = ks2;
-    // the separate-transform route of large groups: slots of the plain plan (at most 64) and x_rht
+    // the separate-transform route (of stacked layers, which takes it at the least): slots of the plain plan (at most 64)
+    // and x_rht
     size_t plain = 0;
-    if (tr_group_plain(total_m_pad, n_pad, B))
+    if (tr_group_plain(total_m_pad, n_pad, B, false) || tr_group_plain(total_m_pad, n_pad, B, true))
         plain = (size_t)n_shards * align256((size_t)B * n_pad * sizeof(f16)) + align256((size_t)64 * B * total_m_pad * sizeof(float));
     const size_t fused = align256((size_t)ks * B * total_m_pad * sizeof(float));
-    // (2..4 tokens of stacked layers, glqh_fused_linear_trellis_3inst_group_rvq2: x_rht and the sums under the K
-    // plan of the tallest layer, which has at least total / n_shards rows)
-    size_t stacked = 0;
-    if (B > 1) {
-        int S = 0, ksb = 0;
-        const int64_t mmin = total_m_pad / n_shards / 32 * 32;
-        glqh_trellis_mma_plan(mmin < 32 ? 32 : mmin, n_pad, &S, &ksb);
-        stacked = (size_t)n_shards * align256((size_t)B * n_pad * sizeof(f16)) +
-                  align256((size_t)ksb * B * total_m_pad * sizeof(float));
-    }
-    const size_t most = plain > fused ? plain : fused;
-    return (size_t)n_shards * 256 + (stacked > most ? stacked : most);
+    return (size_t)n_shards * 256 + (plain > fused ? plain : fused);
 }
 
 // the second stage of stacked layer i of a group (first: it sets the group's rate *R2)
@@ -1076,12 +1070,9 @@ static int tr_group_decode(const void *x, int x_dtype, int64_t x_stride, int64_t
     if (B > TR_GROUP_SMALL_MAX)
         return tr_group_tiles(x, x_dtype, x_stride, B, sv, packed, R, nullptr, 0, nullptr, n_shards, blocks_n, n_blocks_n, bn_meta_dev,
                               in_features, n_pad, ws, ws_bytes, st, c);
-    if (tr_group_plain(total, n_pad, B)) {
-        // one K plan for all layers (that of the tallest), so that the finishing launch sees one slot count
-        int64_t mmax = 0;
-        for (int i = 0; i < n_shards; ++i) mmax = c->m_pads[i] > mmax ? c->m_pads[i] : mmax;
+    if (tr_group_plain(total, n_pad, B, false)) {
         int S = 0;
-        glqh_trellis_mma_plan(mmax, n_pad, &S, &ks);
+        glqh_trellis_mma_plan(glqh_trellis_mma_group_rows(c->m_pads, n_shards), n_pad, &S, &ks);
         const size_t xb = align256((size_t)B * n_pad * sizeof(f16));
         const size_t need = (size_t)n_shards * xb + align256((size_t)ks * B * total * sizeof(float));
         GLQH_REQUIRE(ws && ws_bytes >= need, "trellis group: workspace of %zu bytes needed, got %zu", need, ws_bytes);
@@ -1095,10 +1086,8 @@ static int tr_group_decode(const void *x, int x_dtype, int64_t x_stride, int64_t
         for (int i = 0; i < n_shards; ++i) {
             c->parts[i] = p;
             p += (size_t)ks * B * c->m_pads[i];
-            if (glqh_launch_trellis_mma(x_of[i], B, packed[i], R, c->m_pads[i], n_pad, S, ks, c->parts[i], 0, 1.0f, 0, 0, st))
-                return 1;
         }
-        return 0;
+        return glqh_launch_trellis_mma_group(x_of, B, packed, R, nullptr, 0, nullptr, c->m_pads, n_shards, n_pad, S, ks, c->parts, st);
     }
     const int fi_mode = tr_group_plan(c->m_pads, n_shards, n_pad, B, &steps, &ks);
     GLQH_REQUIRE(fi_mode != 0, "trellis group: shape not eligible");
@@ -1201,13 +1190,11 @@ extern "C" int glqh_fused_linear_trellis_3inst_group_rvq2(const void *x, int x_d
             return 1;
         return tr_group_finish(c, n_shards, B, y_dtype, y_stride, st);
     }
-    if (B > 1) {
-        // 2..16 tokens: one transform launch per distinct sign vector, one small-batch launch per layer that decodes
-        // both streams against the staged activations, under the K plan of the tallest layer, one finishing launch
-        int64_t mmax = 0;
-        for (int i = 0; i < n_shards; ++i) mmax = c.m_pads[i] > mmax ? c.m_pads[i] : mmax;
+    if (tr_group_plain(total, n_pad, B, true)) {
+        // one transform launch, one launch of the small-batch kernel over the strips of all layers that
+        // decodes both streams against the staged activations, one finishing launch
         int S = 0;
-        glqh_trellis_mma_plan(mmax, n_pad, &S, &ks);
+        glqh_trellis_mma_plan(glqh_trellis_mma_group_rows(c.m_pads, n_shards), n_pad, &S, &ks);
         const size_t xb = align256((size_t)B * n_pad * sizeof(f16));
         const size_t need = (size_t)n_shards * xb + align256((size_t)ks * B * total * sizeof(float));
         GLQH_REQUIRE(ws && ws_bytes >= need, "trellis two-stage group: workspace of %zu bytes needed, got %zu", need, ws_bytes);
@@ -1219,11 +1206,9 @@ extern "C" int glqh_fused_linear_trellis_3inst_group_rvq2(const void *x, int x_d
         for (int i = 0; i < n_shards; ++i) {
             c.parts[i] = p;
             p += (size_t)ks * B * c.m_pads[i];
-            glqh_range range("dequant_matmul");
-            if (glqh_launch_trellis_mma_rvq(x_of[i], B, packed[i], packed2[i], R2, rs2[i], c.m_pads[i], n_pad, S, ks,
-                                            c.parts[i], st))
-                return 1;
         }
+        if (glqh_launch_trellis_mma_group(x_of, B, packed, 4, packed2, R2, rs2, c.m_pads, n_shards, n_pad, S, ks, c.parts, st))
+            return 1;
         return glqh_launch_output_rht_group(c.parts, c.su, c.ys, c.scale, c.m_pads, c.outs, n_shards, y_dtype, y_stride,
                                             B, ks, st);
     }

@@ -75,12 +75,14 @@ def test_grouped_many_tokens(ms, n, B, K, shared_sv):
     ((2048, 512, 512), 2048, 17, (4,), False), ((1088, 32), 2368, 32, (3,), True), ((160, 320, 2336, 64), 1088, 33, (2,), False),
     ((11008, 96), 576, 64, (4,), False), ((512, 1088), 704, 20, (4, 2), False), ((2048, 512, 512), 2048, 64, (4, 4), True),
     ((160, 96), 128, 37, (4, 1), False),
+    ((160, 32, 96), 3392, 1, (4, 2), False), ((1088, 96), 5248, 1, (3,), True), ((2048, 512, 512), 2048, 2, (4, 4), False),
+    ((96, 160, 32, 64), 960, 4, (4,), False), ((1056, 64), 2368, 5, (2,), False), ((320, 1088, 32), 704, 16, (4, 1), True),
     ((512, 1088), 704, 65, (4, 2), False), ((2048, 512, 512), 2048, 200, (4, 4), False), ((1184, 96), 2368, 300, (4, 3), True),
     ((4096, 32), 576, 700, (4, 1), False),
 ])
-def test_grouped_few_dozen_tokens_and_stacked_layers(ms, n, B, bits, shared_sv):
+def test_grouped_calls_against_single_layers(ms, n, B, bits, shared_sv):
     from glq_amd import ext, hadamard as H
-    say("grouped few dozen tokens", ms, n, B, bits, shared_sv)
+    say("grouped call", ms, n, B, bits, shared_sv)
     layers, bn, bn_meta = _layers(ms, n, bits[0], 3, shared_sv)
     x = (torch.randn(B, n, generator=torch.Generator().manual_seed(5)) * 0.7).to(torch.bfloat16).to(DEV)
     sv0 = t(layers[0]["sv"])
