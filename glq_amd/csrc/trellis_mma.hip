@@ -923,6 +923,12 @@ int glqh_trellis_mma_plan(int64_t m, int64_t k, int *S_out, int *ksplit_out) {
     if (ks < 1) ks = 1;
     int64_t S = (nkp + ks - 1) / ks;
     S = (S + TR_WAVES - 1) / TR_WAVES * TR_WAVES;
+    // Short slots cost the finishing launch more than they save here: at least two k-pairs per wave, and four where that
+    // still leaves two workgroups per CU or many slots (whole linear, 4 bits, 4 / 16 tokens, kernel us, S = 4 or 8 -> here:
+    // 2048 x 2048 13.0 / 14.1 -> 12.8 / 12.9, 4096 x 4096 17.2 / 20.6 -> 14.9 / 16.8, 2048 x 11008 18.4 / 21.1 -> 16.4 /
+    // 19.7, 1024 x 8192 17.3 / 19.7 -> 13.2 / 14.5).
+    if (S < 2 * TR_WAVES) S = 2 * TR_WAVES;
+    if (S < 4 * TR_WAVES && nkp > 8 * S && wgs * ((nkp + S - 1) / S) >= (int64_t)glqh_device_cus() * 2) S = 4 * TR_WAVES;
     *S_out = (int)S;
     *ksplit_out = (int)((nkp + S - 1) / S);
     return 1;
