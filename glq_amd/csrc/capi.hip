@@ -13,7 +13,7 @@ int glqh_rht_init(void);
 int glqh_e8_init(void);
 int glqh_launch_trellis_decompress(const void *packed, int R, int64_t m, int64_t k, void *out,
                                    hipStream_t stream);
-int glqh_trellis_mma_plan(int64_t m, int64_t k, int *S_out, int *ksplit_out);
+extern "C" int glqh_trellis_mma_plan(int64_t m, int64_t k, int *S_out, int *ksplit_out);
 int glqh_launch_trellis_mma(const void *x_f16, int64_t B, const void *packed, int R, int64_t m, int64_t k,
                             int S, int ksplit, float *part, int direct, float scale, int accum,
                             int64_t out_stride, hipStream_t stream);
@@ -740,6 +740,19 @@ static int tr_group_plan(const int64_t *m_pads, int n_shards, int64_t n_pad, int
     return tr_fusein_plan(m_pads, n_shards, n_pad, B, steps, ks);
 }
 
+// Most K slots that a group of these rows gets from the small-batch kernel's plan.  Layers are whole 64-row strips
+// there, so the group has between total / 64 and total / 64 + n / 2 of them, and the plan is asked for each count:
+// its slots are not monotonic in the rows (2560 -> 2 x 5248: 5 slots at the mean layer's rows, 7 at the group's).
+static int tr_group_small_slots(int64_t total_m_pad, int64_t n_pad, int n_shards) {
+    int most = 1;
+    for (int64_t strips = (total_m_pad + 63) / 64; strips * 64 <= total_m_pad + 32 * (int64_t)n_shards; ++strips) {
+        int S = 0, ks = 0;
+        glqh_trellis_mma_plan(strips * 64, n_pad, &S, &ks);
+        if (ks > most) most = ks;
+    }
+    return most;
+}
+
 extern "C" size_t glqh_fused_linear_trellis_group_workspace_bytes(int64_t B, int64_t n_pad, int64_t total_m_pad,
                                                                   int n_shards) {
     if (B > TR_GROUP_MANY_MIN && n_shards >= 1 && n_shards <= TR_GROUP_MANY_MAX && total_m_pad >= 32 && n_pad >= 64) {
@@ -763,15 +776,9 @@ extern "C" size_t glqh_fused_linear_trellis_group_workspace_bytes(int64_t B, int
         return (size_t)n_shards * (256 + align256(glqh_trellis_tile_xb_bytes(n_pad, B))) +
                align256((size_t)B * n_pad * sizeof(f16)) + align256((size_t)ksb * B * total_m_pad * sizeof(float));
     }
-    if (B > 4) {
-        // x_rht and the partial sums under the K plan of the tallest layer, which has at least total / n_shards
-        // rows (the plan's slot count does not grow with the rows)
-        int S = 0, ksb = 0;
-        const int64_t mmin = total_m_pad / n_shards / 32 * 32;
-        glqh_trellis_mma_plan(mmin < 32 ? 32 : mmin, n_pad, &S, &ksb);
+    if (B > 4)
         return (size_t)n_shards * (256 + align256((size_t)B * n_pad * sizeof(f16))) +
-               align256((size_t)ksb * B * total_m_pad * sizeof(float));
-    }
+               align256((size_t)tr_group_small_slots(total_m_pad, n_pad, n_shards) * B * total_m_pad * sizeof(float));
     int steps = 0, ks = 0;
     // upper bound over how the rows may be split among the layers: the most workgroups (and
     // so the fewest K slots) arise from many short layers, the most slots from one tall layer

@@ -913,8 +913,9 @@ int mma_init_R() {
 }  // namespace
 
 // K slots: S k-pairs (32 columns) each, a multiple of the wave count, chosen from the
-// layer shape only; about four workgroups per CU.
-int glqh_trellis_mma_plan(int64_t m, int64_t k, int *S_out, int *ksplit_out) {
+// layer shape only; about four workgroups per CU.  The slot count is NOT monotonic in the rows: a taller layer may
+// start at a longer slot and miss the step to four k-pairs per wave, and then has more of them.
+extern "C" int glqh_trellis_mma_plan(int64_t m, int64_t k, int *S_out, int *ksplit_out) {
     const int64_t nkp = k / 32;
     const int64_t wgs = (m + 63) / 64;
     const int64_t target = (int64_t)glqh_device_cus() * 4;

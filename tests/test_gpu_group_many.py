@@ -79,6 +79,8 @@ def test_grouped_many_tokens(ms, n, B, K, shared_sv):
     ((96, 160, 32, 64), 960, 4, (4,), False), ((1056, 64), 2368, 5, (2,), False), ((320, 1088, 32), 704, 16, (4, 1), True),
     ((512, 1088), 704, 65, (4, 2), False), ((2048, 512, 512), 2048, 200, (4, 4), False), ((1184, 96), 2368, 300, (4, 3), True),
     ((4096, 32), 576, 700, (4, 1), False),
+    # rows between those of one layer and of the group change the K plan: widths 2112..3072 at 5..16 tokens
+    ((5248, 5248), 2560, 8, (4,), False), ((4096, 4096), 3072, 16, (4, 2), False), ((3072, 3072, 3072), 2816, 5, (2,), True),
 ])
 def test_grouped_calls_against_single_layers(ms, n, B, bits, shared_sv):
     from glq_amd import ext, hadamard as H
