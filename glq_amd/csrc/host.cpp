@@ -14,6 +14,7 @@
 #include <dlfcn.h>
 
 #include <algorithm>
+#include <array>
 #include <vector>
 
 #include <ATen/ATen.h>
@@ -57,7 +58,8 @@ constexpr int64_t MOST_TOKENS = 32768;                         // _MAX_TOKENS_PE
 const c10::DispatchKeySet PLAIN({c10::DispatchKey::CUDA, c10::DispatchKey::ADInplaceOrView, c10::DispatchKey::AutogradCUDA,
                                   c10::DispatchKey::AutocastCUDA});
 
-// an ordinary contiguous GPU tensor of this type, or null
+// An ordinary contiguous GPU tensor of this type, or null.  The pointer is good while this thread has the GIL: a layer's
+// buffers can be replaced by another thread once a call gives it up, so what a call reads after that it holds by value.
 const at::Tensor *gpu(PyObject *o, at::ScalarType dt) {
     if (!o || !THPVariable_CheckExact(o)) return nullptr;
     const at::Tensor &t = THPVariable_Unpack(o);
@@ -178,9 +180,16 @@ PyObject *guarded(F f) {
     return nullptr;
 }
 
+// The tensors of one layer, by value; false where one of them is not what the call recognises.
+bool hold(PyObject *o, at::ScalarType dt, at::Tensor *to) {
+    const at::Tensor *t = gpu(o, dt);
+    if (t) *to = *t;
+    return t != nullptr;
+}
+
 // ---- one trellis linear ------------------------------------------------------------------
 struct trellis_layer {
-    const at::Tensor *sv, *su, *packed, *packed2;              // packed2: null without a second stage
+    at::Tensor sv, su, packed, packed2;                        // packed2: undefined without a second stage
     const int64_t *bn, *bm;
     int64_t n_bn, n_bm;
     const glqh_block_meta *bn_meta, *bm_meta;
@@ -193,9 +202,10 @@ PyObject *run_trellis(const at::Tensor &x, const trellis_layer &l, at::ScalarTyp
     NONE_UNLESS(B >= 1 && B <= MOST_TOKENS);
     NONE_UNLESS(PyDict_GetItem(g_ext, s_dense) == Py_False);
     int64_t most = setting(s_tmax, 0);
-    if (l.packed2) most = std::min(most, setting(s_smax, 0));
-    NONE_UNLESS(B <= most && l.packed->dim() == 2 && (!l.packed2 || l.packed2->dim() == 2));
-    NONE_UNLESS(same_device(x, {l.sv, l.su, l.packed, l.packed2}));
+    const bool two = l.packed2.defined();
+    if (two) most = std::min(most, setting(s_smax, 0));
+    NONE_UNLESS(B <= most && l.packed.dim() == 2 && (!two || l.packed2.dim() == 2));
+    NONE_UNLESS(same_device(x, {&l.sv, &l.su, &l.packed, two ? &l.packed2 : nullptr}));
     return guarded([&]() -> PyObject * {
         c10::DeviceGuard guard(x.device());
         at::Tensor y = like(x, l.out, dt);
@@ -203,10 +213,9 @@ PyObject *run_trellis(const at::Tensor &x, const trellis_layer &l, at::ScalarTyp
         {
             no_gil unlocked;
             scratch ws(L.trellis_ws(B, l.n_pad, l.m_pad));
-            rc = L.trellis(x.const_data_ptr(), lib_type(x.scalar_type()), x.size(-1), B, l.sv->const_data_ptr(), l.su->const_data_ptr(),
-                           l.packed->const_data_ptr(), l.packed->size(0), l.packed->size(1),
-                           l.packed2 ? l.packed2->const_data_ptr() : nullptr, l.packed2 ? l.packed2->size(0) : 0,
-                           l.packed2 ? l.packed2->size(1) : 0, l.bn, l.n_bn, l.bm, l.n_bm, l.bn_meta, l.bm_meta, l.wscale, l.inv2,
+            rc = L.trellis(x.const_data_ptr(), lib_type(x.scalar_type()), x.size(-1), B, l.sv.const_data_ptr(), l.su.const_data_ptr(),
+                           l.packed.const_data_ptr(), l.packed.size(0), l.packed.size(1),
+                           two ? l.packed2.const_data_ptr() : nullptr, two ? l.packed2.size(0) : 0, two ? l.packed2.size(1) : 0, l.bn, l.n_bn, l.bm, l.n_bm, l.bn_meta, l.bm_meta, l.wscale, l.inv2,
                            l.in, l.out, l.n_pad, l.m_pad, y.mutable_data_ptr(), lib_type(dt), l.out, nullptr, 0, ws.p.get(), ws.bytes,
                            stream_of(x));
         }
@@ -220,12 +229,9 @@ PyObject *py_trellis_linear(PyObject *, PyObject *const *a, Py_ssize_t n) {
     NONE_UNLESS(n == 16 && !modes());
     const at::Tensor *x = activations(a[0]);
     NONE_UNLESS(x && x->dim() == 2);
-    trellis_layer l = {gpu(a[1], at::kHalf), gpu(a[2], at::kHalf), gpu(a[3], at::kShort), nullptr};
-    NONE_UNLESS(l.sv && l.su && l.packed);
-    if (a[4] != Py_None) {
-        l.packed2 = gpu(a[4], at::kShort);
-        NONE_UNLESS(l.packed2 && l.packed2->numel() > 0);
-    }
+    trellis_layer l;
+    NONE_UNLESS(hold(a[1], at::kHalf, &l.sv) && hold(a[2], at::kHalf, &l.su) && hold(a[3], at::kShort, &l.packed));
+    if (a[4] != Py_None) NONE_UNLESS(hold(a[4], at::kShort, &l.packed2) && l.packed2.numel() > 0);
     blocks bn, bm;
     NONE_UNLESS(bn.read(a[5]) && bm.read(a[6]));
     NONE_UNLESS(meta(a[7], bn.n, &l.bn_meta) && meta(a[8], bm.n, &l.bm_meta));
@@ -280,47 +286,49 @@ const glqh_block_meta *meta_ptr(const at::Tensor &t) { return t.defined() ? (con
 
 PyObject *item(PyObject *d, PyObject *name) { return PyDict_GetItem(d, name); }
 
-PyObject *add_bias(PyObject *y, PyObject *bias) {
-    if (!y || y == Py_None || !bias || bias == Py_None) return y;
+PyObject *add_bias(PyObject *y, const at::Tensor &bias) {
+    if (!y || y == Py_None || !bias.defined()) return y;
     return guarded([&]() -> PyObject * {
         c10::NoGradGuard no_grad;
         const at::Tensor &t = THPVariable_Unpack(y);
-        t.add_(THPVariable_Unpack(bias).to(t.scalar_type()));
+        t.add_(bias.to(t.scalar_type()));
         return y;
     });
 }
 
+// a layer's bias; undefined if it has none
+bool hold_bias(PyObject *buffers, at::Tensor *to) {
+    PyObject *b = item(buffers, s_bias);
+    return !b || b == Py_None || hold(b, at::kHalf, to);
+}
+
 PyObject *forward_trellis(const plan_t &p, PyObject *buffers, const at::Tensor &x) {
-    PyObject *tlut = item(buffers, s_tlut), *tp2 = item(buffers, s_tp2), *bias = item(buffers, s_bias);
+    PyObject *tlut = item(buffers, s_tlut), *tp2 = item(buffers, s_tp2);
     NONE_UNLESS(tlut && THPVariable_CheckExact(tlut) && THPVariable_Unpack(tlut).numel() == 0);
-    trellis_layer l = {gpu(item(buffers, s_SV), at::kHalf), gpu(item(buffers, s_SU), at::kHalf), gpu(item(buffers, s_tp), at::kShort), nullptr};
-    NONE_UNLESS(l.sv && l.su && l.packed && tp2 && THPVariable_CheckExact(tp2));
-    if (THPVariable_Unpack(tp2).numel() > 0) {
-        l.packed2 = gpu(tp2, at::kShort);
-        NONE_UNLESS(l.packed2);
-    }
-    NONE_UNLESS(!bias || bias == Py_None || gpu(bias, at::kHalf));
+    trellis_layer l;
+    at::Tensor bias;
+    NONE_UNLESS(hold(item(buffers, s_SV), at::kHalf, &l.sv) && hold(item(buffers, s_SU), at::kHalf, &l.su) &&
+                hold(item(buffers, s_tp), at::kShort, &l.packed) && tp2 && THPVariable_CheckExact(tp2));
+    if (THPVariable_Unpack(tp2).numel() > 0) NONE_UNLESS(hold(tp2, at::kShort, &l.packed2));
+    NONE_UNLESS(hold_bias(buffers, &bias));
     l.bn = p.bn.data(); l.n_bn = p.bn.size(); l.bm = p.bm.data(); l.n_bm = p.bm.size();
     l.bn_meta = l.n_bn > 1 ? meta_ptr(p.bn_meta) : nullptr;
     l.bm_meta = l.n_bm > 1 ? meta_ptr(p.bm_meta) : nullptr;
-    l.wscale = p.wscale; l.inv2 = l.packed2 ? p.inv[0] : 0.0; l.in = p.in; l.out = p.out; l.n_pad = p.n_pad; l.m_pad = p.m_pad;
+    l.wscale = p.wscale; l.inv2 = l.packed2.defined() ? p.inv[0] : 0.0; l.in = p.in; l.out = p.out; l.n_pad = p.n_pad; l.m_pad = p.m_pad;
     return add_bias(run_trellis(x, l, x.scalar_type()), bias);
 }
 
 PyObject *forward_shell(const plan_t &p, PyObject *self, PyObject *buffers, const at::Tensor &x) {
     NONE_UNLESS(item(self, s_codebook) == p.codebook[0] && item(self, s_codebook2) == p.codebook[1]);
     for (int i = 0; i < 2; ++i) NONE_UNLESS(!p.cb[i].defined() || (int64_t)p.cb[i]._version() == p.cb_version[i]);
-    const at::Tensor *q[4];
-    for (int i = 0; i < 4; ++i) {
-        q[i] = gpu(item(buffers, s_q[i]), at::kShort);
-        NONE_UNLESS(q[i] && !q[i]->is_inference() && q[i]->const_data_ptr() == p.q_data[i] && (int64_t)q[i]->_version() == p.q_version[i]);
-    }
-    const at::Tensor *sv = gpu(item(buffers, s_SV), at::kHalf), *su = gpu(item(buffers, s_SU), at::kHalf);
-    PyObject *bias = item(buffers, s_bias);
-    NONE_UNLESS(sv && su && (!bias || bias == Py_None || gpu(bias, at::kHalf)));
+    at::Tensor q[4], sv, su, bias;
+    for (int i = 0; i < 4; ++i)
+        NONE_UNLESS(hold(item(buffers, s_q[i]), at::kShort, q + i) && !q[i].is_inference() && q[i].const_data_ptr() == p.q_data[i] &&
+                    (int64_t)q[i]._version() == p.q_version[i]);
+    NONE_UNLESS(hold(item(buffers, s_SV), at::kHalf, &sv) && hold(item(buffers, s_SU), at::kHalf, &su) && hold_bias(buffers, &bias));
     const int64_t B = x.numel() / p.in;
-    NONE_UNLESS(B >= 1 && B <= MOST_TOKENS && q[0]->dim() == 2 && q[0]->size(0) == p.m_pad && q[0]->size(1) * 8 == p.n_pad);
-    NONE_UNLESS(same_device(x, {sv, su, q[0], &p.table[0]}));
+    NONE_UNLESS(B >= 1 && B <= MOST_TOKENS && q[0].dim() == 2 && q[0].size(0) == p.m_pad && q[0].size(1) * 8 == p.n_pad);
+    NONE_UNLESS(same_device(x, {&sv, &su, &q[0], &p.table[0]}));
     // the routes of ext._e8_dense_route: dequantize + library GEMM is Python's
     const int64_t plain_most = setting(s_emax, 0), fold_most = std::max(plain_most, setting(s_efmax, 0));
     glqh_e8_folded f = {};
@@ -347,13 +355,13 @@ PyObject *forward_shell(const plan_t &p, PyObject *self, PyObject *buffers, cons
     PyObject *y = guarded([&]() -> PyObject * {
         c10::DeviceGuard guard(x.device());
         at::Tensor out = like(x, p.out, x.scalar_type());
-        auto stage = [&](int s) { return s < p.stages ? q[s]->const_data_ptr() : nullptr; };
+        auto stage = [&](int s) { return s < p.stages ? q[s].const_data_ptr() : nullptr; };
         const bool t2 = p.stages >= 2;
         int rc;
         {
             no_gil unlocked;
             scratch ws(L.e8_ws(B, p.n_pad, p.m_pad));
-            rc = L.e8(x.const_data_ptr(), lib_type(x.scalar_type()), p.in, B, sv->const_data_ptr(), su->const_data_ptr(), stage(0), stage(1),
+            rc = L.e8(x.const_data_ptr(), lib_type(x.scalar_type()), p.in, B, sv.const_data_ptr(), su.const_data_ptr(), stage(0), stage(1),
                       stage(2), stage(3), (const uint32_t *)p.table[0].const_data_ptr(),
                       t2 ? (const uint32_t *)p.table[1].const_data_ptr() : nullptr, t2 ? p.table[1].size(0) : 0, p.wscale, p.inv[0],
                       p.inv[1], p.inv[2], p.bn.data(), p.bn.size(), p.bm.data(), p.bm.size(),
@@ -387,16 +395,20 @@ PyObject *forward_group(const plan_t &p, PyObject *self, const at::Tensor &x) {
     glqh_trellis_shard sh[GLQH_MAX_SHARDS] = {};
     glqh_trellis_stage2 s2[GLQH_MAX_SHARDS] = {};
     int64_t total_out = 0, total_m = 0;
+    std::array<at::Tensor, 4 * GLQH_MAX_SHARDS> keep;          // the lists can change once the GIL is given up
+    size_t kept = 0;
     for (size_t i = 0; i < n; ++i) {
         const at::Tensor *sv = gpu(PyList_GET_ITEM(svs, i), at::kHalf), *su = gpu(PyList_GET_ITEM(sus, i), at::kHalf);
         const at::Tensor *pk = gpu(PyList_GET_ITEM(ps, i), at::kShort);
         NONE_UNLESS(sv && su && pk && pk->dim() == 2 && pk->numel() > 0 && same_device(x, {sv, su, pk}));
+        for (const at::Tensor *t : {sv, su, pk}) keep[kept++] = *t;
         sh[i] = {sv->const_data_ptr(), su->const_data_ptr(), pk->const_data_ptr(), pk->size(0), pk->size(1), p.shards[i].wscale,
                  p.shards[i].out, p.shards[i].m_pad, nullptr};
         NONE_UNLESS(sh[i].packed_cols == sh[0].packed_cols);
         if (p.two_stage) {
             const at::Tensor *pk2 = gpu(PyList_GET_ITEM(ps2, i), at::kShort);
             NONE_UNLESS(pk2 && pk2->dim() == 2 && pk2->numel() > 0 && same_device(x, {pk2}));
+            keep[kept++] = *pk2;
             s2[i] = {pk2->const_data_ptr(), pk2->size(0), pk2->size(1), p.shards[i].inv2};
             NONE_UNLESS(sh[i].packed_cols == 64 && s2[i].packed2_cols == s2[0].packed2_cols);
         }
@@ -430,12 +442,13 @@ PyObject *forward_group(const plan_t &p, PyObject *self, const at::Tensor &x) {
 PyObject *plan_call(PyObject *self, PyObject *const *a, size_t nargs, PyObject *kw) {
     NONE_UNLESS(PyVectorcall_NARGS(nargs) == 2 && !kw && PyDict_CheckExact(a[0]) && !modes());
     const plan_t &p = *((Plan *)self)->p;
-    const at::Tensor *x = activations(a[1]);
-    NONE_UNLESS(x && x->dim() >= 1 && x->size(-1) == p.in && x->numel() > 0);
-    if (p.kind == GROUP) return forward_group(p, a[0], *x);
+    const at::Tensor *given = activations(a[1]);
+    NONE_UNLESS(given && given->dim() >= 1 && given->size(-1) == p.in && given->numel() > 0);
+    const at::Tensor x = *given;
+    if (p.kind == GROUP) return forward_group(p, a[0], x);
     PyObject *buffers = item(a[0], s_buffers);
     NONE_UNLESS(buffers && PyDict_Check(buffers));
-    return p.kind == TRELLIS ? forward_trellis(p, buffers, *x) : forward_shell(p, a[0], buffers, *x);
+    return p.kind == TRELLIS ? forward_trellis(p, buffers, x) : forward_shell(p, a[0], buffers, x);
 }
 
 void plan_free(PyObject *self) {

@@ -117,3 +117,51 @@ def test_dispatch_modes_take_the_python_route():
     with Count():
         assert lin._fast(lin.__dict__, x) is None
         assert torch.equal(lin(x), ref)
+
+
+@pytest.mark.parametrize("kind", ["trellis2", "shell2", "merged"])
+def test_buffers_replaced_by_another_thread_during_calls(kind):
+    """A thread that keeps replacing a layer's sign vector (and writing over memory of its size) while another one
+    calls the layer: every result is the one of a sign vector that the layer has had."""
+    import threading
+
+    from glq_amd import linear_method as LM
+    say("native forward, buffers replaced by another thread", kind)
+    x = torch.randn(3, 2304, generator=torch.Generator().manual_seed(2)).to(DEV, torch.bfloat16)
+    if kind == "merged":
+        lins = [_layer("trellis", m, 2304, False) for m in (512, 64)]
+        layer = LM.MergedTrellisLinear.from_linears(lins).process_weights_after_loading(DEV)
+        call, put = (lambda: layer.apply(x)), (lambda su: layer.SU._shard_data.__setitem__(0, su))
+        su = layer.SU.get_shard(0)
+    else:
+        layer = _layer(kind, 512, 2304, True)
+        layer.prepare()
+        call, put, su = (lambda: layer(x)), (lambda s: setattr(layer, "SU", s)), layer.SU
+    two = [su, -su]
+    refs = []
+    for s in two:
+        put(s)
+        call()                                                   # the first makes the native form
+        assert layer._fast(layer.__dict__, x) is not None
+        refs.append(call())
+    assert not torch.equal(*refs)
+    stop, failed = threading.Event(), []
+
+    def replace():
+        try:
+            i = 0
+            while not stop.is_set():
+                put(two[i & 1].clone())                          # the only reference: the one before it is freed
+                torch.full_like(su, float("nan"))
+                i += 1
+        except BaseException as e:                               # noqa: BLE001 - reported by the main thread
+            failed.append(e)
+    worker = threading.Thread(target=replace)
+    worker.start()
+    try:
+        got = [call() for _ in range(300)]
+    finally:
+        stop.set()
+        worker.join()
+    assert not failed, failed
+    assert all(torch.equal(y, refs[0]) or torch.equal(y, refs[1]) for y in got)
