@@ -18,6 +18,7 @@
 #include <vector>
 
 #include <ATen/ATen.h>
+#include <ATen/TracerMode.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/core/GradMode.h>
@@ -64,6 +65,7 @@ const at::Tensor *gpu(PyObject *o, at::ScalarType dt) {
     if (!o || !THPVariable_CheckExact(o)) return nullptr;
     const at::Tensor &t = THPVariable_Unpack(o);
     if (!t.defined() || t.scalar_type() != dt || (t.key_set() | PLAIN) != PLAIN || !t.is_cuda() || !t.is_contiguous()) return nullptr;
+    if (t.requires_grad() && c10::GradMode::is_enabled()) return nullptr;   // the operators say that they are not differentiable
     return &t;
 }
 
@@ -74,7 +76,8 @@ const at::Tensor *activations(PyObject *o) {
 
 int lib_type(at::ScalarType t) { return t == at::kHalf ? GLQH_F16 : t == at::kBFloat16 ? GLQH_BF16 : GLQH_F32; }
 
-bool modes() { return c10::impl::TorchDispatchModeTLS::any_modes_set(); }
+// a Python dispatch mode, or torch.jit.trace above the dispatcher: the call has to be seen as an operator
+bool modes() { return c10::impl::TorchDispatchModeTLS::any_modes_set() || at::tracer::impl::is_dispatch_enabled(); }
 
 bool integer(PyObject *o, int64_t *v) {
     if (!PyLong_CheckExact(o)) return false;

@@ -165,3 +165,26 @@ def test_buffers_replaced_by_another_thread_during_calls(kind):
         worker.join()
     assert not failed, failed
     assert all(torch.equal(y, refs[0]) or torch.equal(y, refs[1]) for y in got)
+
+
+@pytest.mark.parametrize("kind", ["trellis", "trellis2"])
+def test_tracing_and_gradients_see_the_operator(kind):
+    """torch.jit.trace records the operator, not its result, and an input that wants a gradient gets an output with the
+    autograd node that says that the operator has no derivative, instead of one that silently needs none."""
+    from glq_amd import custom_ops
+    say("native forward under tracing", kind)
+    custom_ops.register()
+    lin = _layer(kind, 64, 128, False)
+    g = torch.Generator().manual_seed(0)
+    x, other = (torch.randn(2, 128, generator=g).to(DEV, torch.bfloat16) for _ in range(2))
+    lin(x)
+    assert lin._fast(lin.__dict__, x) is not None
+    traced = torch.jit.trace(lin, x)
+    assert torch.equal(traced(other), lin(other))
+    assert any(n.kind().startswith("glq::") for n in traced.graph.nodes())
+    w = x.clone().requires_grad_()
+    assert lin._fast(lin.__dict__, w) is None
+    y = lin(w)
+    assert y.requires_grad and y.grad_fn is not None and torch.equal(y, lin(x))
+    with torch.no_grad():
+        assert lin._fast(lin.__dict__, w) is not None and not lin(w).requires_grad
