@@ -289,14 +289,17 @@ const glqh_block_meta *meta_ptr(const at::Tensor &t) { return t.defined() ? (con
 
 PyObject *item(PyObject *d, PyObject *name) { return PyDict_GetItem(d, name); }
 
+// y + bias in y's place; takes y's reference
 PyObject *add_bias(PyObject *y, const at::Tensor &bias) {
     if (!y || y == Py_None || !bias.defined()) return y;
-    return guarded([&]() -> PyObject * {
+    PyObject *sum = guarded([&]() -> PyObject * {
         c10::NoGradGuard no_grad;
         const at::Tensor &t = THPVariable_Unpack(y);
         t.add_(bias.to(t.scalar_type()));
         return y;
     });
+    if (!sum) Py_DECREF(y);                                    // the addition raised
+    return sum;
 }
 
 // a layer's bias; undefined if it has none

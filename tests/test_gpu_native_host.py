@@ -188,3 +188,17 @@ def test_tracing_and_gradients_see_the_operator(kind):
     assert y.requires_grad and y.grad_fn is not None and torch.equal(y, lin(x))
     with torch.no_grad():
         assert lin._fast(lin.__dict__, w) is not None and not lin(w).requires_grad
+
+
+def test_a_failing_bias_addition_keeps_no_output():
+    say("native forward, bias of a wrong length")
+    lin = _layer("trellis", 512, 2048, True)
+    x = torch.randn(64, 2048, generator=torch.Generator().manual_seed(0)).to(DEV, torch.bfloat16)
+    lin(x)
+    lin.bias = torch.zeros(511, device=DEV).half()
+    held = []
+    for _ in range(3):
+        with pytest.raises(RuntimeError, match="size"):
+            lin._fast(lin.__dict__, x)
+        held.append(torch.cuda.memory_allocated())
+    assert held[0] == held[1] == held[2]
