@@ -117,18 +117,12 @@ struct blocks {
     }
 };
 
-bool meta(PyObject *o, int64_t n_blocks, const glqh_block_meta **p) {
-    *p = nullptr;
-    if (n_blocks <= 1) return true;
-    const at::Tensor *t = gpu(o, at::kInt);
-    if (!t) return false;
-    *p = (const glqh_block_meta *)t->const_data_ptr();
-    return true;
-}
+const glqh_block_meta *meta_ptr(const at::Tensor &t) { return t.defined() ? (const glqh_block_meta *)t.const_data_ptr() : nullptr; }
 
+// undefined tensors are on every device
 bool same_device(const at::Tensor &x, std::initializer_list<const at::Tensor *> ts) {
     for (const at::Tensor *t : ts)
-        if (t && t->device() != x.device()) return false;
+        if (t->defined() && t->device() != x.device()) return false;
     return true;
 }
 
@@ -183,19 +177,22 @@ PyObject *guarded(F f) {
     return nullptr;
 }
 
-// The tensors of one layer, by value; false where one of them is not what the call recognises.
+// a tensor by value; false where it is not what the call recognises
 bool hold(PyObject *o, at::ScalarType dt, at::Tensor *to) {
     const at::Tensor *t = gpu(o, dt);
     if (t) *to = *t;
     return t != nullptr;
 }
 
+// the block table of a transform of several blocks
+bool hold_meta(PyObject *o, int64_t n_blocks, at::Tensor *to) { return n_blocks <= 1 || hold(o, at::kInt, to); }
+
 // ---- one trellis linear ------------------------------------------------------------------
 struct trellis_layer {
     at::Tensor sv, su, packed, packed2;                        // packed2: undefined without a second stage
+    at::Tensor bn_meta, bm_meta;                               // undefined for a single block
     const int64_t *bn, *bm;
     int64_t n_bn, n_bm;
-    const glqh_block_meta *bn_meta, *bm_meta;
     double wscale, inv2;
     int64_t in, out, n_pad, m_pad;
 };
@@ -208,7 +205,7 @@ PyObject *run_trellis(const at::Tensor &x, const trellis_layer &l, at::ScalarTyp
     const bool two = l.packed2.defined();
     if (two) most = std::min(most, setting(s_smax, 0));
     NONE_UNLESS(B <= most && l.packed.dim() == 2 && (!two || l.packed2.dim() == 2));
-    NONE_UNLESS(same_device(x, {&l.sv, &l.su, &l.packed, two ? &l.packed2 : nullptr}));
+    NONE_UNLESS(same_device(x, {&l.sv, &l.su, &l.packed, &l.packed2, &l.bn_meta, &l.bm_meta}));
     return guarded([&]() -> PyObject * {
         c10::DeviceGuard guard(x.device());
         at::Tensor y = like(x, l.out, dt);
@@ -218,7 +215,8 @@ PyObject *run_trellis(const at::Tensor &x, const trellis_layer &l, at::ScalarTyp
             scratch ws(L.trellis_ws(B, l.n_pad, l.m_pad));
             rc = L.trellis(x.const_data_ptr(), lib_type(x.scalar_type()), x.size(-1), B, l.sv.const_data_ptr(), l.su.const_data_ptr(),
                            l.packed.const_data_ptr(), l.packed.size(0), l.packed.size(1),
-                           two ? l.packed2.const_data_ptr() : nullptr, two ? l.packed2.size(0) : 0, two ? l.packed2.size(1) : 0, l.bn, l.n_bn, l.bm, l.n_bm, l.bn_meta, l.bm_meta, l.wscale, l.inv2,
+                           two ? l.packed2.const_data_ptr() : nullptr, two ? l.packed2.size(0) : 0, two ? l.packed2.size(1) : 0, l.bn, l.n_bn, l.bm, l.n_bm, meta_ptr(l.bn_meta),
+                           meta_ptr(l.bm_meta), l.wscale, l.inv2,
                            l.in, l.out, l.n_pad, l.m_pad, y.mutable_data_ptr(), lib_type(dt), l.out, nullptr, 0, ws.p.get(), ws.bytes,
                            stream_of(x));
         }
@@ -237,7 +235,7 @@ PyObject *py_trellis_linear(PyObject *, PyObject *const *a, Py_ssize_t n) {
     if (a[4] != Py_None) NONE_UNLESS(hold(a[4], at::kShort, &l.packed2) && l.packed2.numel() > 0);
     blocks bn, bm;
     NONE_UNLESS(bn.read(a[5]) && bm.read(a[6]));
-    NONE_UNLESS(meta(a[7], bn.n, &l.bn_meta) && meta(a[8], bm.n, &l.bm_meta));
+    NONE_UNLESS(hold_meta(a[7], bn.n, &l.bn_meta) && hold_meta(a[8], bm.n, &l.bm_meta));
     l.bn = bn.p; l.n_bn = bn.n; l.bm = bm.p; l.n_bm = bm.n;
     NONE_UNLESS(real(a[9], &l.wscale) && real(a[10], &l.inv2) && integer(a[11], &l.in) && integer(a[12], &l.out) &&
                 integer(a[13], &l.n_pad) && integer(a[14], &l.m_pad));
@@ -285,8 +283,6 @@ struct Plan {
     plan_t *p;
 };
 
-const glqh_block_meta *meta_ptr(const at::Tensor &t) { return t.defined() ? (const glqh_block_meta *)t.const_data_ptr() : nullptr; }
-
 PyObject *item(PyObject *d, PyObject *name) { return PyDict_GetItem(d, name); }
 
 // y + bias in y's place; takes y's reference
@@ -318,8 +314,8 @@ PyObject *forward_trellis(const plan_t &p, PyObject *buffers, const at::Tensor &
     if (THPVariable_Unpack(tp2).numel() > 0) NONE_UNLESS(hold(tp2, at::kShort, &l.packed2));
     NONE_UNLESS(hold_bias(buffers, &bias));
     l.bn = p.bn.data(); l.n_bn = p.bn.size(); l.bm = p.bm.data(); l.n_bm = p.bm.size();
-    l.bn_meta = l.n_bn > 1 ? meta_ptr(p.bn_meta) : nullptr;
-    l.bm_meta = l.n_bm > 1 ? meta_ptr(p.bm_meta) : nullptr;
+    if (l.n_bn > 1) l.bn_meta = p.bn_meta;
+    if (l.n_bm > 1) l.bm_meta = p.bm_meta;
     l.wscale = p.wscale; l.inv2 = l.packed2.defined() ? p.inv[0] : 0.0; l.in = p.in; l.out = p.out; l.n_pad = p.n_pad; l.m_pad = p.m_pad;
     return add_bias(run_trellis(x, l, x.scalar_type()), bias);
 }
@@ -334,7 +330,7 @@ PyObject *forward_shell(const plan_t &p, PyObject *self, PyObject *buffers, cons
     NONE_UNLESS(hold(item(buffers, s_SV), at::kHalf, &sv) && hold(item(buffers, s_SU), at::kHalf, &su) && hold_bias(buffers, &bias));
     const int64_t B = x.numel() / p.in;
     NONE_UNLESS(B >= 1 && B <= MOST_TOKENS && q[0].dim() == 2 && q[0].size(0) == p.m_pad && q[0].size(1) * 8 == p.n_pad);
-    NONE_UNLESS(same_device(x, {&sv, &su, &q[0], &p.table[0]}));
+    NONE_UNLESS(same_device(x, {&sv, &su, &q[0], &q[1], &q[2], &q[3], &p.table[0], &p.table[1], &p.bn_meta, &p.bm_meta}));
     // the routes of ext._e8_dense_route: dequantize + library GEMM is Python's
     const int64_t plain_most = setting(s_emax, 0), fold_most = std::max(plain_most, setting(s_efmax, 0));
     glqh_e8_folded f = {};
@@ -397,7 +393,7 @@ PyObject *forward_group(const plan_t &p, PyObject *self, const at::Tensor &x) {
         NONE_UNLESS(B <= std::min(setting(s_tmax, 0), setting(s_smax, 0)) && PyDict_GetItem(g_ext, s_dense) == Py_False &&
                     PyDict_GetItem(g_ext, s_fuse) == Py_True);
     PyObject *svs = shard_list(self, s_SV, n), *sus = shard_list(self, s_SU, n), *ps = shard_list(self, s_tp, n), *ps2 = shard_list(self, s_tp2, n);
-    NONE_UNLESS(svs && sus && ps && ps2);
+    NONE_UNLESS(svs && sus && ps && ps2 && (p.bn.size() <= 1 || same_device(x, {&p.bn_meta})));
     glqh_trellis_shard sh[GLQH_MAX_SHARDS] = {};
     glqh_trellis_stage2 s2[GLQH_MAX_SHARDS] = {};
     int64_t total_out = 0, total_m = 0;
@@ -597,11 +593,11 @@ bool projection(PyObject *const *t, const at::Tensor &x, const blocks &bn, const
             w->inv_rs2_dev = irs->const_data_ptr<float>();
         }
     }
-    const glqh_block_meta *bmeta;
-    if (!meta(bnm, bn.n, &bmeta)) return false;
+    at::Tensor bmeta;                                          // the caller's argument keeps it
+    if (!hold_meta(bnm, bn.n, &bmeta) || !same_device(x, {&bmeta})) return false;
     w->packed = pk->const_data_ptr(); w->packed_rows = pk->size(1); w->packed_cols = pk->size(2);
     w->su_f16 = su->const_data_ptr(); w->sv_f16 = sv->const_data_ptr(); w->wscale_dev = ws->const_data_ptr<float>();
-    w->blocks_n = bn.p; w->n_blocks_n = bn.n; w->bn_meta_dev = bmeta; w->blocks_m = bm.p; w->n_blocks_m = bm.n;
+    w->blocks_n = bn.p; w->n_blocks_n = bn.n; w->bn_meta_dev = meta_ptr(bmeta); w->blocks_m = bm.p; w->n_blocks_m = bm.n;
     w->in_features = in; w->out_features = out; w->n_pad = n_pad; w->m_pad = m_pad;
     return true;
 }

@@ -47,6 +47,7 @@ _GLQ_FUSED_TRELLIS_ENABLED = os.environ.get("GLQ_FUSED_TRELLIS", "1") != "0"
 
 class E8RHTLinear(nn.Module):
     _fast = None        # native form of forward (csrc/host.cpp), made by the first forward, dropped with _scalars
+    _fast_device = None # the device it was made for
 
     def __init__(self, in_features: int, out_features: int, bias: bool = False,
                  block_diagonal: bool = False, codebook_type: str = "e8_shell"):
@@ -103,6 +104,10 @@ class E8RHTLinear(nn.Module):
         self._blocks_m_meta_cpu = pack_block_meta(self.blocks_m)
         self._blocks_n_meta_gpu = None
         self._blocks_m_meta_gpu = None
+
+    def _apply(self, fn, recurse=True):
+        self._fast = None                              # moved or converted: it holds tensors of the device it was made for
+        return super()._apply(fn, recurse)
 
     @property
     def weight(self):
@@ -348,6 +353,11 @@ class E8RHTLinear(nn.Module):
         t1, t2, streams, h1, h2 = ext.e8_plan_parts(qs[:n], cb, cb2)
         return h.shell_plan(*args, *sc["inv"], n, self.codebook, self.codebook2, cb, cb2, t1, t2, qs, streams, h1, h2)
 
+    def _keep_native(self, ext, sc, device):
+        """Make the native form where there is none, or one for another device (buffers assigned one by one)."""
+        if self._fast is None or self._fast_device != device:
+            self._fast, self._fast_device = self._native(ext, sc), device
+
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         fast = self._fast
         if fast is not None and _GLQ_FUSED_TRELLIS_ENABLED and not torch.compiler.is_compiling():
@@ -380,8 +390,7 @@ class E8RHTLinear(nn.Module):
                 sc["wscale"], self.in_features, self.out_features, self.n_pad, self.m_pad,
                 bias=self.bias, out_dtype=x.dtype, trellis_packed2=self.trellis_packed2,
                 inv_resid_scale2=sc["inv2"])
-            if fast is None:
-                self._fast = self._native(ext, sc)
+            self._keep_native(ext, sc, x.device)
             return y.reshape(*shape[:-1], self.out_features)
 
         n = sc["n_stages"]
@@ -403,8 +412,7 @@ class E8RHTLinear(nn.Module):
         else:
             y = ext.glq_fused_linear_cuda(*common, int(math.log2(self.n_pad)),
                                           int(math.log2(self.m_pad)), *tail, out_dtype=xin.dtype)
-        if fast is None:
-            self._fast = self._native(ext, sc)
+        self._keep_native(ext, sc, x.device)
         if y.dtype != x.dtype:
             y = y.to(x.dtype)
         if self.bias is not None:

@@ -202,3 +202,42 @@ def test_a_failing_bias_addition_keeps_no_output():
             lin._fast(lin.__dict__, x)
         held.append(torch.cuda.memory_allocated())
     assert held[0] == held[1] == held[2]
+
+
+@pytest.mark.parametrize("kind", ["trellis", "shell2", "merged"])
+def test_block_tables_on_another_device_are_declined(kind):
+    """A plan made while the block tables were elsewhere (here: on the host) does not hand their addresses to the GPU."""
+    from glq_amd import ext, linear_method as LM
+    say("native forward, block tables on another device", kind)
+    x = torch.randn(2, 192, generator=torch.Generator().manual_seed(0)).to(DEV, torch.bfloat16)
+    if kind == "merged":
+        layer = LM.MergedTrellisLinear.from_linears([_layer("trellis", m, 192, False) for m in (96, 64)])
+        layer.process_weights_after_loading(DEV)
+        layer._glq_trellis_meta[0]["_bnm"] = layer._glq_trellis_meta[0]["_bnm"].cpu()
+        layer._make_native(ext, False)
+        assert layer._fast(layer.__dict__, x) is None
+        return
+    lin = _layer(kind, 96, 192, False)
+    lin.prepare()
+    ref, sc = lin(x), lin._scalars
+    h = ext.host()
+    for which in ("_blocks_n_meta_gpu", "_blocks_m_meta_gpu"):
+        kept = getattr(lin, which)
+        setattr(lin, which, kept.cpu())
+        assert lin._native(ext, sc)(lin.__dict__, x) is None
+        if kind == "trellis":
+            assert h.trellis_linear(x, lin.SV, lin.SU, lin.trellis_packed, None, lin._blocks_n_tensor, lin._blocks_m_tensor,
+                                    lin._blocks_n_meta_gpu, lin._blocks_m_meta_gpu, 0.02, 0.0, 192, 96, 192, 96, None) is None
+        setattr(lin, which, kept)
+    # a layer that goes away and comes back has its native form again after one call
+    lin.to("cpu")
+    assert lin._fast is None
+    lin.to(DEV)
+    assert torch.equal(lin(x), ref)
+    y = lin._fast(lin.__dict__, x)
+    assert y is not None and torch.equal(y, ref)
+    # a form made for another device (a layer whose buffers were assigned one by one) is replaced, not kept
+    lin._fast_device = torch.device("cpu")
+    old = lin._fast
+    lin(x.float())                                               # the Python route
+    assert lin._fast is not old and lin._fast_device == x.device

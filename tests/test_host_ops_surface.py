@@ -161,3 +161,12 @@ def test_merged_shell_linear_host_side():
         layer.apply(torch.zeros(1, 960))
     with pytest.raises(RuntimeError, match="E8-shell layers"):
         MergedShellLinear.from_linears([])
+
+
+@pytest.mark.parametrize("codebook_type", ["trellis", "e8_shell"])
+def test_moved_layers_drop_their_native_form(codebook_type):
+    from glq_amd.quantized_linear import E8RHTLinear
+    lin = E8RHTLinear(192, 96, codebook_type=codebook_type)
+    lin._fast = object()
+    torch.nn.Sequential(lin).to("cpu")
+    assert lin._fast is None
