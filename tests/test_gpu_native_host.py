@@ -241,3 +241,21 @@ def test_block_tables_on_another_device_are_declined(kind):
     old = lin._fast
     lin(x.float())                                               # the Python route
     assert lin._fast is not old and lin._fast_device == x.device
+
+
+def test_calls_without_the_native_host_path(monkeypatch):
+    """The same results where the host path cannot be loaded: layers, merged layers and codewords through Python."""
+    from glq_amd import ext, linear_method as LM
+    say("without the native host path")
+    x = torch.randn(3, 192, generator=torch.Generator().manual_seed(0)).to(DEV, torch.bfloat16)
+    lins = [_layer("trellis", m, 192, True) for m in (96, 64)] + [_layer("shell2", 96, 192, False)]
+    merged = LM.MergedTrellisLinear.from_linears([_layer("trellis", m, 192, False) for m in (96, 64)])
+    calls = [lambda l=l: l(x) for l in lins] + [lambda: merged.process_weights_after_loading(DEV).apply(x)]
+    table, v = e8_table_f16().float(), torch.randn(99, 8, generator=torch.Generator().manual_seed(1)).to(DEV)
+    calls.append(lambda: ext.e8_quantize(v, table)[1])
+    refs = [f() for f in calls for _ in range(2)][1::2]
+    monkeypatch.setattr(ext, "_host", ext._NoHost)
+    for l in lins:
+        l._fast = None
+    for f, ref in zip(calls, refs):
+        assert torch.equal(f(), ref) and torch.equal(f(), ref)

@@ -170,3 +170,22 @@ def test_moved_layers_drop_their_native_form(codebook_type):
     lin._fast = object()
     torch.nn.Sequential(lin).to("cpu")
     assert lin._fast is None
+
+
+def test_a_missing_host_path_is_reported_once_and_declines(monkeypatch):
+    """Without _glq_host.so (or with one that does not load) every call is left to the Python code."""
+    import sys
+    import warnings
+
+    import glq_amd
+    from glq_amd import ext
+    monkeypatch.setitem(sys.modules, "glq_amd._glq_host", None)
+    monkeypatch.delattr(glq_amd, "_glq_host", raising=False)
+    monkeypatch.setattr(ext, "_host", None)
+    with pytest.warns(RuntimeWarning, match="_glq_host"):
+        h = ext.host()
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        assert ext.host() is h
+    for name in ("trellis_linear", "moe", "shell_quantize", "trellis_plan", "shell_plan", "group_plan"):
+        assert getattr(h, name)(1, 2, 3) is None
