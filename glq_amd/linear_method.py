@@ -89,7 +89,7 @@ class MergedTrellisLinear:
     KV-shared layers do."""
 
     glq_is_trellis = True
-    _fast = None        # native form of the grouped calls (csrc/host.cpp), made by the first of them
+    _fast = None        # native form of the grouped calls (csrc/host.cpp), made at load time
 
     def __init__(self, in_features, shard_sizes, bpw=4):
         self.glq_in_features = int(in_features)
@@ -132,7 +132,7 @@ class MergedTrellisLinear:
         """Everything that reads the host or allocates, once, before any capture
         (glq_vllm/linear_method.py:1308-1464): buffers to the device, scalars to Python floats,
         the load-time invariants between the recipe and what the checkpoint carries, block lists
-        and device metas per shard, and for a merged 3INST layer the shard-batched output
+        and device metas per shard, the native form of the grouped calls, and for a merged 3INST layer the shard-batched output
         transform's concatenated sign vector and sub-block table."""
         if device is None:
             device = next(t.device for t in self.trellis_packed._shard_data + self.SV._shard_data
@@ -195,6 +195,9 @@ class MergedTrellisLinear:
                     "max_bs": max_bs,
                     "has_s2": any(m["has_s2"] for m in self._glq_trellis_meta),
                 }
+        if device.type == "cuda" and (self._grouped_ok(1) or self._grouped_rvq2_ok(1)):
+            from . import ext
+            self._make_native(ext, self._grouped_rvq2_ok(1))
         return self
 
     # ------------------------------------------------------------------ apply

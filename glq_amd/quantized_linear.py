@@ -46,7 +46,7 @@ _MAX_TOKENS_PER_CALL = 32768
 _GLQ_FUSED_TRELLIS_ENABLED = os.environ.get("GLQ_FUSED_TRELLIS", "1") != "0"
 
 class E8RHTLinear(nn.Module):
-    _fast = None        # native form of forward (csrc/host.cpp), made by the first forward, dropped with _scalars
+    _fast = None        # native form of forward (csrc/host.cpp), made by prepare() or the first forward, dropped with _scalars
     _fast_device = None # the device it was made for
 
     def __init__(self, in_features: int, out_features: int, bias: bool = False,
@@ -187,8 +187,8 @@ class E8RHTLinear(nn.Module):
 
     def prepare(self):
         """Load-time step, to be called once the buffers are on the GPU and the table is attached,
-        before any stream capture: host copies of the scalars, block meta on the device and, for an
-        E8 layer, the packed table(s) and the folded index streams the small-batch and tile kernels
+        before any stream capture: host copies of the scalars, block meta on the device, the native form of
+        forward (the first call is then as fast as the later ones) and, for an E8 layer, the packed table(s) and the folded index streams the small-batch and tile kernels
         read (1.5 x the index bytes; `GLQ_E8_FOLD=0` / `GLQ_E8_FOLD_MAX_BYTES` bound them).  The
         reference's place for this work is `GLQLinearMethod.process_weights_after_loading`
         (glq_vllm/linear_method.py:1031-1110).  A forward call outside capture runs it if the
@@ -209,6 +209,7 @@ class E8RHTLinear(nn.Module):
             held = ext.e8_prepare(self.Qidxs, cb, self.Qidxs2 if n >= 2 else None, cb2,
                                   self.Qidxs3 if n >= 3 else None, self.Qidxs4 if n >= 4 else None)
         self._prepared_for = self._buffer_identity()
+        self._keep_native(ext, sc, dev)
         return held
 
     def _buffer_identity(self):
@@ -340,6 +341,8 @@ class E8RHTLinear(nn.Module):
     def _native(self, ext, sc):
         """The native forward: scalars, block sizes and, for a shell layer, tables and folded streams as they are now.
         The buffers themselves are read again on every call."""
+        if self._is_trellis and not (self._trellis_has_kernel and ext.glq_trellis_kernel_supported(self.m_pad, self.n_pad)):
+            return None                                # forward says why
         h, bd = ext.host(), self._is_trellis or self.block_diagonal
         args = (self.in_features, self.out_features, self.n_pad, self.m_pad, list(self.blocks_n), list(self.blocks_m),
                 self._blocks_n_meta_gpu if bd else None, self._blocks_m_meta_gpu if bd else None, sc["wscale"])

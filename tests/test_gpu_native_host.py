@@ -50,8 +50,11 @@ def test_native_forward_equals_the_python_route(kind, out_f, in_f, bias, dtype, 
     lin = _layer(kind, out_f, in_f, bias)
     lin.prepare()
     x = torch.randn(*shape, in_f, generator=torch.Generator().manual_seed(3)).to(DEV, dtype)
-    assert lin._fast is None
-    ref = lin(x)                                                 # the Python route, which makes the native form
+    assert lin._fast is not None                                 # made by the load-time step
+    y = lin(x)
+    lin._fast = None
+    ref = lin(x)                                                 # the Python route, which makes the native form again
+    assert torch.equal(y, ref)
     y = lin._fast(lin.__dict__, x)
     assert y is not None and y.shape == ref.shape and y.dtype == ref.dtype and torch.equal(y, ref)
     assert torch.equal(lin(x), ref)
@@ -95,7 +98,9 @@ def test_native_merged_forward_equals_the_python_route(bpw, B):
     lins = [_layer("trellis2" if bpw == 6 else "trellis", m, 192, False) for m in (96, 64, 64)]
     ml = LM.MergedTrellisLinear.from_linears(lins, bpw=bpw).process_weights_after_loading(DEV)
     x = torch.randn(B, 192, generator=torch.Generator().manual_seed(B)).to(DEV, torch.bfloat16)
-    ref = ml.apply(x)
+    assert ml._fast is not None                                  # made by the load-time step
+    ml._fast = None
+    ref = ml.apply(x)                                            # the Python route, which makes it again
     y = ml._fast(ml.__dict__, x)
     assert y is not None and torch.equal(y, ref)
     bias = torch.randn(224, generator=torch.Generator().manual_seed(0)).to(DEV)
@@ -214,6 +219,7 @@ def test_block_tables_on_another_device_are_declined(kind):
         layer = LM.MergedTrellisLinear.from_linears([_layer("trellis", m, 192, False) for m in (96, 64)])
         layer.process_weights_after_loading(DEV)
         layer._glq_trellis_meta[0]["_bnm"] = layer._glq_trellis_meta[0]["_bnm"].cpu()
+        layer._fast = None
         layer._make_native(ext, False)
         assert layer._fast(layer.__dict__, x) is None
         return
@@ -259,3 +265,20 @@ def test_calls_without_the_native_host_path(monkeypatch):
         l._fast = None
     for f, ref in zip(calls, refs):
         assert torch.equal(f(), ref) and torch.equal(f(), ref)
+
+
+def test_load_time_steps_make_no_native_form_for_what_forward_refuses():
+    from glq_amd import linear_method as LM
+    say("native form of layers that are refused")
+    lin = _layer("trellis", 64, 128, False)
+    lin.set_codebook(type("natural", (), {"has_kernel": False})())
+    lin.prepare()
+    x = torch.zeros(1, 128, dtype=torch.bfloat16, device=DEV)
+    with pytest.raises(RuntimeError, match="natural-layout"):
+        lin(x)
+    lins = [_layer("trellis", 64, 128, False), _layer("trellis2", 32, 128, False)]
+    mixed = LM.MergedTrellisLinear.from_linears(lins, bpw=4)
+    mixed.trellis_packed2._shard_data[1] = torch.zeros(0, dtype=torch.int16, device=DEV)
+    mixed.trellis_packed._shard_data[1] = torch.zeros(0, dtype=torch.int16, device=DEV)       # never loaded
+    mixed.process_weights_after_loading(DEV)
+    assert mixed._fast is None and float(mixed.apply(x)[:, 64:].abs().max()) == 0.0
