@@ -96,10 +96,9 @@ SIGNATURES = {
         c_int, [c_vp, c_int, c_i64, c_i64, c_vp, c_vp, c_i64, c_i64, c_vp, c_vp, c_i64, c_int, c_vp, c_int,
                 c_i64, c_vp, c_sz, c_vp]),
     "glqh_e8_quantize": (c_int, [c_vp, c_vp, c_vp, c_i64, c_i64, c_vp, c_vp, c_vp]),
-    "glqh_e8_shell_index": (c_int, [c_vp, c_vp, c_i64, c_vp, c_vp, c_vp, c_vp]),
     "glqh_e8_shell_workspace_bytes": (c_sz, [c_i64]),
     "glqh_e8_shell_quantize": (
-        c_int, [c_vp, c_i64, c_vp, c_vp, c_i64, c_vp, c_vp, c_vp, c_vp, c_vp, c_sz, c_vp]),
+        c_int, [c_vp, c_i64, c_vp, c_vp, c_i64, c_vp, c_vp, c_vp, c_sz, c_vp]),
     "glqh_trellis_quantize_workspace_bytes": (c_sz, [c_int, c_i64]),
     "glqh_trellis_quantize_tiles": (c_int, [c_vp, c_i64, c_int, c_vp, c_vp, c_vp, c_sz, c_vp]),
     "glqh_trellis_quantize_matrix_workspace_bytes": (c_sz, [c_int, c_i64, c_i64]),

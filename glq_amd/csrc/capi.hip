@@ -2107,33 +2107,22 @@ extern "C" int glqh_e8_quantize(const float *x, const float *table_f32, const fl
                                    (hipStream_t)stream);
 }
 
-int glqh_launch_e8_shell_index(const float *table, const float *norms, int n, uint32_t *keys, int *vals, int *counts,
-                               hipStream_t stream);
 size_t glqh_e8_shell_ws_bytes(int64_t N);
 int glqh_launch_e8_shell_quantize(const float *x, int64_t N, const float *table, const float *norms, int n_entries,
-                                  const uint32_t *keys, const int *vals, int64_t *idx_out, float *dec_out, void *ws,
-                                  hipStream_t stream);
-
-extern "C" int glqh_e8_shell_index(const float *table_f32, const float *norms_f32, int64_t n_entries, uint32_t *keys_out,
-                                   int32_t *vals_out, int32_t *counts_out, void *stream) {
-    GLQH_INIT();
-    GLQH_REQUIRE(table_f32 && norms_f32 && keys_out && vals_out && counts_out, "e8 shell index: null pointer");
-    GLQH_REQUIRE(n_entries >= 1 && n_entries <= 65536, "e8 shell index: %lld table rows (1..65536)", (long long)n_entries);
-    return glqh_launch_e8_shell_index(table_f32, norms_f32, (int)n_entries, keys_out, vals_out, counts_out, (hipStream_t)stream);
-}
+                                  int64_t *idx_out, float *dec_out, void *ws, hipStream_t stream);
 
 extern "C" size_t glqh_e8_shell_workspace_bytes(int64_t N) { return N >= 1 ? glqh_e8_shell_ws_bytes(N) : 0; }
 
 extern "C" int glqh_e8_shell_quantize(const float *x, int64_t N, const float *table_f32, const float *norms_f32,
-                                      int64_t n_entries, const uint32_t *keys, const int32_t *vals, int64_t *idx_out,
-                                      float *decoded_out, void *ws, size_t ws_bytes, void *stream) {
+                                      int64_t n_entries, int64_t *idx_out, float *decoded_out, void *ws, size_t ws_bytes,
+                                      void *stream) {
     GLQH_INIT();
-    GLQH_REQUIRE(x && table_f32 && norms_f32 && keys && vals && idx_out, "e8 shell quantize: null pointer");
+    GLQH_REQUIRE(x && table_f32 && norms_f32 && idx_out, "e8 shell quantize: null pointer");
     GLQH_REQUIRE(N >= 1, "e8 shell quantize: N=%lld", (long long)N);
     GLQH_REQUIRE(n_entries >= 1 && n_entries <= 65536, "e8 shell quantize: %lld table rows (1..65536)", (long long)n_entries);
     const size_t need = glqh_e8_shell_ws_bytes(N);
     GLQH_REQUIRE(ws && ws_bytes >= need, "e8 shell quantize: workspace of %zu bytes needed, got %zu", need, ws_bytes);
-    return glqh_launch_e8_shell_quantize(x, N, table_f32, norms_f32, (int)n_entries, keys, vals, idx_out, decoded_out, ws,
+    return glqh_launch_e8_shell_quantize(x, N, table_f32, norms_f32, (int)n_entries, idx_out, decoded_out, ws,
                                          (hipStream_t)stream);
 }
 

@@ -16,11 +16,11 @@ typedef float f32x4v __attribute__((ext_vector_type(4)));
 constexpr int EQ_THREADS = 256;
 constexpr int EQ_VPT = 4;
 
-__global__ void __launch_bounds__(EQ_THREADS)
-e8_quantize_kernel(const float *__restrict__ x, const float *__restrict__ table,
-                   const float *__restrict__ norms, int64_t N, int K, int64_t *__restrict__ idx_out,
-                   float *__restrict__ dec_out) {
-    const int64_t v0 = ((int64_t)blockIdx.x * EQ_THREADS + threadIdx.x) * EQ_VPT;
+// the vectors of workgroup `block`
+__device__ __forceinline__ void
+e8_quantize_block(const float *__restrict__ x, const float *__restrict__ table, const float *__restrict__ norms, int64_t N,
+                  int K, int64_t *__restrict__ idx_out, float *__restrict__ dec_out, int64_t block) {
+    const int64_t v0 = (block * EQ_THREADS + threadIdx.x) * EQ_VPT;
     float xv[EQ_VPT][8], best[EQ_VPT];
     int bi[EQ_VPT];
 #pragma unroll
@@ -60,14 +60,26 @@ e8_quantize_kernel(const float *__restrict__ x, const float *__restrict__ table,
     }
 }
 
+__global__ void __launch_bounds__(EQ_THREADS)
+e8_quantize_kernel(const float *__restrict__ x, const float *__restrict__ table,
+                   const float *__restrict__ norms, int64_t N, int K, int64_t *__restrict__ idx_out,
+                   float *__restrict__ dec_out) {
+    e8_quantize_block(x, table, norms, N, K, idx_out, dec_out, blockIdx.x);
+}
+
 // ---- the whole shell table, by its symmetry --------------------------------------------
 // The 65536-row table is every E8 point of norm up to 10 and a part of the shell of norm 12.  A
 // full shell is a union of orbits of the even signed permutations (Weyl group of D8), and on one
 // orbit the largest <x, c> is <y, p>: y = |x| in descending order, its last entry carrying the
 // sign of the product of x's entries, p the orbit's representative ordered the same way.  20 orbits
 // of prefix sums of y replace 56881 distances; the second largest value on an orbit is one of the
-// eight simple reflections of p away, so the gap to every other row is known too.  The index of
-// the row found comes from a hash of the codewords.
+// eight simple reflections of p away, so the gap to every other row is known too.
+//
+// Nothing about a table is taken on trust or kept from one call for the next.  Every E8 point of norm up to 12 has a
+// place of its own (es_map), a matter of the lattice alone; the first launch of a call writes each row's number to its
+// place, and what the search assumes of the table is checked on the way: rows that are such points, with their norms
+// in `norms`, the number of those of norm up to 10, and (in the second launch) that no two rows share a place.  For
+// any other table the third launch walks it, every vector against every row.
 //
 // Which row the table walk above would return depends on fp32 rounding only where two distances are
 // closer than what rounding can move them; `es_margin` bounds that: 128 roundings of
@@ -80,61 +92,70 @@ e8_quantize_kernel(const float *__restrict__ x, const float *__restrict__ table,
 // finite, or have too many points in reach for the list, take the walk itself (e8_walk_kernel).
 //
 // 524288 vectors of N(0, 1): 12.06 ms (walk) -> 98 us (points of norm 12 on the matrix cores, all 8655 rows for
-// every vector they may win) -> 34 us (points in reach only; 38 MB in and out, 8 us); 960 vectors 12.7 ms ->
-// 14 us, latency.
+// every vector they may win) -> 34 us (points in reach only; 38 MB in and out, 8 us) -> 35.4 us with the table read
+// by every call (es_index_kernel 4.5 us; 250 -> 54 us where the table is new); 960 vectors 12.7 ms -> 13.4 ->
+// 20 us: three dependent launches.
 constexpr int ES_THREADS = 256;
-constexpr int ES_SLOTS = 1 << 17;                              // hash slots for at most 65536 keys
-constexpr uint32_t ES_EMPTY = 0xFFFFFFFFu;
+constexpr int ES_PLACES = 117361;                              // E8 points of norm up to 12
+constexpr int ES_FULL = GLQH_E8_SHELL_MIN_ROWS;                // of norm up to 10: all of them are rows of the table
+constexpr int ES_CHECKS = 128;                                 // workgroups, at least, that look for rows of one place
 constexpr int ES_CHUNK = 128;                                  // vectors whose points are listed together,
 constexpr int ES_LIST = 3072;                                  // and the points: 2.5 each at unit scale, up to 106 far out
 constexpr int ES_SPLIT = 128;                                  // parts of the table in the exact walk
 
-__device__ __forceinline__ uint32_t es_hash(uint32_t code) { return (code * 2654435761u) >> 15; }
+// Places.  A point is two halves of four coordinates (2 c + 6 in a nibble each).  Halves are integers or half-integers
+// and have an even or an odd sum of coordinates (of 2 c: 0 or 2 mod 4), and two of them make a point when they agree in
+// both.  With the halves of a class in the order of their norms, those that a first half h can take are a prefix, as
+// long as there are halves of norm up to 12 - |h|^2: the place of (h, l) is base(h) + rank(l).
+struct es_map_t {
+    uint32_t at[65536];                                        // by half: base << 11 | rank; 0 where it is none
+    int places, ranks;
+};
 
-__global__ void __launch_bounds__(256)
-es_clear_kernel(uint32_t *__restrict__ keys, int *__restrict__ counts) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i < ES_SLOTS) keys[i] = ES_EMPTY;
-    if (i < 8) counts[i] = 0;
+constexpr es_map_t es_make_map() {
+    es_map_t m = {};
+    int count[4][50] = {};                                     // halves of a class by 4 * norm, then those before them
+    int base = 0, most = 0;
+    for (int pass = 0; pass < 2; ++pass) {
+        int upto[4][50] = {};                                  // halves of 4 * norm up to n
+        int next[4][50] = {};
+        if (pass == 1)
+            for (int c = 0; c < 4; ++c) {
+                int sum = 0;
+                for (int n = 0; n <= 48; ++n) {
+                    next[c][n] = sum;
+                    sum += count[c][n];
+                    upto[c][n] = sum;
+                }
+                most = sum > most ? sum : most;
+            }
+        for (int odd = 0; odd < 2; ++odd)
+            for (int a = odd; a <= 12; a += 2)
+                for (int b = odd; b <= 12; b += 2)
+                    for (int c = odd; c <= 12; c += 2)
+                        for (int d = odd; d <= 12; d += 2) {
+                            const int n = (a - 6) * (a - 6) + (b - 6) * (b - 6) + (c - 6) * (c - 6) + (d - 6) * (d - 6);
+                            const int k = 2 * odd + (((a + b + c + d) >> 1) & 1);
+                            if (n > 48) continue;
+                            if (pass == 0) ++count[k][n];
+                            else {
+                                m.at[a | b << 4 | c << 8 | d << 12] = (uint32_t)base << 11 | (uint32_t)next[k][n]++;
+                                base += upto[k][48 - n];
+                            }
+                        }
+    }
+    m.places = base;
+    m.ranks = most;
+    return m;
 }
 
-// counts[s]: distinct rows of norm 2s (s = 0..6) that are E8 points with that norm in `norms`;
-// counts[7]: everything else.
-__global__ void __launch_bounds__(256)
-es_index_kernel(const float *__restrict__ table, const float *__restrict__ norms, int n, uint32_t *__restrict__ keys,
-                int *__restrict__ vals, int *__restrict__ counts) {
-    const int r = blockIdx.x * 256 + threadIdx.x;
-    if (r >= n) return;
-    uint32_t code = 0, odd = 0;
-    int sum = 0, n4 = 0;
-    bool ok = true;
-#pragma unroll
-    for (int d = 0; d < 8; ++d) {
-        const float t = 2.0f * table[(int64_t)r * 8 + d] + 6.0f;
-        ok = ok && t >= 0.0f && t <= 12.0f && t == (float)(int)t;
-        const int v = ok ? (int)t : 0;
-        code |= (uint32_t)v << (4 * d);
-        odd += v & 1;
-        sum += v - 6;
-        n4 += (v - 6) * (v - 6);
-    }
-    ok = ok && (odd == 0 || odd == 8) && (sum & 3) == 0 && n4 <= 48 && norms[r] == 0.25f * (float)n4;
-    int s = 7;
-    if (ok) {
-        uint32_t h = es_hash(code);
-        for (int probe = 0; probe < ES_SLOTS; ++probe) {       // ends: fewer keys than slots
-            const uint32_t was = atomicCAS(keys + h, ES_EMPTY, code);
-            if (was == ES_EMPTY) { vals[h] = r; s = n4 >> 3; break; }
-            if (was == code) break;                            // a second row with these values
-            h = (h + 1) & (ES_SLOTS - 1);
-        }
-    }
-    // one add per wave and class: the rows are sorted by norm, so a wave has one or two
-#pragma unroll 1
-    for (int q = 0; q < 8; ++q) {
-        const unsigned long long who = __ballot(s == q);
-        if (s == q && (int)(threadIdx.x & 63) == __builtin_ctzll(who)) atomicAdd(counts + q, __builtin_popcountll(who));
-    }
+__device__ constexpr es_map_t es_map = es_make_map();
+static_assert(es_map.places == ES_PLACES && es_map.ranks <= 2048, "places of the points");
+
+// the place of a point of norm up to 12
+__device__ __forceinline__ int es_place(uint32_t code) {
+    const uint32_t h = es_map.at[code & 0xffffu], l = es_map.at[code >> 16];
+    return (int)((h >> 11) + (l & 2047u));
 }
 
 // the walk's distance of one row
@@ -158,12 +179,43 @@ __device__ __forceinline__ void es_load(const float *__restrict__ x, int64_t v, 
     xv[4] = b.x; xv[5] = b.y; xv[6] = b.z; xv[7] = b.w;
 }
 
+// row_at[place] = row; place_of[row], -1 where the row is not such a point with its norm in `norms`.
+// counts[r / 64]: rows of norm up to 10, negative if one of the 64 rows is no point.
+__global__ void __launch_bounds__(ES_THREADS)
+es_index_kernel(const float *__restrict__ table, const float *__restrict__ norms, int n, int *__restrict__ row_at,
+                int *__restrict__ place_of, int *__restrict__ counts, int *__restrict__ shared_place) {
+    const int r = blockIdx.x * ES_THREADS + threadIdx.x;
+    if (r == 0) *shared_place = 0;
+    if (r >= n) return;
+    float c[8];
+    es_load(table, r, c);
+    const float norm = norms[r];
+    uint32_t code = 0, odd = 0;
+    int sum = 0, n4 = 0;
+    bool ok = true;
+#pragma unroll
+    for (int d = 0; d < 8; ++d) {
+        const float t = 2.0f * c[d] + 6.0f;
+        ok = ok && t >= 0.0f && t <= 12.0f && t == (float)(int)t;
+        const int v = ok ? (int)t : 0;
+        code |= (uint32_t)v << (4 * d);
+        odd += v & 1;
+        sum += v - 6;
+        n4 += (v - 6) * (v - 6);
+    }
+    ok = ok && (odd == 0 || odd == 8) && (sum & 3) == 0 && n4 <= 48 && norm == 0.25f * (float)n4;
+    const int place = ok ? es_place(code) : -1;
+    place_of[r] = place;
+    if (ok) row_at[place] = r;
+    const unsigned long long full = __ballot(ok && n4 <= 40), bad = __ballot(!ok);
+    if ((threadIdx.x & 63) == 0) counts[r >> 6] = bad ? -ES_FULL - 1 : __builtin_popcountll(full);
+}
+
 struct es_args {
     const float *x, *table, *norms;
     int64_t N;
-    const uint32_t *keys;
-    const int *vals;
     int n_entries;
+    int *row_at, *place_of, *counts, *shared_place;            // written by es_index_kernel
     int64_t *idx_out;
     float *dec_out;                                            // may be null
     int *walk_count;                                           // per workgroup of the first kernel
@@ -171,16 +223,10 @@ struct es_args {
     unsigned long long *walk_key;                              // N
 };
 
-// row of a codeword (2 c + 6 in a nibble per coordinate), -1 if the table does not hold it
+// row of a point (2 c + 6 in a nibble per coordinate), -1 if the table does not hold it: its place is then unset
 __device__ __forceinline__ int es_row(const es_args &a, uint32_t code) {
-    uint32_t h = es_hash(code), k = a.keys[h];
-    int row = a.vals[h];                                       // asked for together; unset where the key is empty
-    for (int probe = 0; k != code && k != ES_EMPTY && probe < ES_SLOTS; ++probe) {
-        h = (h + 1) & (ES_SLOTS - 1);
-        k = a.keys[h];
-        row = a.vals[h];
-    }
-    return k == code ? row : -1;
+    const int place = es_place(code), row = a.row_at[place];
+    return (uint32_t)row < (uint32_t)a.n_entries && a.place_of[row] == place ? row : -1;
 }
 
 __device__ __forceinline__ void es_store(const es_args &a, int64_t v, int row) {
@@ -326,6 +372,12 @@ e8_shell_kernel(const es_args a) {
     const int tid = threadIdx.x;
     const int64_t v0 = (int64_t)blockIdx.x * V;
     if (tid == 0) n_flag = n_walk = 0;
+    // two rows of one place: one of them is not the row found there
+    for (int64_t r = (int64_t)blockIdx.x * ES_THREADS + tid; r < a.n_entries; r += (int64_t)gridDim.x * ES_THREADS) {
+        const int place = a.place_of[r];
+        if (place >= 0 && a.row_at[place] != (int)r) *a.shared_place = 1;
+    }
+    if (v0 >= a.N) return;                                     // here for that only
     __syncthreads();
     auto walk = [&](int local) {
         const int64_t at = v0 + atomicAdd(&n_walk, 1);
@@ -358,7 +410,7 @@ e8_shell_kernel(const es_args a) {
         if (q[6] + q[7] != 0) gap = __builtin_fminf(gap, (float)(q[6] + q[7]) * (s.y[6] + s.y[7]));
         if (!(gap > s.margin)) { flags[atomicAdd(&n_flag, 1)] = (unsigned short)local; continue; }
         const uint32_t code = es_code(p, s.k, s.signs, s.flip);
-        a.idx_out[v] = es_row(a, code);
+        a.idx_out[v] = a.row_at[es_place(code)];               // a row of the table, of norm up to 10
         if (a.dec_out) {
             f32x4v lo, hi;
 #pragma unroll
@@ -442,7 +494,7 @@ e8_shell_kernel(const es_args a) {
         if (tid < nc) {
             const int local = flags[c0 + tid];
             if (s_signs[tid] & 512u) walk(local);
-            else es_store(a, v0 + local, (int)(uint32_t)best[tid]);
+            else if (best[tid] != ~0ull) es_store(a, v0 + local, (int)(uint32_t)best[tid]);   // none: not the shell table
         }
         __syncthreads();
     }
@@ -455,13 +507,15 @@ e8_shell_kernel(const es_args a) {
 __global__ void __launch_bounds__(ES_THREADS)
 e8_walk_kernel(const es_args a, int n_src, int per_src) {
     constexpr int ROWS = 65536 / ES_SPLIT;                     // of one part, at most
-    __shared__ int sums[4];
+    __shared__ int sums[4], fulls[4];
     __shared__ int64_t item[64];                               // the vector's list position
     __shared__ unsigned long long keys[4][64];
     __shared__ f32x4v rows[ROWS][2];
     __shared__ float row_norm[ROWS];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    // the vectors' ranks over all source workgroups: a run of sources per thread
+    // what the search assumed of the table, and the vectors' ranks over all source workgroups: a run of sources per thread
+    int full = tid == 0 && *a.shared_place ? -ES_FULL - 1 : 0;
+    for (int i = tid; i < (a.n_entries + 63) / 64; i += ES_THREADS) full += a.counts[i];
     const int per = (n_src + ES_THREADS - 1) / ES_THREADS;
     const int s0 = min(tid * per, n_src), s1 = min(s0 + per, n_src);
     int mine = 0;
@@ -471,15 +525,27 @@ e8_walk_kernel(const es_args a, int n_src, int per_src) {
     for (int o = 1; o < 64; o <<= 1) {
         const int v = __shfl_up(first, o, 64);
         if (lane >= o) first += v;
+        full += __shfl_xor(full, o, 64);
     }
-    if (lane == 63) sums[wave] = first;
+    if (lane == 63) {
+        sums[wave] = first;
+        fulls[wave] = full;
+    }
     __syncthreads();
     int total = 0;
     first -= mine;
+    full = 0;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
         if (q < wave) first += sums[q];
         total += sums[q];
+        full += fulls[q];
+    }
+    if (full != ES_FULL) {                                     // any other table: every vector against every row
+        const int64_t blocks = (a.N + EQ_THREADS * EQ_VPT - 1) / (EQ_THREADS * EQ_VPT);
+        for (int64_t b = blockIdx.x; b < blocks; b += gridDim.x)
+            e8_quantize_block(a.x, a.table, a.norms, a.N, a.n_entries, a.idx_out, a.dec_out, b);
+        return;
     }
     const int64_t work = (int64_t)((total + 63) / 64) * ES_SPLIT;
     for (int64_t w = blockIdx.x; w < work; w += gridDim.x) {
@@ -546,33 +612,34 @@ int glqh_launch_e8_quantize(const float *x, const float *table, const float *nor
     return 0;
 }
 
-int glqh_launch_e8_shell_index(const float *table, const float *norms, int n, uint32_t *keys, int *vals, int *counts,
-                               hipStream_t stream) {
-    hipLaunchKernelGGL(es_clear_kernel, dim3(ES_SLOTS / 256), dim3(256), 0, stream, keys, counts);
-    hipLaunchKernelGGL(es_index_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, table, norms, n, keys, vals,
-                       counts);
-    GLQH_LAUNCH_CHECK("e8 shell index launch");
-    return 0;
+static size_t es_align(size_t v) { return (v + 15) & ~(size_t)15; }
+
+size_t glqh_e8_shell_ws_bytes(int64_t N) {
+    return es_align((size_t)N * 16 + (size_t)((N + 63) / 64) * 4) + (size_t)(ES_PLACES + 65536 + 65536 / 64 + 1) * 4;
 }
 
-size_t glqh_e8_shell_ws_bytes(int64_t N) { return (size_t)N * 16 + (size_t)((N + 63) / 64) * 4; }
-
 int glqh_launch_e8_shell_quantize(const float *x, int64_t N, const float *table, const float *norms, int n_entries,
-                                  const uint32_t *keys, const int *vals, int64_t *idx_out, float *dec_out, void *ws,
-                                  hipStream_t stream) {
+                                  int64_t *idx_out, float *dec_out, void *ws, hipStream_t stream) {
     const int per = es_per_wg(N);
     const int64_t wgs = (N + per - 1) / per;
     GLQH_REQUIRE(N <= 2147483647ll, "e8 quantize: too many vectors");
     es_args a;
-    a.x = x; a.table = table; a.norms = norms; a.N = N; a.keys = keys; a.vals = vals; a.n_entries = n_entries;
+    a.x = x; a.table = table; a.norms = norms; a.N = N; a.n_entries = n_entries;
     a.idx_out = idx_out; a.dec_out = dec_out;
     a.walk_key = (unsigned long long *)ws;
     a.walk_list = (int *)(a.walk_key + N);
     a.walk_arrive = a.walk_list + N;
     a.walk_count = a.walk_arrive + N;
-    if (per == 512) hipLaunchKernelGGL(e8_shell_kernel<512>, dim3((unsigned)wgs), dim3(ES_THREADS), 0, stream, a);
-    else if (per == 256) hipLaunchKernelGGL(e8_shell_kernel<256>, dim3((unsigned)wgs), dim3(ES_THREADS), 0, stream, a);
-    else hipLaunchKernelGGL(e8_shell_kernel<64>, dim3((unsigned)wgs), dim3(ES_THREADS), 0, stream, a);
+    a.row_at = (int *)((char *)ws + es_align((size_t)N * 16 + (size_t)((N + 63) / 64) * 4));
+    a.place_of = a.row_at + ES_PLACES;
+    a.counts = a.place_of + 65536;
+    a.shared_place = a.counts + 65536 / 64;
+    const dim3 grid((unsigned)(wgs > ES_CHECKS ? wgs : ES_CHECKS));
+    hipLaunchKernelGGL(es_index_kernel, dim3((unsigned)((n_entries + ES_THREADS - 1) / ES_THREADS)), dim3(ES_THREADS), 0, stream, table,
+                       norms, n_entries, a.row_at, a.place_of, a.counts, a.shared_place);
+    if (per == 512) hipLaunchKernelGGL(e8_shell_kernel<512>, grid, dim3(ES_THREADS), 0, stream, a);
+    else if (per == 256) hipLaunchKernelGGL(e8_shell_kernel<256>, grid, dim3(ES_THREADS), 0, stream, a);
+    else hipLaunchKernelGGL(e8_shell_kernel<64>, grid, dim3(ES_THREADS), 0, stream, a);
     hipLaunchKernelGGL(e8_walk_kernel, dim3(2 * glqh_device_cus()), dim3(ES_THREADS), 0, stream, a, (int)wgs, per);
     GLQH_LAUNCH_CHECK("e8 shell quantize launch");
     return 0;

@@ -640,14 +640,13 @@ PyObject *py_moe(PyObject *, PyObject *const *a, Py_ssize_t n) {
 }
 
 // ---- E8 codewords ----------------------------------------------------------------------------
-// shell_quantize(x, table, norms, keys, vals, return_decoded) -> (decoded | None, indices)
+// shell_quantize(x, table, norms, return_decoded) -> (decoded | None, indices)
 PyObject *py_shell_quantize(PyObject *, PyObject *const *a, Py_ssize_t n) {
-    NONE_UNLESS(n == 6 && !modes());
+    NONE_UNLESS(n == 4 && !modes());
     const at::Tensor *x = gpu(a[0], at::kFloat), *table = gpu(a[1], at::kFloat), *norms = gpu(a[2], at::kFloat);
-    const at::Tensor *keys = gpu(a[3], at::kInt), *vals = gpu(a[4], at::kInt);
-    NONE_UNLESS(x && table && norms && keys && vals && x->dim() == 2 && x->size(1) == 8 && x->size(0) >= 1);
-    NONE_UNLESS(same_device(*x, {table, norms, keys, vals}));
-    const int decoded = PyObject_IsTrue(a[5]);
+    NONE_UNLESS(x && table && norms && x->dim() == 2 && x->size(1) == 8 && x->size(0) >= 1 && table->dim() == 2 && table->size(1) == 8);
+    NONE_UNLESS(table->size(0) <= 65536 && norms->numel() == table->size(0) && same_device(*x, {table, norms}));
+    const int decoded = PyObject_IsTrue(a[3]);
     NONE_UNLESS(decoded >= 0);
     const int64_t N = x->size(0);
     return guarded([&]() -> PyObject * {
@@ -659,8 +658,8 @@ PyObject *py_shell_quantize(PyObject *, PyObject *const *a, Py_ssize_t n) {
             no_gil unlocked;
             scratch ws(L.shell_ws(N));
             rc = L.shell_quantize(x->const_data_ptr<float>(), N, table->const_data_ptr<float>(), norms->const_data_ptr<float>(), table->size(0),
-                                  (const uint32_t *)keys->const_data_ptr(), vals->const_data_ptr<int32_t>(), idx.mutable_data_ptr<int64_t>(),
-                                  decoded ? dec.mutable_data_ptr<float>() : nullptr, ws.p.get(), ws.bytes, stream_of(*x));
+                                  idx.mutable_data_ptr<int64_t>(), decoded ? dec.mutable_data_ptr<float>() : nullptr, ws.p.get(),
+                                  ws.bytes, stream_of(*x));
         }
         if (rc) return failed();
         return Py_BuildValue("(NN)", decoded ? THPVariable_Wrap(std::move(dec)) : Py_NewRef(Py_None), THPVariable_Wrap(std::move(idx)));
@@ -707,7 +706,7 @@ PyMethodDef methods[] = {
     {"bind", py_bind, METH_VARARGS, "bind(library handle, globals of glq_amd.ext)"},
     {"trellis_linear", (PyCFunction)(void *)py_trellis_linear, METH_FASTCALL, "fused trellis linear, or None"},
     {"moe", (PyCFunction)(void *)py_moe, METH_FASTCALL, "routed trellis experts, or None"},
-    {"shell_quantize", (PyCFunction)(void *)py_shell_quantize, METH_FASTCALL, "codewords of the whole shell table, or None"},
+    {"shell_quantize", (PyCFunction)(void *)py_shell_quantize, METH_FASTCALL, "codewords of a table that may be the shell table, or None"},
     {"trellis_plan", py_trellis_plan, METH_VARARGS, "forward of a trellis E8RHTLinear"},
     {"shell_plan", py_shell_plan, METH_VARARGS, "forward of a shell E8RHTLinear"},
     {"group_plan", py_group_plan, METH_VARARGS, "forward of a merged trellis layer"},

@@ -1154,92 +1154,43 @@ def glq_fused_linear_block_diag_cuda(x, sv, su, qidxs, codebook, wscale, in_feat
 
 
 # ---- encode side ----------------------------------------------------------------------
-_SHELL_PLANS = _DerivedCache()
-_SHELL_COUNTS = (1, 240, 2160, 6720, 17520, 30240)            # E8 points of norm 0, 2, .. 10
-# Tables of a few hundred rows (the secondary table of 3 bpw has 256) are walked in as little time.
-_SHELL_MIN_ROWS = 4096
-
-
-class _ShellPlan:
-    """What the search on the whole shell table needs beside it, derived once per table: fp32 rows and norms
-    and the hash of the rows.  `ok` is False for any other table."""
-
-    def __init__(self, codebook, norms):
-        lib = _lib.load()
-        # copies: the cache must not keep alive the tensors whose end drops its entry
-        self.table = codebook.to(torch.float32, copy=True).contiguous()
-        self.norms = (self.table * self.table).sum(-1) if norms is None else norms.to(self.table, copy=True).contiguous()
-        self.given = None if norms is None else weakref.ref(norms.untyped_storage())
-        self.ok = False
-        if self.table.shape[0] < _SHELL_MIN_ROWS or self.norms.numel() != self.table.shape[0]:
-            return
-        i32 = dict(dtype=torch.int32, device=self.table.device)
-        n = self.table.shape[0]
-        keys, vals, counts = torch.empty(1 << 17, **i32), torch.empty(1 << 17, **i32), torch.empty(8, **i32)
-        check(lib.glqh_e8_shell_index(_p(self.table), _p(self.norms), n, _p(keys), _p(vals), _p(counts), _stream()))
-        counts = counts.tolist()
-        if tuple(counts[:6]) != _SHELL_COUNTS or counts[7] != 0:
-            return
-        self.keys, self.vals = keys, vals
-        self.ok = True
-
-
-_SHELL_SEEN = {}                     # (id, id) of table and norms -> what they were, and the plan found for them
-
-
-def _shell_plan(codebook, norms):
-    """The plan of a table, made on its first use outside stream capture; None where there is none."""
-    if codebook.is_inference() or (norms is not None and norms.is_inference()):
-        return None                                            # tensors that do not count their changes
-    hit = _SHELL_SEEN.get((id(codebook), id(norms)))
-    if hit is not None and hit[0]() is codebook and hit[1] == codebook._version and hit[2] == codebook.data_ptr() and (
-            norms is None or (hit[3]() is norms and hit[4] == norms._version and hit[5] == norms.data_ptr())):
-        return hit[6]
-    plan = _find_shell_plan(codebook, norms)
-    if plan is not None:
-        if len(_SHELL_SEEN) >= 8:                              # bounded: an entry keeps its plan
-            _SHELL_SEEN.clear()
-        _SHELL_SEEN[(id(codebook), id(norms))] = (
-            weakref.ref(codebook), codebook._version, codebook.data_ptr(),
-            *((None, 0, 0) if norms is None else (weakref.ref(norms), norms._version, norms.data_ptr())), plan)
-    return plan
-
-
-def _find_shell_plan(codebook, norms):
-    if codebook.dim() != 2 or codebook.shape[1] != 8 or not _SHELL_MIN_ROWS <= codebook.shape[0] <= 65536:
-        return None
-    extra = () if norms is None else _skey(norms)
-    plan = _SHELL_PLANS.get(codebook, extra)
-    if plan is None or (norms is not None and plan.given() is not norms.untyped_storage()):
-        if torch.cuda.is_current_stream_capturing():
-            return None
-        plan = _SHELL_PLANS.put(codebook, _ShellPlan(codebook, norms), extra)
-    return plan if plan.ok else None
+# Rows of a table that may be the whole shell table: the E8 points of norm up to 10 are this many
+# (GLQH_E8_SHELL_MIN_ROWS).  Smaller tables (the secondary one of 3 bpw has 256) are walked.
+_SHELL_MIN_ROWS = 56881
 
 
 def e8_quantize(x, codebook, codebook_norms=None, return_decoded=True):
     """E8ShellCodebook.quantize (glq/codebook.py:227-278) on the GPU: nearest row of
     `codebook` (K, 8) for every row of x (N, 8), lowest index on ties.  fp32 arithmetic in
-    coordinate order, the reference's CPU branch.  Returns (decoded fp32 (N, 8), idx int64)."""
+    coordinate order, the reference's CPU branch.  Returns (decoded fp32 (N, 8), idx int64).
+    The table is read on every call: what its search assumes of the shell table is checked on the
+    device, and nothing is kept."""
+    lib = _lib.load()
     if x.dim() != 2 or x.shape[1] != 8:
         raise RuntimeError(f"x must be (N, 8), got {tuple(x.shape)}")
-    if x.is_cuda and x.shape[0] and codebook.device == x.device:
-        with torch.cuda.device(x.device):
-            plan = _shell_plan(codebook, codebook_norms)
-        if plan is not None:
-            got = host().shell_quantize(x.contiguous().to(torch.float32), plan.table, plan.norms, plan.keys, plan.vals, return_decoded)
-            if got is not None:
-                return got
-    lib = _lib.load()
     xf = x.contiguous().to(torch.float32)
     _chk(xf, "x", torch.float32)
     N = xf.shape[0]
-    idx = torch.empty(N, dtype=torch.int64, device=x.device)
-    dec = torch.empty(N, 8, dtype=torch.float32, device=x.device) if return_decoded else None
-    if N:
-        with torch.cuda.device(x.device):
-            cb = codebook.contiguous().to(torch.float32)
-            norms = (cb * cb).sum(-1) if codebook_norms is None else codebook_norms.contiguous().to(torch.float32)
+    if N == 0:
+        return (torch.empty(0, 8, dtype=torch.float32, device=x.device) if return_decoded else None,
+                torch.empty(0, dtype=torch.int64, device=x.device))
+    with torch.cuda.device(x.device):
+        cb = codebook.contiguous().to(torch.float32)
+        norms = (cb * cb).sum(-1) if codebook_norms is None else codebook_norms.contiguous().to(torch.float32)
+        _chk(cb, "codebook", torch.float32)
+        _chk(norms, "codebook_norms", torch.float32)
+        shell = _SHELL_MIN_ROWS <= cb.shape[0] <= 65536
+        if shell:
+            got = (_host or host()).shell_quantize(xf, cb, norms, return_decoded)
+            if got is not None:
+                return got
+        idx = torch.empty(N, dtype=torch.int64, device=x.device)
+        dec = torch.empty(N, 8, dtype=torch.float32, device=x.device) if return_decoded else None
+        if shell:
+            ws = _ws(lib.glqh_e8_shell_workspace_bytes(N), x.device)
+            check(lib.glqh_e8_shell_quantize(_p(xf), N, _p(cb), _p(norms), cb.shape[0], _p(idx), _p(dec), _p(ws), ws.numel(),
+                                             _stream()))
+        else:
             check(lib.glqh_e8_quantize(_p(xf), _p(cb), _p(norms), N, cb.shape[0], _p(idx), _p(dec), _stream()))
     return dec, idx
 

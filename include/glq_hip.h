@@ -463,17 +463,15 @@ int glqh_fused_linear_e8_folded(const void *x, int x_dtype, int64_t x_stride, in
 int glqh_e8_quantize(const float *x, const float *table_f32, const float *norms_f32, int64_t N,
                      int64_t n_entries, int64_t *idx_out, float *decoded_out, void *stream);
 
-/* The same search on the shell table itself (every E8 point of norm up to 10 and a part of those of norm 12, norms =
- * |row|^2), in a few hundred operations per vector instead of a walk over the table; same indices, bit for bit.
- * Load time, once per table: glqh_e8_shell_index fills the hash of its rows (2^17 keys and values), and
- * counts_out[s] = distinct rows of norm 2s, s = 0..6, counts_out[7] = all others; the table qualifies when these
- * are 1, 240, 2160, 6720, 17520, 30240, any number and 0. */
-int glqh_e8_shell_index(const float *table_f32, const float *norms_f32, int64_t n_entries, uint32_t *keys_out,
-                        int32_t *vals_out, int32_t *counts_out, void *stream);
+/* The same for tables that may be the shell table itself (every E8 point of norm up to 10 and a part of those of
+ * norm 12, norms = |row|^2), in a few hundred operations per vector instead of a walk over the table; same indices,
+ * bit for bit.  The table is read, and checked on the device, by every call; any other table gives the walk's result
+ * in the walk's time.  One with fewer than GLQH_E8_SHELL_MIN_ROWS rows (the points of norm up to 10) cannot be the
+ * shell table: glqh_e8_quantize serves it without the check. */
+#define GLQH_E8_SHELL_MIN_ROWS 56881
 size_t glqh_e8_shell_workspace_bytes(int64_t N);
 int glqh_e8_shell_quantize(const float *x, int64_t N, const float *table_f32, const float *norms_f32, int64_t n_entries,
-                           const uint32_t *keys, const int32_t *vals, int64_t *idx_out, float *decoded_out, void *ws,
-                           size_t ws_bytes, void *stream);
+                           int64_t *idx_out, float *decoded_out, void *ws, size_t ws_bytes, void *stream);
 
 size_t glqh_trellis_quantize_workspace_bytes(int K, int64_t n_tiles);
 

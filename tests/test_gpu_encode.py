@@ -84,7 +84,95 @@ def test_e8_quantize_on_the_shell_table_equals_the_table_walk(N, scale):
     assert torch.equal(dec, wdec)
     assert torch.equal(ext.e8_quantize(X, cb, norms)[1], walk)   # the caller's norms
     norms[5] += 0.5                                              # a table that no longer qualifies, same memory
-    assert ext._shell_plan(cb, norms) is None
+    X, walk, wdec = X[:2000], walk[:2000], wdec[:2000]
+    _lib.check(_lib.load().glqh_e8_quantize(X.data_ptr(), cb.data_ptr(), norms.data_ptr(), X.shape[0], 65536, walk.data_ptr(),
+                                            wdec.data_ptr(), torch.cuda.current_stream().cuda_stream))
+    dec, idx = ext.e8_quantize(X, cb, norms)
+    assert torch.equal(idx, walk) and torch.equal(dec, wdec)
+
+
+def _walk(X, cb, norms):
+    """Every row against every vector."""
+    from glq_amd import _lib
+    idx, dec = torch.empty(X.shape[0], dtype=torch.int64, device=DEV), torch.empty_like(X)
+    _lib.check(_lib.load().glqh_e8_quantize(X.data_ptr(), cb.data_ptr(), norms.data_ptr(), X.shape[0], cb.shape[0], idx.data_ptr(),
+                                            dec.data_ptr(), torch.cuda.current_stream().cuda_stream))
+    return dec, idx
+
+
+def _changed_table(how):
+    cb = torch.from_numpy(O.e8_table()).to(DEV)
+    if how == "rows in another order":                           # still the shell table
+        return cb[torch.randperm(65536, generator=torch.Generator().manual_seed(1)).to(DEV)].contiguous()
+    if how == "fewer rows of norm 12":
+        return cb[:60000].contiguous()
+    if how == "a row twice, one missing":                        # in number they are as many as before
+        cb[300] = cb[40000]
+    elif how == "a row of norm 12 twice":
+        cb[65535] = cb[60000]
+    elif how == "a row off the lattice":
+        cb[1234, 0] += 0.25
+    elif how == "a row that is not finite":
+        cb[50000, 3] = float("nan")
+    elif how == "scaled":
+        cb *= 2
+    return cb
+
+
+@pytest.mark.parametrize("how", ["rows in another order", "fewer rows of norm 12", "a row twice, one missing", "a row of norm 12 twice",
+                                 "a row off the lattice", "a row that is not finite", "scaled"])
+@pytest.mark.parametrize("N", [3, 1500])
+def test_e8_quantize_reads_its_table_on_every_call(how, N):
+    """The same tensor with other contents, written where PyTorch counts no change, and tables that are almost the
+    shell table: always the walk's rows."""
+    from glq_amd import ext
+    say("e8 shell search, changed table", how, N)
+    cb = torch.from_numpy(O.e8_table()).to(DEV)
+    X = torch.randn(N, 8, generator=torch.Generator().manual_seed(N)) * 1.5
+    X[0] = 0.0                                                   # ties
+    X[1] = torch.from_numpy(O.e8_table())[40000]
+    X = X.to(DEV)
+    norms = (cb * cb).sum(-1)
+    dec, idx = ext.e8_quantize(X, cb, norms)
+    wdec, widx = _walk(X, cb, norms)
+    assert torch.equal(idx, widx) and torch.equal(dec, wdec)
+    new = _changed_table(how)
+    version = cb._version
+    cb.data[:new.shape[0]].copy_(new)
+    cb2, norms2 = cb[:new.shape[0]], norms[:new.shape[0]]
+    norms.data.copy_((cb.data * cb.data).sum(-1))
+    assert cb._version == version
+    for given in (norms2, None):
+        dec, idx = ext.e8_quantize(X, cb2, given)
+        wdec, widx = _walk(X, cb2, norms2)
+        assert torch.equal(idx, widx) and torch.equal(dec, wdec)
+
+
+def test_e8_quantize_under_capture():
+    """Captured on its first use, replayed on other vectors and with other table contents."""
+    from glq_amd import ext
+    say("e8 shell search under capture")
+    g = torch.Generator().manual_seed(0)
+    cb = torch.from_numpy(O.e8_table()).to(DEV)
+    norms = (cb * cb).sum(-1)
+    X = torch.zeros(700, 8, device=DEV)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        dec, idx = ext.e8_quantize(X, cb, norms)
+    for turn in range(4):
+        X.copy_(torch.randn(700, 8, generator=g) * (1 + turn))
+        if turn == 2:
+            cb.copy_(_changed_table("rows in another order"))
+            norms.copy_((cb * cb).sum(-1))
+        if turn == 3:
+            cb.copy_(_changed_table("a row twice, one missing"))
+            norms.copy_((cb * cb).sum(-1))
+        graph.replay()
+        torch.cuda.synchronize()
+        wdec, widx = _walk(X, cb, norms)
+        assert torch.equal(idx, widx) and torch.equal(dec, wdec), turn
 
 
 @pytest.mark.parametrize("K", [1, 2, 3, 4])

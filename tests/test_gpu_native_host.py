@@ -1,6 +1,7 @@
 """The native host path (csrc/host.cpp) against the Python route of the same calls: equal bit for bit where it
 serves a call, None -- and the Python route -- where something is not what it recognises (needs an MI355X)."""
 import copy
+import gc
 
 import pytest
 import torch
@@ -201,6 +202,7 @@ def test_a_failing_bias_addition_keeps_no_output():
     x = torch.randn(64, 2048, generator=torch.Generator().manual_seed(0)).to(DEV, torch.bfloat16)
     lin(x)
     lin.bias = torch.zeros(511, device=DEV).half()
+    gc.collect()                                                 # what earlier tests left in reference cycles
     held = []
     for _ in range(3):
         with pytest.raises(RuntimeError, match="size"):
