@@ -710,19 +710,24 @@ extern "C" int glqh_fused_linear_trellis_3inst_noalloc(
 // Few tokens of a group: one transform launch and one launch of the small-batch kernel over the strips of all layers, or
 // the fused-input launch, every workgroup of which repeats the transform of all tokens for its K slot (as many terms per
 // element as its Hadamard block has slices).  Whole grouped call, kernel us, folded / separate:
-//   4 bits, 1 token   2048-wide q/k/v 10.3 / 13.9, 3072 13.9 / 14.0, 4096 17.4 / 17.6, 5248 20.1 / 18.0, 8192 30.0 / 28.3;
-//                     gate/up 2048 -> 2 x 11008 17.0 / 20.2, 3392 -> 2 x 7040 20.8 / 20.0, 4096 -> 2 x 8192 22.6 / 23.2
+//   4 bits, 1 token   three equal layers: 2048 wide 10.6 / 12.1, 3072 14.2 / 15.1, 3392 16.3 / 15.9, 3584 16.0 / 16.6,
+//                     3840 15.0 / 17.1, 4032 18.6 / 17.2, 4096 16.1 / 18.2, 4352 20.2 / 18.5, 5248 26.5 / 21.4; two
+//                     layers of 56M weights: 3584 20.0 / 18.4, 3840 20.0 / 19.3, 4096 19.8 / 19.2, of 80M: 25.2 / 23.3,
+//                     25.4 / 22.6, 23.0 / 22.4 (2 bits 27.0 / 24.6, 26.3 / 23.7, 26.3 / 24.2)
 //   4 + 2, 1 token    3072 16.6 / 17.0, 4096 23.1 / 21.2, 5248 26.5 / 23.5; 3392 -> 2 x 7040 30.0 / 27.5
 //   4 bits, 2 tokens  960 14.3 / 12.2, 2048 12.8 / 13.3, 3072 18.3 / 14.4; 1024 -> 2 x 2560 11.6 / 12.8,
 //                     2048 -> 2 x 11008 19.6 / 20.9, 3392 -> 2 x 7040 25.1 / 20.8
 //   4 bits, 4 tokens  960 18.0 / 12.6, 2048 15.8 / 13.4; 2048 -> 2 x 11008 22.5 / 21.5
 // and one token of single-stage groups above 96M weights (4096 -> 2 x 14336: 37.4 / 33.9), below 32M (11008 -> 2048, a
-// group of one: 14.3 / 18) never.  The fused-input launches
-// serve up to four tokens, one of stacked layers.
+// group of one: 14.3 / 18) never.  Widths of whole 256-column slots fold better (no workgroup transforms a ragged tail
+// beside its share of the large block): up to 4096 columns, where slots are that short, they cross at 48M weights
+// instead of 32M (40M: 15.1 / 15.9 us, 56M: 20.1 / 19.2).  The fused-input launches serve up to four tokens, one of
+// stacked layers.
 static bool tr_group_plain(int64_t total_m_pad, int64_t n_pad, int64_t B, bool stacked) {
     if (!tr_fuse_input_enabled() || B > 4 || (stacked && B > 1)) return true;
     const int64_t w = total_m_pad * n_pad;
-    if (B == 1) return (n_pad > 3072 && (stacked || n_pad != 4096) && w > ((int64_t)32 << 20)) || (!stacked && w > ((int64_t)96 << 20));
+    const int64_t folds = !stacked && n_pad <= 4096 && n_pad % 256 == 0 ? 48 : 32;
+    if (B == 1) return (n_pad > 3072 && w > folds << 20) || (!stacked && w > ((int64_t)96 << 20));
     return B > 2 || n_pad > 2048 || (n_pad & (n_pad - 1)) != 0;
 }
 // The grouped call at many tokens: more than 64 tokens, at most four layers.  The K split of a group is at most

@@ -81,6 +81,9 @@ def test_grouped_many_tokens(ms, n, B, K, shared_sv):
     ((4096, 32), 576, 700, (4, 1), False),
     # rows between those of one layer and of the group change the K plan: widths 2112..3072 at 5..16 tokens
     ((5248, 5248), 2560, 8, (4,), False), ((4096, 4096), 3072, 16, (4, 2), False), ((3072, 3072, 3072), 2816, 5, (2,), True),
+    # one token, either side of the weights from which the transform is a launch of its own (whole 256-column slots: 48M)
+    ((6528, 6528), 3840, 1, (2,), False), ((6560, 6560), 3840, 1, (2,), False), ((4096, 4096, 4096), 4096, 1, (4,), False),
+    ((4960, 4960), 3392, 1, (4,), True),
 ])
 def test_grouped_calls_against_single_layers(ms, n, B, bits, shared_sv):
     from glq_amd import ext, hadamard as H
