@@ -1306,20 +1306,32 @@ struct moe_plan {
     size_t part_bytes;
 };
 
-// From this many (token, choice) slots on the rows are grouped by expert and every expert's stream is read
-// once per 16 of its rows; below, every slot reads its expert's stream for itself (no routing launch, no
-// separate input transforms).  The grouped form pays three more launches and wins once slots share experts: measured on 128 experts of
-// 2048 -> 2 x 768 -> 2048 with 8 choices, 32 slots 51.7 (per slot) against 54.7 us (grouped), 48 slots 69.0 / 67.8,
-// 64 slots 81.3 / 72.3, 88 slots 105.1 / 78.3.  GLQ_MOE_GROUP_MIN overrides (read once).
-static int64_t moe_group_min(int64_t n_experts) {
+// Whether the rows of this many (token, choice) slots are grouped by expert and every expert's stream is read once per
+// 16 of its rows; otherwise every slot reads its expert's stream for itself (no routing launch, no separate input
+// transforms).  The grouped form pays three more launches and wins once the reads that slots of one expert share are
+// worth more: about slots^2 / (2 * experts) of them with routing at random, times the expert's bytes; a larger constant
+// part stands for what it gains and loses beside them.  The line is fitted to 707 calls in both forms, 8-512 experts of
+// 1024 -> 2 x 512 to 4096 -> 2 x 1536, 2-6 bits, 8-256 slots; it costs 0.6% on average against the better form each
+// time, three eighths of the experts 3.2%, three quarters 5.7%.  4 bits, us, slot by slot / grouped:
+//   16 experts    1024 x 512 at 32 slots 30.0 / 35.7, 2048 x 768 at 16 / 24 slots 34.4 / 38.2, 42.4 / 40.6, 4096 x 1536 at
+//                 16 slots 75.3 / 63.4
+//   32 experts    1024 x 512 at 48 / 64 slots 34.8 / 35.4, 36.6 / 35.4, 2048 x 768 at 24 / 40 42.7 / 45.3, 54.2 / 48.6
+//   64 experts    1024 x 512 at 64 / 96 slots 38.3 / 42.5, 45.6 / 42.1, 2048 x 768 at 32 / 40 48.1 / 51.2, 54.2 / 51.6
+//   128 experts   1024 x 512 at 96 / 128 slots 47.5 / 48.8, 56.1 / 49.5, 2048 x 768 at 40 / 56 55.8 / 57.2, 75.4 / 68.9,
+//                 4096 x 1536 at 16 / 32 77.9 / 78.8, 123.6 / 120.4
+// Four slots per expert are grouped however small the experts are.  GLQ_MOE_GROUP_MIN=<n> (read once): from n slots on.
+static bool moe_grouped(int64_t n_slots, int64_t n_experts, const glqh_moe_proj *w13, const glqh_moe_proj *w2) {
     static const int64_t v = [] {
         const char *e = getenv("GLQ_MOE_GROUP_MIN");
         const long long x = e && *e ? atoll(e) : 0;
         return (int64_t)(x > 0 ? x : 0);
     }();
-    if (v > 0) return v;
-    const int64_t d = 3 * n_experts / 8;
-    return d < 16 ? 16 : d;
+    if (v > 0) return n_slots >= v;
+    if (n_slots < 16) return false;
+    double bytes = 0.0;                                        // of one expert
+    for (const glqh_moe_proj *w : {w13, w2})
+        bytes += 2.0 * (double)w->packed_rows * (double)(w->packed_cols + (w->packed2 ? w->packed2_cols : 0));
+    return n_slots >= 4 * n_experts || (double)n_slots * (double)n_slots * bytes >= 750e6 + 12e6 * (double)n_experts;
 }
 
 // From this many rows per expert on average (slots / experts that can have rows) the grouped form hands over to
@@ -1334,9 +1346,9 @@ static int64_t moe_tile_min_rows() {
     return v;
 }
 
-static bool moe_tile_form(int64_t n_slots, int64_t n_experts) {
+static bool moe_tile_form(int64_t n_slots, int64_t n_experts, bool grouped) {
     const int64_t live = n_experts < n_slots ? n_experts : n_slots, mn = moe_tile_min_rows();
-    return mn > 0 && n_slots >= moe_group_min(n_experts) && n_slots >= mn * live;
+    return mn > 0 && grouped && n_slots >= mn * live;
 }
 
 // GLQ_MOE_FUSE=0 (read once): the launches between and after the decode launches stay separate at every slot count
@@ -1352,7 +1364,7 @@ static bool moe_fuse_enabled() {
 // 112.6 fused, 512 slots 147.1 / 148.2, 1024 slots 161.2 / 161.5, 2048 slots 222 / 215, 8192 slots 531 / 493)
 constexpr int MOE_FUSE_MIN_SLOTS = 1024;
 
-static int moe_proj_plan(const glqh_moe_proj *w, int64_t n_slots, int64_t n_experts, const char *what, moe_plan *p) {
+static int moe_proj_plan(const glqh_moe_proj *w, int64_t n_slots, int64_t n_experts, bool grouped, const char *what, moe_plan *p) {
     GLQH_REQUIRE(w && w->packed && w->su_f16 && w->sv_f16 && w->wscale_dev, "routed experts %s: null pointer", what);
     if (tr_bits_from_packed(w->packed_cols, 0, &p->R1) || tr_check_shape(w->m_pad, w->n_pad, w->packed_rows)) return 1;
     p->R2 = 0;
@@ -1369,11 +1381,11 @@ static int moe_proj_plan(const glqh_moe_proj *w, int64_t n_slots, int64_t n_expe
     GLQH_REQUIRE(w->n_blocks_n > 1 ? (w->bn_meta_dev != nullptr && w->blocks_n != nullptr) : pow2_n,
                  "routed experts %s: input block sizes missing", what);
     p->tile = 0;
-    if (moe_tile_form(n_slots, n_experts)) {
+    if (moe_tile_form(n_slots, n_experts, grouped)) {
         p->tile = 1;
         p->S = 0;
         p->ks = 1;
-    } else if (n_slots >= moe_group_min(n_experts)) {
+    } else if (grouped) {
         // about four workgroups per CU if every expert that can have rows has some
         const int64_t nkp = w->n_pad / 32, wgs = ((w->m_pad + 63) / 64) * (n_experts < n_slots ? n_experts : n_slots);
         int64_t ks = ((int64_t)glqh_device_cus() * 4 + wgs - 1) / wgs;
@@ -1388,7 +1400,7 @@ static int moe_proj_plan(const glqh_moe_proj *w, int64_t n_slots, int64_t n_expe
     // both stages in one launch: the per-slot form and the grouped form's passes of 16 rows add the sums in fp32, the
     // tile form multiplies with one fp16 operand; the grouped form's passes of up to 64 rows keep a launch per stage
     p->fuse2 = p->R2 && p->R1 == 4 && tr_fuse_stages_enabled() &&
-               (p->tile || n_slots < moe_group_min(n_experts) || !glqh_moe_grouped_wide((int)n_slots, (int)n_experts));
+               (p->tile || !grouped || !glqh_moe_grouped_wide((int)n_slots, (int)n_experts));
     p->ks_all = p->R2 && !p->fuse2 ? 2 * p->ks : p->ks;
     p->part_bytes = align256((size_t)p->ks_all * n_slots * w->m_pad * sizeof(float));
     return 0;
@@ -1403,7 +1415,7 @@ struct moe_ws {
 };
 
 static moe_ws moe_ws_layout(const glqh_moe_proj *w13, const glqh_moe_proj *w2, const moe_plan &p13, const moe_plan &p2,
-                            int64_t num_tokens, int64_t n_slots, int64_t n_experts) {
+                            int64_t num_tokens, int64_t n_slots, int64_t n_experts, bool grouped) {
     moe_ws l;
     size_t o = 0;
     l.part13 = o; o += p13.part_bytes;
@@ -1412,7 +1424,7 @@ static moe_ws moe_ws_layout(const glqh_moe_proj *w13, const glqh_moe_proj *w2, c
     l.part2 = o; o += p2.part_bytes;
     l.y = o; o += align256((size_t)n_slots * w2->out_features * sizeof(f16));
     l.perm = l.pexp = l.offs = l.route = l.xhat = o;
-    if (n_slots >= moe_group_min(n_experts)) {
+    if (grouped) {
         l.perm = o; o += align256((size_t)n_slots * sizeof(int));
         l.pexp = o; o += align256((size_t)n_slots * sizeof(int));
         l.offs = o; o += align256((size_t)(n_experts + 1) * sizeof(int));
@@ -1435,10 +1447,11 @@ extern "C" size_t glqh_fused_moe_trellis_workspace_bytes(int64_t num_tokens, int
                                                          const glqh_moe_proj *w13, const glqh_moe_proj *w2) {
     if (glqh_init() != 0 || num_tokens < 1 || top_k < 1 || num_experts < 1 || !w13 || !w2) return 0;
     const int64_t n_slots = num_tokens * top_k;
+    const bool grouped = moe_grouped(n_slots, num_experts, w13, w2);
     moe_plan p13, p2;
-    if (moe_proj_plan(w13, n_slots, num_experts, "w13", &p13) || moe_proj_plan(w2, n_slots, num_experts, "w2", &p2))
+    if (moe_proj_plan(w13, n_slots, num_experts, grouped, "w13", &p13) || moe_proj_plan(w2, n_slots, num_experts, grouped, "w2", &p2))
         return 0;
-    return moe_ws_layout(w13, w2, p13, p2, num_tokens, n_slots, num_experts).total;
+    return moe_ws_layout(w13, w2, p13, p2, num_tokens, n_slots, num_experts, grouped).total;
 }
 
 // one projection, rows grouped by expert: input transform of the rows, then one decode launch per stage
@@ -1527,13 +1540,14 @@ extern "C" int glqh_fused_moe_trellis_3inst(const void *x, int x_dtype, int64_t 
     GLQH_REQUIRE(activation_type >= 0 && activation_type <= 2,
                  "routed experts: gated activations 0 (silu), 1 (gelu-tanh), 2 (relu2) only, got %d", activation_type);
     const int n_slots = (int)(num_tokens * top_k);
+    const bool grouped = moe_grouped(n_slots, num_experts, w13, w2);
     moe_plan p13, p2;
-    if (moe_proj_plan(w13, n_slots, num_experts, "w13", &p13) || moe_proj_plan(w2, n_slots, num_experts, "w2", &p2))
+    if (moe_proj_plan(w13, n_slots, num_experts, grouped, "w13", &p13) || moe_proj_plan(w2, n_slots, num_experts, grouped, "w2", &p2))
         return 1;
     GLQH_REQUIRE(w13->out_features == 2 * intermediate_size && w2->in_features == intermediate_size,
                  "routed experts: w13 yields %lld values, w2 takes %lld, intermediate size %lld (gate | up)",
                  (long long)w13->out_features, (long long)w2->in_features, (long long)intermediate_size);
-    const moe_ws l = moe_ws_layout(w13, w2, p13, p2, num_tokens, n_slots, num_experts);
+    const moe_ws l = moe_ws_layout(w13, w2, p13, p2, num_tokens, n_slots, num_experts, grouped);
     GLQH_REQUIRE(ws && ws_bytes >= l.total, "routed experts: workspace of %zu bytes needed, got %zu", l.total, ws_bytes);
     hipStream_t st = (hipStream_t)stream;
     char *base = (char *)ws;
@@ -1541,7 +1555,6 @@ extern "C" int glqh_fused_moe_trellis_3inst(const void *x, int x_dtype, int64_t 
     f16 *h = (f16 *)(base + l.h), *hact = (f16 *)(base + l.a), *yslot = (f16 *)(base + l.y);
     int *perm = (int *)(base + l.perm), *offs = (int *)(base + l.offs);
     void *xhat = base + l.xhat;
-    const bool grouped = n_slots >= moe_group_min(num_experts);
     GLQH_REQUIRE(!grouped || num_experts <= 65535, "routed experts: at most 65535 experts, got %lld", (long long)num_experts);
     int *pexp = (int *)(base + l.pexp);
     if (grouped && glqh_launch_moe_route(topk_ids, n_slots, (int)num_experts, perm, pexp, offs, (int *)(base + l.route), st))

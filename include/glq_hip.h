@@ -273,9 +273,10 @@ size_t glqh_fused_moe_trellis_workspace_bytes(int64_t num_tokens, int64_t top_k,
  * synchronisation, no allocation: capturable).  Replaces glq_fused_moe_trellis_3inst_cuda
  * (glq/csrc/glq_cuda.cu:5030-5250; grouped matmul glq/csrc/glq_trellis.cu:1475-1540) behind
  * torch.ops.glq.fused_moe_trellis_3inst (glq_vllm/custom_ops.py:22-36).  With few (token,
- * choice) slots every slot is one fused-input GEMV on its expert's stream; from
- * max(16, 3/8 num_experts) slots on a routing launch groups the slots by expert and every
- * expert's stream is read once per 16 of its rows (GLQ_MOE_GROUP_MIN sets that count), once
+ * choice) slots every slot is one fused-input GEMV on its expert's stream; from 16 slots on,
+ * where slots^2 * (bytes of an expert) >= 750 MB + 12 MB * num_experts or there are four slots per
+ * expert, a routing launch groups the slots by expert and every expert's stream is read once per 16
+ * of its rows (GLQ_MOE_GROUP_MIN=<n>: from n slots on), once
  * per up to 64 rows from an average of 12 rows per expert on (GLQ_MOE_WIDE_MIN_ROWS); from an
  * average of 24 rows per expert on (GLQ_MOE_TILE_MIN_ROWS, 0 = never) the expert-sorted slots go
  * through the many-token tile kernel in runs of up to 128-512 rows of one expert, the decoded

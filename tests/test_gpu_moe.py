@@ -217,7 +217,7 @@ def test_refusals(ext):
                                                  (256, 128, 200, 3, 0), (320, 192, 300, 2, 2), (256, 128, 530, 2, 0),
                                                  (256, 128, 1100, 4, 0), (320, 192, 600, 2, 2)])
 def test_many_slots_grouped_by_expert(ext, hidden, inter, T, K, K2):
-    """From max(16, 3/8 of the experts) slots on the rows are grouped by expert.  Skewed routing: every token's first choice is
+    """From four slots per expert on (with small experts) the rows are grouped by expert.  Skewed routing: every token's first choice is
     expert 2 (more than two tiles of 16 rows for it), expert 5 gets nothing, some ids are out of range.  From an
     average of 12 rows per expert on, a pass over an expert's stream takes up to 64 of its rows: the cases give
     expert 2 one pass of 16 (T = 16), of 32 (24), of 64 (33, 40), 64 + 32 (90) and 64 + 16 (80) rows.  From 48 rows
@@ -257,6 +257,21 @@ def test_experts_of_four_five_eight_and_nine_rows(ext, hidden, inter, K2):
     y = ext.glq_fused_moe_trellis_3inst_cuda(x.to(DEV), t(ids), t(w), *ex.device_args(0))
     ref = ex.oracle(x.float().numpy(), ids, w, 0)
     assert max(rel(y[i], ref[i]) for i in range(T)) < 2 * TOL
+
+
+@pytest.mark.parametrize("slots,hidden,inter,K2", [(22, 1088, 1024, 0), (23, 1088, 1024, 0), (16, 1024, 1088, 3), (17, 1024, 1088, 3)])
+def test_either_side_of_the_grouping_line(ext, slots, hidden, inter, K2):
+    """Six experts whose bytes put the line between 22 and 23 slots, and between 16 and 17 with a second stage of three
+    bits."""
+    say("moe grouping line", slots, hidden, inter, K2)
+    ex = experts(6, hidden, inter, 4, K2, seed=9)
+    rng = np.random.default_rng(slots)
+    ids = rng.integers(0, 6, (slots, 1)).astype(np.int64)
+    w = rng.random((slots, 1)).astype(np.float32)
+    x = torch.from_numpy(rng.standard_normal((slots, hidden)).astype(np.float32)).bfloat16()
+    y = ext.glq_fused_moe_trellis_3inst_cuda(x.to(DEV), t(ids), t(w), *ex.device_args(0))
+    ref = ex.oracle(x.float().numpy(), ids, w, 0)
+    assert max(rel(y[i], ref[i]) for i in range(slots)) < 2 * TOL
 
 
 @pytest.mark.parametrize("hidden,inter", [(256, 4096), (8192, 128)])
@@ -331,8 +346,8 @@ def test_both_forms_on_every_case_in_a_fresh_process(group_min, wide_min, tile_m
 @pytest.mark.parametrize("T", [1, 4, 40, 140])
 def test_qwen3_moe_expert_shapes(ext, T):
     """Expert shapes of a Qwen3-MoE layer (hidden 2048, intermediate 768, top-8), 16 of the experts,
-    4 bpw, bf16 activations: every chosen expert decoded whole by the oracle.  One and four tokens run slot by
-    slot, 40 tokens grouped by expert (20 rows each on average), 140 tokens through the tile kernel (70 rows
+    4 bpw, bf16 activations: every chosen expert decoded whole by the oracle.  One token runs slot by slot, four
+    and 40 tokens grouped by expert (2 and 20 rows each on average), 140 tokens through the tile kernel (70 rows
     each, runs of up to 128 positions, 1120 slots: with the fused launches around the second projection)."""
     say("moe qwen3 shapes", T)
     ex = experts(16, 2048, 768, seed=3)
