@@ -397,11 +397,12 @@ input_rht_wide_multi_kernel(const XT *__restrict__ x, int64_t x_stride, rht_in_w
 // Every thread of the workgroup calls.
 // (the first half, what a thread reads: callers that transform several rows in turn request the next row's
 // sums before they transform this one's)
-// acc += the K slots' sums at p, p + stride, ... in order, four of them in flight: one at a time a thread waits for
-// memory once per slot (37 tokens x (11008 -> 2048) at 6 bpw, whole call 33.5 -> 30.7 us)
-template <int E, typename PT>
+// acc += the K slots' sums at p, p + stride, ... in order, C of them in flight.  One at a time a thread waits for memory
+// once per slot: four, for eight elements, take 37 tokens x (11008 -> 2048) at 6 bpw, whole call, from 33.5 to 30.7 us.
+// (Sixteen elements: their registers are the occupancy.  moe_final_row keeps the next choice's sums beside this one's
+// and has one K slot as a rule: one, 112 -> 88 registers.)
+template <int E, int C, typename PT>
 __device__ __forceinline__ void output_wide_sum(float (&acc)[E], const PT *p, int64_t stride, int ks) {
-    constexpr int C = E == 8 ? 4 : 1;                            // (sixteen elements: their registers are the occupancy)
     for (int k0 = 0; k0 < ks; k0 += C) {
         float t[C][E];
 #pragma unroll
@@ -421,7 +422,7 @@ __device__ __forceinline__ void output_wide_sum(float (&acc)[E], const PT *p, in
     }
 }
 
-template <int E>
+template <int E, int C = (E == 8 ? 4 : 1)>
 __device__ __forceinline__ void output_wide_load(float (&v)[E], const glqh_ysrc &src, int64_t b, int m_pad,
                                                  const rht_slice &blk, bool active, int te) {
     const int i = E * te;
@@ -440,8 +441,8 @@ __device__ __forceinline__ void output_wide_load(float (&v)[E], const glqh_ysrc 
 #pragma unroll
                 for (int e = 0; e < E; ++e) acc[e] = 0.0f;
                 const int64_t eoff = ebase + st * src.part_sstride;
-                if (src.part_f16) output_wide_sum<E, f16>(acc, (const f16 *)src.part + eoff, src.part_kstride, src.ksplit);
-                else output_wide_sum<E, float>(acc, src.part + eoff, src.part_kstride, src.ksplit);   // uniform over the launch
+                if (src.part_f16) output_wide_sum<E, C, f16>(acc, (const f16 *)src.part + eoff, src.part_kstride, src.ksplit);
+                else output_wide_sum<E, C, float>(acc, src.part + eoff, src.part_kstride, src.ksplit);   // uniform over the launch
                 const float sc = st == 0 ? src.scale[0] : st == 1 ? src.scale[1]
                                : st == 2 ? src.scale[2] : src.scale[3];
 #pragma unroll
@@ -1316,7 +1317,7 @@ __device__ __forceinline__ void moe_final_row(const moe_out_args &a, const float
         const int64_t e = a.topk_ids[slot];
         ch.valid = e >= 0 && e < a.n_experts;
         const glqh_ysrc src = moe_src(a, ch.valid ? a.wscale_dev[e] : 0.0f);
-        output_wide_load<E>(ch.v, src, slot, a.m_pad, blk, active && ch.valid, role.te);
+        output_wide_load<E, 1>(ch.v, src, slot, a.m_pad, blk, active && ch.valid, role.te);
         ch.w = 0.0f;
 #pragma unroll
         for (int j = 0; j < E; ++j) ch.f[j] = 0.0f;
@@ -1658,7 +1659,9 @@ int glqh_launch_moe_final(const float *part, int ks, int part_f16, int num_token
                             (int)out_features, (int)m_pad};
     // (sixteen elements per thread on half as many threads: slower, the whole call of 32768 slots x 2048 rows 701 -> 714 us
     // -- the registers of two choices in flight cost occupancy)
-    const int lwg = wide_log_wg(ilog2(max_bs), num_tokens, m_pad);
+    // A workgroup holds the largest block, not 4096 points: two tokens of 2048 rows in one of 512 threads leave two
+    // workgroups per CU that wait for each other's barriers, where five of 256 threads fit (32768 slots x 2048 rows 90 -> 74 us).
+    const int lwg = std::min(WIDE_LOG_WG, std::max(WIDE_LOG_WG_MIN, ilog2(max_bs)));
     const dim3 grid((unsigned)wide_grid<false>(margs.canon, lwg, num_tokens)), threads(1u << (lwg - 3));
     const size_t lds = wide_lds_bytes(ilog2(max_bs), lwg, false);
 #define GLQH_MOE_FINAL(YT, BIG)                                                                                  \
