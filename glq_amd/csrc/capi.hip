@@ -1158,7 +1158,8 @@ extern "C" int glqh_fused_linear_trellis_3inst_group_rvq2(const void *x, int x_d
     GLQH_REQUIRE(in_features >= 1 && in_features <= n_pad, "trellis two-stage group: in_features exceeds n_pad");
     GLQH_REQUIRE(y_stride > 0, "trellis two-stage group: y_stride must be positive");
     if (B > TR_GROUP_MANY_MIN) {
-        GLQH_REQUIRE(tr_fuse_stages_enabled(), "trellis two-stage group: more than 16 tokens need both streams in one operand");
+        GLQH_REQUIRE(tr_fuse_stages_enabled(), "trellis two-stage group: %lld tokens need both streams in one operand "
+                                               "(GLQ_TRELLIS_FUSE_STAGES=0)", (long long)B);
         return tr_group_many(x, x_dtype, x_stride, B, shards, stage2, n_shards, blocks_n, n_blocks_n, bn_meta_dev, in_features, n_pad,
                              y_dtype, y_stride, ws, ws_bytes, st);
     }
@@ -1196,7 +1197,8 @@ extern "C" int glqh_fused_linear_trellis_3inst_group_rvq2(const void *x, int x_d
     }
     int steps = 0, ks = 0;
     if (B > TR_GROUP_SMALL_MAX) {
-        GLQH_REQUIRE(tr_fuse_stages_enabled(), "trellis two-stage group: more than 16 tokens need both streams in one operand");
+        GLQH_REQUIRE(tr_fuse_stages_enabled(), "trellis two-stage group: %lld tokens need both streams in one operand "
+                                               "(GLQ_TRELLIS_FUSE_STAGES=0)", (long long)B);
         if (tr_group_tiles(x, x_dtype, x_stride, B, sv, packed, 4, packed2, R2, rs2, n_shards, blocks_n, n_blocks_n, bn_meta_dev,
                            in_features, n_pad, ws, ws_bytes, st, &c))
             return 1;
