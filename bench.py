@@ -370,7 +370,7 @@ def extras(torch, ext, dev):
             us = _graph_time(torch, lambda: [ext.glq_dequant_matmul_cuda(xh, a, cb, 0.02, b, cb, 1 / 3.0)
                                              for a, b in qs], len(qs))
             out[f"e8_2stage_gemv_4096x14336_B{B}_GBs"] = round(m * (n // 8) * 4 / us / 1e3, 1)
-            hbm("e8_mma_kernel<2,FOLD> (whole unfused call; algorithmic bytes = 2 B per index and stage)",
+            hbm("e8_few_kernel<2> (whole unfused call; algorithmic bytes = 2 B per index and stage)",
                 f"configs[2]: E8 two-stage 4 bpw 4096x14336, {B} token(s), 10 index sets in rotation",
                 m * (n // 8) * 4, us)
         # the same kernel where the launch's fixed costs amortise: 16384 x 16384, two stages, uniformly random
@@ -385,7 +385,7 @@ def extras(torch, ext, dev):
             us = _graph_time(torch, lambda: [ext.glq_dequant_matmul_cuda(xh, a, cb, 0.02, b, cb, 1 / 3.0) for a, b in big],
                              len(big))
             out["e8_2stage_gemv_16384x16384_B1_GBs"] = round(mm * (nn // 8) * 4 / us / 1e3, 1)
-            hbm("e8_mma_kernel<2,FOLD> (+ K-slot sum where the plan splits K across workgroups)",
+            hbm("e8_few_kernel<2> (+ K-slot sum where the plan splits K across workgroups)",
                 "E8 two-stage 4 bpw 16384x16384, 1 token, 3 index sets of 134 MB in rotation", mm * (nn // 8) * 4, us)
             for a, b in big:
                 ext.e8_release(a, b)
