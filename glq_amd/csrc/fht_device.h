@@ -255,7 +255,9 @@ __device__ __forceinline__ void fht_thread_levels(float (&v)[E]) {
 
 // Blocks of 16..512 points side by side in one wave, sixteen elements per lane: log_bs is the lane's own block's.
 // Blocks are aligned to their size, so a lane's partner at a level below its block's size is in the same block; a
-// lane whose block is smaller takes no part in the level.
+// lane whose block is smaller takes no part in the level: it adds its partner's value times zero, so an infinity or NaN
+// in one block makes its neighbours NaN.  The caller's row is an input transform, every output sums over all of its
+// blocks, and none of that token's is finite either way.
 __device__ __forceinline__ void fht_lanes_ragged(float (&v)[16], int log_bs, int lane) {
     fht_thread_levels<16>(v);
     fht_lane_level<0>(v, lane, log_bs > 4);

@@ -431,15 +431,15 @@ class _TrellisShard(C.Structure):
 
 def glq_fused_linear_trellis_3inst_group(x, shards, blocks_n, blocks_n_meta, in_features, n_pad,
                                          out_dtype=None, decode_only=False, separate=False):
-    """Several separately quantized trellis layers on the same x (fused q/k/v, gate/up) with
-    one decode launch and one output-transform launch: the per-shard loop of the reference's
-    vLLM linear method (glq_vllm/linear_method.py:664-710) as a single call.
+    """Several separately quantized trellis layers on the same x (fused q/k/v, gate/up) with shared
+    launches: the per-shard loop of the reference's vLLM linear method
+    (glq_vllm/linear_method.py:664-710) as a single call.
 
     shards: sequence of (sv, su, trellis_packed, wscale, out_features, m_pad).  Returns one
     (B, sum(out_features)) tensor, shard s in columns [off_s, off_s + out_features_s).
-    Up to four layers.  1..4 tokens: one decode launch; 5..64: one decode launch per layer (the small-batch
-    kernel to 16 tokens, the small-tile kernel above) between one transform launch per sign vector and one
-    finishing launch; more than 64: one launch of the many-token kernel over the row tiles of all of them.
+    Up to four layers, one decode launch over the rows of all of them and one finishing launch: 1..4 tokens the
+    fused-input launch or, by width and weights, a transform launch and the small-batch kernel; 5..16 those two;
+    17..64 tokens a transform launch and the small-tile kernel; more than 64 the many-token kernel.
     Single-stage layers of one rate and block_decompose block sizes; raises RuntimeError otherwise (callers then use the per-layer op).
     decode_only=True stops after the decode launch (no output transform, returns None): a measurement
     hook.  separate=True (more than 64 tokens): a list of contiguous (B, out_features_s) tensors instead."""
@@ -493,13 +493,13 @@ def glq_fused_linear_trellis_3inst_group_rvq2(x, shards, blocks_n, blocks_n_meta
     """The grouped call for stacked (two-stage) layers: fused q/k/v or
     gate/up of a 5-8 bpw checkpoint, whose per-shard loop in the reference is
     fused_linear_trellis_3inst_yrht_rvq2 per shard + output_rht_shards (glq_vllm/linear_method.py:664-710).
-    One token: one decode launch for both streams of every shard; 2..16: one transform launch for all sign
-    vectors and one decode launch per shard (the small-batch kernel); above: one launch of the tile kernel over
-    the row tiles of all shards; one finishing launch.
+    One decode launch for both streams of every shard and one finishing launch, as in the single-stage call (the
+    fused-input launch at one token only), at any token count; above 2048 tokens whole linears through the library
+    GEMM are faster.
 
     shards: sequence of (sv, su, trellis_packed, trellis_packed2, wscale, inv_resid_scale2, out_features,
     m_pad); first stages of 4 bpw, second stages of one common rate.  Returns (B, sum(out_features)).
-    Raises RuntimeError for other token counts or rates (callers then use the per-layer op)."""
+    Raises RuntimeError for other rates (callers then use the per-layer op)."""
     lib = _lib.load()
     _chk(x, "x", (torch.float16, torch.bfloat16))
     B = x.shape[0]

@@ -193,22 +193,22 @@ size_t glqh_fused_linear_trellis_group_workspace_bytes(int64_t B, int64_t n_pad,
                                                        int n_shards);
 
 /* Separately quantized layers that consume the same x (fused q/k/v, gate/up of a merged
- * linear): one decode launch and one output-transform launch for all of them instead of
- * two or three per layer.  Replaces the per-shard loop of the vLLM linear method
+ * linear): one decode launch and one finishing launch for all of them, and one input transform
+ * launch where the decode launch does not transform itself.  Replaces the per-shard loop of the vLLM linear method
  * (glq_vllm/linear_method.py:664-710: fused_linear_trellis_3inst_yrht per shard, then
  * output_rht_shards; glq/csrc/glq_trellis.cu:1373-1397, glq/csrc/glq_cuda.cu:2882-2916) and
  * gives, per shard, the result of glqh_fused_linear_trellis_3inst on that shard up to the
- * rounding of a different K split.  Single-stage layers of one rate R, at most 4 tokens,
- * canonical (block_decompose) output block sizes; anything else is refused and the caller
- * falls back to per-layer calls.
- * 5..64 tokens: one input transform per distinct sign vector, one decode launch per layer (the small-batch
- * kernel under the K plan of the tallest up to 16 tokens, the small-tile kernel under its own plan above)
- * and one output-transform launch for all layers, or one per layer where their K plans differ (no K-slot
- * sum launches, no shared fp32 buffer in between).
- * More than 64 tokens (up to four layers, every y given): one input transform per distinct sign
- * vector, ONE launch of the many-token kernel over the row tiles of all layers (small layers do not
- * fill the chip one by one) and one output transform per layer.  y_stride 0 there: every layer's rows
- * are packed (row stride = its out_features), so that each layer's output is a contiguous matrix.
+ * rounding of a different K split.  One to four single-stage layers of one rate R, canonical
+ * (block_decompose) output block sizes, any token count; anything else is refused and the caller
+ * falls back to per-layer calls.  All layers share every launch and one K plan:
+ * 1..4 tokens: the fused-input launch (transform and decode), or the transform of x under every distinct
+ * sign vector and the small-batch kernel over the 64-row strips of all layers, by width and weights;
+ * 5..16 tokens: the second of these;
+ * 17..64 tokens: the transform into the tile kernels' layout, the small-tile kernel over the row tiles;
+ * more than 64 tokens (every y given): the same with the many-token kernel, whose sums may be fp16.
+ * y_stride 0 there: every layer's rows are packed (row stride = its out_features), so that each layer's
+ * output is a contiguous matrix.
+ * (Rows or widths that the shared transform launches do not take have one launch per sign vector or layer.)
  */
 int glqh_fused_linear_trellis_3inst_group(const void *x, int x_dtype, int64_t x_stride, int64_t B,
                                           const glqh_trellis_shard *shards, int n_shards,
@@ -226,15 +226,14 @@ typedef struct {
     double inv_resid_scale2;
 } glqh_trellis_stage2;
 
-/* The grouped call for stacked layers at 1..64 tokens (at one token the decode step of fused q/k/v and gate/up of a
+/* The grouped call for stacked layers, any token count (at one token the decode step of fused q/k/v and gate/up of a
  * 5-8 bits/weight checkpoint; the reference runs fused_linear_trellis_3inst_yrht_rvq2 per shard,
- * glq_vllm/linear_method.py:664-710): one decode launch reads both streams of every layer (first
- * stages of 4 bits/weight, second stages of one common rate, stage2[i] belongs to shards[i]) and one
- * launch finishes them.  2..64 tokens: one input transform per distinct sign vector, one launch per layer
- * that decodes both streams (the small-batch kernel to 16 tokens, the small-tile kernel above), one
- * finishing launch.  Workspace:
- * glqh_fused_linear_trellis_group_workspace_bytes(B, ...).  Every shard's y must be given; other token
- * counts and rates are refused (per-layer calls serve them). */
+ * glq_vllm/linear_method.py:664-710): the launches of the single-stage call, the decode launch reading both
+ * streams of every layer (first stages of 4 bits/weight, second stages of one common rate, stage2[i] belongs
+ * to shards[i]); the fused-input launch at one token only, and from 17 tokens on both streams make one
+ * operand (refused under GLQ_TRELLIS_FUSE_STAGES=0).  Workspace:
+ * glqh_fused_linear_trellis_group_workspace_bytes(B, ...).  Every shard's y must be given; other rates are
+ * refused (per-layer calls serve them). */
 int glqh_fused_linear_trellis_3inst_group_rvq2(const void *x, int x_dtype, int64_t x_stride, int64_t B,
                                                const glqh_trellis_shard *shards,
                                                const glqh_trellis_stage2 *stage2, int n_shards,
