@@ -92,12 +92,13 @@ e8_quantize_kernel(const float *__restrict__ x, const float *__restrict__ table,
 // finite, or have too many points in reach for the list, take the walk itself (e8_walk_kernel).
 //
 // 524288 vectors of N(0, 1): 12.06 ms (walk) -> 98 us (points of norm 12 on the matrix cores, all 8655 rows for
-// every vector they may win) -> 34 us (points in reach only; 38 MB in and out, 8 us) -> 35.4 us with the table read
-// by every call (es_index_kernel 4.5 us; 250 -> 54 us where the table is new); 960 vectors 12.7 ms -> 13.4 ->
-// 20 us: three dependent launches.
+// every vector they may win) -> 34 us (points in reach only; 38 MB in and out, 8 us) -> 33.2 us with the table read
+// by every call (es_index_kernel 4 us; 250 -> 52 us where the table is new); 960 vectors 12.7 ms -> 13.4 ->
+// 17.3 us: three dependent launches.
 constexpr int ES_THREADS = 256;
 constexpr int ES_PLACES = 117361;                              // E8 points of norm up to 12
 constexpr int ES_FULL = GLQH_E8_SHELL_MIN_ROWS;                // of norm up to 10: all of them are rows of the table
+enum { ES_SHARED, ES_IN_FULL, ES_WALKS, ES_FOUND };            // two rows of one place; rows of the full shells; vectors to walk
 constexpr int ES_CHECKS = 128;                                 // workgroups, at least, that look for rows of one place
 constexpr int ES_CHUNK = 128;                                  // vectors whose points are listed together,
 constexpr int ES_LIST = 3072;                                  // and the points: 2.5 each at unit scale, up to 106 far out
@@ -183,9 +184,9 @@ __device__ __forceinline__ void es_load(const float *__restrict__ x, int64_t v, 
 // counts[r / 64]: rows of norm up to 10, negative if one of the 64 rows is no point.
 __global__ void __launch_bounds__(ES_THREADS)
 es_index_kernel(const float *__restrict__ table, const float *__restrict__ norms, int n, int *__restrict__ row_at,
-                int *__restrict__ place_of, int *__restrict__ counts, int *__restrict__ shared_place) {
+                int *__restrict__ place_of, int *__restrict__ counts, int *__restrict__ found) {
     const int r = blockIdx.x * ES_THREADS + threadIdx.x;
-    if (r == 0) *shared_place = 0;
+    if (r == 0) found[ES_SHARED] = found[ES_IN_FULL] = found[ES_WALKS] = 0;
     if (r >= n) return;
     float c[8];
     es_load(table, r, c);
@@ -215,7 +216,8 @@ struct es_args {
     const float *x, *table, *norms;
     int64_t N;
     int n_entries;
-    int *row_at, *place_of, *counts, *shared_place;            // written by es_index_kernel
+    int *row_at, *place_of, *counts;                           // written by es_index_kernel
+    int *found;                                                // what the search finds out, cleared by es_index_kernel
     int64_t *idx_out;
     float *dec_out;                                            // may be null
     int *walk_count;                                           // per workgroup of the first kernel
@@ -372,10 +374,18 @@ e8_shell_kernel(const es_args a) {
     const int tid = threadIdx.x;
     const int64_t v0 = (int64_t)blockIdx.x * V;
     if (tid == 0) n_flag = n_walk = 0;
-    // two rows of one place: one of them is not the row found there
+    // two rows of one place: one of them is not the row found there.  (What the last launch asks of the table is summed up
+    // here, so that with nothing to walk it reads three words: 524288 vectors 35.9 -> 33.2 us, 960 20 -> 17.3.)
     for (int64_t r = (int64_t)blockIdx.x * ES_THREADS + tid; r < a.n_entries; r += (int64_t)gridDim.x * ES_THREADS) {
         const int place = a.place_of[r];
-        if (place >= 0 && a.row_at[place] != (int)r) *a.shared_place = 1;
+        if (place >= 0 && a.row_at[place] != (int)r) a.found[ES_SHARED] = 1;
+    }
+    if (blockIdx.x == gridDim.x - 1) {                         // rows of the full shells; other rows make the sum differ
+        int full = 0;
+        for (int i = tid; i < (a.n_entries + 63) / 64; i += ES_THREADS) full += a.counts[i];
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) full += __shfl_xor(full, o, 64);
+        if ((tid & 63) == 0) atomicAdd(a.found + ES_IN_FULL, full);
     }
     if (v0 >= a.N) return;                                     // here for that only
     __syncthreads();
@@ -498,7 +508,10 @@ e8_shell_kernel(const es_args a) {
         }
         __syncthreads();
     }
-    if (tid == 0) a.walk_count[blockIdx.x] = n_walk;
+    if (tid == 0) {
+        a.walk_count[blockIdx.x] = n_walk;
+        if (n_walk) atomicAdd(a.found + ES_WALKS, n_walk);
+    }
 }
 
 // The table walk for the vectors left over, 64 at a time, a lane each: workgroup (64 vectors, part of
@@ -507,15 +520,21 @@ e8_shell_kernel(const es_args a) {
 __global__ void __launch_bounds__(ES_THREADS)
 e8_walk_kernel(const es_args a, int n_src, int per_src) {
     constexpr int ROWS = 65536 / ES_SPLIT;                     // of one part, at most
-    __shared__ int sums[4], fulls[4];
+    __shared__ int sums[4];
     __shared__ int64_t item[64];                               // the vector's list position
     __shared__ unsigned long long keys[4][64];
     __shared__ f32x4v rows[ROWS][2];
     __shared__ float row_norm[ROWS];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    // what the search assumed of the table, and the vectors' ranks over all source workgroups: a run of sources per thread
-    int full = tid == 0 && *a.shared_place ? -ES_FULL - 1 : 0;
-    for (int i = tid; i < (a.n_entries + 63) / 64; i += ES_THREADS) full += a.counts[i];
+    if (a.found[ES_SHARED] != 0 || a.found[ES_IN_FULL] != ES_FULL) {   // not what the search assumed: every vector, every row
+        const int64_t blocks = (a.N + EQ_THREADS * EQ_VPT - 1) / (EQ_THREADS * EQ_VPT);
+        for (int64_t b = blockIdx.x; b < blocks; b += gridDim.x)
+            e8_quantize_block(a.x, a.table, a.norms, a.N, a.n_entries, a.idx_out, a.dec_out, b);
+        return;
+    }
+    const int total = a.found[ES_WALKS];
+    if (total == 0) return;
+    // the vectors' ranks over all source workgroups: a run of sources per thread
     const int per = (n_src + ES_THREADS - 1) / ES_THREADS;
     const int s0 = min(tid * per, n_src), s1 = min(s0 + per, n_src);
     int mine = 0;
@@ -525,28 +544,13 @@ e8_walk_kernel(const es_args a, int n_src, int per_src) {
     for (int o = 1; o < 64; o <<= 1) {
         const int v = __shfl_up(first, o, 64);
         if (lane >= o) first += v;
-        full += __shfl_xor(full, o, 64);
     }
-    if (lane == 63) {
-        sums[wave] = first;
-        fulls[wave] = full;
-    }
+    if (lane == 63) sums[wave] = first;
     __syncthreads();
-    int total = 0;
     first -= mine;
-    full = 0;
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
+    for (int q = 0; q < 4; ++q)
         if (q < wave) first += sums[q];
-        total += sums[q];
-        full += fulls[q];
-    }
-    if (full != ES_FULL) {                                     // any other table: every vector against every row
-        const int64_t blocks = (a.N + EQ_THREADS * EQ_VPT - 1) / (EQ_THREADS * EQ_VPT);
-        for (int64_t b = blockIdx.x; b < blocks; b += gridDim.x)
-            e8_quantize_block(a.x, a.table, a.norms, a.N, a.n_entries, a.idx_out, a.dec_out, b);
-        return;
-    }
     const int64_t work = (int64_t)((total + 63) / 64) * ES_SPLIT;
     for (int64_t w = blockIdx.x; w < work; w += gridDim.x) {
         const int base = (int)(w / ES_SPLIT) * 64, part = (int)(w % ES_SPLIT);
@@ -615,7 +619,7 @@ int glqh_launch_e8_quantize(const float *x, const float *table, const float *nor
 static size_t es_align(size_t v) { return (v + 15) & ~(size_t)15; }
 
 size_t glqh_e8_shell_ws_bytes(int64_t N) {
-    return es_align((size_t)N * 16 + (size_t)((N + 63) / 64) * 4) + (size_t)(ES_PLACES + 65536 + 65536 / 64 + 1) * 4;
+    return es_align((size_t)N * 16 + (size_t)((N + 63) / 64) * 4) + (size_t)(ES_PLACES + 65536 + 65536 / 64 + ES_FOUND) * 4;
 }
 
 int glqh_launch_e8_shell_quantize(const float *x, int64_t N, const float *table, const float *norms, int n_entries,
@@ -633,10 +637,10 @@ int glqh_launch_e8_shell_quantize(const float *x, int64_t N, const float *table,
     a.row_at = (int *)((char *)ws + es_align((size_t)N * 16 + (size_t)((N + 63) / 64) * 4));
     a.place_of = a.row_at + ES_PLACES;
     a.counts = a.place_of + 65536;
-    a.shared_place = a.counts + 65536 / 64;
+    a.found = a.counts + 65536 / 64;
     const dim3 grid((unsigned)(wgs > ES_CHECKS ? wgs : ES_CHECKS));
     hipLaunchKernelGGL(es_index_kernel, dim3((unsigned)((n_entries + ES_THREADS - 1) / ES_THREADS)), dim3(ES_THREADS), 0, stream, table,
-                       norms, n_entries, a.row_at, a.place_of, a.counts, a.shared_place);
+                       norms, n_entries, a.row_at, a.place_of, a.counts, a.found);
     if (per == 512) hipLaunchKernelGGL(e8_shell_kernel<512>, grid, dim3(ES_THREADS), 0, stream, a);
     else if (per == 256) hipLaunchKernelGGL(e8_shell_kernel<256>, grid, dim3(ES_THREADS), 0, stream, a);
     else hipLaunchKernelGGL(e8_shell_kernel<64>, grid, dim3(ES_THREADS), 0, stream, a);
