@@ -12,6 +12,9 @@
 // All arithmetic is fp32 with separate subtract, multiply and add (no contraction), the
 // input is rounded to fp16 first (glq/trellis.py:468).
 //
+// viterbi_kernel does that for every tile of small calls and of 1-bit ones; elsewhere for the few that the search on
+// lower bounds, further down, leaves to it.
+//
 // What bounds it is vector-ALU issue: 65536 states per step, 510 steps per tile.  A workgroup
 // therefore keeps the whole table in registers, two fp16 values to a register (v_fma_mix_f32
 // subtracts the input from either half with fp32 rounding), and a state costs 3.5 instructions:
@@ -267,13 +270,19 @@ __device__ __forceinline__ int64_t vt_step_pos(int t, int64_t ld) {
     return (int64_t)((l >> 2) + 8 * ((j >> 1) & 1)) * ld + 2 * (l & 3) + 8 * (j >> 2) + (j & 1);
 }
 
-// Persistent workgroups walk the tiles with a fixed stride, each owning one slab of cost rows.
-// ld > 0: tiles_in and hat_out are (m, n) matrices of row length ld, the tiles their 16x16 blocks in
-// row-major order; ld == 0: (tiles, 256) rows in step order.
+// Element `t` of a tile.  ld > 0: of (m, n) matrices of row length ld, the tiles their 16x16 blocks in row-major order;
+// ld == 0: of (tiles, 256) rows in step order.
+__device__ __forceinline__ int64_t vt_pos(int64_t tile, int t, int64_t ld) {
+    const int64_t per_row = ld >> 4;
+    return ld ? (tile / per_row) * 16 * ld + (tile % per_row) * 16 + vt_step_pos(t, ld) : tile * VT_T + t;
+}
+
+// Persistent workgroups walk the tiles with a fixed stride, each owning one slab of cost rows.  marked: only tiles whose
+// first state is -1.
 template <int K>
 __global__ void __launch_bounds__(vt_cfg<K>::THREADS, 4)
 viterbi_kernel(const float *__restrict__ tiles_in, int64_t n_tiles, int64_t ld, float *__restrict__ scratch,
-               int32_t *__restrict__ states_out, float *__restrict__ hat_out) {
+               int32_t *states_out, float *__restrict__ hat_out, int marked) {
     using C = vt_cfg<K>;
     constexpr int G = C::G;
     extern __shared__ float best[];                            // ROWS * G floats
@@ -282,6 +291,11 @@ viterbi_kernel(const float *__restrict__ tiles_in, int64_t n_tiles, int64_t ld, 
     __shared__ vt_best red[C::THREADS / 64];
     const int tid = threadIdx.x;
     float *hist = scratch + (int64_t)blockIdx.x * (VT_T / C::DEPTH) * G;
+    if (marked) {
+        bool any = false;
+        for (int64_t tile = blockIdx.x; tile < n_tiles; tile += gridDim.x) any = any || states_out[tile * VT_T] < 0;
+        if (!any) return;
+    }
     f16x2 w[32768 / C::THREADS];
 #pragma unroll
     for (int k = 0; k < C::NK; ++k)
@@ -295,9 +309,8 @@ viterbi_kernel(const float *__restrict__ tiles_in, int64_t n_tiles, int64_t ld, 
                 w[(k * C::UNITS + q) * (C::LOWS / 2) + j / 2] = v;
             }
     for (int64_t tile = blockIdx.x; tile < n_tiles; tile += gridDim.x) {
-        const int64_t per_row = ld >> 4;
-        const int64_t at = ld ? (tile / per_row) * 16 * ld + (tile % per_row) * 16 : tile * VT_T;
-        const int64_t pos = ld ? at + vt_step_pos(tid & 255, ld) : at + (tid & 255);
+        if (marked && states_out[tile * VT_T] >= 0) continue;
+        const int64_t pos = vt_pos(tile, tid & 255, ld);
         if (tid < VT_T) {
             const float v = (float)(f16)tiles_in[pos];
             x[tid] = v;
@@ -314,6 +327,731 @@ viterbi_kernel(const float *__restrict__ tiles_in, int64_t n_tiles, int64_t ld, 
             hat_out[pos] = (float)tr_weight((uint32_t)s);
         }
         __syncthreads();
+    }
+}
+
+// ---- the search on lower bounds ----------------------------------------------------------
+// The costs that decide are fp32, but most of what viterbi_kernel spends on them goes to states that no good path comes
+// near.  Here the forward pass carries LOWER BOUNDS of the costs in packed fp16, two states to an instruction and rounded
+// towards zero, and the few paths that their bounds do not exclude are compared in the exact arithmetic of
+// viterbi_kernel: the same states, the same ties.
+//
+// Bounds (vb_forward).  l_i[g] <= best_i[g] - B_i for every group: the subtraction and the multiply-add of a state
+// round towards zero, a minimum does not round, and every VB_NORM steps the row's minimum moves from the row into B
+// (values stay small, where fp16 is fine; a difference of two fp16 numbers that is >= 0 rounds down too).  The pass runs
+// one step past the last input, so that L = min l_T + B_T bounds the whole search.
+// Backtrack (vb_backtrack, a wave a tile).  From the end, keep every way whose bound (its cost to the end + l + B)
+// is at most L (1 + SLACK): what the fp16 roundings lose is 0.3-0.5 % of the cost, so a level keeps 1.4 ways on average.
+// At the start the cheapest kept path costs U.  If U (1 + 2^-14) is within the limit, no path that was dropped can cost U
+// or less, also after the roundings of 256 fp32 additions (2^-24 each), and the kept ones contain the search's answer and
+// all its ties; else the backtrack runs again with that limit.  Where another kept path is within 2^-14 of the cheapest
+// (3 % of the tiles), fp32 costs are evaluated forward over the kept ways, minima and lowest states as in viterbi_kernel.
+// Tiles that fail (inputs above VB_X, not finite or all equal, more kept ways than fit) are marked by state -1 and
+// left to viterbi_kernel, which skips all others.  2048 x 2048 weights in viterbi_kernel alone -> so: 69.7 -> 31.9 ms at
+// K = 4, 59.0 -> 38.1 at 3, 66.5 -> 36.4 at 2.
+constexpr int VB_THREADS = 512;
+constexpr int VB_NORM = 2;                 // steps between two moves of the row's minimum into B
+constexpr float VB_X = 16.0f;              // largest input: (16 + 4)^2 for 16 / K steps stays far below 65504
+constexpr int VB_MOST = 64;                // kept groups of a step: a lane each
+
+template <int K>
+struct vb_cfg {
+    static constexpr int G = 1 << (16 - K), NK = 1 << K, HI = G >> K;
+    static constexpr int CW = NK / 2;                          // words of a group's predecessor costs
+    static constexpr int DEPTH = K == 2 ? 4 : 2;               // steps per stored row
+    static constexpr int STORED = VT_T / DEPTH;
+    static constexpr float SLACK = K == 4 ? 0.0042f : K == 3 ? 0.0049f : 0.0058f;
+    static constexpr int ROW = K == 4 ? 32 * 72 : K == 3 ? 128 * 36 : 4096 * 2 + 256 * 2;   // words of a row, with its padding
+    static constexpr int ROWS = K == 2 ? 1 : 2;                // cost rows in LDS per tile; one: read by all, then written
+    static constexpr int FEW = K == 2 ? 2 : 1;                 // tiles a workgroup in calls that do not fill the chip
+};
+
+__device__ __forceinline__ f16x2 vb_pair(uint32_t v) { return __builtin_bit_cast(f16x2, v); }
+__device__ __forceinline__ uint32_t vb_bits(f16x2 v) { return __builtin_bit_cast(uint32_t, v); }
+__device__ __forceinline__ float vb_half(uint32_t bits) { return (float)__builtin_bit_cast(f16, (uint16_t)bits); }
+
+// Where cost rows lie in LDS: the NK predecessor costs of a group (a = g >> K) are one run, read in one or two
+// accesses, and what a wave writes of one low digit falls on different banks: runs are padded, and the words of a run
+// (predecessors 2j, 2j+1) exchanged by an exclusive-or that is constant for a reader and for a writer.
+template <int K>
+__device__ __forceinline__ int vb_run(int a) {                 // in words
+    if constexpr (K == 4) return (a >> 3) * 72 + (a & 7) * 8;
+    if constexpr (K == 3) return (a >> 3) * 36 + (a & 7) * 4;
+    return a * 2 + (a >> 4) * 2;
+}
+template <int K>
+__device__ __forceinline__ int vb_word(int a) {
+    if constexpr (K == 4) return (a >> 5) & 7;
+    if constexpr (K == 3) return (a >> 7) & 3;
+    return (a >> 6) & 1;
+}
+// group g's cost, in halves; the groups of a thread's slots are NK halves apart
+template <int K>
+__device__ __forceinline__ int vb_at(int g) {
+    using C = vb_cfg<K>;
+    const int k = g / C::HI, a = g % C::HI;
+    return vb_run<K>(a) * 2 + (((k >> 1) ^ vb_word<K>(a)) << 1) + (k & 1);
+}
+// Stored rows are the runs without the padding: what a thread has read of the row goes out as it is, and the ways into
+// one group, whose digits are the high ones, lie in 64-byte pieces.  Position of group g's cost, and back:
+template <int K>
+__device__ __forceinline__ int vb_stored(int g) {
+    using C = vb_cfg<K>;
+    const int k = g / C::HI, a = g % C::HI;
+    return a * C::NK + (((k >> 1) ^ vb_word<K>(a)) << 1) + (k & 1);
+}
+template <int K>
+__device__ __forceinline__ int vb_group(int at) {
+    using C = vb_cfg<K>;
+    const int a = at >> K, k = at & (C::NK - 1);
+    return ((((k >> 1) ^ vb_word<K>(a)) << 1) + (k & 1)) * C::HI + a;
+}
+
+// the least of a wave's values, in every lane
+__device__ __forceinline__ uint32_t vb_wave_min(uint32_t v) {
+    auto step = [&](uint32_t u) { v = u < v ? u : v; };
+    step((uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x111, 0xf, 0xf, false));   // row_shr:1, 2, 4, 8
+    step((uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x112, 0xf, 0xf, false));
+    step((uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x114, 0xf, 0xf, false));
+    step((uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x118, 0xf, 0xf, false));
+    step((uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x142, 0xa, 0xf, false));   // row_bcast:15, 31
+    step((uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x143, 0xc, 0xf, false));
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
+__device__ __forceinline__ int vb_lane(int v, int from) { return __builtin_amdgcn_readlane(v, from); }
+__device__ __forceinline__ float vb_lane(float v, int from) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), from));
+}
+__device__ __forceinline__ int vb_below(uint64_t mask) {       // lanes of the mask below this one
+    return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0));
+}
+
+// What the two kernels of a pass hand each other, per tile
+struct vb_tile {
+    float pre[VT_T / VB_NORM + 1];         // B at step j * VB_NORM
+    int over;                              // the tail-biting overlap, -1: left to viterbi_kernel
+};
+
+// Tiles first .. first + count - 1 and one of their two passes: 0 on the inputs rolled by T/2, unconstrained; 1 from and
+// to the overlap that the first backtrack found.  rows: STORED rows of G halves per tile.
+struct vb_part {
+    int64_t first;
+    int count, pass;
+    uint16_t *rows;
+    vb_tile *info;
+};
+
+// One forward pass, the rows of every DEPTH-th step to part.rows.  TPW tiles a workgroup: their steps share the table and
+// the barriers; workgroups walk the tiles with a fixed stride.
+//
+// What bounds it is vector issue: 2.5 instructions for two states, 4.4-4.7 clocks each.  A loop of nothing else takes 6.0
+// clocks a state, where subtract, multiply, add and half a minimum in fp32 take 14.4 (fma_mix 4.3, the others 2.5); the
+// pass over 1024 tiles at K = 4 takes 0.93 ms, of which such loops would be 0.65.
+template <int K, int TPW>
+__device__ __forceinline__ void vb_forward(const float *__restrict__ tiles_in, int64_t ld, const vb_part &part, int worker,
+                                           int workers, uint32_t *lds) {
+    using C = vb_cfg<K>;
+    constexpr int THREADS = VB_THREADS;
+    const int64_t first = part.first;
+    const int count = part.count, pass = part.pass;
+    uint16_t *const __restrict__ rows = part.rows;
+    vb_tile *const __restrict__ info = part.info;
+    constexpr int G = C::G, NK = C::NK, CW = C::CW, D = C::DEPTH, ROWS = C::ROWS;
+    // SHARE threads to a predecessor group, UNITS such groups to a thread, LP pairs of their groups
+    constexpr int SHARE = K == 4 ? 2 : 1, LOWS = NK / SHARE, LP = LOWS / 2;
+    constexpr int UNITS = G / THREADS / LOWS;
+    constexpr int ROUND = D > VB_NORM ? D : VB_NORM;
+    __shared__ uint32_t xh[TPW][VT_T];                         // inputs, twice each
+    __shared__ uint32_t low[TPW][2];                           // the least cost of the last row, of alternate moves
+    __shared__ int over[TPW], varied[TPW];
+    const int tid = threadIdx.x, lane = tid & 63;
+    auto row_of = [&](int t, int which) { return lds + (t * ROWS + which) * C::ROW; };
+    // This thread's predecessor group and first slot of unit q.  Below K = 4, units 2i and 2i + 1 are predecessors 2j and
+    // 2j + 1 of the same groups: their costs go out as one word.
+    auto a_of = [&](int q) {
+        const int t = tid / SHARE;
+        if constexpr (K == 4) return t;
+        if constexpr (K == 3) return (t & 127) + 128 * (2 * (t >> 7) + q);
+        return t + THREADS * ((q & 4) | (q & 1) << 1 | (q >> 1 & 1));
+    };
+    const int slot0 = tid % SHARE * LOWS;
+    f16x2 w[UNITS * LP * NK];
+#pragma unroll
+    for (int q = 0; q < UNITS; ++q)
+#pragma unroll
+        for (int p = 0; p < LP; ++p)
+#pragma unroll
+            for (int j = 0; j < NK; ++j) {
+                const int a = a_of(q);
+                const int k = (((j >> 1) ^ vb_word<K>(a)) << 1) + (j & 1);
+                const int s = k * G + a * NK;
+                f16x2 v = {tr_weight((uint32_t)(s + slot0 + 2 * p)), tr_weight((uint32_t)(s + slot0 + 2 * p + 1))};
+                asm volatile("" : "+v"(v));                    // finished here, in the usual rounding
+                w[(q * LP + p) * NK + j] = v;
+            }
+    const int turn = pass ? 0 : VT_T / 2, pairs = (count + TPW - 1) / TPW;
+#pragma unroll 1
+    for (int pair = worker; pair < pairs; pair += workers) {
+        if (tid < TPW) varied[tid] = 0;
+        if (tid < TPW) over[tid] = pair * TPW + tid >= count ? -1 : pass ? info[pair * TPW + tid].over : 0;
+        __syncthreads();
+        {
+            const int t = tid >> 8, i = tid & 255;
+            if (t < TPW) {
+                const bool there = pair * TPW + t < count;
+                const f16 v = there ? (f16)tiles_in[vt_pos(first + pair * TPW + t, i, ld)] : (f16)0.0f;
+                xh[t][i] = vb_bits(f16x2{v, v});
+                if (!(__builtin_fabsf((float)v) <= VB_X)) over[t] = -1;
+            }
+        }
+        __syncthreads();
+        if (pass == 0) {                                       // equal inputs leave every other path a tie
+            const int t = tid >> 8, i = tid & 255;
+            if (t < TPW && xh[t][i] != xh[t][0]) varied[t] = 1;
+            __syncthreads();
+            if (tid < TPW && !varied[tid]) over[tid] = -1;
+            __syncthreads();
+        }
+        bool any = false;
+#pragma unroll
+        for (int t = 0; t < TPW; ++t) any = any || over[t] >= 0;
+        if (pass == 0 && tid < TPW && pair * TPW + tid < count) info[pair * TPW + tid].over = over[tid];
+        if (!any) {
+            __syncthreads();
+            continue;
+        }
+#pragma unroll
+        for (int t = 0; t < TPW; ++t) {
+            uint16_t *r = (uint16_t *)row_of(t, 0);
+            for (int g = tid; g < G; g += THREADS) r[vb_at<K>(g)] = pass == 0 || g == over[t] ? 0 : 0x7C00;
+            if (tid < 2) low[t][tid] = 0xFFFFFFFFu;
+        }
+        __syncthreads();
+        asm volatile("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 2, 2), 3" ::: "memory");   // fp16 rounds towards zero
+        uint32_t xn[TPW];
+        float moved[TPW];
+#pragma unroll
+        for (int t = 0; t < TPW; ++t) {
+            xn[t] = xh[t][turn];
+            moved[t] = 0.0f;
+            if (tid == 0 && pair * TPW + t < count) info[pair * TPW + t].pre[0] = 0.0f;
+        }
+        auto load = [&](int t, int which, uint32_t (&c)[UNITS][CW]) {
+#pragma unroll
+            for (int q = 0; q < UNITS; ++q) {
+                const uint32_t *r = row_of(t, which) + vb_run<K>(a_of(q));
+                if constexpr (CW == 2) {
+                    const u32x2 v = *(const u32x2 *)r;
+                    c[q][0] = v.x; c[q][1] = v.y;
+                } else {
+#pragma unroll
+                    for (int j = 0; j < CW; j += 4) {
+                        const u32x4 v = *(const u32x4 *)(r + j);
+                        c[q][j] = v.x; c[q][j + 1] = v.y; c[q][j + 2] = v.z; c[q][j + 3] = v.w;
+                    }
+                }
+            }
+        };
+        auto keep = [&](int t, int level, uint32_t (&c)[UNITS][CW]) {   // the row of a level, as read
+            uint16_t *h = rows + ((int64_t)(pair * TPW + t) * C::STORED + level - 1) * G;
+#pragma unroll
+            for (int q = 0; q < UNITS; ++q) {
+                if constexpr (K == 4) {                        // two threads have read the same: a half each
+                    const uint32_t odd = 0u - (tid & 1);
+                    u32x4 v;
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) v[j] = c[q][j] ^ ((c[q][j] ^ c[q][j + 4]) & odd);
+                    *(u32x4 *)(h + (uint32_t)(tid * 8)) = v;
+                } else if constexpr (K == 3) {
+                    *(u32x4 *)(h + (uint32_t)(a_of(q) * NK)) = u32x4{c[q][0], c[q][1], c[q][2], c[q][3]};
+                } else {
+                    *(u32x2 *)(h + (uint32_t)(a_of(q) * NK)) = u32x2{c[q][0], c[q][1]};
+                }
+            }
+        };
+#pragma unroll 1
+        for (int i0 = 0; i0 < VT_T; i0 += ROUND)
+#pragma unroll
+        for (int u = 1; u <= ROUND; ++u) {
+            const int i = i0 + u, cur = ROWS == 2 ? (u + 1) & 1 : 0, nxt = ROWS == 2 ? u & 1 : 0;
+            const bool move = u % VB_NORM == 0, least = u % VB_NORM == VB_NORM - 1;
+            f16x2 x[TPW];
+            uint32_t c[TPW][UNITS][CW];
+#pragma unroll
+            for (int t = 0; t < TPW; ++t) {
+                if (ROWS == 2) load(t, cur, c[t]);
+                x[t] = vb_pair(__builtin_amdgcn_readfirstlane(xn[t]));
+                xn[t] = xh[t][(i + turn) & (VT_T - 1)];        // read a step ahead
+            }
+#pragma unroll
+            for (int t = 0; t < TPW; ++t) {
+                if constexpr (ROWS == 1) {
+                    load(t, 0, c[t]);
+                    vt_barrier();                              // read by all: the row may change
+                }
+                f16x2 shift = vb_pair(0);
+                if (move) shift = vb_pair(__builtin_amdgcn_readfirstlane(low[t][i / VB_NORM & 1]));
+                const bool there = pair * TPW + t < count;
+                if ((u - 1) % D == 0 && i > 1 && there) keep(t, (i - 1) / D, c[t]);
+                f16x2 least_of = vb_pair(0x7C007C00u), m[2][LP];
+#pragma unroll
+                for (int q = 0; q < UNITS; ++q) {
+                    f16x2(&mq)[LP] = m[q & 1];
+#pragma unroll
+                    for (int p = 0; p < LP; ++p) {
+                        f16x2 e[NK];
+#pragma unroll
+                        for (int j = 0; j < NK; ++j) {
+                            const f16x2 d = w[(q * LP + p) * NK + j] - x[t], cj = vb_pair(c[t][q][j >> 1]);
+                            e[j] = __builtin_elementwise_fma(d, d, j & 1 ? f16x2{cj.y, cj.y} : f16x2{cj.x, cj.x});
+                        }
+                        f16x2 v = e[0];
+#pragma unroll
+                        for (int j = 1; j + 1 < NK; j += 2)
+                            v = __builtin_elementwise_minimum(__builtin_elementwise_minimum(v, e[j]), e[j + 1]);
+                        mq[p] = __builtin_elementwise_minimum(v, e[NK - 1]);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                    if (move) {
+#pragma unroll
+                        for (int p = 0; p < LP; ++p) mq[p] -= shift;
+                    }
+                    if (least) {
+#pragma unroll
+                        for (int p = 0; p < LP; ++p) least_of = __builtin_elementwise_minimum(least_of, mq[p]);
+                    }
+                    if constexpr (K == 4) {
+                        uint16_t *o = (uint16_t *)row_of(t, nxt) + vb_at<K>((a_of(0) << K) + slot0);
+#pragma unroll
+                        for (int p = 0; p < LP; ++p) {
+                            o[2 * p * NK] = (uint16_t)vb_bits(mq[p]);
+                            o[(2 * p + 1) * NK] = (uint16_t)(vb_bits(mq[p]) >> 16);
+                        }
+                    } else if (q & 1) {
+                        uint32_t *o = row_of(t, nxt) + (vb_at<K>((a_of(q - 1) << K) + slot0) >> 1);
+#pragma unroll
+                        for (int p = 0; p < LP; ++p) {
+                            o[2 * p * CW] = vb_bits(f16x2{m[0][p].x, m[1][p].x});
+                            o[(2 * p + 1) * CW] = vb_bits(f16x2{m[0][p].y, m[1][p].y});
+                        }
+                    }
+                }
+                if (least) {                                   // numbers >= 0 order as their bits
+                    least_of = __builtin_elementwise_minimum(least_of, f16x2{least_of.y, least_of.x});
+                    const uint32_t v = vb_wave_min(vb_bits(least_of));
+                    if (lane == 0) atomicMin(&low[t][(i + 1) / VB_NORM & 1], v);
+                    if (tid == 0 && i > VB_NORM) low[t][i / VB_NORM & 1] = 0xFFFFFFFFu;   // the word of the move before
+                }
+                if (move && tid == 0 && there) {
+                    moved[t] += (float)shift.x;
+                    info[pair * TPW + t].pre[i / VB_NORM] = moved[t];
+                }
+            }
+            if (ROWS == 2) vt_barrier();
+        }
+        vt_barrier();
+#pragma unroll
+        for (int t = 0; t < TPW; ++t) {
+            uint32_t c[UNITS][CW];
+            load(t, 0, c);
+            if (pair * TPW + t < count) keep(t, C::STORED, c);
+        }
+        asm volatile("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 2, 2), 0" ::: "memory");
+        __syncthreads();
+    }
+}
+
+// A tile's working memory in LDS during the backtrack.  Level l is step l * DEPTH; its entries are the
+// kept ways from the groups of level l (parents: where the states lead) to those of level l - 1 (children).
+struct vb_pool {
+    static constexpr int ENTRIES = 768;    // 550 at most in 3 * 10^4 tiles of Gaussian values, 170 on average
+    float cost[ENTRIES];                   // of the entries: to the end
+    uint16_t entry[ENTRIES];               // the digits of its states, nearest step first | parent << 8
+    uint16_t via[ENTRIES];                 // of child j at j: best entry | its parent << 8 | close second << 14
+    uint16_t group[ENTRIES];               // the groups of level l at groups[l]
+    uint8_t child[ENTRIES];
+    uint16_t at[VT_T / 2 + 2], groups[VT_T / 2 + 2];   // entries of level l: at[l] .. at[l-1]
+    float best[VB_MOST];
+    int kept[VB_MOST];
+};
+static_assert(vb_pool::ENTRIES >= VB_MOST, "a level fits");
+// states from group g by the digits p, nearest step first
+template <int K>
+__device__ __forceinline__ void vb_walk(int g, int p, int (&st)[vb_cfg<K>::DEPTH]) {
+    using C = vb_cfg<K>;
+    int at = g;
+#pragma unroll
+    for (int e = 0; e < C::DEPTH; ++e) {
+        st[e] = ((p >> (K * (C::DEPTH - 1 - e))) & (C::NK - 1)) * C::G + at;
+        at = st[e] >> K;
+    }
+}
+
+// The backtrack of one tile by one wave: 0 and the states in `states`; the limit to try next; infinity where the tile
+// has to be searched exactly.
+// n, gv: the groups of step T (a lane each) whose bounds are within `limit`; x[i]: input of step i; the bounds' row of
+// level l at hist + (l - 1) * G; pre[j]: B at step j * VB_NORM; tie: the only group of step 0, or -1; the states up to
+// step `upto` are wanted.
+template <int K>
+__device__ __forceinline__ float vb_trace(int n, int gv, float limit, const float *x, const uint16_t *__restrict__ hist,
+                                          const float *pre, int tie, int upto, vb_pool *P, int *states) {
+    using C = vb_cfg<K>;
+    constexpr int D = C::DEPTH, LEVELS = C::STORED, R = (1 << (K * D)) / 64;
+    const int lane = threadIdx.x & 63;
+    const float close = limit * 0x1p-14f, inf = __builtin_inff();
+    float cv = 0.0f;                                           // lane j: cost from group gv of this level to the end
+    int ne = 0, ns = 0;
+    bool full = false, empty = false;
+    float xn[D], pn = pre[(LEVELS - 1) * D / VB_NORM];         // read a level ahead
+#pragma unroll
+    for (int e = 0; e < D; ++e) xn[e] = x[VT_T - 1 - e];
+    // The ways from a group, R to a lane, by where their bounds lie: digits of a lane's ways, and the first one's place.
+    constexpr int E = 16 - K - K * D;                          // what of the group is left above the digits
+    int ways[R], place;
+    {
+        const int run = K == 4 ? lane >> 2 : K == 3 ? lane >> 3 : lane;   // the digits but the farthest, the nearest lowest
+        const int in = K == 4 ? (lane & 3) * 4 : K == 3 ? lane & 7 : 0;
+        place = (run << (E + K)) + in;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            int k = in + r;
+            k ^= vb_word<K>(run << E) << 1;
+            ways[r] = K == 2 ? (run & 3) << 6 | (run >> 2 & 3) << 4 | run >> 4 << 2 | k : run << K | k;
+        }
+    }
+    // their bounds, in the row below level l (of level 1, whose row is not stored, any row); requested as soon as a level's
+    // first group is known: they take longer than everything else here
+    u32x2 ahead = {0, 0};
+    auto ask = [&](int l, int g, u32x2 &into) {
+        const uint16_t *row = hist + (uint32_t)((l > 1 ? l - 2 : 0) * C::G) + place + (uint32_t)((g >> (K * D)) << K);
+        if constexpr (R == 4) into = *(const u32x2 *)row;
+        else into.x = *row;
+    };
+    auto bound_of = [&](u32x2 v, int r) { return vb_half((r & 2 ? v.y : v.x) >> (16 * (r & 1)) & 0xFFFFu); };
+    ask(LEVELS, vb_lane(gv, 0), ahead);
+#pragma unroll 1
+    for (int l = LEVELS; l > 0; --l) {
+        full = full || ns + n > P->ENTRIES;
+        if (full || empty) break;
+        if (lane == 0) {
+            P->at[l] = (uint16_t)ne;
+            P->groups[l] = (uint16_t)ns;
+        }
+        if (lane < n) P->group[ns + lane] = (uint16_t)gv;
+        ns += n;
+        const float room = limit - pn;
+        float xs[D];
+#pragma unroll
+        for (int e = 0; e < D; ++e) {
+            xs[e] = xn[e];
+            xn[e] = x[((l - 1) * D - 1 - e) & (VT_T - 1)];
+        }
+        pn = pre[(l > 1 ? l - 2 : 0) * D / VB_NORM];
+        // lane j: child j, its cheapest entry, and the next one's cost
+        int m = 0, nn = 0, ng = -1, nvia = lane;
+        float nc = inf, second = inf;
+#pragma unroll 1
+        for (int j = 0; j < n; ++j) {
+            const int g = vb_lane(gv, j);
+            const float c0 = vb_lane(cv, j);
+            const u32x2 bounds = ahead;
+            if (j + 1 < n) ask(l, vb_lane(gv, j + 1), ahead);  // one group ahead, too
+            int front[R];
+            float c[R], bound[R];
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                int st[D];
+                vb_walk<K>(g, ways[r], st);
+                front[r] = st[D - 1] >> K;
+                c[r] = c0;
+#pragma unroll
+                for (int e = 0; e < D; ++e) c[r] += vt_err(st[e], xs[e]);
+            }
+            uint64_t mask[R];
+            int count = 0;
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                bound[r] = l > 1 ? bound_of(bounds, r) : tie < 0 || front[r] == tie ? 0.0f : inf;
+                mask[r] = __ballot(c[r] + bound[r] <= room);
+                count += __builtin_popcountll(mask[r]);
+            }
+            full = full || m + count > 256 || ne + m + count > P->ENTRIES || (n == 1 && count > VB_MOST);
+            if (full) break;
+            if (n == 1 && count) {
+                int g0 = 0;
+#pragma unroll
+                for (int r = R - 1; r >= 0; --r) g0 = mask[r] ? vb_lane(front[r], __builtin_ctzll(mask[r])) : g0;
+                ask(l - 1, g0, ahead);
+            }
+            int k = m;
+            if (n == 1) {                                      // one parent: its children are all different
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    const int to = k + vb_below(mask[r]);
+                    if (c[r] + bound[r] <= room) {
+                        P->entry[ne + to] = (uint16_t)ways[r];
+                        P->kept[to] = front[r];
+                        P->cost[ne + to] = c[r];
+                    }
+                    k += __builtin_popcountll(mask[r]);
+                }
+                if (lane < count) P->child[ne + lane] = (uint8_t)lane;
+                __builtin_amdgcn_wave_barrier();
+                nn = count;
+                ng = P->kept[lane];
+                nc = P->cost[ne + (lane < count ? lane : 0)];
+                __builtin_amdgcn_wave_barrier();
+            } else {                                           // one entry after the other, in registers: there are a few
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    if (c[r] + bound[r] <= room) {
+                        const int to = ne + k + vb_below(mask[r]);
+                        P->entry[to] = (uint16_t)(ways[r] | j << 8);
+                        P->cost[to] = c[r];
+                    }
+#pragma unroll 1
+                    for (uint64_t rest = mask[r]; rest; rest &= rest - 1, ++k) {
+                        const int from = __builtin_ctzll(rest), f = vb_lane(front[r], from);
+                        const float cf = vb_lane(c[r], from);
+                        const uint64_t same = __ballot(ng == f);
+                        const int child = same ? __builtin_ctzll(same) : nn;
+                        nn = __builtin_amdgcn_readfirstlane(nn + (same ? 0 : 1));
+                        P->child[ne + k] = (uint8_t)child;
+                        const bool mine = lane == child, better = mine && cf < nc;
+                        const float other = __builtin_fmaxf(nc, cf);   // the new one's or, where that is better, the old one's
+                        second = mine && other < second ? other : second;
+                        nvia = better ? k | j << 8 : nvia;
+                        nc = better ? cf : nc;
+                        ng = mine ? f : ng;
+                    }
+                }
+            }
+            m += count;
+        }
+        full = full || nn > VB_MOST;
+        empty = m == 0;
+        if (n != 1) ask(l - 1, vb_lane(ng, 0) & (C::G - 1), ahead);
+        if (lane < nn) P->via[ne + lane] = (uint16_t)(nvia | (second - nc <= close ? 1 << 14 : 0));
+        ne += m;
+        n = nn;
+        gv = ng & (C::G - 1);
+        cv = nc;
+    }
+    if (full) return inf;
+    if (empty) return limit * (1.0f + 0.5f * C::SLACK);
+    if (lane == 0) P->at[0] = (uint16_t)ne;
+    float u = inf, second = inf;
+    int take = 0;
+#pragma unroll 1
+    for (int q = 0; q < n; ++q) {
+        const float cq = vb_lane(cv, q);
+        take = cq < u ? q : take;
+        second = __builtin_fminf(second, __builtin_fmaxf(u, cq));
+        u = __builtin_fminf(u, cq);
+    }
+    if (!(u * (1.0f + 0x1p-14f) <= limit)) return vb_lane(u * (1.0f + 0x1p-13f), 0);
+    // the cheapest path, from the start; where no other one is close to it, it is the answer
+    bool near = second - u <= close;
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll 1
+    for (int l0 = 0; l0 * D <= upto; l0 += 64) {
+        const int ats = P->at[l0 + 1 + lane], gs = P->groups[l0 + 1 + lane];
+        int mine = 0;                                          // lane k: the path's way from level l0 + k to the next
+#pragma unroll 1
+        for (int k = 0; k < 64 && (l0 + k) * D <= upto; ++k) {
+            const int v = __builtin_amdgcn_readfirstlane(P->via[vb_lane(ats, k) + take]);
+            mine = lane == k ? v : mine;
+            near = near || (v >> 14);
+            take = v >> 8 & 63;
+        }
+        if ((l0 + lane) * D <= upto) {
+            int st[D];
+            vb_walk<K>(P->group[gs + (mine >> 8 & 63)], P->entry[ats + (mine & 255)] & 255, st);
+#pragma unroll
+            for (int e = 0; e < D; ++e) states[(l0 + lane + 1) * D - 1 - e] = st[e];
+        }
+    }
+    if (!near) return 0.0f;
+
+    // exact costs, forward over the kept ways that a path close to the cheapest may take; lane e: entry e of the level,
+    // best, cheap: exact cost from the start, cost to the end, of group `lane` of the level below
+    float cheap = P->cost[P->at[1] + (P->via[P->at[1] + lane] & 255)];
+    float best = lane < n && cheap <= u + close ? 0.0f : inf;
+#pragma unroll 1
+    for (int l = 1; l <= LEVELS; ++l) {
+        const int eb = P->at[l], m = __builtin_amdgcn_readfirstlane((int)P->at[l - 1] - eb), nb = P->at[l < LEVELS ? l + 1 : l];
+        if (m > 64) return inf;
+        const int e = eb + (lane < m ? lane : 0), en = P->entry[e], parent = en >> 8, child = P->child[e];
+        int st[D];
+        vb_walk<K>(P->group[P->groups[l] + parent], en & 255, st);
+        float v[D], c = __shfl(best, child, GLQH_WAVE);
+        const float room = __shfl(cheap, child, GLQH_WAVE) + close;
+        const uint64_t live = __ballot(lane < m && c < inf && P->cost[e] <= room);
+#pragma unroll
+        for (int d = D - 1; d >= 0; --d) {
+            c = vt_err(st[d], x[l * D - 1 - d]) + c;
+            v[d] = c;
+        }
+        bool least = live >> lane & 1;     // of its parent (at the end: of all): the lowest cost, then the lowest state, step by step
+#pragma unroll 1
+        for (uint64_t rest = live & (live - 1) ? live : 0; rest; rest &= rest - 1) {
+            const int q = __builtin_ctzll(rest);
+            bool under = false, level = l == LEVELS || vb_lane(parent, q) == parent;
+#pragma unroll
+            for (int d = 0; d < D; ++d) {
+                const float vq = vb_lane(v[d], q);
+                const int sq = vb_lane(st[d], q);
+                under = under || (level && (vq < v[d] || (vq == v[d] && sq < st[d])));
+                level = level && vq == v[d] && sq == st[d];
+            }
+            least = least && !under;
+        }
+        const uint64_t won = __ballot(least);
+        if (l == LEVELS) {
+            take = __builtin_ctzll(won);
+            break;
+        }
+        cheap = P->cost[nb + (P->via[nb + lane] & 255)];
+        if ((won & (won - 1)) == 0) {
+            const int q = __builtin_ctzll(won);
+            best = lane == vb_lane(parent, q) ? vb_lane(v[0], q) : inf;
+        } else {
+            P->best[lane] = inf;
+            __builtin_amdgcn_wave_barrier();
+            if (least) P->best[parent] = v[0];
+            __builtin_amdgcn_wave_barrier();
+            best = P->best[lane];
+        }
+        __builtin_amdgcn_wave_barrier();
+        if (least) P->via[nb + parent] = (uint16_t)lane;       // now: the entry that the group's exact cost comes from
+        __builtin_amdgcn_wave_barrier();
+    }
+#pragma unroll 1
+    for (int l = LEVELS; l > 0; --l) {
+        const int at = P->at[l] + take, en = P->entry[at];
+        int st[D];
+        vb_walk<K>(P->group[P->groups[l] + (en >> 8)], en & 255, st);
+        if (lane == 0) {
+#pragma unroll
+            for (int e = 0; e < D; ++e) states[l * D - 1 - e] = st[e];
+        }
+        if (l > 1) take = __builtin_amdgcn_readfirstlane(P->via[P->at[l] + P->child[at]]);
+    }
+    return 0.0f;
+}
+
+// A wave's memory while it walks back
+struct vb_work {
+    vb_pool pool;
+    float x[VT_T], pre[VT_T / VB_NORM + 1];
+    int states[VT_T], start[VB_MOST];
+};
+
+// The backtrack of tile part.first + at (one wave): after pass 0 the overlap, after pass 1 the states and values.
+// What bounds it is latency: a chain of STORED levels, each a look into a row of which only the last level's group tells
+// where (a microsecond), some 150 instructions and trips to LDS.  150 us on average, 340 for the slowest of 256 tiles.
+template <int K>
+__device__ __forceinline__ void vb_backtrack(const float *__restrict__ tiles_in, int64_t ld, const vb_part &part, int at,
+                                             vb_work *W, int32_t *__restrict__ states_out, float *__restrict__ hat_out) {
+    using C = vb_cfg<K>;
+    float *const x = W->x, *const pre = W->pre;
+    int *const states = W->states, *const start = W->start;
+    const int lane = threadIdx.x & 63, pass = part.pass;
+    const int64_t tile = part.first + at;
+    vb_tile *const mine = part.info + at;
+    const int over = __builtin_amdgcn_readfirstlane(mine->over);
+    if (over < 0) {
+        if (pass && lane == 0) states_out[tile * VT_T] = -1;
+        return;
+    }
+    const int turn = pass ? 0 : VT_T / 2, tie = pass ? over : -1;
+    for (int i = lane; i < VT_T; i += 64) x[i] = (float)(f16)tiles_in[vt_pos(tile, (i + turn) & (VT_T - 1), ld)];
+    for (int i = lane; i <= VT_T / VB_NORM; i += 64) pre[i] = mine->pre[i];
+    const uint16_t *hist = part.rows + (int64_t)at * C::STORED * C::G, *last = hist + (int64_t)(C::STORED - 1) * C::G;
+    __builtin_amdgcn_wave_barrier();
+    const float bt = pre[VT_T / VB_NORM];
+    uint32_t lo = 0xFFFFu;                                     // the least bound of the groups that may be last
+    if (pass) {
+        lo = last[vb_stored<K>(tie)];
+    } else {
+#pragma unroll 8
+        for (int g = 0; g < C::G; g += 64) {
+            const uint32_t v = last[g + lane];
+            lo = v < lo ? v : lo;
+        }
+        lo = vb_wave_min(lo);
+    }
+    float limit = vb_lane((vb_half(lo) + bt) * (1.0f + C::SLACK), 0);
+    bool good = false;
+#pragma unroll 1
+    for (int tries = 0; tries < 4; ++tries) {
+        int n = pass;                                          // the groups of step T within the limit
+        if (pass) {
+            if (lane == 0) start[0] = tie;
+        } else {
+#pragma unroll 1
+            for (int g0 = 0; g0 < C::G; g0 += 512) {
+                float b[8], least = __builtin_inff();
+#pragma unroll
+                for (int k = 0; k < 8; ++k) {
+                    b[k] = vb_half(last[g0 + 64 * k + lane]) + bt;
+                    least = __builtin_fminf(least, b[k]);
+                }
+                if (!__ballot(least <= limit)) continue;
+#pragma unroll
+                for (int k = 0; k < 8; ++k) {
+                    const uint64_t mask = __ballot(b[k] <= limit);
+                    const int at = n + vb_below(mask);
+                    if (b[k] <= limit && at < VB_MOST) start[at] = vb_group<K>(g0 + 64 * k + lane);
+                    n += __builtin_popcountll(mask);
+                }
+            }
+        }
+        __builtin_amdgcn_wave_barrier();
+        if (n > VB_MOST) break;
+        n = __builtin_amdgcn_readfirstlane(n);
+        limit = vb_trace<K>(n, lane < n ? start[lane] : 0, limit, x, hist, pre, tie, pass ? VT_T - 1 : VT_T / 2, &W->pool, states);
+        good = limit == 0.0f;
+        if (good || limit == __builtin_inff()) break;
+        __builtin_amdgcn_wave_barrier();
+    }
+    __builtin_amdgcn_wave_barrier();
+    if (pass == 0) {
+        if (lane == 0) mine->over = good ? states[VT_T / 2] >> K : -1;
+        return;
+    }
+    if (!good) {
+        if (lane == 0) states_out[tile * VT_T] = -1;
+        return;
+    }
+    for (int i = lane; i < VT_T; i += 64) {
+        const int s = states[i];
+        states_out[tile * VT_T + i] = s;
+        hat_out[vt_pos(tile, i, ld)] = (float)tr_weight((uint32_t)s);
+    }
+}
+
+// The first workgroups walk back, a tile to each of their first VB_WALK waves; the others run a forward pass.  Neither
+// part reads what the other one writes: a launch walks back over one batch of tiles while the vector units, which that
+// leaves idle, run another batch forward (1024 and 1024 tiles, K = 2: 1.11 ms, 0.91 + 0.40 in two launches).
+constexpr int VB_WALK = 4;
+template <int K, int TPW>
+constexpr int vb_lds() {
+    constexpr int rows = TPW * vb_cfg<K>::ROWS * vb_cfg<K>::ROW * 4, walk = VB_WALK * (int)sizeof(vb_work);
+    return rows > walk ? rows : walk;
+}
+template <int K, int TPW>
+__global__ void __launch_bounds__(VB_THREADS, 4)
+vb_kernel(const float *__restrict__ tiles_in, int64_t ld, vb_part forward, vb_part back, int walkers,
+          int32_t *__restrict__ states_out, float *__restrict__ hat_out) {
+    extern __shared__ uint32_t lds[];
+    if ((int)blockIdx.x < walkers) {
+        const int wave = threadIdx.x >> 6, at = blockIdx.x * VB_WALK + wave;
+        if (wave >= VB_WALK || at >= back.count) return;
+        __builtin_amdgcn_s_setprio(3);
+        vb_backtrack<K>(tiles_in, ld, back, at, (vb_work *)lds + wave, states_out, hat_out);
+    } else {
+        vb_forward<K, TPW>(tiles_in, ld, forward, blockIdx.x - walkers, gridDim.x - walkers, lds);
     }
 }
 
@@ -402,18 +1140,96 @@ int acs_launch(const float *cost, const void *x, const float *lut, float *cost_o
     return 0;
 }
 
+// Two batches of tiles take turns: while one walks back, the other runs forward.  A batch is a chip full of pairs (two
+// workgroups a CU); everything is one batch where that leaves none to overlap with.
+struct vb_plan {
+    int64_t batch;
+    int batches;                           // in flight: 1 or 2
+};
+vb_plan vb_plan_of(int64_t n_tiles) {
+    const int64_t full = 4 * (int64_t)glqh_device_cus();
+    return n_tiles <= full ? vb_plan{n_tiles, 1} : vb_plan{full, 2};
+}
+template <int K>
+size_t vb_bytes(int64_t n_tiles) {
+    const vb_plan p = vb_plan_of(n_tiles);
+    return (size_t)p.batch * p.batches * (vb_cfg<K>::STORED * vb_cfg<K>::G * 2 + sizeof(vb_tile));
+}
+
+template <int K>
+int vb_launch(const float *tiles, int64_t n_tiles, int64_t ld, void *scratch, int32_t *states, float *hat, hipStream_t stream) {
+    using C = vb_cfg<K>;
+    const vb_plan plan = vb_plan_of(n_tiles);
+    const size_t rows = (size_t)plan.batch * C::STORED * C::G;
+    const int cus = glqh_device_cus();
+    auto part = [&](int64_t batch, int pass) {
+        const int64_t first = batch * plan.batch, left = n_tiles - first;
+        const int slab = (int)(batch & 1);
+        return vb_part{first, (int)(left <= 0 ? 0 : left < plan.batch ? left : plan.batch), pass, (uint16_t *)scratch + slab * rows,
+                       (vb_tile *)((uint16_t *)scratch + plan.batches * rows) + slab * plan.batch};
+    };
+    auto launch = [&](const vb_part &forward, const vb_part &back) {
+        const int walkers = (back.count + VB_WALK - 1) / VB_WALK;
+        // one tile a workgroup while that gives no CU more than two workgroups (512 tiles: 1.58 ms at K = 4, 1.52 at 3); at
+        // K = 2, with one cost row and a barrier to both its sides, a second tile is what fills the wait (2.9 -> 1.66)
+        const bool few = forward.count <= 2 * cus;
+        const int per = few ? C::FEW : 2, work = (forward.count + per - 1) / per;
+        const dim3 grid(walkers + (work < 2 * cus ? work : 2 * cus));
+        if (grid.x == 0) return 0;
+        if (few)
+            hipLaunchKernelGGL((vb_kernel<K, C::FEW>), grid, dim3(VB_THREADS), (vb_lds<K, C::FEW>()), stream, tiles, ld, forward, back,
+                               walkers, states, hat);
+        else
+            hipLaunchKernelGGL((vb_kernel<K, 2>), grid, dim3(VB_THREADS), (vb_lds<K, 2>()), stream, tiles, ld, forward, back, walkers,
+                               states, hat);
+        GLQH_LAUNCH_CHECK("viterbi launch");
+        return 0;
+    };
+    // batches 2i and 2i + 1: F0(a) | F0(b) B0(a) | F1(a) B0(b) | F1(b) B1(a) | F0(a') B1(b) | ...
+    vb_part back{0, 0, 0, nullptr, nullptr};
+    for (int64_t b = 0; b * plan.batch < n_tiles; b += 2)
+        for (int turn = 0; turn < 4; ++turn) {
+            const vb_part forward = part(b + (turn & 1), turn >> 1);
+            if (forward.count == 0 || plan.batches == 1) {     // nothing beside it
+                if (launch(vb_part{0, 0, 0, nullptr, nullptr}, back)) return 1;
+                back.count = 0;
+            }
+            if (forward.count == 0) continue;
+            if (launch(forward, back)) return 1;
+            back = forward;
+        }
+    return launch(vb_part{0, 0, 0, nullptr, nullptr}, back);
+}
+
 template <int K>
 int vt_launch(const float *tiles, int64_t n_tiles, int64_t ld, void *scratch, int grid, int32_t *states, float *hat,
               hipStream_t stream) {
+    int marked = 0;
+    if constexpr (K >= 2) {
+        // a tile a CU is as fast without the bounds' chain of launches (256 tiles, exact / on bounds: 1.38 / 1.62 ms at K = 2,
+        // 1.16 / 1.20 at 3, 1.40 / 1.16 at 4; 512: 2.15 / 1.68, 1.89 / 1.52, 2.18 / 1.58)
+        if (K == 4 || n_tiles > glqh_device_cus()) {
+            if (int rc = vb_launch<K>(tiles, n_tiles, ld, scratch, states, hat, stream)) return rc;
+            marked = 1;
+        }
+    }
     constexpr size_t lds = vt_cfg<K>::ROWS * sizeof(float) * (size_t)vt_cfg<K>::G;
     hipLaunchKernelGGL(viterbi_kernel<K>, dim3((unsigned)grid), dim3(vt_cfg<K>::THREADS), lds, stream, tiles, n_tiles, ld,
-                       (float *)scratch, states, hat);
+                       (float *)scratch, states, hat, marked);
     GLQH_LAUNCH_CHECK("viterbi launch");
     return 0;
 }
 
 template <int K>
 int vt_set_lds() {
+    if constexpr (K >= 2) {
+        auto set = [](const void *kernel, int lds) {
+            return glqh_check_hip(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds), "viterbi attribute");
+        };
+        constexpr int FEW = vb_cfg<K>::FEW;
+        if (int rc = set((const void *)vb_kernel<K, FEW>, vb_lds<K, FEW>()) || set((const void *)vb_kernel<K, 2>, vb_lds<K, 2>()))
+            return rc;
+    }
     return glqh_check_hip(hipFuncSetAttribute((const void *)viterbi_kernel<K>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                               (int)(vt_cfg<K>::ROWS * sizeof(float) * vt_cfg<K>::G)),
                           "viterbi attribute");
@@ -432,7 +1248,9 @@ int glqh_viterbi_grid(int K, int64_t n_tiles) {
 size_t glqh_viterbi_scratch_bytes(int K, int64_t n_tiles) {
     const size_t row = sizeof(float) << (16 - K);
     const int depth = K == 1 ? vt_cfg<1>::DEPTH : K == 2 ? vt_cfg<2>::DEPTH : K == 3 ? vt_cfg<3>::DEPTH : vt_cfg<4>::DEPTH;
-    return (size_t)glqh_viterbi_grid(K, n_tiles) * (VT_T / depth) * row;
+    const size_t exact = (size_t)glqh_viterbi_grid(K, n_tiles) * (VT_T / depth) * row;
+    const size_t bound = K == 2 ? vb_bytes<2>(n_tiles) : K == 3 ? vb_bytes<3>(n_tiles) : K == 4 ? vb_bytes<4>(n_tiles) : 0;
+    return (exact > bound ? exact : bound) + 255 & ~(size_t)255;
 }
 
 // ld: 0 for tiles in step order, else the row length of the (m, n) matrices `tiles` and `hat`

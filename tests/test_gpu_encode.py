@@ -251,3 +251,57 @@ def test_quantize_matrix_equals_the_tile_route(K, m, n):
     assert torch.equal(recon, ext.trellis_tiles_to_matrix(hat, m, n))
     if K > 1:                                            # the dequantizer takes 2..4 bits
         assert torch.equal(ext.glq_decompress_trellis_3inst_cuda(packed, m, n).float(), recon)
+
+
+def _search_tiles(n, seed):
+    """Gaussian tiles with some that the search on bounds leaves to the exact one or has to compare exactly: constant and
+    alternating values, wide ones, inputs that are not finite, few distinct values (ties), tiny ones."""
+    g = torch.Generator().manual_seed(seed)
+    X = torch.randn(n, 256, generator=g) * 0.8933837
+    pick = torch.randperm(n, generator=g)
+    special = [torch.full((256,), 0.25), torch.zeros(256), torch.tensor([1.0, -1.0]).repeat(128), torch.randn(256, generator=g) * 3,
+               torch.randn(256, generator=g) * 20, (torch.randn(256, generator=g) * 2).round() / 2, torch.randn(256, generator=g) * 1e-3,
+               torch.randn(256, generator=g).index_fill(0, torch.tensor([7]), float("inf")), torch.linspace(-16, 16, 256)]
+    for j, s in zip(pick[:n // 2].tolist(), special):
+        X[j] = s
+    return X
+
+
+@pytest.mark.parametrize("K", [2, 3, 4])
+@pytest.mark.parametrize("n", [257, 512, 513, 1025, 2051])
+def test_viterbi_on_bounds_equals_the_exact_search(K, n):
+    """Every route of the search on lower bounds (one and two tiles a workgroup, an odd last pair, one batch and batches
+    that take turns): the states of the same tiles searched a few at a time, which at 2 and 3 bits is the exact kernel
+    (itself pinned on the oracle above), and of the oracle on some of them."""
+    from glq_amd import ext
+    say("viterbi on bounds", K, n)
+    X = _search_tiles(n, 100 * K + n)
+    hat, st = ext.trellis_quantize_tiles(X.to(DEV), K)
+    few = [ext.trellis_quantize_tiles(c.to(DEV), K) for c in X.split(200)]
+    assert torch.equal(st, torch.cat([f[1] for f in few])), (st != torch.cat([f[1] for f in few])).any(1).nonzero()[:5]
+    assert torch.equal(hat, torch.cat([f[0] for f in few]))
+    if n == 513:
+        some = torch.cat([X[:12], X[-4:]])
+        _, ref = O.trellis_quantize_tiles(some.numpy(), K)
+        got = torch.cat([st[:12], st[-4:]]).cpu().numpy()
+        finite = torch.isfinite(some).all(1).numpy()
+        assert np.array_equal(got[finite], ref[finite])
+
+
+def test_viterbi_under_capture():
+    """Captured and replayed on other tiles: the launches' batches hand each other their rows through the same memory."""
+    from glq_amd import ext
+    say("viterbi under capture")
+    X = torch.zeros(1100, 256, device=DEV)
+    ext.trellis_quantize_tiles(X[:4], 4)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        hat, st = ext.trellis_quantize_tiles(X, 4)
+    for turn in range(3):
+        X.copy_(_search_tiles(1100, turn))
+        graph.replay()
+        torch.cuda.synchronize()
+        want = ext.trellis_quantize_tiles(X, 4)
+        assert torch.equal(st, want[1]) and torch.equal(hat, want[0]), turn
