@@ -53,6 +53,7 @@ struct tt_args {
     int64_t out_stride;
     int out_f16;                                   // partial sums as fp16 (not with direct)
     int rt0;                                       // first row tile of this launch (RT counts from there)
+    int half_rt;                                   // row tiles behind the RT ones, each done as two tiles of 64 rows
     const uint8_t *packed2;                        // the residual stage's stream of a stacked layer (kernels with R2 > 0)
     float rs2;                                     // and its scale
 };
@@ -116,7 +117,7 @@ __device__ __forceinline__ void tt_barrier() {     // waits for LDS only: global
 // Decode role of a wave in both tile kernels: from half a record (block pair `unit` of the tile, k-pair `kpi` of the
 // step, m-tile `ms`) the two A operands of row groups 2 ms and 2 ms + 1, the two fp16 halves of every weight added
 // first (the dequantizer's rounding), written in operand layout (lane L's 16 bytes at slot L of operand
-// kpi * 8 + unit * 4 + 2 ms + rh).  half = -1: both operands; 0 / 1: operand rh = half only.
+// op + rh, op = kpi * 8 + unit * 4 + 2 ms).  half = -1: both operands; 0 / 1: operand rh = half only.
 template <int R>
 __device__ __forceinline__ void tt_decode(const tr_record<R> &r, int ms, int next1, int next2, u32x4 (&af)[2], int half) {
     uint32_t c0 = ms ? r.c[1] : r.c[0], c1 = ms ? r.c[3] : r.c[2];
@@ -150,13 +151,13 @@ __device__ __forceinline__ void tt_decode(const tr_record<R> &r, int ms, int nex
 }
 
 template <int R>
-__device__ __forceinline__ void tt_emit(const tr_record<R> &r, int unit, int kpi, int ms, int next1, int next2, int lane,
-                                        u32x4 *dst, int half = -1) {
+__device__ __forceinline__ void tt_emit(const tr_record<R> &r, int op, int ms, int next1, int next2, int lane, u32x4 *dst,
+                                        int half = -1) {
     u32x4 af[2];
     tt_decode<R>(r, ms, next1, next2, af, half);
 #pragma unroll
     for (int rh = 0; rh < 2; ++rh)
-        if (half < 0 || rh == half) dst[(kpi * TT_FRAGS + unit * 4 + 2 * ms + rh) * GLQH_WAVE + lane] = af[rh];
+        if (half < 0 || rh == half) dst[(op + rh) * GLQH_WAVE + lane] = af[rh];
 }
 
 // A stacked layer (glq/trellis.py:923-933: W = W1 + inv_resid_scale2 * W2): both stages' weights of the operand,
@@ -164,8 +165,8 @@ __device__ __forceinline__ void tt_emit(const tr_record<R> &r, int unit, int kpi
 // decompressed stages into one fp16 matrix before its GEMM (glq/csrc/glq_trellis.cu:1322-1334,
 // glq/quantized_linear.py:986-1010) -- so the products of a stacked layer are those of a single one.
 template <int R, int R2>
-__device__ __forceinline__ void tt_emit2(const tr_record<R> &r, const tr_record<R2> &rb, float rs2, int unit, int kpi,
-                                         int ms, int next1, int next2, int lane, u32x4 *dst, int half = -1) {
+__device__ __forceinline__ void tt_emit2(const tr_record<R> &r, const tr_record<R2> &rb, float rs2, int op, int ms,
+                                         int next1, int next2, int lane, u32x4 *dst, int half = -1) {
     u32x4 af[2], bf[2];
     tt_decode<R>(r, ms, next1, next2, af, half);
     tt_decode<R2>(rb, ms, next1, next2, bf, half);
@@ -176,7 +177,7 @@ __device__ __forceinline__ void tt_emit2(const tr_record<R> &r, const tr_record<
         f16x8 o;
 #pragma unroll
         for (int e = 0; e < 8; ++e) o[e] = (f16)((float)x[e] + rs2 * (float)y[e]);
-        dst[(kpi * TT_FRAGS + unit * 4 + 2 * ms + rh) * GLQH_WAVE + lane] = __builtin_bit_cast(u32x4, o);
+        dst[(op + rh) * GLQH_WAVE + lane] = __builtin_bit_cast(u32x4, o);
     }
 }
 
@@ -186,7 +187,15 @@ __device__ __forceinline__ void tt_emit2(const tr_record<R> &r, const tr_record<
 // read the operands back from LDS (64 KB per step and workgroup instead of 128, which at 16 or 32 tokens per
 // wave costs more cycles than their products), and a SIMD's decode runs beside its products instead of between
 // them.  Same tiles, K slots and order of summation as the plain form with NTW / 2: the same bits.
-template <int R, int NTW, int MODE, int R2 = 0, bool PC = false>
+//
+// TF: 16-row operands per k-half.  8: tiles of 128 rows, row tiles 0 .. RT - 1.  4 (PC only): tiles of 64 rows, the two
+// halves of the half_rt row tiles behind those, for what would be a last round of 128-row tiles on at most half of the CUs: half
+// the products and half the decode a tile (every decoding wave one m-tile of one block pair), the same activations.  Such a
+// round is bound by a step's chain from record to product more than by the products, so it takes nine tenths of a round of
+// 128-row tiles and not half: grouped gate/up of 2 x 11008 rows x 2048 columns at 512 tokens (256 tiles of 128 rows and 176
+// of 64 in place of 344) 81.0 -> 77.6 us the whole call.  Tiles of 512 tokens have no such form: it took longer than the
+// 256-token tiles of a launch of its own for the last round (14336 x 4096 at 4096 tokens 482 -> 490 us).
+template <int R, int NTW, int MODE, int R2 = 0, bool PC = false, int TF = TT_FRAGS>
 __device__ __forceinline__ void tr_tile_body(const tt_args &a, const tt_group &g, const tt_moe &mo) {
     constexpr bool GROUP = MODE == TT_GROUP, MOE = MODE == TT_MOE;
     constexpr int MW = PC ? 4 : TT_WAVES;                       // multiplying waves
@@ -200,12 +209,15 @@ __device__ __forceinline__ void tr_tile_body(const tt_args &a, const tt_group &g
     // decode role (PC: of waves 4..7, both m-tiles)
     const bool producer = PC && wave >= 4;                      // uniform over the wave
     const int dw = PC ? 2 * (wave & 3) : wave;
-    const int unit = dw >> 2, kpi = (dw >> 1) & 1, ms = dw & 1;
+    constexpr bool HALF = TF == 4;
+    static_assert(!HALF || PC, "tiles of 64 rows have decoding and multiplying waves");
+    const int kpi = HALF ? (wave >> 1) & 1 : (dw >> 1) & 1, ms = HALF ? wave & 1 : dw & 1;
     const int hm = i >> 3, l = 4 * (i & 7) + q;
     const int l1 = (l + 1) & 31, l2 = (l + 2) & 31;
     const int next1 = 16 * (l1 & 3) + 8 * hm + (l1 >> 2), next2 = 16 * (l2 & 3) + 8 * hm + (l2 >> 2);
 
-    int nitems = a.TT * a.KS * a.RT;
+    const int RT = HALF ? 2 * a.half_rt : a.RT;
+    int nitems = a.TT * a.KS * RT;
     if constexpr (MOE) nitems = *mo.n_tiles * a.RT * a.TT;      // one K slot; TT = workgroup tiles per run
     const int per_xcd = (nitems + 7) >> 3;
     const int xcd = blockIdx.x & 7, bx = blockIdx.x >> 3;
@@ -213,8 +225,9 @@ __device__ __forceinline__ void tr_tile_body(const tt_args &a, const tt_group &g
     for (int w = bx; w < per_xcd; w += nbx) {
         const int item = xcd * per_xcd + w;
         if (item >= nitems) break;                              // uniform
-        const int slot = (item / a.RT) % a.KS, tt0 = item / (a.RT * a.KS);
-        int rt = a.rt0 + item % a.RT;                           // row tile of its layer
+        const int slot = (item / RT) % a.KS, tt0 = item / (RT * a.KS);
+        int rt = HALF ? a.RT + (item % RT >> 1) : a.rt0 + item % RT;   // row tile of its layer
+        const int unit = HALF ? item % RT & 1 : dw >> 2;        // block pair of the row tile that this wave decodes
         int lm = a.m;
         const uint8_t *lpacked = a.packed;
         const f16 *lxb = a.xb;
@@ -253,7 +266,8 @@ __device__ __forceinline__ void tr_tile_body(const tt_args &a, const tt_group &g
             }
             active = __builtin_amdgcn_readfirstlane((int)(tok0 < limit)) != 0;
         }
-        const int r0 = rt * TT_ROWS;
+        const int r0 = rt * TT_ROWS + (HALF ? 64 * unit : 0);
+        if (HALF && r0 >= lm) continue;                         // uniform over the workgroup
         const int ds0 = slot * a.slot_ds, ds1 = min(ds0 + a.slot_ds, nds);
 
         const int mp = min(2 * (2 * rt + unit) + hm, mpairs - 1);
@@ -267,18 +281,22 @@ __device__ __forceinline__ void tr_tile_body(const tt_args &a, const tt_group &g
             if constexpr (R2 > 0) r = tr_load_record<RB>(rec_base2 + (int64_t)min(d, ds1 - 1) * 64 * REC2);
             return r;
         };
+        auto emit_tile = [&](const tr_record<R> &r, const tr_record<RB> &rb, int mt, u32x4 *dst, int half = -1) {
+            const int op = kpi * TF + (HALF ? 0 : 4 * unit) + 2 * mt;
+            if constexpr (R2 > 0) tt_emit2<R, RB>(r, rb, lrs2, op, mt, next1, next2, lane, dst, half);
+            else tt_emit<R>(r, op, mt, next1, next2, lane, dst, half);
+        };
         auto emit = [&](const tr_record<R> &r, const tr_record<RB> &rb, u32x4 *dst, int half = -1) {
-            if constexpr (R2 > 0) tt_emit2<R, RB>(r, rb, lrs2, unit, kpi, ms, next1, next2, lane, dst, half);
-            else tt_emit<R>(r, unit, kpi, ms, next1, next2, lane, dst, half);
+            emit_tile(r, rb, ms, dst, half);
         };
         // multiply role: token 16 * tt + i of the wave's tokens; k-pair kp, slot q at xb[(kp * Mp + token) * 4 + q]
         // (the token dimension of xb is padded to whole tiles: no clamping, constant offsets)
         const int64_t bstep = (int64_t)a.Mp * 32;               // elements from one k-pair to the next
         const f16 *xrow = lxb + (int64_t)(tok0 + i) * 32 + q * 8;
 
-        f32x4 acc[TT_FRAGS][NTW];
+        f32x4 acc[TF][NTW];
 #pragma unroll
-        for (int f = 0; f < TT_FRAGS; ++f)
+        for (int f = 0; f < TF; ++f)
 #pragma unroll
             for (int tt = 0; tt < NTW; ++tt) acc[f][tt] = f32x4{0.f, 0.f, 0.f, 0.f};
 
@@ -295,10 +313,11 @@ __device__ __forceinline__ void tr_tile_body(const tt_args &a, const tt_group &g
         if constexpr (PC) {
             if (producer) {                                     // as many barriers as the multiplying waves meet
                 auto emit_both = [&](const tr_record<R> &r, const tr_record<RB> &rb, u32x4 *dst) {
-#pragma unroll
-                    for (int mt = 0; mt < 2; ++mt) {
-                        if constexpr (R2 > 0) tt_emit2<R, RB>(r, rb, lrs2, unit, kpi, mt, next1, next2, lane, dst);
-                        else tt_emit<R>(r, unit, kpi, mt, next1, next2, lane, dst);
+                    if constexpr (HALF) {
+                        emit_tile(r, rb, ms, dst);
+                    } else {
+                        emit_tile(r, rb, 0, dst);
+                        emit_tile(r, rb, 1, dst);
                     }
                 };
                 tr_record<R> p1 = load_rec(ds0 + 1), p2 = load_rec(ds0 + 2);
@@ -358,14 +377,14 @@ __device__ __forceinline__ void tr_tile_body(const tt_args &a, const tt_group &g
             ring[1] = __builtin_bit_cast(f16x8, rd[GLQH_WAVE + lane]);
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int kk = 0; kk < 2 * TT_FRAGS; ++kk) {
-                const int u = kk / TT_FRAGS, f = kk % TT_FRAGS;
+            for (int kk = 0; kk < 2 * TF; ++kk) {
+                const int u = kk / TF, f = kk % TF;
                 if (f == 0) {
                     load_half(bs[(2 * j + u + 2) % 3], 2 * (d - ds0) + u + 2);
                     __builtin_amdgcn_sched_barrier(0);
                 }
                 const f16x8 af = ring[kk & 1];
-                if (kk + 2 < 2 * TT_FRAGS) ring[kk & 1] = __builtin_bit_cast(f16x8, rd[(kk + 2) * GLQH_WAVE + lane]);
+                if (kk + 2 < 2 * TF) ring[kk & 1] = __builtin_bit_cast(f16x8, rd[(kk + 2) * GLQH_WAVE + lane]);
 #pragma unroll
                 for (int tt = 0; tt < NTW; ++tt)
                     acc[f][tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
@@ -397,7 +416,7 @@ __device__ __forceinline__ void tr_tile_body(const tt_args &a, const tt_group &g
         for (int tt = 0; tt < NTW; ++tt) {
             if ((MOE && !active) || producer) break;
 #pragma unroll
-            for (int f = 0; f < TT_FRAGS; ++f)
+            for (int f = 0; f < TF; ++f)
                 *(f32x4 *)(ep + i * TT_EP_STRIDE + 64 * (f >> 2) + 8 * (f & 3) + rlane) = acc[f][tt];
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
             if (!a.direct && a.out_f16) {                       // uniform
@@ -410,7 +429,7 @@ __device__ __forceinline__ void tr_tile_body(const tt_args &a, const tt_group &g
                     f32x4 v1 = *(const f32x4 *)(ep + tl * TT_EP_STRIDE + rl + 4);
                     if constexpr (MOE) { v0 *= osc; v1 *= osc; }
                     else { v0 *= f16sc; v1 *= f16sc; }
-                    if (tok >= limit || row >= lm) continue;    // m is a multiple of 32: whole runs of eight
+                    if (tok >= limit || row >= lm || (HALF && rl >= 64)) continue;   // m is a multiple of 32: whole runs of eight
                     if constexpr (MOE) tok = mo.perm[tok];
                     typedef _Float16 f16x8o __attribute__((ext_vector_type(8)));
                     const int64_t e = ((int64_t)slot * a.M + tok) * lm + row;
@@ -425,7 +444,7 @@ __device__ __forceinline__ void tr_tile_body(const tt_args &a, const tt_group &g
                     int tok = tok0 + 16 * tt + tl;
                     f32x4 v = *(const f32x4 *)(ep + tl * TT_EP_STRIDE + rl);
                     if constexpr (MOE) v *= osc;
-                    if (tok >= limit || row >= lm) continue;
+                    if (tok >= limit || row >= lm || (HALF && rl >= 64)) continue;
                     if constexpr (MOE) tok = mo.perm[tok];
                     if (!a.direct) {
                         *(f32x4 *)(lout + ((int64_t)slot * a.M + tok) * lm + row) = v;
@@ -458,18 +477,27 @@ template <int R, int NTW>
 __global__ void __launch_bounds__(TT_THREADS)
 tr_tile_pc_kernel(const tt_args a) {
     tr_tile_body<R, NTW, TT_PLAIN, 0, true>(a, tt_group{}, tt_moe{});
+    if constexpr (NTW == 4) {
+        if (a.half_rt) tr_tile_body<R, NTW, TT_PLAIN, 0, true, 4>(a, tt_group{}, tt_moe{});
+    }
 }
 
 template <int R2, int NTW>
 __global__ void __launch_bounds__(TT_THREADS)
 tr_tile_rvq_pc_kernel(const tt_args a) {
     tr_tile_body<4, NTW, TT_PLAIN, R2, true>(a, tt_group{}, tt_moe{});
+    if constexpr (NTW == 4) {
+        if (a.half_rt) tr_tile_body<4, NTW, TT_PLAIN, R2, true, 4>(a, tt_group{}, tt_moe{});
+    }
 }
 
 template <int R, int NTW>
 __global__ void __launch_bounds__(TT_THREADS)
 tr_tile_group_pc_kernel(const tt_args a, const tt_group g) {
     tr_tile_body<R, NTW, TT_GROUP, 0, true>(a, g, tt_moe{});
+    if constexpr (NTW == 4) {
+        if (a.half_rt) tr_tile_body<R, NTW, TT_GROUP, 0, true, 4>(a, g, tt_moe{});
+    }
 }
 
 // a stacked layer (first stage 4 bits/weight): both streams decoded into one operand
@@ -496,6 +524,9 @@ template <int R2, int NTW>
 __global__ void __launch_bounds__(TT_THREADS)
 tr_tile_group_rvq_pc_kernel(const tt_args a, const tt_group g) {
     tr_tile_body<4, NTW, TT_GROUP, R2, true>(a, g, tt_moe{});
+    if constexpr (NTW == 4) {
+        if (a.half_rt) tr_tile_body<4, NTW, TT_GROUP, R2, true, 4>(a, g, tt_moe{});
+    }
 }
 
 template <int R, int NTW>
@@ -597,8 +628,9 @@ __device__ __forceinline__ void tr_tile_small_body(const tt_args &a, const tt_gr
             return r;
         };
         auto emit = [&](const tr_record<R> r, const tr_record<RB> rb, u32x4 *dst) {
-            if constexpr (R2 > 0) tt_emit2<R, RB>(r, rb, y.rs2, unit, kpi, ms, next1, next2, lane, dst);
-            else tt_emit<R>(r, unit, kpi, ms, next1, next2, lane, dst);
+            const int op = kpi * TT_FRAGS + 4 * unit + 2 * ms;
+            if constexpr (R2 > 0) tt_emit2<R, RB>(r, rb, y.rs2, op, ms, next1, next2, lane, dst);
+            else tt_emit<R>(r, op, ms, next1, next2, lane, dst);
         };
         // multiply role: token 16 * tt + i of the wave's token group
         const int64_t bstep = (int64_t)a.Mp * 32;               // elements from one k-pair to the next
@@ -854,6 +886,20 @@ bool tt_split_roles(const tt_plan &p, int min_steps) {
     return pc && p.NTW <= 2 && p.slot_ds >= (pc_steps > 0 ? pc_steps : min_steps);
 }
 
+// The last round of 256-token tiles of decoding and multiplying waves (slots of min_steps steps and more): where it would
+// run on at most half of the CUs, its row tiles become tiles of 64 rows in the same launch, twice as many: they end in one
+// round (with more than half of the CUs taken they would need two, each nine tenths of the one they replace).
+void tt_halve_last_round(const tt_plan &p, int min_steps, tt_args *a) {
+    a->half_rt = 0;
+    if (p.NTW != 2 || !tt_split_roles(p, min_steps) || p.KS != 1) return;
+    const int64_t cus = glqh_device_cus(), rounds = (int64_t)p.RT * p.TT / cus;
+    if (rounds < 1) return;
+    const int whole = (int)(rounds * cus / p.TT), rest = p.RT - whole;
+    if (rest <= 0 || 2 * (int64_t)rest * p.TT > cus) return;
+    a->RT = whole;
+    a->half_rt = rest;
+}
+
 template <int R, int NTW>
 int tt_launch(const tt_plan &p, const tt_args &a, hipStream_t stream) {
     hipLaunchKernelGGL((tr_tile_kernel<R, NTW>), dim3((unsigned)p.grid), dim3(TT_THREADS), TT_LDS, stream, a);
@@ -982,6 +1028,7 @@ int glqh_launch_trellis_tile(const void *x_f16, void *xb_scratch, int64_t M, con
     a.out_stride = out_stride;
     a.out_f16 = out_f16;
     a.rt0 = 0;
+    tt_halve_last_round(p, packed2 ? 8 : 16, &a);
     a.packed2 = (const uint8_t *)packed2;
     a.rs2 = rs2;
     if (packed2) {
@@ -1130,6 +1177,7 @@ int glqh_launch_trellis_tile_group(const void *const xb[], int64_t M, const void
     a.TT = p.TT;
     a.KS = p.KS;
     a.slot_ds = p.slot_ds;
+    tt_halve_last_round(p, 8, &a);
     a.out_f16 = out_f16;
     if (packed2) {
         switch (R2) {

@@ -111,6 +111,14 @@ def test_grouped_calls_against_single_layers(ms, n, B, bits, shared_sv):
         off += m
 
 
+@pytest.mark.parametrize("ms,n,B,bits", [((32768, 1056, 544), 1024, 256, (4,)), ((20512, 12384), 576, 200, (2,)),
+                                         ((32640, 288), 1024, 130, (4, 2)), ((10912, 96, 160), 256, 1500, (3,))])
+def test_grouped_last_round_of_half_tiles(ms, n, B, bits):
+    """The last round of row tiles as tiles of 64 rows across the layers of a group: layers that begin in it and layers whose
+    last tile has 32, 96 or all of its rows."""
+    test_grouped_calls_against_single_layers(ms, n, B, bits, False)
+
+
 def test_grouped_many_tokens_refusals():
     from glq_amd import ext
     say("grouped many tokens refusals")

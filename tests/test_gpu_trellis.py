@@ -139,6 +139,23 @@ def test_matmul_large_batch_tiles(ext, m, n, B, K):
     assert rel(first, rows) < 1e-3
 
 
+@pytest.mark.parametrize("m,n,B,K", [(32768 + 32, 1024, 256, 4), (49152, 1024, 200, 3), (32768 + 224, 1024, 129, 2),
+                                     (11392 - 96, 128, 1500, 4), (16384 - 32, 192, 1025, 3), (14336, 320, 2048, 4)])
+def test_matmul_last_round_of_half_tiles(ext, m, n, B, K):
+    """A last round of row tiles on at most half of the CUs runs as tiles of 64 rows: one row tile of 32 rows (its second
+    half is empty), as many as there can be, 96 rows in the last one; tiles of 256 and of 512 tokens, ragged in the tokens.
+    The products are exact in fp32 and added in fp32: n roundings of at most the sum of their sizes, one more of the scale."""
+    say("matmul half tiles", m, n, B, K)
+    pt = t(O.random_packed(m, n, K, seed=5))
+    xt = t((np.random.default_rng(B).standard_normal((B, n)) * 0.5).astype(np.float16))
+    W = ext.glq_decompress_trellis_3inst_cuda(pt, m, n).double()
+    out = ext.glq_decode_matmul_trellis_3inst_cuda(xt, pt, m, n, 0.25)
+    ref, size = 0.25 * (xt.double() @ W.T), 0.25 * (xt.double().abs() @ W.abs().T)
+    assert out.shape == (B, m) and bool(((out.double() - ref).abs() <= (n + 1) * 2.0 ** -24 * size).all())
+    ext.glq_decode_matmul_trellis_3inst_cuda(xt, pt, m, n, 0.25, out=out, accum=True)
+    assert bool(((out.double() - 2 * ref).abs() <= (2 * n + 3) * 2.0 ** -24 * size).all())
+
+
 def _layer_args(art, m, n, dtype):
     from glq_amd import hadamard as H
     bn, bm = art["blocks_n"], art["blocks_m"]
