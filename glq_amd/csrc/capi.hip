@@ -1268,6 +1268,14 @@ int glqh_launch_moe_weighted_sum(const void *y_f16, int64_t y_stride, int num_to
 
 int glqh_moe_mid_eligible(int64_t m_pad13, const int64_t *blocks_m13, int64_t n_blocks_m13, int64_t n_pad2,
                           const int64_t *blocks_n2, int64_t n_blocks_n2);
+int glqh_moe_mid_few_eligible(int64_t m_pad13, const int64_t *blocks_m13, int64_t n_blocks_m13, int64_t n_pad2,
+                              const int64_t *blocks_n2, int64_t n_blocks_n2);
+int glqh_launch_moe_mid_few(const float *part, int ks, int part_f16, int n_slots, int n_experts, const int64_t *topk_ids,
+                            const void *su_base, const float *wscale_dev, int64_t out_features13, int64_t m_pad13,
+                            const int64_t *blocks_m13, int64_t n_blocks_m13, const int *perm, const int *pexp,
+                            const int *n_valid, int64_t intermediate, int act, const void *sv2, int64_t n_pad2,
+                            const int64_t *blocks_n2, int64_t n_blocks_n2, void *out_f16, int layout, int64_t Mp,
+                            hipStream_t stream);
 int glqh_launch_moe_mid(const float *part, int ks, int part_f16, int n_slots, int n_experts, const int64_t *topk_ids,
                         const void *su_base, const float *wscale_dev, int64_t out_features13, int64_t m_pad13,
                         const int64_t *blocks_m13, int64_t n_blocks_m13, const int *perm, const int *pexp, const int *n_valid,
@@ -1281,6 +1289,10 @@ int glqh_moe_route_segments(int n_slots, int n_experts);
 size_t glqh_moe_route_scratch_ints(int n_slots, int n_experts);
 int glqh_launch_moe_route(const int64_t *topk_ids, int n_slots, int n_experts, int *perm, int *pexp, int *offs,
                           int *scratch, hipStream_t stream);
+int glqh_launch_moe_route_input(const int64_t *topk_ids, int n_slots, int n_experts, int *perm, int *pexp, int *offs,
+                                const void *x, int x_dtype, int64_t x_stride, const void *sv, void *out_f16, int64_t rows,
+                                int64_t in_features, int64_t n_pad, const int64_t *blocks_host, int64_t n_blocks,
+                                hipStream_t stream);
 int glqh_moe_grouped_wide(int n_slots, int n_experts);
 int glqh_launch_trellis_mma_moe_grouped(const void *packed, int64_t stride_bytes, int R, const int *perm,
                                         const int *offs, int n_slots, int n_experts, int x_div,
@@ -1362,8 +1374,11 @@ static bool moe_fuse_enabled() {
     }();
     return on;
 }
-// from this many slots on (below, the separate launches are as fast or faster: 128 slots 108.8 us separate against
-// 112.6 fused, 512 slots 147.1 / 148.2, 1024 slots 161.2 / 161.5, 2048 slots 222 / 215, 8192 slots 531 / 493)
+// Between the decode launches one launch always, where the blocks allow it: below MOE_MID_FEW_SLOTS slots the form with a
+// row's blocks side by side, above the one with a row's blocks in turn (both measured beside the kernels).  Behind the second
+// decode launch one launch from MOE_FUSE_MIN_SLOTS slots on (whole call, separate / one: 128 slots 81.4 / 84.4 us with a
+// token's choices side by side, 512 slots 147.1 / 148.2, 1024 slots 161.2 / 161.5, 2048 slots 222 / 215, 8192 slots 531 / 493).
+constexpr int MOE_MID_FEW_SLOTS = 4096;
 constexpr int MOE_FUSE_MIN_SLOTS = 1024;
 
 static int moe_proj_plan(const glqh_moe_proj *w, int64_t n_slots, int64_t n_experts, bool grouped, const char *what, moe_plan *p) {
@@ -1483,9 +1498,11 @@ static int moe_decode_grouped(const glqh_moe_proj *w, const moe_plan &p, const i
 // launch per stage into fp16 sums [stage][slot][row], times the expert's scale (and the second stage's)
 static int moe_decode_tile(const glqh_moe_proj *w, const moe_plan &p, const int *perm, const int *offs, const void *tiles,
                            const int *n_tiles, int n_slots, int n_experts, int x_div, const void *x, int x_dtype,
-                           int64_t x_stride, int64_t x_rows, void *xhat, void *xb, float *part, hipStream_t st) {
+                           int64_t x_stride, int64_t x_rows, void *xhat, void *xb, float *part, hipStream_t st,
+                           bool transformed = false) {
     if (x) {                                                   // nullptr: xb already holds the packed activations
-        if (glqh_launch_input_rht(x, x_dtype, x_stride, w->sv_f16, xhat, GLQH_F16, x_rows, w->in_features, w->n_pad,
+        if (!transformed &&                                    // transformed: xhat already holds the rows
+            glqh_launch_input_rht(x, x_dtype, x_stride, w->sv_f16, xhat, GLQH_F16, x_rows, w->in_features, w->n_pad,
                                   w->bn_meta_dev, w->blocks_n, w->n_blocks_n, 0.0f, st))
             return 1;
         if (glqh_launch_trellis_pack_moe(xhat, xb, perm, offs, n_slots, n_experts, x_div, w->n_pad, st)) return 1;
@@ -1559,7 +1576,15 @@ extern "C" int glqh_fused_moe_trellis_3inst(const void *x, int x_dtype, int64_t 
     void *xhat = base + l.xhat;
     GLQH_REQUIRE(!grouped || num_experts <= 65535, "routed experts: at most 65535 experts, got %lld", (long long)num_experts);
     int *pexp = (int *)(base + l.pexp);
-    if (grouped && glqh_launch_moe_route(topk_ids, n_slots, (int)num_experts, perm, pexp, offs, (int *)(base + l.route), st))
+    // the routing table and, where that is one launch, the rows' input transform in it
+    int rows_in = -1;
+    if (grouped)
+        rows_in = glqh_launch_moe_route_input(topk_ids, n_slots, (int)num_experts, perm, pexp, offs, x, x_dtype, x_stride,
+                                              w13->sv_f16, xhat, num_tokens, w13->in_features, w13->n_pad, w13->blocks_n,
+                                              w13->n_blocks_n, st);
+    if (rows_in > 0) return 1;
+    if (grouped && rows_in < 0 &&
+        glqh_launch_moe_route(topk_ids, n_slots, (int)num_experts, perm, pexp, offs, (int *)(base + l.route), st))
         return 1;
     const bool tile = p13.tile != 0;
     void *xb = base + l.xb, *tiles = base + l.tiles;
@@ -1567,17 +1592,29 @@ extern "C" int glqh_fused_moe_trellis_3inst(const void *x, int x_dtype, int64_t 
     if (tile && glqh_launch_trellis_tile_moe_table(offs, n_slots, (int)num_experts, tiles, n_tiles, st)) return 1;
     // gate | up of every slot: decode on the token's row, output transform with the expert's signs
     if (tile ? moe_decode_tile(w13, p13, perm, offs, tiles, n_tiles, n_slots, (int)num_experts, (int)top_k, x, x_dtype,
-                               x_stride, num_tokens, xhat, xb, part13, st)
-        : grouped ? moe_decode_grouped(w13, p13, perm, offs, n_slots, (int)num_experts, (int)top_k, x, x_dtype, x_stride,
-                                       num_tokens, xhat, part13, st)
+                               x_stride, num_tokens, xhat, xb, part13, st, rows_in == 0)
+        : grouped ? moe_decode_grouped(w13, p13, perm, offs, n_slots, (int)num_experts, (int)top_k, rows_in == 0 ? nullptr : x,
+                                       x_dtype, x_stride, num_tokens, xhat, part13, st)
                   : moe_decode(w13, p13, topk_ids, n_slots, (int)num_experts, (int)top_k, x, x_dtype, x_stride, part13, st))
         return 1;
-    // between the decode launches: one launch per slot row for the grouped forms, three or four otherwise
+    // between the decode launches: one launch, or three or four where the blocks are too large for it
     const bool mid = grouped && n_slots >= MOE_FUSE_MIN_SLOTS && moe_fuse_enabled() &&
                      glqh_moe_mid_eligible(w13->m_pad, w13->blocks_m, w13->n_blocks_m, w2->n_pad, w2->blocks_n,
                                            w2->n_blocks_n);
+    const bool few = n_slots < MOE_MID_FEW_SLOTS && moe_fuse_enabled() &&
+                     glqh_moe_mid_few_eligible(w13->m_pad, w13->blocks_m, w13->n_blocks_m, grouped ? w2->n_pad : 0,
+                                               w2->blocks_n, w2->n_blocks_n);
     const void *x2 = hact;
-    if (mid) {
+    if (few) {
+        const int layout = !grouped ? 3 : tile ? 2 : 0;
+        if (glqh_launch_moe_mid_few(part13, p13.ks_all, tile, n_slots, (int)num_experts, topk_ids, w13->su_f16, w13->wscale_dev,
+                                    w13->out_features, w13->m_pad, w13->blocks_m, w13->n_blocks_m, perm, pexp,
+                                    offs + num_experts, intermediate_size, activation_type, w2->sv_f16, w2->n_pad, w2->blocks_n,
+                                    w2->n_blocks_n, layout == 3 ? (void *)hact : layout == 2 ? xb : xhat, layout,
+                                    tile ? glqh_trellis_tile_moe_padded(n_slots, num_experts) : 0, st))
+            return 1;
+        if (grouped) x2 = nullptr;
+    } else if (mid) {
         if (glqh_launch_moe_mid(part13, p13.ks_all, tile, n_slots, (int)num_experts, topk_ids, w13->su_f16, w13->wscale_dev,
                                 w13->out_features, w13->m_pad, w13->blocks_m, w13->n_blocks_m, perm, pexp, offs + num_experts,
                                 intermediate_size, activation_type, w2->sv_f16, w2->n_pad, w2->blocks_n, w2->n_blocks_n,

@@ -1294,6 +1294,111 @@ moe_mid_kernel(moe_mid_args a, f16 *__restrict__ out, glqh_meta_args m13, glqh_m
     }
 }
 
+// The same for up to a few thousand slots, where a launch is its chain of latencies and not its instructions: the blocks of a
+// row side by side, whole waves each and eight elements a thread, a thread's sums and signs requested at once, four barriers
+// in all (the form above takes the blocks in turn on few waves, which longer than 4096 slots is the cheaper one).
+// LAYOUT 0: workgroup = slot.  LAYOUT 2: workgroup = sorted position.  LAYOUT 3: workgroup = slot, and the activated row
+// itself is stored (slots of an invalid expert: zeros) for a second projection that transforms its own rows.
+// Whole call, the separate launches (3 or 2) -> this one, microseconds: 128 experts of 2048 -> 2 x 768 -> 2048 at 8 / 32 /
+// 128 / 512 slots 27.5 / 52.5 / 85.5 / 126.3 -> 26.6 / 50.5 / 83.3 / 124.0, 32 of 1024 x 512 at 80 slots 35.8 -> 33.2, 16
+// of 2048 x 768 at 384 slots (tile form) 67.9 -> 63.1; against the form above 16 of 1024 x 512 at 2048 slots 75.0 ->
+// 74.1, 128 of 2048 x 768 at 4096 slots 272.7 -> 273.5 (not taken).
+struct mid_part {
+    rht_slice blk;
+    int te;                                                      // the thread's number among those of its block
+    bool any;                                                    // false: past the row's waves
+};
+
+// waves of a block of `bs` points at eight elements a thread
+__host__ __device__ __forceinline__ int mid_waves(int bs) { return bs > 512 ? bs >> 9 : 1; }
+
+__device__ __forceinline__ mid_part mid_part_of(const glqh_meta_args &m, int nb) {
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    mid_part p = {};
+    int w0 = 0;
+    for (int j = 0; j < nb; ++j) {                               // uniform over the wave
+        const rht_slice b = rht_slice_of(m, 0.0f, j);
+        const int nw = mid_waves(b.bs);
+        if (wave >= w0 && wave < w0 + nw) {
+            p.blk = b;
+            p.te = (wave - w0) * 64 + lane;
+            p.any = true;
+        }
+        w0 += nw;
+    }
+    return p;
+}
+
+template <int LAYOUT>
+__global__ void __launch_bounds__(1024)
+moe_mid_few_kernel(moe_mid_args a, f16 *__restrict__ out, glqh_meta_args m13, glqh_meta_args m2) {
+    extern __shared__ float s[];
+    int pos = blockIdx.x, slot = blockIdx.x;
+    int64_t e;
+    if constexpr (LAYOUT == 2) {
+        pos = (pos >> 6) * 64 + (pos & 7) * 8 + ((pos >> 3) & 7);
+        if (pos >= *a.n_valid) return;                           // uniform over the workgroup
+        slot = a.perm[pos];
+        e = a.pexp[pos];
+    } else {
+        e = a.o.topk_ids[slot];
+        if (e < 0 || e >= a.o.n_experts) {                       // uniform over the workgroup
+            if constexpr (LAYOUT == 3)
+                for (int i = threadIdx.x; i < a.intermediate; i += blockDim.x) out[(int64_t)slot * a.intermediate + i] = (f16)0.0f;
+            return;
+        }
+    }
+    f16 *hrow = (f16 *)(s + a.s_floats);
+    const mid_part p13 = mid_part_of(m13, a.nb13);
+    const bool act13 = p13.any && 8 * p13.te < p13.blk.bs;
+    float v[8], f[8];
+    output_wide_load<8>(v, moe_src(a.o, a.o.wscale_dev[e]), slot, a.o.m_pad, p13.blk, act13, p13.te);
+    int idx[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+        idx[q] = p13.blk.off + fht_wave_index<8>(p13.blk.log_len, act13 ? p13.te : 0, q);
+        f[q] = (float)a.o.su_base[e * a.o.m_pad + idx[q]];
+    }
+    if (p13.any) fht_wave<8, true>(v, p13.blk.log_len, s + p13.blk.off, p13.te);
+    else fht_barrier<false>();
+    if (act13) {
+#pragma unroll
+        for (int q = 0; q < 8; ++q) hrow[idx[q]] = (f16)(v[q] * (p13.blk.norm * f[q]));
+    }
+    __syncthreads();
+    auto activated = [&](int i) { return (f16)(moe_gate((float)hrow[i], a.act) * (float)hrow[a.intermediate + i]); };
+    if constexpr (LAYOUT == 3) {
+        for (int i = threadIdx.x; i < a.intermediate; i += blockDim.x) out[(int64_t)slot * a.intermediate + i] = activated(i);
+    } else {
+        const mid_part p2 = mid_part_of(m2, a.nb2);
+        const bool act2 = p2.any && 8 * p2.te < p2.blk.bs;
+        const int i0 = p2.blk.off + 8 * p2.te;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = f[j] = 0.0f;
+        if (act2) {
+            load8<f16>(a.sv2 + i0, f);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) v[j] = i0 + j < a.intermediate ? (float)activated(i0 + j) * f[j] : 0.0f;
+        }
+        if (p2.any) fht_wave<8, true>(v, p2.blk.log_len, s + p2.blk.off, p2.te);
+        else fht_barrier<false>();
+        if (act2) {                                              // hrow has been read: it takes the transformed row
+#pragma unroll
+            for (int q = 0; q < 8; ++q)
+                hrow[p2.blk.off + fht_wave_index<8>(p2.blk.log_len, p2.te, q)] = (f16)(v[q] * p2.blk.norm);
+        }
+        __syncthreads();
+        for (int c = threadIdx.x; c < a.n_pad2 >> 3; c += blockDim.x) {
+            if constexpr (LAYOUT == 2) {
+                const uint32_t *r = (const uint32_t *)hrow + 16 * (c >> 2) + (c & 3);   // columns 2q + {0,1,8,9,16,17,24,25}
+                *(u32x4 *)(out + (((int64_t)(c >> 2) * a.Mp + pos) * 4 + (c & 3)) * 8) = u32x4{r[0], r[4], r[8], r[12]};
+            } else {
+                *(u32x4 *)(out + (int64_t)slot * a.n_pad2 + 8 * c) = *(const u32x4 *)(hrow + 8 * c);
+            }
+        }
+    }
+}
+
 // The second projection's output transform and the weighted sum over a token's choices in one launch, for many
 // tokens: rows = tokens, dealt out like output_rht_wide_kernel's; a thread transforms its part of every choice in
 // turn, rounds it to fp16 as the separate launch stores it, and adds it times the routing weight in fp32, choices
@@ -1423,10 +1528,9 @@ moe_weighted_sum_kernel(const f16 *__restrict__ y, int64_t y_stride, const int64
 // Slots grouped by expert, without a sort: wave e counts the valid slots of experts below e
 // (offs[e]; wave n_experts: the total, offs[n_experts]) and then writes its own slots, in ascending
 // slot order, from that position on.  Fixed by the routing alone: the same table on every call.
-__global__ void __launch_bounds__(256)
-moe_route_kernel(const int64_t *__restrict__ topk_ids, int n_slots, int n_experts, int *__restrict__ perm,
-                 int *__restrict__ pexp, int *__restrict__ offs) {
-    const int e = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+__device__ __forceinline__ void moe_route_body(const int64_t *__restrict__ topk_ids, int n_slots, int n_experts,
+                                               int *__restrict__ perm, int *__restrict__ pexp, int *__restrict__ offs, int wg) {
+    const int e = wg * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (e > n_experts) return;                                   // uniform over the wave
     constexpr int U = 8;                                         // 512 slots requested before the first is looked at
     int below = 0;
@@ -1455,6 +1559,34 @@ moe_route_kernel(const int64_t *__restrict__ topk_ids, int n_slots, int n_expert
             mine += __builtin_popcountll(hit);
         }
     }
+}
+
+__global__ void __launch_bounds__(256)
+moe_route_kernel(const int64_t *__restrict__ topk_ids, int n_slots, int n_experts, int *__restrict__ perm,
+                 int *__restrict__ pexp, int *__restrict__ offs) {
+    moe_route_body(topk_ids, n_slots, n_experts, perm, pexp, offs, blockIdx.x);
+}
+
+// The table and the input transform of the tokens' rows, which wait for nothing of each other, in one launch: the first
+// route_wgs workgroups write the table, the others transform one block of one row each.  Whole call, one launch each -> this:
+// 128 experts of 2048 -> 2 x 768 -> 2048 at 32 / 128 / 512 slots 50.6 / 83.3 / 123.8 -> 48.6 / 81.7 / 121.2 us, 32 of
+// 1024 x 512 at 80 slots 33.2 -> 31.3, 16 of 1024 x 512 at 2048 slots 74.3 -> 71.3.
+template <typename XT>
+__global__ void __launch_bounds__(256)
+moe_route_input_kernel(const int64_t *__restrict__ topk_ids, int n_slots, int n_experts, int *__restrict__ perm,
+                       int *__restrict__ pexp, int *__restrict__ offs, int route_wgs, const XT *__restrict__ x,
+                       int64_t x_stride, const f16 *__restrict__ sv, f16 *__restrict__ out, int in_features, int n_pad, int nb,
+                       glqh_meta_args margs) {
+    extern __shared__ float s[];
+    if ((int)blockIdx.x < route_wgs) {
+        moe_route_body(topk_ids, n_slots, n_experts, perm, pexp, offs, blockIdx.x);
+        return;
+    }
+    const int item = blockIdx.x - route_wgs, token = item / nb;
+    const rht_slice blk = rht_slice_of(margs, 0.0f, item % nb);
+    const wide_role role = {(int)threadIdx.x, 0, 256, 0, true};
+    if (blk.log_bs > 11) input_rht_wide_body<16, XT, f16, 0>(x, x_stride, sv, out, in_features, n_pad, 0, token, blk, s, role);
+    else input_rht_wide_body<8, XT, f16, 0>(x, x_stride, sv, out, in_features, n_pad, 0, token, blk, s, role);
 }
 
 // The same table for many slots, in two launches: the slots in SEG segments, wave (expert, segment) first counts
@@ -1596,6 +1728,70 @@ int glqh_moe_mid_eligible(int64_t m_pad13, const int64_t *blocks_m13, int64_t n_
     return b13 <= (1 << WIDE_LOG_MAX) && b2 <= (1 << WIDE_LOG_MAX) && (m_pad13 & 7) == 0 && (n_pad2 & 31) == 0;
 }
 
+// threads of the few-slot form (0: not served): the waves of the row with more of them, blocks of at most 4096 points
+// (fht_wave of eight elements); n_pad2 0: the activated row is the result
+static int moe_mid_few_threads(int64_t m_pad13, const int64_t *blocks_m13, int64_t n_blocks_m13, int64_t n_pad2,
+                               const int64_t *blocks_n2, int64_t n_blocks_n2) {
+    int64_t pads[2] = {m_pad13, n_pad2};
+    int waves = 0;
+    for (int r = 0; r < (n_pad2 ? 2 : 1); ++r) {
+        const int64_t nb = r ? n_blocks_n2 : n_blocks_m13, *b = r ? blocks_n2 : blocks_m13;
+        glqh_meta_args m;
+        if (pads[r] & (r ? 31 : 7) || pads[r] >= 8192) return 0;
+        if (!glqh_fill_meta_args(&m, nb > 1 ? b : nullptr, nb > 1 ? nb : 1, pads[r]) || m.canon != pads[r]) return 0;
+        int w = 0;
+        for (int l = 12; l >= 3; --l)
+            if (pads[r] >> l & 1) w += mid_waves(1 << l);
+        waves = std::max(waves, w);
+    }
+    return waves <= 16 ? 64 * waves : 0;
+}
+
+int glqh_moe_mid_few_eligible(int64_t m_pad13, const int64_t *blocks_m13, int64_t n_blocks_m13, int64_t n_pad2,
+                              const int64_t *blocks_n2, int64_t n_blocks_n2) {
+    return moe_mid_few_threads(m_pad13, blocks_m13, n_blocks_m13, n_pad2, blocks_n2, n_blocks_n2) > 0;
+}
+
+// layout 3: n_pad2 0, perm, pexp and n_valid unused
+int glqh_launch_moe_mid_few(const float *part, int ks, int part_f16, int n_slots, int n_experts, const int64_t *topk_ids,
+                            const void *su_base, const float *wscale_dev, int64_t out_features13, int64_t m_pad13,
+                            const int64_t *blocks_m13, int64_t n_blocks_m13, const int *perm, const int *pexp,
+                            const int *n_valid, int64_t intermediate, int act, const void *sv2, int64_t n_pad2,
+                            const int64_t *blocks_n2, int64_t n_blocks_n2, void *out_f16, int layout, int64_t Mp,
+                            hipStream_t stream) {
+    glqh_range range("output_rht");
+    const int threads = moe_mid_few_threads(m_pad13, blocks_m13, n_blocks_m13, layout == 3 ? 0 : n_pad2, blocks_n2, n_blocks_n2);
+    GLQH_REQUIRE(threads > 0, "routed experts: block sizes not served by the fused middle launch");
+    GLQH_REQUIRE(act >= 0 && act <= 2, "routed experts: gated activations 0 (silu), 1 (gelu-tanh), 2 (relu2), got %d", act);
+    GLQH_REQUIRE(aligned16(part) && aligned16(su_base) && aligned16(out_f16) && (layout == 3 || aligned16(sv2)),
+                 "routed experts: unaligned rows");
+    glqh_meta_args m13 = {}, m2 = {};
+    m13.canon = (int)m_pad13;
+    m2.canon = (int)n_pad2;
+    moe_mid_args a = {};
+    a.o = {part, ks, part_f16, n_slots, n_experts, topk_ids, (const f16 *)su_base, wscale_dev, (int)out_features13,
+           (int)m_pad13};
+    a.sv2 = (const f16 *)sv2;
+    a.perm = perm;
+    a.pexp = pexp;
+    a.n_valid = n_valid;
+    a.intermediate = (int)intermediate;
+    a.act = act;
+    a.n_pad2 = (int)n_pad2;
+    a.Mp = (int)Mp;
+    a.nb13 = __builtin_popcountll((unsigned long long)m_pad13);
+    a.nb2 = __builtin_popcountll((unsigned long long)n_pad2);
+    const int64_t row = (std::max(m_pad13, layout == 3 ? 0 : n_pad2) + 7) & ~7;
+    a.s_floats = (int)row;
+    const size_t lds = (size_t)row * (sizeof(float) + sizeof(f16));
+    const dim3 grid((unsigned)(layout == 2 ? 64 * ((n_slots + 63) / 64) : n_slots)), block((unsigned)threads);
+    if (layout == 2) hipLaunchKernelGGL(moe_mid_few_kernel<2>, grid, block, lds, stream, a, (f16 *)out_f16, m13, m2);
+    else if (layout == 3) hipLaunchKernelGGL(moe_mid_few_kernel<3>, grid, block, lds, stream, a, (f16 *)out_f16, m13, m2);
+    else hipLaunchKernelGGL(moe_mid_few_kernel<0>, grid, block, lds, stream, a, (f16 *)out_f16, m13, m2);
+    GLQH_LAUNCH_CHECK("routed-expert middle launch, few slots");
+    return 0;
+}
+
 // sums of the first projection -> transformed activations of the second (layout 0: rows by slot; 2: the tile
 // kernel's blocked operand by sorted position, Mp positions), for the slots listed in perm[0 .. *n_valid)
 int glqh_launch_moe_mid(const float *part, int ks, int part_f16, int n_slots, int n_experts, const int64_t *topk_ids,
@@ -1702,6 +1898,33 @@ int glqh_launch_moe_route(const int64_t *topk_ids, int n_slots, int n_experts, i
                            n_experts, seg_slots, n_seg, scratch, perm, pexp, offs);
     }
     GLQH_LAUNCH_CHECK("routed-expert routing launch");
+    return 0;
+}
+
+// routing table and transformed rows (fp16, n_pad apart) in one launch; -1 (nothing launched) where it does not apply
+int glqh_launch_moe_route_input(const int64_t *topk_ids, int n_slots, int n_experts, int *perm, int *pexp, int *offs,
+                                const void *x, int x_dtype, int64_t x_stride, const void *sv, void *out_f16, int64_t rows,
+                                int64_t in_features, int64_t n_pad, const int64_t *blocks_host, int64_t n_blocks,
+                                hipStream_t stream) {
+    glqh_meta_args margs;
+    if (glqh_moe_route_segments(n_slots, n_experts) != 1 || n_pad >= 8192 || (n_pad & 7) || (x_stride & 7)) return -1;
+    if (!glqh_fill_meta_args(&margs, n_blocks > 1 ? blocks_host : nullptr, n_blocks > 1 ? n_blocks : 1, n_pad) ||
+        margs.canon != n_pad)
+        return -1;
+    if (!x || !aligned16(x) || !aligned16(sv) || !aligned16(out_f16) || in_features < 1 || in_features > n_pad) return -1;
+    glqh_range range("input_rht");
+    const int nb = __builtin_popcountll((unsigned long long)n_pad), route_wgs = (n_experts + 1 + 3) / 4;
+    const size_t lds = rht_reg_lds_bytes(63 - __builtin_clzll((unsigned long long)n_pad));
+    const dim3 grid((unsigned)(route_wgs + rows * nb));
+    if (x_dtype == GLQH_F16)
+        hipLaunchKernelGGL(moe_route_input_kernel<f16>, grid, dim3(256), lds, stream, topk_ids, n_slots, n_experts, perm, pexp,
+                           offs, route_wgs, (const f16 *)x, x_stride, (const f16 *)sv, (f16 *)out_f16, (int)in_features,
+                           (int)n_pad, nb, margs);
+    else
+        hipLaunchKernelGGL(moe_route_input_kernel<uint16_t>, grid, dim3(256), lds, stream, topk_ids, n_slots, n_experts, perm,
+                           pexp, offs, route_wgs, (const uint16_t *)x, x_stride, (const f16 *)sv, (f16 *)out_f16,
+                           (int)in_features, (int)n_pad, nb, margs);
+    GLQH_LAUNCH_CHECK("routed-expert routing and input launch");
     return 0;
 }
 

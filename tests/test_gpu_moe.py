@@ -294,6 +294,30 @@ def test_rows_with_a_block_of_8192_points(ext, hidden, inter):
     assert torch.equal(y, ext.glq_fused_moe_trellis_3inst_cuda(x.to(DEV), t(ids), t(w), *a))
 
 
+@pytest.mark.parametrize("hidden,inter,T,K,act,dtype", [
+    (256, 2048, 2, 2, 0, torch.float16),           # per slot; one block of 4096 points, eight waves
+    (64, 448, 12, 2, 1, torch.bfloat16),           # grouped; blocks of 512 .. 128 points side by side, of 256 .. 64 behind them
+    (4032, 192, 40, 2, 2, torch.float16),          # tile form (27 rows an expert); blocks of 2048 .. 64 columns beside the table
+    (64, 1984, 9, 2, 0, torch.bfloat16),           # grouped; nine waves and then six
+    (64, 1984, 3, 2, 0, torch.bfloat16),           # per slot, the same row
+    (64, 4032, 9, 2, 0, torch.float16),            # a row of seventeen waves: the separate launches
+    (4096, 64, 30, 1, 0, torch.bfloat16),          # rows of one block of 4096 columns beside the table
+    (8192, 64, 8, 2, 1, torch.float16)])           # rows too long for that launch
+def test_launches_between_the_projections(ext, hidden, inter, T, K, act, dtype):
+    """One launch between the two decode launches and one for the routing table and the input rows, at the edges of the
+    shapes that they serve, with a choice of no valid expert; the bar is the file's."""
+    say("moe between", hidden, inter, T, K, act)
+    ex = experts(3, hidden, inter, seed=4)
+    ids, w = routing(T, K, 3, T)
+    ids[T // 2, K - 1] = 3
+    x = torch.from_numpy(np.random.default_rng(T).standard_normal((T, hidden)).astype(np.float32)).to(dtype)
+    a = ex.device_args(act)
+    y = ext.glq_fused_moe_trellis_3inst_cuda(x.to(DEV), t(ids), t(w), *a)
+    ref = ex.oracle(x.float().numpy(), ids, w, act)
+    assert rel(y, ref) < TOL, rel(y, ref)
+    assert torch.equal(y, ext.glq_fused_moe_trellis_3inst_cuda(x.to(DEV), t(ids), t(w), *a))
+
+
 def test_large_activations_stay_finite_in_the_tile_form(ext):
     """Squared-ReLU experts on activations of a few units: the second projection's unscaled sums pass the fp16
     range while the result does not; the tile form's fp16 sums carry the expert's scale, so it stays finite and
