@@ -25,6 +25,7 @@
 // while the tiles alone would leave CUs idle; partial sums [slot][token][row] are combined in slot
 // order by the consumer, or, with one slot, the scaled result is written (or added) in place.
 #include <algorithm>
+#include <type_traits>
 #include "common.h"
 #include "trellis_device.h"
 
@@ -665,73 +666,95 @@ __device__ __forceinline__ void tr_tile_small_body(const tt_args &a, const tt_gr
 #pragma unroll
         for (int dd = 0; dd < 4; ++dd) emit(rc[dd], rcb[dd], abuf + dd * TT_BUF);
         tt_barrier();
-        for (int qd = 0; qd < nquads; qd += 2) {
+        // group qd: multiplied out of buffer qd & 1 while the next group is decoded into the other one, from e / eb
+        // (the branches also keep decode and products of a step apart, which two waves per SIMD overlap better than the
+        // compiler does within one: without them where both groups are whole, 14336 x 4096 at 64 tokens 45.7 -> 54.0 us)
+        auto group = [&](int qd, tr_record<R> (&e)[4], tr_record<RB> (&eb)[4]) {
+            const int d0 = ds0 + 4 * qd;
+            const u32x4 *rd = abuf + (qd & 1) * 4 * TT_BUF + rg * GLQH_WAVE + lane;
+            u32x4 *wr = abuf + ((qd & 1) ^ 1) * 4 * TT_BUF;
 #pragma unroll
-            for (int h = 0; h < 2; ++h) {                       // group qd + h: buffer h
-                if (qd + h < nquads) {                          // uniform
-                    const int d0 = ds0 + 4 * (qd + h);
-                    const u32x4 *rd = abuf + h * 4 * TT_BUF + rg * GLQH_WAVE + lane;
-                    u32x4 *wr = abuf + (h ^ 1) * 4 * TT_BUF;
+            for (int dd = 0; dd < 4; ++dd) {
+                // operand kk of the step: half-step kk / TG, operand rg + RG (kk % TG); read PF ahead
+                constexpr int NK = 2 * TG, PF = NK < 4 ? NK : 4;
+                auto frag = [&](int kk) {
+                    return __builtin_bit_cast(f16x8, rd[dd * TT_BUF + ((kk / TG) * TT_FRAGS + RG * (kk % TG)) * GLQH_WAVE]);
+                };
+                f16x8 ring[PF];
 #pragma unroll
-                    for (int dd = 0; dd < 4; ++dd) {
-                        rc[dd] = rn[dd];
-                        rn[dd] = load_rec(d0 + 8 + dd);
-                        rcb[dd] = rnb[dd];
-                        rnb[dd] = load_rec2(d0 + 8 + dd);
+                for (int kk = 0; kk < PF; ++kk) ring[kk] = frag(kk);
+                load_b(b[(dd + 3) & 3], d0 + dd + 3);
+                if (d0 + 4 + dd < ds1) emit(e[dd], eb[dd], wr + dd * TT_BUF);   // operands of the next group, uniform
+                if (d0 + dd < ds1) {                            // uniform: a slot need not be whole groups
+#pragma unroll
+                    for (int kk = 0; kk < NK; ++kk) {
+                        const f16x8 af = ring[kk % PF];
+                        if (kk + PF < NK) ring[kk % PF] = frag(kk + PF);
+#pragma unroll
+                        for (int tt = 0; tt < NTW; ++tt)
+                            acc[kk % TG][tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                                af, __builtin_bit_cast(f16x8, b[dd][tt][kk / TG]), acc[kk % TG][tt], 0, 0, 0);
                     }
-#pragma unroll
-                    for (int dd = 0; dd < 4; ++dd) {
-                        // operand kk of the step: half-step kk / TG, operand rg + RG (kk % TG); read PF ahead
-                        constexpr int NK = 2 * TG, PF = NK < 4 ? NK : 4;
-                        auto frag = [&](int kk) {
-                            return __builtin_bit_cast(f16x8, rd[dd * TT_BUF + ((kk / TG) * TT_FRAGS + RG * (kk % TG)) * GLQH_WAVE]);
-                        };
-                        f16x8 ring[PF];
-#pragma unroll
-                        for (int kk = 0; kk < PF; ++kk) ring[kk] = frag(kk);
-                        load_b(b[(dd + 3) & 3], d0 + dd + 3);
-                        if (d0 + 4 + dd < ds1) emit(rc[dd], rcb[dd], wr + dd * TT_BUF);   // operands of the next group, uniform
-                        if (d0 + dd < ds1) {                    // uniform: a slot need not be whole groups
-#pragma unroll
-                            for (int kk = 0; kk < NK; ++kk) {
-                                const f16x8 af = ring[kk % PF];
-                                if (kk + PF < NK) ring[kk % PF] = frag(kk + PF);
-#pragma unroll
-                                for (int tt = 0; tt < NTW; ++tt)
-                                    acc[kk % TG][tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
-                                        af, __builtin_bit_cast(f16x8, b[dd][tt][kk / TG]), acc[kk % TG][tt], 0, 0, 0);
-                            }
-                        }
-                    }
-                    tt_barrier();                               // rd has been read, wr is written
                 }
             }
+            tt_barrier();                                       // rd has been read, wr is written
+        };
+        // Records of the group after the next one are requested into the set that the previous group has emptied, by turns;
+        // none past the slot's end (2048 x 11008 at 37 tokens, 4 + 2 bits in slots of 11 steps, the call 28.1 -> 27.4 us).
+        // Where nothing is requested it is another piece of code, not a branch around the request: behind that the waits would
+        // have to assume that nothing was (14336 x 4096 at 64 tokens, slots of 32 steps, 47.1 -> 48.6 us).
+        auto request = [&](int qd, tr_record<R> (&r)[4], tr_record<RB> (&rb)[4]) {
+#pragma unroll
+            for (int dd = 0; dd < 4; ++dd) {
+                r[dd] = load_rec(ds0 + 4 * qd + dd);
+                rb[dd] = load_rec2(ds0 + 4 * qd + dd);
+            }
+        };
+        int qd = 0;
+        for (; qd + 3 < nquads; qd += 2) {
+            request(qd + 2, rc, rcb);
+            group(qd, rn, rnb);
+            request(qd + 3, rn, rnb);
+            group(qd + 1, rc, rcb);
         }
+        if (qd + 2 < nquads) {                                  // uniform: three groups left
+            request(qd + 2, rc, rcb);
+            group(qd++, rn, rnb);
+#pragma unroll
+            for (int dd = 0; dd < 4; ++dd) { rn[dd] = rc[dd]; rnb[dd] = rcb[dd]; }
+        }
+        for (; qd < nquads; ++qd) group(qd, rn, rnb);           // the last one decodes nothing
 
         // lane holds four consecutive rows of token i for every (operand, token tile): operand
-        // f = 4 unit' + s covers rows 64 unit' + 32 h + 8 s + (0..7), h = 0, 1
+        // f = 4 unit' + s covers rows 64 unit' + 32 h + 8 s + (0..7), h = 0, 1.  The tile leaves through LDS, 512 bytes of a
+        // token's rows at a time and not as 16-byte pieces from the lanes (with the requests above, whole calls, 4 bits:
+        // 2048 x 11008 at 37 tokens 23.3 -> 22.3 us, 4096 x 14336 at 40 32.4 -> 31.3, 8192 x 8192 at 48 36.0 -> 34.7,
+        // 512 x 512 at 20 12.5 -> 12.0; 4 + 2 bits 2048 x 11008 at 37 28.1 -> 27.0, 14336 x 4096 at 64 47.0 -> 45.9)
         const int rlane = 32 * (q >> 1) + 4 * (q & 1);
+        float *ep = (float *)abuf;
 #pragma unroll
-        for (int tt = 0; tt < NTW; ++tt) {
-            const int tok = 16 * NTW * tg + 16 * tt + i;
-            if (tok >= a.M) continue;
+        for (int tt = 0; tt < NTW; ++tt)
 #pragma unroll
             for (int j = 0; j < TG; ++j) {
                 const int f = rg + RG * j;
-                const int row = r0 + 64 * (f >> 2) + 8 * (f & 3) + rlane;
-                if (row >= y.m) continue;                       // m is a multiple of 32: whole groups of four
-                if (!a.direct) {
-                    *(f32x4 *)(y.out + ((int64_t)slot * a.M + tok) * y.m + row) = acc[j][tt];
+                *(f32x4 *)(ep + (16 * NTW * tg + 16 * tt + i) * TT_EP_STRIDE + 64 * (f >> 2) + 8 * (f & 3) + rlane) = acc[j][tt];
+            }
+        tt_barrier();
+        for (int c = threadIdx.x; c < 32 * a.M; c += TT_THREADS) {
+            const int tok = c >> 5, rl = 4 * (c & 31), row = r0 + rl;
+            if (row >= y.m) continue;                           // m is a multiple of 32: whole groups of four
+            f32x4 v = *(const f32x4 *)(ep + tok * TT_EP_STRIDE + rl);
+            if (!a.direct) {
+                *(f32x4 *)(y.out + ((int64_t)slot * a.M + tok) * y.m + row) = v;
+            } else {
+                float *o = y.out + (int64_t)tok * a.out_stride + row;
+                if ((a.out_stride & 3) == 0) {
+                    v *= a.scale;
+                    if (a.accum) v += *(f32x4 *)o;
+                    *(f32x4 *)o = v;
                 } else {
-                    float *o = y.out + (int64_t)tok * a.out_stride + row;
-                    if ((a.out_stride & 3) == 0) {
-                        f32x4 v = acc[j][tt] * a.scale;
-                        if (a.accum) v += *(f32x4 *)o;
-                        *(f32x4 *)o = v;
-                    } else {
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) o[e] = a.accum ? o[e] + acc[j][tt][e] * a.scale : acc[j][tt][e] * a.scale;
-                    }
+                    for (int e = 0; e < 4; ++e) o[e] = a.accum ? o[e] + v[e] * a.scale : v[e] * a.scale;
                 }
             }
         }

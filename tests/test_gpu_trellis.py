@@ -156,6 +156,23 @@ def test_matmul_last_round_of_half_tiles(ext, m, n, B, K):
     assert bool(((out.double() - 2 * ref).abs() <= (2 * n + 3) * 2.0 ** -24 * size).all())
 
 
+@pytest.mark.parametrize("n,B,K", [(64, 17, 4), (256, 64, 2), (320, 32, 3), (576, 33, 4), (768, 49, 2), (832, 64, 4),
+                                   (1088, 20, 3), (1344, 37, 4)])
+def test_matmul_groups_of_four_steps(ext, n, B, K):
+    """17..64 tokens: one to six groups of four steps in a K slot, whole and ragged, a last row tile of 32 rows, stored and
+    added in place.  The same bound as above."""
+    m = 32768 + 32                                 # more row tiles than CUs: one K slot
+    say("matmul groups", n, B, K)
+    pt = t(O.random_packed(m, n, K, seed=6))
+    xt = t((np.random.default_rng(B).standard_normal((B, n)) * 0.5).astype(np.float16))
+    W = ext.glq_decompress_trellis_3inst_cuda(pt, m, n).double()
+    out = ext.glq_decode_matmul_trellis_3inst_cuda(xt, pt, m, n, 0.25)
+    ref, size = 0.25 * (xt.double() @ W.T), 0.25 * (xt.double().abs() @ W.abs().T)
+    assert out.shape == (B, m) and bool(((out.double() - ref).abs() <= (n + 1) * 2.0 ** -24 * size).all())
+    ext.glq_decode_matmul_trellis_3inst_cuda(xt, pt, m, n, 0.25, out=out, accum=True)
+    assert bool(((out.double() - 2 * ref).abs() <= (2 * n + 3) * 2.0 ** -24 * size).all())
+
+
 def _layer_args(art, m, n, dtype):
     from glq_amd import hadamard as H
     bn, bm = art["blocks_n"], art["blocks_m"]
