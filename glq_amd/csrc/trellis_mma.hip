@@ -105,48 +105,65 @@ __device__ __forceinline__ mma_lane mma_lane_of(int lane) {
 }
 
 // Sum the four waves' accumulators through LDS in wave order and write them out, G row
-// groups per pass (all four when the buffer allows).  red: [TR_WAVES][G][NT][4][4*TP] floats.
+// groups per pass (all four when the buffer allows).
 template <int NT>
 constexpr int mma_red_groups() { return NT <= 2 ? 4 : 2; }
 
+// A wave's sums in LDS: value (row group sg, token tile tt, row 4 q + r of the group's sixteen, token) at
+// sg * SS + (4 tt + r) * RS + q * TP + token.  They are written with the tokens along the lanes, as the products leave them,
+// and read with the rows along the lanes, so that a token's 64 rows leave as one run of 256 bytes and not as 4-byte pieces, a
+// line each (whole calls of 16 tokens, 4 bits: 4096 x 14336 26.8 -> 26.3 us, 14336 x 4096 31.1 -> 30.8, 14336 x 14336 61.1 ->
+// 60.4; 5 tokens at 4 + 2 bits, 14336 x 4096 33.4 -> 33.1); RS and SS put the 64 rows of a token on 64 banks.
 template <int TP, int NT>
-constexpr int mma_red_bytes() { return TR_WAVES * mma_red_groups<NT>() * NT * 4 * 4 * TP * 4; }
+struct mma_red {
+    static constexpr int G = mma_red_groups<NT>();
+    static constexpr int RS = TP == 16 ? 68 : TP == 8 ? 34 : 4 * TP;
+    static constexpr int SS = 4 * NT * RS + (TP > 1 ? 1 : 0);
+    static constexpr int WAVE = G * SS;
+    static constexpr int VALUES = 16 * G * NT * TP;              // of a pass
+    int row, token, at;                                          // row of the pass's strip (s0 = 0), token, place
+    __device__ __forceinline__ explicit mma_red(int e) {
+        const int rl = e % (16 * G), sg = (rl >> 3) % G, i = 8 * (rl / (8 * G)) + (rl & 7);
+        token = e / (16 * G);
+        row = 32 * (i >> 3) + (i & 7) + 8 * sg;
+        at = sg * SS + (4 * (token / TP) + (i & 3)) * RS + (i >> 2) * TP + token % TP;
+    }
+    template <typename ACC>
+    static __device__ __forceinline__ void put(float *red, const ACC &acc, int s0, int cl) {   // cl = q * TP + token
+#pragma unroll
+        for (int sg = 0; sg < G; ++sg)
+#pragma unroll
+            for (int tt = 0; tt < NT; ++tt)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) red[sg * SS + (4 * tt + r) * RS + cl] = acc.v[s0 + sg][tt][r];
+    }
+    static __device__ __forceinline__ float sum(const float *red, int at) {
+        float v = red[at];
+#pragma unroll
+        for (int w = 1; w < TR_WAVES; ++w) v += red[w * WAVE + at];
+        return v;
+    }
+};
+
+template <int TP, int NT>
+constexpr int mma_red_bytes() { return TR_WAVES * mma_red<TP, NT>::WAVE * 4; }
 
 template <int TP, int NT>
 __device__ __forceinline__ void mma_reduce_store(const mma_acc<NT> acc, float *red, const mma_lane a,
                                                  int wave, int B, int m, int tok0, int row0, int slot,
                                                  float *__restrict__ part, int direct, float scale,
                                                  int accum, int64_t out_stride) {
-    constexpr int CL = 4 * TP;
-    constexpr int G = mma_red_groups<NT>();
-    constexpr int PER_WAVE = G * NT * 4 * CL;
+    using L = mma_red<TP, NT>;
 #pragma unroll
-    for (int s0 = 0; s0 < 4; s0 += G) {
+    for (int s0 = 0; s0 < 4; s0 += L::G) {
         __syncthreads();
-        if (a.live) {
-            const int cl = a.q * TP + a.tokl;
-#pragma unroll
-            for (int sg = 0; sg < G; ++sg)
-#pragma unroll
-                for (int tt = 0; tt < NT; ++tt)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r)
-                        red[wave * PER_WAVE + ((sg * NT + tt) * 4 + r) * CL + cl] = acc.v[s0 + sg][tt][r];
-        }
+        if (a.live) L::put(red + wave * L::WAVE, acc, s0, a.q * TP + a.tokl);
         __syncthreads();
-        for (int e = threadIdx.x; e < PER_WAVE; e += TR_THREADS) {
-            const int cl = e % CL;
-            int rest = e / CL;
-            const int r = rest & 3;
-            rest >>= 2;
-            const int tt = rest % NT, sg = rest / NT;
-            const int i = 4 * (cl / TP) + r;
-            const int row = row0 + 32 * (i >> 3) + (i & 7) + 8 * (s0 + sg);
-            const int tok = tok0 + 16 * tt + (cl % TP);
+        for (int e = threadIdx.x; e < L::VALUES; e += TR_THREADS) {
+            const L w(e);
+            const int row = row0 + w.row + 8 * s0, tok = tok0 + 16 * (w.token / TP) + w.token % TP;
             if (tok >= B || row >= m) continue;
-            float v = red[e];
-#pragma unroll
-            for (int w = 1; w < TR_WAVES; ++w) v += red[w * PER_WAVE + e];
+            const float v = L::sum(red, w.at);
             if (direct) {
                 float *o = part + (int64_t)tok * out_stride + row;
                 *o = accum ? (*o + scale * v) : scale * v;
@@ -637,6 +654,9 @@ struct tr_moe_group_args {
     int n_slots, x_div;
 };
 
+template <int TP, int NT>
+constexpr int moe_red_bytes() { return TR_WAVES * mma_red_groups<NT>() * NT * 4 * 4 * TP * 4; }
+
 // One pass over the K slot for NT tiles of TP of the expert's rows, positions [t0, t0 + TP NT) of its run in perm.
 // TP = 4 (NT = 1): an expert of few rows stages a quarter of the operand slots; lanes past the fourth row read a
 // zeroed block behind the chunk.
@@ -711,7 +731,9 @@ __device__ __forceinline__ void moe_group_pass(const tr_moe_group_args &g, const
             for (int tt = 0; tt < NT; ++tt) acc.v[sg][tt] += pscale * accb.v[sg][tt];
         pscale = 1.0f;
     }
-    // the four waves' sums in wave order, G row groups per round, then one row of part per (K slot, slot)
+    // the four waves' sums in wave order, G row groups per round, then one row of part per (K slot, slot).  (Tokens along
+    // the lanes on the way out as well: with the rows along them, mma_red's order, 128 slots of 128 experts 82 -> 84 us,
+    // 960 slots of 64 experts 120 -> 136.)
 #pragma unroll
     for (int s0 = 0; s0 < 4; s0 += G) {
         __syncthreads();
@@ -1295,10 +1317,10 @@ int glqh_launch_trellis_mma_moe_grouped(const void *packed, int64_t stride_bytes
     ch.ch2 = std::min(ch.ch2, s4);
     ch.ch4 = std::min(ch.ch4, s4);
     ch.ch_few = std::min(MOE_FEW_CHUNK, (s4 + 7) & ~7);
-    size_t lds = std::max((size_t)ch.ch1 * mma_slot_bytes(16, 1), (size_t)mma_red_bytes<16, 1>());
+    size_t lds = std::max((size_t)ch.ch1 * mma_slot_bytes(16, 1), (size_t)moe_red_bytes<16, 1>());
     if (wide)
         lds = std::max({lds, (size_t)ch.ch2 * mma_slot_bytes(16, 2), (size_t)ch.ch4 * mma_slot_bytes(16, 4),
-                        (size_t)mma_red_bytes<16, 4>()});
+                        (size_t)moe_red_bytes<16, 4>()});
     else
         lds = std::max({lds, (size_t)(ch.ch_few + 1) * mma_slot_bytes(4, 1), (size_t)(ch.ch_few / 2 + 1) * mma_slot_bytes(8, 1)});
     tr_moe_group_args g = {(const uint8_t *)packed, stride_bytes, (const uint8_t *)packed2, stride2_bytes, perm, offs,
