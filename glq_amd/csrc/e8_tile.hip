@@ -35,6 +35,7 @@
 // (at most 16 KB per table) sits in LDS whole, and a lookup is two 8-byte LDS reads whose result is
 // the operand: no table word comes from L2, nothing is expanded, 128 KB of table fill per workgroup
 // fall away.  The fp16 values and the stage arithmetic are the same, so the results are bit-identical.
+#include <type_traits>
 #include "e8_device.h"
 
 namespace {
@@ -587,56 +588,81 @@ e8_tile_small_kernel(const et_args a) {
 #pragma unroll
         for (int dd = 0; dd < 4; ++dd) decode(dd, abuf + dd * ET_BUF);
         et_barrier();
-        for (int q = 0; q < nquads; q += 2) {
+        // group q is multiplied out of buffer q & 1 while the next one, if there is one (MORE), is decoded into the other
+        // (LEAN: the registers are all taken, the last group as another piece of code spills some)
+        constexpr bool LEAN = NS == 4 && NTW == 2;
+        auto group = [&](auto MORE, int q, int h) {             // h = q & 1
+            const u32x4 *rd = abuf + h * 4 * ET_BUF + rg * GLQH_WAVE + lane;
+            u32x4 *wr = abuf + (h ^ 1) * 4 * ET_BUF;
+            if constexpr (decltype(MORE)::value) {
+                transpose();                                    // the next group's indices take over
+                load_quad(q + 2);
+            }
 #pragma unroll
-            for (int h = 0; h < 2; ++h) {                       // group q + h: buffers and registers h
-                if (q + h < nquads) {                           // uniform
-                    const u32x4 *rd = abuf + h * 4 * ET_BUF + rg * GLQH_WAVE + lane;
-                    u32x4 *wr = abuf + (h ^ 1) * 4 * ET_BUF;
-                    transpose();                                // the next group's indices take over
-                    load_quad(q + h + 2);
+            for (int dd = 0; dd < 4; ++dd) {
+                // operand k of the step: sub-step k / TG, fragment rg + RG (k % TG); read PF ahead
+                constexpr int NK = 2 * TG, PF = NK < 4 ? NK : 4;
+                auto frag = [&](int k) {
+                    return __builtin_bit_cast(f16x8, rd[dd * ET_BUF + ((k / TG) * ET_FRAGS + RG * (k % TG)) * GLQH_WAVE]);
+                };
+                f16x8 ring[PF];
 #pragma unroll
-                    for (int dd = 0; dd < 4; ++dd) {
-                        // operand k of the step: sub-step k / TG, fragment rg + RG (k % TG); read PF ahead
-                        constexpr int NK = 2 * TG, PF = NK < 4 ? NK : 4;
-                        auto frag = [&](int k) {
-                            return __builtin_bit_cast(f16x8, rd[dd * ET_BUF + ((k / TG) * ET_FRAGS + RG * (k % TG)) * GLQH_WAVE]);
-                        };
-                        f16x8 ring[PF];
+                for (int k = 0; k < PF; ++k) ring[k] = frag(k);
+                load_b(b[(dd + 3) & 3], ds0 + 4 * q + dd + 3);
+                if constexpr (decltype(MORE)::value) decode(dd, wr + dd * ET_BUF);
 #pragma unroll
-                        for (int k = 0; k < PF; ++k) ring[k] = frag(k);
-                        load_b(b[(dd + 3) & 3], ds0 + 4 * (q + h) + dd + 3);
-                        decode(dd, wr + dd * ET_BUF);           // operands of the next group (unused after the last)
+                for (int k = 0; k < NK; ++k) {
+                    const f16x8 af = ring[k % PF];
+                    if (k + PF < NK) ring[k % PF] = frag(k + PF);
 #pragma unroll
-                        for (int k = 0; k < NK; ++k) {
-                            const f16x8 af = ring[k % PF];
-                            if (k + PF < NK) ring[k % PF] = frag(k + PF);
-#pragma unroll
-                            for (int tt = 0; tt < NTW; ++tt)
-                                acc[k % TG][tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
-                                    af, __builtin_bit_cast(f16x8, b[dd][tt][k / TG]), acc[k % TG][tt], 0, 0, 0);
-                        }
-                    }
-                    et_barrier();                               // rd has been read, wr is written
+                    for (int tt = 0; tt < NTW; ++tt)
+                        acc[k % TG][tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                            af, __builtin_bit_cast(f16x8, b[dd][tt][k / TG]), acc[k % TG][tt], 0, 0, 0);
                 }
             }
+            et_barrier();                                       // rd has been read, wr is written
+            // (nothing moves from one group into the other: with the two of a round mixed, 14336 x 14336 at 64 tokens, two
+            // stages, 70 -> 88 us)
+            if constexpr (!LEAN) __builtin_amdgcn_sched_barrier(0);
+        };
+        if constexpr (LEAN) {
+            for (int q = 0; q < nquads; q += 2) {
+                group(std::true_type{}, q, 0);
+                if (q + 1 < nquads) group(std::true_type{}, q + 1, 1);   // uniform
+            }
+        } else {
+            int q = 0;
+            for (; q + 2 < nquads; q += 2) {
+                group(std::true_type{}, q, 0);
+                group(std::true_type{}, q + 1, 1);
+            }
+            if (q + 1 < nquads) group(std::true_type{}, q++, 0);
+            group(std::false_type{}, q, q & 1);
         }
-        // lane holds rows 4g .. 4g+3 of token i of every (fragment, token tile)
+        // lane holds rows 4g .. 4g+3 of token i of every (fragment, token tile).  The tile leaves through LDS, a token tile of
+        // every group at a time, in runs of 512 bytes and not as 16-byte pieces from the lanes.  (With that, the last group
+        // decoding nothing and the groups kept apart, whole calls, two stages: 4096 x 14336 at 20 tokens 30.7 -> 28.1 us,
+        // 4096 x 4096 at 64 / 128 21.8 -> 20.3 / 28.8 -> 27.6, 14336 x 14336 at 64 77 -> 71, 960 x 960 at 48 14.6 -> 13.4.)
+        float *ep = (float *)abuf;
         const bool vec = (a.m_pad & 3) == 0;
 #pragma unroll
         for (int tt = 0; tt < NTW; ++tt) {
-            const int tok = 16 * NTW * tg + 16 * tt + i;
-            if (tok >= a.M) continue;
-            float *orow = a.part + ((int64_t)slot * a.M + tok) * a.m_pad;
+            if (tt) et_barrier();                               // the previous tile has been read
 #pragma unroll
-            for (int j = 0; j < TG; ++j) {
-                const int row = r0 + 16 * (rg + RG * j) + 4 * g;
+            for (int j = 0; j < TG; ++j)
+                *(f32x4 *)(ep + (16 * tg + i) * ET_EP_STRIDE + 16 * (rg + RG * j) + 4 * g) = acc[j][tt];
+            et_barrier();
+            for (int c = threadIdx.x; c < 16 * TG * 32; c += ET_THREADS) {
+                const int tl = c >> 5, tok = 16 * NTW * (tl >> 4) + 16 * tt + (tl & 15), rl = 4 * (c & 31), row = r0 + rl;
+                if (tok >= a.M) continue;
+                float *orow = a.part + ((int64_t)slot * a.M + tok) * a.m_pad;
+                const f32x4 v = *(const f32x4 *)(ep + tl * ET_EP_STRIDE + rl);
                 if (vec && row + 3 < a.m_pad) {
-                    *(f32x4 *)(orow + row) = acc[j][tt];
+                    *(f32x4 *)(orow + row) = v;
                 } else {
 #pragma unroll
                     for (int e = 0; e < 4; ++e)
-                        if (row + e < a.m_pad) orow[row + e] = acc[j][tt][e];
+                        if (row + e < a.m_pad) orow[row + e] = v[e];
                 }
             }
         }

@@ -667,8 +667,8 @@ __device__ __forceinline__ void tr_tile_small_body(const tt_args &a, const tt_gr
         for (int dd = 0; dd < 4; ++dd) emit(rc[dd], rcb[dd], abuf + dd * TT_BUF);
         tt_barrier();
         // group qd: multiplied out of buffer qd & 1 while the next group is decoded into the other one, from e / eb
-        // (the branches also keep decode and products of a step apart, which two waves per SIMD overlap better than the
-        // compiler does within one: without them where both groups are whole, 14336 x 4096 at 64 tokens 45.7 -> 54.0 us)
+        // (the branches also keep the steps apart: without them where both groups are whole the compiler mixes one group
+        // into the next, 14336 x 4096 at 64 tokens 45.7 -> 54.0 us; with a scheduling barrier there it is level)
         auto group = [&](int qd, tr_record<R> (&e)[4], tr_record<RB> (&eb)[4]) {
             const int d0 = ds0 + 4 * qd;
             const u32x4 *rd = abuf + (qd & 1) * 4 * TT_BUF + rg * GLQH_WAVE + lane;

@@ -173,6 +173,14 @@ def test_many_token_products_on_folded_streams_equal_products_on_indices(ext, m,
         assert rel(y_fold, x.float().cpu().numpy() @ W.T) < TOL
 
 
+@pytest.mark.parametrize("m,n,B", [(16516, 256, 33), (16518, 512, 64), (16516, 768, 20), (16516, 1024, 200), (16517, 1280, 100)])
+@pytest.mark.parametrize("stages", [1, 2, 3, 4])
+def test_groups_of_four_steps_on_folded_streams(ext, m, n, B, stages):
+    """One to five groups of four steps in the one K slot of a layer with more row tiles than half the CUs; rows that end
+    inside a fragment, whole runs of four and not."""
+    test_many_token_products_on_folded_streams_equal_products_on_indices(ext, m, n, B, stages)
+
+
 def test_fused_linear_on_folded_streams_and_under_capture(ext):
     """The forward path only looks the folded streams up.  A layer that was never prepared runs on its
     indices -- also under capture, with a warning -- and makes nothing; after `e8_prepare` a captured
