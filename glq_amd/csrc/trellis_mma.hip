@@ -123,8 +123,15 @@ struct mma_red {
     static constexpr int VALUES = 16 * G * NT * TP;              // of a pass
     int row, token, at;                                          // row of the pass's strip (s0 = 0), token, place
     __device__ __forceinline__ explicit mma_red(int e) {
-        const int rl = e % (16 * G), sg = (rl >> 3) % G, i = 8 * (rl / (8 * G)) + (rl & 7);
+        int rl = e % (16 * G), sg = (rl >> 3) % G, i = 8 * (rl / (8 * G)) + (rl & 7);
         token = e / (16 * G);
+        if constexpr (TP == 1 && NT == 1) {                      // one token: 64 rows in the order of their places
+            at = e;
+            sg = e >> 4;
+            i = 4 * (e & 3) + ((e >> 2) & 3);
+            row = 32 * (i >> 3) + (i & 7) + 8 * sg;
+            return;
+        }
         row = 32 * (i >> 3) + (i & 7) + 8 * sg;
         at = sg * SS + (4 * (token / TP) + (i & 3)) * RS + (i >> 2) * TP + token % TP;
     }
