@@ -341,7 +341,9 @@ viterbi_kernel(const float *__restrict__ tiles_in, int64_t n_tiles, int64_t ld, 
 // (values stay small, where fp16 is fine; a difference of two fp16 numbers that is >= 0 rounds down too).  The pass runs
 // one step past the last input, so that L = min l_T + B_T bounds the whole search.
 // Backtrack (vb_backtrack, a wave a tile).  From the end, keep every way whose bound (its cost to the end + l + B)
-// is at most L (1 + SLACK): what the fp16 roundings lose is 0.3-0.5 % of the cost, so a level keeps 1.4 ways on average.
+// is at most L (1 + SLACK) + VB_LOST: what the fp16 roundings lose is 0.3-0.5 % of the cost, so a level keeps 1.4 ways on
+// average.  (Below 2^-14 they lose up to 2^-24 a step whatever the cost: on values that are decoded ones again, or a rounding
+// off them, L is 0 where the best path costs 10^-9.)
 // At the start the cheapest kept path costs U.  If U (1 + 2^-14) is within the limit, no path that was dropped can cost U
 // or less, also after the roundings of 256 fp32 additions (2^-24 each), and the kept ones contain the search's answer and
 // all its ties; else the backtrack runs again with that limit.  Where another kept path is within 2^-14 of the cheapest
@@ -353,6 +355,7 @@ constexpr int VB_THREADS = 512;
 constexpr int VB_NORM = 2;                 // steps between two moves of the row's minimum into B
 constexpr float VB_X = 16.0f;              // largest input: (16 + 4)^2 for 16 / K steps stays far below 65504
 constexpr int VB_MOST = 64;                // kept groups of a step: a lane each
+constexpr float VB_LOST = VT_T * 0x1p-24f; // what fp16 roundings of the smallest numbers take off a bound, at most
 
 template <int K>
 struct vb_cfg {
@@ -687,14 +690,14 @@ __device__ __forceinline__ void vb_walk(int g, int p, int (&st)[vb_cfg<K>::DEPTH
     }
 }
 
-// The backtrack of one tile by one wave: 0 and the states in `states`; the limit to try next; infinity where the tile
-// has to be searched exactly.
+// The backtrack of one tile by one wave: true, and the states in `states`; or false, and `limit` the one to try next,
+// infinity where the tile has to be searched exactly.
 // n, gv: the groups of step T (a lane each) whose bounds are within `limit`; x[i]: input of step i; the bounds' row of
 // level l at hist + (l - 1) * G; pre[j]: B at step j * VB_NORM; tie: the only group of step 0, or -1; the states up to
 // step `upto` are wanted.
 template <int K>
-__device__ __forceinline__ float vb_trace(int n, int gv, float limit, const float *x, const uint16_t *__restrict__ hist,
-                                          const float *pre, int tie, int upto, vb_pool *P, int *states) {
+__device__ __forceinline__ bool vb_trace(int n, int gv, float &limit, const float *x, const uint16_t *__restrict__ hist,
+                                         const float *pre, int tie, int upto, vb_pool *P, int *states) {
     using C = vb_cfg<K>;
     constexpr int D = C::DEPTH, LEVELS = C::STORED, R = (1 << (K * D)) / 64;
     const int lane = threadIdx.x & 63;
@@ -837,8 +840,10 @@ __device__ __forceinline__ float vb_trace(int n, int gv, float limit, const floa
         gv = ng & (C::G - 1);
         cv = nc;
     }
-    if (full) return inf;
-    if (empty) return limit * (1.0f + 0.5f * C::SLACK);
+    if (full || empty) {
+        limit = full ? inf : limit * (1.0f + 0.5f * C::SLACK);
+        return false;
+    }
     if (lane == 0) P->at[0] = (uint16_t)ne;
     float u = inf, second = inf;
     int take = 0;
@@ -849,7 +854,10 @@ __device__ __forceinline__ float vb_trace(int n, int gv, float limit, const floa
         second = __builtin_fminf(second, __builtin_fmaxf(u, cq));
         u = __builtin_fminf(u, cq);
     }
-    if (!(u * (1.0f + 0x1p-14f) <= limit)) return vb_lane(u * (1.0f + 0x1p-13f), 0);
+    if (!(u * (1.0f + 0x1p-14f) <= limit)) {
+        limit = vb_lane(u * (1.0f + 0x1p-13f), 0);
+        return false;
+    }
     // the cheapest path, from the start; where no other one is close to it, it is the answer
     bool near = second - u <= close;
     __builtin_amdgcn_wave_barrier();
@@ -871,7 +879,7 @@ __device__ __forceinline__ float vb_trace(int n, int gv, float limit, const floa
             for (int e = 0; e < D; ++e) states[(l0 + lane + 1) * D - 1 - e] = st[e];
         }
     }
-    if (!near) return 0.0f;
+    if (!near) return true;
 
     // exact costs, forward over the kept ways that a path close to the cheapest may take; lane e: entry e of the level,
     // best, cheap: exact cost from the start, cost to the end, of group `lane` of the level below
@@ -880,7 +888,10 @@ __device__ __forceinline__ float vb_trace(int n, int gv, float limit, const floa
 #pragma unroll 1
     for (int l = 1; l <= LEVELS; ++l) {
         const int eb = P->at[l], m = __builtin_amdgcn_readfirstlane((int)P->at[l - 1] - eb), nb = P->at[l < LEVELS ? l + 1 : l];
-        if (m > 64) return inf;
+        if (m > 64) {
+            limit = inf;
+            return false;
+        }
         const int e = eb + (lane < m ? lane : 0), en = P->entry[e], parent = en >> 8, child = P->child[e];
         int st[D];
         vb_walk<K>(P->group[P->groups[l] + parent], en & 255, st);
@@ -937,7 +948,7 @@ __device__ __forceinline__ float vb_trace(int n, int gv, float limit, const floa
         }
         if (l > 1) take = __builtin_amdgcn_readfirstlane(P->via[P->at[l] + P->child[at]]);
     }
-    return 0.0f;
+    return true;
 }
 
 // A wave's memory while it walks back
@@ -960,7 +971,7 @@ __device__ __forceinline__ void vb_backtrack(const float *__restrict__ tiles_in,
     const int64_t tile = part.first + at;
     vb_tile *const mine = part.info + at;
     const int over = __builtin_amdgcn_readfirstlane(mine->over);
-    if (over < 0) {
+    if ((uint32_t)over >= (uint32_t)C::G) {
         if (pass && lane == 0) states_out[tile * VT_T] = -1;
         return;
     }
@@ -981,7 +992,7 @@ __device__ __forceinline__ void vb_backtrack(const float *__restrict__ tiles_in,
         }
         lo = vb_wave_min(lo);
     }
-    float limit = vb_lane((vb_half(lo) + bt) * (1.0f + C::SLACK), 0);
+    float limit = vb_lane((vb_half(lo) + bt) * (1.0f + C::SLACK) + VB_LOST, 0);
     bool good = false;
 #pragma unroll 1
     for (int tries = 0; tries < 4; ++tries) {
@@ -1010,8 +1021,7 @@ __device__ __forceinline__ void vb_backtrack(const float *__restrict__ tiles_in,
         __builtin_amdgcn_wave_barrier();
         if (n > VB_MOST) break;
         n = __builtin_amdgcn_readfirstlane(n);
-        limit = vb_trace<K>(n, lane < n ? start[lane] : 0, limit, x, hist, pre, tie, pass ? VT_T - 1 : VT_T / 2, &W->pool, states);
-        good = limit == 0.0f;
+        good = vb_trace<K>(n, lane < n ? start[lane] : 0, limit, x, hist, pre, tie, pass ? VT_T - 1 : VT_T / 2, &W->pool, states);
         if (good || limit == __builtin_inff()) break;
         __builtin_amdgcn_wave_barrier();
     }

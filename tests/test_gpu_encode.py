@@ -288,6 +288,63 @@ def test_viterbi_on_bounds_equals_the_exact_search(K, n):
         assert np.array_equal(got[finite], ref[finite])
 
 
+def _exact_states(X, K, chunk=256):
+    """The search of the oracle's `trellis_quantize_tiles` step by step on cost rows in memory: the single-step kernel (held
+    to the reference's step in test_gpu_named_surface.py), lowest states on ties, and the walk back here."""
+    from glq_amd import ext
+    lut = t(O.lut_3inst())
+    lutf, G = lut.float(), 1 << (16 - K)
+    state = torch.arange(65536, device=DEV)
+
+    def search(x, over=None):                            # x (b, 256) fp16 -> states (b, 256)
+        cost = (lutf - x[:, :1].float()) ** 2
+        if over is not None:
+            cost = torch.where(state >> K == over[:, None], cost, torch.inf)
+        prev = torch.empty(256, x.shape[0], G, dtype=torch.int32, device=DEV)
+        for i in range(1, 256):
+            cost = ext.viterbi_acs_step(cost, x[:, i].contiguous(), lutf, K, prev[i])
+        if over is not None:
+            cost = torch.where(state & (G - 1) == over[:, None], cost, torch.inf)
+        at = torch.where(cost == cost.min(1, keepdim=True).values, state, 65536).min(1).values
+        states = torch.empty(x.shape, dtype=torch.int64, device=DEV)
+        for i in range(255, -1, -1):
+            states[:, i] = at
+            if i:
+                at = prev[i].gather(1, (at >> K)[:, None])[:, 0].long()
+        return states
+
+    out = []
+    for x in X.to(DEV).half().split(chunk):
+        out.append(search(x, search(x.roll(128, 1))[:, 128] >> K))
+    return torch.cat(out).int()
+
+
+@pytest.mark.parametrize("K", [2, 3, 4])
+@pytest.mark.parametrize("kind", ["decoded", "one value a rounding off", "noise of 1e-5", "noise of 2e-7"])
+def test_viterbi_of_decoded_weights(K, kind):
+    """Tiles that are decoded tail-biting paths, or nearly: their best path costs nothing or so little that all its bounds in
+    fp16 are zero."""
+    from glq_amd import ext
+    say("viterbi of decoded weights", K, kind)
+    n = 300                                              # more than a tile per CU: on bounds at every K
+    lut = torch.from_numpy(O.lut_3inst().astype(np.float16))
+    X = lut[torch.from_numpy(O.trellis_states(O.random_packed(160, 480, K, seed=K), 160, 480).astype(np.int64))].reshape(n, 256).float()
+    g = torch.Generator().manual_seed(K)
+    if kind == "one value a rounding off":
+        at = X.abs().argsort(1)[torch.arange(n), torch.randint(0, 64, (n,), generator=g)]   # one of the smaller values
+        v = X[torch.arange(n), at].half()
+        X[torch.arange(n), at] = torch.nextafter(v, torch.full_like(v, 8.0)).float()
+    elif kind.startswith("noise"):
+        X = X + torch.randn(n, 256, generator=g) * float(kind.split()[-1])
+    hat, st = ext.trellis_quantize_tiles(X.to(DEV), K)
+    ref = _exact_states(X, K)
+    assert torch.equal(st, ref), (st != ref).any(1).nonzero()[:5]
+    assert torch.equal(hat.cpu(), lut[ref.long().cpu()].float())
+    assert np.array_equal(st[:3].cpu().numpy(), O.trellis_quantize_tiles(X[:3].numpy(), K)[1])
+    if kind == "decoded":
+        assert torch.equal(hat.cpu(), X)
+
+
 def test_viterbi_under_capture():
     """Captured and replayed on other tiles: the launches' batches hand each other their rows through the same memory."""
     from glq_amd import ext
