@@ -1601,7 +1601,8 @@ extern "C" int glqh_fused_moe_trellis_3inst(const void *x, int x_dtype, int64_t 
     const bool mid = grouped && n_slots >= MOE_FUSE_MIN_SLOTS && moe_fuse_enabled() &&
                      glqh_moe_mid_eligible(w13->m_pad, w13->blocks_m, w13->n_blocks_m, w2->n_pad, w2->blocks_n,
                                            w2->n_blocks_n);
-    const bool few = n_slots < MOE_MID_FEW_SLOTS && moe_fuse_enabled() &&
+    // (input signs at any address, as the separate launches take them: the one launch reads them in runs of eight)
+    const bool few = n_slots < MOE_MID_FEW_SLOTS && moe_fuse_enabled() && (!grouped || ((uintptr_t)w2->sv_f16 & 15) == 0) &&
                      glqh_moe_mid_few_eligible(w13->m_pad, w13->blocks_m, w13->n_blocks_m, grouped ? w2->n_pad : 0,
                                                w2->blocks_n, w2->n_blocks_n);
     const void *x2 = hact;

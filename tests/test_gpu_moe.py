@@ -318,6 +318,24 @@ def test_launches_between_the_projections(ext, hidden, inter, T, K, act, dtype):
     assert torch.equal(y, ext.glq_fused_moe_trellis_3inst_cuda(x.to(DEV), t(ids), t(w), *a))
 
 
+@pytest.mark.parametrize("T", [2, 30])                # per slot and grouped
+def test_input_signs_at_any_address(ext, T):
+    """Input signs of both projections that are slices of a buffer, not 16-byte aligned."""
+    say("moe unaligned signs", T)
+    ex = experts(3, 256, 192, seed=4)
+    ids, w = routing(T, 2, 3, T)
+    x = torch.from_numpy(np.random.default_rng(T).standard_normal((T, 256)).astype(np.float32)).bfloat16()
+    a = list(ex.device_args(0))
+    for j in (3, 9):                                     # w13_SV, w2_SV
+        buf = torch.zeros(a[j].numel() + 1, dtype=a[j].dtype, device=DEV)
+        buf[1:] = a[j]
+        a[j] = buf[1:]
+        assert a[j].data_ptr() % 16
+    y = ext.glq_fused_moe_trellis_3inst_cuda(x.to(DEV), t(ids), t(w), *a)
+    ref = ex.oracle(x.float().numpy(), ids, w, 0)
+    assert rel(y, ref) < TOL, rel(y, ref)
+
+
 def test_large_activations_stay_finite_in_the_tile_form(ext):
     """Squared-ReLU experts on activations of a few units: the second projection's unscaled sums pass the fp16
     range while the result does not; the tile form's fp16 sums carry the expert's scale, so it stays finite and
