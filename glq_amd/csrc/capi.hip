@@ -1365,8 +1365,8 @@ static bool moe_tile_form(int64_t n_slots, int64_t n_experts, bool grouped) {
     return mn > 0 && grouped && n_slots >= mn * live;
 }
 
-// GLQ_MOE_FUSE=0 (read once): the launches between and after the decode launches stay separate at every slot count
-// (output transform, activation, input transform, repack; output transform, weighted sum).
+// GLQ_MOE_FUSE=0 (read once): the launches before, between and after the decode launches stay separate at every slot count
+// (routing table, input transform; output transform, activation, input transform, repack; output transform, weighted sum).
 static bool moe_fuse_enabled() {
     static const bool on = [] {
         const char *e = getenv("GLQ_MOE_FUSE");
@@ -1578,7 +1578,7 @@ extern "C" int glqh_fused_moe_trellis_3inst(const void *x, int x_dtype, int64_t 
     int *pexp = (int *)(base + l.pexp);
     // the routing table and, where that is one launch, the rows' input transform in it
     int rows_in = -1;
-    if (grouped)
+    if (grouped && moe_fuse_enabled())
         rows_in = glqh_launch_moe_route_input(topk_ids, n_slots, (int)num_experts, perm, pexp, offs, x, x_dtype, x_stride,
                                               w13->sv_f16, xhat, num_tokens, w13->in_features, w13->n_pad, w13->blocks_n,
                                               w13->n_blocks_n, st);

@@ -385,6 +385,40 @@ def test_both_forms_on_every_case_in_a_fresh_process(group_min, wide_min, tile_m
     assert r.returncode == 0, (r.stdout[-3000:], r.stderr[-1000:])
 
 
+_COUNT_LAUNCHES = """
+import ctypes, sys, numpy as np, torch
+sys.path.insert(0, "tests")
+import test_gpu_moe as M
+from glq_amd import _lib, ext
+T = 30
+ids, w = M.routing(T, 2, 3, T)
+args = (torch.randn(T, 256, device=M.DEV).bfloat16(), M.t(ids), M.t(w), *M.experts(3, 256, 192, seed=4).device_args(0))
+ext.glq_fused_moe_trellis_3inst_cuda(*args)
+graph = torch.cuda.CUDAGraph(keep_graph=True)
+with torch.cuda.graph(graph):
+    ext.glq_fused_moe_trellis_3inst_cuda(*args)
+n = ctypes.c_size_t()
+assert _lib.load().hipGraphGetNodes(ctypes.c_void_p(graph.raw_cuda_graph()), None, ctypes.byref(n)) == 0
+print("launches", n.value)
+"""
+
+
+@pytest.mark.parametrize("fuse,launches", [
+    ("1", 6),                                          # table + rows, decode, between, decode, output transform, sum
+    ("0", 9)])                                         # the first two and the three between as launches of their own
+def test_launches_of_a_call_in_a_fresh_process(fuse, launches):
+    """GLQ_MOE_FUSE=0 keeps every launch around the two decode launches separate, the routing table's and the input
+    transform's among them: launches of a captured call of 60 slots."""
+    import os
+    import subprocess
+    import sys
+    say("moe launches, child process", fuse)
+    r = subprocess.run([sys.executable, "-u", "-c", _COUNT_LAUNCHES], env={**os.environ, "GLQ_MOE_FUSE": fuse},
+                       capture_output=True, text=True, timeout=300,
+                       cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
+    assert r.returncode == 0 and f"launches {launches}\n" in r.stdout, (r.stdout[-2000:], r.stderr[-2000:])
+
+
 @pytest.mark.parametrize("T", [1, 4, 40, 140])
 def test_qwen3_moe_expert_shapes(ext, T):
     """Expert shapes of a Qwen3-MoE layer (hidden 2048, intermediate 768, top-8), 16 of the experts,
