@@ -344,10 +344,12 @@ viterbi_kernel(const float *__restrict__ tiles_in, int64_t n_tiles, int64_t ld, 
 // is at most L (1 + SLACK) + VB_LOST: what the fp16 roundings lose is 0.3-0.5 % of the cost, so a level keeps 1.4 ways on
 // average.  (Below 2^-14 they lose up to 2^-24 a step whatever the cost: on values that are decoded ones again, or a rounding
 // off them, L is 0 where the best path costs 10^-9.)
-// At the start the cheapest kept path costs U.  If U (1 + 2^-14) is within the limit, no path that was dropped can cost U
-// or less, also after the roundings of 256 fp32 additions (2^-24 each), and the kept ones contain the search's answer and
-// all its ties; else the backtrack runs again with that limit.  Where another kept path is within 2^-14 of the cheapest
-// (3 % of the tiles), fp32 costs are evaluated forward over the kept ways, minima and lowest states as in viterbi_kernel.
+// At the start the cheapest kept path costs U.  If U (1 + VB_NEAR) is within the limit, no path that was dropped can be the
+// search's answer, and the kept ones contain that and all its ties; else the backtrack runs again with that limit.  (Four
+// fp32 sums stand between the two, each off by at most e = (256 + 8) 2^-24 of itself: U, the bound of what was dropped,
+// and viterbi_kernel's costs of both paths, from which it takes the cheaper; 4 e < VB_NEAR.)  Where another kept path is
+// within VB_NEAR of the cheapest (3 % of the tiles), fp32 costs are evaluated forward over the kept ways, minima and lowest
+// states as in viterbi_kernel.
 // Tiles that fail (inputs above VB_X, not finite or all equal, more kept ways than fit) are marked by state -1 and
 // left to viterbi_kernel, which skips all others.  2048 x 2048 weights in viterbi_kernel alone -> so: 69.7 -> 31.9 ms at
 // K = 4, 59.0 -> 38.1 at 3, 66.5 -> 36.4 at 2.
@@ -355,6 +357,8 @@ constexpr int VB_THREADS = 512;
 constexpr int VB_NORM = 2;                 // steps between two moves of the row's minimum into B
 constexpr float VB_X = 16.0f;              // largest input: (16 + 4)^2 for 16 / K steps stays far below 65504
 constexpr int VB_MOST = 64;                // kept groups of a step: a lane each
+constexpr float VB_NEAR = 1100 * 0x1p-24f; // paths this close, relative to the limit, are compared in viterbi_kernel's sums
+static_assert(4 * (VT_T + 8) * 0x1p-24f < VB_NEAR, "four sums of 256 rounded squares");
 constexpr float VB_LOST = VT_T * 0x1p-24f; // what fp16 roundings of the smallest numbers take off a bound, at most
 
 template <int K>
@@ -701,7 +705,7 @@ __device__ __forceinline__ bool vb_trace(int n, int gv, float &limit, const floa
     using C = vb_cfg<K>;
     constexpr int D = C::DEPTH, LEVELS = C::STORED, R = (1 << (K * D)) / 64;
     const int lane = threadIdx.x & 63;
-    const float close = limit * 0x1p-14f, inf = __builtin_inff();
+    const float close = limit * VB_NEAR, inf = __builtin_inff();
     float cv = 0.0f;                                           // lane j: cost from group gv of this level to the end
     int ne = 0, ns = 0;
     bool full = false, empty = false;
@@ -854,8 +858,8 @@ __device__ __forceinline__ bool vb_trace(int n, int gv, float &limit, const floa
         second = __builtin_fminf(second, __builtin_fmaxf(u, cq));
         u = __builtin_fminf(u, cq);
     }
-    if (!(u * (1.0f + 0x1p-14f) <= limit)) {
-        limit = vb_lane(u * (1.0f + 0x1p-13f), 0);
+    if (!(u * (1.0f + VB_NEAR) <= limit)) {
+        limit = vb_lane(u * (1.0f + 2 * VB_NEAR), 0);
         return false;
     }
     // the cheapest path, from the start; where no other one is close to it, it is the answer
