@@ -29,6 +29,8 @@
 
 #pragma clang fp contract(off)
 
+size_t glqh_viterbi_scratch_bytes(int K, int64_t n_tiles);
+
 namespace {
 
 constexpr int VT_T = 256;
@@ -277,12 +279,19 @@ __device__ __forceinline__ int64_t vt_pos(int64_t tile, int t, int64_t ld) {
     return ld ? (tile / per_row) * 16 * ld + (tile % per_row) * 16 + vt_step_pos(t, ld) : tile * VT_T + t;
 }
 
-// Persistent workgroups walk the tiles with a fixed stride, each owning one slab of cost rows.  marked: only tiles whose
-// first state is -1.
+// Which tiles of a call are searched how: those for the search on bounds, from order[0] on, those that it does not try, from
+// order[n_tiles - 1] back, and those that it tried and left.
+struct vb_lists {
+    int *counts;                           // how many it tries, how many it left; null: no such search
+    int *order, *left;
+};
+
+// Persistent workgroups walk the tiles (lists: those that are not found on bounds) with a fixed stride, each owning one
+// slab of cost rows.
 template <int K>
 __global__ void __launch_bounds__(vt_cfg<K>::THREADS, 4)
 viterbi_kernel(const float *__restrict__ tiles_in, int64_t n_tiles, int64_t ld, float *__restrict__ scratch,
-               int32_t *states_out, float *__restrict__ hat_out, int marked) {
+               int32_t *__restrict__ states_out, float *__restrict__ hat_out, vb_lists lists) {
     using C = vt_cfg<K>;
     constexpr int G = C::G;
     extern __shared__ float best[];                            // ROWS * G floats
@@ -291,11 +300,8 @@ viterbi_kernel(const float *__restrict__ tiles_in, int64_t n_tiles, int64_t ld, 
     __shared__ vt_best red[C::THREADS / 64];
     const int tid = threadIdx.x;
     float *hist = scratch + (int64_t)blockIdx.x * (VT_T / C::DEPTH) * G;
-    if (marked) {
-        bool any = false;
-        for (int64_t tile = blockIdx.x; tile < n_tiles; tile += gridDim.x) any = any || states_out[tile * VT_T] < 0;
-        if (!any) return;
-    }
+    const int64_t untried = lists.counts ? n_tiles - lists.counts[0] : 0, todo = lists.counts ? untried + lists.counts[1] : n_tiles;
+    if ((int64_t)blockIdx.x >= todo) return;
     f16x2 w[32768 / C::THREADS];
 #pragma unroll
     for (int k = 0; k < C::NK; ++k)
@@ -308,8 +314,9 @@ viterbi_kernel(const float *__restrict__ tiles_in, int64_t n_tiles, int64_t ld, 
                 asm volatile("" : "+v"(v));                    // finished here: neither spilled half-done nor recomputed
                 w[(k * C::UNITS + q) * (C::LOWS / 2) + j / 2] = v;
             }
-    for (int64_t tile = blockIdx.x; tile < n_tiles; tile += gridDim.x) {
-        if (marked && states_out[tile * VT_T] >= 0) continue;
+    for (int64_t item = blockIdx.x; item < todo; item += gridDim.x) {
+        int64_t tile = item;
+        if (lists.counts) tile = item < untried ? lists.order[n_tiles - 1 - item] : lists.left[item - untried];
         const int64_t pos = vt_pos(tile, tid & 255, ld);
         if (tid < VT_T) {
             const float v = (float)(f16)tiles_in[pos];
@@ -350,12 +357,23 @@ viterbi_kernel(const float *__restrict__ tiles_in, int64_t n_tiles, int64_t ld, 
 // and viterbi_kernel's costs of both paths, from which it takes the cheaper; 4 e < VB_NEAR.)  Where another kept path is
 // within VB_NEAR of the cheapest (3 % of the tiles), fp32 costs are evaluated forward over the kept ways, minima and lowest
 // states as in viterbi_kernel.
-// Tiles that fail (inputs above VB_X, not finite or all equal, more kept ways than fit) are marked by state -1 and
-// left to viterbi_kernel, which skips all others.  2048 x 2048 weights in viterbi_kernel alone -> so: 69.7 -> 31.9 ms at
+// Tiles with inputs above VB_X, not finite or all equal are not tried, and those with more kept ways than fit are left: lists
+// of both go to viterbi_kernel (with marks instead of lists, every workgroup walking its share of all tiles, it took the
+// time of all of them where half were marked).  Far beyond the weights' range the cost is mostly what no path can avoid,
+// and SLACK of that lets everything through: tiles with more than WIDE of it are not tried either (K = 4: 5 % of those with
+// 2-3 are left, 23 % with 4-5, 64 % with 10-14; K = 3 and 2: 17 and 18 % of the first beyond), nor is a minority of up to two
+// chips full, nor the rest of a call after batches of which more than half were left.  4096 tiles, exact / so, ms:
+//   normal values of sigma      1e-4         0.9          1.6          1.8          2.2          3 and more
+//     K = 4                     17.5 / 17.7  17.5 / 8.2   17.5 / 11.1  17.4 / 15.8  17.4 / 17.6  17.5 / 17.6
+//     K = 3                     14.9 / 10.3  14.7 / 9.6   14.6 / 10.9  14.6 / 11.0  14.6 / 14.8  14.6 / 14.7
+//     K = 2                     16.7 / 8.1   16.7 / 9.6   16.7 / 10.4  16.8 / 10.8  16.7 / 12.2  16.7 / 16.7
+// Slower is what fills the lists and shows nothing beforehand, as slow ramps do (-3 to 3 over the tile's steps): 17.5 / 19.2,
+// 14.6 / 16.2, 16.7 / 18.7, up to 1.4 times in calls of one or two batches.  2048 x 2048 weights in viterbi_kernel alone -> so: 69.7 -> 31.9 ms at
 // K = 4, 59.0 -> 38.1 at 3, 66.5 -> 36.4 at 2.
 constexpr int VB_THREADS = 512;
 constexpr int VB_NORM = 2;                 // steps between two moves of the row's minimum into B
 constexpr float VB_X = 16.0f;              // largest input: (16 + 4)^2 for 16 / K steps stays far below 65504
+constexpr float VB_W = 4.0f;               // the weights' range: 3.97
 constexpr int VB_MOST = 64;                // kept groups of a step: a lane each
 constexpr float VB_NEAR = 1100 * 0x1p-24f; // paths this close, relative to the limit, are compared in viterbi_kernel's sums
 static_assert(4 * (VT_T + 8) * 0x1p-24f < VB_NEAR, "four sums of 256 rounded squares");
@@ -370,6 +388,7 @@ struct vb_cfg {
     static constexpr float SLACK = K == 4 ? 0.0042f : K == 3 ? 0.0049f : 0.0058f;
     static constexpr int ROW = K == 4 ? 32 * 72 : K == 3 ? 128 * 36 : 4096 * 2 + 256 * 2;   // words of a row, with its padding
     static constexpr int ROWS = K == 2 ? 1 : 2;                // cost rows in LDS per tile; one: read by all, then written
+    static constexpr float WIDE = 4.0f * (1 << (2 * (4 - K)));   // of a tile that is tried: cost beyond the weights' range
     static constexpr int FEW = K == 2 ? 2 : 1;                 // tiles a workgroup in calls that do not fill the chip
 };
 
@@ -439,7 +458,7 @@ struct vb_tile {
     int over;                              // the tail-biting overlap, -1: left to viterbi_kernel
 };
 
-// Tiles first .. first + count - 1 and one of their two passes: 0 on the inputs rolled by T/2, unconstrained; 1 from and
+// Tiles order[first .. first + count - 1], as far as that many are tried, and one of their two passes: 0 on the inputs rolled by T/2, unconstrained; 1 from and
 // to the overlap that the first backtrack found.  rows: STORED rows of G halves per tile.
 struct vb_part {
     int64_t first;
@@ -447,6 +466,67 @@ struct vb_part {
     uint16_t *rows;
     vb_tile *info;
 };
+__device__ __forceinline__ int vb_count(const vb_part &part, const vb_lists &lists) {
+    const int64_t left = __builtin_amdgcn_readfirstlane(lists.counts[0]) - part.first;
+    return left < part.count ? (left < 0 ? 0 : (int)left) : part.count;
+}
+
+// The lists, in two launches (10 us together, where the smallest call takes 730): a wave a tile notes in `left` whether it is tried, and one workgroup deals the tiles out.
+__global__ void __launch_bounds__(256)
+vb_try_kernel(const float *__restrict__ tiles_in, int64_t n_tiles, int64_t ld, float most, vb_lists lists) {
+    const int64_t tile = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63;
+    if (tile >= n_tiles) return;
+    float v[VT_T / 64];
+#pragma unroll
+    for (int j = 0; j < VT_T / 64; ++j) v[j] = (float)(f16)tiles_in[vt_pos(tile, 64 * j + lane, ld)];
+    bool within = true, varied = false;                        // equal inputs leave every other path a tie
+    float wide = 0.0f;
+    const float first = __shfl(v[0], 0, GLQH_WAVE);
+#pragma unroll
+    for (int j = 0; j < VT_T / 64; ++j) {
+        within = within && __builtin_fabsf(v[j]) <= VB_X;
+        varied = varied || v[j] != first;
+        const float past = __builtin_fmaxf(__builtin_fabsf(v[j]) - VB_W, 0.0f);
+        wide += past * past;
+    }
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) wide += __shfl_xor(wide, d, GLQH_WAVE);
+    within = __ballot(!within) == 0 && __ballot(varied) != 0 && wide <= most;
+    if (lane == 0) lists.left[tile] = within;
+}
+
+__global__ void __launch_bounds__(1024)
+vb_order_kernel(int n_tiles, int few, vb_lists lists) {
+    __shared__ int of_wave[16];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    int tried = 0;
+    int next = tid < n_tiles ? lists.left[tid] : 0;
+    for (int base = 0; base < n_tiles; base += 1024) {
+        const int i = base + tid, mine = next;
+        next = i + 1024 < n_tiles ? lists.left[i + 1024] : 0;
+        const uint64_t mask = __ballot(mine);
+        if (lane == 0) of_wave[wave] = __builtin_popcountll(mask);
+        __syncthreads();
+        int at = tried + vb_below(mask);
+#pragma unroll
+        for (int w = 0; w < 16; ++w) {
+            at += w < wave ? of_wave[w] : 0;
+            tried += of_wave[w];
+        }
+        if (i < n_tiles) lists.order[mine ? at : n_tiles - 1 - (i - at)] = i;   // i - at: tiles before it that are not tried
+        __syncthreads();
+    }
+    if (tid == 0) {
+        lists.counts[0] = tried <= few && tried < n_tiles - tried ? 0 : tried;
+        lists.counts[1] = 0;
+    }
+}
+
+// Before the batch that begins at `first`: where more than half of those before it were left, it and the rest are not tried.
+__global__ void vb_stop_kernel(int64_t first, vb_lists lists) {
+    if (threadIdx.x == 0 && 2 * (int64_t)lists.counts[1] > first && lists.counts[0] > first) lists.counts[0] = (int)first;
+}
 
 // One forward pass, the rows of every DEPTH-th step to part.rows.  TPW tiles a workgroup: their steps share the table and
 // the barriers; workgroups walk the tiles with a fixed stride.
@@ -455,12 +535,12 @@ struct vb_part {
 // clocks a state, where subtract, multiply, add and half a minimum in fp32 take 14.4 (fma_mix 4.3, the others 2.5); the
 // pass over 1024 tiles at K = 4 takes 0.93 ms, of which such loops would be 0.65.
 template <int K, int TPW>
-__device__ __forceinline__ void vb_forward(const float *__restrict__ tiles_in, int64_t ld, const vb_part &part, int worker,
-                                           int workers, uint32_t *lds) {
+__device__ __forceinline__ void vb_forward(const float *__restrict__ tiles_in, int64_t ld, const vb_lists &lists,
+                                           const vb_part &part, int worker, int workers, uint32_t *lds) {
     using C = vb_cfg<K>;
     constexpr int THREADS = VB_THREADS;
     const int64_t first = part.first;
-    const int count = part.count, pass = part.pass;
+    const int count = vb_count(part, lists), pass = part.pass;
     uint16_t *const __restrict__ rows = part.rows;
     vb_tile *const __restrict__ info = part.info;
     constexpr int G = C::G, NK = C::NK, CW = C::CW, D = C::DEPTH, ROWS = C::ROWS;
@@ -470,7 +550,7 @@ __device__ __forceinline__ void vb_forward(const float *__restrict__ tiles_in, i
     constexpr int ROUND = D > VB_NORM ? D : VB_NORM;
     __shared__ uint32_t xh[TPW][VT_T];                         // inputs, twice each
     __shared__ uint32_t low[TPW][2];                           // the least cost of the last row, of alternate moves
-    __shared__ int over[TPW], varied[TPW];
+    __shared__ int over[TPW];
     const int tid = threadIdx.x, lane = tid & 63;
     auto row_of = [&](int t, int which) { return lds + (t * ROWS + which) * C::ROW; };
     // This thread's predecessor group and first slot of unit q.  Below K = 4, units 2i and 2i + 1 are predecessors 2j and
@@ -499,30 +579,19 @@ __device__ __forceinline__ void vb_forward(const float *__restrict__ tiles_in, i
     const int turn = pass ? 0 : VT_T / 2, pairs = (count + TPW - 1) / TPW;
 #pragma unroll 1
     for (int pair = worker; pair < pairs; pair += workers) {
-        if (tid < TPW) varied[tid] = 0;
         if (tid < TPW) over[tid] = pair * TPW + tid >= count ? -1 : pass ? info[pair * TPW + tid].over : 0;
-        __syncthreads();
         {
             const int t = tid >> 8, i = tid & 255;
             if (t < TPW) {
                 const bool there = pair * TPW + t < count;
-                const f16 v = there ? (f16)tiles_in[vt_pos(first + pair * TPW + t, i, ld)] : (f16)0.0f;
+                const f16 v = there ? (f16)tiles_in[vt_pos(lists.order[first + pair * TPW + t], i, ld)] : (f16)0.0f;
                 xh[t][i] = vb_bits(f16x2{v, v});
-                if (!(__builtin_fabsf((float)v) <= VB_X)) over[t] = -1;
             }
         }
         __syncthreads();
-        if (pass == 0) {                                       // equal inputs leave every other path a tie
-            const int t = tid >> 8, i = tid & 255;
-            if (t < TPW && xh[t][i] != xh[t][0]) varied[t] = 1;
-            __syncthreads();
-            if (tid < TPW && !varied[tid]) over[tid] = -1;
-            __syncthreads();
-        }
         bool any = false;
 #pragma unroll
         for (int t = 0; t < TPW; ++t) any = any || over[t] >= 0;
-        if (pass == 0 && tid < TPW && pair * TPW + tid < count) info[pair * TPW + tid].over = over[tid];
         if (!any) {
             __syncthreads();
             continue;
@@ -966,19 +1035,16 @@ struct vb_work {
 // What bounds it is latency: a chain of STORED levels, each a look into a row of which only the last level's group tells
 // where (a microsecond), some 150 instructions and trips to LDS.  150 us on average, 340 for the slowest of 256 tiles.
 template <int K>
-__device__ __forceinline__ void vb_backtrack(const float *__restrict__ tiles_in, int64_t ld, const vb_part &part, int at,
-                                             vb_work *W, int32_t *__restrict__ states_out, float *__restrict__ hat_out) {
+__device__ __forceinline__ void vb_backtrack(const float *__restrict__ tiles_in, int64_t ld, const vb_lists &lists,
+                                             const vb_part &part, int at, vb_work *W, int32_t *__restrict__ states_out, float *__restrict__ hat_out) {
     using C = vb_cfg<K>;
     float *const x = W->x, *const pre = W->pre;
     int *const states = W->states, *const start = W->start;
     const int lane = threadIdx.x & 63, pass = part.pass;
-    const int64_t tile = part.first + at;
+    const int64_t tile = __builtin_amdgcn_readfirstlane(lists.order[part.first + at]);
     vb_tile *const mine = part.info + at;
-    const int over = __builtin_amdgcn_readfirstlane(mine->over);
-    if ((uint32_t)over >= (uint32_t)C::G) {
-        if (pass && lane == 0) states_out[tile * VT_T] = -1;
-        return;
-    }
+    const int over = pass ? __builtin_amdgcn_readfirstlane(mine->over) : 0;
+    if ((uint32_t)over >= (uint32_t)C::G) return;              // left after the first pass
     const int turn = pass ? 0 : VT_T / 2, tie = pass ? over : -1;
     for (int i = lane; i < VT_T; i += 64) x[i] = (float)(f16)tiles_in[vt_pos(tile, (i + turn) & (VT_T - 1), ld)];
     for (int i = lane; i <= VT_T / VB_NORM; i += 64) pre[i] = mine->pre[i];
@@ -1030,14 +1096,9 @@ __device__ __forceinline__ void vb_backtrack(const float *__restrict__ tiles_in,
         __builtin_amdgcn_wave_barrier();
     }
     __builtin_amdgcn_wave_barrier();
-    if (pass == 0) {
-        if (lane == 0) mine->over = good ? states[VT_T / 2] >> K : -1;
-        return;
-    }
-    if (!good) {
-        if (lane == 0) states_out[tile * VT_T] = -1;
-        return;
-    }
+    if (!good && lane == 0) lists.left[atomicAdd(lists.counts + 1, 1)] = (int)tile;
+    if (pass == 0 && lane == 0) mine->over = good ? states[VT_T / 2] >> K : -1;
+    if (pass == 0 || !good) return;
     for (int i = lane; i < VT_T; i += 64) {
         const int s = states[i];
         states_out[tile * VT_T + i] = s;
@@ -1056,16 +1117,16 @@ constexpr int vb_lds() {
 }
 template <int K, int TPW>
 __global__ void __launch_bounds__(VB_THREADS, 4)
-vb_kernel(const float *__restrict__ tiles_in, int64_t ld, vb_part forward, vb_part back, int walkers,
+vb_kernel(const float *__restrict__ tiles_in, int64_t ld, vb_lists lists, vb_part forward, vb_part back, int walkers,
           int32_t *__restrict__ states_out, float *__restrict__ hat_out) {
-    extern __shared__ uint32_t lds[];
+    extern __shared__ __attribute__((aligned(16))) uint32_t lds[];   // (at 4, with the rows read 16 bytes at a time: a pass 228 -> 267 us)
     if ((int)blockIdx.x < walkers) {
         const int wave = threadIdx.x >> 6, at = blockIdx.x * VB_WALK + wave;
-        if (wave >= VB_WALK || at >= back.count) return;
+        if (wave >= VB_WALK || at >= vb_count(back, lists)) return;
         __builtin_amdgcn_s_setprio(3);
-        vb_backtrack<K>(tiles_in, ld, back, at, (vb_work *)lds + wave, states_out, hat_out);
+        vb_backtrack<K>(tiles_in, ld, lists, back, at, (vb_work *)lds + wave, states_out, hat_out);
     } else {
-        vb_forward<K, TPW>(tiles_in, ld, forward, blockIdx.x - walkers, gridDim.x - walkers, lds);
+        vb_forward<K, TPW>(tiles_in, ld, lists, forward, blockIdx.x - walkers, gridDim.x - walkers, lds);
     }
 }
 
@@ -1170,9 +1231,22 @@ size_t vb_bytes(int64_t n_tiles) {
     return (size_t)p.batch * p.batches * (vb_cfg<K>::STORED * vb_cfg<K>::G * 2 + sizeof(vb_tile));
 }
 
+// The lists, behind everything else (viterbi_kernel's rows take the place of the bounds'), the counts last
+size_t vb_list_bytes(int64_t n_tiles) { return 2 * (((size_t)n_tiles * sizeof(int) + 255) & ~(size_t)255) + 256; }
+vb_lists vb_lists_at(char *end, int64_t n_tiles) {
+    char *at = end - vb_list_bytes(n_tiles);
+    const size_t one = ((size_t)n_tiles * sizeof(int) + 255) & ~(size_t)255;
+    return vb_lists{(int *)(at + 2 * one), (int *)at, (int *)(at + one)};
+}
+
 template <int K>
-int vb_launch(const float *tiles, int64_t n_tiles, int64_t ld, void *scratch, int32_t *states, float *hat, hipStream_t stream) {
+int vb_launch(const float *tiles, int64_t n_tiles, int64_t ld, void *scratch, const vb_lists &lists, int32_t *states, float *hat,
+              hipStream_t stream) {
     using C = vb_cfg<K>;
+    hipLaunchKernelGGL(vb_try_kernel, dim3((unsigned)((n_tiles + 3) / 4)), dim3(256), 0, stream, tiles, n_tiles, ld, C::WIDE, lists);
+    hipLaunchKernelGGL(vb_order_kernel, dim3(1), dim3(1024), 0, stream, (int)n_tiles,
+                       8 * glqh_device_cus(), lists);
+    GLQH_LAUNCH_CHECK("viterbi lists launch");
     const vb_plan plan = vb_plan_of(n_tiles);
     const size_t rows = (size_t)plan.batch * C::STORED * C::G;
     const int cus = glqh_device_cus();
@@ -1191,17 +1265,18 @@ int vb_launch(const float *tiles, int64_t n_tiles, int64_t ld, void *scratch, in
         const dim3 grid(walkers + (work < 2 * cus ? work : 2 * cus));
         if (grid.x == 0) return 0;
         if (few)
-            hipLaunchKernelGGL((vb_kernel<K, C::FEW>), grid, dim3(VB_THREADS), (vb_lds<K, C::FEW>()), stream, tiles, ld, forward, back,
-                               walkers, states, hat);
+            hipLaunchKernelGGL((vb_kernel<K, C::FEW>), grid, dim3(VB_THREADS), (vb_lds<K, C::FEW>()), stream, tiles, ld, lists, forward,
+                               back, walkers, states, hat);
         else
-            hipLaunchKernelGGL((vb_kernel<K, 2>), grid, dim3(VB_THREADS), (vb_lds<K, 2>()), stream, tiles, ld, forward, back, walkers,
-                               states, hat);
+            hipLaunchKernelGGL((vb_kernel<K, 2>), grid, dim3(VB_THREADS), (vb_lds<K, 2>()), stream, tiles, ld, lists, forward, back,
+                               walkers, states, hat);
         GLQH_LAUNCH_CHECK("viterbi launch");
         return 0;
     };
     // batches 2i and 2i + 1: F0(a) | F0(b) B0(a) | F1(a) B0(b) | F1(b) B1(a) | F0(a') B1(b) | ...
     vb_part back{0, 0, 0, nullptr, nullptr};
-    for (int64_t b = 0; b * plan.batch < n_tiles; b += 2)
+    for (int64_t b = 0; b * plan.batch < n_tiles; b += 2) {
+        if (b) hipLaunchKernelGGL(vb_stop_kernel, dim3(1), dim3(64), 0, stream, b * plan.batch, lists);
         for (int turn = 0; turn < 4; ++turn) {
             const vb_part forward = part(b + (turn & 1), turn >> 1);
             if (forward.count == 0 || plan.batches == 1) {     // nothing beside it
@@ -1212,24 +1287,27 @@ int vb_launch(const float *tiles, int64_t n_tiles, int64_t ld, void *scratch, in
             if (launch(forward, back)) return 1;
             back = forward;
         }
+    }
     return launch(vb_part{0, 0, 0, nullptr, nullptr}, back);
 }
+
+// a tile a CU is as fast without the bounds' chain of launches (256 tiles, exact / on bounds: 1.38 / 1.62 ms at K = 2,
+// 1.16 / 1.20 at 3, 1.40 / 1.16 at 4; 512: 2.15 / 1.68, 1.89 / 1.52, 2.18 / 1.58)
+bool vb_takes(int K, int64_t n_tiles) { return K == 4 || (K >= 2 && n_tiles > glqh_device_cus()); }
 
 template <int K>
 int vt_launch(const float *tiles, int64_t n_tiles, int64_t ld, void *scratch, int grid, int32_t *states, float *hat,
               hipStream_t stream) {
-    int marked = 0;
+    vb_lists lists = {};
     if constexpr (K >= 2) {
-        // a tile a CU is as fast without the bounds' chain of launches (256 tiles, exact / on bounds: 1.38 / 1.62 ms at K = 2,
-        // 1.16 / 1.20 at 3, 1.40 / 1.16 at 4; 512: 2.15 / 1.68, 1.89 / 1.52, 2.18 / 1.58)
-        if (K == 4 || n_tiles > glqh_device_cus()) {
-            if (int rc = vb_launch<K>(tiles, n_tiles, ld, scratch, states, hat, stream)) return rc;
-            marked = 1;
+        if (vb_takes(K, n_tiles)) {
+            lists = vb_lists_at((char *)scratch + glqh_viterbi_scratch_bytes(K, n_tiles), n_tiles);
+            if (int rc = vb_launch<K>(tiles, n_tiles, ld, scratch, lists, states, hat, stream)) return rc;
         }
     }
     constexpr size_t lds = vt_cfg<K>::ROWS * sizeof(float) * (size_t)vt_cfg<K>::G;
     hipLaunchKernelGGL(viterbi_kernel<K>, dim3((unsigned)grid), dim3(vt_cfg<K>::THREADS), lds, stream, tiles, n_tiles, ld,
-                       (float *)scratch, states, hat, marked);
+                       (float *)scratch, states, hat, lists);
     GLQH_LAUNCH_CHECK("viterbi launch");
     return 0;
 }
@@ -1263,8 +1341,9 @@ size_t glqh_viterbi_scratch_bytes(int K, int64_t n_tiles) {
     const size_t row = sizeof(float) << (16 - K);
     const int depth = K == 1 ? vt_cfg<1>::DEPTH : K == 2 ? vt_cfg<2>::DEPTH : K == 3 ? vt_cfg<3>::DEPTH : vt_cfg<4>::DEPTH;
     const size_t exact = (size_t)glqh_viterbi_grid(K, n_tiles) * (VT_T / depth) * row;
-    const size_t bound = K == 2 ? vb_bytes<2>(n_tiles) : K == 3 ? vb_bytes<3>(n_tiles) : K == 4 ? vb_bytes<4>(n_tiles) : 0;
-    return (exact > bound ? exact : bound) + 255 & ~(size_t)255;
+    if (!vb_takes(K, n_tiles)) return exact;
+    const size_t bound = K == 2 ? vb_bytes<2>(n_tiles) : K == 3 ? vb_bytes<3>(n_tiles) : vb_bytes<4>(n_tiles);
+    return (((exact > bound ? exact : bound) + 255) & ~(size_t)255) + vb_list_bytes(n_tiles);
 }
 
 // ld: 0 for tiles in step order, else the row length of the (m, n) matrices `tiles` and `hat`

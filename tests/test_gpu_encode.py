@@ -345,6 +345,65 @@ def test_viterbi_of_decoded_weights(K, kind):
         assert torch.equal(hat.cpu(), X)
 
 
+def _quantize_counts(X, K):
+    """States, and how many tiles the search on bounds tried and left (the counts that end its workspace)."""
+    from glq_amd import _lib
+    lib, n = _lib.load(), X.shape[0]
+    X, states, hat = X.to(DEV), torch.empty(n, 256, dtype=torch.int32, device=DEV), torch.empty(n, 256, device=DEV)
+    ws = torch.zeros(lib.glqh_trellis_quantize_workspace_bytes(K, n), dtype=torch.uint8, device=DEV)
+    _lib.check(lib.glqh_trellis_quantize_tiles(X.data_ptr(), n, K, states.data_ptr(), hat.data_ptr(), ws.data_ptr(), ws.numel(),
+                                               torch.cuda.current_stream().cuda_stream))
+    return states, *ws[-256:].view(torch.int32)[:2].tolist()
+
+
+@pytest.mark.parametrize("K", [2, 3, 4])
+@pytest.mark.parametrize("kind", ["normal", "wide", "wide among normal", "normal among wide", "ramps"])
+def test_viterbi_tiles_on_either_search(K, kind):
+    """Which tiles the search on bounds tries, how many it leaves, and the exact states of all of them: normal values (tried,
+    and a few in a thousand left), values far beyond the weights' range (not tried), both mixed, a majority (only the
+    normal ones) and a minority of normal ones (none), and ramps, which the lists do not hold: not tried to the end."""
+    say("viterbi on either search", K, kind)
+    n = 2500 if kind == "ramps" else 700
+    g = torch.Generator().manual_seed(K)
+    X = torch.randn(n, 256, generator=g) * 0.9
+    wide = torch.zeros(n, dtype=torch.bool)
+    if kind.startswith("wide"):
+        wide[:] = kind == "wide"
+        wide[::3] = True
+    elif kind == "normal among wide":
+        wide[:] = True
+        wide[::3] = False
+    X[wide] *= 7
+    if kind == "ramps":
+        X = torch.linspace(-3, 3, 256) + X * 1e-3
+    states, tried, left = _quantize_counts(X, K)
+    if kind == "ramps":
+        assert n > tried and left > tried // 2, (tried, left)
+    else:
+        assert tried == {"normal": n, "wide": 0, "wide among normal": n - int(wide.sum()), "normal among wide": 0}[kind], tried
+        assert left <= n // 50, left
+    ref = _exact_states(X, K)
+    assert torch.equal(states, ref), (states != ref).any(1).nonzero()[:5]
+
+
+@pytest.mark.parametrize("K,m,n", [(2, 256, 320), (3, 288, 256), (4, 512, 576)])
+def test_quantize_matrix_on_bounds_equals_the_tile_route(K, m, n):
+    """More tiles than CUs, whose places in the matrix the lists tell, all but two of them on bounds: the tile route, bit for bit."""
+    from glq_amd import ext
+    say("quantize matrix on bounds", K, m, n)
+    W = torch.randn(m, n, generator=torch.Generator().manual_seed(K)) * 0.9
+    W[:16, :16] = 0.25
+    W[-16:, 32:48] *= 8
+    W = W.to(DEV)
+    packed, recon = ext.trellis_quantize_matrix(W, K)
+    tiles = ext.trellis_matrix_to_tiles(W)
+    states, tried, _ = _quantize_counts(tiles, K)
+    assert tried == tiles.shape[0] - 2
+    assert torch.equal(packed, ext.trellis_pack_states(states, m, n, K))
+    assert torch.equal(recon, ext.trellis_tiles_to_matrix(ext.trellis_quantize_tiles(tiles, K)[0], m, n))
+    assert torch.equal(ext.glq_decompress_trellis_3inst_cuda(packed, m, n).float(), recon)
+
+
 def test_viterbi_under_capture():
     """Captured and replayed on other tiles: the launches' batches hand each other their rows through the same memory."""
     from glq_amd import ext
