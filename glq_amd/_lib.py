@@ -100,6 +100,7 @@ SIGNATURES = {
     "glqh_e8_shell_quantize": (
         c_int, [c_vp, c_i64, c_vp, c_vp, c_i64, c_vp, c_vp, c_vp, c_sz, c_vp]),
     "glqh_trellis_quantize_workspace_bytes": (c_sz, [c_int, c_i64]),
+    "glqh_trellis_quantize_least_workspace_bytes": (c_sz, [c_int, c_i64]),
     "glqh_trellis_quantize_tiles": (c_int, [c_vp, c_i64, c_int, c_vp, c_vp, c_vp, c_sz, c_vp]),
     "glqh_trellis_quantize_matrix_workspace_bytes": (c_sz, [c_int, c_i64, c_i64]),
     "glqh_trellis_quantize_matrix": (c_int, [c_vp, c_i64, c_i64, c_int, c_vp, c_vp, c_vp, c_sz, c_vp]),

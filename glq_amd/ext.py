@@ -1195,6 +1195,13 @@ def e8_quantize(x, codebook, codebook_norms=None, return_decoded=True):
     return dec, idx
 
 
+def _quantize_ws(nbytes, least, device):
+    try:
+        return _ws(nbytes, device)
+    except torch.OutOfMemoryError:                            # the search in smaller batches
+        return _ws(least, device)
+
+
 def trellis_quantize_tiles(tiles, K):
     """bitshift_codebook.quantize (glq/trellis.py:467-484) on the GPU: (B, 256) tiles in step
     order -> (hat (B, 256) fp32, states (B, 256) int32), tail-biting Viterbi, K = 1..4."""
@@ -1208,8 +1215,8 @@ def trellis_quantize_tiles(tiles, K):
     hat = torch.empty(B, 256, dtype=torch.float32, device=x.device)
     if B:
         with torch.cuda.device(x.device):
-            nb = lib.glqh_trellis_quantize_workspace_bytes(int(K), B)
-            ws = _ws(max(nb, 256), x.device)
+            ws = _quantize_ws(lib.glqh_trellis_quantize_workspace_bytes(int(K), B),
+                              lib.glqh_trellis_quantize_least_workspace_bytes(int(K), B), x.device)
             check(lib.glqh_trellis_quantize_tiles(_p(x), B, int(K), _p(states), _p(hat), _p(ws), ws.numel(),
                                                   _stream()))
     return hat, states
@@ -1288,6 +1295,8 @@ def trellis_quantize_matrix(W_rht, K):
     packed = torch.empty(((m // 16) * (n // 16), 16 * int(K)), dtype=torch.int16, device=W.device)
     recon = torch.empty_like(W)
     with torch.cuda.device(W.device):
-        ws = _ws(lib.glqh_trellis_quantize_matrix_workspace_bytes(int(K), m, n), W.device)
+        tiles = (m // 16) * (n // 16)
+        ws = _quantize_ws(lib.glqh_trellis_quantize_matrix_workspace_bytes(int(K), m, n),
+                          lib.glqh_trellis_quantize_least_workspace_bytes(int(K), tiles) + 1024 * tiles, W.device)
         check(lib.glqh_trellis_quantize_matrix(_p(W), m, n, int(K), _p(packed), _p(recon), _p(ws), ws.numel(), _stream()))
     return packed, recon

@@ -475,6 +475,10 @@ int glqh_e8_shell_quantize(const float *x, int64_t N, const float *table_f32, co
 
 size_t glqh_trellis_quantize_workspace_bytes(int K, int64_t n_tiles);
 
+/* Less than that does too, at a tenth more time (calls of more than four tiles per CU, half as much); the matrix
+ * entry below takes this and the states, 1024 bytes per tile. */
+size_t glqh_trellis_quantize_least_workspace_bytes(int K, int64_t n_tiles);
+
 /* Tail-biting Viterbi search of the 3INST trellis for n_tiles sequences of 256 fp32 values
  * (a 16x16 tile in step order): states_out (n_tiles, 256) int32, hat_out (n_tiles, 256) fp32 =
  * decode_3inst(state).  Inputs are rounded to fp16 first, costs are fp32, ties go to the

@@ -404,6 +404,43 @@ def test_quantize_matrix_on_bounds_equals_the_tile_route(K, m, n):
     assert torch.equal(ext.glq_decompress_trellis_3inst_cuda(packed, m, n).float(), recon)
 
 
+@pytest.mark.parametrize("K,n", [(2, 1025), (3, 2000), (4, 1700), (1, 600), (4, 3)])
+def test_viterbi_in_the_least_workspace(K, n, monkeypatch):
+    """Where the larger workspace is not to be had: the least one, half of it for many tiles, gives the same states; a byte
+    less is refused."""
+    from glq_amd import _lib, ext
+    say("viterbi least workspace", K, n)
+    lib = _lib.load()
+    most, least = lib.glqh_trellis_quantize_workspace_bytes(K, n), lib.glqh_trellis_quantize_least_workspace_bytes(K, n)
+    assert least < 0.51 * most if K > 1 and n > 1000 else least <= most
+    X = _search_tiles(n, n)
+    hat, states = ext.trellis_quantize_tiles(X.to(DEV), K)
+    W = torch.randn(512, 1024, generator=torch.Generator().manual_seed(K)).to(DEV)
+    want = ext.trellis_quantize_matrix(W, K)
+    taken, plain = [], ext._ws
+    larger = {most} - {least}
+    if K > 1:
+        larger.add(lib.glqh_trellis_quantize_matrix_workspace_bytes(K, 512, 1024))
+
+    def short(nbytes, device):
+        taken.append(nbytes)
+        if nbytes in larger:
+            raise torch.OutOfMemoryError("short of memory")
+        return plain(nbytes, device)
+
+    monkeypatch.setattr(ext, "_ws", short)
+    got = ext.trellis_quantize_tiles(X.to(DEV), K)
+    assert taken[-1] == least
+    assert torch.equal(got[1], states) and torch.equal(got[0], hat)
+    assert all(torch.equal(a, b) for a, b in zip(ext.trellis_quantize_matrix(W, K), want))
+    monkeypatch.undo()
+    ws = torch.empty(least - 1, dtype=torch.uint8, device=DEV)
+    x = X.to(DEV)
+    with pytest.raises(RuntimeError, match="workspace"):
+        _lib.check(lib.glqh_trellis_quantize_tiles(x.data_ptr(), n, K, states.data_ptr(), hat.data_ptr(), ws.data_ptr(), ws.numel(),
+                                                   torch.cuda.current_stream().cuda_stream))
+
+
 def test_viterbi_under_capture():
     """Captured and replayed on other tiles: the launches' batches hand each other their rows through the same memory."""
     from glq_amd import ext
