@@ -271,12 +271,15 @@ def _search_tiles(n, seed):
 @pytest.mark.parametrize("n", [257, 512, 513, 1025, 2051])
 def test_viterbi_on_bounds_equals_the_exact_search(K, n):
     """Every route of the search on lower bounds (one and two tiles a workgroup, an odd last pair, one batch and batches
-    that take turns): the states of the same tiles searched a few at a time, which at 2 and 3 bits is the exact kernel
-    (itself pinned on the oracle above), and of the oracle on some of them."""
+    that take turns): the states of all tiles step by step on cost rows in memory, of the same tiles searched a few at a
+    time, which at 2 and 3 bits is the exact kernel (itself pinned on the oracle above), and of the oracle on some of them."""
     from glq_amd import ext
     say("viterbi on bounds", K, n)
     X = _search_tiles(n, 100 * K + n)
     hat, st = ext.trellis_quantize_tiles(X.to(DEV), K)
+    exact = _exact_states(X, K)
+    assert torch.equal(st, exact), (st != exact).any(1).nonzero()[:5]
+    assert torch.equal(hat.cpu(), torch.from_numpy(O.lut_3inst().astype(np.float32))[exact.cpu().long()])
     few = [ext.trellis_quantize_tiles(c.to(DEV), K) for c in X.split(200)]
     assert torch.equal(st, torch.cat([f[1] for f in few])), (st != torch.cat([f[1] for f in few])).any(1).nonzero()[:5]
     assert torch.equal(hat, torch.cat([f[0] for f in few]))
@@ -446,6 +449,7 @@ def test_viterbi_under_capture():
     from glq_amd import ext
     say("viterbi under capture")
     X = torch.zeros(1100, 256, device=DEV)
+    lut = t(O.lut_3inst().astype(np.float32))
     ext.trellis_quantize_tiles(X[:4], 4)
     side = torch.cuda.Stream()
     side.wait_stream(torch.cuda.current_stream())
@@ -456,5 +460,5 @@ def test_viterbi_under_capture():
         X.copy_(_search_tiles(1100, turn))
         graph.replay()
         torch.cuda.synchronize()
-        want = ext.trellis_quantize_tiles(X, 4)
-        assert torch.equal(st, want[1]) and torch.equal(hat, want[0]), turn
+        assert torch.equal(st, _exact_states(X, 4)), turn
+        assert torch.equal(hat, lut[st.long()]), turn
