@@ -112,11 +112,17 @@ def test_grouped_calls_against_single_layers(ms, n, B, bits, shared_sv):
 
 
 @pytest.mark.parametrize("ms,n,B,bits", [((32768, 1056, 544), 1024, 256, (4,)), ((20512, 12384), 576, 200, (2,)),
-                                         ((32640, 288), 1024, 130, (4, 2)), ((10912, 96, 160), 256, 1500, (3,))])
+                                         ((32640, 288), 1024, 130, (4, 2)), ((10528, 96, 160), 1024, 1000, (3,)),
+                                         ((10528, 96, 160), 512, 1020, (4, 2))])
 def test_grouped_last_round_of_half_tiles(ms, n, B, bits):
-    """The last round of row tiles as tiles of 64 rows across the layers of a group: layers that begin in it and layers whose
-    last tile has 32, 96 or all of its rows."""
+    """The last round of 256-token tiles as tiles of 64 rows across the layers of a group (K slots of 8 steps of 64 columns and
+    more): layers that begin in it and layers whose last tile has 32, 96 or all of its rows, one and four token tiles."""
     test_grouped_calls_against_single_layers(ms, n, B, bits, False)
+
+
+def test_grouped_512_token_tiles_of_short_rows():
+    """Rows of four steps, tiles of 512 tokens."""
+    test_grouped_calls_against_single_layers((10912, 96, 160), 256, 1500, (3,), False)
 
 
 def test_grouped_many_tokens_refusals():

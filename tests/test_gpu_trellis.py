@@ -140,10 +140,11 @@ def test_matmul_large_batch_tiles(ext, m, n, B, K):
 
 
 @pytest.mark.parametrize("m,n,B,K", [(32768 + 32, 1024, 256, 4), (49152, 1024, 200, 3), (32768 + 224, 1024, 129, 2),
-                                     (11392 - 96, 128, 1500, 4), (16384 - 32, 192, 1025, 3), (14336, 320, 2048, 4)])
+                                     (10976, 1024, 1000, 4), (11008, 1088, 1024, 3), (10848, 1024, 1020, 2)])
 def test_matmul_last_round_of_half_tiles(ext, m, n, B, K):
-    """A last round of row tiles on at most half of the CUs runs as tiles of 64 rows: one row tile of 32 rows (its second
-    half is empty), as many as there can be, 96 rows in the last one; tiles of 256 and of 512 tokens, ragged in the tokens.
+    """A last round of 256-token tiles on at most half of the CUs runs as tiles of 64 rows (K slots of 16 steps of 64 columns
+    and more): one row tile of 32 rows (its second half is empty), as many as there can be, 96 rows in the last one; one
+    and four token tiles, whole and ragged.
     The products are exact in fp32 and added in fp32: n roundings of at most the sum of their sizes, one more of the scale."""
     say("matmul half tiles", m, n, B, K)
     pt = t(O.random_packed(m, n, K, seed=5))
@@ -154,6 +155,34 @@ def test_matmul_last_round_of_half_tiles(ext, m, n, B, K):
     assert out.shape == (B, m) and bool(((out.double() - ref).abs() <= (n + 1) * 2.0 ** -24 * size).all())
     ext.glq_decode_matmul_trellis_3inst_cuda(xt, pt, m, n, 0.25, out=out, accum=True)
     assert bool(((out.double() - 2 * ref).abs() <= (2 * n + 3) * 2.0 ** -24 * size).all())
+
+
+@pytest.mark.parametrize("m,n,B,K", [(11392 - 96, 128, 1500, 4), (16384 - 32, 192, 1025, 3), (14336, 320, 2048, 4)])
+def test_matmul_last_round_behind_512_token_tiles(ext, m, n, B, K):
+    """A last round of 512-token tiles on at most half of the CUs: 256-token tiles in a launch of their own.  The same bound."""
+    test_matmul_last_round_of_half_tiles(ext, m, n, B, K)
+
+
+@pytest.mark.parametrize("m,n,B,K2", [(32768 + 32, 512, 200, 2), (32768 + 224, 576, 130, 1), (32768 + 96, 512, 129, 4),
+                                      (10976, 1024, 999, 3)])
+def test_two_stage_last_round_of_half_tiles(ext, m, n, B, K2):
+    """The same round of a layer whose two streams are decoded into one operand (K slots of 8 steps and more), with fp16 sums:
+    the same tokens 50 at a time, which are tiles of 128 rows throughout."""
+    say("two-stage half tiles", m, n, B, K2)
+    _, sv = O.rht_signs(m, n, 3)
+    su, _ = O.rht_signs(m, n, 4)
+    art = {"trellis_packed": O.random_packed(m, n, 4, 5), "trellis_packed2": O.random_packed(m, n, K2, 6), "SU": su, "SV": sv,
+           "Wscale": np.float32(0.05), "inv_resid_scale2": np.float32(0.3), "blocks_m": O.block_decompose(m),
+           "blocks_n": O.block_decompose(n)}
+    a = _layer_args(art, m, n, torch.bfloat16)
+    x = torch.randn(B, n, generator=torch.Generator().manual_seed(B)).to(torch.bfloat16).to(DEV)
+
+    def layer(rows):
+        return ext.glq_fused_linear_trellis_3inst_rvq2_cuda(
+            rows.contiguous(), a["sv"], a["su"], a["packed"], a["packed2"], a["bn"], a["bm"], a["bn_meta"], a["bm_meta"],
+            a["wscale"], a["inv2"], n, m, n, m, out_dtype=torch.bfloat16)
+
+    assert rel(layer(x), torch.cat([layer(r) for r in x.split(50)])) < 4e-3
 
 
 @pytest.mark.parametrize("n,B,K", [(64, 17, 4), (256, 64, 2), (320, 32, 3), (576, 33, 4), (768, 49, 2), (832, 64, 4),
