@@ -589,7 +589,8 @@ e8_tile_small_kernel(const et_args a) {
         for (int dd = 0; dd < 4; ++dd) decode(dd, abuf + dd * ET_BUF);
         et_barrier();
         // group q is multiplied out of buffer q & 1 while the next one, if there is one (MORE), is decoded into the other
-        // (LEAN: the registers are all taken, the last group as another piece of code spills some)
+        // (LEAN: the registers are all taken, the last group as another piece of code spills some, so that it decodes once
+        // more, unused).  Index runs and activations past the slot's end are requests for its last ones.
         constexpr bool LEAN = NS == 4 && NTW == 2;
         auto group = [&](auto MORE, int q, int h) {             // h = q & 1
             const u32x4 *rd = abuf + h * 4 * ET_BUF + rg * GLQH_WAVE + lane;

@@ -1302,7 +1302,8 @@ moe_mid_kernel(moe_mid_args a, f16 *__restrict__ out, glqh_meta_args m13, glqh_m
 // Whole call, the separate launches (3 or 2) -> this one, microseconds: 128 experts of 2048 -> 2 x 768 -> 2048 at 8 / 32 /
 // 128 / 512 slots 27.5 / 52.5 / 85.5 / 126.3 -> 26.6 / 50.5 / 83.3 / 124.0, 32 of 1024 x 512 at 80 slots 35.8 -> 33.2, 16
 // of 2048 x 768 at 384 slots (tile form) 67.9 -> 63.1; against the form above 16 of 1024 x 512 at 2048 slots 75.0 ->
-// 74.1, 128 of 2048 x 768 at 4096 slots 272.7 -> 273.5 (not taken).
+// 74.1, 128 of 2048 x 768 at 4096 slots 272.7 -> 273.5 (not taken).  The butterflies begin in another order than those of the
+// separate launches: the same widths throughout, but not the same bits (5e-4 of the experts' result, some fp16 roundings).
 struct mid_part {
     rht_slice blk;
     int te;                                                      // the thread's number among those of its block
@@ -1570,7 +1571,8 @@ moe_route_kernel(const int64_t *__restrict__ topk_ids, int n_slots, int n_expert
 // The table and the input transform of the tokens' rows, which wait for nothing of each other, in one launch: the first
 // route_wgs workgroups write the table, the others transform one block of one row each.  Whole call, one launch each -> this:
 // 128 experts of 2048 -> 2 x 768 -> 2048 at 32 / 128 / 512 slots 50.6 / 83.3 / 123.8 -> 48.6 / 81.7 / 121.2 us, 32 of
-// 1024 x 512 at 80 slots 33.2 -> 31.3, 16 of 1024 x 512 at 2048 slots 74.3 -> 71.3.
+// 1024 x 512 at 80 slots 33.2 -> 31.3, 16 of 1024 x 512 at 2048 slots 74.3 -> 71.3.  (Up to 64 rows the launch of their
+// own sums in another order, so some roundings of the rows to fp16 differ.)
 template <typename XT>
 __global__ void __launch_bounds__(256)
 moe_route_input_kernel(const int64_t *__restrict__ topk_ids, int n_slots, int n_experts, int *__restrict__ perm,

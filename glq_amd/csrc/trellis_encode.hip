@@ -12,8 +12,8 @@
 // All arithmetic is fp32 with separate subtract, multiply and add (no contraction), the
 // input is rounded to fp16 first (glq/trellis.py:468).
 //
-// viterbi_kernel does that for every tile of small calls and of 1-bit ones; elsewhere for the few that the search on
-// lower bounds, further down, leaves to it.
+// viterbi_kernel does that for every tile of 1-bit calls and, at 2 and 3 bits, of small ones; elsewhere for those that the
+// search on lower bounds, further down, does not try or leaves to it.
 //
 // What bounds it is vector-ALU issue: 65536 states per step, 510 steps per tile.  A workgroup
 // therefore keeps the whole table in registers, two fp16 values to a register (v_fma_mix_f32
@@ -368,8 +368,8 @@ viterbi_kernel(const float *__restrict__ tiles_in, int64_t n_tiles, int64_t ld, 
 //     K = 3                     14.9 / 10.3  14.7 / 9.6   14.6 / 10.9  14.6 / 11.0  14.6 / 14.8  14.6 / 14.7
 //     K = 2                     16.7 / 8.1   16.7 / 9.6   16.7 / 10.4  16.8 / 10.8  16.7 / 12.2  16.7 / 16.7
 // Slower is what fills the lists and shows nothing beforehand, as slow ramps do (-3 to 3 over the tile's steps): 17.5 / 19.2,
-// 14.6 / 16.2, 16.7 / 18.7, up to 1.4 times in calls of one or two batches.  2048 x 2048 weights in viterbi_kernel alone -> so: 69.7 -> 31.9 ms at
-// K = 4, 59.0 -> 38.1 at 3, 66.5 -> 36.4 at 2.
+// 14.6 / 16.2, 16.7 / 18.7, up to 1.4 times in calls of one or two batches.  2048 x 2048 weights: 69.6 -> 32.7 at K = 4,
+// 58.6 -> 37.5 at 3, 66.6 -> 35.5 at 2.
 constexpr int VB_THREADS = 512;
 constexpr int VB_NORM = 2;                 // steps between two moves of the row's minimum into B
 constexpr float VB_X = 16.0f;              // largest input: (16 + 4)^2 for 16 / K steps stays far below 65504

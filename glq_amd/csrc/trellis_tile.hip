@@ -700,7 +700,7 @@ __device__ __forceinline__ void tr_tile_small_body(const tt_args &a, const tt_gr
             tt_barrier();                                       // rd has been read, wr is written
         };
         // Records of the group after the next one are requested into the set that the previous group has emptied, by turns;
-        // none past the slot's end (2048 x 11008 at 37 tokens, 4 + 2 bits in slots of 11 steps, the call 28.1 -> 27.4 us).
+        // no group of them past the slot's last (2048 x 11008 at 37 tokens, 4 + 2 bits in slots of 11 steps, the call 28.1 -> 27.4 us).
         // Where nothing is requested it is another piece of code, not a branch around the request: behind that the waits would
         // have to assume that nothing was (14336 x 4096 at 64 tokens, slots of 32 steps, 47.1 -> 48.6 us).
         auto request = [&](int qd, tr_record<R> (&r)[4], tr_record<RB> (&rb)[4]) {
