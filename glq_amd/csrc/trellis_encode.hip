@@ -361,7 +361,7 @@ viterbi_kernel(const float *__restrict__ tiles_in, int64_t n_tiles, int64_t ld, 
 // of both go to viterbi_kernel (with marks instead of lists, every workgroup walking its share of all tiles, it took the
 // time of all of them where half were marked).  Far beyond the weights' range the cost is mostly what no path can avoid,
 // and SLACK of that lets everything through: tiles with more than WIDE of it are not tried either (K = 4: 5 % of those with
-// 2-3 are left, 23 % with 4-5, 64 % with 10-14; K = 3 and 2: 17 and 18 % of the first beyond), nor is a minority of up to two
+// 2-3 are left, 23 % with 4-5, 64 % with 10-14; K = 3 and 2: 20 and 18 % of the first beyond), nor is a minority of up to two
 // chips full, nor the rest of a call after batches of which more than half were left.  4096 tiles, exact / so, ms:
 //   normal values of sigma      1e-4         0.9          1.6          1.8          2.2          3 and more
 //     K = 4                     17.5 / 17.7  17.5 / 8.2   17.5 / 11.1  17.4 / 15.8  17.4 / 17.6  17.5 / 17.6
