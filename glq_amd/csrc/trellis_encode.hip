@@ -24,6 +24,8 @@
 // state and step, compare and two selects per state, a byte of arg-min per step and group) -> 69.6 ms,
 // vector ALUs issuing in 74 % of the cycles at 2.4 GHz (30.8 M instructions per SIMD, of which 29.9 M
 // are the 3.5 per state).
+#include <algorithm>
+#include <type_traits>
 #include "common.h"
 #include "trellis_device.h"
 
@@ -282,7 +284,7 @@ __device__ __forceinline__ int64_t vt_pos(int64_t tile, int t, int64_t ld) {
 // Which tiles of a call are searched how: those for the search on bounds, from order[0] on, those that it does not try, from
 // order[n_tiles - 1] back, and those that it tried and left.
 struct vb_lists {
-    int *counts;                           // how many it tries, how many it left; null: no such search
+    int *counts;                           // how many it tries, how many it left, and before this batch; null: no such search
     int *order, *left;
 };
 
@@ -357,19 +359,20 @@ viterbi_kernel(const float *__restrict__ tiles_in, int64_t n_tiles, int64_t ld, 
 // and viterbi_kernel's costs of both paths, from which it takes the cheaper; 4 e < VB_NEAR.)  Where another kept path is
 // within VB_NEAR of the cheapest (3 % of the tiles), fp32 costs are evaluated forward over the kept ways, minima and lowest
 // states as in viterbi_kernel.
-// Tiles with inputs above VB_X, not finite or all equal are not tried, and those with more kept ways than fit are left: lists
-// of both go to viterbi_kernel (with marks instead of lists, every workgroup walking its share of all tiles, it took the
+// Tiles with inputs above VB_X, not finite or all equal are not tried, and those with more kept ways than fit, also at half the
+// slack, are left: lists of both go to viterbi_kernel (with marks instead of lists, every workgroup walking its share of all tiles, it took the
 // time of all of them where half were marked).  Far beyond the weights' range the cost is mostly what no path can avoid,
 // and SLACK of that lets everything through: tiles with more than WIDE of it are not tried either (K = 4: 5 % of those with
 // 2-3 are left, 23 % with 4-5, 64 % with 10-14; K = 3 and 2: 20 and 18 % of the first beyond), nor is a minority of up to two
 // chips full, nor the rest of a call after batches of which more than half were left.  4096 tiles, exact / so, ms:
 //   normal values of sigma      1e-4         0.9          1.6          1.8          2.2          3 and more
 //     K = 4                     17.5 / 17.7  17.5 / 8.2   17.5 / 11.1  17.4 / 15.8  17.4 / 17.6  17.5 / 17.6
+//     K = 4, through vm_kernel         10.4         6.4          9.4         15.4         17.6         17.6
 //     K = 3                     14.9 / 10.3  14.7 / 9.6   14.6 / 10.9  14.6 / 11.0  14.6 / 14.8  14.6 / 14.7
 //     K = 2                     16.7 / 8.1   16.7 / 9.6   16.7 / 10.4  16.8 / 10.8  16.7 / 12.2  16.7 / 16.7
 // Slower is what fills the lists and shows nothing beforehand, as slow ramps do (-3 to 3 over the tile's steps): 17.5 / 19.2,
-// 14.6 / 16.2, 16.7 / 18.7, up to 1.4 times in calls of one or two batches.  2048 x 2048 weights: 69.6 -> 32.7 at K = 4,
-// 58.6 -> 37.5 at 3, 66.6 -> 35.5 at 2.
+// 14.6 / 16.2, 16.7 / 18.7, up to 1.4 times in calls of one or two batches.  2048 x 2048 weights: 69.6 -> 32.7 at K = 4
+// (25.7 through vm_kernel), 58.6 -> 37.5 at 3, 66.6 -> 35.5 at 2.
 constexpr int VB_THREADS = 512;
 constexpr int VB_NORM = 2;                 // steps between two moves of the row's minimum into B
 constexpr float VB_X = 16.0f;              // largest input: (16 + 4)^2 for 16 / K steps stays far below 65504
@@ -465,6 +468,7 @@ struct vb_part {
     int count, pass;
     uint16_t *rows;
     vb_tile *info;
+    bool product;                          // bounds of vm_kernel
 };
 __device__ __forceinline__ int vb_count(const vb_part &part, const vb_lists &lists) {
     const int64_t left = __builtin_amdgcn_readfirstlane(lists.counts[0]) - part.first;
@@ -525,7 +529,16 @@ vb_order_kernel(int n_tiles, int few, vb_lists lists) {
 
 // Before the batch that begins at `first`: where more than half of those before it were left, it and the rest are not tried.
 __global__ void vb_stop_kernel(int64_t first, vb_lists lists) {
-    if (threadIdx.x == 0 && 2 * (int64_t)lists.counts[1] > first && lists.counts[0] > first) lists.counts[0] = (int)first;
+    if (threadIdx.x != 0) return;
+    if (2 * (int64_t)lists.counts[1] > first && lists.counts[0] > first) lists.counts[0] = (int)first;
+    lists.counts[2] = lists.counts[1];
+}
+
+// Between the passes of a large batch: where more than half were left in the first one, none of it is tried
+__global__ void vm_stop_kernel(int64_t first, int count, vb_lists lists) {
+    if (threadIdx.x != 0 || 2 * (lists.counts[1] - lists.counts[2]) <= count) return;
+    lists.counts[0] = (int)first;
+    lists.counts[1] = lists.counts[2];
 }
 
 // One forward pass, the rows of every DEPTH-th step to part.rows.  TPW tiles a workgroup: their steps share the table and
@@ -737,10 +750,236 @@ __device__ __forceinline__ void vb_forward(const float *__restrict__ tiles_in, i
     }
 }
 
+// ---- the forward pass on the matrix cores (K = 4, chips full of tiles) ---------------------
+// w^2 - 2xw + c is a product of matrices: rows are states, with w, w^2 and a one, columns are tiles, with -2x, a one and c.
+// w and x are fp16 numbers, w^2 two of them (rounded, and what that left), c the bound of the predecessor's group as it is
+// stored: the products are exact, and the sums are fp32.  A v_mfma_f32_32x32x16_f16 costs 1024 states in 32 clocks, where
+// vb_forward's two packed instructions take 75, and leaves the vector units the minima, three numbers to an instruction, and
+// x^2 and what moves into B once to a minimum.
+//
+// Operands.  Of the sixteen numbers of a row a product needs three and the one: a lane's eight hold two states each (its
+// halves of tw, of their squares and of what those lack), and lanes 32-63 two more; columns are sixteen tiles, twice, and
+// pick by their zeros: the first product of a pair takes the states of lanes 0-31 (their first halves in columns 0-15, their
+// second ones in 16-31), the second product those of lanes 32-63.  The ones meet the bounds in lanes 0-31 only, whose rows
+// 0-15 and 16-31 are two neighbouring predecessor groups a, in the order of their low digits, at one high digit k; bounds of
+// two such groups lie in one word.  So a pair of products costs the states of 4 predecessor groups at 2 high digits, eight
+// pairs are all 16 digits (a unit), and the minimum over them stays in its lane.
+//
+// A workgroup has sixteen tiles, a CU to itself: one row of bounds, 128 KB, is read by all and written by all in turn, and
+// eight waves have eight units each, with their table in 64 registers and the new bounds, until all have read, in 64 more.
+//
+// Rounding.  A sum is off by at most VM_OFF times its terms' magnitudes (2.6 * 2^-24 is the most that 3 * 10^7 sums of such
+// terms showed, and a rounding follows); with e the state's cost those are at most (2 |x| + sqrt e)^2 <= 5 x^2 + 5 e, and c, and
+// what moves, which is no more than c.  So 5 VM_OFF x^2 comes off every step's bounds, with what w^2 may lack below fp16's
+// smallest numbers, and VM_LESS of c + e.  Bounds are rounded once a step, towards zero; a row's least one stays at VM_FLOOR,
+// above what comes off until the next move, so that none is negative.
+//
+// 4096 tiles, a pass: 2.6 ms, where vb_forward takes 3.7, and 0.65 for the walk back, which nothing overlaps.  Vector ALUs issue
+// in 59 % of the cycles (three quarters of that the minima) and the matrix cores work in 39 %, at 2.0 GHz; the rows on their
+// way to memory take 0.4 ms of it.  Measured and not kept: products a pair ahead of the minima (2.6, with the rows in one
+// piece; no registers for more), four waves a SIMD (eight tiles a workgroup, 128 registers: 3.4), eight tiles and two rows
+// (2.8), priorities of waves (level).
+constexpr int VM_TILES = 16, VM_THREADS = 512;
+constexpr float VM_OFF = 6 * 0x1p-24f, VM_LESS = 0x1p-19f, VM_FLOOR = 0x1p-9f;
+static_assert(5 * VM_OFF < VM_LESS && VB_NORM * 2 * 5 * VM_OFF * VB_X * VB_X < 0.99f * VM_FLOOR, "all of a sum; no bound is negative");
+constexpr int VM_ROW = 2048 * VM_TILES, VM_LDS = (VM_ROW + VT_T * VM_TILES) * 4;   // words of the row; bytes
+
+template <int N, int END, typename F>
+__device__ __forceinline__ void vm_unroll(const F &f) {        // f(0), f(1), ... for more than a pragma unrolls
+    if constexpr (N < END) {
+        f(std::integral_constant<int, N>());
+        vm_unroll<N + 1, END>(f);
+    }
+}
+__device__ __forceinline__ float vm_loss(float x) { return 5 * VM_OFF * x * x + 0x1p-24f; }
+
+// Word of the bounds of groups k * 256 + 2p and + 1 (p < 128), tile t.  A product's lanes read 16 tiles at one or two p, what goes
+// to memory is 32 p at two k of one tile: the exclusive-or keeps both on different banks.
+__device__ __forceinline__ int vm_word(int k, int p, int t) { return (k * 128 + p) * VM_TILES + (t ^ ((p >> 2 & 7) | (k >> 3) << 3)); }
+
+__global__ void __launch_bounds__(VM_THREADS, 2)
+vm_kernel(const float *__restrict__ tiles_in, int64_t ld, vb_lists lists, vb_part part) {
+    using C = vb_cfg<4>;
+    typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+    typedef float f32x16 __attribute__((ext_vector_type(16)));
+    extern __shared__ __attribute__((aligned(16))) uint32_t lds[];
+    uint32_t *const xs = lds + VM_ROW;                         // inputs [step][tile], twice each
+    __shared__ uint32_t low[2][VM_TILES];                      // the least bound of the last row, of alternate moves
+    __shared__ int over[VM_TILES];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int half = lane >> 5, t = lane & 15, second = lane >> 4 & 1;
+    const int first = blockIdx.x * VM_TILES, count = vb_count(part, lists) - first;
+    if (count <= 0) return;
+    if (tid < VM_TILES) over[tid] = tid < count && part.pass ? part.info[first + tid].over : -1;
+    if (tid < 2 * VM_TILES) low[tid >> 4][tid & 15] = 0xFFFFFFFFu;
+    for (int i = tid; i < VT_T * VM_TILES; i += VM_THREADS) {
+        const int to = i >> 8, step = i & 255;
+        const f16 v = to < count ? (f16)tiles_in[vt_pos(lists.order[part.first + first + to], step, ld)] : (f16)0.0f;
+        xs[step * VM_TILES + to] = vb_bits(f16x2{v, v});
+    }
+    __syncthreads();
+    for (int i = tid; i < VM_ROW; i += VM_THREADS) {           // step 0: the group that the overlap names, or all
+        const int to = i & 15, p = i >> 4 & 127, k = i >> 11, g = over[to] - k * 256 - 2 * p;
+        const f16 in = (f16)VM_FLOOR, out = (f16)30000.0f;     // (far above any that matters, and finite: zeros meet it)
+        lds[vm_word(k, p, to)] = part.pass ? vb_bits(f16x2{g == 0 ? in : out, g == 1 ? in : out}) : vb_bits(f16x2{in, in});
+    }
+    uint32_t tw[8][8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const uint32_t s = (uint32_t)((2 * j + half) * C::G + (4 * (8 * wave + u) + second) * C::NK + t);
+            tw[u][j] = vb_bits(f16x2{tr_weight(s), tr_weight(s + 2 * C::NK)});
+            asm volatile("" : "+v"(tw[u][j]));                 // finished here
+        }
+    // the operands' fixed parts, kept apart from what changes
+    const uint32_t pick = second ? 0xFFFF0000u : 0x0000FFFFu, one = 0x3C003C00u & pick;
+    const uint32_t pick1 = half ? 0 : pick, pick2 = half ? pick : 0;
+    u32x4 a = {0, 0, 0, half ? 0u : second ? 0x3C000000u : 0x00003C00u}, b1[2], b2[2];
+    asm volatile("" : "+v"(a));
+#pragma unroll
+    for (int n = 0; n < 2; ++n) {
+        b1[n] = half ? u32x4{0, 0, 0, 0} : u32x4{0, one, one, 0};
+        b2[n] = half ? u32x4{0, one, one, 0} : u32x4{0, 0, 0, 0};
+        asm volatile("" : "+v"(b1[n]), "+v"(b2[n]));
+    }
+    const int read0 = (16 * wave + second) * VM_TILES * 4 + ((t ^ (wave & 1) << 2) << 2);
+    const int write0 = (2 * wave * 128 + 16 * second + 2 * half) * VM_TILES * 4 + ((t ^ second << 2 ^ (wave >> 2) << 3) << 2);
+    char *const row = (char *)lds;
+    const int turn = part.pass ? 0 : VT_T / 2;
+    float moved = -VM_FLOOR;
+    if (tid < VM_TILES && tid < count) part.info[first + tid].pre[0] = 0.0f;
+    __syncthreads();
+
+    // An eighth of what a wave writes of a level's row: 32 words p at eight of the digits, of one of its two tiles
+    const int high = lane & 1;
+    auto fetch = [&](int q, u32x4 (&v)[2]) __attribute__((always_inline)) {
+        const int to = 2 * wave + (q >> 2), p = 32 * (q & 3) + (lane >> 1), w = p >> 4 & 7;
+        const int from = vm_word(8 * high, p, to) * 4;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            typedef __attribute__((address_space(3))) const uint32_t lds_word;
+            __attribute__((address_space(3))) const char *at = (__attribute__((address_space(3))) const char *)row + (from + ((j ^ (w & 3)) << 14));
+            v[0][j] = *(lds_word *)at;
+            v[1][j] = *(lds_word *)(at + 8192);
+        }
+    };
+    auto keep = [&](int level, int q, const u32x4 (&v)[2]) __attribute__((always_inline)) {
+        const int to = 2 * wave + (q >> 2), p = 32 * (q & 3) + (lane >> 1), w = p >> 4 & 7;
+        uint16_t *o = part.rows + ((int64_t)(first + to) * C::STORED + level - 1) * C::G + 2 * p * C::NK + 8 * (high ^ w >> 2);
+        u32x4 even, odd;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            even[j] = __builtin_amdgcn_perm(v[1][j], v[0][j], 0x05040100u);
+            odd[j] = __builtin_amdgcn_perm(v[1][j], v[0][j], 0x07060302u);
+        }
+        if (to < count) {
+            *(u32x4 *)o = even;
+            *(u32x4 *)(o + C::NK) = odd;
+        }
+    };
+    uint32_t next = xs[turn * VM_TILES + t];
+#pragma unroll 1
+    for (int i = 1; i <= VT_T; ++i) {
+        const bool move = i % VB_NORM == 0;
+        const uint32_t xh = next;
+        next = xs[((i + turn) & (VT_T - 1)) * VM_TILES + t];   // read a step ahead
+        const float x = vb_half(xh & 0xFFFFu);
+        float shift = 0.0f;
+        if (move) {
+            shift = vb_half(low[i / VB_NORM & 1][t] & 0xFFFFu) - VM_FLOOR;
+            moved += shift;
+            if (tid < VM_TILES && tid < count) part.info[first + tid].pre[i / VB_NORM] = moved;
+        }
+        const bool store = !move && i > 1;                     // the row that this step reads
+        const float add = x * x * (1 - VM_LESS) - shift - vm_loss(x);
+        const uint32_t twice = vb_bits(vb_pair(xh) * f16x2{(f16)-2.0f, (f16)-2.0f});
+#pragma unroll
+        for (int n = 0; n < 2; ++n) {
+            b1[n].x = twice & pick1;
+            b2[n].x = twice & pick2;
+        }
+        f32x16 least;
+        u32x4 kept[2];
+        int at[2];
+        uint32_t out[8][8];
+        auto ask = [&](int n) {                                // the bounds of pair n
+            const int u = n >> 3, k = 2 * (n & 7);
+            if ((n & 15) == 0) {
+#pragma unroll
+                for (int q = 0; q < 2; ++q) {
+                    at[q] = (read0 ^ ((u >> 1 | q << 3) << 2)) + q * 65536;
+                    asm volatile("" : "+v"(at[q]));            // addresses of their own would all be kept
+                }
+            }
+            typedef __attribute__((address_space(3))) const volatile char lds_byte;   // volatile: into the operand, not two at once and moved
+            typedef __attribute__((address_space(3))) const volatile uint32_t lds_word;
+            lds_byte *from = (lds_byte *)row + at[k >> 3] + ((k & 7) * 8192 + u * 128);
+            b1[n & 1].w = *(lds_word *)from;
+            b2[n & 1].w = *(lds_word *)(from + 8192);
+        };
+        ask(0);
+        ask(1);
+        vm_unroll<0, 64>([&](auto at_n) __attribute__((always_inline)) {
+            constexpr int n = decltype(at_n)::value;
+            u32x4 &p1 = b1[n & 1], &p2 = b2[n & 1];
+            if (n % 8 == 0 && store) fetch(n >> 3, kept);
+            if (n % 8 == 4 && store) keep((i - 1) / C::DEPTH, n >> 3, kept);
+            a.x = tw[n >> 3][n & 7];
+            asm volatile("" : "+v"(a.x));                      // or the squares of all would be kept, for which there is no room
+            const f16x2 w = vb_pair(a.x), sq = w * w;
+            a.y = vb_bits(sq);
+            a.z = vb_bits(__builtin_elementwise_fma(w, w, -sq));
+            const f32x16 d1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, p1), f32x16{}, 0, 0, 0);
+            const f32x16 d2 = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, p2), f32x16{}, 0, 0, 0);
+            asm("" : "+v"(a), "+v"(p1), "+v"(p2));             // changed in place
+            if (n + 2 < 64) ask(n + 2);
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                least[r] = n % 8 == 0 ? __builtin_elementwise_minimum(d1[r], d2[r])
+                                      : __builtin_elementwise_minimum(__builtin_elementwise_minimum(least[r], d1[r]), d2[r]);
+            if (n % 8 == 3) asm volatile("" : "+v"(least));    // here, and not behind the branch
+            if (n % 8 == 7) {
+#pragma unroll
+                for (int r = 0; r < 8; ++r) {
+                    out[n >> 3][r] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(__builtin_fmaf(least[2 * r], 1 - VM_LESS, add),
+                                                                                                      __builtin_fmaf(least[2 * r + 1], 1 - VM_LESS, add)));
+                    asm volatile("" : "+v"(out[n >> 3][r]));   // now, and not where it is written: there is no room for the products
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        });
+        vt_barrier();                                          // read by all
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+#pragma unroll
+            for (int r = 0; r < 8; ++r)
+                *(uint32_t *)(row + (write0 ^ (r >> 1) << 2) + (u >> 2) * 8192 + (u & 3) * 2048 + (r >> 1) * 256 + (r & 1) * 64) = out[u][r];
+        if (!move) {                                           // numbers >= 0 order as their bits
+            f16x2 v = vb_pair(0x7C007C00u);
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+#pragma unroll
+                for (int r = 0; r < 8; r += 2)
+                    v = __builtin_elementwise_minimum(__builtin_elementwise_minimum(v, vb_pair(out[u][r])), vb_pair(out[u][r + 1]));
+            v = __builtin_elementwise_minimum(v, f16x2{v.y, v.x});
+            atomicMin(&low[(i + 1) / VB_NORM & 1][t], vb_bits(v) & 0xFFFFu);
+            if (tid < VM_TILES && i > VB_NORM) low[i / VB_NORM & 1][tid] = 0xFFFFFFFFu;   // the word of the move before
+        }
+        vt_barrier();
+    }
+#pragma unroll 1
+    for (int q = 0; q < 8; ++q) {
+        u32x4 v[2];
+        fetch(q, v);
+        keep(C::STORED, q, v);
+    }
+}
+
 // A tile's working memory in LDS during the backtrack.  Level l is step l * DEPTH; its entries are the
 // kept ways from the groups of level l (parents: where the states lead) to those of level l - 1 (children).
 struct vb_pool {
-    static constexpr int ENTRIES = 768;    // 550 at most in 3 * 10^4 tiles of Gaussian values, 170 on average
+    static constexpr int ENTRIES = 672;    // 550 at most in 3 * 10^4 tiles of Gaussian values, 170 on average
     float cost[ENTRIES];                   // of the entries: to the end
     uint16_t entry[ENTRIES];               // the digits of its states, nearest step first | parent << 8
     uint16_t via[ENTRIES];                 // of child j at j: best entry | its parent << 8 | close second << 14
@@ -769,8 +1008,8 @@ __device__ __forceinline__ void vb_walk(int g, int p, int (&st)[vb_cfg<K>::DEPTH
 // level l at hist + (l - 1) * G; pre[j]: B at step j * VB_NORM; tie: the only group of step 0, or -1; the states up to
 // step `upto` are wanted.
 template <int K>
-__device__ __forceinline__ bool vb_trace(int n, int gv, float &limit, const float *x, const uint16_t *__restrict__ hist,
-                                         const float *pre, int tie, int upto, vb_pool *P, int *states) {
+__device__ __forceinline__ bool vb_trace(int n, int gv, float &limit, const f16 *x, const uint16_t *__restrict__ hist,
+                                         const float *pre, int tie, int upto, vb_pool *P, uint16_t *states) {
     using C = vb_cfg<K>;
     constexpr int D = C::DEPTH, LEVELS = C::STORED, R = (1 << (K * D)) / 64;
     const int lane = threadIdx.x & 63;
@@ -780,7 +1019,7 @@ __device__ __forceinline__ bool vb_trace(int n, int gv, float &limit, const floa
     bool full = false, empty = false;
     float xn[D], pn = pre[(LEVELS - 1) * D / VB_NORM];         // read a level ahead
 #pragma unroll
-    for (int e = 0; e < D; ++e) xn[e] = x[VT_T - 1 - e];
+    for (int e = 0; e < D; ++e) xn[e] = (float)x[VT_T - 1 - e];
     // The ways from a group, R to a lane, by where their bounds lie: digits of a lane's ways, and the first one's place.
     constexpr int E = 16 - K - K * D;                          // what of the group is left above the digits
     int ways[R], place;
@@ -820,7 +1059,7 @@ __device__ __forceinline__ bool vb_trace(int n, int gv, float &limit, const floa
 #pragma unroll
         for (int e = 0; e < D; ++e) {
             xs[e] = xn[e];
-            xn[e] = x[((l - 1) * D - 1 - e) & (VT_T - 1)];
+            xn[e] = (float)x[((l - 1) * D - 1 - e) & (VT_T - 1)];
         }
         pn = pre[(l > 1 ? l - 2 : 0) * D / VB_NORM];
         // lane j: child j, its cheapest entry, and the next one's cost
@@ -949,7 +1188,7 @@ __device__ __forceinline__ bool vb_trace(int n, int gv, float &limit, const floa
             int st[D];
             vb_walk<K>(P->group[gs + (mine >> 8 & 63)], P->entry[ats + (mine & 255)] & 255, st);
 #pragma unroll
-            for (int e = 0; e < D; ++e) states[(l0 + lane + 1) * D - 1 - e] = st[e];
+            for (int e = 0; e < D; ++e) states[(l0 + lane + 1) * D - 1 - e] = (uint16_t)st[e];
         }
     }
     if (!near) return true;
@@ -973,7 +1212,7 @@ __device__ __forceinline__ bool vb_trace(int n, int gv, float &limit, const floa
         const uint64_t live = __ballot(lane < m && c < inf && P->cost[e] <= room);
 #pragma unroll
         for (int d = D - 1; d >= 0; --d) {
-            c = vt_err(st[d], x[l * D - 1 - d]) + c;
+            c = vt_err(st[d], (float)x[l * D - 1 - d]) + c;
             v[d] = c;
         }
         bool least = live >> lane & 1;     // of its parent (at the end: of all): the lowest cost, then the lowest state, step by step
@@ -1017,7 +1256,7 @@ __device__ __forceinline__ bool vb_trace(int n, int gv, float &limit, const floa
         vb_walk<K>(P->group[P->groups[l] + (en >> 8)], en & 255, st);
         if (lane == 0) {
 #pragma unroll
-            for (int e = 0; e < D; ++e) states[l * D - 1 - e] = st[e];
+            for (int e = 0; e < D; ++e) states[l * D - 1 - e] = (uint16_t)st[e];
         }
         if (l > 1) take = __builtin_amdgcn_readfirstlane(P->via[P->at[l] + P->child[at]]);
     }
@@ -1027,9 +1266,12 @@ __device__ __forceinline__ bool vb_trace(int n, int gv, float &limit, const floa
 // A wave's memory while it walks back
 struct vb_work {
     vb_pool pool;
-    float x[VT_T], pre[VT_T / VB_NORM + 1];
-    int states[VT_T], start[VB_MOST];
+    float pre[VT_T / VB_NORM + 1];
+    f16 x[VT_T];
+    uint16_t states[VT_T];
+    int start[VB_MOST];
 };
+static_assert(sizeof(vb_work) <= 160 * 1024 / 16, "sixteen on a CU");
 
 // The backtrack of tile part.first + at (one wave): after pass 0 the overlap, after pass 1 the states and values.
 // What bounds it is latency: a chain of STORED levels, each a look into a row of which only the last level's group tells
@@ -1038,15 +1280,24 @@ template <int K>
 __device__ __forceinline__ void vb_backtrack(const float *__restrict__ tiles_in, int64_t ld, const vb_lists &lists,
                                              const vb_part &part, int at, vb_work *W, int32_t *__restrict__ states_out, float *__restrict__ hat_out) {
     using C = vb_cfg<K>;
-    float *const x = W->x, *const pre = W->pre;
-    int *const states = W->states, *const start = W->start;
+    float *const pre = W->pre;
+    f16 *const x = W->x;
+    uint16_t *const states = W->states;
+    int *const start = W->start;
     const int lane = threadIdx.x & 63, pass = part.pass;
     const int64_t tile = __builtin_amdgcn_readfirstlane(lists.order[part.first + at]);
     vb_tile *const mine = part.info + at;
     const int over = pass ? __builtin_amdgcn_readfirstlane(mine->over) : 0;
     if ((uint32_t)over >= (uint32_t)C::G) return;              // left after the first pass
     const int turn = pass ? 0 : VT_T / 2, tie = pass ? over : -1;
-    for (int i = lane; i < VT_T; i += 64) x[i] = (float)(f16)tiles_in[vt_pos(tile, (i + turn) & (VT_T - 1), ld)];
+    float lost = 0.0f;                                         // off the bounds, beside their roundings
+    for (int i = lane; i < VT_T; i += 64) {
+        x[i] = (f16)tiles_in[vt_pos(tile, (i + turn) & (VT_T - 1), ld)];
+        lost += vm_loss((float)x[i]);
+    }
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) lost += __shfl_xor(lost, d, GLQH_WAVE);
+    lost = K == 4 && part.product ? VT_T * VM_FLOOR * 0x1p-10f + lost : VB_LOST;   // (2^-10: a rounding of the least bounds)
     for (int i = lane; i <= VT_T / VB_NORM; i += 64) pre[i] = mine->pre[i];
     const uint16_t *hist = part.rows + (int64_t)at * C::STORED * C::G, *last = hist + (int64_t)(C::STORED - 1) * C::G;
     __builtin_amdgcn_wave_barrier();
@@ -1062,7 +1313,8 @@ __device__ __forceinline__ void vb_backtrack(const float *__restrict__ tiles_in,
         }
         lo = vb_wave_min(lo);
     }
-    float limit = vb_lane((vb_half(lo) + bt) * (1.0f + C::SLACK) + VB_LOST, 0);
+    const float least = vb_lane(vb_half(lo) + bt, 0);
+    float limit = vb_lane(least * (1.0f + C::SLACK) + lost, 0), lower = limit - 0.5f * (limit - least);
     bool good = false;
 #pragma unroll 1
     for (int tries = 0; tries < 4; ++tries) {
@@ -1089,10 +1341,15 @@ __device__ __forceinline__ void vb_backtrack(const float *__restrict__ tiles_in,
             }
         }
         __builtin_amdgcn_wave_barrier();
-        if (n > VB_MOST) break;
         n = __builtin_amdgcn_readfirstlane(n);
-        good = vb_trace<K>(n, lane < n ? start[lane] : 0, limit, x, hist, pre, tie, pass ? VT_T - 1 : VT_T / 2, &W->pool, states);
-        if (good || limit == __builtin_inff()) break;
+        if (n > VB_MOST) limit = __builtin_inff();
+        else good = vb_trace<K>(n, lane < n ? start[lane] : 0, limit, x, hist, pre, tie, pass ? VT_T - 1 : VT_T / 2, &W->pool, states);
+        if (good) break;
+        if (limit == __builtin_inff()) {                       // too many ways for the lists: half the slack may do
+            limit = lower;
+            lower = __builtin_inff();
+        }
+        if (limit == __builtin_inff()) break;
         __builtin_amdgcn_wave_barrier();
     }
     __builtin_amdgcn_wave_barrier();
@@ -1128,6 +1385,14 @@ vb_kernel(const float *__restrict__ tiles_in, int64_t ld, vb_lists lists, vb_par
     } else {
         vb_forward<K, TPW>(tiles_in, ld, lists, forward, blockIdx.x - walkers, gridDim.x - walkers, lds);
     }
+}
+
+// The walk back over tiles that vm_kernel has run forward, a wave a workgroup: as many at a time as the LDS holds
+__global__ void __launch_bounds__(GLQH_WAVE, 4)
+vm_walk_kernel(const float *__restrict__ tiles_in, int64_t ld, vb_lists lists, vb_part back, int32_t *__restrict__ states_out,
+               float *__restrict__ hat_out) {
+    __shared__ vb_work work;
+    if ((int)blockIdx.x < vb_count(back, lists)) vb_backtrack<4>(tiles_in, ld, lists, back, blockIdx.x, &work, states_out, hat_out);
 }
 
 // states (tiles in row-major tile order, 256 steps each) -> packed kernel layout: the chunk of
@@ -1217,20 +1482,30 @@ int acs_launch(const float *cost, const void *x, const float *lut, float *cost_o
 
 // Two batches of tiles take turns: while one walks back, the other runs forward.  A batch is a chip full of pairs (two
 // workgroups a CU); everything is one batch where that leaves none to overlap with.  least: batches of half as many, in the
-// scratch that viterbi_kernel alone takes (16384 tiles 1 GB and 35.5 ms instead of 2 and 32.7 at K = 4, 2 GB and 37.2 instead
+// scratch that viterbi_kernel alone takes (16384 tiles 1 GB and 35.5 ms instead of 4 and 25.7 at K = 4, 2 GB and 37.2 instead
 // of 4 and 38.0 at 3, 38.9 instead of 35.7 at 2).
+//
+// At K = 4 chips full of sixteen tiles a CU come first, through vm_kernel, one after the other, and the rest too where that is
+// VM_FEWEST tiles a CU or more: a part of a chip takes its whole time (3072 tiles 6.2 and 6.0 ms, 4096 8.2 and 6.5).
 struct vb_plan {
     int64_t batch;
     int batches;                           // in flight: 1 or 2
 };
+constexpr int VM_FEWEST = 12;
+template <int K>
+int64_t vm_tiles(int64_t n_tiles, int least) {
+    const int64_t full = VM_TILES * (int64_t)glqh_device_cus(), rest = n_tiles % full;
+    return K != 4 || least ? 0 : rest < VM_FEWEST * (int64_t)glqh_device_cus() ? n_tiles - rest : n_tiles;
+}
 vb_plan vb_plan_of(int64_t n_tiles, int least) {
     const int64_t full = (least ? 2 : 4) * (int64_t)glqh_device_cus();
     return n_tiles <= full ? vb_plan{n_tiles, 1} : vb_plan{full, 2};
 }
 template <int K>
 size_t vb_bytes(int64_t n_tiles, int least) {
-    const vb_plan p = vb_plan_of(n_tiles, least);
-    return (size_t)p.batch * p.batches * (vb_cfg<K>::STORED * vb_cfg<K>::G * 2 + sizeof(vb_tile));
+    const int64_t products = vm_tiles<K>(n_tiles, least), chip = std::min(products, VM_TILES * (int64_t)glqh_device_cus());
+    const vb_plan p = vb_plan_of(n_tiles - products, least);
+    return (size_t)std::max(chip, p.batch * p.batches) * (vb_cfg<K>::STORED * vb_cfg<K>::G * 2 + sizeof(vb_tile));
 }
 
 // The lists, behind everything else (viterbi_kernel's rows take the place of the bounds'), the counts last
@@ -1249,15 +1524,17 @@ int vb_launch(const float *tiles, int64_t n_tiles, int64_t ld, void *scratch, in
     hipLaunchKernelGGL(vb_order_kernel, dim3(1), dim3(1024), 0, stream, (int)n_tiles,
                        8 * glqh_device_cus(), lists);
     GLQH_LAUNCH_CHECK("viterbi lists launch");
-    const vb_plan plan = vb_plan_of(n_tiles, least);
-    const size_t rows = (size_t)plan.batch * C::STORED * C::G;
     const int cus = glqh_device_cus();
+    const int64_t products = vm_tiles<K>(n_tiles, least);
+    const vb_plan plan = vb_plan_of(n_tiles - products, least);
+    const size_t rows = (size_t)plan.batch * C::STORED * C::G;
     auto part = [&](int64_t batch, int pass) {
-        const int64_t first = batch * plan.batch, left = n_tiles - first;
+        const int64_t first = products + batch * plan.batch, left = n_tiles - first;
         const int slab = (int)(batch & 1);
         return vb_part{first, (int)(left <= 0 ? 0 : left < plan.batch ? left : plan.batch), pass, (uint16_t *)scratch + slab * rows,
-                       (vb_tile *)((uint16_t *)scratch + plan.batches * rows) + slab * plan.batch};
+                       (vb_tile *)((uint16_t *)scratch + plan.batches * rows) + slab * plan.batch, false};
     };
+    const vb_part none{0, 0, 0, nullptr, nullptr, false};
     auto launch = [&](const vb_part &forward, const vb_part &back) {
         const int walkers = (back.count + VB_WALK - 1) / VB_WALK;
         // one tile a workgroup while that gives no CU more than two workgroups (512 tiles: 1.58 ms at K = 4, 1.52 at 3); at
@@ -1275,14 +1552,28 @@ int vb_launch(const float *tiles, int64_t n_tiles, int64_t ld, void *scratch, in
         GLQH_LAUNCH_CHECK("viterbi launch");
         return 0;
     };
+    if constexpr (K == 4) {
+        const int64_t chip = std::min(products, VM_TILES * (int64_t)cus);
+        for (int64_t first = 0; first < products; first += chip) {
+            hipLaunchKernelGGL(vb_stop_kernel, dim3(1), dim3(64), 0, stream, first, lists);
+            const int count = (int)std::min(products - first, chip);
+            for (int pass = 0; pass < 2; ++pass) {
+                const vb_part all{first, count, pass, (uint16_t *)scratch, (vb_tile *)((uint16_t *)scratch + chip * C::STORED * C::G), true};
+                hipLaunchKernelGGL(vm_kernel, dim3((count + VM_TILES - 1) / VM_TILES), dim3(VM_THREADS), VM_LDS, stream, tiles, ld, lists, all);
+                hipLaunchKernelGGL(vm_walk_kernel, dim3(count), dim3(GLQH_WAVE), 0, stream, tiles, ld, lists, all, states, hat);
+                if (pass == 0) hipLaunchKernelGGL(vm_stop_kernel, dim3(1), dim3(64), 0, stream, first, count, lists);
+                GLQH_LAUNCH_CHECK("viterbi launch");
+            }
+        }
+    }
     // batches 2i and 2i + 1: F0(a) | F0(b) B0(a) | F1(a) B0(b) | F1(b) B1(a) | F0(a') B1(b) | ...
-    vb_part back{0, 0, 0, nullptr, nullptr};
-    for (int64_t b = 0; b * plan.batch < n_tiles; b += 2) {
-        if (b) hipLaunchKernelGGL(vb_stop_kernel, dim3(1), dim3(64), 0, stream, b * plan.batch, lists);
+    vb_part back = none;
+    for (int64_t b = 0; products + b * plan.batch < n_tiles; b += 2) {
+        if (products + b) hipLaunchKernelGGL(vb_stop_kernel, dim3(1), dim3(64), 0, stream, products + b * plan.batch, lists);
         for (int turn = 0; turn < 4; ++turn) {
             const vb_part forward = part(b + (turn & 1), turn >> 1);
             if (forward.count == 0 || plan.batches == 1) {     // nothing beside it
-                if (launch(vb_part{0, 0, 0, nullptr, nullptr}, back)) return 1;
+                if (launch(none, back)) return 1;
                 back.count = 0;
             }
             if (forward.count == 0) continue;
@@ -1290,7 +1581,7 @@ int vb_launch(const float *tiles, int64_t n_tiles, int64_t ld, void *scratch, in
             back = forward;
         }
     }
-    return launch(vb_part{0, 0, 0, nullptr, nullptr}, back);
+    return launch(none, back);
 }
 
 // a tile a CU is as fast without the bounds' chain of launches (256 tiles, exact / on bounds: 1.38 / 1.62 ms at K = 2,
@@ -1323,6 +1614,8 @@ int vt_set_lds() {
         constexpr int FEW = vb_cfg<K>::FEW;
         if (int rc = set((const void *)vb_kernel<K, FEW>, vb_lds<K, FEW>()) || set((const void *)vb_kernel<K, 2>, vb_lds<K, 2>()))
             return rc;
+        if constexpr (K == 4)
+            if (int rc = set((const void *)vm_kernel, VM_LDS)) return rc;
     }
     return glqh_check_hip(hipFuncSetAttribute((const void *)viterbi_kernel<K>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                               (int)(vt_cfg<K>::ROWS * sizeof(float) * vt_cfg<K>::G)),

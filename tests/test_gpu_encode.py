@@ -462,3 +462,41 @@ def test_viterbi_under_capture():
         torch.cuda.synchronize()
         assert torch.equal(st, _exact_states(X, 4)), turn
         assert torch.equal(hat, lut[st.long()]), turn
+
+
+@pytest.mark.parametrize("n", [3072, 3081, 4396])
+def test_viterbi_by_products_equals_the_exact_search(n):
+    """Calls that fill the chip at K = 4, whose forward pass is matrix products: the smallest of them, a last workgroup with one
+    tile, and a full chip with a rest for the other route; special tiles among them, decoded ones, and some whose best path costs
+    about what the bounds are made for, or more.  A few in a thousand may be left to the exact search, not more."""
+    say("viterbi by products", n)
+    X = _search_tiles(n, n)
+    X[-1] = torch.randn(256, generator=torch.Generator().manual_seed(n)) * 0.9   # the last workgroup's, in order and tried
+    X[100:140] *= torch.linspace(1, 2.4, 40)[:, None]
+    lut = torch.from_numpy(O.lut_3inst().astype(np.float32))
+    X[200:260] = lut[torch.from_numpy(O.trellis_states(O.random_packed(96, 160, 4, seed=4), 96, 160).astype(np.int64))].reshape(60, 256)
+    X[230:260] += torch.randn(30, 256, generator=torch.Generator().manual_seed(1)) * 1e-3
+    states, tried, left = _quantize_counts(X, 4)
+    assert tried > n - 40 and left <= n // 100, (tried, left)
+    ref = _exact_states(X, 4)
+    assert torch.equal(states, ref), (states != ref).any(1).nonzero()[:5]
+
+
+def test_viterbi_by_products_under_capture():
+    """Captured and replayed on other tiles, with eager work between."""
+    from glq_amd import ext
+    say("viterbi by products under capture")
+    n = 3100
+    X = torch.zeros(n, 256, device=DEV)
+    ext.trellis_quantize_tiles(X[:4], 4)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        _, st = ext.trellis_quantize_tiles(X, 4)
+    for turn in range(3):
+        X.copy_(_search_tiles(n, turn))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(st, ext.trellis_quantize_tiles(X, 4)[1]), turn
+    assert torch.equal(st, _exact_states(X.cpu(), 4))
