@@ -115,16 +115,11 @@ e8_tile_kernel(const et_args a) {
 #pragma unroll
     for (int s = 0; s < 3; ++s) rs[s] = f16x2{(f16)a.r[s], (f16)a.r[s]};
 
-    // Workgroups with equal blockIdx % 8 run on one XCD and share its L2: each XCD takes a
-    // contiguous range of the item list, whose fastest index is the row tile, so its CUs read
+    // Each XCD takes a contiguous range of the item list, whose fastest index is the row tile, so its CUs read
     // the same activations at the same time.
     const int nitems = a.TT * a.KS * a.RT;
-    const int per_xcd = (nitems + 7) >> 3;
-    const int xcd = blockIdx.x & 7, bx = blockIdx.x >> 3;
-    const int nbx = ((int)gridDim.x - xcd + 7) >> 3;
-    for (int w = bx; w < per_xcd; w += nbx) {
-        const int item = xcd * per_xcd + w;
-        if (item >= nitems) break;                              // uniform
+    const glqh_share share = glqh_xcd_share(nitems);
+    for (int item = share.first; item < share.end; item += share.step) {
         const int rt = item % a.RT, slot = (item / a.RT) % a.KS, tt0 = item / (a.RT * a.KS);
         const int r0 = rt * ET_ROWS, tok0 = tt0 * (ET_WAVES * 16 * NTW) + wave * 16 * NTW;
         const int ds0 = slot * a.slot_ds, ds1 = min(ds0 + a.slot_ds, nds);
@@ -740,29 +735,26 @@ static int et_plan_for(int NTW, int64_t m_pad, int64_t n_pad, int64_t M, et_plan
     return 1;
 }
 
-// Expected microseconds of a plan, as for the trellis tile kernel: rounds x steps x the time of a step (2.75 us
-// with 512-token tiles, 1.65 with 256: two-stage layers on folded streams, full chip), a last round of at least
-// half, +0.6 x the idle share when a single round leaves CUs idle, and the K slots' fp32 sums written and read
-// at about 4 TB/s.
+// Expected microseconds of a plan, as for the trellis tile kernel: the steps of a round cost what the chip's power allows (1.8 us
+// with all CUs on 512-token tiles, 1.13 on 256: one- and two-stage layers on folded streams) in proportion to the CUs that have a
+// tile, and no less than a step's chain (1.57, 1.02); and the K slots' fp32 sums.
 static double et_plan_cost(const et_plan &p, int64_t m_pad, int64_t M) {
     const int cus = glqh_device_cus();
-    const int64_t items = (int64_t)p.RT * p.TT * p.KS;
-    const int64_t full = items / cus, rem = items % cus;
-    double rounds = (double)full, slow = 1.0;
-    if (full == 0) {
-        rounds = 1.0;
-        slow = 1.0 + 0.6 * (1.0 - (double)items / cus);
-    } else if (rem > 0) {
-        rounds += std::max(0.5, (double)rem / cus);
-    }
-    double t = rounds * p.slot_ds * (p.NTW == 4 ? 2.75 : 1.65) * slow;
-    if (p.KS > 1) t += 2.0 * p.KS * (double)M * (double)m_pad * 4.0 / 4.0e6;
+    const int64_t items = (int64_t)p.RT * p.TT * p.KS, full = items / cus, rem = items % cus;
+    auto step = [&](double share) { return p.NTW == 4 ? std::max(1.57, 1.8 * share) : std::max(1.02, 1.13 * share); };
+    double t = (double)full * step(1.0);
+    if (rem) t += step((double)rem / cus);
+    t *= p.slot_ds;
+    if (p.KS > 1) t += 0.1e-6 * 4 * p.KS * (double)M * (double)m_pad;
     return t;
 }
 
-// Above 256 tokens: 512-token tiles (one- and two-stage layers) unless 256-token tiles are expected to be at
-// least 5 % faster, which they are where row tiles are few (11008 x 11008 at 1024 tokens: 548 -> 384 us,
-// 11008 x 2048: 151 -> 115).  GLQ_ET_NTW forces a tile.
+// Above 256 tokens: 512-token tiles (one- and two-stage layers) unless 256-token tiles are expected to be 3 % faster, which
+// they are where they waste less on padding or need fewer K slots (5120 x 5120 at 768 tokens 74 -> 68 us, the whole call).  Over
+// 72 shapes (2048-14336 rows and columns, 300-4096 tokens) the rule takes the faster one but for 0.02 % of the sum; 512-token
+// tiles throughout lose 0.6 %.  (A step slower by 0.6 of the idle share, which was the second round of glqh_xcd_share's comment, and
+// a last round that counted in proportion, lost 4.8 %: 5120 x 5120 at 2048 tokens 194 -> 149 us, 14336 x 4096 at 512 97 -> 84.)
+// GLQ_ET_NTW forces a tile.
 int et_make_plan(int64_t m_pad, int64_t n_pad, int64_t M, int nstages, et_plan *p) {
     if (M < 1 || m_pad < 1 || n_pad < 256 || (n_pad & 255) || M > ((int64_t)1 << 22) || m_pad > ((int64_t)1 << 24))
         return 0;
@@ -772,7 +764,7 @@ int et_make_plan(int64_t m_pad, int64_t n_pad, int64_t M, int nstages, et_plan *
     if (top < 4 || forced) return 1;
     et_plan p2;
     et_plan_for(2, m_pad, n_pad, M, &p2);
-    if (et_plan_cost(p2, m_pad, M) < 0.95 * et_plan_cost(*p, m_pad, M)) *p = p2;
+    if (et_plan_cost(p2, m_pad, M) < 0.97 * et_plan_cost(*p, m_pad, M)) *p = p2;
     return 1;
 }
 

@@ -220,12 +220,8 @@ __device__ __forceinline__ void tr_tile_body(const tt_args &a, const tt_group &g
     const int RT = HALF ? 2 * a.half_rt : a.RT;
     int nitems = a.TT * a.KS * RT;
     if constexpr (MOE) nitems = *mo.n_tiles * a.RT * a.TT;      // one K slot; TT = workgroup tiles per run
-    const int per_xcd = (nitems + 7) >> 3;
-    const int xcd = blockIdx.x & 7, bx = blockIdx.x >> 3;
-    const int nbx = ((int)gridDim.x - xcd + 7) >> 3;
-    for (int w = bx; w < per_xcd; w += nbx) {
-        const int item = xcd * per_xcd + w;
-        if (item >= nitems) break;                              // uniform
+    const glqh_share share = glqh_xcd_share(nitems);
+    for (int item = share.first; item < share.end; item += share.step) {
         const int slot = (item / RT) % a.KS, tt0 = item / (RT * a.KS);
         int rt = HALF ? a.RT + (item % RT >> 1) : a.rt0 + item % RT;   // row tile of its layer
         const int unit = HALF ? item % RT & 1 : dw >> 2;        // block pair of the row tile that this wave decodes
@@ -850,48 +846,47 @@ void tt_plan_for(int NTW, int64_t m, int64_t k, int64_t M, tt_plan *p) {
     p->grid = (int)(items < cus ? items : cus);
 }
 
-// Microseconds a plan is expected to take: rounds of workgroups x steps x the time of a step (2.26 us with
-// 512-token tiles, 1.7 with 256), a last round that counts at least half, a step that is slower when a single
-// round leaves CUs idle (+ 0.6 x the idle share: 172 workgroups on 256 CUs take 2.75 / 2.0 us per step, measured),
-// and what K slots cost on top (their sums, esz bytes each, written and read again at about 4 TB/s).
-double tt_plan_cost(const tt_plan &p, int64_t m, int64_t M, int esz) {
+bool tt_split_roles(const tt_plan &p, int min_steps);
+int tt_rest(const tt_plan &p);
+
+// Microseconds a plan for more than 256 tokens is expected to take, but for what all plans share.  Steps of a round cost what
+// the chip's power allows (1.76 us with all CUs on 512-token tiles, 1.03 on 256) in proportion to the CUs that have a tile, and
+// no less than a step's chain (1.32, 0.82); a last round on few of them may run as half tiles (0.53 us a step) or, of a layer
+// on its own, as 256-token tiles; K slots add their sums, 3 bytes each (between fp16 and fp32: the K-slot query and the launch
+// must arrive at the same plan, whatever the width the sums leave with).
+double tt_plan_cost(const tt_plan &p, int64_t m, int64_t M, bool alone) {
     const int cus = glqh_device_cus();
-    const int64_t items = (int64_t)p.RT * p.TT * p.KS;
-    const int64_t full = items / cus, rem = items % cus;
-    double rounds = (double)full, slow = 1.0;
-    if (full == 0) {
-        rounds = 1.0;
-        slow = 1.0 + 0.6 * (1.0 - (double)items / cus);
-    } else if (rem > 0) {
-        rounds += std::max(0.5, (double)rem / cus);
+    const int64_t items = (int64_t)p.RT * p.TT * p.KS, full = items / cus, rem = items % cus;
+    auto step = [&](int ntw, double share) { return ntw == 4 ? std::max(1.32, 1.76 * share) : std::max(0.82, 1.03 * share); };
+    double t = (double)full * step(p.NTW, 1.0);
+    if (rem) {
+        double last = step(p.NTW, (double)rem / cus);
+        if (full && p.KS == 1 && p.NTW == 4 && alone && 2 * rem <= cus)
+            last = step(2, std::min(1.0, (double)((rem + p.TT - 1) / p.TT * ((M + 255) / 256)) / cus));
+        else if (full && p.NTW == 2 && tt_split_roles(p, alone ? 16 : 8) && tt_rest(p) > 0)
+            last = 0.53;
+        t += last;
     }
-    const double step = p.NTW == 4 ? 2.26 : p.NTW == 2 ? 1.7 : 1.3;
-    double t = rounds * p.slot_ds * step * slow;
-    if (p.KS > 1) t += 2.0 * p.KS * (double)M * (double)m * esz / 4.0e6;
+    t *= p.slot_ds;
+    if (p.KS > 1) t += 0.08e-6 * 3 * p.KS * (double)M * (double)m;
     return t;
 }
 
-// Up to 256 tokens the tile follows the token count; above, 512-token tiles unless 256-token tiles are expected
-// to be at least 5 % faster: few row tiles (small layers, a few hundred tokens) fill the chip with neither, and
-// the smaller tile then needs fewer K slots or leaves a shorter last round (2048 x 2048 at 2048 tokens: 4 x 4
-// tiles x 2 slots -> 8 x 4 tiles x 1 slot, 73 -> 58 us; 11008 x 11008 at 1024 tokens: 172 tiles in one round ->
-// 344 in two short ones, 474 -> 366 us).  The model is rough: on a sweep of 15 shapes (512..14336 rows x
-// 2048..11008 columns) x 512..4096 tokens through the matmul entry it ends within 3 % of the faster tile in 48 of
-// 60 cases, 25 % off at worst (14336 x 2048 at 512 tokens, a gain it misses), 3 % below 512-token tiles everywhere
-// in total; the seven linears of a 3B-shape layer: 505 -> 444 us at 1024 tokens.  GLQ_TT_NTW forces a tile
-// above 256 tokens.
+// Up to 256 tokens the tile follows the token count; above, 512-token tiles unless 256-token tiles are expected to be 3 %
+// faster: where they waste less on padding (2 x 14336 rows x 4096 columns at 768 tokens 261 -> 236 us, the whole call), need
+// fewer K slots (2048 x 2048 at 2048 tokens 73 -> 58) or leave a shorter last round.  Over 70 shapes (fused q/k/v and gate/up,
+// layers of 2048-14336 rows and columns; 300-4096 tokens) the rule takes the faster one but for 0.3 % of the sum; 512-token tiles
+// throughout lose 1 % of it.  GLQ_TT_NTW forces a tile above 256 tokens.
 // max_ntw = 2: a stacked layer decoded into one operand (two streams' records and temporaries do not fit beside the
 // accumulators of a 512-token tile).
-void tt_make_plan(int64_t m, int64_t k, int64_t M, tt_plan *p, int max_ntw = 4) {
+void tt_make_plan(int64_t m, int64_t k, int64_t M, tt_plan *p, int max_ntw = 4, bool alone = true) {
     const int top = std::min(tt_ntw(M), max_ntw);
     tt_plan_for(top, m, k, M, p);
     static const bool forced = getenv("GLQ_TT_NTW") != nullptr;
     if (top < 4 || forced) return;
     tt_plan p2;
     tt_plan_for(2, m, k, M, &p2);
-    // (3 bytes per sum, between fp16 and fp32: the K-slot query and the launch must arrive at the same plan,
-    // whatever the width the sums leave with)
-    if (tt_plan_cost(p2, m, M, 3) < 0.95 * tt_plan_cost(*p, m, M, 3)) *p = p2;
+    if (tt_plan_cost(p2, m, M, alone) < 0.97 * tt_plan_cost(*p, m, M, alone)) *p = p2;
 }
 
 // Tiles of up to 256 tokens run with decoding and multiplying waves (the tr_tile_*_pc_kernel forms) when a K
@@ -912,15 +907,15 @@ bool tt_split_roles(const tt_plan &p, int min_steps) {
 // The last round of 256-token tiles of decoding and multiplying waves (slots of min_steps steps and more): where it would
 // run on at most half of the CUs, its row tiles become tiles of 64 rows in the same launch, twice as many: they end in one
 // round (with more than half of the CUs taken they would need two, each nine tenths of the one they replace).
-void tt_halve_last_round(const tt_plan &p, int min_steps, tt_args *a) {
-    a->half_rt = 0;
-    if (p.NTW != 2 || !tt_split_roles(p, min_steps) || p.KS != 1) return;
+int tt_rest(const tt_plan &p) {                                // row tiles of such a round, 0: none
     const int64_t cus = glqh_device_cus(), rounds = (int64_t)p.RT * p.TT / cus;
-    if (rounds < 1) return;
-    const int whole = (int)(rounds * cus / p.TT), rest = p.RT - whole;
-    if (rest <= 0 || 2 * (int64_t)rest * p.TT > cus) return;
-    a->RT = whole;
-    a->half_rt = rest;
+    if (p.KS != 1 || rounds < 1) return 0;
+    const int rest = p.RT - (int)(rounds * cus / p.TT);
+    return rest > 0 && 2 * (int64_t)rest * p.TT <= cus ? rest : 0;
+}
+void tt_halve_last_round(const tt_plan &p, int min_steps, tt_args *a) {
+    a->half_rt = p.NTW == 2 && tt_split_roles(p, min_steps) ? tt_rest(p) : 0;
+    a->RT = p.RT - a->half_rt;
 }
 
 template <int R, int NTW>
@@ -1125,7 +1120,7 @@ namespace {
 void tt_make_group_plan(const int64_t *m, int n_layers, int64_t k, int64_t M, int two_stage, tt_plan *p) {
     int64_t rt = 0;
     for (int l = 0; l < n_layers; ++l) rt += (m[l] + TT_ROWS - 1) / TT_ROWS;
-    tt_make_plan(TT_ROWS * rt, k, M, p, two_stage ? 2 : 4);     // same rule, on the row tiles of all layers
+    tt_make_plan(TT_ROWS * rt, k, M, p, two_stage ? 2 : 4, false);   // same rule, on the row tiles of all layers
 }
 
 #define GLQH_TTG(...)                                                                                      \

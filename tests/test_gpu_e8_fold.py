@@ -181,6 +181,12 @@ def test_groups_of_four_steps_on_folded_streams(ext, m, n, B, stages):
     test_many_token_products_on_folded_streams_equal_products_on_indices(ext, m, n, B, stages)
 
 
+@pytest.mark.parametrize("m,n,B,stages", [(100, 512, 300, 2), (1376, 512, 300, 1), (5500, 256, 600, 2), (11008, 512, 600, 2), (1300, 768, 150, 3)])
+def test_tiles_in_uneven_shares_on_folded_streams(ext, m, n, B, stages):
+    """Tiles that the XCDs cannot share evenly: 1, 11, 86 and 172 of 512 tokens, 11 of 256 in K slots."""
+    test_many_token_products_on_folded_streams_equal_products_on_indices(ext, m, n, B, stages)
+
+
 def test_fused_linear_on_folded_streams_and_under_capture(ext):
     """The forward path only looks the folded streams up.  A layer that was never prepared runs on its
     indices -- also under capture, with a warning -- and makes nothing; after `e8_prepare` a captured

@@ -163,6 +163,14 @@ def test_matmul_last_round_behind_512_token_tiles(ext, m, n, B, K):
     test_matmul_last_round_of_half_tiles(ext, m, n, B, K)
 
 
+@pytest.mark.parametrize("m,n,B,K", [(96, 512, 300, 4), (1376, 512, 300, 2), (5504, 512, 600, 4), (11008, 1024, 700, 3),
+                                     (22016 - 96, 1024, 760, 4)])
+def test_matmul_tiles_in_uneven_shares(ext, m, n, B, K):
+    """Tiles that the XCDs cannot share evenly: 1, 11, 86 and 172 of 512 tokens, and three 256-token tiles with a last round of
+    half tiles.  The same bound."""
+    test_matmul_last_round_of_half_tiles(ext, m, n, B, K)
+
+
 @pytest.mark.parametrize("m,n,B,K2", [(32768 + 32, 512, 200, 2), (32768 + 224, 576, 130, 1), (32768 + 96, 512, 129, 4),
                                       (10976, 1024, 999, 3)])
 def test_two_stage_last_round_of_half_tiles(ext, m, n, B, K2):
