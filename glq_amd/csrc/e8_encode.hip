@@ -94,14 +94,26 @@ e8_quantize_kernel(const float *__restrict__ x, const float *__restrict__ table,
 // 524288 vectors of N(0, 1): 12.06 ms (walk) -> 98 us (points of norm 12 on the matrix cores, all 8655 rows for
 // every vector they may win) -> 34 us (points in reach only; 38 MB in and out, 8 us) -> 33.2 us with the table read
 // by every call (es_index_kernel 4 us; 250 -> 52 us where the table is new); 960 vectors 12.7 ms -> 13.4 ->
-// 17.3 us: three dependent launches.
+// 17.3 us: three dependent launches.  Then the lists, which a workgroup had filled an addition at a time and walked level
+// by level, a barrier each: with the first points and their children from the 25 known orbits, counted before they are placed,
+// and the rest to each wave alone, 33.5 -> 32 us, 131072 vectors 22.6 -> 19.7, 960 18.2 -> 16.7; of scale 2, where nearly all
+// vectors have them, 131072 vectors 110 -> 50 us, and of scale 20, 200 -> 176.  Of 32 us the kernel takes 28: half of that
+// the first pass (bound by VALU instructions), a quarter the first points, the rest trips through the lists and the table.
+// (Of scale 0.5, with a vector or two for a workgroup to list, 524288 take 21.6 us, not 21.)
 constexpr int ES_THREADS = 256;
 constexpr int ES_PLACES = 117361;                              // E8 points of norm up to 12
 constexpr int ES_FULL = GLQH_E8_SHELL_MIN_ROWS;                // of norm up to 10: all of them are rows of the table
 enum { ES_SHARED, ES_IN_FULL, ES_WALKS, ES_FOUND };            // two rows of one place; rows of the full shells; vectors to walk
 constexpr int ES_CHECKS = 128;                                 // workgroups, at least, that look for rows of one place
-constexpr int ES_CHUNK = 128;                                  // vectors whose points are listed together,
-constexpr int ES_LIST = 3072;                                  // and the points: 2.5 each at unit scale, up to 106 far out
+constexpr int ES_CHUNK = 128;                                  // vectors whose points are listed together, fewer far out,
+constexpr int ES_LIST = 3584;                                  // and the points: 3.6 each at unit scale, up to 106 far out
+constexpr int ES_GROWN = ES_LIST - 1200;                       // (four workgroups' lists fill a CU's LDS); the nearest points
+constexpr int ES_WAVE = ES_GROWN / 4;                          // of the orbits behind this, the others in a part for each wave
+// Points in wait from which a wave takes a lane for each rather than eight: times of 16, 24, 40, 64 are 149, 149, 152, 169 us
+// at 131072 vectors of scale 4 and level at unit scale.
+constexpr int ES_MANY = 24;
+static_assert(ES_THREADS == 2 * ES_CHUNK && 16 * 25 <= ES_LIST - ES_GROWN && 16 * 25 * 8 <= 2 * ES_GROWN,
+              "two threads a vector; the orbits of the fewest vectors fit, and most of their points' children");
 constexpr int ES_SPLIT = 128;                                  // parts of the table in the exact walk
 
 // Places.  A point is two halves of four coordinates (2 c + 6 in a nibble each).  Halves are integers or half-integers
@@ -225,12 +237,6 @@ struct es_args {
     unsigned long long *walk_key;                              // N
 };
 
-// row of a point (2 c + 6 in a nibble per coordinate), -1 if the table does not hold it: its place is then unset
-__device__ __forceinline__ int es_row(const es_args &a, uint32_t code) {
-    const int place = es_place(code), row = a.row_at[place];
-    return (uint32_t)row < (uint32_t)a.n_entries && a.place_of[row] == place ? row : -1;
-}
-
 __device__ __forceinline__ void es_store(const es_args &a, int64_t v, int row) {
     a.idx_out[v] = row;
     if (a.dec_out) {
@@ -340,7 +346,8 @@ __device__ __forceinline__ void es_orbits_12(const float y[8], F f) {
 }
 
 // f(gap, child) for the children of point p in its orbit's tree whose distance is at most `room` more than p's: a
-// simple reflection that takes p further away, and is the first to bring the child back.
+// simple reflection that takes p further away, and is the first to bring the child back.  (Of points known at compile time little
+// but the comparisons with `room` is left.)
 template <typename F>
 __device__ __forceinline__ void es_children(uint32_t p, const float y[8], float room, F f) {
     int q[8];
@@ -361,15 +368,64 @@ __device__ __forceinline__ void es_children(uint32_t p, const float y[8], float 
         f(gap, (p & 0x00FFFFFFu) | (uint32_t)(6 - q[7]) << 24 | (uint32_t)(6 - q[6]) << 28);
 }
 
+// The same with eight lanes to a point, lane i: whether reflection i (7: of the last two places, with their signs) makes a child, and how
+// much further away it is.  ya, yb: y of the two places.
+__device__ __forceinline__ bool es_child(uint32_t p, int i, float ya, float yb, float room, float &gap) {
+    const int k = i < 7 ? i : 6, qa = es_q(p, k), qb = es_q(p, k + 1), qp = es_q(p, i < 7 ? max(i - 1, 0) : 5);
+    // the pairs ahead of (i - 1, i) descend
+    const uint32_t descends = (uint32_t)(__ballot(qa >= qb) >> (threadIdx.x & 56)) & 255u;
+    const uint32_t ahead = i == 7 ? 31u : (1u << max(i - 1, 0)) - 1u;
+    bool child = (descends & ahead) == ahead;
+    if (i < 7) {
+        gap = (float)(qa - qb) * (ya - yb);
+        child = child && qa > qb && (i == 0 || qp >= qb);
+    } else {
+        gap = (float)(qa + qb) * (ya + yb);
+        child = child && qp >= -qb && qa >= qb && qa + qb > 0;
+    }
+    return child && gap <= room;
+}
+__device__ __forceinline__ uint32_t es_reflect(uint32_t p, int i) {
+    if (i == 7) return (p & 0x00FFFFFFu) | (uint32_t)(6 - es_q(p, 7)) << 24 | (uint32_t)(6 - es_q(p, 6)) << 28;
+    const uint32_t d = ((p >> (4 * i)) ^ (p >> (4 * i + 4))) & 15u;
+    return p ^ (d << (4 * i)) ^ (d << (4 * i + 4));
+}
+
+// The lanes' counts up to this one's, and of all of them.  The whole wave calls.
+__device__ __forceinline__ int es_before(int count, int &total) {
+    int sum = count;
+    sum += __builtin_amdgcn_update_dpp(0, sum, 0x111, 0xf, 0xf, true);   // row_shr:1, 2, 4, 8
+    sum += __builtin_amdgcn_update_dpp(0, sum, 0x112, 0xf, 0xf, true);
+    sum += __builtin_amdgcn_update_dpp(0, sum, 0x114, 0xf, 0xf, true);
+    sum += __builtin_amdgcn_update_dpp(0, sum, 0x118, 0xf, 0xf, true);
+    sum += __builtin_amdgcn_update_dpp(0, sum, 0x142, 0xa, 0xf, false);  // row_bcast:15, 31
+    sum += __builtin_amdgcn_update_dpp(0, sum, 0x143, 0xc, 0xf, false);
+    total = __builtin_amdgcn_readlane(sum, 63);
+    return sum - count;
+}
+// Places for `count` entries of each lane in a list of the workgroup, in one addition to its length: this lane's first one.  The
+// whole wave calls.  (An addition for each
+// orbit would be 25 trips to LDS, one after the other.)
+__device__ __forceinline__ int es_places(int count, int *length) {
+    int total;
+    const int before = es_before(count, total);
+    if (total == 0) return 0;
+    int at = 0;
+    if ((threadIdx.x & 63) == 0) at = atomicAdd(length, total);
+    return __builtin_amdgcn_readfirstlane(at) + before;
+}
+
 template <int V>                                               // vectors of a workgroup
 __global__ void __launch_bounds__(ES_THREADS, 4)
 e8_shell_kernel(const es_args a) {
-    __shared__ int n_flag, n_walk, n_list;
+    __shared__ int n_flag, n_walk, n_seed, n_child, n_grown[4], n_left[4];
     __shared__ unsigned short flags[V];
-    __shared__ uint32_t list_p[ES_LIST], sk[ES_CHUNK][8];
+    __shared__ uint32_t list_p[ES_LIST], sk[8][ES_CHUNK];
     __shared__ unsigned char list_j[ES_LIST];
     __shared__ float list_room[ES_LIST];
-    __shared__ uint32_t s_signs[ES_CHUNK];                     // bit 8: flip, bit 9: left to the walk
+    __shared__ uint32_t s_signs[ES_CHUNK];                     // bit 8: flip
+    __shared__ unsigned char s_walk[ES_CHUNK];                 // left to the walk
+    __shared__ float s_margin[ES_CHUNK];
     __shared__ unsigned long long best[ES_CHUNK];
     const int tid = threadIdx.x;
     const int64_t v0 = (int64_t)blockIdx.x * V;
@@ -418,7 +474,17 @@ e8_shell_kernel(const es_args a) {
         for (int r = 0; r < 7; ++r)
             if (q[r] != q[r + 1]) gap = __builtin_fminf(gap, (float)(q[r] - q[r + 1]) * (s.y[r] - s.y[r + 1]));
         if (q[6] + q[7] != 0) gap = __builtin_fminf(gap, (float)(q[6] + q[7]) * (s.y[6] + s.y[7]));
-        if (!(gap > s.margin)) { flags[atomicAdd(&n_flag, 1)] = (unsigned short)local; continue; }
+        if (!(gap > s.margin)) {
+            const int at = atomicAdd(&n_flag, 1);
+            flags[at] = (unsigned short)local;
+            if (at < ES_CHUNK) {                               // the first chunk's are at hand
+#pragma unroll
+                for (int r = 0; r < 8; ++r) sk[r][at] = s.k[r];
+                s_signs[at] = s.signs | (s.flip ? 256u : 0u);
+                s_margin[at] = s.margin;
+            }
+            continue;
+        }
         const uint32_t code = es_code(p, s.k, s.signs, s.flip);
         a.idx_out[v] = a.row_at[es_place(code)];               // a row of the table, of norm up to 10
         if (a.dec_out) {
@@ -434,79 +500,212 @@ e8_shell_kernel(const es_args a) {
     }
     __syncthreads();
     const int nf = n_flag;
-    // 128 vectors at a time, or 32 where many have points in reach: those have many each
-    const int step = nf * 2 < V ? ES_CHUNK : 32;
-    for (int c0 = 0; c0 < nf; c0 += step) {
+    // As many vectors at a time as the lists hold the first points of, with room for as many again.  (32 where more than half are
+    // here and 128 otherwise, without the second try below: 1.5 and 2 times as long at scale 4 and 2.)
+    int step = ES_CHUNK;
+    for (int c0 = 0; c0 < nf;) {
         const int nc = nf - c0 < step ? nf - c0 : step;
-        if (tid == 0) n_list = 0;
+        if (tid == 0) n_seed = n_child = 0;
+        if (tid < ES_CHUNK) s_walk[tid] = 0;
         __syncthreads();
-        auto push = [&](uint32_t p, int j, float room) {
-            const int at = atomicAdd(&n_list, 1);
-            if (at < ES_LIST) {
+        auto put = [&](int at, int end, uint32_t p, int j, float room) {
+            if (at < end) {
                 list_p[at] = p;
                 list_j[at] = (unsigned char)j;
                 list_room[at] = room;
-            } else atomicOr(&s_signs[j], 512u);
+            } else s_walk[j] = 1;
         };
-        if (tid < nc) {                                        // the nearest points of the orbits in reach
-            float xv[8];
-            es_load(a.x, v0 + flags[c0 + tid], xv);
-            es_vec s;
-            es_sort(xv, s);
+        // the nearest points of the orbits in reach, and their children: half of the orbits each to two threads of a vector
+        const int mine = tid & (ES_CHUNK - 1), half = __builtin_amdgcn_readfirstlane(tid / ES_CHUNK);
+        if ((mine & ~63) < nc) {
+            const bool on = mine < nc;
+            const int slot = on ? mine : 0;
+            float y[8], margin;
+            if (c0 == 0) {
 #pragma unroll
-            for (int r = 0; r < 8; ++r) sk[tid][r] = s.k[r];
-            s_signs[tid] = s.signs | (s.flip ? 256u : 0u);
-            best[tid] = ~0ull;
-            float b1 = __builtin_inff();
-            es_orbits(s.y, [&](float d, uint32_t) { b1 = __builtin_fminf(b1, d); });
-            const float reach = b1 + s.margin;
-            auto seed = [&](float d, uint32_t code) { if (d <= reach) push(code, tid, reach - d); };
-            es_orbits(s.y, seed);
-            es_orbits_12(s.y, seed);
+                for (int r = 0; r < 8; ++r) y[r] = __builtin_bit_cast(float, sk[r][slot] & ~7u);
+                if (s_signs[slot] & 256u) y[7] = -y[7];
+                margin = s_margin[slot];
+            } else {
+                float xv[8];
+                es_load(a.x, v0 + flags[c0 + slot], xv);
+                es_vec s;
+                es_sort(xv, s);
+                if (on && half == 0) {
+#pragma unroll
+                    for (int r = 0; r < 8; ++r) sk[r][mine] = s.k[r];
+                    s_signs[mine] = s.signs | (s.flip ? 256u : 0u);
+                }
+#pragma unroll
+                for (int r = 0; r < 8; ++r) y[r] = s.y[r];
+                margin = s.margin;
+            }
+            if (on && half == 0) best[mine] = ~0ull;
+            float b1 = __builtin_inff(), room[25];
+            int o = 0;
+            es_orbits(y, [&](float v, uint32_t) {
+                b1 = __builtin_fminf(b1, v);
+                room[o++] = v;
+            });
+            es_orbits_12(y, [&](float v, uint32_t) { room[o++] = v; });
+            const float reach = b1 + margin;
+#pragma unroll
+            for (o = 0; o < 25; ++o) room[o] = on ? reach - room[o] : -1.0f;
+            int seeds = 0, children = 0;
+            o = 0;
+            auto count = [&](float, uint32_t code) {
+                if (o / 13 == half) {
+                    seeds += room[o] >= 0.0f;
+                    es_children(code, y, room[o], [&](float, uint32_t) { ++children; });
+                }
+                ++o;
+            };
+            es_orbits(y, count);
+            es_orbits_12(y, count);
+            int at = ES_GROWN + es_places(seeds, &n_seed), to = es_places(children, &n_child);
+            if (step == 16 || __ballot(at + seeds > ES_LIST || to + children > ES_GROWN / 2) == 0) {
+                o = 0;
+                auto list = [&](float, uint32_t code) {
+                    if (o / 13 == half) {
+                        if (room[o] >= 0.0f) put(at++, ES_LIST, code, mine, 0.0f);
+                        es_children(code, y, room[o], [&](float gap, uint32_t child) {   // dealt out to the waves
+                            put((to & 3) * ES_WAVE + (to >> 2), ((to & 3) + 1) * ES_WAVE, child, mine, room[o] - gap);
+                            ++to;
+                        });
+                    }
+                    ++o;
+                };
+                es_orbits(y, list);
+                es_orbits_12(y, list);
+            }
         }
         __syncthreads();
-        for (int done = 0, n = n_list < ES_LIST ? n_list : ES_LIST; done < n;) {     // level by level
+        if (step > 16 && (n_seed > ES_LIST - ES_GROWN || n_child > ES_GROWN / 2)) {
+            int of = 1;                                        // too many for the lists: again with fewer vectors
+            do of *= 2;
+            while (step > 16 * of && (n_seed > of * (ES_LIST - ES_GROWN) || n_child > of * (ES_GROWN / 2)));
+            step /= of;
             __syncthreads();
-            for (int e = done + tid; e < n; e += ES_THREADS) {
-                const int j = list_j[e];
-                const float room = list_room[e];
-                float y[8];
-#pragma unroll
-                for (int r = 0; r < 8; ++r) y[r] = __builtin_bit_cast(float, sk[j][r] & ~7u);
-                if (s_signs[j] & 256u) y[7] = -y[7];
-                es_children(list_p[e], y, room, [&](float gap, uint32_t child) { push(child, j, room - gap); });
-            }
-            __syncthreads();
-            done = n;
-            n = n_list < ES_LIST ? n_list : ES_LIST;
+            continue;
         }
-        const int n = n_list < ES_LIST ? n_list : ES_LIST;
-        for (int e = tid; e < n; e += ES_THREADS) {
-            const int j = list_j[e];
-            uint32_t k[8];
+        const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), first = wave * ES_WAVE;
+        int n = min((n_child + 3 - wave) >> 2, ES_WAVE), done = 0, seeds = min(n_seed, ES_LIST - ES_GROWN);
+        for (;;) {
+            // a wave's own points, with no wait for the others, until none is added or its part of the list is full: a lane
+            // each while there are many, eight lanes each when there are few
+            while (done < n) {
+                if (n - done >= ES_MANY) {
+                    // the last added ones first where the list fills up, so that fewer wait
+                    const bool last = n > ES_WAVE / 2 && n - done >= 128;
+                    const int at = (last ? n - 64 : done) + (tid & 63), e = first + min(at, n - 1), j = list_j[e];
+                    const float room = at < n ? list_room[e] : -1.0f;
+                    const uint32_t p = list_p[e];
+                    if (last) {                                // they change places with the longest waiting
+                        const int with = first + done + (tid & 63);
+                        const uint32_t wp = list_p[with];
+                        const unsigned char wj = list_j[with];
+                        const float wr = list_room[with];
+                        list_p[with] = p;
+                        list_j[with] = (unsigned char)j;
+                        list_room[with] = room;
+                        list_p[e] = wp;
+                        list_j[e] = wj;
+                        list_room[e] = wr;
+                    }
+                    float y[8];
 #pragma unroll
-            for (int r = 0; r < 8; ++r) k[r] = sk[j][r];
-            float xv[8], c[8];
-            es_load(a.x, v0 + flags[c0 + j], xv);
-            const uint32_t code = es_code(list_p[e], k, s_signs[j], (s_signs[j] >> 8) & 1u);
-            const int row = es_row(a, code);
-            if (row < 0) continue;
-            int n4 = 0;
-#pragma unroll
-            for (int d = 0; d < 8; ++d) {
-                const int q = es_q(code, d);
-                c[d] = 0.5f * (float)q;
-                n4 += q * q;
+                    for (int r = 0; r < 8; ++r) y[r] = __builtin_bit_cast(float, sk[r][j] & ~7u);
+                    if (s_signs[j] & 256u) y[7] = -y[7];
+                    int children = 0, total;
+                    es_children(p, y, room, [&](float, uint32_t) { ++children; });
+                    int to = first + n + es_before(children, total);
+                    if (n + total > ES_WAVE && done > 0) break;
+                    es_children(p, y, room, [&](float gap, uint32_t child) { put(to++, first + ES_WAVE, child, j, room - gap); });
+                    done = min(done + 64, n);
+                    n = min(n + total, ES_WAVE);
+                    __builtin_amdgcn_wave_barrier();
+                    continue;
+                }
+                const int i = tid & 7, k = i < 7 ? i : 6, at = done + (tid >> 3 & 7), e = first + min(at, n - 1), j = list_j[e];
+                const float room = list_room[e];
+                const uint32_t p = list_p[e], kb = sk[k + 1][j] & ~7u;
+                const float ya = __builtin_bit_cast(float, sk[k][j] & ~7u);
+                const float yb = __builtin_bit_cast(float, k == 6 && (s_signs[j] & 256u) ? kb ^ 0x80000000u : kb);
+                float gap;
+                const bool child = es_child(p, i, ya, yb, room, gap) && at < n;
+                const unsigned long long all = __ballot(child);
+                if (n + __builtin_popcountll(all) > ES_WAVE && done > 0) break;
+                const int to = n + __builtin_amdgcn_mbcnt_hi((uint32_t)(all >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)all, 0));
+                if (child) put(first + to, first + ES_WAVE, es_reflect(p, i), j, room - gap);
+                done = min(done + 8, n);
+                n = min(n + __builtin_popcountll(all), ES_WAVE);
+                __builtin_amdgcn_wave_barrier();
             }
-            atomicMin(&best[j], es_key(es_dist(xv, c, 0.25f * (float)n4), row));
+            if ((tid & 63) == 0) {
+                n_grown[wave] = done;
+                n_left[wave] = n - done;
+            }
+            __syncthreads();
+            // the points that the table holds, by the walk's arithmetic, two at a time: three trips to memory each
+            const int g0 = n_grown[0], g1 = g0 + n_grown[1], g2 = g1 + n_grown[2], g3 = g2 + n_grown[3];
+            const int some = g3 + seeds;
+            for (int q0 = tid; q0 < some; q0 += 2 * ES_THREADS) {
+                int j[2], row[2];
+                uint32_t code[2];
+                float xv[2][8];
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    const int q = min(q0 + u * ES_THREADS, some - 1);
+                    const int e = q < g0 ? q : q < g1 ? ES_WAVE + q - g0 : q < g2 ? 2 * ES_WAVE + q - g1 : q < g3 ? 3 * ES_WAVE + q - g2 : ES_GROWN + q - g3;
+                    j[u] = list_j[e];
+                    es_load(a.x, v0 + flags[c0 + j[u]], xv[u]);
+                    uint32_t k[8];
+#pragma unroll
+                    for (int r = 0; r < 8; ++r) k[r] = sk[r][j[u]];
+                    code[u] = es_code(list_p[e], k, s_signs[j[u]], (s_signs[j[u]] >> 8) & 1u);
+                }
+                int place[2];
+#pragma unroll
+                for (int u = 0; u < 2; ++u) place[u] = es_place(code[u]);
+#pragma unroll
+                for (int u = 0; u < 2; ++u) row[u] = a.row_at[place[u]];
+#pragma unroll
+                for (int u = 0; u < 2; ++u)                        // not held: the place is not set
+                    if ((uint32_t)row[u] >= (uint32_t)a.n_entries || a.place_of[row[u]] != place[u]) row[u] = -1;
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    if (row[u] < 0 || q0 + u * ES_THREADS >= some) continue;
+                    float c[8];
+                    int n4 = 0;
+#pragma unroll
+                    for (int d = 0; d < 8; ++d) {
+                        const int q = es_q(code[u], d);
+                        c[d] = 0.5f * (float)q;
+                        n4 += q * q;
+                    }
+                    atomicMin(&best[j[u]], es_key(es_dist(xv[u], c, 0.25f * (float)n4), row[u]));
+                }
+            }
+            if ((n_left[0] | n_left[1] | n_left[2] | n_left[3]) == 0) break;
+            __syncthreads();
+            // those that are not tried for children yet go to the front
+            for (int e = tid & 63; e < n - done; e += 64) {
+                list_p[first + e] = list_p[first + done + e];
+                list_j[first + e] = list_j[first + done + e];
+                list_room[first + e] = list_room[first + done + e];
+            }
+            __builtin_amdgcn_wave_barrier();
+            n -= done;
+            done = seeds = 0;
         }
         __syncthreads();
         if (tid < nc) {
             const int local = flags[c0 + tid];
-            if (s_signs[tid] & 512u) walk(local);
+            if (s_walk[tid]) walk(local);
             else if (best[tid] != ~0ull) es_store(a, v0 + local, (int)(uint32_t)best[tid]);   // none: not the shell table
         }
         __syncthreads();
+        c0 += step;
     }
     if (tid == 0) {
         a.walk_count[blockIdx.x] = n_walk;

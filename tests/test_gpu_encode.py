@@ -100,6 +100,28 @@ def _walk(X, cb, norms):
     return dec, idx
 
 
+@pytest.mark.parametrize("N,scale", [(63, 20.0), (70001, 2.0), (65600, 20.0), (262200, 6.0)])
+def test_e8_quantize_of_many_points_in_reach(N, scale):
+    """Where the lists of a workgroup take fewer vectors at a time, are emptied on the way, or run over: all vectors
+    outside the table, at each number of vectors to a workgroup, some of whole workgroups with hundreds of points at one
+    distance (equal entries, zeros).  The walk's own index and codeword throughout."""
+    from glq_amd import ext
+    say("e8 shell search, many points", N, scale)
+    g = torch.Generator().manual_seed(N)
+    X = torch.randn(N, 8, generator=g) * scale
+    for first, of in ((0, [1.0, 0, 0, 0, 0, 0, 0, 0]), (N // 4, [1.0] * 8), (N // 2, [1.0, 1.0, 1.0, 1.0, 0, 0, 0, 0]),
+                      (3 * N // 4, [3.0, 1.0, 1.0, 1.0, 1.0, 1.0, 1.0, -1.0])):
+        n = min(600, N // 8)
+        X[first:first + n] = torch.tensor(of) * (scale * (1 + torch.rand(n, 1, generator=g)))
+        X[first + n // 2:first + n] += 1e-5 * torch.randn(n - n // 2, 8, generator=g)
+    cb = torch.from_numpy(O.e8_table()).to(DEV)
+    X = X.to(DEV)
+    dec, idx = ext.e8_quantize(X, cb)
+    wdec, walk = _walk(X, cb, (cb * cb).sum(-1))
+    assert torch.equal(idx, walk), int((idx != walk).sum())
+    assert torch.equal(dec, wdec)
+
+
 def _changed_table(how):
     cb = torch.from_numpy(O.e8_table()).to(DEV)
     if how == "rows in another order":                           # still the shell table
