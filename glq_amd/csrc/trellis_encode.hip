@@ -372,7 +372,7 @@ viterbi_kernel(const float *__restrict__ tiles_in, int64_t n_tiles, int64_t ld, 
 //     K = 2                     16.7 / 8.1   16.7 / 9.6   16.7 / 10.4  16.8 / 10.8  16.7 / 12.2  16.7 / 16.7
 // Slower is what fills the lists and shows nothing beforehand, as slow ramps do (-3 to 3 over the tile's steps): 17.5 / 19.2,
 // 14.6 / 16.2, 16.7 / 18.7, up to 1.4 times in calls of one or two batches.  2048 x 2048 weights: 69.6 -> 32.7 at K = 4
-// (25.7 through vm_kernel), 58.6 -> 37.5 at 3, 66.6 -> 35.5 at 2.
+// (24.0 through vm_kernel), 58.6 -> 37.5 at 3, 66.6 -> 35.5 at 2.
 constexpr int VB_THREADS = 512;
 constexpr int VB_NORM = 2;                 // steps between two moves of the row's minimum into B
 constexpr float VB_X = 16.0f;              // largest input: (16 + 4)^2 for 16 / K steps stays far below 65504
@@ -436,6 +436,22 @@ __device__ __forceinline__ int vb_group(int at) {
     return ((((k >> 1) ^ vb_word<K>(a)) << 1) + (k & 1)) * C::HI + a;
 }
 
+// vm_kernel's rows have all ways into a group in one piece, its NK^DEPTH runs one after the other (512 bytes at K = 4, where
+// sixteen pieces of 32 touch sixteen cache lines: the walk back over 4096 tiles 694 -> 612 us).  vb_forward's threads write a run
+// each of neighbouring groups, which would scatter.  Where a place of theirs lies then, and back:
+template <int K>
+__device__ __forceinline__ int vb_together(int at) {
+    constexpr int E = 16 - K - K * vb_cfg<K>::DEPTH, HIGH = 16 - 2 * K - E;   // bits of a that the ways share, and the others
+    const int a = at >> K;
+    return ((a & ((1 << E) - 1)) << HIGH | a >> E) << K | (at & (vb_cfg<K>::NK - 1));
+}
+template <int K>
+__device__ __forceinline__ int vb_apart(int at) {
+    constexpr int E = 16 - K - K * vb_cfg<K>::DEPTH, HIGH = 16 - 2 * K - E;
+    const int a = at >> K;
+    return ((a & ((1 << HIGH) - 1)) << E | a >> HIGH) << K | (at & (vb_cfg<K>::NK - 1));
+}
+
 // the least of a wave's values, in every lane
 __device__ __forceinline__ uint32_t vb_wave_min(uint32_t v) {
     auto step = [&](uint32_t u) { v = u < v ? u : v; };
@@ -462,7 +478,7 @@ struct vb_tile {
 };
 
 // Tiles order[first .. first + count - 1], as far as that many are tried, and one of their two passes: 0 on the inputs rolled by T/2, unconstrained; 1 from and
-// to the overlap that the first backtrack found.  rows: STORED rows of G halves per tile.
+// to the overlap that the first backtrack found.  rows: of every tile a row of G halves, STORED times.
 struct vb_part {
     int64_t first;
     int count, pass;
@@ -642,7 +658,7 @@ __device__ __forceinline__ void vb_forward(const float *__restrict__ tiles_in, i
             }
         };
         auto keep = [&](int t, int level, uint32_t (&c)[UNITS][CW]) {   // the row of a level, as read
-            uint16_t *h = rows + ((int64_t)(pair * TPW + t) * C::STORED + level - 1) * G;
+            uint16_t *h = rows + ((int64_t)(level - 1) * part.count + pair * TPW + t) * G;
 #pragma unroll
             for (int q = 0; q < UNITS; ++q) {
                 if constexpr (K == 4) {                        // two threads have read the same: a half each
@@ -774,7 +790,7 @@ __device__ __forceinline__ void vb_forward(const float *__restrict__ tiles_in, i
 // smallest numbers, and VM_LESS of c + e.  Bounds are rounded once a step, towards zero; a row's least one stays at VM_FLOOR,
 // above what comes off until the next move, so that none is negative.
 //
-// 4096 tiles, a pass: 2.6 ms, where vb_forward takes 3.7, and 0.65 for the walk back, which nothing overlaps.  Vector ALUs issue
+// 4096 tiles, a pass: 2.6 ms, where vb_forward takes 3.7, and 0.58 for the walk back, which nothing overlaps.  Vector ALUs issue
 // in 59 % of the cycles (three quarters of that the minima) and the matrix cores work in 39 %, at 2.0 GHz; the rows on their
 // way to memory take 0.4 ms of it.  Measured and not kept: products a pair ahead of the minima (2.6, with the rows in one
 // piece; no registers for more), four waves a SIMD (eight tiles a workgroup, 128 registers: 3.4), eight tiles and two rows
@@ -866,7 +882,7 @@ vm_kernel(const float *__restrict__ tiles_in, int64_t ld, vb_lists lists, vb_par
     };
     auto keep = [&](int level, int q, const u32x4 (&v)[2]) __attribute__((always_inline)) {
         const int to = 2 * wave + (q >> 2), p = 32 * (q & 3) + (lane >> 1), w = p >> 4 & 7;
-        uint16_t *o = part.rows + ((int64_t)(first + to) * C::STORED + level - 1) * C::G + 2 * p * C::NK + 8 * (high ^ w >> 2);
+        uint16_t *o = part.rows + ((int64_t)(level - 1) * part.count + first + to) * C::G + vb_together<4>(2 * p * C::NK) + 8 * (high ^ w >> 2);
         u32x4 even, odd;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -875,7 +891,7 @@ vm_kernel(const float *__restrict__ tiles_in, int64_t ld, vb_lists lists, vb_par
         }
         if (to < count) {
             *(u32x4 *)o = even;
-            *(u32x4 *)(o + C::NK) = odd;
+            *(u32x4 *)(o + vb_together<4>(C::NK)) = odd;
         }
     };
     uint32_t next = xs[turn * VM_TILES + t];
@@ -1005,11 +1021,11 @@ __device__ __forceinline__ void vb_walk(int g, int p, int (&st)[vb_cfg<K>::DEPTH
 // The backtrack of one tile by one wave: true, and the states in `states`; or false, and `limit` the one to try next,
 // infinity where the tile has to be searched exactly.
 // n, gv: the groups of step T (a lane each) whose bounds are within `limit`; x[i]: input of step i; the bounds' row of
-// level l at hist + (l - 1) * G; pre[j]: B at step j * VB_NORM; tie: the only group of step 0, or -1; the states up to
+// level l at hist + (l - 1) * step; pre[j]: B at step j * VB_NORM; tie: the only group of step 0, or -1; the states up to
 // step `upto` are wanted.
 template <int K>
 __device__ __forceinline__ bool vb_trace(int n, int gv, float &limit, const f16 *x, const uint16_t *__restrict__ hist,
-                                         const float *pre, int tie, int upto, vb_pool *P, uint16_t *states) {
+                                         int64_t step, bool together, const float *pre, int tie, int upto, vb_pool *P, uint16_t *states) {
     using C = vb_cfg<K>;
     constexpr int D = C::DEPTH, LEVELS = C::STORED, R = (1 << (K * D)) / 64;
     const int lane = threadIdx.x & 63;
@@ -1017,16 +1033,16 @@ __device__ __forceinline__ bool vb_trace(int n, int gv, float &limit, const f16 
     float cv = 0.0f;                                           // lane j: cost from group gv of this level to the end
     int ne = 0, ns = 0;
     bool full = false, empty = false;
-    float xn[D], pn = pre[(LEVELS - 1) * D / VB_NORM];         // read a level ahead
-#pragma unroll
-    for (int e = 0; e < D; ++e) xn[e] = (float)x[VT_T - 1 - e];
+    typedef f16 inputs __attribute__((ext_vector_type(D)));
+    inputs xn = *(const inputs *)(x + VT_T - D);               // read a level ahead
+    float pn = pre[(LEVELS - 1) * D / VB_NORM];
     // The ways from a group, R to a lane, by where their bounds lie: digits of a lane's ways, and the first one's place.
     constexpr int E = 16 - K - K * D;                          // what of the group is left above the digits
     int ways[R], place;
     {
         const int run = K == 4 ? lane >> 2 : K == 3 ? lane >> 3 : lane;   // the digits but the farthest, the nearest lowest
         const int in = K == 4 ? (lane & 3) * 4 : K == 3 ? lane & 7 : 0;
-        place = (run << (E + K)) + in;
+        place = (run << (together ? K : E + K)) + in;
 #pragma unroll
         for (int r = 0; r < R; ++r) {
             int k = in + r;
@@ -1038,114 +1054,153 @@ __device__ __forceinline__ bool vb_trace(int n, int gv, float &limit, const f16 
     // first group is known: they take longer than everything else here
     u32x2 ahead = {0, 0};
     auto ask = [&](int l, int g, u32x2 &into) {
-        const uint16_t *row = hist + (uint32_t)((l > 1 ? l - 2 : 0) * C::G) + place + (uint32_t)((g >> (K * D)) << K);
+        const uint16_t *row = hist + (l > 1 ? l - 2 : 0) * step + place + (uint32_t)((g >> (K * D)) << (together ? K * D : K));
         if constexpr (R == 4) into = *(const u32x2 *)row;
         else into.x = *row;
     };
     auto bound_of = [&](u32x2 v, int r) { return vb_half((r & 2 ? v.y : v.x) >> (16 * (r & 1)) & 0xFFFFu); };
+    // of the ways from group g, c0 from the end: the groups they come from, their costs, the lanes of those within the limit
+    float xs[D], room;
+    auto look = [&](int l, int g, float c0, u32x2 bounds, int (&front)[R], float (&c)[R], uint64_t (&mask)[R]) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            int st[D];
+            vb_walk<K>(g, ways[r], st);
+            front[r] = st[D - 1] >> K;
+            c[r] = c0;
+#pragma unroll
+            for (int e = 0; e < D; ++e) c[r] += vt_err(st[e], xs[e]);
+        }
+        if (l == 1) {                                          // from the start, or from its only group
+            auto start = [&](int r) { return tie < 0 || front[r] == tie ? 0u : 0x7C00u; };
+            bounds.x = start(0) | (R > 1 ? start(R > 1 ? 1 : 0) << 16 : 0u);
+            if constexpr (R == 4) bounds.y = start(2) | start(3) << 16;
+        }
+        int count = 0;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            mask[r] = __ballot(c[r] + bound_of(bounds, r) <= room);
+            count += __builtin_popcountll(mask[r]);
+        }
+        return count;
+    };
     ask(LEVELS, vb_lane(gv, 0), ahead);
 #pragma unroll 1
     for (int l = LEVELS; l > 0; --l) {
-        full = full || ns + n > P->ENTRIES;
-        if (full || empty) break;
-        if (lane == 0) {
-            P->at[l] = (uint16_t)ne;
-            P->groups[l] = (uint16_t)ns;
-        }
-        if (lane < n) P->group[ns + lane] = (uint16_t)gv;
-        ns += n;
-        const float room = limit - pn;
-        float xs[D];
+        full = ns + n > P->ENTRIES;
+        if (full) break;
+        room = limit - pn;
 #pragma unroll
-        for (int e = 0; e < D; ++e) {
-            xs[e] = xn[e];
-            xn[e] = (float)x[((l - 1) * D - 1 - e) & (VT_T - 1)];
-        }
+        for (int e = 0; e < D; ++e) xs[e] = (float)xn[D - 1 - e];
+        xn = *(const inputs *)(x + ((l - 2) * D & (VT_T - 1)));
         pn = pre[(l > 1 ? l - 2 : 0) * D / VB_NORM];
-        // lane j: child j, its cheapest entry, and the next one's cost
-        int m = 0, nn = 0, ng = -1, nvia = lane;
-        float nc = inf, second = inf;
-#pragma unroll 1
-        for (int j = 0; j < n; ++j) {
-            const int g = vb_lane(gv, j);
-            const float c0 = vb_lane(cv, j);
-            const u32x2 bounds = ahead;
-            if (j + 1 < n) ask(l, vb_lane(gv, j + 1), ahead);  // one group ahead, too
-            int front[R];
-            float c[R], bound[R];
+        int front[R];
+        float c[R];
+        uint64_t mask[R];
+        if (n == 1) {                                          // one group: its ways lead to different ones
+            const int g = vb_lane(gv, 0), m = look(l, g, vb_lane(cv, 0), ahead, front, c, mask);
+            full = ne + m > P->ENTRIES || m > VB_MOST;
+            empty = m == 0;
+            if (full || empty) break;
+            int cs = __builtin_bit_cast(int, c[R - 1]), ws = ways[R - 1];   // a lane's first way in reach
+            uint64_t first = mask[R - 1];
 #pragma unroll
-            for (int r = 0; r < R; ++r) {
-                int st[D];
-                vb_walk<K>(g, ways[r], st);
-                front[r] = st[D - 1] >> K;
-                c[r] = c0;
-#pragma unroll
-                for (int e = 0; e < D; ++e) c[r] += vt_err(st[e], xs[e]);
+            for (int r = R - 2; r >= 0; --r) {
+                const bool in = mask[r] >> lane & 1;
+                cs = in ? __builtin_bit_cast(int, c[r]) : cs;
+                ws = in ? ways[r] : ws;
+                first = mask[r] ? mask[r] : first;
             }
-            uint64_t mask[R];
-            int count = 0;
-#pragma unroll
-            for (int r = 0; r < R; ++r) {
-                bound[r] = l > 1 ? bound_of(bounds, r) : tie < 0 || front[r] == tie ? 0.0f : inf;
-                mask[r] = __ballot(c[r] + bound[r] <= room);
-                count += __builtin_popcountll(mask[r]);
+            const int from = __builtin_ctzll(first), way = vb_lane(ws, from);
+            int st[D];
+            vb_walk<K>(g, way, st);
+            ask(l - 1, st[D - 1] >> K, ahead);
+            if (lane == 0) {
+                P->at[l] = (uint16_t)ne;
+                P->groups[l] = (uint16_t)ns;
+                P->group[ns] = (uint16_t)g;
             }
-            full = full || m + count > 256 || ne + m + count > P->ENTRIES || (n == 1 && count > VB_MOST);
-            if (full) break;
-            if (n == 1 && count) {
-                int g0 = 0;
-#pragma unroll
-                for (int r = R - 1; r >= 0; --r) g0 = mask[r] ? vb_lane(front[r], __builtin_ctzll(mask[r])) : g0;
-                ask(l - 1, g0, ahead);
-            }
-            int k = m;
-            if (n == 1) {                                      // one parent: its children are all different
+            if (m == 1) {                                      // three levels in four
+                gv = st[D - 1] >> K;
+                cv = __builtin_bit_cast(float, vb_lane(cs, from));
+                if (lane == 0) {
+                    P->entry[ne] = (uint16_t)way;
+                    P->cost[ne] = cv;
+                    P->child[ne] = 0;
+                    P->via[ne] = 0;
+                }
+            } else {
+                int k = 0;
 #pragma unroll
                 for (int r = 0; r < R; ++r) {
                     const int to = k + vb_below(mask[r]);
-                    if (c[r] + bound[r] <= room) {
+                    if (mask[r] >> lane & 1) {
                         P->entry[ne + to] = (uint16_t)ways[r];
                         P->kept[to] = front[r];
                         P->cost[ne + to] = c[r];
                     }
                     k += __builtin_popcountll(mask[r]);
                 }
-                if (lane < count) P->child[ne + lane] = (uint8_t)lane;
                 __builtin_amdgcn_wave_barrier();
-                nn = count;
-                ng = P->kept[lane];
-                nc = P->cost[ne + (lane < count ? lane : 0)];
+                gv = P->kept[lane];
+                cv = P->cost[ne + (lane < m ? lane : 0)];
+                if (lane < m) {
+                    P->child[ne + lane] = (uint8_t)lane;
+                    P->via[ne + lane] = (uint16_t)lane;
+                }
                 __builtin_amdgcn_wave_barrier();
-            } else {                                           // one entry after the other, in registers: there are a few
-#pragma unroll
-                for (int r = 0; r < R; ++r) {
-                    if (c[r] + bound[r] <= room) {
-                        const int to = ne + k + vb_below(mask[r]);
-                        P->entry[to] = (uint16_t)(ways[r] | j << 8);
-                        P->cost[to] = c[r];
-                    }
+            }
+            ns += 1;
+            ne += m;
+            n = m;
+            continue;
+        }
+        if (lane == 0) {
+            P->at[l] = (uint16_t)ne;
+            P->groups[l] = (uint16_t)ns;
+        }
+        if (lane < n) P->group[ns + lane] = (uint16_t)gv;
+        ns += n;
+        // lane j: child j, its cheapest entry, and the next one's cost
+        int m = 0, nn = 0, ng = -1, nvia = lane;
+        float nc = inf, second = inf;
 #pragma unroll 1
-                    for (uint64_t rest = mask[r]; rest; rest &= rest - 1, ++k) {
-                        const int from = __builtin_ctzll(rest), f = vb_lane(front[r], from);
-                        const float cf = vb_lane(c[r], from);
-                        const uint64_t same = __ballot(ng == f);
-                        const int child = same ? __builtin_ctzll(same) : nn;
-                        nn = __builtin_amdgcn_readfirstlane(nn + (same ? 0 : 1));
-                        P->child[ne + k] = (uint8_t)child;
-                        const bool mine = lane == child, better = mine && cf < nc;
-                        const float other = __builtin_fmaxf(nc, cf);   // the new one's or, where that is better, the old one's
-                        second = mine && other < second ? other : second;
-                        nvia = better ? k | j << 8 : nvia;
-                        nc = better ? cf : nc;
-                        ng = mine ? f : ng;
-                    }
+        for (int j = 0; j < n; ++j) {
+            const u32x2 bounds = ahead;
+            if (j + 1 < n) ask(l, vb_lane(gv, j + 1), ahead);  // one group ahead, too
+            const int count = look(l, vb_lane(gv, j), vb_lane(cv, j), bounds, front, c, mask);
+            full = m + count > 256 || ne + m + count > P->ENTRIES;
+            if (full) break;
+            int k = m;                                         // one entry after the other, in registers: there are a few
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                if (mask[r] >> lane & 1) {
+                    const int to = ne + k + vb_below(mask[r]);
+                    P->entry[to] = (uint16_t)(ways[r] | j << 8);
+                    P->cost[to] = c[r];
+                }
+#pragma unroll 1
+                for (uint64_t rest = mask[r]; rest; rest &= rest - 1, ++k) {
+                    const int from = __builtin_ctzll(rest), f = vb_lane(front[r], from);
+                    const float cf = vb_lane(c[r], from);
+                    const uint64_t same = __ballot(ng == f);
+                    const int child = same ? __builtin_ctzll(same) : nn;
+                    nn = __builtin_amdgcn_readfirstlane(nn + (same ? 0 : 1));
+                    P->child[ne + k] = (uint8_t)child;
+                    const bool mine = lane == child, better = mine && cf < nc;
+                    const float other = __builtin_fmaxf(nc, cf);   // the new one's or, where that is better, the old one's
+                    second = mine && other < second ? other : second;
+                    nvia = better ? k | j << 8 : nvia;
+                    nc = better ? cf : nc;
+                    ng = mine ? f : ng;
                 }
             }
             m += count;
         }
         full = full || nn > VB_MOST;
         empty = m == 0;
-        if (n != 1) ask(l - 1, vb_lane(ng, 0) & (C::G - 1), ahead);
+        if (full || empty) break;
+        ask(l - 1, vb_lane(ng, 0) & (C::G - 1), ahead);
         if (lane < nn) P->via[ne + lane] = (uint16_t)(nvia | (second - nc <= close ? 1 << 14 : 0));
         ne += m;
         n = nn;
@@ -1195,24 +1250,42 @@ __device__ __forceinline__ bool vb_trace(int n, int gv, float &limit, const f16 
 
     // exact costs, forward over the kept ways that a path close to the cheapest may take; lane e: entry e of the level,
     // best, cheap: exact cost from the start, cost to the end, of group `lane` of the level below
+    // (what of a level is known beforehand is read a level ahead: trips to LDS, each behind the last, were half of its time)
+    struct level_data {
+        int m, nb, parent, child, way, group;
+        float cost, cheap;                                     // of the entry; of group `lane` of the level above
+    };
+    auto read = [&](int l) {
+        level_data L;
+        const int eb = P->at[l];
+        L.m = (int)P->at[l - 1] - eb, L.nb = P->at[l < LEVELS ? l + 1 : l];
+        const int e = eb + (lane < L.m ? lane : 0), en = P->entry[e];
+        L.parent = en >> 8, L.way = en & 255, L.child = P->child[e], L.cost = P->cost[e];
+        L.group = P->group[P->groups[l] + L.parent];
+        L.cheap = P->cost[L.nb + (P->via[L.nb + lane] & 255)];
+        return L;
+    };
     float cheap = P->cost[P->at[1] + (P->via[P->at[1] + lane] & 255)];
     float best = lane < n && cheap <= u + close ? 0.0f : inf;
+    level_data next = read(1);
 #pragma unroll 1
     for (int l = 1; l <= LEVELS; ++l) {
-        const int eb = P->at[l], m = __builtin_amdgcn_readfirstlane((int)P->at[l - 1] - eb), nb = P->at[l < LEVELS ? l + 1 : l];
+        const level_data L = next;
+        next = read(l < LEVELS ? l + 1 : l);
+        const int m = __builtin_amdgcn_readfirstlane(L.m), nb = L.nb, parent = L.parent;
         if (m > 64) {
             limit = inf;
             return false;
         }
-        const int e = eb + (lane < m ? lane : 0), en = P->entry[e], parent = en >> 8, child = P->child[e];
         int st[D];
-        vb_walk<K>(P->group[P->groups[l] + parent], en & 255, st);
-        float v[D], c = __shfl(best, child, GLQH_WAVE);
-        const float room = __shfl(cheap, child, GLQH_WAVE) + close;
-        const uint64_t live = __ballot(lane < m && c < inf && P->cost[e] <= room);
+        vb_walk<K>(L.group, L.way, st);
+        float v[D], c = __shfl(best, L.child, GLQH_WAVE);
+        const float room = __shfl(cheap, L.child, GLQH_WAVE) + close;
+        const uint64_t live = __ballot(lane < m && c < inf && L.cost <= room);
+        const inputs xl = *(const inputs *)(x + (l - 1) * D);
 #pragma unroll
         for (int d = D - 1; d >= 0; --d) {
-            c = vt_err(st[d], (float)x[l * D - 1 - d]) + c;
+            c = vt_err(st[d], (float)xl[D - 1 - d]) + c;
             v[d] = c;
         }
         bool least = live >> lane & 1;     // of its parent (at the end: of all): the lowest cost, then the lowest state, step by step
@@ -1234,7 +1307,7 @@ __device__ __forceinline__ bool vb_trace(int n, int gv, float &limit, const f16 
             take = __builtin_ctzll(won);
             break;
         }
-        cheap = P->cost[nb + (P->via[nb + lane] & 255)];
+        cheap = L.cheap;
         if ((won & (won - 1)) == 0) {
             const int q = __builtin_ctzll(won);
             best = lane == vb_lane(parent, q) ? vb_lane(v[0], q) : inf;
@@ -1250,15 +1323,20 @@ __device__ __forceinline__ bool vb_trace(int n, int gv, float &limit, const f16 
         __builtin_amdgcn_wave_barrier();
     }
 #pragma unroll 1
-    for (int l = LEVELS; l > 0; --l) {
-        const int at = P->at[l] + take, en = P->entry[at];
-        int st[D];
-        vb_walk<K>(P->group[P->groups[l] + (en >> 8)], en & 255, st);
-        if (lane == 0) {
-#pragma unroll
-            for (int e = 0; e < D; ++e) states[l * D - 1 - e] = (uint16_t)st[e];
+    for (int l0 = LEVELS; l0 > 0; l0 -= 64) {
+        const int ats = P->at[l0 - lane], gs = P->groups[l0 - lane];
+        int mine = 0;                                          // lane k: the path's entry of level l0 - k
+#pragma unroll 1
+        for (int k = 0; k < 64; ++k) {
+            mine = lane == k ? take : mine;
+            const int at = vb_lane(ats, k);
+            if (l0 - k > 1) take = __builtin_amdgcn_readfirstlane(P->via[at + P->child[at + take]]);
         }
-        if (l > 1) take = __builtin_amdgcn_readfirstlane(P->via[P->at[l] + P->child[at]]);
+        const int en = P->entry[ats + mine];
+        int st[D];
+        vb_walk<K>(P->group[gs + (en >> 8)], en & 255, st);
+#pragma unroll
+        for (int e = 0; e < D; ++e) states[(l0 - lane) * D - 1 - e] = (uint16_t)st[e];
     }
     return true;
 }
@@ -1267,7 +1345,7 @@ __device__ __forceinline__ bool vb_trace(int n, int gv, float &limit, const f16 
 struct vb_work {
     vb_pool pool;
     float pre[VT_T / VB_NORM + 1];
-    f16 x[VT_T];
+    alignas(8) f16 x[VT_T];
     uint16_t states[VT_T];
     int start[VB_MOST];
 };
@@ -1276,6 +1354,10 @@ static_assert(sizeof(vb_work) <= 160 * 1024 / 16, "sixteen on a CU");
 // The backtrack of tile part.first + at (one wave): after pass 0 the overlap, after pass 1 the states and values.
 // What bounds it is latency: a chain of STORED levels, each a look into a row of which only the last level's group tells
 // where (a microsecond), some 150 instructions and trips to LDS.  150 us on average, 340 for the slowest of 256 tiles.
+// Sixteen waves a CU over 4096 tiles of vm_kernel: 0.19 ms on average, 0.46 for the slowest tile, which is what the launch takes (four ways
+// a level, and another near).  0.73 -> 0.58 by the kept groups' bounds in one piece, a short way where one way is in reach, and
+// the exact comparison's levels read ahead and its path found by the lanes.  (Two groups at a time, or the next level's
+// first two asked for: 0.69, in spilled scalar registers; a loop of its own for levels of one way: level.)
 template <int K>
 __device__ __forceinline__ void vb_backtrack(const float *__restrict__ tiles_in, int64_t ld, const vb_lists &lists,
                                              const vb_part &part, int at, vb_work *W, int32_t *__restrict__ states_out, float *__restrict__ hat_out) {
@@ -1299,12 +1381,13 @@ __device__ __forceinline__ void vb_backtrack(const float *__restrict__ tiles_in,
     for (int d = 1; d < 64; d <<= 1) lost += __shfl_xor(lost, d, GLQH_WAVE);
     lost = K == 4 && part.product ? VT_T * VM_FLOOR * 0x1p-10f + lost : VB_LOST;   // (2^-10: a rounding of the least bounds)
     for (int i = lane; i <= VT_T / VB_NORM; i += 64) pre[i] = mine->pre[i];
-    const uint16_t *hist = part.rows + (int64_t)at * C::STORED * C::G, *last = hist + (int64_t)(C::STORED - 1) * C::G;
+    const int64_t step = (int64_t)part.count * C::G;
+    const uint16_t *hist = part.rows + (int64_t)at * C::G, *last = hist + (C::STORED - 1) * step;
     __builtin_amdgcn_wave_barrier();
     const float bt = pre[VT_T / VB_NORM];
     uint32_t lo = 0xFFFFu;                                     // the least bound of the groups that may be last
     if (pass) {
-        lo = last[vb_stored<K>(tie)];
+        lo = last[part.product ? vb_together<K>(vb_stored<K>(tie)) : vb_stored<K>(tie)];
     } else {
 #pragma unroll 8
         for (int g = 0; g < C::G; g += 64) {
@@ -1335,7 +1418,7 @@ __device__ __forceinline__ void vb_backtrack(const float *__restrict__ tiles_in,
                 for (int k = 0; k < 8; ++k) {
                     const uint64_t mask = __ballot(b[k] <= limit);
                     const int at = n + vb_below(mask);
-                    if (b[k] <= limit && at < VB_MOST) start[at] = vb_group<K>(g0 + 64 * k + lane);
+                    if (b[k] <= limit && at < VB_MOST) start[at] = vb_group<K>(part.product ? vb_apart<K>(g0 + 64 * k + lane) : g0 + 64 * k + lane);
                     n += __builtin_popcountll(mask);
                 }
             }
@@ -1343,7 +1426,7 @@ __device__ __forceinline__ void vb_backtrack(const float *__restrict__ tiles_in,
         __builtin_amdgcn_wave_barrier();
         n = __builtin_amdgcn_readfirstlane(n);
         if (n > VB_MOST) limit = __builtin_inff();
-        else good = vb_trace<K>(n, lane < n ? start[lane] : 0, limit, x, hist, pre, tie, pass ? VT_T - 1 : VT_T / 2, &W->pool, states);
+        else good = vb_trace<K>(n, lane < n ? start[lane] : 0, limit, x, hist, step, part.product, pre, tie, pass ? VT_T - 1 : VT_T / 2, &W->pool, states);
         if (good) break;
         if (limit == __builtin_inff()) {                       // too many ways for the lists: half the slack may do
             limit = lower;
@@ -1482,7 +1565,7 @@ int acs_launch(const float *cost, const void *x, const float *lut, float *cost_o
 
 // Two batches of tiles take turns: while one walks back, the other runs forward.  A batch is a chip full of pairs (two
 // workgroups a CU); everything is one batch where that leaves none to overlap with.  least: batches of half as many, in the
-// scratch that viterbi_kernel alone takes (16384 tiles 1 GB and 35.5 ms instead of 4 and 25.7 at K = 4, 2 GB and 37.2 instead
+// scratch that viterbi_kernel alone takes (16384 tiles 1 GB and 35.5 ms instead of 4 and 24.0 at K = 4, 2 GB and 37.2 instead
 // of 4 and 38.0 at 3, 38.9 instead of 35.7 at 2).
 //
 // At K = 4 chips full of sixteen tiles a CU come first, through vm_kernel, one after the other, and the rest too where that is
