@@ -109,17 +109,21 @@ __device__ __forceinline__ attn_kregs attn_load_k(const uint16_t *__restrict__ K
     return r;
 }
 
-// four rows of V of a thread's round (rows j0 + u * 4 * AT_WAVES; 16 lanes per row, 16 bytes each)
+// four rows of V of a thread's round (rows j0 + u * 4 * AT_WAVES; 16 lanes per row, 16 / PARTS bytes each)
+template <int PARTS>
 struct attn_vregs {
-    u32x4 v[4];
+    typedef uint32_t words __attribute__((ext_vector_type(4 / PARTS)));
+    words v[4];
 };
 
-__device__ __forceinline__ attn_vregs attn_load_v(const uint16_t *__restrict__ V, int j0, int last) {
+template <int PARTS>
+__device__ __forceinline__ attn_vregs<PARTS> attn_load_v(const uint16_t *__restrict__ V, int j0, int last) {
     constexpr int D = 128;
     const int vcol = threadIdx.x & 15;
-    attn_vregs r;
+    attn_vregs<PARTS> r;
 #pragma unroll
-    for (int u = 0; u < 4; ++u) r.v[u] = *(const u32x4 *)(V + (int64_t)min(j0 + u * 4 * AT_WAVES, last) * D + 8 * vcol);
+    for (int u = 0; u < 4; ++u)
+        r.v[u] = *(const typename attn_vregs<PARTS>::words *)(V + (int64_t)min(j0 + u * 4 * AT_WAVES, last) * D + 8 / PARTS * vcol);
     return r;
 }
 
@@ -130,14 +134,16 @@ __device__ __forceinline__ attn_vregs attn_load_v(const uint16_t *__restrict__ V
 // L2 of this XCD for the workgroup that merges the shares) instead of the finished row to `out`.
 constexpr int AT_PART = 2 + 128;
 
-template <bool NEWROW, bool FIRST = false>
+// PARTS: the workgroup makes one of the row's PARTS runs of 128 / PARTS columns, and V, vnew and out begin
+// there: all scores, but only that much of V.  Every column is summed in the order that PARTS = 1 takes.
+template <bool NEWROW, bool FIRST = false, int PARTS = 1>
 __device__ __forceinline__ void attn_core(const float *qs, const uint16_t *__restrict__ K,
                                           const uint16_t *__restrict__ V, int n, const uint16_t *knew,
                                           const uint16_t *vnew, float *sc, float *red,
                                           float (*part)[128], uint16_t *__restrict__ out,
                                           const attn_kregs first_k = {}, int j_lo = 0, int j_hi = -1,
                                           float *pbuf = nullptr) {
-    constexpr int D = 128;
+    constexpr int DV = 128 / PARTS, C = 8 / PARTS;             // columns of the workgroup, of a lane
     if (j_hi < 0) j_hi = n;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     // last row that is read from the cache (row n - 1 comes from knew / vnew when NEWROW)
@@ -180,7 +186,7 @@ __device__ __forceinline__ void attn_core(const float *qs, const uint16_t *__res
     // is requested here, ahead of the softmax, every later one a round ahead of its use.
     const int vr = lane >> 4, vcol = lane & 15;
     const int vj0 = j_lo + wave * 4 + vr;
-    attn_vregs vcur = attn_load_v(V, vj0, last);
+    attn_vregs<PARTS> vcur = attn_load_v<PARTS>(V, vj0, last);
     mx = wave_max(mx);
     if (lane == 0) red[wave] = mx;
     __syncthreads();
@@ -200,23 +206,23 @@ __device__ __forceinline__ void attn_core(const float *qs, const uint16_t *__res
     float tot = 0.0f;
 #pragma unroll
     for (int w = 0; w < AT_WAVES; ++w) tot += red[w];
-    float a[8];
+    float a[C];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) a[e] = 0.0f;
+    for (int e = 0; e < C; ++e) a[e] = 0.0f;
     for (int j0 = vj0; j0 < j_hi; j0 += 4 * 4 * AT_WAVES) {
-        attn_vregs vnext = vcur;
-        if (j0 + 4 * 4 * AT_WAVES < j_hi) vnext = attn_load_v(V, j0 + 4 * 4 * AT_WAVES, last);
+        attn_vregs<PARTS> vnext = vcur;
+        if (j0 + 4 * 4 * AT_WAVES < j_hi) vnext = attn_load_v<PARTS>(V, j0 + 4 * 4 * AT_WAVES, last);
         float pw[4];
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             const int j = j0 + u * 4 * AT_WAVES;
-            if (NEWROW && j == n - 1) vcur.v[u] = *(const u32x4 *)(vnew + 8 * vcol);
+            if (NEWROW && j == n - 1) vcur.v[u] = *(const typename attn_vregs<PARTS>::words *)(vnew + C * vcol);
             pw[u] = j < j_hi ? sc[j - j_lo] : 0.0f;
         }
 #pragma unroll
         for (int u = 0; u < 4; ++u)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
+            for (int e = 0; e < C / 2; ++e) {
                 const uint32_t w = vcur.v[u][e];
                 a[2 * e] += pw[u] * bf16_bits_to_f32((uint16_t)(w & 0xFFFFu));
                 a[2 * e + 1] += pw[u] * bf16_bits_to_f32((uint16_t)(w >> 16));
@@ -224,16 +230,16 @@ __device__ __forceinline__ void attn_core(const float *qs, const uint16_t *__res
         vcur = vnext;
     }
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {                               // the wave's four row lanes
+    for (int e = 0; e < C; ++e) {                               // the wave's four row lanes
         a[e] += __shfl_xor(a[e], 16, GLQH_WAVE);
         a[e] += __shfl_xor(a[e], 32, GLQH_WAVE);
     }
     if (vr == 0) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) part[wave][8 * vcol + e] = a[e];
+        for (int e = 0; e < C; ++e) part[wave][C * vcol + e] = a[e];
     }
     __syncthreads();
-    if (threadIdx.x < D) {
+    if (threadIdx.x < DV) {
         float acc = 0.0f;
 #pragma unroll
         for (int w = 0; w < AT_WAVES; ++w) acc += part[w][threadIdx.x];
@@ -600,7 +606,11 @@ __device__ __forceinline__ rht_slice slice_of_row(int m, int row, int log_slice)
     return blk;
 }
 
-template <bool SHARED>
+// PARTS workgroups (blockIdx.z) make 128 / PARTS columns of a head's row each: the scores and what leads to them are made by
+// all of them, V is read by one each.  A head's 512 cached positions are 128 KB of V behind 128 KB of K, and one CU draws some 50
+// bytes a ns: the launch 11.3 -> 10.2 us, a step of 8 layers at 8 / 128 / 512 / 1000 positions 567 / 584 / 603 / 626 -> 561 / 579 / 593 /
+// 615 us.  (The first rounds of V requested beside the keys instead: 10.8 -> 11.6.)
+template <bool SHARED, int PARTS>
 __global__ void __launch_bounds__(AT_THREADS)
 out_rope_attn_kernel(qkv_fin a, int ksplit, const int64_t *__restrict__ pos_ptr,
                      const uint16_t *__restrict__ cos_t, const uint16_t *__restrict__ sin_t,
@@ -614,7 +624,7 @@ out_rope_attn_kernel(qkv_fin a, int ksplit, const int64_t *__restrict__ pos_ptr,
     __shared__ float part[AT_WAVES][D];
     __shared__ __align__(16) uint16_t knew[D], vnew[D];
     float *sc = lds;
-    const int h = blockIdx.x, per = heads / kv_heads, g = h / per;
+    const int h = blockIdx.x, per = heads / kv_heads, g = h / per, col0 = PARTS > 1 ? (int)blockIdx.z * (D / PARTS) : 0;
     const int64_t p = pos_ptr[0];
     if (p < 0 || p >= max_len) return;             // position outside the cache and the score buffer
     const int n = (int)p + 1;
@@ -691,7 +701,7 @@ out_rope_attn_kernel(qkv_fin a, int ksplit, const int64_t *__restrict__ pos_ptr,
             uint16_t *nw = grp == 1 ? knew : vnew;
             nw[d] = o0;
             nw[d + half] = o1;
-            if (h % per == 0 && share == 0) {                    // one writer per key/value head
+            if (h % per == 0 && share == 0 && col0 == 0) {       // one writer per key/value head
                 uint16_t *dst = (grp == 1 ? kc : vc) + ((int64_t)g * max_len + p) * D;
                 dst[d] = o0;
                 dst[d + half] = o1;
@@ -700,11 +710,11 @@ out_rope_attn_kernel(qkv_fin a, int ksplit, const int64_t *__restrict__ pos_ptr,
     }
     fht_barrier<true>();                           // qs, knew, vnew are in LDS
     if constexpr (!SHARED) {
-        attn_core<true, true>(qs, Kh, Vh, n, knew, vnew, sc, red, part, out + (int64_t)h * D, first_k);
+        attn_core<true, true, PARTS>(qs, Kh, Vh + col0, n, knew, vnew + col0, sc, red, part, out + (int64_t)h * D + col0, first_k);
     } else {
         float *hbuf = split_buf + (int64_t)h * gridDim.y * AT_PART;
         attn_core<true, true>(qs, Kh, Vh, n, knew, vnew, sc, red, part, out + (int64_t)h * D, first_k, j_lo, j_hi,
-                        ns > 1 ? hbuf + share * AT_PART : nullptr);
+                              ns > 1 ? hbuf + share * AT_PART : nullptr);
         if (ns > 1) attn_merge_shares(hbuf, split_cnt + h, ns, out + (int64_t)h * D, (int *)red);
     }
 }
@@ -993,14 +1003,19 @@ int glqh_launch_out_rope_attn(const float *const part[3], const void *const su[3
                  (long long)max_len);
     unsigned int *cnt = (unsigned int *)split_state;
     float *sbuf = split_state ? (float *)((char *)split_state + ATTN_SPLIT_MAX_HEADS * sizeof(unsigned int)) : nullptr;
-#define GLQH_ATTN_LAUNCH(SHARED)                                                                              \
-    hipLaunchKernelGGL(out_rope_attn_kernel<SHARED>, dim3((unsigned)heads, (unsigned)shares), dim3(AT_THREADS), lds, \
-                       stream, a, ksplit, pos, (const uint16_t *)cos_t, (const uint16_t *)sin_t,                  \
+    // Without shares, as many parts of a row as there are CUs for.  (With them the workgroups that retire at once cost what the
+    // parts save: 4 layers at 8 / 700 / 2000 positions of 2048 340.0 / 365.5 / 379.8 -> 345.9 / 368.7 / 381.7 us.)
+    const int64_t parts = 4 * heads <= glqh_device_cus() ? 4 : 2 * heads <= glqh_device_cus() ? 2 : 1;
+#define GLQH_ATTN_LAUNCH(SHARED, PARTS)                                                                       \
+    hipLaunchKernelGGL((out_rope_attn_kernel<SHARED, PARTS>), dim3((unsigned)heads, (unsigned)shares, PARTS),         \
+                       dim3(AT_THREADS), lds, stream, a, ksplit, pos, (const uint16_t *)cos_t, (const uint16_t *)sin_t,                  \
                        (uint16_t *)k_cache, (uint16_t *)v_cache, (uint16_t *)out, (int)heads, (int)kv_heads,      \
                        (int)max_len, apply_rope, 1.0f / sqrtf((float)head_dim), log_slice, sc_floats, buf_floats, \
                        sbuf, cnt, ATTN_SPLIT_MIN)
-    if (shares > 1) GLQH_ATTN_LAUNCH(true);
-    else GLQH_ATTN_LAUNCH(false);
+    if (shares > 1) GLQH_ATTN_LAUNCH(true, 1);
+    else if (parts == 4) GLQH_ATTN_LAUNCH(false, 4);
+    else if (parts == 2) GLQH_ATTN_LAUNCH(false, 2);
+    else GLQH_ATTN_LAUNCH(false, 1);
 #undef GLQH_ATTN_LAUNCH
     GLQH_LAUNCH_CHECK("out+rope+attention launch");
     return 0;

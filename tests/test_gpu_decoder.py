@@ -241,6 +241,34 @@ def test_attention_with_shared_keys(L, positions):
         assert e < 6e-3, (p, e)
 
 
+@pytest.mark.parametrize("heads,kvh", [(16, 4), (96, 8), (160, 8)])
+def test_attention_row_in_parts(heads, kvh):
+    """Four, two and one workgroups to a head's row, by the number of heads: the bits of the separate launches, which
+    never part a row, at the edges of a round of V (256 rows) and of the keys (512)."""
+    from glq_amd import decoder as D
+    say("attention in parts", heads, kvh)
+    g = torch.Generator(device=DEV).manual_seed(heads)
+    hidden, hd, L = 256, 128, 600
+    q, k, v = (D._Linear(heads * hd, hidden, 4, g, DEV), D._Linear(kvh * hd, hidden, 4, g, DEV),
+               D._Linear(kvh * hd, hidden, 4, g, DEV))
+    h = torch.randn(1, hidden, generator=g, device=DEV).to(torch.bfloat16)
+    cos = torch.rand(L, hd, generator=g, device=DEV).to(torch.bfloat16)
+    sin = torch.rand(L, hd, generator=g, device=DEV).to(torch.bfloat16)
+    kc0 = torch.randn(kvh, L, hd, generator=g, device=DEV).to(torch.bfloat16)
+    vc0 = torch.randn(kvh, L, hd, generator=g, device=DEV).to(torch.bfloat16)
+    for p in (0, 1, 255, 256, 511, 512, 599):
+        pos = torch.tensor([p], device=DEV)
+        qr, kc, vc = torch.zeros(1, heads * hd, dtype=torch.bfloat16, device=DEV), kc0.clone(), vc0.clone()
+        D._qkv_rope_store(q, k, v, h, pos, cos, sin, qr, kc, vc, hd, L, 1)
+        ref = torch.zeros_like(qr)
+        D.check(D._lib.load().glqh_attn_decode_bf16(qr.data_ptr(), kc.data_ptr(), vc.data_ptr(), pos.data_ptr(), ref.data_ptr(),
+                                                    heads, kvh, hd, L, D._stream()))
+        kc1, vc1, out = kc0.clone(), vc0.clone(), torch.zeros_like(qr)
+        D._qkv_rope_attn(q, k, v, h, pos, cos, sin, kc1, vc1, out, heads, kvh, hd, L, 1)
+        assert torch.count_nonzero(ref) > 0
+        assert torch.equal(out, ref) and torch.equal(kc1, kc) and torch.equal(vc1, vc), p
+
+
 @pytest.mark.parametrize("hidden,vocab", [(2048, 128256), (4096, 1000), (2048, 7)])
 def test_output_head_and_argmax(hidden, vocab):
     """Logits of the library's output head against a float64 product, its arg-max against the
