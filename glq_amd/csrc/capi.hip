@@ -42,7 +42,7 @@ static int e8_tile_ks(int64_t m_pad, int64_t n_pad, int64_t B, int nstages, bool
     return B > GLQH_E8_SMALL_BATCH ? glqh_e8_tile_ksplit(m_pad, n_pad, B, nstages, fold) : 0;
 }
 
-int glqh_trellis_mma_fusein_plan(int64_t wgs_rows, int64_t k, int64_t B, int *S_out, int *ksplit_out);
+int glqh_trellis_mma_fusein_plan(int64_t wgs_rows, int64_t k, int64_t B, int n_stages, int n_layers, int *S_out, int *ksplit_out);
 int glqh_launch_trellis_mma_rvq(const void *x_f16, int64_t B, const void *packed, const void *packed2, int R2, float rs2,
                                 int64_t m, int64_t k, int S, int ksplit, float *part, hipStream_t stream);
 int64_t glqh_trellis_mma_group_rows(const int64_t m[], int n);
@@ -67,10 +67,11 @@ int glqh_launch_trellis_mma_fusein(const void *const packed[], const void *const
 // smaller workgroups of the v_dot2 form spread it over more CUs.
 #define GLQH_FUSEIN_MMA_MIN_STRIPS 32
 static int tr_fusein_plan(const int64_t *m_pads, int n, int64_t n_pad, int64_t B, int *S, int *ks,
-                          int mma_min_strips = GLQH_FUSEIN_MMA_MIN_STRIPS) {
+                          bool both_stages = false) {          // of a stacked layer in one launch: the MFMA form at every height
     int64_t total = 0, wgs = 0;
     for (int i = 0; i < n; ++i) { total += m_pads[i]; wgs += (m_pads[i] + 63) / 64; }
-    if (wgs >= mma_min_strips) return glqh_trellis_mma_fusein_plan(wgs, n_pad, B, S, ks) ? 2 : 0;
+    if (both_stages || wgs >= GLQH_FUSEIN_MMA_MIN_STRIPS)
+        return glqh_trellis_mma_fusein_plan(wgs, n_pad, B, both_stages ? 2 : 1, n, S, ks) ? 2 : 0;
     return glqh_trellis_fusein_plan(total, n_pad, B, S, ks) ? 1 : 0;
 }
 // many-token kernel (trellis_tile.hip): weights decoded once per 128-row x 512-token tile
@@ -454,7 +455,7 @@ static size_t tr_fused_part_bytes(int64_t B, int64_t n_pad, int64_t m_pad) {
     int steps = 0, ks2 = 0;
     if (tr_fusein_plan(&m_pad, 1, n_pad, B, &steps, &ks2) && ks2 > ks) ks = ks2;
     // one token of a two-stage layer plans the MFMA form at every height
-    if (B == 1 && tr_fusein_plan(&m_pad, 1, n_pad, B, &steps, &ks2, 1) && ks2 > ks) ks = ks2;
+    if (B == 1 && tr_fusein_plan(&m_pad, 1, n_pad, B, &steps, &ks2, true) && ks2 > ks) ks = ks2;
     return align256((size_t)ks * B * m_pad * sizeof(float));
 }
 
@@ -547,7 +548,7 @@ extern "C" int glqh_fused_linear_trellis_3inst(
     const bool fi_pays = tr_fuse_input_enabled() && m_pad * n_pad <= ((int64_t)(fuse2 ? 128 : 32) << 20) &&
                          (B == 1 || (B == 2 && pow2_n && n_pad <= 4096 && m_pad <= 4096));
     if (fi_pays && fi_blocks && (x_dtype == GLQH_F16 || x_dtype == GLQH_BF16) &&
-        (fi_mode = tr_fusein_plan(&m_pad, 1, n_pad, B, &fi_steps, &ks, fuse2 ? 1 : GLQH_FUSEIN_MMA_MIN_STRIPS)) != 0 &&
+        (fi_mode = tr_fusein_plan(&m_pad, 1, n_pad, B, &fi_steps, &ks, fuse2)) != 0 &&
         (!has_s2 || (B == 1 && fi_mode == 2 && (merge2 || fuse2)))) {
         if (n_blocks_n > 1) {
             int64_t sum = 0;
@@ -789,7 +790,7 @@ extern "C" size_t glqh_fused_linear_trellis_group_workspace_bytes(int64_t B, int
     // so the fewest K slots) arise from many short layers, the most slots from one tall layer
     int ks2 = 0;
     if (!glqh_trellis_fusein_plan(total_m_pad, n_pad, B, &steps, &ks)) return 0;
-    if (glqh_trellis_mma_fusein_plan((total_m_pad + 63) / 64, n_pad, B, &steps, &ks2) && ks2 > ks) ks = ks2;
+    if (glqh_trellis_mma_fusein_plan((total_m_pad + 63) / 64, n_pad, B, 2, 1, &steps, &ks2) && ks2 > ks) ks = ks2;
     // the separate-transform route (of stacked layers, which takes it at the least): slots of the plain plan (at most 64)
     // and x_rht
     size_t plain = 0;
@@ -1226,7 +1227,7 @@ extern "C" int glqh_fused_linear_trellis_3inst_group_rvq2(const void *x, int x_d
         return glqh_launch_output_rht_group(c.parts, c.su, c.ys, c.scale, c.m_pads, c.outs, n_shards, y_dtype, y_stride,
                                             B, ks, st);
     }
-    GLQH_REQUIRE(tr_fuse_input_enabled() && tr_fusein_plan(c.m_pads, n_shards, n_pad, 1, &steps, &ks, 1) == 2,
+    GLQH_REQUIRE(tr_fuse_input_enabled() && tr_fusein_plan(c.m_pads, n_shards, n_pad, 1, &steps, &ks, true) == 2,
                  "trellis two-stage group: shape not eligible");
     const size_t need = align256((size_t)ks * total * sizeof(float));
     GLQH_REQUIRE(ws && ws_bytes >= need, "trellis two-stage group: workspace of %zu bytes needed, got %zu", need, ws_bytes);
@@ -1411,7 +1412,7 @@ static int moe_proj_plan(const glqh_moe_proj *w, int64_t n_slots, int64_t n_expe
         p->S = (int)S;
         p->ks = (int)((nkp + S - 1) / S);
     } else {
-        GLQH_REQUIRE(glqh_trellis_mma_fusein_plan((w->m_pad / 64) * n_slots, w->n_pad, 1, &p->S, &p->ks),
+        GLQH_REQUIRE(glqh_trellis_mma_fusein_plan((w->m_pad / 64) * n_slots, w->n_pad, 1, p->R2 ? 2 : 1, (int)n_slots, &p->S, &p->ks),
                      "routed experts %s: no plan", what);
     }
     // both stages in one launch: the per-slot form and the grouped form's passes of 16 rows add the sums in fp32, the

@@ -516,8 +516,15 @@ tr_mma_fusein_body(const uint8_t *__restrict__ packed, const XT *__restrict__ x,
                             0, pscale, 0, 0);
 }
 
+// Four waves a SIMD: without the bound the compiler puts the products' sums into accumulation registers beside 117-133 others,
+// which makes three waves and a second round of any launch of more than 768 workgroups (4096 x 8192, one token: 20.6 -> 17.7 us,
+// 4 + 2 bits 25.4 -> 22.1; 14336 x 4096 at 4 + 2 31.4 -> 28.3; q/k/v of a 4096-wide model 16.2 -> 14.0; two slots of 4096 -> 2 x
+// 2048 experts 32.4 -> 28.4).  With it they are vector registers, up to 128 and no scratch.  (The kernels on transformed
+// activations have room for five to seven waves either way: 0-1 % slower with the sums moved.)
+constexpr int FI_PER_SIMD = 4;
+
 template <int R, typename XT, int TP>
-__global__ void __launch_bounds__(TR_THREADS)
+__global__ void __launch_bounds__(TR_THREADS, FI_PER_SIMD)
 tr_mma_fusein_kernel(const uint8_t *__restrict__ packed, const XT *__restrict__ x, int64_t x_stride,
                      const f16 *__restrict__ sv, int B, int m, int k, int in_features, int S,
                      const glqh_block_meta *__restrict__ bn_meta, int n_blocks, glqh_meta_args margs,
@@ -530,7 +537,7 @@ tr_mma_fusein_kernel(const uint8_t *__restrict__ packed, const XT *__restrict__ 
 // Both stages of a stacked layer (first stage 4 bits/weight, as every recipe of the reference has it:
 // glq_vllm/linear_method.py trellis recipes 5..8 bpw = 4 + 1..4), one token.
 template <int R2, typename XT>
-__global__ void __launch_bounds__(TR_THREADS)
+__global__ void __launch_bounds__(TR_THREADS, FI_PER_SIMD)
 tr_mma_fusein_rvq_kernel(const uint8_t *__restrict__ packed, const uint8_t *__restrict__ packed2, float rs2,
                          const XT *__restrict__ x, int64_t x_stride, const f16 *__restrict__ sv, int m, int k,
                          int in_features, int S, const glqh_block_meta *__restrict__ bn_meta, int n_blocks,
@@ -552,7 +559,7 @@ struct tr_fusein_group {
 };
 
 template <int R, typename XT, int TP>
-__global__ void __launch_bounds__(TR_THREADS)
+__global__ void __launch_bounds__(TR_THREADS, FI_PER_SIMD)
 tr_mma_fusein_group_kernel(tr_fusein_group g, const XT *__restrict__ x, int64_t x_stride, int B, int k,
                            int in_features, int S, const glqh_block_meta *__restrict__ bn_meta,
                            int n_blocks, glqh_meta_args margs) {
@@ -577,7 +584,7 @@ struct tr_fusein_group_rvq {
 };
 
 template <int R2, typename XT>
-__global__ void __launch_bounds__(TR_THREADS)
+__global__ void __launch_bounds__(TR_THREADS, FI_PER_SIMD)
 tr_mma_fusein_group_rvq_kernel(tr_fusein_group g, tr_fusein_group_rvq g2, const XT *__restrict__ x, int64_t x_stride,
                                int k, int in_features, int S, const glqh_block_meta *__restrict__ bn_meta,
                                int n_blocks, glqh_meta_args margs) {
@@ -613,7 +620,7 @@ struct tr_moe_args {
 };
 
 template <int R, typename XT>
-__global__ void __launch_bounds__(TR_THREADS)
+__global__ void __launch_bounds__(TR_THREADS, FI_PER_SIMD)
 tr_mma_fusein_moe_kernel(tr_moe_args g, const XT *__restrict__ x, int64_t x_stride, const f16 *__restrict__ sv,
                          int m, int k, int in_features, int S, const glqh_block_meta *__restrict__ bn_meta,
                          int n_blocks, glqh_meta_args margs) {
@@ -630,7 +637,7 @@ tr_mma_fusein_moe_kernel(tr_moe_args g, const XT *__restrict__ x, int64_t x_stri
 // Two-stage experts (first stage 4 bits/weight): both streams of the slot's expert in the same launch, the second
 // one's sums times the expert's inv_resid_scale2 (read on the device) added in registers.
 template <int R2, typename XT>
-__global__ void __launch_bounds__(TR_THREADS)
+__global__ void __launch_bounds__(TR_THREADS, FI_PER_SIMD)
 tr_mma_fusein_moe_rvq_kernel(tr_moe_args g, const uint8_t *__restrict__ packed2, int64_t stride2_bytes,
                              const XT *__restrict__ x, int64_t x_stride, const f16 *__restrict__ sv, int m, int k,
                              int in_features, int S, const glqh_block_meta *__restrict__ bn_meta, int n_blocks,
@@ -1037,22 +1044,39 @@ int glqh_launch_trellis_mma_group(const f16 *const x[], int64_t B, const void *c
 }
 
 // ---- fused-input GEMV (MFMA form): plan and launch -----------------------------------
-// S k-pairs per K slot: a power of two >= 8 chosen so that about four workgroups per CU are
-// in flight; the slice 32*S is capped by LDS (8192 columns at one token, 4096 at 2..4).
-int glqh_trellis_mma_fusein_plan(int64_t wgs_rows, int64_t k, int64_t B, int *S_out, int *ksplit_out) {
+// S k-pairs per K slot: a power of two >= 8; the slice 32*S is capped by LDS (8192 columns at one token, 4096 at 2..4).
+// More rows never get more slots, nor do single-stage layers, in groups or alone, more than a stacked one of their size:
+// workspaces rely on it.
+int glqh_trellis_mma_fusein_plan(int64_t wgs_rows, int64_t k, int64_t B, int n_stages, int n_layers, int *S_out, int *ksplit_out) {
     if (B < 1 || B > 4 || wgs_rows < 1) return 0;
-    const int64_t nkp = k / 32;
-    const int64_t target = (int64_t)glqh_device_cus() * 4;
-    int64_t ks_target = (target + wgs_rows - 1) / wgs_rows;
-    if (ks_target < 1) ks_target = 1;
+    const int64_t nkp = k / 32, cus = glqh_device_cus();
+    const int64_t ks_target = std::max<int64_t>((cus * 4 + wgs_rows - 1) / wgs_rows, 1);   // four workgroups per CU at most
     const int64_t want = (nkp + ks_target - 1) / ks_target;
     int64_t S = 2 * TR_WAVES;                                   // at least 256 columns per slot
     // Every workgroup sums the (block / slice) sub-slices of its Hadamard block before it
     // decodes anything: 256-column slices of a block of 4096 points or more are 16+ terms in
     // front of two records per wave (4096 x 4096: 17.6 us per linear with them, 11.9 us with
-    // 512-column slices).
+    // 512-column slices; 2048 x 8192, one stage: 12.5 us with those, 11.4 with 1024-column slices, but 15.5 / 16.5 at 4 + 2
+    // bits, whose records outweigh the terms).
     if (k >= 4096) S = 4 * TR_WAVES;
+    if (k >= 8192 && B == 1 && n_stages == 1) S = 8 * TR_WAVES;
     while (S < want) S <<= 1;
+    // One token: a fourth workgroup on a CU costs more in transforms and in sums for the finishing launch to read (from the
+    // memory side, at 25-50 bytes a ns) than it hides.  Up to 1024-column slices, which the registers transform (2048: +4 us).
+    // Whole linear, us, at S = 8 / 16 / 32, by workgroups:
+    //   1024 at 16   4096 x 8192 - / 17.7 / 14.5, 8192 x 4096 - / 17.5 / 14.6
+    //    896         2048 x 14336 - / 16.8 / 14.0, 4096 x 7168 - / 15.9 / 13.9
+    //    768         8192 x 3072 - / 14.5 / 13.9, 6144 x 4096 - / 12.9 / 13.3, 4096 x 6144 - / 13.2 / 13.4
+    //    512         4096 x 4096 - / 11.4 / 11.6
+    //   1024 at 8    8192 x 2048 14.7 / 12.0 / 11.5
+    //    512         8192 x 1024 10.2 / 9.2 / 10.0, 4096 x 2048 10.1 / 9.9 / 11.3, but 1024 -> 2 x 4096 9.2 / 9.3 / 10.3
+    //    384         3072 x 2048 8.8 / 8.9 / 10.2
+    //   4 + 2 bits   1024: 8192 x 2048 16.8 / 14.8 / 16.3, 8192 x 4096 - / 22.3 / 20.8; 512: 4096 x 2048 11.4 / 12.2 / 16.3
+    auto many = [&] {
+        const int64_t wgs = wgs_rows * ((nkp + S - 1) / S);
+        return S == 2 * TR_WAVES && n_stages == 1 && n_layers == 1 ? wgs >= 2 * cus : wgs > 3 * cus;
+    };
+    while (B == 1 && S < std::min<int64_t>(8 * TR_WAVES, nkp) && many()) S <<= 1;
     const int64_t cap = B == 1 ? FI_MAX_S : FI_MAX_S_TP4;
     if (S > cap) S = cap;
     *S_out = (int)S;

@@ -181,6 +181,50 @@ def test_few_tokens_of_two_stage_layers(m, n, K, K2, in_f):
         assert float(wide[:, :32].min()) == 7.0 and float(wide[:, 32 + m:].max()) == 7.0
 
 
+@pytest.mark.parametrize("ms,n,K,K2,in_f", [
+    ((8192,), 1024, 4, 0, 1024), ((8160,), 1024, 4, 0, 1000), ((24608,), 512, 2, 0, 512), ((8192,), 2048, 3, 0, 2048),
+    ((2048,), 8192, 4, 0, 8100), ((2080,), 8256, 4, 0, 8256), ((3104,), 4096 + 512, 2, 0, 4608), ((4096,), 4096 - 64, 4, 0, 4032),
+    ((8192,), 2048, 4, 2, 2048), ((1024,), 8192, 4, 2, 8192), ((12320,), 1024, 4, 1, 1024),
+    ((4096, 4128), 1024, 4, 0, 1024), ((3072, 1024, 1056), 3072, 4, 0, 3072), ((8192, 32), 2048, 4, 2, 2000)])
+def test_one_token_at_each_length_of_k_slot(ms, n, K, K2, in_f):
+    """One token through layers, and groups of layers, whose rows and columns lie on either side of the lines between
+    K slots of 256, 512 and 1024 columns, with ragged last slots, strips and input widths: against the oracle, and equal
+    bit for bit on a second call."""
+    from glq_amd import ext, hadamard as H
+    say("one token, K slots", ms, n, K, K2, in_f)
+    bn = O.block_decompose(n)
+    bnt, bnm = torch.tensor(bn), H.pack_block_meta(bn).to(DEV)
+    x = (torch.randn(1, in_f, generator=torch.Generator().manual_seed(sum(ms) + n)) * 0.7).to(torch.bfloat16)
+    xp = np.zeros((1, n), np.float32)                         # columns past in_features are zero padding
+    xp[:, :in_f] = x.float().numpy()
+    refs, layers, one = [], [], None
+    for i, m in enumerate(ms):
+        su, sv = O.rht_signs(m, n, 43 + i)
+        packed = [O.random_packed(m, n, k, 13 + i) for k in (K, K2) if k]
+        W = O.decode_layer(packed[0], m, n, fast=True).astype(np.float32)
+        if K2:
+            W = W + O.decode_layer(packed[1], m, n, fast=True) * np.float32(0.3)
+        bm = O.block_decompose(m)
+        refs.append(O.linear_forward_rht(xp, W * np.float32(0.02), su.astype(np.float32), sv.astype(np.float32), bn, bm, n, m))
+        svd, sud, ps = t(sv.astype(np.float16)), t(su.astype(np.float16)), [t(p) for p in packed]
+        if len(ms) == 1 and not K2:
+            one = lambda: ext.glq_fused_linear_trellis_3inst_cuda(
+                x.to(DEV), svd, sud, ps[0], bnt, torch.tensor(bm), bnm, H.pack_block_meta(bm).to(DEV), 0.02, in_f, m, n, m,
+                out_dtype=torch.bfloat16)
+        elif len(ms) == 1:
+            one = lambda: ext.glq_fused_linear_trellis_3inst_rvq2_cuda(
+                x.to(DEV), svd, sud, *ps, bnt, torch.tensor(bm), bnm, H.pack_block_meta(bm).to(DEV), 0.02, 0.3, in_f, m, n, m,
+                out_dtype=torch.bfloat16)
+        layers.append((svd, sud, *ps, 0.02, 0.3, m, m) if K2 else (svd, sud, *ps, 0.02, m, m))
+    if one is None:
+        call = ext.glq_fused_linear_trellis_3inst_group_rvq2 if K2 else ext.glq_fused_linear_trellis_3inst_group
+        one = lambda: call(x.to(DEV), layers, bnt, bnm, in_f, n, out_dtype=torch.bfloat16)
+    y = one()
+    ref = np.concatenate(refs, axis=1)
+    assert y.shape == ref.shape and rel(y, ref) < TOL, rel(y, ref)
+    assert torch.equal(y, one())
+
+
 def test_two_stage_layers_with_a_launch_per_stage_in_a_fresh_process():
     """GLQ_TRELLIS_FUSE_STAGES=0 (read once by the library): two-stage layers decode their stages in two launches
     at every token count; the two-stage cases of this file and of the module tests against the oracle that way, in
