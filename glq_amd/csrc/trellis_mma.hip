@@ -362,7 +362,7 @@ __device__ __forceinline__ void
 tr_mma_fusein_body(const uint8_t *__restrict__ packed, const XT *__restrict__ x, int64_t x_stride,
                    const f16 *__restrict__ sv, int B, int m, int k, int in_features, int S,
                    const glqh_block_meta *__restrict__ bn_meta, int n_blocks, glqh_meta_args margs,
-                   float *__restrict__ part, float pscale, u32x4 *lds, int part_B = 0,
+                   float *__restrict__ part, float pscale, u32x4 *lds, int strip, int part_B = 0,
                    const uint8_t *__restrict__ packed2 = nullptr, float rs2 = 0.0f) {
     constexpr int TPS = mma_tps<TP>();
     const int Ls = S << 5;
@@ -378,7 +378,7 @@ tr_mma_fusein_body(const uint8_t *__restrict__ packed, const XT *__restrict__ x,
     const int kp0 = slot * S;
     const int kp1 = min(kp0 + S, nkp);
     const int c0 = kp0 << 5;
-    const int mp = min(2 * (int)blockIdx.x + a.hm, mpairs - 1);
+    const int mp = min(2 * strip + a.hm, mpairs - 1);
 
     constexpr int REC = 4 * R;
     const uint8_t *lane_base = packed + ((int64_t)mp * nkp * 32 + a.l) * REC;
@@ -512,7 +512,7 @@ tr_mma_fusein_body(const uint8_t *__restrict__ packed, const XT *__restrict__ x,
     }
     // part_B: rows per K slot of the partial-sum array when it holds more rows than this call's
     // tokens (the routed-expert launch: one row per (token, expert) slot, `part` offset to this one)
-    mma_reduce_store<TP, 1>(acc, (float *)lds, a, wave, part_B > 0 ? part_B : B, m, 0, 64 * blockIdx.x, slot, part,
+    mma_reduce_store<TP, 1>(acc, (float *)lds, a, wave, part_B > 0 ? part_B : B, m, 0, 64 * strip, slot, part,
                             0, pscale, 0, 0);
 }
 
@@ -531,7 +531,7 @@ tr_mma_fusein_kernel(const uint8_t *__restrict__ packed, const XT *__restrict__ 
                      float *__restrict__ part, float pscale) {
     extern __shared__ u32x4 xs_lds[];
     tr_mma_fusein_body<R, XT, TP>(packed, x, x_stride, sv, B, m, k, in_features, S, bn_meta, n_blocks, margs,
-                                  part, pscale, xs_lds);
+                                  part, pscale, xs_lds, blockIdx.x);
 }
 
 // Both stages of a stacked layer (first stage 4 bits/weight, as every recipe of the reference has it:
@@ -544,18 +544,19 @@ tr_mma_fusein_rvq_kernel(const uint8_t *__restrict__ packed, const uint8_t *__re
                          glqh_meta_args margs, float *__restrict__ part) {
     extern __shared__ u32x4 xs_lds[];
     tr_mma_fusein_body<4, XT, 1, R2>(packed, x, x_stride, sv, 1, m, k, in_features, S, bn_meta, n_blocks, margs,
-                                     part, 1.0f, xs_lds, 0, packed2, rs2);
+                                     part, 1.0f, xs_lds, blockIdx.x, 0, packed2, rs2);
 }
 
 // Several layers that read the same activations (fused q/k/v, gate/up:
-// glq_vllm/linear_method.py:664-710) in one launch: blockIdx.z picks the layer, each with
-// its own packed stream, input signs and partial-sum buffer; workgroups past a layer's rows
-// retire.
+// glq_vllm/linear_method.py:664-710) in one launch: blockIdx.x walks the 64-row strips of all of them, each with
+// its own packed stream, input signs and partial-sum buffer.  (With a plane of the grid per layer, as tall as the tallest,
+// half of q/k/v's workgroups had no rows and cost their launch: 2048 -> 2048 + 512 + 512 9.4 -> 9.0 us, 4096 -> 4096 + 1024 + 1024
+// 14.1 -> 13.4, 7168 -> 2048 + 512 + 512 17.3 -> 13.1, at 4 + 2 bits 23.8 -> 17.2; decode step of 8 layers 593 -> 576.)
 struct tr_fusein_group {
     const uint8_t *packed[GLQH_MAX_GROUP];
     const f16 *sv[GLQH_MAX_GROUP];
     float *part[GLQH_MAX_GROUP];
-    int m[GLQH_MAX_GROUP];
+    int m[GLQH_MAX_GROUP], strip0[GLQH_MAX_GROUP];              // first strip (layers past the last: past the grid)
 };
 
 template <int R, typename XT, int TP>
@@ -564,20 +565,20 @@ tr_mma_fusein_group_kernel(tr_fusein_group g, const XT *__restrict__ x, int64_t 
                            int in_features, int S, const glqh_block_meta *__restrict__ bn_meta,
                            int n_blocks, glqh_meta_args margs) {
     extern __shared__ u32x4 xs_lds[];
-    const int z = blockIdx.z;
     const uint8_t *packed = g.packed[0];
     const f16 *sv = g.sv[0];
     float *part = g.part[0];
-    int m = g.m[0];
+    int m = g.m[0], strip = blockIdx.x;
 #pragma unroll
     for (int i = 1; i < GLQH_MAX_GROUP; ++i)
-        if (i == z) { packed = g.packed[i]; sv = g.sv[i]; part = g.part[i]; m = g.m[i]; }
-    if ((int)blockIdx.x * 64 >= m) return;
+        if ((int)blockIdx.x >= g.strip0[i]) {
+            packed = g.packed[i]; sv = g.sv[i]; part = g.part[i]; m = g.m[i]; strip = blockIdx.x - g.strip0[i];
+        }
     tr_mma_fusein_body<R, XT, TP>(packed, x, x_stride, sv, B, m, k, in_features, S, bn_meta, n_blocks, margs,
-                                  part, 1.0f, xs_lds);
+                                  part, 1.0f, xs_lds, strip);
 }
 
-// several stacked layers (4 + R2 bits/weight each) on the same token: blockIdx.z = layer
+// several stacked layers (4 + R2 bits/weight each) on the same token
 struct tr_fusein_group_rvq {
     const uint8_t *packed2[GLQH_MAX_GROUP];
     float rs2[GLQH_MAX_GROUP];
@@ -589,18 +590,19 @@ tr_mma_fusein_group_rvq_kernel(tr_fusein_group g, tr_fusein_group_rvq g2, const 
                                int k, int in_features, int S, const glqh_block_meta *__restrict__ bn_meta,
                                int n_blocks, glqh_meta_args margs) {
     extern __shared__ u32x4 xs_lds[];
-    const int z = blockIdx.z;
     const uint8_t *packed = g.packed[0], *packed2 = g2.packed2[0];
     const f16 *sv = g.sv[0];
     float *part = g.part[0];
     float rs2 = g2.rs2[0];
-    int m = g.m[0];
+    int m = g.m[0], strip = blockIdx.x;
 #pragma unroll
     for (int i = 1; i < GLQH_MAX_GROUP; ++i)
-        if (i == z) { packed = g.packed[i]; packed2 = g2.packed2[i]; rs2 = g2.rs2[i]; sv = g.sv[i]; part = g.part[i]; m = g.m[i]; }
-    if ((int)blockIdx.x * 64 >= m) return;
+        if ((int)blockIdx.x >= g.strip0[i]) {
+            packed = g.packed[i]; packed2 = g2.packed2[i]; rs2 = g2.rs2[i]; sv = g.sv[i]; part = g.part[i]; m = g.m[i];
+            strip = blockIdx.x - g.strip0[i];
+        }
     tr_mma_fusein_body<4, XT, 1, R2>(packed, x, x_stride, sv, 1, m, k, in_features, S, bn_meta, n_blocks, margs, part, 1.0f,
-                                     xs_lds, 0, packed2, rs2);
+                                     xs_lds, strip, 0, packed2, rs2);
 }
 
 // Routed experts of a mixture-of-experts layer, one token each (glq/csrc/glq_cuda.cu:5030-5250,
@@ -631,7 +633,7 @@ tr_mma_fusein_moe_kernel(tr_moe_args g, const XT *__restrict__ x, int64_t x_stri
     tr_mma_fusein_body<R, XT, 1>(g.packed + e * g.stride_bytes, x + (int64_t)(slot / g.x_div) * x_stride, x_stride,
                                  sv, 1, m, k, in_features, S, bn_meta, n_blocks, margs,
                                  g.part + (int64_t)slot * m, g.pscale_dev ? g.pscale_dev[e] : 1.0f, xs_lds,
-                                 g.n_slots);
+                                 blockIdx.x, g.n_slots);
 }
 
 // Two-stage experts (first stage 4 bits/weight): both streams of the slot's expert in the same launch, the second
@@ -648,7 +650,7 @@ tr_mma_fusein_moe_rvq_kernel(tr_moe_args g, const uint8_t *__restrict__ packed2,
     if (e < 0 || e >= g.n_experts) return;                      // uniform over the workgroup
     tr_mma_fusein_body<4, XT, 1, R2>(g.packed + e * g.stride_bytes, x + (int64_t)(slot / g.x_div) * x_stride, x_stride,
                                      sv, 1, m, k, in_features, S, bn_meta, n_blocks, margs,
-                                     g.part + (int64_t)slot * m, 1.0f, xs_lds, g.n_slots, packed2 + e * stride2_bytes,
+                                     g.part + (int64_t)slot * m, 1.0f, xs_lds, blockIdx.x, g.n_slots, packed2 + e * stride2_bytes,
                                      g.pscale_dev[e]);
 }
 
@@ -1071,12 +1073,14 @@ int glqh_trellis_mma_fusein_plan(int64_t wgs_rows, int64_t k, int64_t B, int n_s
     //   1024 at 8    8192 x 2048 14.7 / 12.0 / 11.5
     //    512         8192 x 1024 10.2 / 9.2 / 10.0, 4096 x 2048 10.1 / 9.9 / 11.3, but 1024 -> 2 x 4096 9.2 / 9.3 / 10.3
     //    384         3072 x 2048 8.8 / 8.9 / 10.2
-    //   4 + 2 bits   1024: 8192 x 2048 16.8 / 14.8 / 16.3, 8192 x 4096 - / 22.3 / 20.8; 512: 4096 x 2048 11.4 / 12.2 / 16.3
+    //   4 + 2 bits   1024: 8192 x 2048 16.8 / 14.8 / 16.3, 8192 x 4096 - / 22.3 / 20.8, 2752 -> 2 x 5504 - / 21.8 / 22.3, 2944 -> 2 x
+    //                5888 - / 23.6 / 23.8; 512: 4096 x 2048 11.4 / 12.2 / 16.3
     auto many = [&] {
         const int64_t wgs = wgs_rows * ((nkp + S - 1) / S);
         return S == 2 * TR_WAVES && n_stages == 1 && n_layers == 1 ? wgs >= 2 * cus : wgs > 3 * cus;
     };
-    while (B == 1 && S < std::min<int64_t>(8 * TR_WAVES, nkp) && many()) S <<= 1;
+    const int64_t longest = n_stages > 1 && k < 4096 ? 4 * TR_WAVES : 8 * TR_WAVES;
+    while (B == 1 && S < std::min(longest, nkp) && many()) S <<= 1;
     const int64_t cap = B == 1 ? FI_MAX_S : FI_MAX_S_TP4;
     if (S > cap) S = cap;
     *S_out = (int)S;
@@ -1085,7 +1089,7 @@ int glqh_trellis_mma_fusein_plan(int64_t wgs_rows, int64_t k, int64_t B, int n_s
 }
 
 template <int R, typename XT, int TP>
-static int launch_mma_fusein(const tr_fusein_group &g, int n_layers, int64_t max_m, const void *x,
+static int launch_mma_fusein(const tr_fusein_group &g, int n_layers, int strips, const void *x,
                              int64_t x_stride, int64_t B, int64_t k, int64_t in_features, int S, int ksplit,
                              const glqh_block_meta *bn_meta, const int64_t *blocks_host, int n_blocks,
                              float pscale, hipStream_t stream) {
@@ -1094,13 +1098,12 @@ static int launch_mma_fusein(const tr_fusein_group &g, int n_layers, int64_t max
     const glqh_block_meta *meta = n_blocks > 1 ? bn_meta : nullptr;
     const int nb = n_blocks > 1 ? n_blocks : 1;
     const size_t lds = fi_lds_bytes<TP>(S);
+    const dim3 grid((unsigned)strips, (unsigned)ksplit);
     if (n_layers == 1) {
-        dim3 grid((unsigned)((max_m + 63) / 64), (unsigned)ksplit, 1);
         hipLaunchKernelGGL((tr_mma_fusein_kernel<R, XT, TP>), grid, dim3(TR_THREADS), lds, stream, g.packed[0],
                            (const XT *)x, x_stride, g.sv[0], (int)B, g.m[0], (int)k, (int)in_features, S, meta, nb,
                            margs, g.part[0], pscale);
     } else {
-        dim3 grid((unsigned)((max_m + 63) / 64), (unsigned)ksplit, (unsigned)n_layers);
         hipLaunchKernelGGL((tr_mma_fusein_group_kernel<R, XT, TP>), grid, dim3(TR_THREADS), lds, stream, g,
                            (const XT *)x, x_stride, (int)B, (int)k, (int)in_features, S, meta, nb, margs);
     }
@@ -1119,16 +1122,17 @@ int glqh_launch_trellis_mma_fusein(const void *const packed[], const void *const
     GLQH_REQUIRE(n_layers == 1 || pscale == 1.0f, "trellis group: pre-scaled partial sums are a single-layer option");
     GLQH_REQUIRE(B >= 1 && B <= 4, "fused-input trellis kernel serves 1..4 tokens");
     tr_fusein_group g = {};
-    int64_t max_m = 0;
+    int strips = 0;
     for (int i = 0; i < GLQH_MAX_GROUP; ++i) {
         const int j = i < n_layers ? i : 0;
+        g.strip0[i] = i < n_layers ? strips : INT32_MAX;
+        if (i < n_layers) strips += (int)((m[j] + 63) / 64);
         g.packed[i] = (const uint8_t *)packed[j];
         g.sv[i] = (const f16 *)sv[j];
         g.part[i] = part[j];
         g.m[i] = (int)m[j];
-        if (m[j] > max_m) max_m = m[j];
     }
-#define GLQH_FI(RR, XT, TP) launch_mma_fusein<RR, XT, TP>(g, n_layers, max_m, x, x_stride, B, k, in_features, S, \
+#define GLQH_FI(RR, XT, TP) launch_mma_fusein<RR, XT, TP>(g, n_layers, strips, x, x_stride, B, k, in_features, S, \
                                                           ksplit, bn_meta, blocks_host, n_blocks, pscale, stream)
 #define GLQH_FI_R(RR)                                                                   \
     (B == 1 ? (x_dtype == GLQH_F16 ? GLQH_FI(RR, f16, 1) : GLQH_FI(RR, uint16_t, 1))     \
@@ -1161,18 +1165,19 @@ int glqh_launch_trellis_mma_fusein_rvq(const void *const packed[], const void *c
     const size_t lds = fi_lds_bytes<1>(S);
     tr_fusein_group g = {};
     tr_fusein_group_rvq g2 = {};
-    int64_t max_m = 0;
+    int strips = 0;
     for (int i = 0; i < GLQH_MAX_GROUP; ++i) {
         const int j = i < n_layers ? i : 0;
+        g.strip0[i] = i < n_layers ? strips : INT32_MAX;
+        if (i < n_layers) strips += (int)((m[j] + 63) / 64);
         g.packed[i] = (const uint8_t *)packed[j];
         g.sv[i] = (const f16 *)sv[j];
         g.part[i] = part[j];
         g.m[i] = (int)m[j];
         g2.packed2[i] = (const uint8_t *)packed2[j];
         g2.rs2[i] = rs2[j];
-        if (m[j] > max_m) max_m = m[j];
     }
-    const dim3 grid((unsigned)((max_m + 63) / 64), (unsigned)ksplit, (unsigned)n_layers);
+    const dim3 grid((unsigned)strips, (unsigned)ksplit);
 #define GLQH_FI2(RR, XT)                                                                                        \
     do {                                                                                                        \
         if (n_layers == 1)                                                                                      \
