@@ -545,7 +545,12 @@ extern "C" int glqh_fused_linear_trellis_3inst(
     // 28.7 / 35.2, 8192 x 8192 32.4 / 41.2, 16384 x 8192 52.3 / 59.2; 28672 x 8192: 94.4 / 95.4 at 4+4 but
     // 108.8 / 98.6 at 4+2, hence the bound).
     const bool fuse2 = has_s2 && B == 1 && R1 == 4 && tr_fuse_stages_enabled();
-    const bool fi_pays = tr_fuse_input_enabled() && m_pad * n_pad <= ((int64_t)(fuse2 ? 128 : 32) << 20) &&
+    // One stage, one token: widths of whole 256-column slots fold up to 48 Mi weights and powers of two to 64 (folded /
+    // separate, us: 4096 x 11008 17.5 / 19.7, 11008 x 4096 16.8 / 18.9, 20480 x 2048 16.8 / 19.2, 5056 x 9984 19.1 / 20.6, 14336 x 4096
+    // 18.8 / 19.9, 16384 x 4096 21.7 / 22.9, 8192 x 8192 22.5 / 22.8; past the line 7168 x 7168 18.8 / 17.8, 14336 x 5120 23.1 / 22.6,
+    // 5120 x 13824 23.9 / 21.2; widths of many small blocks 10016 x 5056 22.7 / 20.4, 6688 x 8128 21.7 / 18.4).
+    const int64_t fi_most = fuse2 ? 128 : has_s2 || n_pad % 256 || B > 1 ? 32 : pow2_n && n_pad <= 8192 ? 64 : 48;
+    const bool fi_pays = tr_fuse_input_enabled() && m_pad * n_pad <= fi_most << 20 &&
                          (B == 1 || (B == 2 && pow2_n && n_pad <= 4096 && m_pad <= 4096));
     if (fi_pays && fi_blocks && (x_dtype == GLQH_F16 || x_dtype == GLQH_BF16) &&
         (fi_mode = tr_fusein_plan(&m_pad, 1, n_pad, B, &fi_steps, &ks, fuse2)) != 0 &&
