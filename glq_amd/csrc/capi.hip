@@ -724,17 +724,25 @@ extern "C" int glqh_fused_linear_trellis_3inst_noalloc(
 //   4 bits, 2 tokens  960 14.3 / 12.2, 2048 12.8 / 13.3, 3072 18.3 / 14.4; 1024 -> 2 x 2560 11.6 / 12.8,
 //                     2048 -> 2 x 11008 19.6 / 20.9, 3392 -> 2 x 7040 25.1 / 20.8
 //   4 bits, 4 tokens  960 18.0 / 12.6, 2048 15.8 / 13.4; 2048 -> 2 x 11008 22.5 / 21.5
-// and one token of single-stage groups above 96M weights (4096 -> 2 x 14336: 37.4 / 33.9), below 32M (11008 -> 2048, a
-// group of one: 14.3 / 18) never.  Widths of whole 256-column slots fold better (no workgroup transforms a ragged tail
-// beside its share of the large block): up to 4096 columns, where slots are that short, they cross at 48M weights
-// instead of 32M (40M: 15.1 / 15.9 us, 56M: 20.1 / 19.2).  The fused-input launches serve up to four tokens, one of
-// stacked layers.
+// The lines at one token are drawn with four waves a SIMD and one grid over all strips (the kernels above had three and a
+// plane per layer; two and four tokens stand).  Whole call, us, folded / separate, 4 bits and 4 + 2, by Mi weights of the group:
+//   whole slots (256)  4608 wide 36 14.4 / 16.4, 20.8 / 23.1; 5120 35 16.2 / 16.7, 23.5 / 22.9; 6144 48 16.6 / 17.5, 24.0 / 24.9; 7168 42 16.6 /
+//                      17.6, 24.0 / 25.1; 8192 48 17.4 / 18.6, 25.2 / 26.0, 80 28.2 / 25.5, 43 / 37; 4096 48 16.1 / 17.1, 24.1 / 24.8, 56 18.2 /
+//                      18.2, 27.9 / 27.0, 64 19.3 / 20.2, 28.9 / 29.8, 86 26.6 / 24.6; 3840 60 19.7 / 19.2; 3584 56 17.5 / 18.8, 24.6 / 27.2,
+//                      65 21.2 / 20.4
+//   other widths       (a workgroup at the end of a row transforms many small blocks) 2752 29 15.9 / 14.7, 20.6 / 20.1; 2944 33 16.8 /
+//                      15.2, 22.0 / 21.1; 3136 38 16.1 / 15.6; 3520 48 18.0 / 17.1; 3136 14 10.4 / 11.5; 2240 19 12.5 / 13.6, 16.4 / 17.5
+// Single-stage groups above 96 Mi never fold (4096 -> 2 x 14336: 31.1 / 27.4).  The fused-input launches serve up to four tokens,
+// one of stacked layers.
 static bool tr_group_plain(int64_t total_m_pad, int64_t n_pad, int64_t B, bool stacked) {
     if (!tr_fuse_input_enabled() || B > 4 || (stacked && B > 1)) return true;
     const int64_t w = total_m_pad * n_pad;
-    const int64_t folds = !stacked && n_pad <= 4096 && n_pad % 256 == 0 ? 48 : 32;
-    if (B == 1) return (n_pad > 3072 && w > folds << 20) || (!stacked && w > ((int64_t)96 << 20));
-    return B > 2 || n_pad > 2048 || (n_pad & (n_pad - 1)) != 0;
+    const bool pow2_n = (n_pad & (n_pad - 1)) == 0;
+    if (B > 1) return B > 2 || n_pad > 2048 || !pow2_n;
+    if (n_pad % 256 && n_pad > 2048) return w > (int64_t)28 << 20;
+    if (n_pad > 4096 || (stacked && n_pad > 3072)) return w > (int64_t)48 << 20;
+    if (n_pad > 3072) return w > (int64_t)(pow2_n ? 64 : 56) << 20;
+    return !stacked && w > (int64_t)96 << 20;
 }
 // The grouped call at many tokens: more than 64 tokens, at most four layers.  The K split of a group is at most
 // that of a single 128-row layer of the same width (fewer row tiles, more slots).
