@@ -185,11 +185,13 @@ def test_few_tokens_of_two_stage_layers(m, n, K, K2, in_f):
     ((8192,), 1024, 4, 0, 1024), ((8160,), 1024, 4, 0, 1000), ((24608,), 512, 2, 0, 512), ((8192,), 2048, 3, 0, 2048),
     ((2048,), 8192, 4, 0, 8100), ((2080,), 8256, 4, 0, 8256), ((3104,), 4096 + 512, 2, 0, 4608), ((4096,), 4096 - 64, 4, 0, 4032),
     ((8192,), 2048, 4, 2, 2048), ((1024,), 8192, 4, 2, 8192), ((12320,), 1024, 4, 1, 1024),
-    ((4096, 4128), 1024, 4, 0, 1024), ((3072, 1024, 1056), 3072, 4, 0, 3072), ((8192, 32), 2048, 4, 2, 2000)])
+    ((4096, 4128), 1024, 4, 0, 1024), ((3072, 1024, 1056), 3072, 4, 0, 3072), ((8192, 32), 2048, 4, 2, 2000),
+    ((32, 96, 2048, 64), 5120, 4, 0, 5120), ((11008,), 4096, 4, 0, 4096), ((5504, 5536), 2752, 2, 0, 2700),
+    ((4608, 4640), 4608, 3, 0, 4600)])
 def test_one_token_at_each_length_of_k_slot(ms, n, K, K2, in_f):
     """One token through layers, and groups of layers, whose rows and columns lie on either side of the lines between
-    K slots of 256, 512 and 1024 columns, with ragged last slots, strips and input widths: against the oracle, and equal
-    bit for bit on a second call."""
+    K slots of 256, 512 and 1024 columns, and of the lines up to which the input transform folds in, with ragged last
+    slots, strips and input widths: against the oracle, and equal bit for bit on a second call."""
     from glq_amd import ext, hadamard as H
     say("one token, K slots", ms, n, K, K2, in_f)
     bn = O.block_decompose(n)
