@@ -539,7 +539,7 @@ extern "C" int glqh_fused_linear_trellis_3inst(
     // 5120 x 5120 17.0 / 15.8 -- the one loss; two tokens: 4096 x 4096 15.0 / 16.1, but 3072 x 8192 19.3 / 16.2 and
     // 6144 x 2048 14.7 / 13.2, hence the size bound on two tokens).
     // One token of a two-stage layer (first stage 4 bits/weight) takes the MFMA form at every height and up to
-    // four times the size, both streams in one launch: the alternative is a transform, two decode launches
+    // 128 Mi weights, both streams in one launch: the alternative is a transform, two decode launches
     // and a finishing one (whole linear, us, one launch / two or three: 4096 x 4096 at 4+2 15.5 / 22.0, 2048 x 2048
     // 9.5 / 14.4, 11008 x 2048 17.7 / 25.0, 512 x 2048 8.7 / 15.0, 128 x 4096 10.9 / 17.0, 14336 x 4096 at 4+4
     // 28.7 / 35.2, 8192 x 8192 32.4 / 41.2, 16384 x 8192 52.3 / 59.2; 28672 x 8192: 94.4 / 95.4 at 4+4 but
