@@ -1058,10 +1058,9 @@ int glqh_trellis_mma_fusein_plan(int64_t wgs_rows, int64_t k, int64_t B, int n_s
     // Every workgroup sums the (block / slice) sub-slices of its Hadamard block before it
     // decodes anything: 256-column slices of a block of 4096 points or more are 16+ terms in
     // front of two records per wave (4096 x 4096: 17.6 us per linear with them, 11.9 us with
-    // 512-column slices; 2048 x 8192, one stage: 12.5 us with those, 11.4 with 1024-column slices, but 15.5 / 16.5 at 4 + 2
-    // bits, whose records outweigh the terms).
+    // 512-column slices).  1024-column slices of widths from 8192 on, where the rows leave CUs idle, are for nothing over all rates:
+    // 2048 x 8192 11.9 -> 10.8 us at 4 bits, 12.8 -> 13.8 at 2, 13.3 -> 13.9 at 3, 2048 x 11008 13.3 -> 13.1, 13.7 -> 14.8, 13.8 -> 14.9.
     if (k >= 4096) S = 4 * TR_WAVES;
-    if (k >= 8192 && B == 1 && n_stages == 1) S = 8 * TR_WAVES;
     while (S < want) S <<= 1;
     // One token: a fourth workgroup on a CU costs more in transforms and in sums for the finishing launch to read (from the
     // memory side, at 25-50 bytes a ns) than it hides.  Up to 1024-column slices, which the registers transform (2048: +4 us).

@@ -227,6 +227,27 @@ def test_one_token_at_each_length_of_k_slot(ms, n, K, K2, in_f):
     assert torch.equal(y, one())
 
 
+@pytest.mark.parametrize("K", [2, 3, 4])
+def test_down_projection_at_one_token_in_slots_of_512_columns(K):
+    """2048 x 11008 at one token: 22 K slots of sums, and nothing behind them.  The finishing launch adds them in their order, so
+    the bits of the decode step hang on their number."""
+    from glq_amd import _lib
+    say("down projection, slots", K)
+    lib, m, n = _lib.load(), 2048, 11008
+    bn = torch.tensor(O.block_decompose(n))
+    meta = t(O.pack_block_meta(O.block_decompose(n)))
+    su, sv = (t(s.astype(np.float16)) for s in O.rht_signs(m, n, 5))
+    packed = t(O.random_packed(m, n, K, 7))
+    x, y = torch.ones(1, n, dtype=torch.bfloat16, device=DEV), torch.empty(1, m, dtype=torch.bfloat16, device=DEV)
+    ws = torch.full((lib.glqh_fused_linear_trellis_workspace_bytes(1, n, m),), 255, dtype=torch.uint8, device=DEV)   # NaN
+    _lib.check(lib.glqh_fused_linear_trellis_3inst(
+        x.data_ptr(), _lib.GLQH_BF16, n, 1, sv.data_ptr(), su.data_ptr(), packed.data_ptr(), packed.shape[0], packed.shape[1], None,
+        0, 0, bn.data_ptr(), bn.numel(), None, 1, meta.data_ptr(), None, 0.02, 0.0, n, m, n, m, y.data_ptr(), _lib.GLQH_BF16, m, None,
+        0, ws.data_ptr(), ws.numel(), torch.cuda.current_stream().cuda_stream))
+    written = ~ws[(2 * n + 255) // 256 * 256:].view(torch.float32).isnan()
+    assert int(written.sum()) == 22 * m and bool(written[:22 * m].all())
+
+
 def test_two_stage_layers_with_a_launch_per_stage_in_a_fresh_process():
     """GLQ_TRELLIS_FUSE_STAGES=0 (read once by the library): two-stage layers decode their stages in two launches
     at every token count; the two-stage cases of this file and of the module tests against the oracle that way, in
