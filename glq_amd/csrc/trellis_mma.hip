@@ -1074,9 +1074,15 @@ int glqh_trellis_mma_fusein_plan(int64_t wgs_rows, int64_t k, int64_t B, int n_s
     //    384         3072 x 2048 8.8 / 8.9 / 10.2
     //   4 + 2 bits   1024: 8192 x 2048 16.8 / 14.8 / 16.3, 8192 x 4096 - / 22.3 / 20.8, 2752 -> 2 x 5504 - / 21.8 / 22.3, 2944 -> 2 x
     //                5888 - / 23.6 / 23.8; 512: 4096 x 2048 11.4 / 12.2 / 16.3
+    // Widths that are not whole 256-column slots take a fourth workgroup at 512 columns: their tails' small blocks make the longer slots
+    // dear, at 2 and 3 bits above all (S = 16 / 32 at 2, 3, 4 bits: 774 workgroups, 2752 -> 3 x 2752 12.4 / 13.8, 12.2 / 14.3,
+    // 12.2 / 12.8; 828, 2944 -> 3 x 2944 13.3 / 14.8, 13.2 / 14.9, 12.9 / 13.5; 940, 2240 -> 2 x 6016 13.2 / 13.4, 13.1 / 14.0, 13.1 / 12.9;
+    // 1029, 3136 -> 3 x 3136 13.1 / 12.8, 13.0 / 12.8, 12.9 / 12.2).  Below 1024 columns two short slots are too few (S = 8 / 16: 8192 x
+    // 960 11.4 / 12.0, 11.5 / 12.1, 11.4 / 11.3).
     auto many = [&] {
         const int64_t wgs = wgs_rows * ((nkp + S - 1) / S);
-        return S == 2 * TR_WAVES && n_stages == 1 && n_layers == 1 ? wgs >= 2 * cus : wgs > 3 * cus;
+        if (S == 2 * TR_WAVES && n_stages == 1 && n_layers == 1 && k >= 1024) return wgs >= 2 * cus;
+        return wgs > (S > 2 * TR_WAVES && k % 256 ? 4 : 3) * cus;
     };
     const int64_t longest = n_stages > 1 && k < 4096 ? 4 * TR_WAVES : 8 * TR_WAVES;
     while (B == 1 && S < std::min(longest, nkp) && many()) S <<= 1;

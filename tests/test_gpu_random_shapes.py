@@ -248,6 +248,36 @@ def test_down_projection_at_one_token_in_slots_of_512_columns(K):
     assert int(written.sum()) == 22 * m and bool(written[:22 * m].all())
 
 
+@pytest.mark.parametrize("K", [2, 3, 4])
+@pytest.mark.parametrize("ms,n,slots", [((2752, 2752, 2752), 2752, 6), ((2944, 2944, 2944), 2944, 6), ((6016, 6016), 2240, 5),
+                                        ((3136, 3136, 2496), 3136, 7), ((8192,), 960, 4), ((8192,), 1024, 2)])
+def test_slots_of_ragged_widths_at_one_token(ms, n, slots, K):
+    """Groups whose width is not whole 256-column slots keep slots of 512 columns up to four workgroups a CU, a single layer
+    below 1024 columns those of 256 up to three."""
+    from glq_amd import ext, hadamard as H
+    say("ragged widths, slots", ms, n, K)
+    g = torch.Generator(device=DEV).manual_seed(n)
+    sign = lambda k: (torch.randint(0, 2, (k,), generator=g, device=DEV) * 2 - 1).to(torch.float16)
+    layers = [(sign(n), sign(m), torch.randint(-32768, 32768, (m // 16 * (n // 16), 16 * K), generator=g, device=DEV, dtype=torch.int16),
+               0.02, m, m) for m in ms]
+    bn = O.block_decompose(n)
+    taken, plain = [], ext._ws
+
+    def kept(nbytes, device):
+        taken.append(torch.full((nbytes,), 255, dtype=torch.uint8, device=device))   # NaN
+        return taken[-1]
+
+    ext._ws = kept
+    try:
+        ext.glq_fused_linear_trellis_3inst_group(torch.ones(1, n, dtype=torch.bfloat16, device=DEV), layers, torch.tensor(bn),
+                                                 H.pack_block_meta(bn).to(DEV), n, n, out_dtype=torch.bfloat16)
+    finally:
+        ext._ws = plain
+    assert len(taken) == 1
+    written = ~taken[0][:taken[0].numel() // 4 * 4].view(torch.float32).isnan()
+    assert int(written.sum()) == slots * sum(ms) and bool(written[:slots * sum(ms)].all()), int(written.sum()) / sum(ms)
+
+
 def test_two_stage_layers_with_a_launch_per_stage_in_a_fresh_process():
     """GLQ_TRELLIS_FUSE_STAGES=0 (read once by the library): two-stage layers decode their stages in two launches
     at every token count; the two-stage cases of this file and of the module tests against the oracle that way, in
