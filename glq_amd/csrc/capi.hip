@@ -732,6 +732,14 @@ extern "C" int glqh_fused_linear_trellis_3inst_noalloc(
 //                      65 21.2 / 20.4
 //   other widths       (a workgroup at the end of a row transforms many small blocks) 2752 29 15.9 / 14.7, 20.6 / 20.1; 2944 33 16.8 /
 //                      15.2, 22.0 / 21.1; 3136 38 16.1 / 15.6; 3520 48 18.0 / 17.1; 3136 14 10.4 / 11.5; 2240 19 12.5 / 13.6, 16.4 / 17.5
+// Stacked groups wider than 4096 columns are a few long workgroups to a CU (1024-column slots), which the separate route is not: up to 48 Mi
+// they fold where those are two, or three on most CUs, a slot of 768 columns or more counting as one (by workgroups, 4 + 2 bits; 4 + 1
+// and 4 + 4 alike):
+//   up to 512          4608 30 19.6 / 20.1, 36 20.0 / 22.2; 5120 30 19.1 / 19.8; 5632 33 19.0 / 20.9; 6144 30 19.8 / 20.2; 7424 33 19.1 / 20.1;
+//                      8192 32 19.6 / 20.4
+//   520 to 600         4608 40 23.5 / 22.4; 4864 33 21.8 / 20.4; 5120 34 22.9 / 22.2, 38 22.9 / 22.2; 5376 34 23.1 / 22.5; 5632 36 23.0 / 22.3;
+//                      5888 32 21.1 / 19.3; 6144 33 22.1 / 21.0, 36 23.3 / 22.3; 7168 35 22.2 / 21.3; 8192 33 23.2 / 22.4
+//   660 and more       5632 45 23.7 / 24.4; 6144 42 23.5 / 23.2; 7168 42 23.4 / 24.5; 8192 48 25.2 / 26.0
 // Single-stage groups above 96 Mi never fold (4096 -> 2 x 14336: 31.1 / 27.4).  The fused-input launches serve up to four tokens,
 // one of stacked layers.
 static bool tr_group_plain(int64_t total_m_pad, int64_t n_pad, int64_t B, bool stacked) {
@@ -740,7 +748,12 @@ static bool tr_group_plain(int64_t total_m_pad, int64_t n_pad, int64_t B, bool s
     const bool pow2_n = (n_pad & (n_pad - 1)) == 0;
     if (B > 1) return B > 2 || n_pad > 2048 || !pow2_n;
     if (n_pad % 256 && n_pad > 2048) return w > (int64_t)28 << 20;
-    if (n_pad > 4096 || (stacked && n_pad > 3072)) return w > (int64_t)48 << 20;
+    if (stacked && n_pad > 4096) {
+        const int64_t cus = glqh_device_cus(), wgs = (total_m_pad + 63) / 64 * ((n_pad + 256) / 1024);
+        if (wgs > 2 * cus && wgs <= 5 * cus / 2) return true;
+    }
+    if (n_pad > 4096) return w > (int64_t)48 << 20;
+    if (stacked && n_pad > 3072) return w > (int64_t)48 << 20;
     if (n_pad > 3072) return w > (int64_t)(pow2_n ? 64 : 56) << 20;
     return !stacked && w > (int64_t)96 << 20;
 }

@@ -278,6 +278,37 @@ def test_slots_of_ragged_widths_at_one_token(ms, n, slots, K):
     assert int(written.sum()) == slots * sum(ms) and bool(written[:slots * sum(ms)].all()), int(written.sum()) / sum(ms)
 
 
+@pytest.mark.parametrize("ms,n,folds", [((4608, 2304, 2304), 4608, False), ((5120, 1280, 1280), 5120, False), ((4096, 1024, 1024), 6144, False),
+                                        ((3072, 1344, 1344), 5888, False), ((4608, 1792, 1792), 4608, True), ((4096, 1024, 1024), 5120, True),
+                                        ((2048, 1024, 1024), 8192, True), ((4096, 1024, 1024), 7168, True), ((4096, 4096, 4096), 4096, True)])
+def test_where_the_input_transform_of_stacked_groups_folds_in(ms, n, folds):
+    """One token of stacked groups on either side of the line: the workspace begins with the transformed activations where
+    they have a launch of their own, with partial sums where they have not."""
+    from glq_amd import ext, hadamard as H
+    say("stacked groups, route", ms, n)
+    g = torch.Generator(device=DEV).manual_seed(n)
+    sign = lambda k: (torch.randint(0, 2, (k,), generator=g, device=DEV) * 2 - 1).to(torch.float16)
+    bits = lambda m, K: torch.randint(-32768, 32768, (m // 16 * (n // 16), 16 * K), generator=g, device=DEV, dtype=torch.int16)
+    layers = [(sign(n), sign(m), bits(m, 4), bits(m, 2), 0.02, 0.3, m, m) for m in ms]
+    bn = O.block_decompose(n)
+    bnt, bnm = torch.tensor(bn), H.pack_block_meta(bn).to(DEV)
+    x = torch.randn(1, n, generator=g, device=DEV).to(torch.bfloat16)
+    x_rht = torch.empty(1, n, dtype=torch.float16, device=DEV)
+    ext.glq_input_rht_blockdiag_cuda(x, layers[0][0], x_rht, n, n, bnt, bnm)
+    taken, plain = [], ext._ws
+
+    def kept(nbytes, device):
+        taken.append(plain(nbytes, device))
+        return taken[-1]
+
+    ext._ws = kept
+    try:
+        ext.glq_fused_linear_trellis_3inst_group_rvq2(x, layers, bnt, bnm, n, n, out_dtype=torch.bfloat16)
+    finally:
+        ext._ws = plain
+    assert len(taken) == 1 and torch.equal(taken[0][:2 * n].view(torch.float16), x_rht[0]) != folds
+
+
 def test_two_stage_layers_with_a_launch_per_stage_in_a_fresh_process():
     """GLQ_TRELLIS_FUSE_STAGES=0 (read once by the library): two-stage layers decode their stages in two launches
     at every token count; the two-stage cases of this file and of the module tests against the oracle that way, in
