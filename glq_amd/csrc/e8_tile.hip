@@ -749,12 +749,25 @@ static double et_plan_cost(const et_plan &p, int64_t m_pad, int64_t M) {
     return t;
 }
 
+// K slots above 256 tokens, by rounds of workgroups that end together: as for the trellis tile kernel, they decide what a call returns
+// and do not follow the tile that runs them.
+static double et_split_cost(const et_plan &p, int64_t m_pad, int64_t M) {
+    const int cus = glqh_device_cus();
+    const int64_t items = (int64_t)p.RT * p.TT * p.KS, full = items / cus, rem = items % cus;
+    double rounds = (double)full, slow = 1.0;
+    if (full == 0) {
+        rounds = 1.0;
+        slow = 1.0 + 0.6 * (1.0 - (double)items / cus);
+    } else if (rem > 0) {
+        rounds += std::max(0.5, (double)rem / cus);
+    }
+    double t = rounds * p.slot_ds * (p.NTW == 4 ? 2.75 : 1.65) * slow;
+    if (p.KS > 1) t += 2.0 * p.KS * (double)M * (double)m_pad * 4.0 / 4.0e6;
+    return t;
+}
+
 // Above 256 tokens: 512-token tiles (one- and two-stage layers) unless 256-token tiles are expected to be 3 % faster, which
-// they are where they waste less on padding or need fewer K slots (5120 x 5120 at 768 tokens 74 -> 68 us, the whole call).  Over
-// 72 shapes (2048-14336 rows and columns, 300-4096 tokens) the rule takes the faster one but for 0.02 % of the sum; 512-token
-// tiles throughout lose 0.6 %.  (A step slower by 0.6 of the idle share, which was the second round of glqh_xcd_share's comment, and
-// a last round that counted in proportion, lost 4.8 %: 5120 x 5120 at 2048 tokens 194 -> 149 us, 14336 x 4096 at 512 97 -> 84.)
-// GLQ_ET_NTW forces a tile.
+// they are where they waste less on padding (5120 x 5120 at 768 tokens 74 -> 68 us, the whole call).  GLQ_ET_NTW forces a tile.
 int et_make_plan(int64_t m_pad, int64_t n_pad, int64_t M, int nstages, et_plan *p) {
     if (M < 1 || m_pad < 1 || n_pad < 256 || (n_pad & 255) || M > ((int64_t)1 << 22) || m_pad > ((int64_t)1 << 24))
         return 0;
@@ -764,6 +777,13 @@ int et_make_plan(int64_t m_pad, int64_t n_pad, int64_t M, int nstages, et_plan *
     if (top < 4 || forced) return 1;
     et_plan p2;
     et_plan_for(2, m_pad, n_pad, M, &p2);
+    const et_plan &split = et_split_cost(p2, m_pad, M) < 0.95 * et_split_cost(*p, m_pad, M) ? p2 : *p;
+    const int KS = split.KS, slot_ds = split.slot_ds;
+    for (et_plan *q : {p, &p2}) {
+        q->KS = KS;
+        q->slot_ds = slot_ds;
+        q->grid = (int)std::min<int64_t>((int64_t)q->RT * q->TT * KS, glqh_device_cus());
+    }
     if (et_plan_cost(p2, m_pad, M) < 0.97 * et_plan_cost(*p, m_pad, M)) *p = p2;
     return 1;
 }

@@ -872,11 +872,29 @@ double tt_plan_cost(const tt_plan &p, int64_t m, int64_t M, bool alone) {
     return t;
 }
 
+// K slots above 256 tokens: those that 512-token tiles need to fill the chip, or those that 256-token tiles need where that
+// is expected to be 5 % faster, by rounds of workgroups that end together.  Slots are sums of their own, up to 16 of them rounded to
+// fp16: their number decides what a call returns, and whether in fp32, so it hangs on this rule alone and not on the tile
+// that runs them, which is a matter of time.  (With the slots of the faster tile the outputs of a prompt moved wherever the costs below
+// did, sums of 17-21 slots went from fp32 to fp16, and fp16 ones to fp32 and 12 % more time: 512 x 14336 at 1024 tokens 51.1 -> 57.4 us.)
+double tt_split_cost(const tt_plan &p, int64_t m, int64_t M) {
+    const int cus = glqh_device_cus();
+    const int64_t items = (int64_t)p.RT * p.TT * p.KS, full = items / cus, rem = items % cus;
+    double rounds = (double)full, slow = 1.0;
+    if (full == 0) {
+        rounds = 1.0;
+        slow = 1.0 + 0.6 * (1.0 - (double)items / cus);
+    } else if (rem > 0) {
+        rounds += std::max(0.5, (double)rem / cus);
+    }
+    double t = rounds * p.slot_ds * (p.NTW == 4 ? 2.26 : 1.7) * slow;
+    if (p.KS > 1) t += 2.0 * p.KS * (double)M * (double)m * 3 / 4.0e6;
+    return t;
+}
+
 // Up to 256 tokens the tile follows the token count; above, 512-token tiles unless 256-token tiles are expected to be 3 %
-// faster: where they waste less on padding (2 x 14336 rows x 4096 columns at 768 tokens 261 -> 236 us, the whole call), need
-// fewer K slots (2048 x 2048 at 2048 tokens 73 -> 58) or leave a shorter last round.  Over 70 shapes (fused q/k/v and gate/up,
-// layers of 2048-14336 rows and columns; 300-4096 tokens) the rule takes the faster one but for 0.3 % of the sum; 512-token tiles
-// throughout lose 1 % of it.  GLQ_TT_NTW forces a tile above 256 tokens.
+// faster: where they waste less on padding (2 x 14336 rows x 4096 columns at 768 tokens 261 -> 236 us, the whole call) or leave a
+// shorter last round.  GLQ_TT_NTW forces a tile above 256 tokens.
 // max_ntw = 2: a stacked layer decoded into one operand (two streams' records and temporaries do not fit beside the
 // accumulators of a 512-token tile).
 void tt_make_plan(int64_t m, int64_t k, int64_t M, tt_plan *p, int max_ntw = 4, bool alone = true) {
@@ -886,6 +904,13 @@ void tt_make_plan(int64_t m, int64_t k, int64_t M, tt_plan *p, int max_ntw = 4, 
     if (top < 4 || forced) return;
     tt_plan p2;
     tt_plan_for(2, m, k, M, &p2);
+    const tt_plan &split = tt_split_cost(p2, m, M) < 0.95 * tt_split_cost(*p, m, M) ? p2 : *p;
+    const int KS = split.KS, slot_ds = split.slot_ds;
+    for (tt_plan *q : {p, &p2}) {
+        q->KS = KS;
+        q->slot_ds = slot_ds;
+        q->grid = (int)std::min<int64_t>((int64_t)q->RT * q->TT * KS, glqh_device_cus());
+    }
     if (tt_plan_cost(p2, m, M, alone) < 0.97 * tt_plan_cost(*p, m, M, alone)) *p = p2;
 }
 

@@ -391,3 +391,35 @@ def test_fusein_gemv_matches_unfused_pipeline(ext):
     # the fused kernel builds its slice of the transform in a different summation order
     assert rel(out, ref) < 1e-3, rel(out, ref)
     assert torch.equal(out, ext.glq_decode_matvec_trellis_3inst_fusein_cuda(x_raw, sv, p, m, n, inf, 0.01371))
+
+
+@pytest.mark.parametrize("m,B", [(800, 600), (864, 561)])
+def test_sums_of_more_than_16_slots_stay_fp32(ext, m, B):
+    """16384 columns in 18 K slots, activations that the transform leaves exact (one column each: x_rht = +-1), fp32 results: what is
+    left is the products' and transforms' fp32 rounding, a few 2^-24 times the root of the number of terms each; sums
+    rounded to fp16 are off by 1.6e-4."""
+    n = 16384
+    say("more than 16 slots", m, B)
+    g = torch.Generator(device=DEV).manual_seed(m)
+    packed = torch.randint(-32768, 32768, (m // 16 * (n // 16), 64), generator=g, device=DEV, dtype=torch.int16)
+    sv, su = (torch.randint(0, 2, (k,), generator=g, device=DEV).mul_(2).sub_(1).to(torch.float16) for k in (n, m))
+    at = torch.randint(0, n, (B,), generator=g, device=DEV)
+    x = torch.zeros(B, n, dtype=torch.bfloat16, device=DEV)
+    x[torch.arange(B, device=DEV), at] = 128.0
+    bm = O.block_decompose(m)
+    from glq_amd import hadamard as H
+    y = ext.glq_fused_linear_trellis_3inst_cuda(x, sv, su, packed, torch.tensor([n]), torch.tensor(bm), H.pack_block_meta([n]).to(DEV),
+                                                H.pack_block_meta(bm).to(DEV), 0.01, n, m, n, m, out_dtype=torch.float32)
+
+    def fht(a):
+        h, k = 1, a.shape[-1]
+        while h < k:
+            a = a.reshape(-1, k // (2 * h), 2, h)
+            a = torch.stack((a[:, :, 0] + a[:, :, 1], a[:, :, 0] - a[:, :, 1]), 2)
+            h *= 2
+        return a.reshape(-1, k) / k ** 0.5
+
+    W = ext.glq_decompress_trellis_3inst_cuda(packed, m, n).double()
+    z = fht(x.double() * sv.double()) @ W.T * 0.01
+    ref = torch.cat([fht(b) for b in z.split(bm, 1)], 1) * su.double()
+    assert rel(y.double(), ref) < 2e-5, rel(y.double(), ref)

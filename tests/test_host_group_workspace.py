@@ -37,3 +37,15 @@ def test_workspace_of_5_to_16_tokens_holds_the_groups_slots(n, B):
                 if got < need:
                     short.append((k, shards, got, need))
     assert not short, (len(short), short[:4])
+
+
+@pytest.mark.parametrize("entry,m,k,B,slots", [
+    ("trellis_gemv", 2048, 11008, 600, 8), ("trellis_gemv", 2048, 11008, 1139, 5), ("trellis_gemv", 2048, 2048, 1600, 4),
+    ("trellis_gemv", 2048, 2048, 2000, 2), ("trellis_gemv", 2048, 2048, 3100, 2), ("trellis_gemv", 2048, 2048, 4000, 1),
+    ("trellis_gemv", 800, 16384, 600, 18), ("trellis_gemv", 512, 14336, 1024, 16), ("e8_matmul", 3264, 1792, 1347, 1),
+    ("e8_matmul", 2048, 4096, 2000, 2), ("e8_matmul", 2048, 11008, 1139, 3)])
+def test_slots_of_many_tokens(entry, m, k, B, slots):
+    """K slots on either side of the line between those of 512- and of 256-token tiles: the order of a prompt's sums, and
+    whether they are rounded to fp16 (up to 16 slots), hang on their number.  (256 CUs)"""
+    got = getattr(_lib.load(), f"glqh_{entry}_workspace_bytes")(m, k, B)
+    assert got == _align(4 * slots * B * m) + (B + 511) // 512 * 512 * k * 2
