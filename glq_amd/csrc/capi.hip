@@ -2212,9 +2212,16 @@ extern "C" int glqh_e8_shell_quantize(const float *x, int64_t N, const float *ta
 }
 
 int glqh_viterbi_init(void);
-size_t glqh_viterbi_scratch_bytes(int K, int64_t n_tiles, int least);
-int glqh_launch_viterbi(const float *tiles, int64_t n_tiles, int64_t ld, int K, void *scratch, int least, int32_t *states,
+size_t glqh_viterbi_scratch_bytes(int K, int64_t n_tiles, int less);
+int glqh_launch_viterbi(const float *tiles, int64_t n_tiles, int64_t ld, int K, void *scratch, int less, int32_t *states,
                         float *hat, hipStream_t stream);
+
+// how much less than the search is fastest with `bytes` are: 0, 1, or 2, the least that it can do with
+static int viterbi_less(int K, int64_t n_tiles, size_t bytes) {
+    int less = 0;
+    while (less < 2 && bytes < glqh_viterbi_scratch_bytes(K, n_tiles, less)) ++less;
+    return less;
+}
 
 extern "C" size_t glqh_trellis_quantize_workspace_bytes(int K, int64_t n_tiles) {
     if (K < 1 || K > 4 || n_tiles < 1) return 0;
@@ -2225,7 +2232,7 @@ extern "C" size_t glqh_trellis_quantize_workspace_bytes(int K, int64_t n_tiles) 
 extern "C" size_t glqh_trellis_quantize_least_workspace_bytes(int K, int64_t n_tiles) {
     if (K < 1 || K > 4 || n_tiles < 1) return 0;
     glqh_init();
-    return glqh_viterbi_scratch_bytes(K, n_tiles, 1);
+    return glqh_viterbi_scratch_bytes(K, n_tiles, 2);
 }
 
 extern "C" int glqh_trellis_quantize_tiles(const float *tiles, int64_t n_tiles, int K, int32_t *states_out,
@@ -2234,10 +2241,10 @@ extern "C" int glqh_trellis_quantize_tiles(const float *tiles, int64_t n_tiles, 
     GLQH_REQUIRE(tiles && states_out && hat_out, "trellis quantize: null pointer");
     GLQH_REQUIRE(K >= 1 && K <= 4, "trellis encoder supports K (bits/weight) 1-4, got %d", K);
     GLQH_REQUIRE(n_tiles >= 1, "trellis quantize: n_tiles=%lld", (long long)n_tiles);
-    const int least = ws_bytes < glqh_viterbi_scratch_bytes(K, n_tiles, 0);
-    const size_t need = glqh_viterbi_scratch_bytes(K, n_tiles, least);
+    const int less = viterbi_less(K, n_tiles, ws_bytes);
+    const size_t need = glqh_viterbi_scratch_bytes(K, n_tiles, less);
     GLQH_REQUIRE(ws && ws_bytes >= need, "trellis quantize: workspace of %zu bytes needed, got %zu", need, ws_bytes);
-    return glqh_launch_viterbi(tiles, n_tiles, 0, K, ws, least, states_out, hat_out, (hipStream_t)stream);
+    return glqh_launch_viterbi(tiles, n_tiles, 0, K, ws, less, states_out, hat_out, (hipStream_t)stream);
 }
 
 extern "C" size_t glqh_trellis_quantize_matrix_workspace_bytes(int K, int64_t m, int64_t n) {
@@ -2257,12 +2264,13 @@ extern "C" int glqh_trellis_quantize_matrix(const float *w, int64_t m, int64_t n
     GLQH_REQUIRE(glqh_trellis_kernel_supported(m, n), "trellis pack: m %% 32 and n %% 64 must be 0 (m=%lld, n=%lld)",
                  (long long)m, (long long)n);
     const int64_t tiles = (m / 16) * (n / 16);
-    const int least = ws_bytes < glqh_trellis_quantize_matrix_workspace_bytes(K, m, n);
-    const size_t scratch = glqh_viterbi_scratch_bytes(K, tiles, least);                  // a multiple of 256
-    const size_t need = scratch + (size_t)tiles * 256 * sizeof(int32_t);
+    const size_t states_bytes = (size_t)tiles * 256 * sizeof(int32_t);
+    const int less = viterbi_less(K, tiles, ws_bytes > states_bytes ? ws_bytes - states_bytes : 0);
+    const size_t scratch = glqh_viterbi_scratch_bytes(K, tiles, less);                   // a multiple of 256
+    const size_t need = scratch + states_bytes;
     GLQH_REQUIRE(ws && ws_bytes >= need, "trellis quantize: workspace of %zu bytes needed, got %zu", need, ws_bytes);
     int32_t *states = (int32_t *)((char *)ws + scratch);
-    int rc = glqh_launch_viterbi(w, tiles, n, K, ws, least, states, recon_out, (hipStream_t)stream);
+    int rc = glqh_launch_viterbi(w, tiles, n, K, ws, less, states, recon_out, (hipStream_t)stream);
     return rc ? rc : glqh_launch_pack_states(states, m, n, K, packed_out, (hipStream_t)stream);
 }
 

@@ -31,7 +31,7 @@
 
 #pragma clang fp contract(off)
 
-size_t glqh_viterbi_scratch_bytes(int K, int64_t n_tiles, int least);
+size_t glqh_viterbi_scratch_bytes(int K, int64_t n_tiles, int less);
 
 namespace {
 
@@ -1564,9 +1564,9 @@ int acs_launch(const float *cost, const void *x, const float *lut, float *cost_o
 }
 
 // Two batches of tiles take turns: while one walks back, the other runs forward.  A batch is a chip full of pairs (two
-// workgroups a CU); everything is one batch where that leaves none to overlap with.  least: batches of half as many, in the
-// scratch that viterbi_kernel alone takes (16384 tiles 1 GB and 35.5 ms instead of 4 and 24.0 at K = 4, 2 GB and 37.2 instead
-// of 4 and 38.0 at 3, 38.9 instead of 35.7 at 2).
+// workgroups a CU); everything is one batch where that leaves none to overlap with.  less, what a caller short of memory has:
+// 1, no vm_kernel; 2, batches of half as many besides, in the scratch that viterbi_kernel alone takes.  16384 tiles at K = 4
+// 4 GB 24.8 ms, 2 GB 31.0, 1 GB 36.0 (4096: 6.5, 7.7, 9.1); at K = 3, where the first two are one, 4 GB 38.8, 2 GB 39.2, at 2 35.8, 38.9.
 //
 // At K = 4 chips full of sixteen tiles a CU come first, through vm_kernel, one after the other, and the rest too where that is
 // VM_FEWEST tiles a CU or more: a part of a chip takes its whole time (3072 tiles 6.2 and 6.0 ms, 4096 8.2 and 6.5).
@@ -1576,18 +1576,18 @@ struct vb_plan {
 };
 constexpr int VM_FEWEST = 12;
 template <int K>
-int64_t vm_tiles(int64_t n_tiles, int least) {
+int64_t vm_tiles(int64_t n_tiles, int less) {
     const int64_t full = VM_TILES * (int64_t)glqh_device_cus(), rest = n_tiles % full;
-    return K != 4 || least ? 0 : rest < VM_FEWEST * (int64_t)glqh_device_cus() ? n_tiles - rest : n_tiles;
+    return K != 4 || less ? 0 : rest < VM_FEWEST * (int64_t)glqh_device_cus() ? n_tiles - rest : n_tiles;
 }
-vb_plan vb_plan_of(int64_t n_tiles, int least) {
-    const int64_t full = (least ? 2 : 4) * (int64_t)glqh_device_cus();
+vb_plan vb_plan_of(int64_t n_tiles, int less) {
+    const int64_t full = (less > 1 ? 2 : 4) * (int64_t)glqh_device_cus();
     return n_tiles <= full ? vb_plan{n_tiles, 1} : vb_plan{full, 2};
 }
 template <int K>
-size_t vb_bytes(int64_t n_tiles, int least) {
-    const int64_t products = vm_tiles<K>(n_tiles, least), chip = std::min(products, VM_TILES * (int64_t)glqh_device_cus());
-    const vb_plan p = vb_plan_of(n_tiles - products, least);
+size_t vb_bytes(int64_t n_tiles, int less) {
+    const int64_t products = vm_tiles<K>(n_tiles, less), chip = std::min(products, VM_TILES * (int64_t)glqh_device_cus());
+    const vb_plan p = vb_plan_of(n_tiles - products, less);
     return (size_t)std::max(chip, p.batch * p.batches) * (vb_cfg<K>::STORED * vb_cfg<K>::G * 2 + sizeof(vb_tile));
 }
 
@@ -1600,7 +1600,7 @@ vb_lists vb_lists_at(char *end, int64_t n_tiles) {
 }
 
 template <int K>
-int vb_launch(const float *tiles, int64_t n_tiles, int64_t ld, void *scratch, int least, const vb_lists &lists, int32_t *states,
+int vb_launch(const float *tiles, int64_t n_tiles, int64_t ld, void *scratch, int less, const vb_lists &lists, int32_t *states,
               float *hat, hipStream_t stream) {
     using C = vb_cfg<K>;
     hipLaunchKernelGGL(vb_try_kernel, dim3((unsigned)((n_tiles + 3) / 4)), dim3(256), 0, stream, tiles, n_tiles, ld, C::WIDE, lists);
@@ -1608,8 +1608,8 @@ int vb_launch(const float *tiles, int64_t n_tiles, int64_t ld, void *scratch, in
                        8 * glqh_device_cus(), lists);
     GLQH_LAUNCH_CHECK("viterbi lists launch");
     const int cus = glqh_device_cus();
-    const int64_t products = vm_tiles<K>(n_tiles, least);
-    const vb_plan plan = vb_plan_of(n_tiles - products, least);
+    const int64_t products = vm_tiles<K>(n_tiles, less);
+    const vb_plan plan = vb_plan_of(n_tiles - products, less);
     const size_t rows = (size_t)plan.batch * C::STORED * C::G;
     auto part = [&](int64_t batch, int pass) {
         const int64_t first = products + batch * plan.batch, left = n_tiles - first;
@@ -1672,13 +1672,13 @@ int vb_launch(const float *tiles, int64_t n_tiles, int64_t ld, void *scratch, in
 bool vb_takes(int K, int64_t n_tiles) { return K == 4 || (K >= 2 && n_tiles > glqh_device_cus()); }
 
 template <int K>
-int vt_launch(const float *tiles, int64_t n_tiles, int64_t ld, void *scratch, int least, int grid, int32_t *states, float *hat,
+int vt_launch(const float *tiles, int64_t n_tiles, int64_t ld, void *scratch, int less, int grid, int32_t *states, float *hat,
               hipStream_t stream) {
     vb_lists lists = {};
     if constexpr (K >= 2) {
         if (vb_takes(K, n_tiles)) {
-            lists = vb_lists_at((char *)scratch + glqh_viterbi_scratch_bytes(K, n_tiles, least), n_tiles);
-            if (int rc = vb_launch<K>(tiles, n_tiles, ld, scratch, least, lists, states, hat, stream)) return rc;
+            lists = vb_lists_at((char *)scratch + glqh_viterbi_scratch_bytes(K, n_tiles, less), n_tiles);
+            if (int rc = vb_launch<K>(tiles, n_tiles, ld, scratch, less, lists, states, hat, stream)) return rc;
         }
     }
     constexpr size_t lds = vt_cfg<K>::ROWS * sizeof(float) * (size_t)vt_cfg<K>::G;
@@ -1715,25 +1715,25 @@ int glqh_viterbi_grid(int K, int64_t n_tiles) {
     return (int)(n_tiles < g ? n_tiles : g);
 }
 
-// least: what the search can do with, not what it is fastest with
-size_t glqh_viterbi_scratch_bytes(int K, int64_t n_tiles, int least) {
+// less: 0, what the search is fastest with; 1 and 2, what it can do with too
+size_t glqh_viterbi_scratch_bytes(int K, int64_t n_tiles, int less) {
     const size_t row = sizeof(float) << (16 - K);
     const int depth = K == 1 ? vt_cfg<1>::DEPTH : K == 2 ? vt_cfg<2>::DEPTH : K == 3 ? vt_cfg<3>::DEPTH : vt_cfg<4>::DEPTH;
     const size_t exact = (size_t)glqh_viterbi_grid(K, n_tiles) * (VT_T / depth) * row;
     if (!vb_takes(K, n_tiles)) return exact;
-    const size_t bound = K == 2 ? vb_bytes<2>(n_tiles, least) : K == 3 ? vb_bytes<3>(n_tiles, least) : vb_bytes<4>(n_tiles, least);
+    const size_t bound = K == 2 ? vb_bytes<2>(n_tiles, less) : K == 3 ? vb_bytes<3>(n_tiles, less) : vb_bytes<4>(n_tiles, less);
     return (((exact > bound ? exact : bound) + 255) & ~(size_t)255) + vb_list_bytes(n_tiles);
 }
 
 // ld: 0 for tiles in step order, else the row length of the (m, n) matrices `tiles` and `hat`
-int glqh_launch_viterbi(const float *tiles, int64_t n_tiles, int64_t ld, int K, void *scratch, int least, int32_t *states,
+int glqh_launch_viterbi(const float *tiles, int64_t n_tiles, int64_t ld, int K, void *scratch, int less, int32_t *states,
                         float *hat, hipStream_t stream) {
     const int grid = glqh_viterbi_grid(K, n_tiles);
     switch (K) {
-    case 1: return vt_launch<1>(tiles, n_tiles, ld, scratch, least, grid, states, hat, stream);
-    case 2: return vt_launch<2>(tiles, n_tiles, ld, scratch, least, grid, states, hat, stream);
-    case 3: return vt_launch<3>(tiles, n_tiles, ld, scratch, least, grid, states, hat, stream);
-    case 4: return vt_launch<4>(tiles, n_tiles, ld, scratch, least, grid, states, hat, stream);
+    case 1: return vt_launch<1>(tiles, n_tiles, ld, scratch, less, grid, states, hat, stream);
+    case 2: return vt_launch<2>(tiles, n_tiles, ld, scratch, less, grid, states, hat, stream);
+    case 3: return vt_launch<3>(tiles, n_tiles, ld, scratch, less, grid, states, hat, stream);
+    case 4: return vt_launch<4>(tiles, n_tiles, ld, scratch, less, grid, states, hat, stream);
     }
     return glqh_fail("trellis encoder supports K (bits/weight) 1-4, got %d", K);
 }

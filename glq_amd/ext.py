@@ -1198,8 +1198,14 @@ def e8_quantize(x, codebook, codebook_norms=None, return_decoded=True):
 def _quantize_ws(nbytes, least, device):
     try:
         return _ws(nbytes, device)
-    except torch.OutOfMemoryError:                            # the search in smaller batches
-        return _ws(least, device)
+    except torch.OutOfMemoryError:
+        pass
+    if 2 * least < nbytes:                                    # the search without its largest batches
+        try:
+            return _ws(2 * least, device)
+        except torch.OutOfMemoryError:
+            pass
+    return _ws(least, device)                                 # in smaller ones
 
 
 def trellis_quantize_tiles(tiles, K):

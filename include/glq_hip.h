@@ -475,8 +475,9 @@ int glqh_e8_shell_quantize(const float *x, int64_t N, const float *table_f32, co
 
 size_t glqh_trellis_quantize_workspace_bytes(int K, int64_t n_tiles);
 
-/* Less than that does too, at a tenth more time, at 4 bits and sixteen tiles per CU or more a third (half as much for more
- * than four tiles per CU, a quarter there); the matrix entry below takes this and the states, 1024 bytes per tile. */
+/* Less than that does too: the least, half of it for more than four tiles per CU, at up to a tenth more time.  At 4 bits and twelve
+ * tiles per CU or more the least is a third to a quarter of it, at about half as much time again; twice the least then takes
+ * a quarter more.  The matrix entry below takes this and the states, 1024 bytes per tile. */
 size_t glqh_trellis_quantize_least_workspace_bytes(int K, int64_t n_tiles);
 
 /* Tail-biting Viterbi search of the 3INST trellis for n_tiles sequences of 256 fp32 values

@@ -466,6 +466,47 @@ def test_viterbi_in_the_least_workspace(K, n, monkeypatch):
                                                    torch.cuda.current_stream().cuda_stream))
 
 
+def _quantize_in(X, K, nbytes):
+    """States from a workspace of that many bytes, and the last of them that were written."""
+    from glq_amd import _lib
+    n = X.shape[0]
+    x, states, hat = X.to(DEV), torch.empty(n, 256, dtype=torch.int32, device=DEV), torch.empty(n, 256, device=DEV)
+    ws = torch.full((nbytes,), 0xA5, dtype=torch.uint8, device=DEV)
+    _lib.check(_lib.load().glqh_trellis_quantize_tiles(x.data_ptr(), n, K, states.data_ptr(), hat.data_ptr(), ws.data_ptr(), nbytes,
+                                                       torch.cuda.current_stream().cuda_stream))
+    changed = (ws.view(-1, 256) != 0xA5).any(1).nonzero()
+    return states, 256 * (int(changed[-1]) + 1)
+
+
+@pytest.mark.parametrize("n", [3072, 4500])
+def test_viterbi_between_the_least_workspace_and_the_most(n, monkeypatch):
+    """At K = 4 from twelve tiles per CU on: twice the least workspace is used as such (batches of four tiles per CU), the most
+    as such, and the least; the exact states from each of them.  The Python entry tries them in turn."""
+    from glq_amd import _lib, ext
+    say("viterbi between least and most", n)
+    lib = _lib.load()
+    most, least = lib.glqh_trellis_quantize_workspace_bytes(4, n), lib.glqh_trellis_quantize_least_workspace_bytes(4, n)
+    assert 2 * least < most
+    X = _search_tiles(n, n)
+    ref = _exact_states(X, 4)
+    for nbytes, lo, hi in ((most, most, most), (most - 256, 1.9 * least, 2 * least), (2 * least, 1.9 * least, 2 * least),
+                           (least, least, least)):
+        states, used = _quantize_in(X, 4, nbytes)
+        assert lo <= used <= hi, (nbytes, used)
+        assert torch.equal(states, ref), (nbytes, (states != ref).any(1).nonzero()[:5])
+    taken, plain = [], ext._ws
+
+    def short(nbytes, device):
+        taken.append(nbytes)
+        if nbytes > 2 * least:
+            raise torch.OutOfMemoryError("short of memory")
+        return plain(nbytes, device)
+
+    monkeypatch.setattr(ext, "_ws", short)
+    assert torch.equal(ext.trellis_quantize_tiles(X.to(DEV), 4)[1], ref)
+    assert taken == [most, 2 * least]
+
+
 def test_viterbi_under_capture():
     """Captured and replayed on other tiles: the launches' batches hand each other their rows through the same memory."""
     from glq_amd import ext
