@@ -411,6 +411,15 @@ def test_viterbi_tiles_on_either_search(K, kind):
     assert torch.equal(states, ref), (states != ref).any(1).nonzero()[:5]
 
 
+def test_ramps_at_2_bits_are_left_at_their_first_overflow():
+    """Slow ramps fill the lists of the walk back: at K = 2 all go to the exact search without a second walk, and come out exact."""
+    say("ramps at 2 bits")
+    X = torch.linspace(-3, 3, 256) + torch.randn(1024, 256, generator=torch.Generator().manual_seed(2)) * 1e-3
+    states, tried, left = _quantize_counts(X, 2)
+    assert (tried, left) == (1024, 1024)
+    assert torch.equal(states, _exact_states(X, 2))
+
+
 @pytest.mark.parametrize("K,m,n", [(2, 256, 320), (3, 288, 256), (4, 512, 576)])
 def test_quantize_matrix_on_bounds_equals_the_tile_route(K, m, n):
     """More tiles than CUs, whose places in the matrix the lists tell, all but two of them on bounds: the tile route, bit for bit."""
