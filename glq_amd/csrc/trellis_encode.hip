@@ -284,7 +284,8 @@ __device__ __forceinline__ int64_t vt_pos(int64_t tile, int t, int64_t ld) {
 // Which tiles of a call are searched how: those for the search on bounds, from order[0] on, those that it does not try, from
 // order[n_tiles - 1] back, and those that it tried and left.
 struct vb_lists {
-    int *counts;                           // how many it tries, how many it left, and before this batch; null: no such search
+    int *counts;                           // how many it tries, how many it left, and before this batch, and how many of the first go
+                                           // through vm_kernel; null: no such search
     int *order, *left;
 };
 
@@ -477,7 +478,7 @@ struct vb_tile {
     int over;                              // the tail-biting overlap, -1: left to viterbi_kernel
 };
 
-// Tiles order[first .. first + count - 1], as far as that many are tried, and one of their two passes: 0 on the inputs rolled by T/2, unconstrained; 1 from and
+// Tiles order[vb_first .. vb_first + count - 1], as far as that many are tried, and one of their two passes: 0 on the inputs rolled by T/2, unconstrained; 1 from and
 // to the overlap that the first backtrack found.  rows: of every tile a row of G halves, STORED times.
 struct vb_part {
     int64_t first;
@@ -486,9 +487,19 @@ struct vb_part {
     vb_tile *info;
     bool product;                          // bounds of vm_kernel
 };
+__device__ __forceinline__ int64_t vb_first(const vb_part &part, const vb_lists &lists) {
+    return part.first + (part.product ? 0 : __builtin_amdgcn_readfirstlane(lists.counts[3]));   // behind vm_kernel's
+}
 __device__ __forceinline__ int vb_count(const vb_part &part, const vb_lists &lists) {
-    const int64_t left = __builtin_amdgcn_readfirstlane(lists.counts[0]) - part.first;
+    const int tried = __builtin_amdgcn_readfirstlane(lists.counts[0]), products = __builtin_amdgcn_readfirstlane(lists.counts[3]);
+    const int64_t left = (part.product && products < tried ? products : tried) - vb_first(part, lists);
     return left < part.count ? (left < 0 ? 0 : (int)left) : part.count;
+}
+
+// How many of `tiles` go through vm_kernel: whole chips of them, and the rest where it is `fewest` or more
+__host__ __device__ __forceinline__ int64_t vm_share(int64_t tiles, int64_t chip, int64_t fewest) {
+    const int64_t rest = tiles % chip;
+    return rest < fewest ? tiles - rest : tiles;
 }
 
 // The lists, in two launches (10 us together, where the smallest call takes 730): a wave a tile notes in `left` whether it is tried, and one workgroup deals the tiles out.
@@ -517,7 +528,7 @@ vb_try_kernel(const float *__restrict__ tiles_in, int64_t n_tiles, int64_t ld, f
 }
 
 __global__ void __launch_bounds__(1024)
-vb_order_kernel(int n_tiles, int few, vb_lists lists) {
+vb_order_kernel(int n_tiles, int few, int chip, int fewest, vb_lists lists) {
     __shared__ int of_wave[16];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     int tried = 0;
@@ -538,22 +549,28 @@ vb_order_kernel(int n_tiles, int few, vb_lists lists) {
         __syncthreads();
     }
     if (tid == 0) {
-        lists.counts[0] = tried <= few && tried < n_tiles - tried ? 0 : tried;
+        tried = tried <= few && tried < n_tiles - tried ? 0 : tried;
+        lists.counts[0] = tried;
         lists.counts[1] = 0;
+        lists.counts[3] = chip ? vm_share(tried, chip, fewest) : 0;
     }
 }
 
-// Before the batch that begins at `first`: where more than half of those before it were left, it and the rest are not tried.
-__global__ void vb_stop_kernel(int64_t first, vb_lists lists) {
+// Before a batch: where more than half of those before it were left, it and the rest are not tried.
+__global__ void vb_stop_kernel(vb_part part, vb_lists lists) {
     if (threadIdx.x != 0) return;
+    const int64_t first = vb_first(part, lists);
     if (2 * (int64_t)lists.counts[1] > first && lists.counts[0] > first) lists.counts[0] = (int)first;
     lists.counts[2] = lists.counts[1];
 }
 
-// Between the passes of a large batch: where more than half were left in the first one, none of it is tried
-__global__ void vm_stop_kernel(int64_t first, int count, vb_lists lists) {
-    if (threadIdx.x != 0 || 2 * (lists.counts[1] - lists.counts[2]) <= count) return;
-    lists.counts[0] = (int)first;
+// Between the passes of a large batch: where the first one left fewer than `worth` of those tried, none of it is tried.  (The exact
+// search takes as long over three tiles a CU as the second pass over any number.  Given up at half of a chip, 8192 tiles that are half
+// slow ramps took 36.1 ms, not 33, and 4096 that are 70 % ramps 20.7, not 19.)
+__global__ void vm_stop_kernel(vb_part part, int worth, vb_lists lists) {
+    const int count = vb_count(part, lists);
+    if (threadIdx.x != 0 || count == 0 || count - (lists.counts[1] - lists.counts[2]) >= worth) return;
+    lists.counts[0] = (int)part.first;
     lists.counts[1] = lists.counts[2];
 }
 
@@ -568,8 +585,9 @@ __device__ __forceinline__ void vb_forward(const float *__restrict__ tiles_in, i
                                            const vb_part &part, int worker, int workers, uint32_t *lds) {
     using C = vb_cfg<K>;
     constexpr int THREADS = VB_THREADS;
-    const int64_t first = part.first;
+    const int64_t first = vb_first(part, lists);
     const int count = vb_count(part, lists), pass = part.pass;
+    if (count <= 0) return;
     uint16_t *const __restrict__ rows = part.rows;
     vb_tile *const __restrict__ info = part.info;
     constexpr int G = C::G, NK = C::NK, CW = C::CW, D = C::DEPTH, ROWS = C::ROWS;
@@ -1351,7 +1369,7 @@ struct vb_work {
 };
 static_assert(sizeof(vb_work) <= 160 * 1024 / 16, "sixteen on a CU");
 
-// The backtrack of tile part.first + at (one wave): after pass 0 the overlap, after pass 1 the states and values.
+// The backtrack of tile vb_first + at (one wave): after pass 0 the overlap, after pass 1 the states and values.
 // What bounds it is latency: a chain of STORED levels, each a look into a row of which only the last level's group tells
 // where (a microsecond), some 150 instructions and trips to LDS.  150 us on average, 340 for the slowest of 256 tiles.
 // Sixteen waves a CU over 4096 tiles of vm_kernel: 0.19 ms on average, 0.46 for the slowest tile, which is what the launch takes (four ways
@@ -1367,7 +1385,7 @@ __device__ __forceinline__ void vb_backtrack(const float *__restrict__ tiles_in,
     uint16_t *const states = W->states;
     int *const start = W->start;
     const int lane = threadIdx.x & 63, pass = part.pass;
-    const int64_t tile = __builtin_amdgcn_readfirstlane(lists.order[part.first + at]);
+    const int64_t tile = __builtin_amdgcn_readfirstlane(lists.order[vb_first(part, lists) + at]);
     vb_tile *const mine = part.info + at;
     const int over = pass ? __builtin_amdgcn_readfirstlane(mine->over) : 0;
     if ((uint32_t)over >= (uint32_t)C::G) return;              // left after the first pass
@@ -1572,7 +1590,10 @@ int acs_launch(const float *cost, const void *x, const float *lut, float *cost_o
 // 4 GB 24.8 ms, 2 GB 31.0, 1 GB 36.0 (4096: 6.5, 7.7, 9.1); at K = 3, where the first two are one, 4 GB 38.8, 2 GB 39.2, at 2 35.8, 38.9.
 //
 // At K = 4 chips full of sixteen tiles a CU come first, through vm_kernel, one after the other, and the rest too where that is
-// VM_FEWEST tiles a CU or more: a part of a chip takes its whole time (3072 tiles 6.2 and 6.0 ms, 4096 8.2 and 6.5).
+// VM_FEWEST tiles a CU or more: a part of a chip takes its whole time (3072 tiles 6.2 and 6.0 ms, 4096 8.2 and 6.5).  What counts is
+// how many tiles are tried, which the device knows (vm_share): the launches of both ways are there, and those of one do nothing.
+// (4096 tiles, all tried, 6.30 -> 6.33 ms for them.  By the tiles of the call alone 3072 of which 55 % were tried took 12.6 ms, not
+// 10.1, 8192 28.1, not 23.9.)
 struct vb_plan {
     int64_t batch;
     int batches;                           // in flight: 1 or 2
@@ -1580,8 +1601,14 @@ struct vb_plan {
 constexpr int VM_FEWEST = 12;
 template <int K>
 int64_t vm_tiles(int64_t n_tiles, int less) {
-    const int64_t full = VM_TILES * (int64_t)glqh_device_cus(), rest = n_tiles % full;
-    return K != 4 || less ? 0 : rest < VM_FEWEST * (int64_t)glqh_device_cus() ? n_tiles - rest : n_tiles;
+    const int64_t cus = glqh_device_cus();
+    return K != 4 || less ? 0 : vm_share(n_tiles, VM_TILES * cus, VM_FEWEST * cus);
+}
+// tiles, at most, behind them
+template <int K>
+int64_t vb_rest(int64_t n_tiles, int less) {
+    const int64_t most = VM_FEWEST * (int64_t)glqh_device_cus() - 1;
+    return vm_tiles<K>(n_tiles, less) == 0 ? n_tiles : std::min(n_tiles, most);
 }
 vb_plan vb_plan_of(int64_t n_tiles, int less) {
     const int64_t full = (less > 1 ? 2 : 4) * (int64_t)glqh_device_cus();
@@ -1590,7 +1617,7 @@ vb_plan vb_plan_of(int64_t n_tiles, int less) {
 template <int K>
 size_t vb_bytes(int64_t n_tiles, int less) {
     const int64_t products = vm_tiles<K>(n_tiles, less), chip = std::min(products, VM_TILES * (int64_t)glqh_device_cus());
-    const vb_plan p = vb_plan_of(n_tiles - products, less);
+    const vb_plan p = vb_plan_of(vb_rest<K>(n_tiles, less), less);
     return (size_t)std::max(chip, p.batch * p.batches) * (vb_cfg<K>::STORED * vb_cfg<K>::G * 2 + sizeof(vb_tile));
 }
 
@@ -1607,15 +1634,15 @@ int vb_launch(const float *tiles, int64_t n_tiles, int64_t ld, void *scratch, in
               float *hat, hipStream_t stream) {
     using C = vb_cfg<K>;
     hipLaunchKernelGGL(vb_try_kernel, dim3((unsigned)((n_tiles + 3) / 4)), dim3(256), 0, stream, tiles, n_tiles, ld, C::WIDE, lists);
-    hipLaunchKernelGGL(vb_order_kernel, dim3(1), dim3(1024), 0, stream, (int)n_tiles,
-                       8 * glqh_device_cus(), lists);
-    GLQH_LAUNCH_CHECK("viterbi lists launch");
     const int cus = glqh_device_cus();
-    const int64_t products = vm_tiles<K>(n_tiles, less);
-    const vb_plan plan = vb_plan_of(n_tiles - products, less);
+    const int64_t products = vm_tiles<K>(n_tiles, less), rest = vb_rest<K>(n_tiles, less);
+    hipLaunchKernelGGL(vb_order_kernel, dim3(1), dim3(1024), 0, stream, (int)n_tiles, 8 * cus, products ? VM_TILES * cus : 0,
+                       VM_FEWEST * cus, lists);
+    GLQH_LAUNCH_CHECK("viterbi lists launch");
+    const vb_plan plan = vb_plan_of(rest, less);
     const size_t rows = (size_t)plan.batch * C::STORED * C::G;
     auto part = [&](int64_t batch, int pass) {
-        const int64_t first = products + batch * plan.batch, left = n_tiles - first;
+        const int64_t first = batch * plan.batch, left = rest - first;
         const int slab = (int)(batch & 1);
         return vb_part{first, (int)(left <= 0 ? 0 : left < plan.batch ? left : plan.batch), pass, (uint16_t *)scratch + slab * rows,
                        (vb_tile *)((uint16_t *)scratch + plan.batches * rows) + slab * plan.batch, false};
@@ -1625,7 +1652,9 @@ int vb_launch(const float *tiles, int64_t n_tiles, int64_t ld, void *scratch, in
         const int walkers = (back.count + VB_WALK - 1) / VB_WALK;
         // one tile a workgroup while that gives no CU more than two workgroups (512 tiles: 1.58 ms at K = 4, 1.52 at 3); at
         // K = 2, with one cost row and a barrier to both its sides, a second tile is what fills the wait (2.9 -> 1.66)
-        const bool few = forward.count <= 2 * cus;
+        // (by the tiles that are there when all are tried)
+        const int64_t all = n_tiles - products - forward.first;
+        const bool few = (all > 0 ? std::min<int64_t>(all, forward.count) : forward.count) <= 2 * cus;
         const int per = few ? C::FEW : 2, work = (forward.count + per - 1) / per;
         const dim3 grid(walkers + (work < 2 * cus ? work : 2 * cus));
         if (grid.x == 0) return 0;
@@ -1641,21 +1670,21 @@ int vb_launch(const float *tiles, int64_t n_tiles, int64_t ld, void *scratch, in
     if constexpr (K == 4) {
         const int64_t chip = std::min(products, VM_TILES * (int64_t)cus);
         for (int64_t first = 0; first < products; first += chip) {
-            hipLaunchKernelGGL(vb_stop_kernel, dim3(1), dim3(64), 0, stream, first, lists);
             const int count = (int)std::min(products - first, chip);
             for (int pass = 0; pass < 2; ++pass) {
                 const vb_part all{first, count, pass, (uint16_t *)scratch, (vb_tile *)((uint16_t *)scratch + chip * C::STORED * C::G), true};
+                if (pass == 0) hipLaunchKernelGGL(vb_stop_kernel, dim3(1), dim3(64), 0, stream, all, lists);
                 hipLaunchKernelGGL(vm_kernel, dim3((count + VM_TILES - 1) / VM_TILES), dim3(VM_THREADS), VM_LDS, stream, tiles, ld, lists, all);
                 hipLaunchKernelGGL(vm_walk_kernel, dim3(count), dim3(GLQH_WAVE), 0, stream, tiles, ld, lists, all, states, hat);
-                if (pass == 0) hipLaunchKernelGGL(vm_stop_kernel, dim3(1), dim3(64), 0, stream, first, count, lists);
+                if (pass == 0) hipLaunchKernelGGL(vm_stop_kernel, dim3(1), dim3(64), 0, stream, all, 3 * cus, lists);
                 GLQH_LAUNCH_CHECK("viterbi launch");
             }
         }
     }
     // batches 2i and 2i + 1: F0(a) | F0(b) B0(a) | F1(a) B0(b) | F1(b) B1(a) | F0(a') B1(b) | ...
     vb_part back = none;
-    for (int64_t b = 0; products + b * plan.batch < n_tiles; b += 2) {
-        if (products + b) hipLaunchKernelGGL(vb_stop_kernel, dim3(1), dim3(64), 0, stream, products + b * plan.batch, lists);
+    for (int64_t b = 0; b * plan.batch < rest; b += 2) {
+        if (products + b) hipLaunchKernelGGL(vb_stop_kernel, dim3(1), dim3(64), 0, stream, part(b, 0), lists);
         for (int turn = 0; turn < 4; ++turn) {
             const vb_part forward = part(b + (turn & 1), turn >> 1);
             if (forward.count == 0 || plan.batches == 1) {     // nothing beside it

@@ -475,6 +475,44 @@ def test_viterbi_in_the_least_workspace(K, n, monkeypatch):
                                                    torch.cuda.current_stream().cuda_stream))
 
 
+@pytest.mark.parametrize("kind,n", [("wide among normal", 3200), ("wide among normal", 8300), ("1500 normal, then ramps", 4300),
+                                    ("500 normal, then ramps", 4300), ("ramps", 4200), ("ramps, then wide", 6000)])
+def test_viterbi_by_products_over_chips_that_are_not_full(kind, n):
+    """At K = 4 a chip of tiles goes through the matrix products only where twelve tiles a CU of it are tried (not 1760 of 3200, whose
+    rows then fill 2 GB, nor what 4565 of 8300 leave behind the first chip); one of whose tiles the first pass leaves all
+    but three a CU is given up, others are not; the exact states of all tiles throughout."""
+    from glq_amd import _lib
+    say("viterbi by products, chips not full", kind, n)
+    g = torch.Generator().manual_seed(n)
+    X = torch.randn(n, 256, generator=g) * 0.9
+    ramps = torch.linspace(-3, 3, 256) + torch.randn(n, 256, generator=g) * 1e-3
+    wide = n * 9 // 20
+    if kind == "wide among normal":
+        X[torch.randperm(n, generator=g)[:wide]] *= 7
+    elif kind == "ramps, then wide":
+        X *= 7
+        X[:3200] = ramps[:3200]
+    else:
+        first = int(kind.split()[0]) if kind != "ramps" else 0
+        X[first:] = ramps[first:]
+    lib, x = _lib.load(), X.to(DEV)
+    states, hat = torch.empty(n, 256, dtype=torch.int32, device=DEV), torch.empty(n, 256, device=DEV)
+    ws = torch.full((lib.glqh_trellis_quantize_workspace_bytes(4, n),), 0xA5, dtype=torch.uint8, device=DEV)
+    _lib.check(lib.glqh_trellis_quantize_tiles(x.data_ptr(), n, 4, states.data_ptr(), hat.data_ptr(), ws.data_ptr(), ws.numel(),
+                                               torch.cuda.current_stream().cuda_stream))
+    tried, left = ws[-256:].view(torch.int32)[:2].tolist()
+    if kind == "wide among normal":
+        assert tried == n - wide and left <= n // 100, (tried, left)
+        untouched = int((ws[2200 << 20:3000 << 20] != 0xA5).sum()) == 0   # (a failing assertion would list a tensor compared in it)
+        assert untouched == (n == 3200)
+    elif kind == "1500 normal, then ramps":
+        assert tried == 4096 and 2560 <= left <= 2620, (tried, left)
+    else:
+        assert (tried, left) == (0, 0), (tried, left)
+    ref = _exact_states(X, 4)
+    assert torch.equal(states, ref), (states != ref).any(1).nonzero()[:5]
+
+
 def _quantize_in(X, K, nbytes):
     """States from a workspace of that many bytes, and the last of them that were written."""
     from glq_amd import _lib
