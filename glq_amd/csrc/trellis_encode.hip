@@ -360,7 +360,7 @@ viterbi_kernel(const float *__restrict__ tiles_in, int64_t n_tiles, int64_t ld, 
 // and viterbi_kernel's costs of both paths, from which it takes the cheaper; 4 e < VB_NEAR.)  Where another kept path is
 // within VB_NEAR of the cheapest (3 % of the tiles), fp32 costs are evaluated forward over the kept ways, minima and lowest
 // states as in viterbi_kernel.
-// Tiles with inputs above VB_X, not finite or all equal are not tried, and those with more kept ways than fit, at K = 3 and 4 also at half the
+// Tiles with inputs above VB_X, not finite or all equal are not tried, and those with more kept ways than fit, at K = 4 also at half the
 // slack, are left: lists of both go to viterbi_kernel (with marks instead of lists, every workgroup walking its share of all tiles, it took the
 // time of all of them where half were marked).  Far beyond the weights' range the cost is mostly what no path can avoid,
 // and SLACK of that lets everything through: tiles with more than WIDE of it are not tried either (K = 4: 5 % of those with
@@ -1416,9 +1416,9 @@ __device__ __forceinline__ void vb_backtrack(const float *__restrict__ tiles_in,
     }
     const float least = vb_lane(vb_half(lo) + bt, 0);
     float limit = vb_lane(least * (1.0f + C::SLACK) + lost, 0);
-    // at K = 2 a second walk saves few tiles that the exact search would not take in that time (1024 slow ramps 5.2 -> 7.1 ms with it;
-    // normal values of sigma 2.2, where it saves 180 of 4096, 11.0 -> 11.4)
-    float lower = K == 2 ? __builtin_inff() : limit - 0.5f * (limit - least);
+    // below K = 4 a second walk takes longer than the exact search over what it saves (K = 2, 1024 slow ramps 5.2 -> 7.1 ms with it, normal
+    // values of sigma 2.2, where it saves 180 of 4096, 11.0 -> 11.4; K = 3, sigma 2.0, where it saves 210, 12.7 -> 13.0)
+    float lower = K < 4 ? __builtin_inff() : limit - 0.5f * (limit - least);
     bool good = false;
 #pragma unroll 1
     for (int tries = 0; tries < 4; ++tries) {
@@ -1449,7 +1449,7 @@ __device__ __forceinline__ void vb_backtrack(const float *__restrict__ tiles_in,
         if (n > VB_MOST) limit = __builtin_inff();
         else good = vb_trace<K>(n, lane < n ? start[lane] : 0, limit, x, hist, step, part.product, pre, tie, pass ? VT_T - 1 : VT_T / 2, &W->pool, states);
         if (good) break;
-        if (limit == __builtin_inff()) {                       // too many ways for the lists: half the slack may do at K = 3 and 4
+        if (limit == __builtin_inff()) {                       // too many ways for the lists: half the slack may do at K = 4
             limit = lower;
             lower = __builtin_inff();
         }

@@ -420,6 +420,16 @@ def test_ramps_at_2_bits_are_left_at_their_first_overflow():
     assert torch.equal(states, _exact_states(X, 2))
 
 
+def test_wide_tiles_at_3_bits_are_left_at_their_first_overflow():
+    """Normal values of sigma 2: the lists of the walk back hold most tiles' ways, and at K = 3 the others (6-8 % of those tried; half the
+    slack would leave 1 %) go to the exact search without a second walk."""
+    say("wide tiles at 3 bits")
+    X = torch.randn(2000, 256, generator=torch.Generator().manual_seed(3)) * 2.0
+    states, tried, left = _quantize_counts(X, 3)
+    assert tried > 1200 and left > tried // 25, (tried, left)
+    assert torch.equal(states, _exact_states(X, 3))
+
+
 @pytest.mark.parametrize("K,m,n", [(2, 256, 320), (3, 288, 256), (4, 512, 576)])
 def test_quantize_matrix_on_bounds_equals_the_tile_route(K, m, n):
     """More tiles than CUs, whose places in the matrix the lists tell, all but two of them on bounds: the tile route, bit for bit."""
