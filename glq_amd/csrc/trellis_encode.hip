@@ -802,8 +802,8 @@ __device__ __forceinline__ void vb_forward(const float *__restrict__ tiles_in, i
 // A workgroup has sixteen tiles, a CU to itself: one row of bounds, 128 KB, is read by all and written by all in turn, and
 // eight waves have eight units each, with their table in 64 registers and the new bounds, until all have read, in 64 more.
 //
-// Rounding.  A sum is off by at most VM_OFF times its terms' magnitudes (2.6 * 2^-24 is the most that 3 * 10^7 sums of such
-// terms showed, and a rounding follows); with e the state's cost those are at most (2 |x| + sqrt e)^2 <= 5 x^2 + 5 e, and c, and
+// Rounding.  A sum is off by at most VM_OFF times its terms' magnitudes (measured, not derived: 2.6 * 2^-24 is the most that 3 * 10^7 sums
+// of such terms showed, and a rounding follows; the rows that come of it are held to costs in 64 bits, group by group); with e the state's cost those are at most (2 |x| + sqrt e)^2 <= 5 x^2 + 5 e, and c, and
 // what moves, which is no more than c.  So 5 VM_OFF x^2 comes off every step's bounds, with what w^2 may lack below fp16's
 // smallest numbers, and VM_LESS of c + e.  Bounds are rounded once a step, towards zero; a row's least one stays at VM_FLOOR,
 // above what comes off until the next move, so that none is negative.

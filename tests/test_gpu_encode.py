@@ -602,6 +602,58 @@ def test_viterbi_by_products_equals_the_exact_search(n):
     assert torch.equal(states, ref), (states != ref).any(1).nonzero()[:5]
 
 
+def test_bounds_of_the_products_are_bounds():
+    """What the matrix products leave in the workspace, against the costs in float64: no bound of any group at any stored step
+    is above the least cost from the start (beyond the roundings of what moves out of the rows, 2^-24 of it each time), and the
+    limit of the walk back is not below the best path's cost.  Normal tiles, tiny ones, decoded paths whose sums cancel to nothing,
+    and the largest values that are tried, alone and several."""
+    from glq_amd import _lib
+    say("bounds of the products")
+    n, K, G, levels = 3072, 4, 4096, 128
+    g = torch.Generator().manual_seed(11)
+    X = torch.randn(n, 256, generator=g) * 0.9
+    X[16:24] *= torch.linspace(1.1, 1.7, 8)[:, None]
+    X[24:28] *= 0.05
+    X[28:32, 100] = torch.tensor([5.98, -5.98, 5.5, -5.0])
+    X[32:36, ::64] = 4.98 * torch.tensor([1.0, -1.0, 1.0, -1.0])
+    lut = torch.from_numpy(O.lut_3inst().astype(np.float32))
+    X[36:44] = lut[torch.from_numpy(O.trellis_states(O.random_packed(32, 64, 4, seed=4), 32, 64).astype(np.int64))].reshape(-1, 256)
+    X[40:44] += 1e-3 * torch.randn(4, 256, generator=g)
+    lib, x = _lib.load(), X.to(DEV)
+    states, hat = torch.empty(n, 256, dtype=torch.int32, device=DEV), torch.empty(n, 256, device=DEV)
+    ws = torch.zeros(lib.glqh_trellis_quantize_workspace_bytes(K, n), dtype=torch.uint8, device=DEV)
+    _lib.check(lib.glqh_trellis_quantize_tiles(x.data_ptr(), n, K, states.data_ptr(), hat.data_ptr(), ws.data_ptr(), ws.numel(),
+                                               torch.cuda.current_stream().cuda_stream))
+    assert ws[-256:].view(torch.int32)[:2].tolist() == [n, 0]    # all are tried, in their order, and none left: the rows are as they were
+    T = 48
+    rows = ws[:levels * n * G * 2].view(torch.float16).view(levels, n, G)
+    info = ws[levels * n * G * 2:levels * n * G * 2 + n * 520].view(n, 130, 4)[:T].contiguous()
+    pre, over = info[:, :129].contiguous().view(torch.float32)[:, :, 0].double(), info[:, 129].contiguous().view(torch.int32)[:, 0].long()
+    group = torch.arange(G, device=DEV)                          # where a row holds a group's bound
+    k, a = group >> 8, group & 255
+    at = a * 16 + (((k >> 1) ^ (a >> 5 & 7)) << 1) + (k & 1)
+    a = at >> 4
+    at = ((a & 15) << 4 | a >> 4) << 4 | (at & 15)
+    assert torch.equal(at.sort().values, group)
+    w, v = lut.to(DEV).double(), x[:T].half().double()
+    cost = torch.full((T, 16, G), torch.inf, dtype=torch.float64, device=DEV)   # of states by their high digit and group
+    cost[torch.arange(T, device=DEV), :, over] = 0.0
+    for i in range(256):
+        least = cost.amin(1)
+        if i and i % 2 == 0:
+            bound, moved = rows[i // 2 - 1, :T][:, at].double(), pre[:, i // 2, None]
+            assert float((bound + moved - least - i // 2 * 2 ** -24 * moved).max()) <= 0.0, i
+        # state s follows the groups s >> 4
+        cost = (least.repeat_interleave(16, 1) + (v[:, i, None] - w) ** 2).view(T, 16, G)
+    best = cost.amin(1).gather(1, over[:, None])[:, 0]
+    bound, moved = rows[127, :T][:, at].double().gather(1, over[:, None])[:, 0], pre[:, 128]
+    assert float((bound + moved - best - 128 * 2 ** -24 * moved).max()) <= 0.0
+    lost = 256 * 2 ** -19 + (30 * 2 ** -24 * v * v + 2 ** -24).sum(1)
+    room = (bound + moved) * 1.0042 + lost - best
+    say("least room under the limit, relative", float((room / best.clamp_min(1e-3)).min()))
+    assert float(room.min()) >= 0.0
+
+
 def test_viterbi_by_products_under_capture():
     """Captured and replayed on other tiles, with eager work between."""
     from glq_amd import ext
