@@ -654,6 +654,27 @@ def test_bounds_of_the_products_are_bounds():
     assert float(room.min()) >= 0.0
 
 
+def test_quantize_matrix_by_products_over_several_chips():
+    """2048 x 1088 at K = 4: two chips of tiles one after the other through the same rows, and a rest, read and written in the
+    matrix; some tiles left in either chip and some not tried.  The packed exact states."""
+    from glq_amd import ext
+    say("quantize matrix by products")
+    m, n = 2048, 1088
+    g = torch.Generator().manual_seed(8)
+    X = torch.randn(m * n // 256, 256, generator=g) * 0.9
+    X[::40] = torch.linspace(-3, 3, 256) + 1e-3 * torch.randn(X[::40].shape, generator=g)   # ramps show nothing beforehand and fill the lists
+    X[5::500] *= 8
+    W = ext.trellis_tiles_to_matrix(X.to(DEV), m, n)
+    packed, recon = ext.trellis_quantize_matrix(W, 4)
+    tiles = ext.trellis_matrix_to_tiles(W)
+    states, tried, left = _quantize_counts(tiles.cpu(), 4)
+    assert tried == X.shape[0] - 18 and left >= 200, (tried, left)
+    ref = _exact_states(X, 4)
+    assert torch.equal(tiles.cpu(), X) and torch.equal(states, ref)
+    assert torch.equal(packed, ext.trellis_pack_states(ref, m, n, 4))
+    assert torch.equal(ext.glq_decompress_trellis_3inst_cuda(packed, m, n).float(), recon)
+
+
 def test_viterbi_by_products_under_capture():
     """Captured and replayed on other tiles, with eager work between."""
     from glq_amd import ext
