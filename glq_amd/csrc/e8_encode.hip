@@ -7,6 +7,7 @@
 // expansion, 8 FMAs + 1 FMA + compare + 2 selects per (vector, row).  The dot product is
 // summed in coordinate order in fp32 with fused multiply-adds and the distance is
 // fma(-2, dot, norm): for fp32 inputs this is the arithmetic of the reference's CPU branch.
+#include <type_traits>
 #include "common.h"
 
 namespace {
@@ -99,7 +100,6 @@ e8_quantize_kernel(const float *__restrict__ x, const float *__restrict__ table,
 // and the rest to each wave alone, 33.5 -> 32 us, 131072 vectors 22.6 -> 19.7, 960 18.2 -> 16.7; of scale 2, where nearly all
 // vectors have them, 131072 vectors 110 -> 50 us, and of scale 20, 200 -> 176.  Of 32 us the kernel takes 28: half of that
 // the first pass (bound by VALU instructions), a quarter the first points, the rest trips through the lists and the table.
-// (Of scale 0.5, with a vector or two for a workgroup to list, 524288 take 21.6 us, not 21.)
 constexpr int ES_THREADS = 256;
 constexpr int ES_PLACES = 117361;                              // E8 points of norm up to 12
 constexpr int ES_FULL = GLQH_E8_SHELL_MIN_ROWS;                // of norm up to 10: all of them are rows of the table
@@ -112,6 +112,10 @@ constexpr int ES_WAVE = ES_GROWN / 4;                          // of the orbits 
 // Points in wait from which a wave takes a lane for each rather than eight: times of 16, 24, 40, 64 are 149, 149, 152, 169 us
 // at 131072 vectors of scale 4 and level at unit scale.
 constexpr int ES_MANY = 24;
+// Vectors to list up to which a workgroup's first points go to the waves as they are found.  (Those of the known orbits and their
+// children, counted and then placed, are some 1500 instructions, whoever has them: with them for every workgroup 960 vectors of scale 0.5 took
+// 13.6 us, not 12.5, 8000 of scale 0.25 13.8, not 12.7, 524288 21.6, not 21.0.  At 8 and 16 vectors for the line level or slower.)
+constexpr int ES_FEW = 32;
 static_assert(ES_THREADS == 2 * ES_CHUNK && 16 * 25 <= ES_LIST - ES_GROWN && 16 * 25 * 8 <= 2 * ES_GROWN,
               "two threads a vector; the orbits of the fewest vectors fit, and most of their points' children");
 constexpr int ES_SPLIT = 128;                                  // parts of the table in the exact walk
@@ -551,32 +555,45 @@ e8_shell_kernel(const es_args a) {
             const float reach = b1 + margin;
 #pragma unroll
             for (o = 0; o < 25; ++o) room[o] = on ? reach - room[o] : -1.0f;
-            int seeds = 0, children = 0;
-            o = 0;
-            auto count = [&](float, uint32_t code) {
-                if (o / 13 == half) {
-                    seeds += room[o] >= 0.0f;
-                    es_children(code, y, room[o], [&](float, uint32_t) { ++children; });
-                }
-                ++o;
-            };
-            es_orbits(y, count);
-            es_orbits_12(y, count);
-            int at = ES_GROWN + es_places(seeds, &n_seed), to = es_places(children, &n_child);
-            if (step == 16 || __ballot(at + seeds > ES_LIST || to + children > ES_GROWN / 2) == 0) {
+            if (nf <= ES_FEW) {                                // points like the others, whose children the waves find
                 o = 0;
                 auto list = [&](float, uint32_t code) {
-                    if (o / 13 == half) {
-                        if (room[o] >= 0.0f) put(at++, ES_LIST, code, mine, 0.0f);
-                        es_children(code, y, room[o], [&](float gap, uint32_t child) {   // dealt out to the waves
-                            put((to & 3) * ES_WAVE + (to >> 2), ((to & 3) + 1) * ES_WAVE, child, mine, room[o] - gap);
-                            ++to;
-                        });
+                    if (o / 13 == half && room[o] >= 0.0f) {
+                        const int to = atomicAdd(&n_child, 1);
+                        put((to & 3) * ES_WAVE + (to >> 2), ((to & 3) + 1) * ES_WAVE, code, mine, room[o]);
                     }
                     ++o;
                 };
                 es_orbits(y, list);
                 es_orbits_12(y, list);
+            } else {
+                int seeds = 0, children = 0;
+                o = 0;
+                auto count = [&](float, uint32_t code) {
+                    if (o / 13 == half) {
+                        seeds += room[o] >= 0.0f;
+                        es_children(code, y, room[o], [&](float, uint32_t) { ++children; });
+                    }
+                    ++o;
+                };
+                es_orbits(y, count);
+                es_orbits_12(y, count);
+                int at = ES_GROWN + es_places(seeds, &n_seed), to = es_places(children, &n_child);
+                if (step == 16 || __ballot(at + seeds > ES_LIST || to + children > ES_GROWN / 2) == 0) {
+                    o = 0;
+                    auto list = [&](float, uint32_t code) {
+                        if (o / 13 == half) {
+                            if (room[o] >= 0.0f) put(at++, ES_LIST, code, mine, 0.0f);
+                            es_children(code, y, room[o], [&](float gap, uint32_t child) {   // dealt out to the waves
+                                put((to & 3) * ES_WAVE + (to >> 2), ((to & 3) + 1) * ES_WAVE, child, mine, room[o] - gap);
+                                ++to;
+                            });
+                        }
+                        ++o;
+                    };
+                    es_orbits(y, list);
+                    es_orbits_12(y, list);
+                }
             }
         }
         __syncthreads();
@@ -646,15 +663,17 @@ e8_shell_kernel(const es_args a) {
                 n_left[wave] = n - done;
             }
             __syncthreads();
-            // the points that the table holds, by the walk's arithmetic, two at a time: three trips to memory each
+            // the points that the table holds, by the walk's arithmetic: three trips to memory each, two points at a time where there
+            // are more than threads (where there are not, the second one's trips cost 0.1-0.3 us)
             const int g0 = n_grown[0], g1 = g0 + n_grown[1], g2 = g1 + n_grown[2], g3 = g2 + n_grown[3];
             const int some = g3 + seeds;
-            for (int q0 = tid; q0 < some; q0 += 2 * ES_THREADS) {
-                int j[2], row[2];
-                uint32_t code[2];
-                float xv[2][8];
+            auto compare = [&](int q0, auto points) {
+                constexpr int U = decltype(points)::value;
+                int j[U], row[U];
+                uint32_t code[U];
+                float xv[U][8];
 #pragma unroll
-                for (int u = 0; u < 2; ++u) {
+                for (int u = 0; u < U; ++u) {
                     const int q = min(q0 + u * ES_THREADS, some - 1);
                     const int e = q < g0 ? q : q < g1 ? ES_WAVE + q - g0 : q < g2 ? 2 * ES_WAVE + q - g1 : q < g3 ? 3 * ES_WAVE + q - g2 : ES_GROWN + q - g3;
                     j[u] = list_j[e];
@@ -664,16 +683,16 @@ e8_shell_kernel(const es_args a) {
                     for (int r = 0; r < 8; ++r) k[r] = sk[r][j[u]];
                     code[u] = es_code(list_p[e], k, s_signs[j[u]], (s_signs[j[u]] >> 8) & 1u);
                 }
-                int place[2];
+                int place[U];
 #pragma unroll
-                for (int u = 0; u < 2; ++u) place[u] = es_place(code[u]);
+                for (int u = 0; u < U; ++u) place[u] = es_place(code[u]);
 #pragma unroll
-                for (int u = 0; u < 2; ++u) row[u] = a.row_at[place[u]];
+                for (int u = 0; u < U; ++u) row[u] = a.row_at[place[u]];
 #pragma unroll
-                for (int u = 0; u < 2; ++u)                        // not held: the place is not set
+                for (int u = 0; u < U; ++u)                        // not held: the place is not set
                     if ((uint32_t)row[u] >= (uint32_t)a.n_entries || a.place_of[row[u]] != place[u]) row[u] = -1;
 #pragma unroll
-                for (int u = 0; u < 2; ++u) {
+                for (int u = 0; u < U; ++u) {
                     if (row[u] < 0 || q0 + u * ES_THREADS >= some) continue;
                     float c[8];
                     int n4 = 0;
@@ -685,6 +704,11 @@ e8_shell_kernel(const es_args a) {
                     }
                     atomicMin(&best[j[u]], es_key(es_dist(xv[u], c, 0.25f * (float)n4), row[u]));
                 }
+            };
+            if (some <= ES_THREADS) {
+                if (tid < some) compare(tid, std::integral_constant<int, 1>());
+            } else {
+                for (int q0 = tid; q0 < some; q0 += 2 * ES_THREADS) compare(q0, std::integral_constant<int, 2>());
             }
             if ((n_left[0] | n_left[1] | n_left[2] | n_left[3]) == 0) break;
             __syncthreads();

@@ -122,6 +122,24 @@ def test_e8_quantize_of_many_points_in_reach(N, scale):
     assert torch.equal(dec, wdec)
 
 
+@pytest.mark.parametrize("N,V", [(256, 63), (65600, 256), (262200, 256)])
+def test_e8_quantize_on_either_side_of_few_vectors_to_list(N, V):
+    """Workgroups with one vector outside the table, with 31, 32 and 33 (the most whose points go to the waves as they are found), and with
+    none: the walk's own index and codeword."""
+    from glq_amd import ext
+    say("e8 shell search, few to list", N)
+    g = torch.Generator().manual_seed(N)
+    X = torch.randn(N, 8, generator=g) * 0.05
+    for i, k in enumerate((1, 31, 32, 33, 0, 48)):
+        at = i * 1024 % N + torch.randperm(min(V, 256), generator=g)[:k]
+        X[at] = torch.randn(k, 8, generator=g) * 3 + 1
+    cb = torch.from_numpy(O.e8_table()).to(DEV)
+    X = X.to(DEV)
+    dec, idx = ext.e8_quantize(X, cb)
+    wdec, walk = _walk(X, cb, (cb * cb).sum(-1))
+    assert torch.equal(idx, walk) and torch.equal(dec, wdec), int((idx != walk).sum())
+
+
 def _changed_table(how):
     cb = torch.from_numpy(O.e8_table()).to(DEV)
     if how == "rows in another order":                           # still the shell table
