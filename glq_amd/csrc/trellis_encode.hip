@@ -360,7 +360,7 @@ viterbi_kernel(const float *__restrict__ tiles_in, int64_t n_tiles, int64_t ld, 
 // and viterbi_kernel's costs of both paths, from which it takes the cheaper; 4 e < VB_NEAR.)  Where another kept path is
 // within VB_NEAR of the cheapest (3 % of the tiles), fp32 costs are evaluated forward over the kept ways, minima and lowest
 // states as in viterbi_kernel.
-// Tiles with inputs above VB_X, not finite or all equal are not tried, and those with more kept ways than fit, at K = 4 also at half the
+// Tiles with inputs above VB_X, not finite or all equal are not tried, and those with more kept ways than fit, behind vm_kernel also at half the
 // slack, are left: lists of both go to viterbi_kernel (with marks instead of lists, every workgroup walking its share of all tiles, it took the
 // time of all of them where half were marked).  Far beyond the weights' range the cost is mostly what no path can avoid,
 // and SLACK of that lets everything through: tiles with more than WIDE of it are not tried either (K = 4: 5 % of those with
@@ -1012,8 +1012,11 @@ vm_kernel(const float *__restrict__ tiles_in, int64_t ld, vb_lists lists, vb_par
 
 // A tile's working memory in LDS during the backtrack.  Level l is step l * DEPTH; its entries are the
 // kept ways from the groups of level l (parents: where the states lead) to those of level l - 1 (children).
+template <bool PRODUCT>
 struct vb_pool {
-    static constexpr int ENTRIES = 672;    // 550 at most in 3 * 10^4 tiles of Gaussian values, 170 on average
+    // 550 at most in 3 * 10^4 tiles of Gaussian values, 170 on average; behind vm_kernel what lets sixteen walk on a CU.  (672 behind
+    // vb_kernel too: of 2048 tiles of sigma 0.0001 891 left, not 657, 9.8 ms, not 8.9; of 0.001 368, not 133.)
+    static constexpr int ENTRIES = PRODUCT ? 672 : 768;
     float cost[ENTRIES];                   // of the entries: to the end
     uint16_t entry[ENTRIES];               // the digits of its states, nearest step first | parent << 8
     uint16_t via[ENTRIES];                 // of child j at j: best entry | its parent << 8 | close second << 14
@@ -1023,7 +1026,7 @@ struct vb_pool {
     float best[VB_MOST];
     int kept[VB_MOST];
 };
-static_assert(vb_pool::ENTRIES >= VB_MOST, "a level fits");
+static_assert(vb_pool<true>::ENTRIES >= VB_MOST, "a level fits");
 // states from group g by the digits p, nearest step first
 template <int K>
 __device__ __forceinline__ void vb_walk(int g, int p, int (&st)[vb_cfg<K>::DEPTH]) {
@@ -1041,9 +1044,9 @@ __device__ __forceinline__ void vb_walk(int g, int p, int (&st)[vb_cfg<K>::DEPTH
 // n, gv: the groups of step T (a lane each) whose bounds are within `limit`; x[i]: input of step i; the bounds' row of
 // level l at hist + (l - 1) * step; pre[j]: B at step j * VB_NORM; tie: the only group of step 0, or -1; the states up to
 // step `upto` are wanted.
-template <int K>
+template <int K, bool PRODUCT>
 __device__ __forceinline__ bool vb_trace(int n, int gv, float &limit, const f16 *x, const uint16_t *__restrict__ hist,
-                                         int64_t step, bool together, const float *pre, int tie, int upto, vb_pool *P, uint16_t *states) {
+                                         int64_t step, const float *pre, int tie, int upto, vb_pool<PRODUCT> *P, uint16_t *states) {
     using C = vb_cfg<K>;
     constexpr int D = C::DEPTH, LEVELS = C::STORED, R = (1 << (K * D)) / 64;
     const int lane = threadIdx.x & 63;
@@ -1060,7 +1063,7 @@ __device__ __forceinline__ bool vb_trace(int n, int gv, float &limit, const f16 
     {
         const int run = K == 4 ? lane >> 2 : K == 3 ? lane >> 3 : lane;   // the digits but the farthest, the nearest lowest
         const int in = K == 4 ? (lane & 3) * 4 : K == 3 ? lane & 7 : 0;
-        place = (run << (together ? K : E + K)) + in;
+        place = (run << (PRODUCT ? K : E + K)) + in;
 #pragma unroll
         for (int r = 0; r < R; ++r) {
             int k = in + r;
@@ -1072,7 +1075,7 @@ __device__ __forceinline__ bool vb_trace(int n, int gv, float &limit, const f16 
     // first group is known: they take longer than everything else here
     u32x2 ahead = {0, 0};
     auto ask = [&](int l, int g, u32x2 &into) {
-        const uint16_t *row = hist + (l > 1 ? l - 2 : 0) * step + place + (uint32_t)((g >> (K * D)) << (together ? K * D : K));
+        const uint16_t *row = hist + (l > 1 ? l - 2 : 0) * step + place + (uint32_t)((g >> (K * D)) << (PRODUCT ? K * D : K));
         if constexpr (R == 4) into = *(const u32x2 *)row;
         else into.x = *row;
     };
@@ -1360,14 +1363,15 @@ __device__ __forceinline__ bool vb_trace(int n, int gv, float &limit, const f16 
 }
 
 // A wave's memory while it walks back
+template <bool PRODUCT>
 struct vb_work {
-    vb_pool pool;
+    vb_pool<PRODUCT> pool;
     float pre[VT_T / VB_NORM + 1];
     alignas(8) f16 x[VT_T];
     uint16_t states[VT_T];
     int start[VB_MOST];
 };
-static_assert(sizeof(vb_work) <= 160 * 1024 / 16, "sixteen on a CU");
+static_assert(sizeof(vb_work<true>) <= 160 * 1024 / 16, "sixteen on a CU");
 
 // The backtrack of tile vb_first + at (one wave): after pass 0 the overlap, after pass 1 the states and values.
 // What bounds it is latency: a chain of STORED levels, each a look into a row of which only the last level's group tells
@@ -1376,9 +1380,9 @@ static_assert(sizeof(vb_work) <= 160 * 1024 / 16, "sixteen on a CU");
 // a level, and another near).  0.73 -> 0.58 by the kept groups' bounds in one piece, a short way where one way is in reach, and
 // the exact comparison's levels read ahead and its path found by the lanes.  (Two groups at a time, or the next level's
 // first two asked for: 0.69, in spilled scalar registers; a loop of its own for levels of one way: level.)
-template <int K>
+template <int K, bool PRODUCT>
 __device__ __forceinline__ void vb_backtrack(const float *__restrict__ tiles_in, int64_t ld, const vb_lists &lists,
-                                             const vb_part &part, int at, vb_work *W, int32_t *__restrict__ states_out, float *__restrict__ hat_out) {
+                                             const vb_part &part, int at, vb_work<PRODUCT> *W, int32_t *__restrict__ states_out, float *__restrict__ hat_out) {
     using C = vb_cfg<K>;
     float *const pre = W->pre;
     f16 *const x = W->x;
@@ -1397,7 +1401,7 @@ __device__ __forceinline__ void vb_backtrack(const float *__restrict__ tiles_in,
     }
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) lost += __shfl_xor(lost, d, GLQH_WAVE);
-    lost = K == 4 && part.product ? VT_T * VM_FLOOR * 0x1p-10f + lost : VB_LOST;   // (2^-10: a rounding of the least bounds)
+    lost = PRODUCT ? VT_T * VM_FLOOR * 0x1p-10f + lost : VB_LOST;   // (2^-10: a rounding of the least bounds)
     for (int i = lane; i <= VT_T / VB_NORM; i += 64) pre[i] = mine->pre[i];
     const int64_t step = (int64_t)part.count * C::G;
     const uint16_t *hist = part.rows + (int64_t)at * C::G, *last = hist + (C::STORED - 1) * step;
@@ -1405,7 +1409,7 @@ __device__ __forceinline__ void vb_backtrack(const float *__restrict__ tiles_in,
     const float bt = pre[VT_T / VB_NORM];
     uint32_t lo = 0xFFFFu;                                     // the least bound of the groups that may be last
     if (pass) {
-        lo = last[part.product ? vb_together<K>(vb_stored<K>(tie)) : vb_stored<K>(tie)];
+        lo = last[PRODUCT ? vb_together<K>(vb_stored<K>(tie)) : vb_stored<K>(tie)];
     } else {
 #pragma unroll 8
         for (int g = 0; g < C::G; g += 64) {
@@ -1416,9 +1420,9 @@ __device__ __forceinline__ void vb_backtrack(const float *__restrict__ tiles_in,
     }
     const float least = vb_lane(vb_half(lo) + bt, 0);
     float limit = vb_lane(least * (1.0f + C::SLACK) + lost, 0);
-    // below K = 4 a second walk takes longer than the exact search over what it saves (K = 2, 1024 slow ramps 5.2 -> 7.1 ms with it, normal
-    // values of sigma 2.2, where it saves 180 of 4096, 11.0 -> 11.4; K = 3, sigma 2.0, where it saves 210, 12.7 -> 13.0)
-    float lower = K < 4 ? __builtin_inff() : limit - 0.5f * (limit - least);
+    // behind vb_kernel a second walk takes longer than the exact search over what it saves, a tile a CU at a time (K = 2, 1024 slow ramps 5.2 ->
+    // 7.1 ms with it; K = 3, 4096 tiles of sigma 2.0 12.7 -> 13.0; K = 4, 1024 of 1.5 3.8 -> 4.4, though 3000 of 1.7 10.4 -> 9.6)
+    float lower = PRODUCT ? limit - 0.5f * (limit - least) : __builtin_inff();
     bool good = false;
 #pragma unroll 1
     for (int tries = 0; tries < 4; ++tries) {
@@ -1439,7 +1443,7 @@ __device__ __forceinline__ void vb_backtrack(const float *__restrict__ tiles_in,
                 for (int k = 0; k < 8; ++k) {
                     const uint64_t mask = __ballot(b[k] <= limit);
                     const int at = n + vb_below(mask);
-                    if (b[k] <= limit && at < VB_MOST) start[at] = vb_group<K>(part.product ? vb_apart<K>(g0 + 64 * k + lane) : g0 + 64 * k + lane);
+                    if (b[k] <= limit && at < VB_MOST) start[at] = vb_group<K>(PRODUCT ? vb_apart<K>(g0 + 64 * k + lane) : g0 + 64 * k + lane);
                     n += __builtin_popcountll(mask);
                 }
             }
@@ -1447,9 +1451,9 @@ __device__ __forceinline__ void vb_backtrack(const float *__restrict__ tiles_in,
         __builtin_amdgcn_wave_barrier();
         n = __builtin_amdgcn_readfirstlane(n);
         if (n > VB_MOST) limit = __builtin_inff();
-        else good = vb_trace<K>(n, lane < n ? start[lane] : 0, limit, x, hist, step, part.product, pre, tie, pass ? VT_T - 1 : VT_T / 2, &W->pool, states);
+        else good = vb_trace<K, PRODUCT>(n, lane < n ? start[lane] : 0, limit, x, hist, step, pre, tie, pass ? VT_T - 1 : VT_T / 2, &W->pool, states);
         if (good) break;
-        if (limit == __builtin_inff()) {                       // too many ways for the lists: half the slack may do at K = 4
+        if (limit == __builtin_inff()) {                       // too many ways for the lists: half the slack may do
             limit = lower;
             lower = __builtin_inff();
         }
@@ -1473,7 +1477,7 @@ __device__ __forceinline__ void vb_backtrack(const float *__restrict__ tiles_in,
 constexpr int VB_WALK = 4;
 template <int K, int TPW>
 constexpr int vb_lds() {
-    constexpr int rows = TPW * vb_cfg<K>::ROWS * vb_cfg<K>::ROW * 4, walk = VB_WALK * (int)sizeof(vb_work);
+    constexpr int rows = TPW * vb_cfg<K>::ROWS * vb_cfg<K>::ROW * 4, walk = VB_WALK * (int)sizeof(vb_work<false>);
     return rows > walk ? rows : walk;
 }
 template <int K, int TPW>
@@ -1485,7 +1489,7 @@ vb_kernel(const float *__restrict__ tiles_in, int64_t ld, vb_lists lists, vb_par
         const int wave = threadIdx.x >> 6, at = blockIdx.x * VB_WALK + wave;
         if (wave >= VB_WALK || at >= vb_count(back, lists)) return;
         __builtin_amdgcn_s_setprio(3);
-        vb_backtrack<K>(tiles_in, ld, lists, back, at, (vb_work *)lds + wave, states_out, hat_out);
+        vb_backtrack<K, false>(tiles_in, ld, lists, back, at, (vb_work<false> *)lds + wave, states_out, hat_out);
     } else {
         vb_forward<K, TPW>(tiles_in, ld, lists, forward, blockIdx.x - walkers, gridDim.x - walkers, lds);
     }
@@ -1495,8 +1499,8 @@ vb_kernel(const float *__restrict__ tiles_in, int64_t ld, vb_lists lists, vb_par
 __global__ void __launch_bounds__(GLQH_WAVE, 4)
 vm_walk_kernel(const float *__restrict__ tiles_in, int64_t ld, vb_lists lists, vb_part back, int32_t *__restrict__ states_out,
                float *__restrict__ hat_out) {
-    __shared__ vb_work work;
-    if ((int)blockIdx.x < vb_count(back, lists)) vb_backtrack<4>(tiles_in, ld, lists, back, blockIdx.x, &work, states_out, hat_out);
+    __shared__ vb_work<true> work;
+    if ((int)blockIdx.x < vb_count(back, lists)) vb_backtrack<4, true>(tiles_in, ld, lists, back, blockIdx.x, &work, states_out, hat_out);
 }
 
 // states (tiles in row-major tile order, 256 steps each) -> packed kernel layout: the chunk of

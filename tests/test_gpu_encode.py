@@ -448,6 +448,16 @@ def test_wide_tiles_at_3_bits_are_left_at_their_first_overflow():
     assert torch.equal(states, _exact_states(X, 3))
 
 
+def test_tiny_values_at_4_bits_fit_the_lists():
+    """Normal values of sigma 1e-4 keep many ways: lists of 768 leave three tiles in ten (of 672 four and more), a call of less
+    than twelve tiles a CU without a second walk; the exact states."""
+    say("tiny values at 4 bits")
+    X = torch.randn(1024, 256, generator=torch.Generator().manual_seed(4)) * 1e-4
+    states, tried, left = _quantize_counts(X, 4)
+    assert tried == 1024 and 256 <= left <= 384, (tried, left)
+    assert torch.equal(states, _exact_states(X, 4))
+
+
 @pytest.mark.parametrize("K,m,n", [(2, 256, 320), (3, 288, 256), (4, 512, 576)])
 def test_quantize_matrix_on_bounds_equals_the_tile_route(K, m, n):
     """More tiles than CUs, whose places in the matrix the lists tell, all but two of them on bounds: the tile route, bit for bit."""
