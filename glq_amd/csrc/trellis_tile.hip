@@ -851,13 +851,16 @@ int tt_rest(const tt_plan &p);
 
 // Microseconds a plan for more than 256 tokens is expected to take, but for what all plans share.  Steps of a round cost what
 // the chip's power allows (1.76 us with all CUs on 512-token tiles, 1.03 on 256) in proportion to the CUs that have a tile, and
-// no less than a step's chain (1.32, 0.82); a last round on few of them may run as half tiles (0.53 us a step) or, of a layer
-// on its own, as 256-token tiles; K slots add their sums, 3 bytes each (between fp16 and fp32: the K-slot query and the launch
-// must arrive at the same plan, whatever the width the sums leave with).
-double tt_plan_cost(const tt_plan &p, int64_t m, int64_t M, bool alone) {
+// no less than a step's chain (1.32, 0.82); at 2 and 3 bits, whose records take more instructions to part, 1.9, 0.95, 1.7 and 0.9.  A last
+// round on few of them may run as half tiles (0.53 us a step) or, of a layer on its own, as 256-token tiles; K slots add their
+// sums, 3 bytes each (between fp16 and fp32).
+double tt_plan_cost(const tt_plan &p, int64_t m, int64_t M, bool alone, int R) {
     const int cus = glqh_device_cus();
     const int64_t items = (int64_t)p.RT * p.TT * p.KS, full = items / cus, rem = items % cus;
-    auto step = [&](int ntw, double share) { return ntw == 4 ? std::max(1.32, 1.76 * share) : std::max(0.82, 1.03 * share); };
+    auto step = [&](int ntw, double share) {
+        if (R < 4) return ntw == 4 ? std::max(1.7, 1.9 * share) : std::max(0.9, 0.95 * share);
+        return ntw == 4 ? std::max(1.32, 1.76 * share) : std::max(0.82, 1.03 * share);
+    };
     double t = (double)full * step(p.NTW, 1.0);
     if (rem) {
         double last = step(p.NTW, (double)rem / cus);
@@ -894,10 +897,12 @@ double tt_split_cost(const tt_plan &p, int64_t m, int64_t M) {
 
 // Up to 256 tokens the tile follows the token count; above, 512-token tiles unless 256-token tiles are expected to be 3 %
 // faster: where they waste less on padding (2 x 14336 rows x 4096 columns at 768 tokens 261 -> 236 us, the whole call) or leave a
-// shorter last round.  GLQ_TT_NTW forces a tile above 256 tokens.
+// shorter last round.  Over 600 random calls (512-14336 rows and columns, groups up to 60160 rows, 257-4096 tokens) the rule loses 0.2 % of
+// the sum to the faster tile at 4 bits, 0.1 at 2 and 0.4 at 3; with the costs of 4 bits it lost 3.5 and 1.9 there (7168 x 5888 at
+// 1087 tokens and 2 bits 182 us, not 166; 4352 x 8192 at 2048 and 3 bits 257, not 229).  GLQ_TT_NTW forces a tile above 256 tokens.
 // max_ntw = 2: a stacked layer decoded into one operand (two streams' records and temporaries do not fit beside the
 // accumulators of a 512-token tile).
-void tt_make_plan(int64_t m, int64_t k, int64_t M, tt_plan *p, int max_ntw = 4, bool alone = true) {
+void tt_make_plan(int64_t m, int64_t k, int64_t M, tt_plan *p, int R, int max_ntw = 4, bool alone = true) {
     const int top = std::min(tt_ntw(M), max_ntw);
     tt_plan_for(top, m, k, M, p);
     static const bool forced = getenv("GLQ_TT_NTW") != nullptr;
@@ -911,7 +916,7 @@ void tt_make_plan(int64_t m, int64_t k, int64_t M, tt_plan *p, int max_ntw = 4, 
         q->slot_ds = slot_ds;
         q->grid = (int)std::min<int64_t>((int64_t)q->RT * q->TT * KS, glqh_device_cus());
     }
-    if (tt_plan_cost(p2, m, M, alone) < 0.97 * tt_plan_cost(*p, m, M, alone)) *p = p2;
+    if (tt_plan_cost(p2, m, M, alone, R) < 0.97 * tt_plan_cost(*p, m, M, alone, R)) *p = p2;
 }
 
 // Tiles of up to 256 tokens run with decoding and multiplying waves (the tr_tile_*_pc_kernel forms) when a K
@@ -1025,7 +1030,7 @@ size_t glqh_trellis_tile_xb_bytes(int64_t k, int64_t M) { return (size_t)tt_padd
 // K slots the many-token kernel uses for this call (1: it can write the result in place)
 int glqh_trellis_tile_ksplit(int64_t m, int64_t k, int64_t M, int two_stage) {
     tt_plan p;
-    tt_make_plan(m, k, M, &p, two_stage ? 2 : 4);
+    tt_make_plan(m, k, M, &p, 4, two_stage ? 2 : 4);            // (the slots are those of every rate)
     return p.KS;
 }
 
@@ -1043,7 +1048,7 @@ int glqh_launch_trellis_tile(const void *x_f16, void *xb_scratch, int64_t M, con
                              hipStream_t stream, int out_f16, const void *packed2, int R2, float rs2) {
     if (packed2 && R != 4) return glqh_fail("trellis tile kernel: two streams in one operand need a first stage of 4 bits/weight");
     tt_plan p;
-    tt_make_plan(m, k, M, &p, packed2 ? 2 : 4);
+    tt_make_plan(m, k, M, &p, R, packed2 ? 2 : 4);
     if (direct && p.KS != 1) return glqh_fail("trellis tile kernel: in-place output needs a single K slot");
     if (out_f16 && (direct || M <= 64)) return glqh_fail("trellis tile kernel: fp16 sums are partial sums of the large tiles");
     const int Mp = (int)tt_padded_tokens(M);
@@ -1142,10 +1147,10 @@ int glqh_launch_trellis_tile(const void *x_f16, void *xb_scratch, int64_t M, con
 
 // ---- several layers in one launch (more than 16 tokens) -------------------------------------------
 namespace {
-void tt_make_group_plan(const int64_t *m, int n_layers, int64_t k, int64_t M, int two_stage, tt_plan *p) {
+void tt_make_group_plan(const int64_t *m, int n_layers, int64_t k, int64_t M, int two_stage, tt_plan *p, int R = 4) {
     int64_t rt = 0;
     for (int l = 0; l < n_layers; ++l) rt += (m[l] + TT_ROWS - 1) / TT_ROWS;
-    tt_make_plan(TT_ROWS * rt, k, M, p, two_stage ? 2 : 4, false);   // same rule, on the row tiles of all layers
+    tt_make_plan(TT_ROWS * rt, k, M, p, R, two_stage ? 2 : 4, false);   // same rule, on the row tiles of all layers
 }
 
 #define GLQH_TTG(...)                                                                                      \
@@ -1196,7 +1201,7 @@ int glqh_launch_trellis_tile_group(const void *const xb[], int64_t M, const void
     GLQH_REQUIRE(M > 16 && (M > 64 || !out_f16), "trellis tile group: more than 16 tokens (64 for fp16 sums)");
     GLQH_REQUIRE(!packed2 || R == 4, "trellis tile group: two streams in one operand need first stages of 4 bits/weight");
     tt_plan p;
-    tt_make_group_plan(m, n_layers, k, M, packed2 != nullptr, &p);
+    tt_make_group_plan(m, n_layers, k, M, packed2 != nullptr, &p, R);
     tt_args a = {};
     tt_group g = {};
     g.n = n_layers;

@@ -171,6 +171,12 @@ def test_matmul_tiles_in_uneven_shares(ext, m, n, B, K):
     test_matmul_last_round_of_half_tiles(ext, m, n, B, K)
 
 
+@pytest.mark.parametrize("m,n,B,K", [(16992, 1024, 269, 2), (16992, 1024, 269, 3), (17984, 1024, 261, 2), (16992, 1024, 269, 4)])
+def test_matmul_tiles_by_rate(ext, m, n, B, K):
+    """Calls that run as 256-token tiles at 2 and 3 bits and as 512-token tiles at 4.  The same bound."""
+    test_matmul_last_round_of_half_tiles(ext, m, n, B, K)
+
+
 @pytest.mark.parametrize("m,n,B,K2", [(32768 + 32, 512, 200, 2), (32768 + 224, 576, 130, 1), (32768 + 96, 512, 129, 4),
                                       (10976, 1024, 999, 3)])
 def test_two_stage_last_round_of_half_tiles(ext, m, n, B, K2):
