@@ -50,15 +50,15 @@ struct glqh_range {
     } while (0)
 
 // ---- small device helpers -----------------------------------------------------
-// This workgroup's share of n items in a persistent grid: first, first + step, ... below end.  Workgroups whose numbers are
-// equal mod 8 run on one XCD and share its L2; each XCD takes a run of items, as long as it has workgroups for them where there
-// is a workgroup to an item.  (Runs of ceil(n / 8) gave 22 items to XCDs with 21 of 172 workgroups, and the call a second round:
-// 2 x 11008 rows of 2048 columns, tiles of 512 tokens, 102 us instead of 57.)
-struct glqh_share { int first, end, step; };
+// This workgroup's share of n items in a persistent grid: items from + w, w = first, first + step, ... below count.  Workgroups whose
+// numbers are equal mod 8 run on one XCD and share its L2; each XCD takes a run of items, as long as it has workgroups for them where
+// there is a workgroup to an item.  (Runs of ceil(n / 8) gave 22 items to XCDs with 21 of 172 workgroups, and the call a second round:
+// 2 x 11008 rows of 2048 columns, tiles of 512 tokens, 102 us instead of 57.  A loop over the items themselves makes three-stage
+// layers 2-3 % slower: 2048 x 14016 at 2118 tokens 264.7 -> 271.5.)
+struct glqh_share { int from, first, count, step; };
 __device__ __forceinline__ glqh_share glqh_xcd_share(int n) {
     const int xcd = blockIdx.x & 7, each = n >> 3, more = n & 7;
-    const int start = xcd * each + (xcd < more ? xcd : more);
-    return {start + (int)(blockIdx.x >> 3), start + each + (xcd < more ? 1 : 0), ((int)gridDim.x - xcd + 7) >> 3};
+    return {xcd * each + (xcd < more ? xcd : more), (int)(blockIdx.x >> 3), each + (xcd < more ? 1 : 0), ((int)gridDim.x - xcd + 7) >> 3};
 }
 
 __device__ __forceinline__ float bf16_bits_to_f32(uint16_t b) {

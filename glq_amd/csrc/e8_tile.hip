@@ -119,7 +119,8 @@ e8_tile_kernel(const et_args a) {
     // the same activations at the same time.
     const int nitems = a.TT * a.KS * a.RT;
     const glqh_share share = glqh_xcd_share(nitems);
-    for (int item = share.first; item < share.end; item += share.step) {
+    for (int w = share.first; w < share.count; w += share.step) {
+        const int item = share.from + w;
         const int rt = item % a.RT, slot = (item / a.RT) % a.KS, tt0 = item / (a.RT * a.KS);
         const int r0 = rt * ET_ROWS, tok0 = tt0 * (ET_WAVES * 16 * NTW) + wave * 16 * NTW;
         const int ds0 = slot * a.slot_ds, ds1 = min(ds0 + a.slot_ds, nds);

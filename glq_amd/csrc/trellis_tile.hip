@@ -221,7 +221,8 @@ __device__ __forceinline__ void tr_tile_body(const tt_args &a, const tt_group &g
     int nitems = a.TT * a.KS * RT;
     if constexpr (MOE) nitems = *mo.n_tiles * a.RT * a.TT;      // one K slot; TT = workgroup tiles per run
     const glqh_share share = glqh_xcd_share(nitems);
-    for (int item = share.first; item < share.end; item += share.step) {
+    for (int w = share.first; w < share.count; w += share.step) {
+        const int item = share.from + w;
         const int slot = (item / RT) % a.KS, tt0 = item / (RT * a.KS);
         int rt = HALF ? a.RT + (item % RT >> 1) : a.rt0 + item % RT;   // row tile of its layer
         const int unit = HALF ? item % RT & 1 : dw >> 2;        // block pair of the row tile that this wave decodes
