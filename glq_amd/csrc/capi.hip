@@ -725,7 +725,9 @@ extern "C" int glqh_fused_linear_trellis_3inst_noalloc(
 //                     2048 -> 2 x 11008 19.6 / 20.9, 3392 -> 2 x 7040 25.1 / 20.8
 //   4 bits, 4 tokens  960 18.0 / 12.6, 2048 15.8 / 13.4; 2048 -> 2 x 11008 22.5 / 21.5
 // The lines at one token are drawn with four waves a SIMD and one grid over all strips (the kernels above had three and a
-// plane per layer; two and four tokens stand).  Whole call, us, folded / separate, 4 bits and 4 + 2, by Mi weights of the group:
+// plane per layer).  At two tokens these kernels are level with those, 0.997 of the time over 82 layers and 38 groups at 2 and 4 bits, and the
+// lines 1.5-2.1 % above the faster route.  Whole call, one token, us, folded / separate, 4 bits and 4 + 2, by Mi weights of the group (the
+// same lines at 2 and 3 bits are 2 % above the faster route over 53 groups, those of single layers 1 % over 98):
 //   whole slots (256)  4608 wide 36 14.4 / 16.4, 20.8 / 23.1; 5120 35 16.2 / 16.7, 23.5 / 22.9; 6144 48 16.6 / 17.5, 24.0 / 24.9; 7168 42 16.6 /
 //                      17.6, 24.0 / 25.1; 8192 48 17.4 / 18.6, 25.2 / 26.0, 80 28.2 / 25.5, 43 / 37; 4096 48 16.1 / 17.1, 24.1 / 24.8, 56 18.2 /
 //                      18.2, 27.9 / 27.0, 64 19.3 / 20.2, 28.9 / 29.8, 86 26.6 / 24.6; 3840 60 19.7 / 19.2; 3584 56 17.5 / 18.8, 24.6 / 27.2,

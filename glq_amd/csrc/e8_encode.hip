@@ -97,8 +97,8 @@ e8_quantize_kernel(const float *__restrict__ x, const float *__restrict__ table,
 // by every call (es_index_kernel 4 us; 250 -> 52 us where the table is new); 960 vectors 12.7 ms -> 13.4 ->
 // 17.3 us: three dependent launches.  Then the lists, which a workgroup had filled an addition at a time and walked level
 // by level, a barrier each: with the first points and their children from the 25 known orbits, counted before they are placed,
-// and the rest to each wave alone, 33.5 -> 32 us, 131072 vectors 22.6 -> 19.7, 960 18.2 -> 16.7; of scale 2, where nearly all
-// vectors have them, 131072 vectors 110 -> 50 us, and of scale 20, 200 -> 176.  Of 32 us the kernel takes 28: half of that
+// and the rest to each wave alone, 33.5 -> 32 us, 131072 vectors 21.4 -> 18.5, 960 17.7 -> 15.8; of scale 2, where nearly all
+// vectors have them, 131072 vectors 109 -> 49 us, and of scale 20, 201 -> 175.  Of 32 us the kernel takes 28: half of that
 // the first pass (bound by VALU instructions), a quarter the first points, the rest trips through the lists and the table.
 constexpr int ES_THREADS = 256;
 constexpr int ES_PLACES = 117361;                              // E8 points of norm up to 12

@@ -367,13 +367,13 @@ viterbi_kernel(const float *__restrict__ tiles_in, int64_t n_tiles, int64_t ld, 
 // 2-3 are left, 23 % with 4-5, 64 % with 10-14; K = 3 and 2: 20 and 18 % of the first beyond), nor is a minority of up to two
 // chips full, nor the rest of a call after batches of which more than half were left.  4096 tiles, exact / so, ms:
 //   normal values of sigma      1e-4         0.9          1.6          1.8          2.2          3 and more
-//     K = 4                     17.5 / 17.7  17.5 / 8.2   17.5 / 11.1  17.4 / 15.8  17.4 / 17.6  17.5 / 17.6
-//     K = 4, through vm_kernel         10.4         6.4          9.4         15.4         17.6         17.6
-//     K = 3                     14.9 / 10.3  14.7 / 9.6   14.6 / 10.9  14.6 / 11.0  14.6 / 14.8  14.6 / 14.7
-//     K = 2                     16.7 / 8.1   16.7 / 9.6   16.7 / 10.4  16.8 / 10.8  16.7 / 12.2  16.7 / 16.7
-// Slower is what fills the lists and shows nothing beforehand, as slow ramps do (-3 to 3 over the tile's steps): 17.5 / 19.2,
-// 14.6 / 16.2, 16.7 / 18.7, up to 1.4 times in calls of one or two batches.  2048 x 2048 weights: 69.6 -> 32.7 at K = 4
-// (24.0 through vm_kernel), 58.6 -> 37.5 at 3, 66.6 -> 35.5 at 2.
+//     K = 4                     17.5 / 17.2  17.5 / 7.9   17.5 / 10.9  17.5 / 15.6  17.5 / 17.5  17.5 / 17.6
+//     K = 4, through vm_kernel         9.8          6.3          9.0         15.0         17.5         17.5
+//     K = 3                     14.7 / 9.9   14.7 / 9.5   14.6 / 10.8  14.6 / 11.0  14.6 / 14.5  14.6 / 14.6
+//     K = 2                     16.7 / 8.0   16.7 / 8.9   16.7 / 9.0   16.7 / 10.4  16.7 / 11.0  16.7 / 16.6
+// Slower is what fills the lists and shows nothing beforehand, as slow ramps do (-3 to 3 over the tile's steps): 17.5 / 19.1 (20.4
+// through vm_kernel, whose batches are larger; 70 % of a chip behind normal tiles 18.2 / 19.5), 14.6 / 16.3, 16.7 / 18.6, up to 1.3 times
+// in calls of one or two batches.  2048 x 2048 weights: 69.6 -> 32.7 at K = 4 (24.0 through vm_kernel), 58.6 -> 38.0 at 3, 66.6 -> 35.4 at 2.
 constexpr int VB_THREADS = 512;
 constexpr int VB_NORM = 2;                 // steps between two moves of the row's minimum into B
 constexpr float VB_X = 16.0f;              // largest input: (16 + 4)^2 for 16 / K steps stays far below 65504
@@ -808,8 +808,8 @@ __device__ __forceinline__ void vb_forward(const float *__restrict__ tiles_in, i
 // smallest numbers, and VM_LESS of c + e.  Bounds are rounded once a step, towards zero; a row's least one stays at VM_FLOOR,
 // above what comes off until the next move, so that none is negative.
 //
-// 4096 tiles, a pass: 2.6 ms, where vb_forward takes 3.7, and 0.58 for the walk back, which nothing overlaps.  Vector ALUs issue
-// in 59 % of the cycles (three quarters of that the minima) and the matrix cores work in 39 %, at 2.0 GHz; the rows on their
+// 4096 tiles, a pass: 2.6 ms, where vb_forward takes 3.7, and 0.6 for the walk back, which nothing overlaps.  Vector ALUs issue
+// in 62 % of the cycles (three quarters of that the minima) and the matrix cores work in 38 %, at 2.1 GHz; the rows on their
 // way to memory take 0.4 ms of it.  Measured and not kept: products a pair ahead of the minima (2.6, with the rows in one
 // piece; no registers for more), four waves a SIMD (eight tiles a workgroup, 128 registers: 3.4), eight tiles and two rows
 // (2.8), priorities of waves (level).
