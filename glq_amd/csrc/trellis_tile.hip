@@ -898,7 +898,7 @@ double tt_split_cost(const tt_plan &p, int64_t m, int64_t M) {
 
 // Up to 256 tokens the tile follows the token count; above, 512-token tiles unless 256-token tiles are expected to be 3 %
 // faster: where they waste less on padding (2 x 14336 rows x 4096 columns at 768 tokens 261 -> 236 us, the whole call) or leave a
-// shorter last round.  Over 600 random calls (512-14336 rows and columns, groups up to 60160 rows, 257-4096 tokens) the rule loses 0.2 % of
+// shorter last round.  Over 450 random calls (512-14336 rows and columns, groups up to 60160 rows, 257-4096 tokens) the rule loses 0.2 % of
 // the sum to the faster tile at 4 bits, 0.1 at 2 and 0.4 at 3; with the costs of 4 bits it lost 3.5 and 1.9 there (7168 x 5888 at
 // 1087 tokens and 2 bits 182 us, not 166; 4352 x 8192 at 2048 and 3 bits 257, not 229).  GLQ_TT_NTW forces a tile above 256 tokens.
 // max_ntw = 2: a stacked layer decoded into one operand (two streams' records and temporaries do not fit beside the
